@@ -1,6 +1,7 @@
-"""ctypes loader for libmemorax_amd.so (the C ABI declared in include/memorax_amd.h).
+"""Loader for libmemorax_amd.so (the C ABI declared in include/memorax_amd.h) and for the torch side of its
+calls, the extension module memorax_amd._native (csrc/host_ops.cpp), which is bound to the loaded library.
 
-There is no CPU fallback: if the library is missing, or a call returns a
+There is no CPU fallback: if the library or the module is missing, or a call returns a
 non-zero status, a RuntimeError is raised.
 """
 from __future__ import annotations
@@ -63,11 +64,12 @@ SIGNATURES = {
 }
 
 _lib = None
+_native = None
 
 
 def load():
-    """Load the shared library once and attach the prototypes."""
-    global _lib
+    """Load the shared library once, attach the prototypes and bind the extension module to it."""
+    global _lib, _native
     if _lib is not None:
         return _lib
     if not os.path.exists(LIB_PATH):
@@ -79,8 +81,20 @@ def load():
         fn = getattr(lib, name)  # AttributeError if the ABI is incomplete
         fn.restype = res
         fn.argtypes = args
-    _lib = lib
+    try:
+        from . import _native as module
+    except ImportError as e:
+        raise RuntimeError("memorax_amd._native not found: build it with memorax_amd/csrc/build.sh") from e
+    module.bind({name: ctypes.cast(getattr(lib, name), _P).value for name in SIGNATURES})
+    _lib, _native = lib, module
     return lib
+
+
+def native():
+    """The extension module, bound to the library."""
+    if _lib is None:
+        load()
+    return _native
 
 
 def check(status: int, what: str) -> None:

@@ -8,6 +8,8 @@
 #                          chunked kernels without their arithmetic); only bench.py loads it, for the share of a
 #                          wave's time that delta_bwd_kernel spends inside products and for what the kernels'
 #                          access pattern alone costs
+#   ../_native.so          the extension module memorax_amd._native: the torch side of the library's calls
+#                          (host_ops.cpp, host code only; bound to a build of the library when it is loaded)
 #   memorax_amd/csrc/build.sh
 set -euo pipefail
 cd "$(dirname "$0")"
@@ -37,6 +39,11 @@ SRCS=(chunk_bwd.hip)
 compile _clk -DMRX_PHASE_CLOCKS=1
 SRCS=(pattern_probe.hip)
 compile ""
+TORCH=$(python3 -c 'import os, torch; print(os.path.dirname(torch.__file__))')
+g++ -O2 -std=c++17 -fPIC -shared -fvisibility=hidden -Wall -D__HIP_PLATFORM_AMD__=1 -DUSE_ROCM=1 -I../../include \
+    -isystem "$TORCH/include" -isystem "$TORCH/include/torch/csrc/api/include" -isystem /opt/rocm/include $(python3-config --includes) \
+    host_ops.cpp -o ../_native.so -L"$TORCH/lib" -ltorch -ltorch_cpu -ltorch_hip -lc10 -lc10_hip -ltorch_python -Wl,-rpath,"$TORCH/lib" &
+pids+=($!)
 SRCS=("${ALL_SRCS[@]}")
 for p in "${pids[@]}"; do wait "$p"; done
 HD32_OBJS=$(printf '%s_hd32.o ' "${HD32_SRCS[@]%.hip}")
@@ -45,4 +52,4 @@ HD32_OBJS=$(printf '%s_hd32.o ' "${HD32_SRCS[@]%.hip}")
 CLK_OBJS=$(printf '%s.o ' "${SRCS[@]%.hip}" | sed 's/chunk_bwd\.o/chunk_bwd_clk.o/')
 "$HIPCC" --offload-arch=gfx950 -shared -fPIC -o libmemorax_amd_clk.so $CLK_OBJS pattern_probe.o $HD32_OBJS
 rm -f ./*.o
-echo "built $(pwd)/libmemorax_amd.so, libmemorax_amd_c64.so and libmemorax_amd_clk.so"
+echo "built $(pwd)/libmemorax_amd.so, libmemorax_amd_c64.so, libmemorax_amd_clk.so and ../_native.so"

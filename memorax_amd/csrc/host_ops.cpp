@@ -1,0 +1,1242 @@
+// The host side of the library for torch: what runs between a Python call and the kernel launches behind it, as
+// native code (the extension module memorax_amd._native).
+//
+// A call on a small rollout is bound by the host: checking the arguments, allocating the outputs, filling in a
+// C call and -- by far the most -- recording and running the autograd node.  As Python (ctypes calls inside
+// torch.autograd.Function) a forward and backward pair took 125-165 us whatever the arrays' size, most of it in
+// the backward, where the engine's thread had to fetch the interpreter's lock from the thread that waits for it.
+// Here the nodes are C++ (no interpreter in the backward at all) and one layer of functions does checks,
+// allocation and launch for them and for memorax_amd/kernels.py alike.
+//
+// The entry points of the C ABI are bound at run time (bind()) from whatever build of the library Python has
+// loaded; nothing here links against it.
+#include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <ATen/hip/HIPContextLight.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include <array>
+
+#include "memorax_amd.h"
+
+namespace py = pybind11;
+
+namespace {
+
+using at::Tensor;
+using c10::IntArrayRef;
+using c10::ScalarType;
+using OptTensor = std::optional<Tensor>;
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+
+// ------------------------------------------------------------------------------------------------ entry points
+#define MRX_BOUND(X)                                                                                                 \
+    X(mrx_status_string) X(mrx_chunk_size) X(mrx_delta_chunk_size) X(mrx_linear_scan_fwd) X(mrx_linear_scan_bwd)     \
+    X(mrx_linear_scan_last) X(mrx_mingru_scan_fwd) X(mrx_mingru_scan_bwd) X(mrx_mlstm_gates_fwd)                     \
+    X(mrx_mlstm_gates_bwd) X(mrx_rms_norm_fwd) X(mrx_rms_norm_bwd) X(mrx_layer_norm_fwd) X(mrx_layer_norm_bwd)       \
+    X(mrx_silu_gate_fwd) X(mrx_silu_gate_bwd) X(mrx_linear_attn_fwd) X(mrx_linear_attn_bwd)                          \
+    X(mrx_linear_attn_fwd_chunk_parallel) X(mrx_linear_attn_bwd_chunk_parallel)                                      \
+    X(mrx_linear_attn_chunk_parallel_pays) X(mrx_linear_attn_norm_fwd) X(mrx_linear_attn_norm_bwd)                   \
+    X(mrx_gated_linear_attn_fwd) X(mrx_gated_linear_attn_bwd) X(mrx_delta_rule_fwd) X(mrx_delta_rule_bwd)            \
+    X(mrx_delta_rule_fwd_noalloc) X(mrx_deltanet_fwd) X(mrx_deltanet_bwd) X(mrx_linear_attn_step)                    \
+    X(mrx_gated_linear_attn_step) X(mrx_delta_rule_step)
+struct {
+#define MRX_MEMBER(name) decltype(&::name) name = nullptr;
+    MRX_BOUND(MRX_MEMBER)
+#undef MRX_MEMBER
+} lib;
+
+void bind(const py::dict &addresses)
+{
+#define MRX_TAKE(name) lib.name = reinterpret_cast<decltype(&::name)>(addresses[#name].cast<uintptr_t>());
+    MRX_BOUND(MRX_TAKE)
+#undef MRX_TAKE
+}
+
+void check(int status, const char *what)
+{
+    TORCH_CHECK(status == MRX_OK, what, " failed: ", lib.mrx_status_string(status), " (status ", status, ")");
+}
+
+// --------------------------------------------------------------------------------------------------- arguments
+void *stream() { return c10::hip::getCurrentHIPStream().stream(); }
+
+template <typename P = void> P *ptr(const Tensor &t) { return t.defined() ? static_cast<P *>(t.data_ptr()) : nullptr; }
+template <typename P = void> P *ptr(const OptTensor &t) { return t.has_value() ? ptr<P>(*t) : nullptr; }
+float *fptr(const Tensor &t) { return ptr<float>(t); }
+float *fptr(const OptTensor &t) { return ptr<float>(t); }
+
+int code(ScalarType dt)
+{
+    switch (dt) {
+    case at::kFloat: return MRX_F32;
+    case at::kBFloat16: return MRX_BF16;
+    case at::kComplexFloat: return MRX_C64;
+    default: return -1;
+    }
+}
+
+void chk(const Tensor &t, const char *name)
+{
+    TORCH_CHECK_VALUE(t.is_cuda(), name, " must live on the GPU (memorax_amd has no CPU path)");
+    TORCH_CHECK_VALUE(t.is_contiguous(), name, " must be contiguous");
+}
+void chk(const Tensor &t, const char *name, ScalarType dt)
+{
+    chk(t, name);
+    TORCH_CHECK_VALUE(t.scalar_type() == dt, name, " must be ", dt, ", got ", t.scalar_type());
+}
+void chk(const Tensor &t, const char *name, ScalarType dt, IntArrayRef shape)
+{
+    chk(t, name, dt);
+    TORCH_CHECK_VALUE(t.sizes() == shape, name, " must have shape ", shape, ", got ", t.sizes());
+}
+void chk(const OptTensor &t, const char *name, ScalarType dt, IntArrayRef shape)
+{
+    if (t.has_value() && t->defined()) chk(*t, name, dt, shape);
+}
+
+Tensor fresh(IntArrayRef shape, ScalarType dt, const Tensor &like)
+{
+    return at::detail::empty_cuda(shape, dt, like.device(), std::nullopt);
+}
+Tensor fresh_like(const Tensor &t) { return fresh(t.sizes(), t.scalar_type(), t); }
+
+// Reset flags (B,T): bool, uint8 and float32 go to the kernels as they are, anything else as flag != 0.
+struct Done {
+    Tensor t;
+    int dtype;
+    Done(const Tensor &done, int64_t B, int64_t T)
+    {
+        TORCH_CHECK_VALUE(done.dim() == 2 && done.size(0) == B && done.size(1) == T, "done must have shape [", B, ", ", T, "], got ",
+                          done.sizes());
+        const auto dt = done.scalar_type();
+        t = (dt == at::kBool || dt == at::kByte || dt == at::kFloat) ? done.contiguous() : done.ne(0).contiguous();
+        dtype = dt == at::kFloat ? MRX_DONE_F32 : MRX_DONE_U8;
+        TORCH_CHECK_VALUE(t.is_cuda(), "done must live on the GPU (memorax_amd has no CPU path)");
+    }
+    const void *p() const { return t.data_ptr(); }
+};
+
+int64_t chunk_size(ScalarType dt, bool delta) { return delta ? lib.mrx_delta_chunk_size(code(dt)) : lib.mrx_chunk_size(code(dt)); }
+
+int compute_units(const Tensor &t) { return at::cuda::getDeviceProperties(t.get_device())->multiProcessorCount; }
+
+// ----------------------------------------------------------------------------------- checks, allocation, launch
+// ---- diagonal scans
+struct ScanOut {
+    Tensor h, h_last, P_last;
+};
+
+void chk_scan_dtype(ScalarType dt, bool complex, const char *what)
+{
+    TORCH_CHECK_VALUE(dt == at::kFloat || dt == at::kBFloat16 || (complex && dt == at::kComplexFloat), what, " supports float32, ",
+                      complex ? "complex64 and bfloat16" : "bfloat16");
+}
+
+ScanOut scan_fwd(const Tensor &a, const Tensor &b, const Tensor &done_, const OptTensor &h0, const OptTensor &P0, bool want_P)
+{
+    TORCH_CHECK_VALUE(b.dim() == 3, "b must be (B,T,D)");
+    const int64_t B = b.size(0), T = b.size(1), D = b.size(2);
+    const auto dt = b.scalar_type();
+    chk_scan_dtype(dt, true, "linear_scan");
+    const auto ct = dt == at::kBFloat16 ? at::kFloat : dt;   // the carries' type
+    const bool ti = a.dim() == 1;
+    if (ti) chk(a, "a", dt, {D});
+    else chk(a, "a", dt, {B, T, D});
+    chk(b, "b");
+    chk(h0, "h0", ct, {B, D});
+    chk(P0, "P0", ct, {B, D});
+    const Done done(done_, B, T);
+    ScanOut r{fresh_like(b), fresh({B, D}, ct, b), want_P ? fresh({B, D}, ct, b) : Tensor()};
+    check(lib.mrx_linear_scan_fwd(stream(), ptr(a), ptr(b), done.p(), ptr(h0), ptr(P0), ptr(r.h), ptr(r.h_last), ptr(r.P_last), B, T, D,
+                                  code(dt), done.dtype, ti),
+          "mrx_linear_scan_fwd");
+    return r;
+}
+
+struct ScanGrads {
+    Tensor da, db, dh0;
+};
+
+ScanGrads scan_bwd(const Tensor &a, const Tensor &h, const Tensor &done_, const OptTensor &h0, const Tensor &g, const OptTensor &g_last,
+                   bool sum_da)
+{
+    TORCH_CHECK_VALUE(g.dim() == 3, "g must be (B,T,D)");
+    const int64_t B = g.size(0), T = g.size(1), D = g.size(2);
+    const auto dt = g.scalar_type();
+    chk_scan_dtype(dt, true, "linear_scan");
+    const auto ct = dt == at::kBFloat16 ? at::kFloat : dt;
+    const bool ti = a.dim() == 1;
+    if (ti) chk(a, "a", dt, {D});
+    else chk(a, "a", dt, {B, T, D});
+    chk(h, "h", dt, {B, T, D});
+    chk(g, "g", dt);
+    chk(h0, "h0", ct, {B, D});
+    chk(g_last, "g_last", ct, {B, D});
+    const Done done(done_, B, T);
+    TORCH_CHECK_VALUE(ti || !sum_da, "sum_da belongs to a time-invariant a");
+    ScanGrads r{sum_da ? fresh({B, D}, ct, g) : fresh_like(g), fresh_like(g), fresh({B, D}, ct, g)};
+    check(lib.mrx_linear_scan_bwd(stream(), ptr(a), ptr(h), done.p(), ptr(h0), ptr(g), ptr(g_last), ptr(r.da), ptr(r.db), ptr(r.dh0), B, T, D,
+                                  code(dt), done.dtype, sum_da ? MRX_A_TIME_INVARIANT_SUM_DA : int(ti)),
+          "mrx_linear_scan_bwd");
+    return r;
+}
+
+Tensor scan_last(const Tensor &a, const Tensor &b, const Tensor &done_, const OptTensor &h0)
+{
+    TORCH_CHECK_VALUE(b.dim() == 3, "b must be (B,T,D)");
+    const int64_t B = b.size(0), T = b.size(1), D = b.size(2);
+    const auto dt = b.scalar_type();
+    TORCH_CHECK_VALUE(dt == at::kFloat || dt == at::kComplexFloat, "linear_scan_last supports float32 and complex64");
+    TORCH_CHECK_VALUE(a.dim() == 3 && a.size(0) == B && a.size(1) == T && a.size(2) > 0 && D % a.size(2) == 0,
+                      "a must be (B,T,D/group), got ", a.sizes(), " for b ", b.sizes());
+    chk(a, "a", dt);
+    chk(b, "b", dt);
+    chk(h0, "h0", dt, {B, D});
+    const Done done(done_, B, T);
+    Tensor h_last = fresh({B, D}, dt, b);
+    check(lib.mrx_linear_scan_last(stream(), ptr(a), ptr(b), done.p(), ptr(h0), ptr(h_last), B, T, D, D / a.size(2), code(dt), done.dtype),
+          "mrx_linear_scan_last");
+    return h_last;
+}
+
+ScanOut mingru_fwd(const Tensor &z, const Tensor &x, const Tensor &done_, const OptTensor &h0, const OptTensor &P0, bool want_P)
+{
+    TORCH_CHECK_VALUE(z.dim() == 3, "z must be (B,T,D)");
+    const int64_t B = z.size(0), T = z.size(1), D = z.size(2);
+    const auto dt = z.scalar_type();
+    chk_scan_dtype(dt, false, "mingru_scan");
+    chk(z, "z");
+    chk(x, "h_tilde", dt, z.sizes());
+    chk(h0, "h0", at::kFloat, {B, D});
+    chk(P0, "P0", at::kFloat, {B, D});
+    const Done done(done_, B, T);
+    ScanOut r{fresh_like(z), fresh({B, D}, at::kFloat, z), want_P ? fresh({B, D}, at::kFloat, z) : Tensor()};
+    check(lib.mrx_mingru_scan_fwd(stream(), ptr(z), ptr(x), done.p(), fptr(h0), fptr(P0), ptr(r.h), fptr(r.h_last), fptr(r.P_last), B, T, D,
+                                  code(dt), done.dtype),
+          "mrx_mingru_scan_fwd");
+    return r;
+}
+
+ScanGrads mingru_bwd(const Tensor &z, const Tensor &x, const Tensor &h, const Tensor &done_, const OptTensor &h0, const Tensor &g,
+                     const OptTensor &g_last)
+{
+    TORCH_CHECK_VALUE(g.dim() == 3, "g must be (B,T,D)");
+    const int64_t B = g.size(0), T = g.size(1), D = g.size(2);
+    const auto dt = g.scalar_type();
+    chk_scan_dtype(dt, false, "mingru_scan");
+    chk(z, "z", dt, g.sizes());
+    chk(x, "h_tilde", dt, g.sizes());
+    chk(h, "h", dt, g.sizes());
+    chk(g, "g");
+    chk(h0, "h0", at::kFloat, {B, D});
+    chk(g_last, "g_last", at::kFloat, {B, D});
+    const Done done(done_, B, T);
+    ScanGrads r{fresh_like(g), fresh_like(g), fresh({B, D}, at::kFloat, g)};
+    check(lib.mrx_mingru_scan_bwd(stream(), ptr(z), ptr(x), ptr(h), done.p(), fptr(h0), ptr(g), fptr(g_last), ptr(r.da), ptr(r.db),
+                                  fptr(r.dh0), B, T, D, code(dt), done.dtype),
+          "mrx_mingru_scan_bwd");
+    return r;
+}
+
+// ---- the mLSTM stabiliser
+std::array<Tensor, 3> mlstm_gates_fwd(const Tensor &li, const Tensor &lf, const Tensor &done_, const OptTensor &m0, double g_floor)
+{
+    TORCH_CHECK_VALUE(li.dim() == 3, "log_i must be (B,T,H)");
+    const int64_t B = li.size(0), T = li.size(1), H = li.size(2);
+    chk(li, "log_i", at::kFloat);
+    chk(lf, "log_f", at::kFloat, {B, T, H});
+    chk(m0, "m0", at::kFloat, {B, H});
+    const Done done(done_, B, T);
+    std::array<Tensor, 3> r{fresh_like(li), fresh_like(li), fresh_like(li)};
+    check(lib.mrx_mlstm_gates_fwd(stream(), fptr(li), fptr(lf), done.p(), fptr(m0), fptr(r[0]), fptr(r[1]), fptr(r[2]), B, T, H, done.dtype,
+                                  (float)g_floor),
+          "mrx_mlstm_gates_fwd");
+    return r;
+}
+
+std::array<Tensor, 3> mlstm_gates_bwd(const Tensor &li, const Tensor &lf, const Tensor &done_, const OptTensor &m0, const Tensor &m,
+                                      const OptTensor &dm, const OptTensor &dg, const OptTensor &dw, double g_floor, bool want_dm0)
+{
+    TORCH_CHECK_VALUE(li.dim() == 3, "log_i must be (B,T,H)");
+    const int64_t B = li.size(0), T = li.size(1), H = li.size(2);
+    chk(li, "log_i", at::kFloat);
+    chk(lf, "log_f", at::kFloat, {B, T, H});
+    chk(m, "m", at::kFloat, {B, T, H});
+    chk(dm, "dm", at::kFloat, {B, T, H});
+    chk(dg, "dg", at::kFloat, {B, T, H});
+    chk(dw, "dw", at::kFloat, {B, T, H});
+    chk(m0, "m0", at::kFloat, {B, H});
+    const Done done(done_, B, T);
+    std::array<Tensor, 3> r{fresh_like(li), fresh_like(li), want_dm0 ? fresh({B, H}, at::kFloat, li) : Tensor()};
+    check(lib.mrx_mlstm_gates_bwd(stream(), fptr(li), fptr(lf), done.p(), fptr(m0), fptr(m), fptr(dm), fptr(dg), fptr(dw), fptr(r[0]),
+                                  fptr(r[1]), fptr(r[2]), B, T, H, done.dtype, (float)g_floor),
+          "mrx_mlstm_gates_bwd");
+    return r;
+}
+
+// ---- norms and the gate
+void chk_norm_dtype(ScalarType dt)
+{
+    TORCH_CHECK_VALUE(dt == at::kFloat || dt == at::kBFloat16, "the norm kernels take float32 or bfloat16 arrays");
+}
+
+Tensor norm_fwd(const Tensor &x, const OptTensor &scale, const OptTensor &bias, double eps, std::optional<ScalarType> out_dtype, bool center)
+{
+    TORCH_CHECK_VALUE(x.dim() >= 1, "x must have a feature axis");
+    const int64_t D = x.size(-1);
+    const auto dt = x.scalar_type(), od = out_dtype.value_or(dt);
+    chk_norm_dtype(dt);
+    chk_norm_dtype(od);
+    chk(x, "x");
+    chk(scale, "scale", at::kFloat, {D});
+    chk(bias, "bias", at::kFloat, {D});
+    Tensor y = fresh(x.sizes(), od, x);
+    if (x.numel() == 0) return y;
+    const int64_t rows = x.numel() / D;
+    if (center)
+        check(lib.mrx_layer_norm_fwd(stream(), ptr(x), fptr(scale), fptr(bias), ptr(y), rows, D, code(dt), code(od), (float)eps),
+              "mrx_layer_norm_fwd");
+    else
+        check(lib.mrx_rms_norm_fwd(stream(), ptr(x), fptr(scale), ptr(y), rows, D, code(dt), code(od), (float)eps), "mrx_rms_norm_fwd");
+    return y;
+}
+
+struct NormGrads {
+    Tensor dx, dscale, dbias;
+};
+
+NormGrads norm_bwd(const Tensor &x, const OptTensor &scale, const Tensor &dy, double eps, bool want_dparams, const OptTensor &dx_add,
+                   bool center)
+{
+    TORCH_CHECK_VALUE(x.dim() >= 1, "x must have a feature axis");
+    const int64_t D = x.size(-1);
+    const auto dt = x.scalar_type(), yd = dy.scalar_type();
+    chk_norm_dtype(dt);
+    chk_norm_dtype(yd);
+    chk(x, "x");
+    chk(dy, "dy", yd, x.sizes());
+    chk(dx_add, "dx_add", dt, x.sizes());
+    chk(scale, "scale", at::kFloat, {D});
+    NormGrads r{fresh_like(x), {}, {}};
+    Tensor work;
+    if (want_dparams) {
+        r.dscale = fresh({D}, at::kFloat, x);
+        if (center) r.dbias = fresh({D}, at::kFloat, x);
+        work = fresh({(center ? 2 : 1) * MRX_RMS_NORM_PARTS, D}, at::kFloat, x);
+    }
+    if (x.numel() == 0) {   // dx (and dx_add) are empty
+        if (r.dscale.defined()) r.dscale.zero_();
+        if (r.dbias.defined()) r.dbias.zero_();
+        return r;
+    }
+    const int64_t rows = x.numel() / D;
+    if (center)
+        check(lib.mrx_layer_norm_bwd(stream(), ptr(x), fptr(scale), ptr(dy), ptr(dx_add), ptr(r.dx), fptr(r.dscale), fptr(r.dbias), fptr(work),
+                                     rows, D, code(dt), code(yd), (float)eps),
+              "mrx_layer_norm_bwd");
+    else
+        check(lib.mrx_rms_norm_bwd(stream(), ptr(x), fptr(scale), ptr(dy), ptr(dx_add), ptr(r.dx), fptr(r.dscale), fptr(work), rows, D,
+                                   code(dt), code(yd), (float)eps),
+              "mrx_rms_norm_bwd");
+    return r;
+}
+
+Tensor silu_gate_fwd(const Tensor &h, const Tensor &g)
+{
+    const auto dt = h.scalar_type();
+    TORCH_CHECK_VALUE(dt == at::kFloat || dt == at::kBFloat16, "silu_gate takes float32 or bfloat16 arrays");
+    chk(h, "h");
+    chk(g, "g", dt, h.sizes());
+    Tensor y = fresh_like(h);
+    if (h.numel()) check(lib.mrx_silu_gate_fwd(stream(), ptr(h), ptr(g), ptr(y), h.numel(), code(dt)), "mrx_silu_gate_fwd");
+    return y;
+}
+
+std::array<Tensor, 2> silu_gate_bwd(const Tensor &h, const Tensor &g, const Tensor &dy)
+{
+    const auto dt = h.scalar_type();
+    TORCH_CHECK_VALUE(dt == at::kFloat || dt == at::kBFloat16, "silu_gate takes float32 or bfloat16 arrays");
+    chk(h, "h");
+    chk(g, "g", dt, h.sizes());
+    chk(dy, "dy", dt, h.sizes());
+    std::array<Tensor, 2> r{fresh_like(h), fresh_like(h)};
+    if (h.numel())
+        check(lib.mrx_silu_gate_bwd(stream(), ptr(h), ptr(g), ptr(dy), ptr(r[0]), ptr(r[1]), h.numel(), code(dt)), "mrx_silu_gate_bwd");
+    return r;
+}
+
+// ---- chunked attention
+struct Shape {
+    int64_t B, T, H, dk, dv;
+    ScalarType dt;
+    Shape(const Tensor &q, const Tensor &k, const Tensor &v)
+    {
+        TORCH_CHECK_VALUE(q.dim() == 4 && v.dim() == 4, "q, k, v must be (B,T,H,d)");
+        B = q.size(0), T = q.size(1), H = q.size(2), dk = q.size(3), dv = v.size(3);
+        dt = q.scalar_type();
+        TORCH_CHECK_VALUE(dt == at::kFloat || dt == at::kBFloat16, "chunked kernels support float32 and bfloat16");
+        chk(q, "q");
+        chk(k, "k", dt, {B, T, H, dk});
+        chk(v, "v", dt, {B, T, H, dv});
+    }
+    int64_t chunks(bool delta = false) const { return (T + chunk_size(dt, delta) - 1) / chunk_size(dt, delta); }
+    std::array<int64_t, 4> state() const { return {B, H, dv, dk}; }
+};
+
+struct AttnOut {
+    Tensor o, S_last, S_chk;
+    bool parallel;   // S_chk is dense, from the pair of kernels that cuts the work along time
+};
+
+AttnOut linear_attn_fwd(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &done_, const OptTensor &S0, int fmap, bool save_chk,
+                        std::optional<bool> chunk_parallel)
+{
+    const Shape s(q, k, v);
+    chk(S0, "S0", at::kFloat, s.state());
+    const Done done(done_, s.B, s.T);
+    const bool par = chunk_parallel.has_value() ? *chunk_parallel : lib.mrx_linear_attn_chunk_parallel_pays(s.B, s.T, s.H, code(s.dt)) != 0;
+    AttnOut r{fresh_like(v), fresh(s.state(), at::kFloat, q), {}, par};
+    if (save_chk || par) r.S_chk = fresh({s.B, s.H, s.chunks(), s.dv, s.dk}, at::kFloat, q);
+    if (par)
+        check(lib.mrx_linear_attn_fwd_chunk_parallel(stream(), ptr(q), ptr(k), ptr(v), done.p(), fptr(S0), ptr(r.o), fptr(r.S_last),
+                                                     fptr(r.S_chk), s.B, s.T, s.H, s.dk, s.dv, code(s.dt), done.dtype, fmap),
+              "mrx_linear_attn_fwd_chunk_parallel");
+    else
+        check(lib.mrx_linear_attn_fwd(stream(), ptr(q), ptr(k), ptr(v), done.p(), fptr(S0), ptr(r.o), fptr(r.S_last), fptr(r.S_chk), s.B, s.T,
+                                      s.H, s.dk, s.dv, code(s.dt), done.dtype, fmap),
+              "mrx_linear_attn_fwd");
+    if (!save_chk) r.S_chk = Tensor();
+    return r;
+}
+
+struct AttnGrads {
+    Tensor dq, dk, dv, extra, dS0, dz0;   // extra: the gradient of the gate (gated: dg, delta rule: dbeta)
+};
+
+AttnGrads linear_attn_bwd(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &done_, const Tensor &S_chk, const OptTensor &S_last,
+                          const Tensor &dout, const OptTensor &dS_last, int fmap, bool want_dS0)
+{
+    const Shape s(q, k, v);
+    chk(dout, "do", s.dt, v.sizes());
+    chk(S_chk, "S_chk", at::kFloat, {s.B, s.H, s.chunks(), s.dv, s.dk});
+    chk(S_last, "S_last", at::kFloat, s.state());
+    chk(dS_last, "dS_last", at::kFloat, s.state());
+    const Done done(done_, s.B, s.T);
+    AttnGrads r{fresh_like(q), fresh_like(k), fresh_like(v), {}, want_dS0 ? fresh(s.state(), at::kFloat, q) : Tensor(), {}};
+    if (!(S_last.has_value() && S_last->defined())) {   // residuals of the chunk-parallel pair
+        const Tensor ws = fresh_like(S_chk);
+        check(lib.mrx_linear_attn_bwd_chunk_parallel(stream(), ptr(q), ptr(k), ptr(v), done.p(), fptr(S_chk), ptr(dout), fptr(dS_last),
+                                                     ptr(r.dq), ptr(r.dk), ptr(r.dv), fptr(r.dS0), fptr(ws), s.B, s.T, s.H, s.dk, s.dv,
+                                                     code(s.dt), done.dtype, fmap),
+              "mrx_linear_attn_bwd_chunk_parallel");
+        return r;
+    }
+    check(lib.mrx_linear_attn_bwd(stream(), ptr(q), ptr(k), ptr(v), done.p(), fptr(S_chk), fptr(S_last), ptr(dout), fptr(dS_last), ptr(r.dq),
+                                  ptr(r.dk), ptr(r.dv), fptr(r.dS0), s.B, s.T, s.H, s.dk, s.dv, code(s.dt), done.dtype, fmap),
+          "mrx_linear_attn_bwd");
+    return r;
+}
+
+struct NormAttnOut {
+    Tensor o, den, S_last, z_last, S_chk, z_chk, ss;
+};
+
+NormAttnOut linear_attn_norm_fwd(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &done_, const OptTensor &S0,
+                                 const OptTensor &z0, int fmap, double eps, bool save_chk, bool want_ss)
+{
+    const Shape s(q, k, v);
+    chk(S0, "S0", at::kFloat, s.state());
+    chk(z0, "z0", at::kFloat, {s.B, s.H, s.dk});
+    const Done done(done_, s.B, s.T);
+    NormAttnOut r;
+    r.o = fresh_like(v);
+    r.den = fresh({s.B, s.H, s.T}, at::kFloat, q);
+    r.S_last = fresh(s.state(), at::kFloat, q);
+    r.z_last = fresh({s.B, s.H, s.dk}, at::kFloat, q);
+    if (save_chk) {
+        r.S_chk = fresh({s.B, s.H, s.chunks(), s.dv, s.dk}, at::kFloat, q);
+        r.z_chk = fresh({s.B, s.H, s.chunks(), s.dk}, at::kFloat, q);
+    }
+    if (want_ss) r.ss = fresh({s.B, s.H, s.T}, at::kFloat, q);
+    check(lib.mrx_linear_attn_norm_fwd(stream(), ptr(q), ptr(k), ptr(v), done.p(), fptr(S0), fptr(z0), ptr(r.o), fptr(r.den), fptr(r.ss),
+                                       fptr(r.S_last), fptr(r.z_last), fptr(r.S_chk), fptr(r.z_chk), s.B, s.T, s.H, s.dk, s.dv, code(s.dt),
+                                       done.dtype, fmap, (float)eps),
+          "mrx_linear_attn_norm_fwd");
+    return r;
+}
+
+AttnGrads linear_attn_norm_bwd(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &done_, const Tensor &S_chk,
+                               const Tensor &z_chk, const Tensor &S_last, const Tensor &o, const Tensor &den, const Tensor &dout,
+                               const OptTensor &dS_last, const OptTensor &dz_last, int fmap, double eps, bool want_d0, const OptTensor &d_ss)
+{
+    const Shape s(q, k, v);
+    chk(S_last, "S_last", at::kFloat, s.state());
+    chk(dout, "do", s.dt, v.sizes());
+    chk(o, "o", s.dt, v.sizes());
+    chk(den, "den", at::kFloat, {s.B, s.H, s.T});
+    chk(S_chk, "S_chk", at::kFloat, {s.B, s.H, s.chunks(), s.dv, s.dk});
+    chk(z_chk, "z_chk", at::kFloat, {s.B, s.H, s.chunks(), s.dk});
+    chk(dS_last, "dS_last", at::kFloat, s.state());
+    chk(dz_last, "dz_last", at::kFloat, {s.B, s.H, s.dk});
+    chk(d_ss, "d_ss", at::kFloat, {s.B, s.H, s.T});
+    const Done done(done_, s.B, s.T);
+    AttnGrads r{fresh_like(q), fresh_like(k), fresh_like(v), {}, want_d0 ? fresh(s.state(), at::kFloat, q) : Tensor(),
+                want_d0 ? fresh({s.B, s.H, s.dk}, at::kFloat, q) : Tensor()};
+    check(lib.mrx_linear_attn_norm_bwd(stream(), ptr(q), ptr(k), ptr(v), done.p(), fptr(S_chk), fptr(S_last), fptr(z_chk), ptr(o), fptr(den),
+                                       ptr(dout), fptr(d_ss), fptr(dS_last), fptr(dz_last), ptr(r.dq), ptr(r.dk), ptr(r.dv), fptr(r.dS0),
+                                       fptr(r.dz0), s.B, s.T, s.H, s.dk, s.dv, code(s.dt), done.dtype, fmap, (float)eps),
+          "mrx_linear_attn_norm_bwd");
+    return r;
+}
+
+AttnOut gated_linear_attn_fwd(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &g, const Tensor &done_, const OptTensor &S0,
+                              int fmap, bool save_chk)
+{
+    const Shape s(q, k, v);
+    chk(g, "g", at::kFloat, {s.B, s.T, s.H});
+    chk(S0, "S0", at::kFloat, s.state());
+    const Done done(done_, s.B, s.T);
+    AttnOut r{fresh_like(v), fresh(s.state(), at::kFloat, q), {}, false};
+    if (save_chk) r.S_chk = fresh({s.B, s.H, s.chunks(), s.dv, s.dk}, s.dt, q);
+    check(lib.mrx_gated_linear_attn_fwd(stream(), ptr(q), ptr(k), ptr(v), fptr(g), done.p(), fptr(S0), ptr(r.o), fptr(r.S_last), ptr(r.S_chk),
+                                        s.B, s.T, s.H, s.dk, s.dv, code(s.dt), done.dtype, fmap),
+          "mrx_gated_linear_attn_fwd");
+    return r;
+}
+
+AttnGrads gated_linear_attn_bwd(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &g, const Tensor &done_, const Tensor &S_chk,
+                                const Tensor &dout, const OptTensor &dS_last, int fmap, bool want_dS0, const OptTensor &S_last)
+{
+    const Shape s(q, k, v);
+    chk(g, "g", at::kFloat, {s.B, s.T, s.H});
+    chk(dout, "do", s.dt, v.sizes());
+    chk(S_chk, "S_chk", s.dt, {s.B, s.H, s.chunks(), s.dv, s.dk});
+    chk(dS_last, "dS_last", at::kFloat, s.state());
+    chk(S_last, "S_last", at::kFloat, s.state());
+    TORCH_CHECK_VALUE(!ptr(dS_last) || ptr(S_last), "S_last is required with dS_last");
+    const Done done(done_, s.B, s.T);
+    AttnGrads r{fresh_like(q), fresh_like(k), fresh_like(v), fresh_like(g), want_dS0 ? fresh(s.state(), at::kFloat, q) : Tensor(), {}};
+    check(lib.mrx_gated_linear_attn_bwd(stream(), ptr(q), ptr(k), ptr(v), fptr(g), done.p(), ptr(S_chk), fptr(S_last), ptr(dout),
+                                        fptr(dS_last), ptr(r.dq), ptr(r.dk), ptr(r.dv), fptr(r.extra), fptr(r.dS0), s.B, s.T, s.H, s.dk, s.dv,
+                                        code(s.dt), done.dtype, fmap),
+          "mrx_gated_linear_attn_bwd");
+    return r;
+}
+
+// ---- delta rule
+struct DeltaOut {
+    Tensor o, S_last, S_chk, Tm_chk;
+};
+
+// out: an earlier call's results to write into instead of allocating (S_chk undefined there: no residuals).
+// tm_scratch (only without residuals): whether the library is given a buffer for the triangular factors anyway, which lets it
+// compute them chunk-parallel; unset: when it would use one (float32; bfloat16 with at most two sequences per compute unit).
+DeltaOut delta_rule_fwd(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &beta, const Tensor &done_, const OptTensor &S0,
+                        bool save_chk, const std::optional<std::array<OptTensor, 4>> &out, bool prologue, std::optional<bool> tm_scratch,
+                        int factors, int resets)
+{
+    const Shape s(q, k, v);
+    chk(beta, "beta", s.dt, {s.B, s.T, s.H});
+    chk(S0, "S0", at::kFloat, s.state());
+    const Done done(done_, s.B, s.T);
+    const int64_t C = chunk_size(s.dt, true), NC = s.chunks(true);
+    DeltaOut r;
+    if (out.has_value()) {
+        auto take = [](const OptTensor &t) { return t.has_value() ? *t : Tensor(); };
+        r = {take((*out)[0]), take((*out)[1]), take((*out)[2]), take((*out)[3])};
+        chk((*out)[0], "out o", s.dt, v.sizes());
+        chk((*out)[1], "out S_last", at::kFloat, s.state());
+        chk((*out)[2], "out S_chk", s.dt, {s.B, s.H, NC, s.dv, s.dk});
+        chk((*out)[3], "out Tm_chk", s.dt, {s.B, s.H, NC, C, C});
+        TORCH_CHECK_VALUE(r.o.defined() && r.S_last.defined(), "out needs o and S_last");
+    } else {
+        r.o = fresh_like(v);
+        r.S_last = fresh(s.state(), at::kFloat, q);
+        if (save_chk) r.S_chk = fresh({s.B, s.H, NC, s.dv, s.dk}, s.dt, q);
+        const bool factor_buffer =
+            save_chk || (tm_scratch.has_value() ? *tm_scratch : s.dt == at::kFloat || s.B * s.H <= 2 * compute_units(q));
+        if (factor_buffer) r.Tm_chk = fresh({s.B, s.H, NC, C, C}, s.dt, q);
+    }
+    check((prologue ? lib.mrx_deltanet_fwd : lib.mrx_delta_rule_fwd)(stream(), ptr(q), ptr(k), ptr(v), ptr(beta), done.p(), fptr(S0), ptr(r.o),
+                                                                     fptr(r.S_last), ptr(r.S_chk), ptr(r.Tm_chk), s.B, s.T, s.H, s.dk, s.dv,
+                                                                     code(s.dt), done.dtype, factors, resets),
+          prologue ? "mrx_deltanet_fwd" : "mrx_delta_rule_fwd");
+    return r;
+}
+
+AttnGrads delta_rule_bwd(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &beta, const Tensor &done_, const Tensor &S_chk,
+                         const Tensor &Tm_chk, const Tensor &dout, const OptTensor &dS_last, bool want_dS0,
+                         const std::optional<std::array<OptTensor, 5>> &out, bool prologue, int resets)
+{
+    const Shape s(q, k, v);
+    const int64_t C = chunk_size(s.dt, true), NC = s.chunks(true);
+    chk(Tm_chk, "Tm_chk", s.dt, {s.B, s.H, NC, C, C});
+    chk(beta, "beta", s.dt, {s.B, s.T, s.H});
+    chk(dout, "do", s.dt, v.sizes());
+    chk(S_chk, "S_chk", s.dt, {s.B, s.H, NC, s.dv, s.dk});
+    chk(dS_last, "dS_last", at::kFloat, s.state());
+    const Done done(done_, s.B, s.T);
+    AttnGrads r;
+    if (out.has_value()) {
+        const auto &o = *out;
+        for (int i = 0; i < 4; ++i) TORCH_CHECK_VALUE(ptr(o[i]), "out needs dq, dk, dv and dbeta");
+        chk(o[0], "out dq", s.dt, q.sizes());
+        chk(o[1], "out dk", s.dt, k.sizes());
+        chk(o[2], "out dv", s.dt, v.sizes());
+        chk(o[3], "out dbeta", s.dt, beta.sizes());
+        chk(o[4], "out dS0", at::kFloat, s.state());
+        r = {*o[0], *o[1], *o[2], *o[3], o[4].has_value() ? *o[4] : Tensor(), {}};
+    } else {
+        r = {fresh_like(q), fresh_like(k), fresh_like(v), fresh_like(beta), want_dS0 ? fresh(s.state(), at::kFloat, q) : Tensor(), {}};
+    }
+    check((prologue ? lib.mrx_deltanet_bwd : lib.mrx_delta_rule_bwd)(stream(), ptr(q), ptr(k), ptr(v), ptr(beta), done.p(), ptr(S_chk),
+                                                                     ptr(Tm_chk), ptr(dout), fptr(dS_last), ptr(r.dq), ptr(r.dk), ptr(r.dv),
+                                                                     ptr(r.extra), fptr(r.dS0), s.B, s.T, s.H, s.dk, s.dv, code(s.dt),
+                                                                     done.dtype, resets),
+          prologue ? "mrx_deltanet_bwd" : "mrx_delta_rule_bwd");
+    return r;
+}
+
+std::array<Tensor, 2> delta_rule_fwd_noalloc(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &beta, const Tensor &done_,
+                                             const OptTensor &S0, const OptTensor &o, const OptTensor &S_last)
+{
+    const Shape s(q, k, v);
+    chk(beta, "beta", s.dt, {s.B, s.T, s.H});
+    chk(S0, "S0", at::kFloat, s.state());
+    const Done done(done_, s.B, s.T);
+    chk(o, "out o", s.dt, v.sizes());
+    chk(S_last, "out S_last", at::kFloat, s.state());
+    std::array<Tensor, 2> r{o.has_value() ? *o : fresh_like(v), S_last.has_value() ? *S_last : fresh(s.state(), at::kFloat, q)};
+    check(lib.mrx_delta_rule_fwd_noalloc(stream(), ptr(q), ptr(k), ptr(v), ptr(beta), done.p(), fptr(S0), ptr(r[0]), fptr(r[1]), s.B, s.T, s.H,
+                                         s.dk, s.dv, code(s.dt), done.dtype),
+          "mrx_delta_rule_fwd_noalloc");
+    return r;
+}
+
+// ---- single time steps: q, k, v (B,H,d), done (B)
+struct StepShape {
+    int64_t B, H, dk, dv;
+    ScalarType dt;
+    StepShape(const Tensor &q, const Tensor &k, const Tensor &v)
+    {
+        TORCH_CHECK_VALUE(q.dim() == 3 && v.dim() == 3, "q must be (B,H,d), got ", q.sizes());
+        B = q.size(0), H = q.size(1), dk = q.size(2), dv = v.size(2);
+        dt = q.scalar_type();
+        TORCH_CHECK_VALUE(dt == at::kFloat || dt == at::kBFloat16, "unsupported dtype ", dt);
+        chk(q, "q");
+        chk(k, "k", dt, {B, H, dk});
+        chk(v, "v", dt, {B, H, dv});
+    }
+    std::array<int64_t, 4> state() const { return {B, H, dv, dk}; }
+    Tensor next(const OptTensor &S, bool inplace, const Tensor &like) const
+    {
+        return inplace && S.has_value() ? *S : fresh(state(), at::kFloat, like);
+    }
+};
+
+struct StepOut {
+    Tensor o, S, z;
+};
+
+StepOut linear_attn_step(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &done_, const OptTensor &S, const OptTensor &z,
+                         int fmap, bool normalise, double eps, bool inplace)
+{
+    const StepShape s(q, k, v);
+    chk(S, "S", at::kFloat, s.state());
+    chk(z, "z", at::kFloat, {s.B, s.H, s.dk});
+    const Done done(done_.reshape({s.B, 1}), s.B, 1);
+    StepOut r{fresh_like(v), s.next(S, inplace, q), {}};
+    if (normalise) r.z = inplace && z.has_value() ? *z : fresh({s.B, s.H, s.dk}, at::kFloat, q);
+    check(lib.mrx_linear_attn_step(stream(), ptr(q), ptr(k), ptr(v), done.p(), fptr(S), normalise ? fptr(z) : nullptr, ptr(r.o), fptr(r.S),
+                                   fptr(r.z), s.B, s.H, s.dk, s.dv, code(s.dt), done.dtype, fmap, (float)eps),
+          "mrx_linear_attn_step");
+    return r;
+}
+
+StepOut gated_linear_attn_step(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &g, const Tensor &done_, const OptTensor &S,
+                               int fmap, bool inplace)
+{
+    const StepShape s(q, k, v);
+    chk(g, "g", at::kFloat, {s.B, s.H});
+    chk(S, "S", at::kFloat, s.state());
+    const Done done(done_.reshape({s.B, 1}), s.B, 1);
+    StepOut r{fresh_like(v), s.next(S, inplace, q), {}};
+    check(lib.mrx_gated_linear_attn_step(stream(), ptr(q), ptr(k), ptr(v), fptr(g), done.p(), fptr(S), ptr(r.o), fptr(r.S), s.B, s.H, s.dk,
+                                         s.dv, code(s.dt), done.dtype, fmap),
+          "mrx_gated_linear_attn_step");
+    return r;
+}
+
+StepOut delta_rule_step(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &beta, const Tensor &done_, const OptTensor &S,
+                        bool inplace)
+{
+    const StepShape s(q, k, v);
+    chk(beta, "beta", s.dt, {s.B, s.H});
+    chk(S, "S", at::kFloat, s.state());
+    const Done done(done_.reshape({s.B, 1}), s.B, 1);
+    StepOut r{fresh_like(v), s.next(S, inplace, q), {}};
+    check(lib.mrx_delta_rule_step(stream(), ptr(q), ptr(k), ptr(v), ptr(beta), done.p(), fptr(S), ptr(r.o), fptr(r.S), s.B, s.H, s.dk, s.dv,
+                                  code(s.dt), done.dtype),
+          "mrx_delta_rule_step");
+    return r;
+}
+
+// ------------------------------------------------------------------------------------------------ autograd nodes
+// One node type for every operator: Op holds what is no tensor of the graph (flags, scalars, the reset flags) and
+//     static constexpr int SAVED          how many tensors the backward reads
+//     static const char *name()
+//     variable_list backward(node, saved, grads)
+template <class Op> struct OpNode final : torch::autograd::Node {
+    Op op;
+    std::array<SavedVariable, Op::SAVED> saved;
+    std::array<bool, Op::SAVED> output{};
+
+    void keep(int i, const Tensor &t, bool is_output = false)
+    {
+        saved[i] = SavedVariable(t, is_output);
+        output[i] = is_output;
+    }
+    variable_list apply(variable_list &&grads) override
+    {
+        std::lock_guard<std::mutex> lock(mutex_);
+        std::array<Tensor, Op::SAVED> s;
+        for (int i = 0; i < Op::SAVED; ++i) s[i] = saved[i].unpack(output[i] ? shared_from_this() : nullptr);
+        at::AutoDispatchBelowADInplaceOrView below;
+        return op.backward(*this, s, grads);
+    }
+    void release_variables() override
+    {
+        std::lock_guard<std::mutex> lock(mutex_);
+        for (auto &s : saved) s.reset_data();
+    }
+    std::string name() const override { return Op::name(); }
+    bool wants(size_t i) const { return task_should_compute_output(i); }
+};
+
+template <class Op, typename... Ts> std::shared_ptr<OpNode<Op>> record(Op &&op, const Ts &...inputs)
+{
+    auto node = std::shared_ptr<OpNode<Op>>(new OpNode<Op>(), torch::autograd::deleteNode);
+    node->op = std::move(op);
+    node->set_next_edges(torch::autograd::collect_next_edges(inputs...));
+    return node;
+}
+
+bool differentiable(const Tensor &t) { return t.defined() && t.requires_grad(); }
+bool differentiable(const OptTensor &t) { return t.has_value() && differentiable(*t); }
+template <typename... Ts> bool need_grad(const Ts &...ts) { return at::GradMode::is_enabled() && (differentiable(ts) || ...); }
+
+Tensor unwrap(const OptTensor &t) { return t.has_value() ? *t : Tensor(); }
+OptTensor some(const Tensor &t) { return t.defined() ? OptTensor(t) : std::nullopt; }
+// contiguous and in the given type; the tensor itself where it is that already
+Tensor as(const Tensor &t, ScalarType dt) { return t.defined() ? t.to(dt).contiguous() : t; }
+Tensor grad_or_zeros(const Tensor &g, const Tensor &like) { return g.defined() ? g.contiguous() : at::zeros_like(like); }
+Tensor unless(bool skip, const Tensor &t) { return skip ? Tensor() : t; }
+
+struct LinearScanOp {
+    static constexpr int SAVED = 3;   // a, h, h0
+    static const char *name() { return "MemoraxLinearScanBackward"; }
+    Tensor done;
+    variable_list backward(OpNode<LinearScanOp> &node, std::array<Tensor, 3> &s, variable_list &grads)
+    {
+        const Tensor &a = s[0], &h = s[1];
+        const bool ti = a.dim() == 1;   // a broadcast coefficient: the kernel sums its gradient over time, the rest is (B,D)
+        auto r = scan_bwd(a, h, done, some(s[2]), grad_or_zeros(grads[0], h), some(as(grads[1], s[2].defined() ? s[2].scalar_type() : carry(h))),
+                          ti);
+        if (ti && node.wants(0)) r.da = r.da.sum(0).to(a.scalar_type());
+        return {unless(!node.wants(0), r.da), unless(!node.wants(1), r.db), unless(!node.wants(2), r.dh0)};
+    }
+    static ScalarType carry(const Tensor &h) { return h.scalar_type() == at::kBFloat16 ? at::kFloat : h.scalar_type(); }
+};
+
+std::tuple<Tensor, Tensor, Tensor> linear_scan(const Tensor &a, const Tensor &b, const Tensor &done, const OptTensor &h0, const OptTensor &P0)
+{
+    const bool need = need_grad(a, b, h0);
+    Tensor a_, h0_;
+    ScanOut r;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        auto carried = [&](const OptTensor &t) {   // bfloat16 arrays: float32 carries
+            return !t.has_value() ? Tensor() : b.scalar_type() == at::kBFloat16 ? as(*t, at::kFloat) : t->contiguous();
+        };
+        a_ = a.contiguous();
+        h0_ = carried(h0);
+        r = scan_fwd(a_, b.contiguous(), done, some(h0_), some(carried(P0)), true);
+    }
+    if (need) {
+        auto node = record(LinearScanOp{done}, a, b, unwrap(h0));
+        torch::autograd::set_history(r.h, node);
+        torch::autograd::set_history(r.h_last, node);
+        node->keep(0, a_);
+        node->keep(1, r.h, true);
+        node->keep(2, h0_);
+    }
+    return {r.h, r.h_last, r.P_last};
+}
+
+struct MinGruOp {
+    static constexpr int SAVED = 4;   // z, h~, h, h0
+    static const char *name() { return "MemoraxMinGruScanBackward"; }
+    Tensor done;
+    variable_list backward(OpNode<MinGruOp> &node, std::array<Tensor, 4> &s, variable_list &grads)
+    {
+        auto r = mingru_bwd(s[0], s[1], s[2], done, some(s[3]), grad_or_zeros(grads[0], s[2]), some(as(grads[1], at::kFloat)));
+        return {unless(!node.wants(0), r.da), unless(!node.wants(1), r.db), unless(!node.wants(2), r.dh0)};
+    }
+};
+
+std::tuple<Tensor, Tensor, Tensor> mingru_scan(const Tensor &z, const Tensor &x, const Tensor &done, const OptTensor &h0, const OptTensor &P0)
+{
+    const bool need = need_grad(z, x, h0);
+    Tensor z_, x_, h0_;
+    ScanOut r;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        z_ = z.contiguous();
+        x_ = as(x, z.scalar_type());
+        h0_ = as(unwrap(h0), at::kFloat);   // the carries are float32 whatever the arrays are
+        r = mingru_fwd(z_, x_, done, some(h0_), some(as(unwrap(P0), at::kFloat)), true);
+    }
+    if (need) {
+        auto node = record(MinGruOp{done}, z, x, unwrap(h0));
+        torch::autograd::set_history(r.h, node);
+        torch::autograd::set_history(r.h_last, node);
+        node->keep(0, z_);
+        node->keep(1, x_);
+        node->keep(2, r.h, true);
+        node->keep(3, h0_);
+    }
+    return {r.h, r.h_last, r.P_last};
+}
+
+struct LinearAttentionOp {
+    static constexpr int SAVED = 5;   // q, k, v, S_chk, S_last (undefined: the chunk-parallel pair ran)
+    static const char *name() { return "MemoraxLinearAttentionBackward"; }
+    Tensor done;
+    int fmap;
+    bool parallel;
+    variable_list backward(OpNode<LinearAttentionOp> &node, std::array<Tensor, 5> &s, variable_list &grads)
+    {
+        auto r = linear_attn_bwd(s[0], s[1], s[2], done, s[3], parallel ? std::nullopt : some(s[4]), grad_or_zeros(grads[0], s[2]),
+                                 some(as(grads[1], at::kFloat)), fmap, node.wants(3));
+        return {r.dq, r.dk, r.dv, r.dS0};
+    }
+};
+
+// Acting (one time step, no gradients: memoroid.py:93-109 with T = 1) goes to the single-step kernels; in_place lets them
+// update the carried state where it lies, which they do only on the caller's own array (a converted copy is a new one already).
+std::tuple<Tensor, Tensor> linear_attention(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &done, const OptTensor &S0, int fmap,
+                                            bool in_place)
+{
+    const bool need = need_grad(q, k, v, S0);
+    Tensor q_, k_, v_, S0_;
+    AttnOut r;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        q_ = q.contiguous(), k_ = k.contiguous(), v_ = v.contiguous();
+        S0_ = as(unwrap(S0), at::kFloat);
+        if (q_.size(1) == 1 && !need) {
+            auto st = linear_attn_step(q_.select(1, 0), k_.select(1, 0), v_.select(1, 0), done.select(1, 0), some(S0_), std::nullopt, fmap, false,
+                                       1e-6, in_place && S0.has_value() && S0_.is_same(*S0));
+            return {st.o.unsqueeze(1), st.S};
+        }
+        r = linear_attn_fwd(q_, k_, v_, done, some(S0_), fmap, need, std::nullopt);
+    }
+    if (need) {
+        auto node = record(LinearAttentionOp{done, fmap, r.parallel}, q, k, v, unwrap(S0));
+        torch::autograd::set_history(r.o, node);
+        torch::autograd::set_history(r.S_last, node);
+        node->keep(0, q_);
+        node->keep(1, k_);
+        node->keep(2, v_);
+        node->keep(3, r.S_chk);
+        if (!r.parallel) node->keep(4, r.S_last, true);
+    }
+    return {r.o, r.S_last};
+}
+
+struct NormalisedOp {
+    static constexpr int SAVED = 8;   // q, k, v, o, den, S_chk, z_chk, S_last
+    static const char *name() { return "MemoraxNormalisedLinearAttentionBackward"; }
+    Tensor done;
+    int fmap;
+    double eps;
+    bool has_ss;
+    variable_list backward(OpNode<NormalisedOp> &node, std::array<Tensor, 8> &s, variable_list &grads)
+    {
+        auto r = linear_attn_norm_bwd(s[0], s[1], s[2], done, s[5], s[6], s[7], s[3], s[4], grad_or_zeros(grads[0], s[2]),
+                                      some(as(grads[1], at::kFloat)), some(as(grads[2], at::kFloat)), fmap, eps, node.wants(3) || node.wants(4),
+                                      has_ss ? some(as(grads[3], at::kFloat)) : std::nullopt);
+        return {r.dq, r.dk, r.dv, unless(!node.wants(3), r.dS0), unless(!node.wants(4), r.dz0)};
+    }
+};
+
+std::tuple<Tensor, Tensor, Tensor, OptTensor> normalised_linear_attention(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &done,
+                                                                          const OptTensor &S0, const OptTensor &z0, int fmap, double eps,
+                                                                          bool want_ss, bool in_place)
+{
+    const bool need = need_grad(q, k, v, S0, z0);
+    Tensor q_, k_, v_;
+    NormAttnOut r;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        q_ = q.contiguous(), k_ = k.contiguous(), v_ = v.contiguous();
+        const Tensor S0_ = as(unwrap(S0), at::kFloat), z0_ = as(unwrap(z0), at::kFloat);
+        if (q_.size(1) == 1 && !need) {
+            const bool own = in_place && S0.has_value() && S0_.is_same(*S0) && z0.has_value() && z0_.is_same(*z0);
+            auto st = linear_attn_step(q_.select(1, 0), k_.select(1, 0), v_.select(1, 0), done.select(1, 0), some(S0_), some(z0_), fmap, true,
+                                       eps, own);
+            OptTensor ss;
+            if (want_ss) ss = st.o.to(at::kFloat).square().sum(-1).unsqueeze(-1);   // (B,H,1)
+            return {st.o.unsqueeze(1), st.S, st.z, ss};
+        }
+        r = linear_attn_norm_fwd(q_, k_, v_, done, some(S0_), some(z0_), fmap, eps, need, want_ss);
+    }
+    if (need) {
+        auto node = record(NormalisedOp{done, fmap, eps, want_ss}, q, k, v, unwrap(S0), unwrap(z0));
+        torch::autograd::set_history(r.o, node);
+        torch::autograd::set_history(r.S_last, node);
+        torch::autograd::set_history(r.z_last, node);
+        if (want_ss) torch::autograd::set_history(r.ss, node);
+        node->keep(0, q_);
+        node->keep(1, k_);
+        node->keep(2, v_);
+        node->keep(3, r.o, true);
+        node->keep(4, r.den);
+        node->keep(5, r.S_chk);
+        node->keep(6, r.z_chk);
+        node->keep(7, r.S_last, true);
+    }
+    return {r.o, r.S_last, r.z_last, some(r.ss)};
+}
+
+struct GatedOp {
+    static constexpr int SAVED = 6;   // q, k, v, g, S_chk, S_last
+    static const char *name() { return "MemoraxGatedLinearAttentionBackward"; }
+    Tensor done;
+    int fmap;
+    variable_list backward(OpNode<GatedOp> &node, std::array<Tensor, 6> &s, variable_list &grads)
+    {
+        auto r = gated_linear_attn_bwd(s[0], s[1], s[2], s[3], done, s[4], grad_or_zeros(grads[0], s[2]), some(as(grads[1], at::kFloat)), fmap,
+                                       node.wants(4), some(s[5]));
+        return {r.dq, r.dk, r.dv, r.extra, r.dS0};
+    }
+};
+
+std::tuple<Tensor, Tensor> gated_linear_attention(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &g, const Tensor &done,
+                                                  const OptTensor &S0, int fmap, bool in_place)
+{
+    const bool need = need_grad(q, k, v, g, S0);
+    Tensor q_, k_, v_, g_;
+    AttnOut r;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        q_ = q.contiguous(), k_ = k.contiguous(), v_ = v.contiguous(), g_ = as(g, at::kFloat);
+        const Tensor S0_ = as(unwrap(S0), at::kFloat);
+        if (q_.size(1) == 1 && !need) {
+            auto st = gated_linear_attn_step(q_.select(1, 0), k_.select(1, 0), v_.select(1, 0), g_.select(1, 0), done.select(1, 0), some(S0_), fmap,
+                                             in_place && S0.has_value() && S0_.is_same(*S0));
+            return {st.o.unsqueeze(1), st.S};
+        }
+        r = gated_linear_attn_fwd(q_, k_, v_, g_, done, some(S0_), fmap, need);
+    }
+    if (need) {
+        auto node = record(GatedOp{done, fmap}, q, k, v, g, unwrap(S0));
+        torch::autograd::set_history(r.o, node);
+        torch::autograd::set_history(r.S_last, node);
+        node->keep(0, q_);
+        node->keep(1, k_);
+        node->keep(2, v_);
+        node->keep(3, g_);
+        node->keep(4, r.S_chk);
+        node->keep(5, r.S_last, true);
+    }
+    return {r.o, r.S_last};
+}
+
+struct DeltaOp {
+    static constexpr int SAVED = 6;   // q, k, v, beta, S_chk, Tm_chk
+    static const char *name() { return "MemoraxDeltaRuleBackward"; }
+    Tensor done;
+    bool prologue;
+    int resets;
+    variable_list backward(OpNode<DeltaOp> &node, std::array<Tensor, 6> &s, variable_list &grads)
+    {
+        auto r = delta_rule_bwd(s[0], s[1], s[2], s[3], done, s[4], s[5], grad_or_zeros(grads[0], s[2]), some(as(grads[1], at::kFloat)),
+                                node.wants(4), std::nullopt, prologue, resets);
+        return {r.dq, r.dk, r.dv, r.extra, r.dS0};
+    }
+};
+
+std::tuple<Tensor, Tensor> delta_rule(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &beta, const Tensor &done,
+                                      const OptTensor &S0, bool prologue, int resets, bool in_place)
+{
+    const bool need = need_grad(q, k, v, beta, S0);
+    Tensor q_, k_, v_, b_;
+    DeltaOut r;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        q_ = q.contiguous(), k_ = k.contiguous(), v_ = v.contiguous(), b_ = beta.contiguous();
+        const Tensor S0_ = as(unwrap(S0), at::kFloat);
+        if (q_.size(1) == 1 && !need) {
+            Tensor k1 = k_.select(1, 0), b1 = b_.select(1, 0);
+            if (prologue) {   // a (B,H,d) array: the prologue as array operations costs nothing here
+                const Tensor kf = k1.to(at::kFloat);
+                k1 = kf.div(kf.norm(2, {-1}, true).clamp_min(1e-12)).to(k_.scalar_type());
+                b1 = b1.to(at::kFloat).sigmoid().to(b_.scalar_type());
+            }
+            auto st = delta_rule_step(q_.select(1, 0), k1, v_.select(1, 0), b1, done.select(1, 0), some(S0_),
+                                      in_place && S0.has_value() && S0_.is_same(*S0));
+            return {st.o.unsqueeze(1), st.S};
+        }
+        r = delta_rule_fwd(q_, k_, v_, b_, done, some(S0_), need, std::nullopt, prologue, std::nullopt, MRX_FACTORS_AUTO, resets);
+    }
+    if (need) {
+        auto node = record(DeltaOp{done, prologue, resets}, q, k, v, beta, unwrap(S0));
+        torch::autograd::set_history(r.o, node);
+        torch::autograd::set_history(r.S_last, node);
+        node->keep(0, q_);
+        node->keep(1, k_);
+        node->keep(2, v_);
+        node->keep(3, b_);
+        node->keep(4, r.S_chk);
+        node->keep(5, r.Tm_chk);
+    }
+    return {r.o, r.S_last};
+}
+
+struct MlstmGatesOp {
+    static constexpr int SAVED = 4;   // log_i, log_f, m, m0
+    static const char *name() { return "MemoraxMlstmGatesBackward"; }
+    Tensor done;
+    double g_floor;
+    variable_list backward(OpNode<MlstmGatesOp> &node, std::array<Tensor, 4> &s, variable_list &grads)
+    {
+        auto r = mlstm_gates_bwd(s[0], s[1], done, some(s[3]), s[2], some(as(grads[0], at::kFloat)), some(as(grads[1], at::kFloat)),
+                                 some(as(grads[2], at::kFloat)), g_floor, node.wants(2));
+        return {r[0], r[1], r[2]};
+    }
+};
+
+std::tuple<Tensor, Tensor, Tensor> mlstm_gates(const Tensor &log_i, const Tensor &log_f, const Tensor &done, const OptTensor &m0, double g_floor)
+{
+    const bool need = need_grad(log_i, log_f, m0);
+    Tensor li, lf, m0_;
+    std::array<Tensor, 3> r;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        li = as(log_i, at::kFloat), lf = as(log_f, at::kFloat), m0_ = as(unwrap(m0), at::kFloat);
+        r = mlstm_gates_fwd(li, lf, done, some(m0_), g_floor);
+    }
+    if (need) {
+        auto node = record(MlstmGatesOp{done, g_floor}, log_i, log_f, unwrap(m0));
+        for (auto &t : r) torch::autograd::set_history(t, node);
+        node->keep(0, li);
+        node->keep(1, lf);
+        node->keep(2, r[0], true);
+        node->keep(3, m0_);
+    }
+    return {r[0], r[1], r[2]};
+}
+
+struct SiluGateOp {
+    static constexpr int SAVED = 2;   // h, g
+    static const char *name() { return "MemoraxSiluGateBackward"; }
+    variable_list backward(OpNode<SiluGateOp> &, std::array<Tensor, 2> &s, variable_list &grads)
+    {
+        if (!grads[0].defined()) return {Tensor(), Tensor()};
+        auto r = silu_gate_bwd(s[0], s[1], as(grads[0], s[0].scalar_type()));
+        return {r[0], r[1]};
+    }
+};
+
+Tensor silu_gate(const Tensor &h, const Tensor &g)
+{
+    Tensor hc, gc, y;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        auto dt = c10::promoteTypes(h.scalar_type(), g.scalar_type());
+        if (dt != at::kFloat && dt != at::kBFloat16) dt = at::kFloat;
+        hc = as(h, dt), gc = as(g, dt);
+        y = silu_gate_fwd(hc, gc);
+    }
+    if (need_grad(h, g)) {
+        auto node = record(SiluGateOp{}, h, g);
+        torch::autograd::set_history(y, node);
+        node->keep(0, hc);
+        node->keep(1, gc);
+    }
+    return y;
+}
+
+// RMS norm (center false) or layer norm; fork: the input is handed on beside its norm -- (x, norm(x)) -- so that the
+// gradients of both meet in the norm's backward kernel instead of in a pass of their own.
+struct NormOp {
+    static constexpr int SAVED = 2;   // x, scale
+    static const char *name() { return "MemoraxNormBackward"; }
+    double eps;
+    bool center, fork;
+    variable_list backward(OpNode<NormOp> &node, std::array<Tensor, 2> &s, variable_list &grads)
+    {
+        const Tensor &x = s[0], dres = fork ? grads[0] : Tensor(), &dy = grads[fork];
+        if (!dy.defined()) return {dres, Tensor(), Tensor()};   // the norm's branch was not used
+        const Tensor dyc = dy.scalar_type() == at::kFloat || dy.scalar_type() == at::kBFloat16 ? dy.contiguous() : as(dy, at::kFloat);
+        auto r = norm_bwd(x, some(s[1]), dyc, eps, node.wants(1) || node.wants(2), some(as(dres, x.scalar_type())), center);
+        return {r.dx, unless(!node.wants(1), r.dscale), unless(!node.wants(2), r.dbias)};
+    }
+};
+
+std::tuple<Tensor, Tensor> norm(const Tensor &x, const OptTensor &scale, const OptTensor &bias, double eps, std::optional<ScalarType> out_dtype,
+                                bool center, bool fork)
+{
+    Tensor xc, sc, y, res;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        xc = x.scalar_type() == at::kFloat || x.scalar_type() == at::kBFloat16 ? x.contiguous() : as(x, at::kFloat);
+        sc = as(unwrap(scale), at::kFloat);
+        y = norm_fwd(xc, some(sc), some(as(unwrap(bias), at::kFloat)), eps, out_dtype, center);
+        if (fork)   // x under a second name, with x's version counter: writing to either is noticed by the saved tensor
+            res = xc.scalar_type() != x.scalar_type()
+                      ? xc.to(x.scalar_type())
+                      : Tensor(xc.unsafeGetTensorImpl()->shallow_copy_and_detach(torch::autograd::impl::version_counter(xc), false));
+    }
+    if (need_grad(x, scale, bias)) {
+        auto node = record(NormOp{eps, center, fork}, x, unwrap(scale), unwrap(bias));
+        if (fork) torch::autograd::set_history(res, node);
+        torch::autograd::set_history(y, node);
+        node->keep(0, xc);
+        node->keep(1, sc);
+    }
+    return {fork ? res : x, y};
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_native, m)
+{
+    m.def("bind", &bind);
+    // the other calls touch no Python object: they run without the interpreter's lock
+    auto def = [&](const char *name, auto f) { m.def(name, f, py::call_guard<py::gil_scoped_release>()); };
+    def("chunk_size", &chunk_size);
+    // checks, allocation, launch (memorax_amd/kernels.py)
+    auto opt = [](const Tensor &t) { return some(t); };
+    def("linear_scan_fwd", [=](const Tensor &a, const Tensor &b, const Tensor &done, const OptTensor &h0, const OptTensor &P0, bool want_P) {
+        auto r = scan_fwd(a, b, done, h0, P0, want_P);
+        return std::make_tuple(r.h, r.h_last, opt(r.P_last));
+    });
+    def("linear_scan_bwd", [](const Tensor &a, const Tensor &h, const Tensor &done, const OptTensor &h0, const Tensor &g,
+                                const OptTensor &g_last, bool sum_da) {
+        auto r = scan_bwd(a, h, done, h0, g, g_last, sum_da);
+        return std::make_tuple(r.da, r.db, r.dh0);
+    });
+    def("linear_scan_last", &scan_last);
+    def("mingru_scan_fwd", [=](const Tensor &z, const Tensor &x, const Tensor &done, const OptTensor &h0, const OptTensor &P0, bool want_P) {
+        auto r = mingru_fwd(z, x, done, h0, P0, want_P);
+        return std::make_tuple(r.h, r.h_last, opt(r.P_last));
+    });
+    def("mingru_scan_bwd", [](const Tensor &z, const Tensor &x, const Tensor &h, const Tensor &done, const OptTensor &h0, const Tensor &g,
+                                const OptTensor &g_last) {
+        auto r = mingru_bwd(z, x, h, done, h0, g, g_last);
+        return std::make_tuple(r.da, r.db, r.dh0);
+    });
+    def("mlstm_gates_fwd", [](const Tensor &li, const Tensor &lf, const Tensor &done, const OptTensor &m0, double g_floor) {
+        auto r = mlstm_gates_fwd(li, lf, done, m0, g_floor);
+        return std::make_tuple(r[0], r[1], r[2]);
+    });
+    def("mlstm_gates_bwd", [=](const Tensor &li, const Tensor &lf, const Tensor &done, const OptTensor &m0, const Tensor &mm, const OptTensor &dm,
+                                 const OptTensor &dg, const OptTensor &dw, double g_floor, bool want_dm0) {
+        auto r = mlstm_gates_bwd(li, lf, done, m0, mm, dm, dg, dw, g_floor, want_dm0);
+        return std::make_tuple(r[0], r[1], opt(r[2]));
+    });
+    def("norm_fwd", &norm_fwd);
+    def("norm_bwd", [=](const Tensor &x, const OptTensor &scale, const Tensor &dy, double eps, bool want, const OptTensor &dx_add, bool center) {
+        auto r = norm_bwd(x, scale, dy, eps, want, dx_add, center);
+        return std::make_tuple(r.dx, opt(r.dscale), opt(r.dbias));
+    });
+    def("silu_gate_fwd", &silu_gate_fwd);
+    def("silu_gate_bwd", [](const Tensor &h, const Tensor &g, const Tensor &dy) {
+        auto r = silu_gate_bwd(h, g, dy);
+        return std::make_tuple(r[0], r[1]);
+    });
+    def("linear_attn_fwd", [=](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &done, const OptTensor &S0, int fmap,
+                                 bool save_chk, std::optional<bool> chunk_parallel) {
+        auto r = linear_attn_fwd(q, k, v, done, S0, fmap, save_chk, chunk_parallel);
+        return std::make_tuple(r.o, r.S_last, opt(r.S_chk), r.parallel);
+    });
+    def("linear_attn_bwd", [=](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &done, const Tensor &S_chk,
+                                 const OptTensor &S_last, const Tensor &dout, const OptTensor &dS_last, int fmap, bool want_dS0) {
+        auto r = linear_attn_bwd(q, k, v, done, S_chk, S_last, dout, dS_last, fmap, want_dS0);
+        return std::make_tuple(r.dq, r.dk, r.dv, opt(r.dS0));
+    });
+    def("linear_attn_norm_fwd", [=](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &done, const OptTensor &S0,
+                                      const OptTensor &z0, int fmap, double eps, bool save_chk, bool want_ss) {
+        auto r = linear_attn_norm_fwd(q, k, v, done, S0, z0, fmap, eps, save_chk, want_ss);
+        return std::make_tuple(r.o, r.den, r.S_last, r.z_last, opt(r.S_chk), opt(r.z_chk), opt(r.ss));
+    });
+    def("linear_attn_norm_bwd", [=](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &done, const Tensor &S_chk,
+                                      const Tensor &z_chk, const Tensor &S_last, const Tensor &o, const Tensor &den, const Tensor &dout,
+                                      const OptTensor &dS_last, const OptTensor &dz_last, int fmap, double eps, bool want_d0,
+                                      const OptTensor &d_ss) {
+        auto r = linear_attn_norm_bwd(q, k, v, done, S_chk, z_chk, S_last, o, den, dout, dS_last, dz_last, fmap, eps, want_d0, d_ss);
+        return std::make_tuple(r.dq, r.dk, r.dv, opt(r.dS0), opt(r.dz0));
+    });
+    def("gated_linear_attn_fwd", [=](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &g, const Tensor &done,
+                                       const OptTensor &S0, int fmap, bool save_chk) {
+        auto r = gated_linear_attn_fwd(q, k, v, g, done, S0, fmap, save_chk);
+        return std::make_tuple(r.o, r.S_last, opt(r.S_chk));
+    });
+    def("gated_linear_attn_bwd", [=](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &g, const Tensor &done,
+                                       const Tensor &S_chk, const Tensor &dout, const OptTensor &dS_last, int fmap, bool want_dS0,
+                                       const OptTensor &S_last) {
+        auto r = gated_linear_attn_bwd(q, k, v, g, done, S_chk, dout, dS_last, fmap, want_dS0, S_last);
+        return std::make_tuple(r.dq, r.dk, r.dv, r.extra, opt(r.dS0));
+    });
+    def("delta_rule_fwd", [=](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &beta, const Tensor &done, const OptTensor &S0,
+                                bool save_chk, const std::optional<std::array<OptTensor, 4>> &out, bool prologue, std::optional<bool> tm_scratch,
+                                int factors, int resets) {
+        auto r = delta_rule_fwd(q, k, v, beta, done, S0, save_chk, out, prologue, tm_scratch, factors, resets);
+        return std::make_tuple(r.o, r.S_last, opt(r.S_chk), opt(r.Tm_chk));
+    });
+    def("delta_rule_bwd", [=](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &beta, const Tensor &done, const Tensor &S_chk,
+                                const Tensor &Tm_chk, const Tensor &dout, const OptTensor &dS_last, bool want_dS0,
+                                const std::optional<std::array<OptTensor, 5>> &out, bool prologue, int resets) {
+        auto r = delta_rule_bwd(q, k, v, beta, done, S_chk, Tm_chk, dout, dS_last, want_dS0, out, prologue, resets);
+        return std::make_tuple(r.dq, r.dk, r.dv, r.extra, opt(r.dS0));
+    });
+    def("delta_rule_fwd_noalloc", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &beta, const Tensor &done,
+                                       const OptTensor &S0, const OptTensor &o, const OptTensor &S_last) {
+        auto r = delta_rule_fwd_noalloc(q, k, v, beta, done, S0, o, S_last);
+        return std::make_tuple(r[0], r[1]);
+    });
+    def("linear_attn_step", [=](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &done, const OptTensor &S, const OptTensor &z,
+                                  int fmap, bool normalise, double eps, bool inplace) {
+        auto r = linear_attn_step(q, k, v, done, S, z, fmap, normalise, eps, inplace);
+        return std::make_tuple(r.o, r.S, opt(r.z));
+    });
+    def("gated_linear_attn_step", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &g, const Tensor &done, const OptTensor &S,
+                                       int fmap, bool inplace) {
+        auto r = gated_linear_attn_step(q, k, v, g, done, S, fmap, inplace);
+        return std::make_tuple(r.o, r.S);
+    });
+    def("delta_rule_step", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &beta, const Tensor &done, const OptTensor &S,
+                                bool inplace) {
+        auto r = delta_rule_step(q, k, v, beta, done, S, inplace);
+        return std::make_tuple(r.o, r.S);
+    });
+    // differentiable operators (memorax_amd/functional.py)
+    def("linear_scan", &linear_scan);
+    def("mingru_scan", &mingru_scan);
+    def("linear_attention", &linear_attention);
+    def("normalised_linear_attention", &normalised_linear_attention);
+    def("gated_linear_attention", &gated_linear_attention);
+    def("delta_rule", &delta_rule);
+    def("mlstm_gates", &mlstm_gates);
+    def("silu_gate", &silu_gate);
+    def("norm", &norm);
+}
