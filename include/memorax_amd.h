@@ -369,6 +369,54 @@ int mrx_silu_gate_fwd(void *stream, const void *h, const void *g, void *y, int64
 int mrx_silu_gate_bwd(void *stream, const void *h, const void *g, const void *dy, void *dh, void *dg,
                       int64_t n, int dtype);
 
+/* ---- Mamba and mLSTM cells: the passes around their recurrence -----------------
+ * The causal depthwise convolution over time with silu behind it (mamba.py:88-106, mlstm.py:110-125):
+ *     s_t = bias + sum_j w_j x_{t-K+1+j} ,  y_t = silu(s_t)     (x = 0 before the call's first step; resets do not cut it)
+ * x, dx: rows of C features ld_x (ld_dx) floats apart, time steps of a sequence consecutive; y, dy: (B,T,C) dense; w: (C,K);
+ * C a multiple of 4, K <= 4; all float32.  Backward: param_grads receives [dw (C,K) | dbias (C)]; workspace:
+ * MRX_CONV_PARTS * C * (K + 1) floats, overwritten (per-workgroup partial sums, added in a fixed order). */
+#define MRX_CONV_PARTS 256
+int mrx_causal_conv_silu_fwd(void *stream, const float *x, int64_t ld_x, const float *w, const float *bias,
+                             float *y, int64_t B, int64_t T, int64_t C, int64_t K);
+int mrx_causal_conv_silu_bwd(void *stream, const float *x, int64_t ld_x, const float *w, const float *bias,
+                             const float *dy, float *dx, int64_t ld_dx, float *param_grads, float *workspace,
+                             int64_t B, int64_t T, int64_t C, int64_t K);
+
+/* MambaCell's elements (mamba.py:88-122) from its projections: that convolution over the hidden channels (up, the first
+ * H*P columns of rows ld_up apart), B's (b_in) and C's (c_in: (B,T,H*N) each), and
+ *     v = hidden ,  k = B dt ,  q = C ,  dt = softplus(dt_in + dt_bias) ,  g = -dt exp(A_log)
+ * v: (B,T,H,P), k, q: (B,T,H,N), g: (B,T,H) -- the operands of mrx_gated_linear_attn_*.  conv_w: (H*P + 2*H*N, K).
+ * P a multiple of 4; N a power of two from 4 to 256; K <= 4; all float32.
+ * Backward: dv, dk, dq, dg are the gradients of the elements, d_o that of the read-out's sum o + D hidden (its share D d_o
+ * of hidden's gradient is added here).  d_up: rows ld_dup apart, only the first H*P columns are written.  param_grads:
+ * with C = H*P + 2*H*N, [dconv_w (C,K) | dconv_b (C) | ddt_bias (H) | dA_log (H) | dD (H, P/4): still to be summed over
+ * its last axis]; workspace: MRX_CONV_PARTS times that many floats. */
+int mrx_mamba_elements_fwd(void *stream, const float *up, int64_t ld_up, const float *b_in, const float *c_in,
+                           const float *dt_in, const float *conv_w, const float *conv_b, const float *dt_bias,
+                           const float *A_log, float *v, float *k, float *q, float *g, int64_t B, int64_t T,
+                           int64_t H, int64_t P, int64_t N, int64_t K);
+int mrx_mamba_elements_bwd(void *stream, const float *up, int64_t ld_up, const float *b_in, const float *c_in,
+                           const float *dt_in, const float *conv_w, const float *conv_b, const float *dt_bias,
+                           const float *A_log, const float *D, const float *dv, const float *dk, const float *dq,
+                           const float *dg, const float *d_o, float *d_up, int64_t ld_dup, float *db_in,
+                           float *dc_in, float *ddt_in, float *param_grads, float *workspace, int64_t B, int64_t T,
+                           int64_t H, int64_t P, int64_t N, int64_t K);
+
+/* The carry's decay leaf after a call (mamba.py:119-122 under memoroid.py:60-91):
+ *     decay_last = (no reset in the call ? decay0 : 1) * exp(sum of g from the last reset on, its step included)
+ * g: (B,T,H) float32; decay0, decay_last: (B,H). */
+int mrx_decay_last(void *stream, const float *g, const void *done, const float *decay0, float *decay_last, int64_t B,
+                   int64_t T, int64_t H, int done_dtype);
+
+/* MambaCell.read up to its output projection (mamba.py:124-144): y = rms_norm(o + D hidden) * scale * silu(z) over rows of
+ * H*P features (a multiple of 4 per head, at most 2048); z, dz: rows ld_z (ld_dz) floats apart; D: (H), scale: (H*P); float32.
+ * Backward: d_o (the gradient of o + D hidden), dz, dscale; workspace: MRX_RMS_NORM_PARTS * H * P floats. */
+int mrx_mamba_readout_fwd(void *stream, const float *o, const float *hidden, const float *z, int64_t ld_z,
+                          const float *D, const float *scale, float *y, int64_t rows, int64_t H, int64_t P, float eps);
+int mrx_mamba_readout_bwd(void *stream, const float *o, const float *hidden, const float *z, int64_t ld_z,
+                          const float *D, const float *scale, const float *dy, float *d_o, float *dz, int64_t ld_dz,
+                          float *dscale, float *workspace, int64_t rows, int64_t H, int64_t P, float eps);
+
 /* ---- mLSTM: the stabiliser of the cell's gates ---------------------------------
  * mLSTMCell's elements (C, log_f, n, m) combine by the max-stabilised gated sum of mlstm.py:190-206
  * (m = max(m_a + log_f_b, m_b), both sides rescaled by exp(. - m)) under Memoroid.scan_fn's select-reset

@@ -59,6 +59,13 @@ SIGNATURES = {
     "mrx_layer_norm_bwd": (_I, [_P] * 9 + [_L] * 2 + [_I, _I, ctypes.c_float]),
     "mrx_silu_gate_fwd": (_I, [_P] * 4 + [_L, _I]),
     "mrx_silu_gate_bwd": (_I, [_P] * 6 + [_L, _I]),
+    "mrx_causal_conv_silu_fwd": (_I, [_P, _P, _L, _P, _P, _P] + [_L] * 4),
+    "mrx_causal_conv_silu_bwd": (_I, [_P, _P, _L, _P, _P, _P, _P, _L, _P, _P] + [_L] * 4),
+    "mrx_mamba_elements_fwd": (_I, [_P, _P, _L] + [_P] * 11 + [_L] * 6),
+    "mrx_mamba_elements_bwd": (_I, [_P, _P, _L] + [_P] * 14 + [_L] + [_P] * 5 + [_L] * 6),
+    "mrx_decay_last": (_I, [_P] * 5 + [_L] * 3 + [_I]),
+    "mrx_mamba_readout_fwd": (_I, [_P] * 4 + [_L] + [_P] * 3 + [_L] * 3 + [ctypes.c_float]),
+    "mrx_mamba_readout_bwd": (_I, [_P] * 4 + [_L] + [_P] * 5 + [_L] + [_P] * 2 + [_L] * 3 + [ctypes.c_float]),
     "mrx_rms_norm_fwd": (_I, [_P] * 4 + [_L] * 2 + [_I, _I, ctypes.c_float]),
     "mrx_rms_norm_bwd": (_I, [_P] * 8 + [_L] * 2 + [_I, _I, ctypes.c_float]),
 }

@@ -44,7 +44,9 @@ using torch::autograd::variable_list;
     X(mrx_linear_attn_chunk_parallel_pays) X(mrx_linear_attn_norm_fwd) X(mrx_linear_attn_norm_bwd)                   \
     X(mrx_gated_linear_attn_fwd) X(mrx_gated_linear_attn_bwd) X(mrx_delta_rule_fwd) X(mrx_delta_rule_bwd)            \
     X(mrx_delta_rule_fwd_noalloc) X(mrx_deltanet_fwd) X(mrx_deltanet_bwd) X(mrx_linear_attn_step)                    \
-    X(mrx_gated_linear_attn_step) X(mrx_delta_rule_step)
+    X(mrx_gated_linear_attn_step) X(mrx_delta_rule_step) X(mrx_causal_conv_silu_fwd) X(mrx_causal_conv_silu_bwd)     \
+    X(mrx_mamba_elements_fwd) X(mrx_mamba_elements_bwd) X(mrx_decay_last) X(mrx_mamba_readout_fwd)                   \
+    X(mrx_mamba_readout_bwd)
 struct {
 #define MRX_MEMBER(name) decltype(&::name) name = nullptr;
     MRX_BOUND(MRX_MEMBER)
@@ -1116,6 +1118,108 @@ std::tuple<Tensor, Tensor> norm(const Tensor &x, const OptTensor &scale, const O
     return {fork ? res : x, y};
 }
 
+// ---- the Mamba cell between its projections: elements, recurrence, gated read-out (conv_cells.hip)
+struct MambaSizes {
+    int64_t B, T, H, P, N, K, W;   // W = H * P, the hidden width; up holds (hidden | z): rows of 2 W
+};
+
+struct MambaOp {
+    enum { UP, BIN, CIN, DTIN, CONVW, CONVB, DTB, ALOG, D_, SCALE, V, K_, Q, G, O, SCHK, SLAST, SAVED };
+    static const char *name() { return "MemoraxMambaBackward"; }
+    Tensor done;
+    MambaSizes n;
+    double eps;
+    variable_list backward(OpNode<MambaOp> &node, std::array<Tensor, SAVED> &s, variable_list &grads)
+    {
+        const Tensor dy = grad_or_zeros(grads[0], s[V].view({n.B, n.T, n.W})), &up = s[UP];
+        const Tensor d_up = fresh_like(up), d_o = fresh_like(s[O]), dscale = fresh({n.W}, at::kFloat, up);
+        Tensor work = fresh({MRX_RMS_NORM_PARTS, n.W}, at::kFloat, up);
+        check(lib.mrx_mamba_readout_bwd(stream(), fptr(s[O]), fptr(s[V]), fptr(up) + n.W, 2 * n.W, fptr(s[D_]), fptr(s[SCALE]), fptr(dy),
+                                        fptr(d_o), fptr(d_up) + n.W, 2 * n.W, fptr(dscale), fptr(work), n.B * n.T, n.H, n.P, (float)eps),
+              "mrx_mamba_readout_bwd");
+        auto r = gated_linear_attn_bwd(s[Q], s[K_], s[V], s[G], done, s[SCHK], d_o, some(as(grads[1], at::kFloat)), 0, node.wants(10), s[SLAST]);
+        Tensor ddecay0;
+        if (grads[2].defined()) {   // the decay leaf handed on: it depends on every g from the last reset on
+            const Tensor behind = done.ne(0).to(at::kInt).flip(1).cumsum(1).flip(1);   // resets at or after each step
+            const Tensor live = (behind - done.ne(0).to(at::kInt)).eq(0).to(at::kFloat).unsqueeze(-1), intact = behind.slice(1, 0, 1).eq(0).to(at::kFloat);
+            const Tensor total = (s[G] * live).sum(1).exp() * grads[2].to(at::kFloat);   // (B,H), per unit of the decay it started from
+            ddecay0 = total * intact;
+            r.extra = r.extra + live * ((at::where(intact.ne(0), decay0, at::ones_like(decay0)) * total).unsqueeze(1));
+        }
+        const int64_t C = n.W + 2 * n.H * n.N, cols = C * (n.K + 1) + 2 * n.H + n.W / 4;
+        const Tensor params = fresh({cols}, at::kFloat, up), db_in = fresh_like(s[BIN]), dc_in = fresh_like(s[CIN]), ddt = fresh_like(s[DTIN]);
+        work = fresh({MRX_CONV_PARTS, cols}, at::kFloat, up);
+        check(lib.mrx_mamba_elements_bwd(stream(), fptr(up), 2 * n.W, fptr(s[BIN]), fptr(s[CIN]), fptr(s[DTIN]), fptr(s[CONVW]), fptr(s[CONVB]),
+                                         fptr(s[DTB]), fptr(s[ALOG]), fptr(s[D_]), fptr(r.dv), fptr(r.dk), fptr(r.dq), fptr(r.extra), fptr(d_o),
+                                         fptr(d_up), 2 * n.W, fptr(db_in), fptr(dc_in), fptr(ddt), fptr(params), fptr(work), n.B, n.T, n.H, n.P,
+                                         n.N, n.K),
+              "mrx_mamba_elements_bwd");
+        auto part = [&, at = int64_t(0)](int64_t len) mutable { return params.narrow(0, std::exchange(at, at + len), len); };
+        const Tensor dw = part(C * n.K).view({C, 1, n.K}), dcb = part(C), ddtb = part(n.H), dA = part(n.H), dD = part(n.W / 4).view({n.H, n.P / 4}).sum(1);
+        return {d_up, db_in, dc_in, ddt, dw, dcb, ddtb, dA, dD, dscale, r.dS0, ddecay0};
+    }
+    Tensor decay0;
+};
+
+// up (B,T,2HP), b_in, c_in (B,T,HN), dt_in (B,T,H) and the cell's parameters, all float32 -> y (B,T,HP) before the output
+// projection, S_last (B,H,P,N), decay_last (B,H).  Acting (one step, no gradients) runs the single-step kernel.
+std::tuple<Tensor, Tensor, Tensor> mamba_mix(const Tensor &up, const Tensor &b_in, const Tensor &c_in, const Tensor &dt_in, const Tensor &conv_w,
+                                             const Tensor &conv_b, const Tensor &dt_bias, const Tensor &A_log, const Tensor &D,
+                                             const Tensor &scale, const Tensor &done_, const Tensor &S0, const Tensor &decay0, double eps,
+                                             bool in_place)
+{
+    TORCH_CHECK_VALUE(up.dim() == 3 && S0.dim() == 4 && conv_w.dim() == 3, "mamba_mix: up (B,T,2HP), S0 (B,H,P,N), conv_w (C,1,K)");
+    MambaSizes n{up.size(0), up.size(1), S0.size(1), S0.size(2), S0.size(3), conv_w.size(2), S0.size(1) * S0.size(2)};
+    const int64_t C = n.W + 2 * n.H * n.N;
+    chk(up, "up", at::kFloat, {n.B, n.T, 2 * n.W});
+    chk(b_in, "b_in", at::kFloat, {n.B, n.T, n.H * n.N});
+    chk(c_in, "c_in", at::kFloat, {n.B, n.T, n.H * n.N});
+    chk(dt_in, "dt_in", at::kFloat, {n.B, n.T, n.H});
+    chk(conv_w, "conv_w", at::kFloat, {C, 1, n.K});
+    chk(conv_b, "conv_b", at::kFloat, {C});
+    chk(dt_bias, "dt_bias", at::kFloat, {n.H});
+    chk(A_log, "A_log", at::kFloat, {n.H});
+    chk(D, "D", at::kFloat, {n.H});
+    chk(scale, "scale", at::kFloat, {n.W});
+    const bool need = need_grad(up, b_in, c_in, dt_in, conv_w, conv_b, dt_bias, A_log, D, scale, S0, decay0);
+    Tensor v, k, q, g, o, S_chk, S_last, y, decay0_, decay_last;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const Tensor S0_ = as(S0, at::kFloat);
+        decay0_ = as(decay0, at::kFloat);
+        chk(decay0_, "decay0", at::kFloat, {n.B, n.H});
+        const Done done(done_, n.B, n.T);
+        v = fresh({n.B, n.T, n.H, n.P}, at::kFloat, up), k = fresh({n.B, n.T, n.H, n.N}, at::kFloat, up), q = fresh_like(k), g = fresh_like(dt_in);
+        check(lib.mrx_mamba_elements_fwd(stream(), fptr(up), 2 * n.W, fptr(b_in), fptr(c_in), fptr(dt_in), fptr(conv_w), fptr(conv_b),
+                                         fptr(dt_bias), fptr(A_log), fptr(v), fptr(k), fptr(q), fptr(g), n.B, n.T, n.H, n.P, n.N, n.K),
+              "mrx_mamba_elements_fwd");
+        if (n.T == 1 && !need) {
+            auto st = gated_linear_attn_step(q.select(1, 0), k.select(1, 0), v.select(1, 0), g.select(1, 0), done.t.select(1, 0), S0_, 0,
+                                             in_place && S0_.is_same(S0));
+            o = st.o, S_last = st.S;
+        } else {
+            auto r = gated_linear_attn_fwd(q, k, v, g, done.t, S0_, 0, need);
+            o = r.o, S_last = r.S_last, S_chk = r.S_chk;
+        }
+        y = fresh({n.B, n.T, n.W}, at::kFloat, up);
+        check(lib.mrx_mamba_readout_fwd(stream(), fptr(o), fptr(v), fptr(up) + n.W, 2 * n.W, fptr(D), fptr(scale), fptr(y), n.B * n.T, n.H, n.P,
+                                        (float)eps),
+              "mrx_mamba_readout_fwd");
+        decay_last = fresh({n.B, n.H}, at::kFloat, up);
+        check(lib.mrx_decay_last(stream(), fptr(g), done.p(), fptr(decay0_), fptr(decay_last), n.B, n.T, n.H, done.dtype), "mrx_decay_last");
+    }
+    if (need) {
+        auto node = record(MambaOp{done_, n, eps, decay0_}, up, b_in, c_in, dt_in, conv_w, conv_b, dt_bias, A_log, D, scale, S0, decay0);
+        torch::autograd::set_history(y, node);
+        torch::autograd::set_history(S_last, node);
+        torch::autograd::set_history(decay_last, node);
+        const Tensor *kept[] = {&up, &b_in, &c_in, &dt_in, &conv_w, &conv_b, &dt_bias, &A_log, &D, &scale, &v, &k, &q, &g, &o, &S_chk};
+        for (int i = 0; i < MambaOp::SLAST; ++i) node->keep(i, *kept[i]);
+        node->keep(MambaOp::SLAST, S_last, true);
+    }
+    return {y, S_last, decay_last};
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_native, m)
@@ -1239,4 +1343,5 @@ PYBIND11_MODULE(_native, m)
     def("mlstm_gates", &mlstm_gates);
     def("silu_gate", &silu_gate);
     def("norm", &norm);
+    def("mamba_mix", &mamba_mix);
 }

@@ -13,6 +13,7 @@
 // partial sums that a second small kernel adds up in a fixed order.  CENTER selects the layer norm.
 #include <math.h>
 
+#include "col_sum.h"
 #include "common.h"
 
 namespace mrx {
@@ -202,34 +203,6 @@ norm_bwd_kernel(const XT *__restrict__ x, const float *__restrict__ scale, const
     }
 }
 
-// out_y[col] = sum over the nparts rows of block y of parts, in a fixed order (y = 0: dscale, y = 1: dbias): 64 columns
-// per workgroup, sixteen threads per column that each add every sixteenth row, four independent sums in flight per thread.
-constexpr int RD_GROUPS = 16;
-__global__ void __launch_bounds__(64 * RD_GROUPS) norm_param_grad_kernel(const float *__restrict__ parts, float *__restrict__ dscale,
-                                                                      float *__restrict__ dbias, int nparts, int D)
-{
-    __shared__ float red[RD_GROUPS][64];
-    const int c = threadIdx.x & 63, g = threadIdx.x >> 6, col = blockIdx.x * 64 + c;
-    parts += (int64_t)blockIdx.y * nparts * D;
-    float *out = blockIdx.y ? dbias : dscale;
-    float s[4] = {0.f, 0.f, 0.f, 0.f};
-    if (col < D) {
-        int p = g;
-        for (; p + 3 * RD_GROUPS < nparts; p += 4 * RD_GROUPS)
-#pragma unroll
-            for (int u = 0; u < 4; ++u) s[u] += parts[(int64_t)(p + u * RD_GROUPS) * D + col];
-        for (; p < nparts; p += RD_GROUPS) s[0] += parts[(int64_t)p * D + col];
-    }
-    red[g][c] = (s[0] + s[1]) + (s[2] + s[3]);
-    __syncthreads();
-    if (g == 0 && col < D) {
-        float t = 0.f;
-#pragma unroll
-        for (int j = 0; j < RD_GROUPS; ++j) t += red[j][c];
-        out[col] = t;
-    }
-}
-
 bool known(int dtype) { return dtype == MRX_F32 || dtype == MRX_BF16; }
 // rows are read and written four elements at a time
 bool quad_aligned(const void *p, int dtype) { return aligned(p, dtype == MRX_F32 ? 16 : 8); }
@@ -326,8 +299,7 @@ template <bool CENTER> int norm_bwd(BwdCall a, int x_dtype, int dy_dtype)
     else
         rc = dy_dtype == MRX_F32 ? bwd_by_width<__bf16, float, CENTER>(a) : bwd_by_width<__bf16, __bf16, CENTER>(a);
     if (rc != MRX_OK || !a.dscale) return rc;
-    return launch_kernel(norm_param_grad_kernel, dim3((unsigned)((a.D + 63) / 64), CENTER ? 2u : 1u), dim3(64 * RD_GROUPS), 0, a.st,
-                         a.workspace, a.dscale, a.dbias, (int)a.grid, a.D);
+    return launch_column_sum(a.st, a.workspace, a.dscale, CENTER ? a.dbias : nullptr, (int)a.grid, a.D);
 }
 
 }  // namespace

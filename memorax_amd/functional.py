@@ -38,6 +38,11 @@ def step_in_place():
         _step_in_place = before
 
 
+def stepping_in_place():
+    """Whether the caller has allowed it (step_in_place)."""
+    return _step_in_place
+
+
 _FMAP = {None: 0, "none": 0, 0: 0, "elu1": 1, 1: 1}
 _HD = 64  # widest head dim of the kernels (d_k = d_v = 64 or 32)
 

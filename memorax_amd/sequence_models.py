@@ -29,9 +29,11 @@ import torch.nn.functional as F
 
 from typing import NamedTuple
 
+from ._lib import native
 from .dense import Dense, autocast_dtype, dense_group
 from .functional import (deltanet, gated_linear_attention, linear_attention, linear_scan, mingru_scan, mlstm_gates,
-                         normalised_linear_attention, layer_norm, layer_norm_fork, rms_norm, rms_norm_fork, silu_gate)
+                         normalised_linear_attention, layer_norm, layer_norm_fork, rms_norm, rms_norm_fork, silu_gate,
+                         stepping_in_place)
 from .kernels import RMS_NORM_MAX_D as _RMS_NORM_MAX_D
 
 
@@ -75,6 +77,10 @@ class MemoroidCellBase(nn.Module):
 
     def initialize_carry(self, key, input_shape):
         raise NotImplementedError
+
+    def whole(self, x, done, initial_carry):
+        """read(scan(self(x))) as one operation, (next_carry, y), where a cell has it for these arrays; else None."""
+        return None
 
     def scan(self, z, initial_carry, done):
         """Reset-aware inclusive scan of the cell's algebra over time, carry-in
@@ -147,6 +153,9 @@ class Memoroid(SequenceModel):
     def forward(self, inputs, done, initial_carry=None, **kwargs):
         if initial_carry is None:
             initial_carry = self.cell.initialize_carry(None, get_input_shape(inputs))
+        whole = self.cell.whole(inputs, done, initial_carry)
+        if whole is not None:
+            return whole
         z = self.cell(inputs, **kwargs)
         h, next_carry = self.cell.scan(z, initial_carry, done)
         y = self.cell.read(h, inputs, **kwargs)
@@ -604,6 +613,22 @@ class MambaCell(MemoroidCellBase):
         carry = (S_last.transpose(-1, -2)[:, None], torch.exp(G_last)[:, None, :, None, None])
         return o, carry
 
+    def whole(self, x, done, initial_carry):
+        """Elements, recurrence and gated read-out in one native operation (conv_cells.hip around the gated kernels): float32
+        on the device, sizes the kernels take as they are.  The composition below -- projections formed in ``forward`` and
+        again in ``read``, the library's convolution between transposes -- takes ten times as long."""
+        P, N = self.head_dim, self.state_dim
+        if not (x.is_cuda and x.dtype == torch.float32 and x.dim() == 3 and x.shape[0] * x.shape[1] > 0 and autocast_dtype(x) is None
+                and self.conv.weight.dtype == torch.float32 and P % 4 == 0 and P <= 64 and N in (4, 8, 16, 32, 64)
+                and self.conv_dim <= 4 and self.num_heads * P <= _RMS_NORM_MAX_D):
+            return None
+        h0, decay0 = initial_carry
+        up, b_in, c_in, dt_in = dense_group(x, [self.input_projection, self.B, self.C, self.dt])
+        y, S_last, decay = native().mamba_mix(up, b_in, c_in, dt_in, self.conv.weight, self.conv.bias, self.dt_bias, self.A_log, self.D,
+                                              self.norm.scale, done, h0[:, 0].transpose(-1, -2), decay0[:, 0, :, 0, 0], self.norm.eps,
+                                              stepping_in_place())
+        return (S_last.transpose(-1, -2)[:, None], decay[:, None, :, None, None]), self.output_projection(y)
+
     def read(self, o, x, **kwargs):
         Bn, T, _ = x.shape
         hidden, _, _, z, _ = self._project(x)
@@ -613,8 +638,8 @@ class MambaCell(MemoroidCellBase):
 
     def initialize_carry(self, key, input_shape):
         *batch, _ = input_shape
-        dev = self.A_log.device
-        return (torch.zeros(*batch, 1, self.num_heads, self.state_dim, self.head_dim, device=dev),
+        dev = self.A_log.device   # (N, P) in shape, laid out as the kernels hold it: (P, N)
+        return (torch.zeros(*batch, 1, self.num_heads, self.head_dim, self.state_dim, device=dev).transpose(-1, -2),
                 torch.ones(*batch, 1, self.num_heads, 1, 1, device=dev))
 
 

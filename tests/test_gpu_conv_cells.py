@@ -1,0 +1,68 @@
+"""The Mamba cell as one operation (MambaCell.whole: conv_cells.hip around the gated kernels) against the cell's own
+composition of array operations -- elements, scan, read -- in values, carry and every gradient, where the passes can go
+wrong: lengths around the time tiles and the convolution's width, channel counts around the 256-channel tiles."""
+import pytest
+import torch
+
+from gpu_util import relerr
+
+pytestmark = pytest.mark.gpu
+
+
+def _np(t):
+    return t.detach().cpu().numpy()
+
+
+def _step(cell, x, done, carry, gy, gc, whole):
+    leaves = [x, *carry, *cell.parameters()]
+    for t in leaves:
+        t.grad = None
+    if whole:
+        out = cell.whole(x, done, carry)
+        assert out is not None
+        nxt, y = out
+    else:
+        h, nxt = cell.scan(cell(x), carry, done)
+        y = cell.read(h, x)
+    loss = (y * gy).sum() + sum((c * g).sum() for c, g in zip(nxt, gc))
+    loss.backward()
+    return [y, *nxt], [t.grad.clone() for t in leaves]
+
+
+@pytest.mark.parametrize("B,T,H,P,N,K", [
+    (2, 1, 2, 64, 64, 4), (1, 2, 1, 16, 4, 4), (3, 3, 2, 16, 16, 3), (2, 31, 3, 48, 32, 2), (2, 33, 4, 64, 16, 1), (1, 130, 8, 64, 64, 4),
+    (5, 65, 5, 52, 64, 4), (70, 34, 2, 32, 32, 4)])
+def test_mamba_cell_whole_equals_its_composition(B, T, H, P, N, K):
+    from memorax_amd import sequence_models as sm
+    torch.manual_seed(T)
+    Fe = 24
+    cell = sm.MambaCell(Fe, num_heads=H, head_dim=P, state_dim=N, conv_dim=K).cuda()
+    g = torch.Generator(device="cuda").manual_seed(B)
+    rand = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    x = rand(B, T, Fe).requires_grad_()
+    done = torch.rand(B, T, device="cuda", generator=g) < 0.05
+    carry = [rand(B, 1, H, N, P).requires_grad_(), torch.rand(B, 1, H, 1, 1, device="cuda", generator=g).requires_grad_()]
+    gy, gc = rand(B, T, Fe), [rand(B, 1, H, N, P) * 0.1, rand(B, 1, H, 1, 1)]
+    print(f"case mamba {B} {T} {H} {P} {N} {K}", flush=True)
+    outs, grads = _step(cell, x, done, carry, gy, gc, True)
+    ref_outs, ref_grads = _step(cell, x, done, carry, gy, gc, False)
+    names = ["y", "S", "decay"] + ["dx", "dS0", "ddecay0"] + [n for n, _ in cell.named_parameters()]
+    for n, a, b in zip(names, outs + grads, ref_outs + ref_grads):
+        assert a.shape == b.shape, n
+        assert relerr(a, _np(b)) <= 2e-4, (n, relerr(a, _np(b)))
+
+
+def test_mamba_cell_acting_equals_its_composition():
+    from memorax_amd import sequence_models as sm
+    torch.manual_seed(3)
+    B, Fe, H, d = 37, 32, 2, 32
+    cell = sm.MambaCell(Fe, num_heads=H, head_dim=d, state_dim=d).cuda()
+    carry = ref = cell.initialize_carry(None, (B, Fe))
+    with torch.no_grad():
+        for t in range(4):
+            x, done = torch.randn(B, 1, Fe, device="cuda"), torch.rand(B, 1, device="cuda") < 0.2
+            carry, y = sm.Memoroid(cell)(x, done, carry)
+            h, ref = cell.scan(cell(x), ref, done)
+            assert relerr(y, _np(cell.read(h, x))) <= 1e-4
+            for a, b in zip(carry, ref):
+                assert a.shape == b.shape and relerr(a, _np(b)) <= 1e-4
