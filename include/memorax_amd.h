@@ -529,6 +529,38 @@ int mrx_delta_rule_step(void *stream, const void *q, const void *k,
                         int64_t H, int64_t dk, int64_t dv, int dtype,
                         int done_dtype);
 
+/* The same with the DeltaNet cell's prologue: k and beta_raw are the raw projections, k / max(|k|, 1e-12) and
+ * sigmoid(beta_raw) are formed in the kernel (the T = 1 case of mrx_deltanet_fwd). */
+int mrx_deltanet_step(void *stream, const void *q, const void *k,
+                      const void *v, const void *beta_raw, const void *done,
+                      const float *S_in, void *o, float *S_out, int64_t B,
+                      int64_t H, int64_t dk, int64_t dv, int dtype,
+                      int done_dtype);
+
+/* MinGRU (min_gru.py:49-90), carry in the cell's log-space leaves, with the gated read-out of the block around it:
+ *     h = (done ? 0 : sigma(-z) exp(log_state)) + sigma(z) g(h~) ;  log_state' = log h
+ *     log_decay' = (done ? 0 : log_decay) + log sigma(-z) ;  y = h * silu(gate)   (gate NULL: y = h)
+ * z, h_tilde, gate, y: (B,D) in `dtype`, MRX_F32 or MRX_BF16; the carry's leaves: (B,D) fp32, updated in place where
+ * the outputs are the inputs; done: (B,). */
+int mrx_mingru_step(void *stream, const void *z, const void *h_tilde, const void *gate, const void *done,
+                    const float *log_state, const float *log_decay, void *y, float *log_state_out,
+                    float *log_decay_out, int64_t B, int64_t D, int dtype, int done_dtype);
+
+/* ---- Dense layers on few rows (acting) -----------------------------------------
+ * Up to MRX_ROW_DENSE_LAYERS dense layers that read the same rows, the norm before them and the residual addition behind
+ * them in one launch (blocks/normalization.py:30-31, residual.py:23-26 around the cells' flax.linen.Dense layers):
+ *     y_l = norm(x) W_l^T + b_l ,  or  y_0 = residual + (norm(x) W_0^T + b_0)  with residual given (one layer, y float32)
+ * x: (rows,K) in x_dtype; norm: 0 none, 1 RMS norm (scale), 2 layer norm (scale, norm_bias), over K with eps; W_l: (n_out[l],K)
+ * in w_dtype; b_l: (n_out[l]) in b_dtype or NULL; y_l: (rows,n_out[l]) in y_dtype.  product_dtype: MRX_BF16 rounds the
+ * normalised rows, weights, biases and results to bfloat16 (float32 sums), MRX_F32 multiplies in float32; round_norm: the
+ * normalised rows pass through bfloat16 in either case.  weights, biases, outs, n_out: HOST arrays of `layers` entries.
+ * K a multiple of 8, at most 2048; x, W and the norm's vectors 16-byte aligned. */
+#define MRX_ROW_DENSE_LAYERS 4
+int mrx_row_dense(void *stream, const void *x, const float *scale, const float *norm_bias, int norm, int round_norm,
+                  const void *const *weights, const void *const *biases, void *const *outs, const int64_t *n_out,
+                  int layers, const float *residual, int64_t rows, int64_t K, int x_dtype, int w_dtype, int b_dtype,
+                  int y_dtype, int product_dtype, float eps);
+
 #ifdef __cplusplus
 }
 #endif

@@ -46,7 +46,7 @@ using torch::autograd::variable_list;
     X(mrx_delta_rule_fwd_noalloc) X(mrx_deltanet_fwd) X(mrx_deltanet_bwd) X(mrx_linear_attn_step)                    \
     X(mrx_gated_linear_attn_step) X(mrx_delta_rule_step) X(mrx_causal_conv_silu_fwd) X(mrx_causal_conv_silu_bwd)     \
     X(mrx_mamba_elements_fwd) X(mrx_mamba_elements_bwd) X(mrx_decay_last) X(mrx_mamba_readout_fwd)                   \
-    X(mrx_mamba_readout_bwd)
+    X(mrx_mamba_readout_bwd) X(mrx_deltanet_step) X(mrx_mingru_step) X(mrx_row_dense)
 struct {
 #define MRX_MEMBER(name) decltype(&::name) name = nullptr;
     MRX_BOUND(MRX_MEMBER)
@@ -676,18 +676,81 @@ StepOut gated_linear_attn_step(const Tensor &q, const Tensor &k, const Tensor &v
     return r;
 }
 
+// prologue: k and beta are the raw projections of the DeltaNet cell
 StepOut delta_rule_step(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &beta, const Tensor &done_, const OptTensor &S,
-                        bool inplace)
+                        bool inplace, bool prologue)
 {
     const StepShape s(q, k, v);
     chk(beta, "beta", s.dt, {s.B, s.H});
     chk(S, "S", at::kFloat, s.state());
     const Done done(done_.reshape({s.B, 1}), s.B, 1);
     StepOut r{fresh_like(v), s.next(S, inplace, q), {}};
-    check(lib.mrx_delta_rule_step(stream(), ptr(q), ptr(k), ptr(v), ptr(beta), done.p(), fptr(S), ptr(r.o), fptr(r.S), s.B, s.H, s.dk, s.dv,
-                                  code(s.dt), done.dtype),
-          "mrx_delta_rule_step");
+    check((prologue ? lib.mrx_deltanet_step : lib.mrx_delta_rule_step)(stream(), ptr(q), ptr(k), ptr(v), ptr(beta), done.p(), fptr(S), ptr(r.o),
+                                                                       fptr(r.S), s.B, s.H, s.dk, s.dv, code(s.dt), done.dtype),
+          prologue ? "mrx_deltanet_step" : "mrx_delta_rule_step");
     return r;
+}
+
+// ---- acting: dense layers on few rows, the MinGRU cell's step
+// norm: 0 none, 1 RMS, 2 layer norm.  The results keep x's leading axes; residual (float32, x's leading axes): added to the one
+// layer's result.
+std::vector<Tensor> row_dense(const Tensor &x, int norm, const OptTensor &scale, const OptTensor &nbias, double eps, bool round_norm,
+                              const std::vector<Tensor> &weights, const std::vector<OptTensor> &biases, ScalarType product, ScalarType out_dtype,
+                              const OptTensor &residual)
+{
+    TORCH_CHECK_VALUE(x.dim() >= 2 && !weights.empty() && weights.size() <= MRX_ROW_DENSE_LAYERS && biases.size() == weights.size(),
+                      "row_dense takes rows and 1 to ", MRX_ROW_DENSE_LAYERS, " layers");
+    const int64_t K = x.size(-1), rows = x.numel() / K;
+    chk(x, "x");
+    chk(scale, "scale", at::kFloat, {K});
+    chk(nbias, "bias of the norm", at::kFloat, {K});
+    const auto wd = weights[0].scalar_type();
+    auto bd = at::kFloat;
+    std::array<const void *, MRX_ROW_DENSE_LAYERS> w{}, b{};
+    std::array<void *, MRX_ROW_DENSE_LAYERS> y{};
+    std::array<int64_t, MRX_ROW_DENSE_LAYERS> n{};
+    std::vector<Tensor> out;
+    out.reserve(weights.size());
+    c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
+    bool first_bias = true;
+    for (size_t l = 0; l < weights.size(); ++l) {
+        n[l] = weights[l].size(0);
+        chk(weights[l], "weight", wd, {n[l], K});
+        if (biases[l].has_value()) {
+            if (std::exchange(first_bias, false)) bd = biases[l]->scalar_type();
+            chk(*biases[l], "bias", bd, {n[l]});
+        }
+        shape.back() = n[l];
+        out.push_back(fresh(shape, out_dtype, x));
+        w[l] = ptr(weights[l]), b[l] = ptr(biases[l]), y[l] = ptr(out[l]);
+    }
+    chk(residual, "residual", at::kFloat, out[0].sizes());
+    check(lib.mrx_row_dense(stream(), ptr(x), fptr(scale), fptr(nbias), norm, round_norm, w.data(), b.data(), y.data(), n.data(),
+                            (int)weights.size(), fptr(residual), rows, K, code(x.scalar_type()), code(wd), code(bd), code(out_dtype),
+                            code(product), (float)eps),
+          "mrx_row_dense");
+    return out;
+}
+
+// z, h~, gate (B,1,D), done (B,1), the carry's leaves (B,1,D) float32 -> y, log_state, log_decay
+std::tuple<Tensor, Tensor, Tensor> mingru_step(const Tensor &z, const Tensor &x, const OptTensor &gate, const Tensor &done_,
+                                               const Tensor &log_state, const Tensor &log_decay, bool in_place)
+{
+    TORCH_CHECK_VALUE(z.dim() == 3 && z.size(1) == 1, "mingru_step takes one time step");
+    const int64_t B = z.size(0), D = z.size(2);
+    const auto dt = z.scalar_type();
+    chk_scan_dtype(dt, false, "mingru_step");
+    chk(z, "z");
+    chk(x, "h_tilde", dt, z.sizes());
+    chk(gate, "gate", dt, z.sizes());
+    chk(log_state, "log_state", at::kFloat, z.sizes());
+    chk(log_decay, "log_decay", at::kFloat, z.sizes());
+    const Done done(done_, B, 1);
+    const Tensor y = fresh_like(z), ls = in_place ? log_state : fresh_like(log_state), ld = in_place ? log_decay : fresh_like(log_decay);
+    check(lib.mrx_mingru_step(stream(), ptr(z), ptr(x), ptr(gate), done.p(), fptr(log_state), fptr(log_decay), ptr(y), fptr(ls), fptr(ld), B, D,
+                              code(dt), done.dtype),
+          "mrx_mingru_step");
+    return {y, ls, ld};
 }
 
 // ------------------------------------------------------------------------------------------------ autograd nodes
@@ -987,14 +1050,8 @@ std::tuple<Tensor, Tensor> delta_rule(const Tensor &q, const Tensor &k, const Te
         q_ = q.contiguous(), k_ = k.contiguous(), v_ = v.contiguous(), b_ = beta.contiguous();
         const Tensor S0_ = as(unwrap(S0), at::kFloat);
         if (q_.size(1) == 1 && !need) {
-            Tensor k1 = k_.select(1, 0), b1 = b_.select(1, 0);
-            if (prologue) {   // a (B,H,d) array: the prologue as array operations costs nothing here
-                const Tensor kf = k1.to(at::kFloat);
-                k1 = kf.div(kf.norm(2, {-1}, true).clamp_min(1e-12)).to(k_.scalar_type());
-                b1 = b1.to(at::kFloat).sigmoid().to(b_.scalar_type());
-            }
-            auto st = delta_rule_step(q_.select(1, 0), k1, v_.select(1, 0), b1, done.select(1, 0), some(S0_),
-                                      in_place && S0.has_value() && S0_.is_same(*S0));
+            auto st = delta_rule_step(q_.select(1, 0), k_.select(1, 0), v_.select(1, 0), b_.select(1, 0), done.select(1, 0), some(S0_),
+                                      in_place && S0.has_value() && S0_.is_same(*S0), prologue);
             return {st.o.unsqueeze(1), st.S};
         }
         r = delta_rule_fwd(q_, k_, v_, b_, done, some(S0_), need, std::nullopt, prologue, std::nullopt, MRX_FACTORS_AUTO, resets);
@@ -1330,9 +1387,11 @@ PYBIND11_MODULE(_native, m)
     });
     def("delta_rule_step", [](const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &beta, const Tensor &done, const OptTensor &S,
                                 bool inplace) {
-        auto r = delta_rule_step(q, k, v, beta, done, S, inplace);
+        auto r = delta_rule_step(q, k, v, beta, done, S, inplace, false);
         return std::make_tuple(r.o, r.S);
     });
+    def("row_dense", &row_dense);
+    def("mingru_step", &mingru_step);
     // differentiable operators (memorax_amd/functional.py)
     def("linear_scan", &linear_scan);
     def("mingru_scan", &mingru_scan);

@@ -1300,3 +1300,66 @@ extern "C" int mrx_mingru_scan_bwd(void *stream, const void *z, const void *h_ti
     return launch_bwd<float, true>((hipStream_t)stream, z, h_tilde, h, done, done_dtype, h0, g, g_last, dz, dh_tilde,
                                    dh0, B, T, D, 0);
 }
+
+namespace {
+
+// One acting step of the MinGRU cell with its carry in the reference's log-space leaves, and the gated read-out of the
+// block around it: exp of the carried state, the element map, the update, its logarithm and the product with silu(gate) are
+// one pass over (B,D) arrays of a few hundred kilobytes -- eight launches as separate operations.
+template <typename S, int VEC>
+__global__ void __launch_bounds__(256) mingru_step_kernel(const S *__restrict__ z, const S *__restrict__ x, const S *__restrict__ gate,
+                                                          const void *__restrict__ done, int done_f32, const float *log_state,
+                                                          const float *log_decay, S *__restrict__ y, float *log_state_out,
+                                                          float *log_decay_out, int64_t n, int64_t D)  // the carry may be updated in place
+{
+    const int64_t at = ((int64_t)blockIdx.x * 256 + threadIdx.x) * VEC;
+    if (at >= n) return;
+    const bool reset = done_at(done, done_f32, at / D);
+    const Vec<float, VEC> zv = cvtv<S, float, VEC>(ldraw<S, VEC>(z + at)), xv = cvtv<S, float, VEC>(ldraw<S, VEC>(x + at));
+    Vec<float, VEC> gv = vfill<float, VEC>(0.f), ls = *reinterpret_cast<const Vec<float, VEC> *>(log_state + at),
+                    ld = *reinterpret_cast<const Vec<float, VEC> *>(log_decay + at), out;
+    if (gate) gv = cvtv<S, float, VEC>(ldraw<S, VEC>(gate + at));
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+        float a = zv.v[i], b = xv.v[i];
+        const float log_a = -(fmaxf(a, 0.f) + log1pf(expf(-fabsf(a))));   // log sigma(-z)
+        MinGru::coeffs(a, b);
+        const float h = reset ? b : a * expf(ls.v[i]) + b;
+        ls.v[i] = logf(h);
+        ld.v[i] = reset ? log_a : ld.v[i] + log_a;
+        const float hs = (float)(S)h, g = gv.v[i];   // the state as the cell hands it on
+        out.v[i] = gate ? hs * g / (1.f + __expf(-g)) : hs;
+    }
+    *reinterpret_cast<Vec<float, VEC> *>(log_state_out + at) = ls;
+    *reinterpret_cast<Vec<float, VEC> *>(log_decay_out + at) = ld;
+    stv<S, float, VEC>(y + at, out);
+}
+
+}  // namespace
+
+extern "C" int mrx_mingru_step(void *stream, const void *z, const void *h_tilde, const void *gate, const void *done, const float *log_state,
+                               const float *log_decay, void *y, float *log_state_out, float *log_decay_out, int64_t B, int64_t D, int dtype,
+                               int done_dtype)
+{
+    if (!z || !h_tilde || !done || !log_state || !log_decay || !y || !log_state_out || !log_decay_out || B <= 0 || D <= 0)
+        return MRX_ERR_INVALID_ARG;
+    if ((dtype != MRX_F32 && dtype != MRX_BF16) || (done_dtype != MRX_DONE_U8 && done_dtype != MRX_DONE_F32)) return MRX_ERR_INVALID_ARG;
+    if (B >= (1ll << 31) || D >= (1ll << 31)) return MRX_ERR_INVALID_ARG;
+    if (const int rc = prepare_device(); rc != MRX_OK) return rc;
+    bool quads = D % 4 == 0;   // rows of whole quads, every array on a 16-byte boundary
+    for (const void *p : {z, h_tilde, gate, (const void *)log_state, (const void *)log_decay, (const void *)y, (const void *)log_state_out,
+                          (const void *)log_decay_out})
+        quads = quads && aligned(p, 16);
+    const int64_t n = B * D, wgs = (n / (quads ? 4 : 1) + 255) / 256;
+    if (wgs >= (1ll << 31)) return MRX_ERR_INVALID_ARG;
+    auto go = [&](auto s, auto vec) {
+        using S = decltype(s);
+        return launch_kernel(mingru_step_kernel<S, decltype(vec)::value>, dim3((unsigned)wgs), dim3(256), 0, (hipStream_t)stream,
+                             (const S *)z, (const S *)h_tilde, (const S *)gate, done, int(done_dtype == MRX_DONE_F32), log_state, log_decay,
+                             (S *)y, log_state_out, log_decay_out, n, D);
+    };
+    using One = std::integral_constant<int, 1>;
+    using Four = std::integral_constant<int, 4>;
+    if (dtype == MRX_BF16) return quads ? go(__bf16(), Four{}) : go(__bf16(), One{});
+    return quads ? go(float(), Four{}) : go(float(), One{});
+}

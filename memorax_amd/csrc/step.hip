@@ -54,7 +54,9 @@ __device__ __forceinline__ float dot4(const f32x4 &a, const f32x4 &b)
 
 // NARROW: narrow heads -- q, k, z are dka wide, v, o dva, the state
 // [dva][dka]; lanes and rows beyond take no part.
-template <typename T, bool DELTA, bool FMAP, bool NARROW = false>
+// PRO (delta rule): k and beta are the raw projections, k / max(|k|, 1e-12) and sigmoid(beta) are formed here, rounded to T as
+// a caller-side prologue would store them.
+template <typename T, bool DELTA, bool FMAP, bool NARROW = false, bool PRO = false>
 __global__ void __launch_bounds__(256)
 step_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restrict__ v,
             const T *__restrict__ beta, const float *__restrict__ glog, const void *__restrict__ done, int done_f32,
@@ -78,6 +80,11 @@ step_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restric
             q4[e] = elu1(q4[e]);
         }
     }
+    if (PRO) {
+        const float inv = 1.f / fmaxf(sqrtf(reduce_row(dot4(k4, k4))), 1e-12f);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) k4[e] = (float)(T)(k4[e] * inv);
+    }
     const float *Sp = S_in ? S_in + bh * dvw * dkw : nullptr;
     const float decay = (!DELTA && glog) ? __expf(glog[bh]) : 1.f;  // gated linear attention: the carried state decays first
     f32x4 s[NP];
@@ -94,7 +101,8 @@ step_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restric
 #pragma unroll
     for (int p = 0; p < NP; ++p) s[p] = reset ? zero4 : s[p] * decay;
     if (DELTA) {
-        const float bb = (float)beta[bh];
+        float bb = (float)beta[bh];
+        if (PRO) bb = (float)(T)(1.f / (1.f + __expf(-bb)));
 #pragma unroll
         for (int p = 0; p < NP; ++p) u[p] = bb * (u[p] - reduce_row(dot4(s[p], k4)));
     }
@@ -142,13 +150,13 @@ int check_step(const void *q, const void *k, const void *v, const void *done, co
     return MRX_OK;
 }
 
-template <typename T, bool DELTA, bool FMAP>
+template <typename T, bool DELTA, bool FMAP, bool PRO = false>
 int launch_step(hipStream_t st, const void *q, const void *k, const void *v, const void *beta, const void *done,
                 int done_f32, const float *S_in, const float *z_in, void *o, float *S_out, float *z_out,
                 int64_t B, int64_t H, float eps, int64_t dka = HD, int64_t dva = HD, const float *glog = nullptr)
 {
     auto go = [&](auto narrow) {
-        return launch_kernel((step_kernel<T, DELTA, FMAP, decltype(narrow)::value>), dim3((unsigned)(B * H)), dim3(256), 0, st,
+        return launch_kernel((step_kernel<T, DELTA, FMAP, decltype(narrow)::value, PRO>), dim3((unsigned)(B * H)), dim3(256), 0, st,
                              (const T *)q, (const T *)k, (const T *)v, (const T *)beta, glog, done, done_f32, S_in, z_in,
                              (T *)o, S_out, z_out, (int)H, eps, (int)dka, (int)dva);
     };
@@ -201,6 +209,24 @@ MRX_EXPORT int MRX_API(mrx_gated_linear_attn_step)(void *stream, const void *q, 
 #undef MRX_ARGS
 }
 
+namespace {
+inline namespace MRX_HD_NS {
+template <bool PRO>
+int delta_step(void *stream, const void *q, const void *k, const void *v, const void *beta, const void *done, const float *S_in, void *o,
+               float *S_out, int64_t B, int64_t H, int64_t dk, int64_t dv, int dtype, int done_dtype)
+{
+    const int rc = check_step(q, k, v, done, S_in, o, S_out, B, H, dk, dv, dtype, done_dtype, true);
+    if (rc != MRX_OK) return rc;
+    if (!beta) return MRX_ERR_INVALID_ARG;
+    hipStream_t st = (hipStream_t)stream;
+    const int df = done_dtype == MRX_DONE_F32;
+    if (dtype == MRX_BF16)
+        return launch_step<__bf16, true, false, PRO>(st, q, k, v, beta, done, df, S_in, nullptr, o, S_out, nullptr, B, H, 0.f, dk, dv);
+    return launch_step<float, true, false, PRO>(st, q, k, v, beta, done, df, S_in, nullptr, o, S_out, nullptr, B, H, 0.f, dk, dv);
+}
+}  // namespace MRX_HD_NS
+}  // namespace
+
 MRX_EXPORT int MRX_API(mrx_delta_rule_step)(void *stream, const void *q, const void *k, const void *v, const void *beta,
                                    const void *done, const float *S_in, void *o, float *S_out, int64_t B,
                                    int64_t H, int64_t dk, int64_t dv, int dtype, int done_dtype)
@@ -208,12 +234,15 @@ MRX_EXPORT int MRX_API(mrx_delta_rule_step)(void *stream, const void *q, const v
 #if MRX_HD == 64
     if (dk <= 32 && dv <= 32) return mrx_delta_rule_step_hd32(stream, q, k, v, beta, done, S_in, o, S_out, B, H, dk, dv, dtype, done_dtype);
 #endif
-    const int rc = check_step(q, k, v, done, S_in, o, S_out, B, H, dk, dv, dtype, done_dtype, true);
-    if (rc != MRX_OK) return rc;
-    if (!beta) return MRX_ERR_INVALID_ARG;
-    hipStream_t st = (hipStream_t)stream;
-    const int df = done_dtype == MRX_DONE_F32;
-    if (dtype == MRX_BF16)
-        return launch_step<__bf16, true, false>(st, q, k, v, beta, done, df, S_in, nullptr, o, S_out, nullptr, B, H, 0.f, dk, dv);
-    return launch_step<float, true, false>(st, q, k, v, beta, done, df, S_in, nullptr, o, S_out, nullptr, B, H, 0.f, dk, dv);
+    return delta_step<false>(stream, q, k, v, beta, done, S_in, o, S_out, B, H, dk, dv, dtype, done_dtype);
+}
+
+MRX_EXPORT int MRX_API(mrx_deltanet_step)(void *stream, const void *q, const void *k, const void *v, const void *beta_raw,
+                                 const void *done, const float *S_in, void *o, float *S_out, int64_t B,
+                                 int64_t H, int64_t dk, int64_t dv, int dtype, int done_dtype)
+{
+#if MRX_HD == 64
+    if (dk <= 32 && dv <= 32) return mrx_deltanet_step_hd32(stream, q, k, v, beta_raw, done, S_in, o, S_out, B, H, dk, dv, dtype, done_dtype);
+#endif
+    return delta_step<true>(stream, q, k, v, beta_raw, done, S_in, o, S_out, B, H, dk, dv, dtype, done_dtype);
 }

@@ -62,6 +62,10 @@ class SequenceModel(nn.Module):
     def initialize_carry(self, key, input_shape):  # pragma: no cover
         raise NotImplementedError
 
+    def acting(self, x, norm, done, carry):
+        """The pre-norm residual block around this model for one acting step; see MemoroidCellBase.acting."""
+        return None
+
 
 class MemoroidCellBase(nn.Module):
     """memoroid.py:20-33 plus the kernel hook ``scan``."""
@@ -80,6 +84,11 @@ class MemoroidCellBase(nn.Module):
 
     def whole(self, x, done, initial_carry):
         """read(scan(self(x))) as one operation, (next_carry, y), where a cell has it for these arrays; else None."""
+        return None
+
+    def acting(self, x, norm, done, carry):
+        """(next_carry, x + read(scan(self(norm(x))))) for one time step without gradients (``_acts``), where a cell has its
+        launches fused for these arrays; else None."""
         return None
 
     def scan(self, z, initial_carry, done):
@@ -160,6 +169,9 @@ class Memoroid(SequenceModel):
         h, next_carry = self.cell.scan(z, initial_carry, done)
         y = self.cell.read(h, inputs, **kwargs)
         return next_carry, y
+
+    def acting(self, x, norm, done, carry):
+        return self.cell.acting(x, norm, done, self.cell.initialize_carry(None, get_input_shape(x)) if carry is None else carry)
 
     def initialize_carry(self, key, input_shape):
         return self.cell.initialize_carry(key, input_shape)
@@ -396,8 +408,55 @@ class GatedLinearRecurrence(SequenceModel):
         h, next_carry = self.cell.scan(self.cell.elements(z, h_tilde), initial_carry, done)
         return next_carry, self.out(_gated(h[0], gate))
 
+    def acting(self, x, norm, done, carry):
+        layers = [self.cell.z, self.cell.h, self.gate]
+        if not (type(self).forward is GatedLinearRecurrence.forward and self.cell.fused and _row_layers(x, [*layers, self.out])):
+            return None
+        if carry is None:
+            carry = self.cell.initialize_carry(None, get_input_shape(x))
+        product = autocast_dtype(x) or x.dtype
+        z, h_tilde, gate = _rows(x, norm, layers, product, product)
+        self.cell.intermediates.sow("gate", lambda z=z: z.float().mean())
+        y, *carry = native().mingru_step(z, h_tilde, gate, done, *carry, stepping_in_place())
+        return tuple(carry), _rows(y, None, [self.out], product, x.dtype, x)[0]
+
     def initialize_carry(self, key, input_shape):
         return self.cell.initialize_carry(key, input_shape)
+
+
+# ----------------------------------------------------------------------------------
+# acting: one time step without gradients (ppo.py:105-143), rows = environments
+# ----------------------------------------------------------------------------------
+_ACTING_ROWS = 4096   # up to here a row-dense launch beats the array library's products and what surrounds them
+
+
+def _acts(x, done, norm):
+    """Whether a pre-norm residual block on ``x`` is an acting step that the row kernels take."""
+    return (not torch.is_grad_enabled() and x.dim() == 3 and x.shape[1] == 1 and 0 < x.shape[0] <= _ACTING_ROWS and x.is_cuda
+            and x.dtype == torch.float32 and x.shape[2] % 8 == 0 and x.is_contiguous() and autocast_dtype(x) in (None, torch.bfloat16)
+            and (type(norm) is _RMSNorm or (type(norm) is _LayerNorm and norm.elementwise_affine)))
+
+
+def _row_layers(x, layers):
+    """Whether the row kernels multiply with these layers' weights as they are (under autocast: whatever dtype the products run in)."""
+    wd = layers[0].weight.dtype
+    plain = (torch.float32,) if autocast_dtype(x) is None else (torch.float32, torch.bfloat16)
+    return wd in plain and all(m.weight.dtype == wd and m.weight.shape[1] % 8 == 0 and m.weight.shape[1] <= _RMS_NORM_MAX_D
+                               and (m.bias is None or m.bias.dtype in (torch.float32, torch.bfloat16)) for m in layers)
+
+
+def _rows(x, norm, layers, product, out_dtype, residual=None):
+    """norm(x) through the layers in one launch, as _RMSNorm / _LayerNorm / Dense would compute it; residual: added to the one result."""
+    rms = type(norm) is _RMSNorm
+    kind = 0 if norm is None else 1 if rms else 2
+    scale = None if norm is None else norm.scale if rms else norm.weight
+    return native().row_dense(x, kind, scale, None if norm is None or rms else norm.bias, 0.0 if norm is None else norm.eps,
+                              x.dtype == torch.bfloat16, [m.weight for m in layers], [m.bias for m in layers], product, out_dtype, residual)
+
+
+def _as_written(cell, cls):
+    """A subclass that overrides what the whole-cell operations stand for runs its own composition."""
+    return type(cell) is cls or all(getattr(type(cell), n) is getattr(cls, n) for n in ("forward", "scan", "read"))
 
 
 # ----------------------------------------------------------------------------------
@@ -483,6 +542,15 @@ class LinearAttentionCell(MemoroidCellBase):
         1024 x 128 x 4 x 64.)"""
         return self.output_projection(self.norm(h.reshape(*x.shape[:2], -1)).to(x.dtype))
 
+    def acting(self, x, norm, done, carry):
+        layers = [self.value, self.key, self.query]
+        if not (_as_written(self, LinearAttentionCell) and _row_layers(x, [*layers, self.output_projection])):
+            return None
+        product = autocast_dtype(x) or x.dtype
+        z = tuple(self._heads(t) for t in _rows(x, norm, layers, product, product))
+        h, carry = self.scan(z, carry, done)
+        return carry, _rows(h.reshape(*x.shape[:2], -1), self.norm, [self.output_projection], product, x.dtype, x)[0]
+
     def initialize_carry(self, key, input_shape):
         *batch, _ = input_shape
         dev = self.key.weight.device
@@ -540,6 +608,16 @@ class DeltaNetCell(MemoroidCellBase):
     def read(self, h, x, **kwargs):
         out = h.reshape(*x.shape[:2], -1)
         return self.output_projection(self.norm(out).to(x.dtype))
+
+    def acting(self, x, norm, done, carry):
+        layers = [self.query, self.key, self.value, self.beta]
+        if not (_as_written(self, DeltaNetCell) and self.dtype in (torch.float32, torch.bfloat16)
+                and _row_layers(x, [*layers, self.output_projection])):
+            return None
+        product = autocast_dtype(x) or x.dtype
+        q, k, v, beta = _rows(x, norm, layers, product, self.dtype)
+        h, carry = self.scan((self._heads(q), self._heads(k), self._heads(v), beta), carry, done)
+        return carry, _rows(h.reshape(*x.shape[:2], -1), self.norm, [self.output_projection], product, x.dtype, x)[0]
 
     def initialize_carry(self, key, input_shape):
         *batch, _ = input_shape
@@ -617,17 +695,30 @@ class MambaCell(MemoroidCellBase):
         """Elements, recurrence and gated read-out in one native operation (conv_cells.hip around the gated kernels): float32
         on the device, sizes the kernels take as they are.  The composition below -- projections formed in ``forward`` and
         again in ``read``, the library's convolution between transposes -- takes ten times as long."""
-        P, N = self.head_dim, self.state_dim
-        if not (x.is_cuda and x.dtype == torch.float32 and x.dim() == 3 and x.shape[0] * x.shape[1] > 0 and autocast_dtype(x) is None
-                and self.conv.weight.dtype == torch.float32 and P % 4 == 0 and P <= 64 and N in (4, 8, 16, 32, 64)
-                and self.conv_dim <= 4 and self.num_heads * P <= _RMS_NORM_MAX_D):
+        if not (self._native_sizes() and _as_written(self, MambaCell) and x.is_cuda and x.dtype == torch.float32 and x.dim() == 3 and x.shape[0] * x.shape[1] > 0 and autocast_dtype(x) is None):
             return None
-        h0, decay0 = initial_carry
-        up, b_in, c_in, dt_in = dense_group(x, [self.input_projection, self.B, self.C, self.dt])
-        y, S_last, decay = native().mamba_mix(up, b_in, c_in, dt_in, self.conv.weight, self.conv.bias, self.dt_bias, self.A_log, self.D,
+        y, carry = self._mix(dense_group(x, [self.input_projection, self.B, self.C, self.dt]), done, initial_carry)
+        return carry, self.output_projection(y)
+
+    def _native_sizes(self):
+        P = self.head_dim
+        return (P % 4 == 0 and P <= 64 and self.state_dim in (4, 8, 16, 32, 64) and self.conv_dim <= 4
+                and self.num_heads * P <= _RMS_NORM_MAX_D and self.conv.weight.dtype == torch.float32)
+
+    def _mix(self, projections, done, carry):
+        h0, decay0 = carry
+        y, S_last, decay = native().mamba_mix(*projections, self.conv.weight, self.conv.bias, self.dt_bias, self.A_log, self.D,
                                               self.norm.scale, done, h0[:, 0].transpose(-1, -2), decay0[:, 0, :, 0, 0], self.norm.eps,
                                               stepping_in_place())
-        return (S_last.transpose(-1, -2)[:, None], decay[:, None, :, None, None]), self.output_projection(y)
+        return y, (S_last.transpose(-1, -2)[:, None], decay[:, None, :, None, None])
+
+    def acting(self, x, norm, done, carry):
+        layers = [self.input_projection, self.B, self.C, self.dt]
+        if not (self._native_sizes() and _as_written(self, MambaCell) and autocast_dtype(x) is None
+                and _row_layers(x, [*layers, self.output_projection])):
+            return None
+        y, carry = self._mix(_rows(x, norm, layers, x.dtype, x.dtype), done, carry)
+        return carry, _rows(y, None, [self.output_projection], x.dtype, x.dtype, x)[0]
 
     def read(self, o, x, **kwargs):
         Bn, T, _ = x.shape
@@ -846,6 +937,10 @@ class Residual(nn.Module):
 
     def forward(self, inputs, done=None, initial_carry=None, **kwargs):
         inner = self.module
+        if type(inner) is PreNorm and not kwargs and hasattr(inner.module, "acting") and _acts(inputs, done, inner.norm):
+            acted = inner.module.acting(inputs, inner.norm, done, initial_carry)
+            if acted is not None:
+                return acted
         if isinstance(inner, PreNorm) and hasattr(inner.norm, "fork"):   # x + f(norm(x)): one kernel takes both gradients of x
             inputs, normed = inner.norm.fork(inputs)
             carry, y = inner.module(normed, done, initial_carry, **kwargs)

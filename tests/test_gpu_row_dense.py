@@ -1,0 +1,99 @@
+"""Dense layers on few rows with the norm before and the residual behind (mrx_row_dense), the MinGRU and DeltaNet acting steps,
+and the pre-norm residual blocks that act through them, against array operations."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from gpu_util import relerr
+
+pytestmark = pytest.mark.gpu
+BF, F32 = torch.bfloat16, torch.float32
+
+
+def _np(t):
+    return t.detach().float().cpu().numpy()
+
+
+@pytest.mark.parametrize("rows,K,ns", [
+    (1, 8, [1]), (15, 24, [3, 64]), (16, 256, [64, 63, 4]), (33, 264, [65]), (100, 520, [200, 5, 17, 128]), (513, 256, [256, 256, 256, 4]),
+    (2050, 512, [100]), (7, 1032, [40]), (4, 2048, [12])])
+@pytest.mark.parametrize("xd,wd,product,out", [(F32, F32, F32, F32), (F32, F32, BF, BF), (BF, BF, BF, BF), (F32, BF, BF, F32), (BF, F32, F32, BF)])
+@pytest.mark.parametrize("norm", [0, 1, 2])
+def test_row_dense_against_array_operations(rows, K, ns, xd, wd, product, out, norm):
+    from memorax_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(rows + K)
+    rand = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    x = rand(rows, 1, K).to(xd)
+    scale, nbias = rand(K), rand(K)
+    ws = [(rand(n, K) / K ** 0.5).to(wd) for n in ns]
+    bs = [rand(n) if i % 2 == 0 else None for i, n in enumerate(ns)]
+    residual = rand(rows, 1, ns[0]) if len(ns) == 1 else None
+    od = F32 if residual is not None else out
+    print(f"case rows {rows} {K} {ns} {xd} {wd} {product} {norm}", flush=True)
+    got = _lib.native().row_dense(x, norm, scale if norm else None, nbias if norm == 2 else None, 1e-6, xd == BF, ws, bs, product, od,
+                                  residual)
+    h = x.double()
+    if norm == 1:
+        h = h * torch.rsqrt(h.square().mean(-1, keepdim=True) + 1e-6) * scale.double()
+    elif norm == 2:
+        h = F.layer_norm(h, (K,), scale.double(), nbias.double(), 1e-6)
+    if product == BF or (norm and xd == BF):
+        h = h.float().to(BF)
+    for y, w, b in zip(got, ws, bs):
+        w, b = (w.to(BF), None if b is None else b.to(BF)) if product == BF else (w, b)
+        ref = F.linear(h.double(), w.double(), None if b is None else b.double())
+        if residual is not None:
+            ref = ref + residual.double()
+        assert y.dtype == od and y.shape == ref.shape
+        tol = 1e-5 if product == F32 and od == F32 and not (norm and xd == BF) else 2e-2
+        assert relerr(y, _np(ref)) <= tol, relerr(y, _np(ref))
+
+
+@pytest.mark.parametrize("B,D,dtype", [(1, 1, F32), (3, 5, F32), (70, 256, BF), (33, 12, F32), (5, 7, BF)])
+def test_mingru_step_against_the_scan(B, D, dtype):
+    from memorax_amd import _lib
+    from memorax_amd import functional as Fn
+    g = torch.Generator(device="cuda").manual_seed(B * D)
+    z, x, gate = (torch.randn(B, 1, D, device="cuda", generator=g).to(dtype) for _ in range(3))
+    done = torch.rand(B, 1, device="cuda", generator=g) < 0.3
+    ls, ld = torch.randn(B, 1, D, device="cuda", generator=g), -torch.rand(B, 1, D, device="cuda", generator=g)
+    if B > 1:
+        ls[1] = -float("inf")
+    h, h_last, P_last = Fn.mingru_scan(z, x, done, ls[:, 0].exp(), ld[:, 0].exp())
+    want = (h.float() * F.silu(gate.float())).to(dtype)
+    tol = 1e-5 if dtype == F32 else 1e-2
+    for in_place in (False, True):
+        a, b = ls.clone(), ld.clone()
+        y, s, d = _lib.native().mingru_step(z, x, gate, done, a, b, in_place)
+        assert (s.data_ptr() == a.data_ptr()) == in_place
+        assert relerr(y, _np(want)) <= tol
+        assert relerr(s[:, 0].exp(), _np(h_last)) <= 1e-5 and relerr(d[:, 0].exp(), _np(P_last)) <= 1e-5
+    y, _, _ = _lib.native().mingru_step(z, x, None, done, ls, ld, False)
+    assert relerr(y, _np(h)) <= tol
+
+
+@pytest.mark.parametrize("d", [16, 32, 64])
+@pytest.mark.parametrize("autocast", [False, True])
+def test_acting_blocks_equal_their_composition(d, autocast):
+    """With gradients enabled a block runs its composition; without, at T = 1, the fused acting step."""
+    from memorax_amd import sequence_models as sm
+    torch.manual_seed(d)
+    B, Fe, H = 37, 64, 2
+    cells = [sm.Memoroid(sm.DeltaNetCell(Fe, d, H)), sm.Memoroid(sm.DeltaNetCell(Fe, d, H, dtype=F32)), sm.GatedLinearRecurrence(Fe, 40),
+             sm.Memoroid(sm.LinearAttentionCell(Fe, d, H)), sm.Memoroid(sm.MambaCell(Fe, H, d, d))]
+    for cell in cells[:4] if autocast else cells:
+        for norm in (sm.RMSNorm, sm.LayerNorm):
+            block = sm.Residual(sm.PreNorm(cell, Fe, norm=norm)).cuda()
+            carry = ref = block.initialize_carry(None, (B, Fe))
+            for t in range(3):
+                x, done = torch.randn(B, 1, Fe, device="cuda"), torch.rand(B, 1, device="cuda") < 0.3
+                with torch.autocast("cuda", dtype=BF, enabled=autocast):
+                    ref, want = block(x, done, ref)
+                    with torch.no_grad():
+                        carry, y = block(x, done, carry)
+                tol = 2e-2 if autocast or isinstance(getattr(cell, "cell", None), sm.DeltaNetCell) else 1e-4
+                name = f"{type(cell).__name__} {type(getattr(cell, 'cell', cell)).__name__} {norm} {t}"
+                assert y.dtype == want.dtype and relerr(y, _np(want)) <= tol, (name, relerr(y, _np(want)))
+                for a, b in zip(carry, ref):
+                    assert a.shape == b.shape and a.dtype == b.dtype and relerr(a, _np(b)) <= tol, (name, relerr(a, _np(b)))
+                ref = tuple(c.detach() for c in ref)
