@@ -5,8 +5,8 @@
 //
 // The library's products take such a call apart into a kernel per layer, a kernel per cast of a weight or an input, the norm
 // before them and the addition behind them -- a dozen launches of 2-5 us each for a few microseconds of reading weights.
-// Here one launch does all of it: a workgroup of four waves owns MT rows and 64 columns, normalises the rows on their way into
-// LDS (every workgroup needs whole rows for the product anyway), and each wave multiplies them with its sixteen weight rows,
+// Here one launch does all of it: a workgroup of four waves owns MT rows and 64 CT columns, normalises the rows on their way into
+// LDS (every workgroup needs whole rows for the product anyway), and each wave multiplies them with its 16 or 32 weight rows,
 // which it reads from memory as they are (float32 or bfloat16; L2-resident: all row tiles read the same ones) and requests
 // before it touches x, so that both trips to memory overlap.
 //
@@ -19,9 +19,8 @@
 namespace mrx {
 namespace {
 
-constexpr int RD_WAVES = 4, RD_THREADS = 64 * RD_WAVES, RD_COLS = 16 * RD_WAVES;
+constexpr int RD_WAVES = 4, RD_THREADS = 64 * RD_WAVES;
 constexpr int RD_MAX_K = 2048;
-constexpr int RD_AHEAD = 8;   // k steps whose weight fragments are requested at once
 
 struct RowDenseArgs {
     const void *x;
@@ -53,10 +52,20 @@ template <bool BF> __device__ __forceinline__ Quad quad_of(const void *p, int64_
     return q;
 }
 
+// Sum over a wave, in every lane: within rows of sixteen lanes by DPP moves (one instruction each, where a shuffle is a trip to
+// LDS), the four rows by shuffles.
 __device__ __forceinline__ float wave_total(float x)
 {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off);
+    auto add = [&](auto ctrl) {
+        const int moved = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, true);
+        x += __builtin_bit_cast(float, moved);
+    };
+    add(std::integral_constant<int, 0xB1>{});    // quad_perm [1,0,3,2]
+    add(std::integral_constant<int, 0x4E>{});    // quad_perm [2,3,0,1]
+    add(std::integral_constant<int, 0x141>{});   // row_half_mirror
+    add(std::integral_constant<int, 0x140>{});   // row_mirror
+    x += __shfl_xor(x, 16);
+    x += __shfl_xor(x, 32);
     return x;
 }
 
@@ -96,12 +105,14 @@ template <typename T, bool WBF> __device__ __forceinline__ typename TT<T>::frag 
     return f;
 }
 
-// T: the products' type; MT: rows per workgroup (16 or 32); NV: 256-feature groups a lane holds of a row (K <= 256 NV).
-template <typename T, bool WBF, int MT, int NV>
+// T: the products' type; MT: rows per workgroup (16 or 32); NV: 256-feature groups a lane holds of a row (K <= 256 NV);
+// CT: 16-column tiles per wave.
+template <typename T, bool WBF, int MT, int NV, int CT>
 __global__ void __launch_bounds__(RD_THREADS) row_dense_kernel(RowDenseArgs a)
 {
     using F = typename TT<T>::frag;
     constexpr int KP = TT<T>::KP, KB = TT<T>::KB, RT = MT / 16, RPW = MT / RD_WAVES;
+    constexpr int AHEAD = 8 / CT;   // k steps whose weight fragments are requested at once
     extern __shared__ __align__(16) unsigned char smem[];
     T *sx = reinterpret_cast<T *>(smem);
     const int kpad = (a.K + KB - 1) / KB * KB, ld = kpad + pad_of<T>(), steps = kpad / KB;
@@ -111,18 +122,19 @@ __global__ void __launch_bounds__(RD_THREADS) row_dense_kernel(RowDenseArgs a)
     const int64_t r0 = (int64_t)(blockIdx.x / (unsigned)tiles) * MT;
     int l = 0;
     while (tile >= a.first_tile[l + 1]) ++l;
-    const int n0 = (tile - a.first_tile[l]) * RD_COLS + wv * 16, N = a.n[l];
+    const int n0 = ((tile - a.first_tile[l]) * RD_WAVES + wv) * 16 * CT, N = a.n[l];
     const void *w = a.w[l];
-    const int wrow = n0 + i16;   // this lane's weight row as an operand of the products
 
-    RawFrag<T, WBF> next[RD_AHEAD];
+    RawFrag<T, WBF> next[AHEAD][CT];
     auto fetch = [&](int s0) {
 #pragma unroll
-        for (int s = 0; s < RD_AHEAD; ++s) {
-            const int k = (s0 + s) * KB + KP * g;
-            if (wrow < N && k < a.K) next[s] = weight_raw<T, WBF>(w, (int64_t)wrow * a.K + k);   // K is a multiple of KP
-            else next[s] = RawFrag<T, WBF>{};
-        }
+        for (int s = 0; s < AHEAD; ++s)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) {
+                const int k = (s0 + s) * KB + KP * g, row = n0 + ct * 16 + i16;   // K is a multiple of KP
+                if (row < N && k < a.K) next[s][ct] = weight_raw<T, WBF>(w, (int64_t)row * a.K + k);
+                else next[s][ct] = RawFrag<T, WBF>{};
+            }
     };
     fetch(0);
 
@@ -186,60 +198,84 @@ __global__ void __launch_bounds__(RD_THREADS) row_dense_kernel(RowDenseArgs a)
     }
     __syncthreads();
 
-    f32x4 acc[RT];
+    f32x4 acc[RT][CT];
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) acc[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int s0 = 0; s0 < steps; s0 += RD_AHEAD) {
-        RawFrag<T, WBF> cur[RD_AHEAD];
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-        for (int s = 0; s < RD_AHEAD; ++s) cur[s] = next[s];
-        if (s0 + RD_AHEAD < steps) fetch(s0 + RD_AHEAD);
+        for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < steps; s0 += AHEAD) {
+        RawFrag<T, WBF> cur[AHEAD][CT];
 #pragma unroll
-        for (int s = 0; s < RD_AHEAD; ++s) {
+        for (int s = 0; s < AHEAD; ++s)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) cur[s][ct] = next[s][ct];
+        if (s0 + AHEAD < steps) fetch(s0 + AHEAD);
+#pragma unroll
+        for (int s = 0; s < AHEAD; ++s) {
             if (s0 + s >= steps) break;
-            const F wf = weight_frag<T, WBF>(cur[s]);
+            F wf[CT];
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-                acc[rt] = TT<T>::mma(wf, TT<T>::template load<ROWK>(sx, ld, rt * 16, (s0 + s) * KB, lane), acc[rt]);
+            for (int ct = 0; ct < CT; ++ct) wf[ct] = weight_frag<T, WBF>(cur[s][ct]);
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                const F xf = TT<T>::template load<ROWK>(sx, ld, rt * 16, (s0 + s) * KB, lane);
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = TT<T>::mma(wf[ct], xf, acc[rt][ct]);
+            }
         }
     }
 
-    // lane (i16, g) holds columns n0 + 4 g + 0..3 of row i16 of each row tile
-    const int c0 = n0 + 4 * g;
-    float bias[4];
+    // lane (i16, g) holds columns c0 .. c0 + 3 of row i16 of each row tile: one store where rows are whole quads
+    const bool quads = N % 4 == 0;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        bias[e] = 0.f;
-        if (a.b[l] && c0 + e < N) {
-            bias[e] = a.b_bf16 ? (float)static_cast<const __bf16 *>(a.b[l])[c0 + e] : static_cast<const float *>(a.b[l])[c0 + e];
-            if (std::is_same<T, __bf16>::value) bias[e] = (float)(__bf16)bias[e];
-        }
-    }
+    for (int ct = 0; ct < CT; ++ct) {
+        const int c0 = n0 + ct * 16 + 4 * g;
+        if (c0 >= N) continue;
+        float bias[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-        const int64_t r = r0 + rt * 16 + i16;
-        if (r >= a.rows) continue;
+        for (int e = 0; e < 4; ++e)
+            if (a.b[l] && c0 + e < N) {
+                bias[e] = a.b_bf16 ? (float)static_cast<const __bf16 *>(a.b[l])[c0 + e] : static_cast<const float *>(a.b[l])[c0 + e];
+                if (std::is_same<T, __bf16>::value) bias[e] = (float)(__bf16)bias[e];
+            }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            if (c0 + e >= N) break;
-            float y = acc[rt][e] + bias[e];
-            if (std::is_same<T, __bf16>::value) y = (float)(__bf16)y;
-            const int64_t at = r * N + c0 + e;
-            if (a.residual) static_cast<float *>(a.y[l])[at] = a.residual[at] + y;
-            else if (a.y_bf16) static_cast<__bf16 *>(a.y[l])[at] = (__bf16)y;
-            else static_cast<float *>(a.y[l])[at] = y;
+        for (int rt = 0; rt < RT; ++rt) {
+            const int64_t r = r0 + rt * 16 + i16, at = r * N + c0;
+            if (r >= a.rows) continue;
+            f32x4 y;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                y[e] = acc[rt][ct][e] + bias[e];
+                if (std::is_same<T, __bf16>::value) y[e] = (float)(__bf16)y[e];
+            }
+            float *yf = static_cast<float *>(a.y[l]) + at;
+            __bf16 *yb = static_cast<__bf16 *>(a.y[l]) + at;
+            if (quads) {
+                if (a.residual) y += *reinterpret_cast<const f32x4 *>(a.residual + at);
+                if (a.y_bf16) *reinterpret_cast<bf16x4 *>(yb) = TT<__bf16>::pack(y[0], y[1], y[2], y[3]);
+                else *reinterpret_cast<f32x4 *>(yf) = y;
+                continue;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (c0 + e >= N) break;
+                if (a.residual) y[e] += a.residual[at + e];
+                if (a.y_bf16) yb[e] = (__bf16)y[e];
+                else yf[e] = y[e];
+            }
         }
     }
 }
 
-template <typename T, bool WBF, int MT> int launch_rows(hipStream_t st, const RowDenseArgs &a)
+template <typename T, bool WBF, int MT, int CT> int launch_rows(hipStream_t st, RowDenseArgs &a)
 {
-    constexpr int KB = TT<T>::KB;
+    constexpr int KB = TT<T>::KB, COLS = 16 * CT * RD_WAVES;
+    for (int l = 0; l < a.layers; ++l) a.first_tile[l + 1] = a.first_tile[l] + (a.n[l] + COLS - 1) / COLS;
     const size_t lds = (size_t)MT * ((a.K + KB - 1) / KB * KB + pad_of<T>()) * sizeof(T);
     const int64_t grid = (a.rows + MT - 1) / MT * a.first_tile[a.layers];
     if (grid >= (1ll << 31)) return MRX_ERR_INVALID_ARG;
     auto go = [&](auto nv) {
-        return launch_kernel(row_dense_kernel<T, WBF, MT, decltype(nv)::value>, dim3((unsigned)grid), dim3(RD_THREADS), lds, st, a);
+        return launch_kernel(row_dense_kernel<T, WBF, MT, decltype(nv)::value, CT>, dim3((unsigned)grid), dim3(RD_THREADS), lds, st, a);
     };
     if (a.K <= 256) return go(std::integral_constant<int, 1>{});
     if constexpr (MT == 16) {
@@ -248,20 +284,37 @@ template <typename T, bool WBF, int MT> int launch_rows(hipStream_t st, const Ro
     }
     return go(std::integral_constant<int, 2>{});
 }
+// Rows and columns per workgroup.  Few workgroups finish soonest small (16 rows x 64 columns: the call is one trip to memory and
+// back); once they outnumber the compute units a few times over, larger ones read every weight and every row less often.
+// Measured inside a HIP graph, 256 features (us): q, k, v and beta of 1 024 environments 8.1 / 7.7 / 7.7 at 16 x 64 / 32 x 64 /
+// 32 x 128, of 2 048 12.0 / 10.9 / 9.6, of 4 096 19.4 / 17.4 / 14.2; a single 256-column layer 5.3 / 7.3 / 9.0 at 1 024 rows,
+// 6.3 / 7.5 / 9.3 at 2 048, 9.2 / 8.8 / 9.4 at 4 096.  (The library's products alone, without the norm: 14.8, 15.8, 19.7 for the
+// first three.)  Wide rows stay at 16: their registers and LDS would not fit otherwise.
+template <typename T, bool WBF> int by_shape(hipStream_t st, RowDenseArgs &a)
+{
+    int64_t small = 0;
+    for (int l = 0; l < a.layers; ++l) small += (a.n[l] + 63) / 64;
+    small *= (a.rows + 15) / 16;
+    if (small <= 512 || a.K > 512) return launch_rows<T, WBF, 16, 1>(st, a);
+    if (small <= 1024) return launch_rows<T, WBF, 32, 1>(st, a);
+    return launch_rows<T, WBF, 32, 2>(st, a);
+}
 
 // Dynamic LDS beyond the default limit of 64 KB: float32 rows of more than 500 (32 rows) or 1 000 features (16 rows).
 constexpr int RD_MAX_LDS = 16 * (RD_MAX_K + 4) * 4;
 const KernelRegistrar registrars[] = {
-    {reinterpret_cast<const void *>(row_dense_kernel<float, false, 16, 8>), RD_MAX_LDS},
-    {reinterpret_cast<const void *>(row_dense_kernel<float, true, 16, 8>), RD_MAX_LDS},
-    {reinterpret_cast<const void *>(row_dense_kernel<float, false, 16, 4>), RD_MAX_LDS},
-    {reinterpret_cast<const void *>(row_dense_kernel<float, true, 16, 4>), RD_MAX_LDS},
-    {reinterpret_cast<const void *>(row_dense_kernel<float, false, 32, 2>), RD_MAX_LDS},
-    {reinterpret_cast<const void *>(row_dense_kernel<float, true, 32, 2>), RD_MAX_LDS},
-    {reinterpret_cast<const void *>(row_dense_kernel<__bf16, false, 16, 8>), RD_MAX_LDS},
-    {reinterpret_cast<const void *>(row_dense_kernel<__bf16, true, 16, 8>), RD_MAX_LDS},
-    {reinterpret_cast<const void *>(row_dense_kernel<__bf16, false, 16, 4>), RD_MAX_LDS},
-    {reinterpret_cast<const void *>(row_dense_kernel<__bf16, true, 16, 4>), RD_MAX_LDS},
+    {reinterpret_cast<const void *>(row_dense_kernel<float, false, 16, 8, 1>), RD_MAX_LDS},
+    {reinterpret_cast<const void *>(row_dense_kernel<float, true, 16, 8, 1>), RD_MAX_LDS},
+    {reinterpret_cast<const void *>(row_dense_kernel<float, false, 16, 4, 1>), RD_MAX_LDS},
+    {reinterpret_cast<const void *>(row_dense_kernel<float, true, 16, 4, 1>), RD_MAX_LDS},
+    {reinterpret_cast<const void *>(row_dense_kernel<float, false, 32, 2, 1>), RD_MAX_LDS},
+    {reinterpret_cast<const void *>(row_dense_kernel<float, true, 32, 2, 1>), RD_MAX_LDS},
+    {reinterpret_cast<const void *>(row_dense_kernel<float, false, 32, 2, 2>), RD_MAX_LDS},
+    {reinterpret_cast<const void *>(row_dense_kernel<float, true, 32, 2, 2>), RD_MAX_LDS},
+    {reinterpret_cast<const void *>(row_dense_kernel<__bf16, false, 16, 8, 1>), RD_MAX_LDS},
+    {reinterpret_cast<const void *>(row_dense_kernel<__bf16, true, 16, 8, 1>), RD_MAX_LDS},
+    {reinterpret_cast<const void *>(row_dense_kernel<__bf16, false, 16, 4, 1>), RD_MAX_LDS},
+    {reinterpret_cast<const void *>(row_dense_kernel<__bf16, true, 16, 4, 1>), RD_MAX_LDS},
 };
 
 }  // namespace
@@ -290,18 +343,10 @@ extern "C" int mrx_row_dense(void *stream, const void *x, const float *scale, co
         if (!weights[l] || !outs[l] || !aligned(weights[l], 16) || !aligned(outs[l], 4)) return MRX_ERR_INVALID_ARG;
         if (n_out[l] <= 0 || n_out[l] > (1 << 24)) return MRX_ERR_INVALID_ARG;
         a.w[l] = weights[l], a.b[l] = biases[l], a.y[l] = outs[l], a.n[l] = (int)n_out[l];
-        a.first_tile[l + 1] = a.first_tile[l] + (int)((n_out[l] + RD_COLS - 1) / RD_COLS);
     }
     if (const int rc = prepare_device(); rc != MRX_OK) return rc;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const bool bf = product_dtype == MRX_BF16;
-    // 32 rows per workgroup read every weight half as often; 16 where that leaves workgroups for the compute units, and where
-    // a row is so wide that its registers (eight rows per wave) or its LDS would not fit
-    const bool wide = K <= 512 && (rows + 31) / 32 * a.first_tile[layers] >= 256;
-    if (bf) {
-        if (a.w_bf16) return wide ? launch_rows<__bf16, true, 32>(st, a) : launch_rows<__bf16, true, 16>(st, a);
-        return wide ? launch_rows<__bf16, false, 32>(st, a) : launch_rows<__bf16, false, 16>(st, a);
-    }
-    if (a.w_bf16) return wide ? launch_rows<float, true, 32>(st, a) : launch_rows<float, true, 16>(st, a);
-    return wide ? launch_rows<float, false, 32>(st, a) : launch_rows<float, false, 16>(st, a);
+    if (bf) return a.w_bf16 ? by_shape<__bf16, true>(st, a) : by_shape<__bf16, false>(st, a);
+    return a.w_bf16 ? by_shape<float, true>(st, a) : by_shape<float, false>(st, a);
 }

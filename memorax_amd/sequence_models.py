@@ -427,7 +427,7 @@ class GatedLinearRecurrence(SequenceModel):
 # ----------------------------------------------------------------------------------
 # acting: one time step without gradients (ppo.py:105-143), rows = environments
 # ----------------------------------------------------------------------------------
-_ACTING_ROWS = 4096   # up to here a row-dense launch beats the array library's products and what surrounds them
+_ACTING_ROWS = 16384   # up to here a row-dense launch beats the array library's products and what surrounds them
 
 
 def _acts(x, done, norm):
