@@ -40,7 +40,7 @@ compile _clk -DMRX_PHASE_CLOCKS=1
 SRCS=(pattern_probe.hip)
 compile ""
 TORCH=$(python3 -c 'import os, torch; print(os.path.dirname(torch.__file__))')
-g++ -O2 -std=c++17 -fPIC -shared -fvisibility=hidden -Wall -D__HIP_PLATFORM_AMD__=1 -DUSE_ROCM=1 -I../../include \
+g++ -O2 -std=c++20 -fPIC -shared -fvisibility=hidden -Wall -D__HIP_PLATFORM_AMD__=1 -DUSE_ROCM=1 -I../../include \
     -isystem "$TORCH/include" -isystem "$TORCH/include/torch/csrc/api/include" -isystem /opt/rocm/include $(python3-config --includes) \
     host_ops.cpp -o ../_native.so -L"$TORCH/lib" -ltorch -ltorch_cpu -ltorch_hip -lc10 -lc10_hip -ltorch_python -Wl,-rpath,"$TORCH/lib" &
 pids+=($!)

@@ -11,6 +11,7 @@
 // The entry points of the C ABI are bound at run time (bind()) from whatever build of the library Python has
 // loaded; nothing here links against it.
 #include <ATen/ATen.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/HIPContextLight.h>
 #include <c10/hip/HIPStream.h>
@@ -732,6 +733,8 @@ std::vector<Tensor> row_dense(const Tensor &x, int norm, const OptTensor &scale,
     return out;
 }
 
+constexpr int64_t ROW_DENSE_ROWS = 16384;   // up to here one launch beats the array library's products and casts
+
 // z, h~, gate (B,1,D), done (B,1), the carry's leaves (B,1,D) float32 -> y, log_state, log_decay
 std::tuple<Tensor, Tensor, Tensor> mingru_step(const Tensor &z, const Tensor &x, const OptTensor &gate, const Tensor &done_,
                                                const Tensor &log_state, const Tensor &log_decay, bool in_place)
@@ -780,6 +783,7 @@ template <class Op> struct OpNode final : torch::autograd::Node {
     {
         std::lock_guard<std::mutex> lock(mutex_);
         for (auto &s : saved) s.reset_data();
+        if constexpr (requires(Op & o) { o.release(); }) op.release();
     }
     std::string name() const override { return Op::name(); }
     bool wants(size_t i) const { return task_should_compute_output(i); }
@@ -1175,6 +1179,178 @@ std::tuple<Tensor, Tensor> norm(const Tensor &x, const OptTensor &scale, const O
     return {fork ? res : x, y};
 }
 
+// ---- dense layers (memorax_amd/dense.py): the array library's products in a shape it runs well
+constexpr int64_t SLICE_ROWS = 2048, MAX_SLICES = 128;   // rows per slice of the weight-gradient product
+
+// Into how many slices the rows of a weight-gradient product are cut: none while the result has tiles enough to fill the
+// device or the rows are few.
+int64_t weight_gradient_slices(int64_t rows, int64_t n_out, int64_t n_in)
+{
+    if (rows < 4 * SLICE_ROWS || rows < 32 * std::max(n_out, n_in)) return 1;
+    int64_t s = 1;
+    while (s < MAX_SLICES && rows % (2 * s) == 0 && rows / (2 * s) >= SLICE_ROWS) s *= 2;
+    return s;
+}
+
+bool half(ScalarType dt) { return dt == at::kBFloat16 || dt == at::kHalf; }
+ScalarType wide(ScalarType dt) { return half(dt) ? at::kFloat : dt; }
+
+// dy^T x for dy (rows, n_out), x (rows, n_in); float32 from 16-bit operands
+Tensor weight_gradient(const Tensor &dy, const Tensor &x)
+{
+    const int64_t rows = dy.size(0), n_out = dy.size(1), n_in = x.size(1);
+    const int64_t s = dy.is_cuda() ? weight_gradient_slices(rows, n_out, n_in) : 1;
+    // a ragged batch: its even part in slices, the rest by itself
+    const int64_t even = rows - rows % (4 * SLICE_ROWS);
+    if (dy.is_cuda() && rows != even && s < weight_gradient_slices(even, n_out, n_in))
+        return weight_gradient(dy.narrow(0, 0, even), x.narrow(0, 0, even)) +
+               at::mm(dy.narrow(0, even, rows - even).t(), x.narrow(0, even, rows - even));
+    if (s == 1) return at::mm(dy.t(), x).to(wide(dy.scalar_type()));
+    const Tensor a = dy.reshape({s, rows / s, n_out}).transpose(1, 2), b = x.reshape({s, rows / s, n_in});
+    return (half(dy.scalar_type()) ? at::bmm(a, b, at::kFloat) : at::bmm(a, b)).sum(0);
+}
+
+// The dtype the array library's autocast would run a product on x in.
+std::optional<ScalarType> autocast_dtype(const Tensor &x)
+{
+    if (x.is_cuda() && x.is_floating_point() && at::autocast::is_autocast_enabled(at::kCUDA)) return at::autocast::get_autocast_dtype(at::kCUDA);
+    return std::nullopt;
+}
+
+// Several dense layers on one input: one cast of it, and the gradients with respect to it accumulated by the products
+// themselves (each adds onto the sum so far) instead of by a pass per layer.
+struct DenseOp {
+    static constexpr int SAVED = 1;   // x as the products read it; the weights follow in `weights`
+    static const char *name() { return "MemoraxDenseBackward"; }
+    std::vector<SavedVariable> weights;
+    std::vector<bool> has_bias;
+    ScalarType x_dtype;
+    variable_list backward(OpNode<DenseOp> &node, std::array<Tensor, 1> &s, variable_list &grads)
+    {
+        c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
+        const Tensor &x = s[0], x2 = x.reshape({-1, x.size(-1)});
+        const size_t n = weights.size();
+        variable_list out(1 + 2 * n);
+        for (size_t l = 0; l < n; ++l) {
+            if (!grads[l].defined()) continue;   // an output nobody used costs no products
+            const Tensor w = weights[l].unpack(), dy = grads[l].to(x.scalar_type()).reshape({-1, w.size(0)});
+            if (node.wants(0)) {
+                if (out[0].defined()) out[0].addmm_(dy, w);
+                else out[0] = at::mm(dy, w);
+            }
+            if (node.wants(1 + l)) out[1 + l] = weight_gradient(dy, x2);
+            if (has_bias[l] && node.wants(1 + n + l)) out[1 + n + l] = dy.sum({0}, false, wide(dy.scalar_type()));
+        }
+        if (out[0].defined()) out[0] = out[0].view(x.sizes()).to(x_dtype);
+        return out;
+    }
+    void release()
+    {
+        for (auto &w : weights) w.reset_data();
+    }
+};
+
+// Few rows without gradients: the layers as one launch of the row kernel, where it takes the arrays as they are.
+bool rows_suit(const Tensor &x, const std::vector<Tensor> &weights, const std::vector<OptTensor> &biases, std::optional<ScalarType> cast)
+{
+    const int64_t K = x.size(-1);
+    auto suits = [](ScalarType dt) { return dt == at::kFloat || dt == at::kBFloat16; };
+    auto fits = [](const Tensor &t) { return t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+    const auto wd = weights[0].scalar_type();
+    if (!x.is_cuda() || x.dim() < 2 || x.numel() == 0 || weights.size() > MRX_ROW_DENSE_LAYERS || K % 8 != 0 || K > 2048) return false;
+    if (x.numel() / K > ROW_DENSE_ROWS || !suits(x.scalar_type()) || !suits(wd) || !fits(x)) return false;
+    if (cast.has_value() ? *cast != at::kBFloat16 : wd != x.scalar_type()) return false;
+    for (size_t l = 0; l < weights.size(); ++l) {
+        if (weights[l].scalar_type() != wd || weights[l].dim() != 2 || weights[l].size(1) != K || weights[l].size(0) == 0 || !fits(weights[l])) return false;
+        if (biases[l].has_value() && (biases[l]->scalar_type() != wd || !biases[l]->is_contiguous())) return false;
+    }
+    return true;
+}
+
+std::vector<Tensor> dense_group(const Tensor &x, const std::vector<Tensor> &weights, const std::vector<OptTensor> &biases)
+{
+    TORCH_CHECK_VALUE(!weights.empty() && biases.size() == weights.size(), "dense_group takes one bias (or None) per weight");
+    const auto cast = autocast_dtype(x);
+    bool need = need_grad(x);
+    for (size_t l = 0; l < weights.size(); ++l) need = need || need_grad(weights[l], biases[l]);
+    c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
+    std::vector<Tensor> out;
+    out.reserve(weights.size());
+    std::vector<Tensor> ws;
+    Tensor xc;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        if (!need && rows_suit(x, weights, biases, cast)) {
+            const auto product = cast.value_or(x.scalar_type());
+            return row_dense(x, 0, std::nullopt, std::nullopt, 0.0, false, weights, biases, product, product, std::nullopt);
+        }
+        xc = cast.has_value() ? x.to(*cast) : x;
+        for (size_t l = 0; l < weights.size(); ++l) {
+            ws.push_back(cast.has_value() ? weights[l].to(*cast) : weights[l]);
+            out.push_back(at::linear(xc, ws[l], biases[l].has_value() && cast.has_value() ? OptTensor(biases[l]->to(*cast)) : biases[l]));
+        }
+    }
+    if (need) {
+        auto node = std::shared_ptr<OpNode<DenseOp>>(new OpNode<DenseOp>(), torch::autograd::deleteNode);
+        torch::autograd::edge_list edges = torch::autograd::collect_next_edges(x);
+        for (const Tensor &w : weights) edges.push_back(torch::autograd::impl::gradient_edge(w));
+        for (const OptTensor &b : biases) edges.push_back(b.has_value() ? torch::autograd::impl::gradient_edge(*b) : torch::autograd::Edge());
+        node->set_next_edges(std::move(edges));
+        node->op.x_dtype = x.scalar_type();
+        for (Tensor &y : out) torch::autograd::set_history(y, node);
+        node->keep(0, xc);
+        for (size_t l = 0; l < ws.size(); ++l) {
+            node->op.weights.emplace_back(ws[l], false);
+            node->op.has_bias.push_back(biases[l].has_value());
+        }
+    }
+    return out;
+}
+
+// ---- causal depthwise convolution over time with silu behind it (conv_cells.hip)
+struct ConvSiluOp {
+    static constexpr int SAVED = 3;   // x, weight, bias
+    static const char *name() { return "MemoraxCausalConvSiluBackward"; }
+    variable_list backward(OpNode<ConvSiluOp> &, std::array<Tensor, 3> &s, variable_list &grads)
+    {
+        if (!grads[0].defined()) return {Tensor(), Tensor(), Tensor()};
+        const Tensor &x = s[0];
+        const int64_t B = x.size(0), T = x.size(1), C = x.size(2), K = s[1].size(2);
+        const Tensor dy = grads[0].contiguous(), dx = fresh(x.sizes(), at::kFloat, x), params = fresh({C * (K + 1)}, at::kFloat, x),
+                     work = fresh({MRX_CONV_PARTS, C * (K + 1)}, at::kFloat, x);
+        check(lib.mrx_causal_conv_silu_bwd(stream(), fptr(x), x.stride(1), fptr(s[1]), fptr(s[2]), fptr(dy), fptr(dx), C, fptr(params),
+                                           fptr(work), B, T, C, K),
+              "mrx_causal_conv_silu_bwd");
+        return {dx, params.narrow(0, 0, C * K).view({C, 1, K}), params.narrow(0, C * K, C)};
+    }
+};
+
+// x (B,T,C) float32, dense or the leading columns of wider rows; weight (C,1,K), bias (C).
+Tensor causal_conv_silu(const Tensor &x_, const Tensor &weight, const Tensor &bias)
+{
+    TORCH_CHECK_VALUE(x_.dim() == 3 && weight.dim() == 3 && x_.is_cuda() && x_.scalar_type() == at::kFloat,
+                      "causal_conv_silu takes (B,T,C) float32 arrays on the GPU");
+    const int64_t B = x_.size(0), T = x_.size(1), C = x_.size(2), K = weight.size(2);
+    chk(weight, "weight", at::kFloat, {C, 1, K});
+    chk(bias, "bias", at::kFloat, {C});
+    Tensor x, y;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const bool rows = x_.stride(2) == 1 && x_.stride(1) % 4 == 0 && x_.stride(0) == T * x_.stride(1) && ((uintptr_t)x_.data_ptr()) % 16 == 0;
+        x = rows ? x_ : x_.contiguous();
+        y = fresh({B, T, C}, at::kFloat, x);
+        check(lib.mrx_causal_conv_silu_fwd(stream(), fptr(x), x.stride(1), fptr(weight), fptr(bias), fptr(y), B, T, C, K), "mrx_causal_conv_silu_fwd");
+    }
+    if (need_grad(x_, weight, bias)) {
+        auto node = record(ConvSiluOp{}, x_, weight, bias);
+        torch::autograd::set_history(y, node);
+        node->keep(0, x);
+        node->keep(1, weight);
+        node->keep(2, bias);
+    }
+    return y;
+}
+
 // ---- the Mamba cell between its projections: elements, recurrence, gated read-out (conv_cells.hip)
 struct MambaSizes {
     int64_t B, T, H, P, N, K, W;   // W = H * P, the hidden width; up holds (hidden | z): rows of 2 W
@@ -1402,5 +1578,9 @@ PYBIND11_MODULE(_native, m)
     def("mlstm_gates", &mlstm_gates);
     def("silu_gate", &silu_gate);
     def("norm", &norm);
+    def("dense_group", &dense_group);
+    def("weight_gradient", &weight_gradient);
+    def("weight_gradient_slices", &weight_gradient_slices);
+    def("causal_conv_silu", &causal_conv_silu);
     def("mamba_mix", &mamba_mix);
 }

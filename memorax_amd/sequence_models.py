@@ -30,7 +30,7 @@ import torch.nn.functional as F
 from typing import NamedTuple
 
 from ._lib import native
-from .dense import Dense, autocast_dtype, dense_group
+from .dense import Dense, Weights, autocast_dtype, dense, dense_group
 from .functional import (deltanet, gated_linear_attention, linear_attention, linear_scan, mingru_scan, mlstm_gates,
                          normalised_linear_attention, layer_norm, layer_norm_fork, rms_norm, rms_norm_fork, silu_gate,
                          stepping_in_place)
@@ -198,6 +198,23 @@ class _DiagonalCell(MemoroidCellBase):
         return (h, None), (h_last[:, None], P_last[:, None])
 
 
+def _complex_states(x, weight):
+    """x B^T for real x (B,T,F) and complex B given as (N, 2, F) (real and imaginary rows): one real product whose columns are
+    the complex result's components.  A complex product of x with a zero imaginary part is four times the arithmetic, and its
+    weight gradient -- a small complex result over every row -- took nine tenths of an LRU layer's update."""
+    N = weight.shape[0]
+    with torch.autocast(x.device.type, enabled=False):   # the recurrence runs in complex64 whatever surrounds it
+        out = dense(x.float(), weight.reshape(2 * N, -1).float())
+    return torch.view_as_complex(out.view(*out.shape[:-1], N, 2))
+
+
+def _real_read_out(state, weight):
+    """Re(state C^T) for complex state (B,T,N), C given as (F, N, 2) with (Re C, -Im C): one real product."""
+    flat = torch.view_as_real(state).flatten(-2)
+    with torch.autocast(state.device.type, enabled=False):
+        return dense(flat, weight.flatten(-2).to(flat.dtype))
+
+
 class LRUCell(_DiagonalCell):
     """Linear Recurrent Unit, complex diagonal recurrence (lru.py:32-108).  The decay
     lambda is time-invariant and is passed to the kernel as an (N,) vector instead of
@@ -220,15 +237,11 @@ class LRUCell(_DiagonalCell):
         self.D = nn.Parameter(torch.randn(features))
 
     def forward(self, x, **kwargs):
-        lam = torch.exp(torch.complex(-torch.exp(self.nu_log), torch.exp(self.theta_log)))
-        B_norm = torch.complex(self.B_real, self.B_imag) * torch.exp(self.gamma_log)[:, None]
-        state = x.to(torch.complex64) @ B_norm.T
-        return (state.contiguous(), lam.to(torch.complex64))
+        lam = torch.polar(torch.exp(-torch.exp(self.nu_log)), torch.exp(self.theta_log))
+        return (_complex_states(x, torch.stack([self.B_real, self.B_imag], 1) * torch.exp(self.gamma_log)[:, None, None]), lam)
 
     def read(self, h, x, **kwargs):
-        state, _ = h
-        C = torch.complex(self.C_real, self.C_imag)
-        return (state @ C.T).real + self.D * x
+        return _real_read_out(h[0], torch.stack([self.C_real, -self.C_imag], -1)) + self.D * x
 
     def initialize_carry(self, key, input_shape):
         *batch, _ = input_shape
@@ -292,13 +305,10 @@ class S5Cell(_DiagonalCell):
 
     def forward(self, x, **kwargs):
         lambda_bar, b_bar, _ = self._discretized_params()
-        state = x.to(torch.complex64) @ b_bar.T
-        return (state.contiguous(), lambda_bar.to(torch.complex64))
+        return (_complex_states(x, torch.view_as_real(b_bar).transpose(1, 2)), lambda_bar.to(torch.complex64))
 
-    def read(self, h, x, **kwargs):
-        _, _, c_tilde = self._discretized_params()
-        state, _ = h
-        return (state @ c_tilde.T).real + self.d * x
+    def read(self, h, x, **kwargs):   # c_tilde is C as it is learned: (F, N, 2)
+        return _real_read_out(h[0], torch.stack([self.C[..., 0], -self.C[..., 1]], -1)) + self.d * x
 
     def initialize_carry(self, key, input_shape):
         *batch, _ = input_shape
@@ -427,7 +437,7 @@ class GatedLinearRecurrence(SequenceModel):
 # ----------------------------------------------------------------------------------
 # acting: one time step without gradients (ppo.py:105-143), rows = environments
 # ----------------------------------------------------------------------------------
-_ACTING_ROWS = 16384   # up to here a row-dense launch beats the array library's products and what surrounds them
+_ACTING_ROWS = 16384   # as in csrc/host_ops.cpp: up to here one launch beats the array library's products and casts
 
 
 def _acts(x, done, norm):
@@ -625,6 +635,16 @@ class DeltaNetCell(MemoroidCellBase):
         return (torch.zeros(*batch, 1, self.num_heads, self.head_dim, self.head_dim, device=dev),)
 
 
+def _causal_conv_silu(x, conv):
+    """silu of a depthwise convolution over time that sees the steps up to its own and nothing before the call's first
+    (mamba.py:88-106): the library's kernel where it takes the arrays, else the array library's operations."""
+    K = conv.kernel_size[0]
+    if (x.is_cuda and x.dtype == torch.float32 and conv.weight.dtype == torch.float32 and autocast_dtype(x) is None and K <= 4
+            and x.shape[2] % 4 == 0 and x.numel() > 0):
+        return native().causal_conv_silu(x, conv.weight, conv.bias)
+    return F.silu(conv(F.pad(x.transpose(1, 2), (K - 1, 0)))).transpose(1, 2)
+
+
 class MambaCell(MemoroidCellBase):
     """Mamba-2 style selective state space cell (mamba.py:33-144).  Elements are
     (h_t = (B_t dt_t) (x) x_t : (H,N,P), decay_t = exp(dt_t A) : (H,1,1)) combined by the diagonal
@@ -658,8 +678,7 @@ class MambaCell(MemoroidCellBase):
         H, P, N = self.num_heads, self.head_dim, self.state_dim
         up, B_in, C_in, dt_in = dense_group(x, [self.input_projection, self.B, self.C, self.dt])
         hidden, z = up.chunk(2, dim=-1)
-        ci = torch.cat([hidden, B_in, C_in], dim=-1).transpose(1, 2)      # (B, channels, T)
-        ci = F.silu(self.conv(F.pad(ci, (self.conv_dim - 1, 0)))).transpose(1, 2)   # causal, per call
+        ci = _causal_conv_silu(torch.cat([hidden, B_in, C_in], dim=-1), self.conv)   # causal, per call
         hidden = ci[..., :H * P].reshape(Bn, T, H, P)
         B_proj = ci[..., H * P:H * P + H * N].reshape(Bn, T, H, N)
         C_proj = ci[..., H * P + H * N:].reshape(Bn, T, H, N)
@@ -749,6 +768,12 @@ class _BlockDiagonalDense(nn.Module):
         bs = features // num_heads
         self.num_heads = num_heads
         self.kernel = nn.Parameter(torch.randn(num_heads, bs, bs) * math.sqrt(2.0 / (5.0 * bs)))
+        self.register_buffer("_eye", torch.eye(num_heads), persistent=False)
+
+    def whole_weight(self):
+        """The map as one (features, features) matrix, zero off the diagonal blocks."""
+        h, o, d = self.kernel.shape
+        return (self.kernel[:, :, None, :] * self._eye.to(self.kernel.dtype)[:, None, :, None]).reshape(h * o, h * d)
 
     def forward(self, x):
         *batch, f = x.shape
@@ -796,19 +821,44 @@ class mLSTMCell(MemoroidCellBase):
         Bn, T, _ = x.shape
         d = self.hidden_dim // self.num_heads
         x_mlstm, z = self.up_projection(x).chunk(2, dim=-1)
-        u = F.silu(self.causal_conv(F.pad(x_mlstm.transpose(1, 2), (self.conv_kernel_size - 1, 0))).transpose(1, 2))
+        u = _causal_conv_silu(x_mlstm, self.causal_conv)
         heads = lambda t: t.reshape(Bn, T, self.num_heads, d)  # noqa: E731
-        return heads(self.query(u)), heads(self.key(u)), heads(self.value(x_mlstm)), z, u
+        if self._heads_as_one(x):
+            q, k = dense_group(u, [Weights(self.query.whole_weight()), Weights(self.key.whole_weight())])
+            v = dense(x_mlstm.contiguous(), self.value.whole_weight())
+        else:
+            q, k, v = self.query(u), self.key(u), self.value(x_mlstm)
+        return heads(q), heads(k), heads(v), z, u
+
+    def _heads_as_one(self, x):
+        """Heads of up to 64 features go through one product with the block-diagonal matrix: a batched product of such narrow
+        blocks, its permutations and its weight gradients over every row cost several times the zeros' arithmetic."""
+        return x.is_cuda and autocast_dtype(x) is None and self.hidden_dim // self.num_heads <= 64 and self.num_heads <= 8
 
     def forward(self, x, **kwargs):
         """Elements in kernel form: (k / sqrt(d), v, log_i, log_f, q)."""
-        Bn, T, _ = x.shape
-        q, k, v, _, _ = self._project(x)
-        gate_input = torch.cat([q, k, v], dim=-1).reshape(Bn, T, -1)
-        i_pre, f_pre = dense_group(gate_input, [self.i_gate, self.f_gate])
+        return self._elements(*self._project(x)[:3])
+
+    def _elements(self, q, k, v):
+        Bn, T, H, d = q.shape
+        if self._heads_as_one(q):   # the gates read (q | k | v) head by head: three products that add up instead of that array
+            w = torch.cat([self.i_gate.weight, self.f_gate.weight]).view(2 * H, H, 3, d)
+            parts = [dense(t.reshape(Bn, T, H * d), w[:, :, i].reshape(2 * H, H * d)) for i, t in enumerate((q, k, v))]
+            i_pre, f_pre = (parts[0] + parts[1] + parts[2] + torch.cat([self.i_gate.bias, self.f_gate.bias])).chunk(2, dim=-1)
+        else:
+            gate_input = torch.cat([q, k, v], dim=-1).reshape(Bn, T, -1)
+            i_pre, f_pre = dense_group(gate_input, [self.i_gate, self.f_gate])
         log_i = i_pre.float()
-        log_f = -F.softplus(-f_pre.float())
-        return (k / math.sqrt(k.shape[-1]), v, log_i, log_f, q)
+        log_f = F.logsigmoid(f_pre.float())
+        return (k / math.sqrt(d), v, log_i, log_f, q)
+
+    def whole(self, x, done, initial_carry):
+        """The composition below with the projections formed once (``read`` forms them again)."""
+        if not (x.is_cuda and x.dim() == 3 and _as_written(self, mLSTMCell)):
+            return None
+        q, k, v, z, u = self._project(x)
+        h, carry = self.scan(self._elements(q, k, v), initial_carry, done)
+        return carry, self._read_out(h, x, z, u)
 
     def binary_operator(self, a, b):
         C_a, log_f_a, n_a, m_a = a
@@ -849,8 +899,10 @@ class mLSTMCell(MemoroidCellBase):
         return h_tilde, carry
 
     def read(self, h_tilde, x, **kwargs):
+        return self._read_out(h_tilde, x, *self._project(x)[3:])
+
+    def _read_out(self, h_tilde, x, z, u):
         Bn, T, _ = x.shape
-        _, _, _, z, u = self._project(x)
         y = F.layer_norm(h_tilde, (h_tilde.shape[-1],), eps=1e-5) * (1.0 + self.norm_weight)[None, None]
         y = y.reshape(Bn, T, self.hidden_dim) + self.learnable_skip * u
         return self.output_projection(_gated(y, z).to(x.dtype))
