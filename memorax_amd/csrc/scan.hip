@@ -46,9 +46,26 @@ template <> struct Ops<c64> {
     }
 };
 
-template <typename E, int VEC> struct alignas(sizeof(E) * VEC) Vec {
+// VEC consecutive channels.  Only as aligned as one of them: rows of any width take vectors (see first_col), and the
+// device's vector accesses need no more than that.
+template <typename E, int VEC> struct Vec {
     E v[VEC];
 };
+
+// The same in LDS, where a whole vector moves at once.
+template <typename E, int VEC> struct alignas(sizeof(E) * VEC) LdsVec {
+    Vec<E, VEC> x;
+};
+
+// First of the VEC channels a thread owns when threads are laid along a row: the last thread of a row whose width is no
+// multiple of VEC moves back to end with it, i.e. it shares channels with its neighbour -- both compute and write the same
+// values.  (One channel per lane instead, the earlier answer to odd widths, halves what a load instruction brings in: bfloat16
+// MinGRU forward + backward at 2367 x 36 x 645 494 us, a third of the rate of an even width.)
+template <int VEC> __device__ __forceinline__ int64_t first_col(int64_t vec_index, int64_t D)
+{
+    const int64_t c = vec_index * VEC;
+    return c + VEC <= D ? c : D - VEC;
+}
 
 template <typename E, int VEC> __device__ __forceinline__ Vec<E, VEC> vfill(E x)
 {
@@ -62,24 +79,29 @@ template <typename E, int VEC> __device__ __forceinline__ Vec<E, VEC> vfill(E x)
 // stores are non-temporal, so that the stream does not sit in the caches at the expense of itself (measured at
 // 512 x 1024 x 1024 float32: forward 5.77 -> 6.05 TB/s, backward 5.74 -> 6.27 TB/s).  The built-ins take
 // scalars and vectors of the language, so a Vec or a raw word group goes through a word type of its size.
-template <int BYTES> struct StreamWord;
-template <> struct StreamWord<2> { using type = uint16_t; };
-template <> struct StreamWord<4> { using type = uint32_t; };
-template <> struct StreamWord<8> { typedef uint32_t type __attribute__((ext_vector_type(2))); };
-template <> struct StreamWord<16> { typedef uint32_t type __attribute__((ext_vector_type(4))); };
-template <typename X> __device__ __forceinline__ X ld_stream(const void *p)
+// AL: the alignment of one element.
+template <int BYTES, int AL> struct StreamWord;
+#define MRX_STREAM_WORD(AL)                                                                                          \
+    template <> struct StreamWord<4, AL> { typedef uint32_t type __attribute__((aligned(AL))); };                      \
+    template <> struct StreamWord<8, AL> { typedef uint32_t type __attribute__((ext_vector_type(2), aligned(AL))); };  \
+    template <> struct StreamWord<16, AL> { typedef uint32_t type __attribute__((ext_vector_type(4), aligned(AL))); };
+template <> struct StreamWord<2, 2> { using type = uint16_t; };
+MRX_STREAM_WORD(2)
+MRX_STREAM_WORD(4)
+#undef MRX_STREAM_WORD
+template <typename X, int AL> __device__ __forceinline__ X ld_stream(const void *p)
 {
     if constexpr (sizeof(X) <= 16) {
-        using W = typename StreamWord<sizeof(X)>::type;
+        using W = typename StreamWord<sizeof(X), AL>::type;
         return __builtin_bit_cast(X, __builtin_nontemporal_load(reinterpret_cast<const W *>(p)));
     } else {
         return *reinterpret_cast<const X *>(p);  // wider than one instruction moves (complex64 x 4)
     }
 }
-template <typename X> __device__ __forceinline__ void st_stream(void *p, const X &x)
+template <typename X, int AL> __device__ __forceinline__ void st_stream(void *p, const X &x)
 {
     if constexpr (sizeof(X) <= 16) {
-        using W = typename StreamWord<sizeof(X)>::type;
+        using W = typename StreamWord<sizeof(X), AL>::type;
         __builtin_nontemporal_store(__builtin_bit_cast(W, x), reinterpret_cast<W *>(p));
     } else {
         *reinterpret_cast<X *>(p) = x;
@@ -91,9 +113,9 @@ template <typename X> __device__ __forceinline__ void st_stream(void *p, const X
 template <typename S, typename E, int VEC> __device__ __forceinline__ Vec<E, VEC> ldv(const S *p)
 {
     if constexpr (std::is_same<S, E>::value) {
-        return ld_stream<Vec<E, VEC>>(p);
+        return ld_stream<Vec<E, VEC>, alignof(E)>(p);
     } else {
-        const Vec<S, VEC> raw = ld_stream<Vec<S, VEC>>(p);
+        const Vec<S, VEC> raw = ld_stream<Vec<S, VEC>, alignof(S)>(p);
         Vec<E, VEC> r;
 #pragma unroll
         for (int i = 0; i < VEC; ++i) r.v[i] = (E)raw.v[i];
@@ -123,7 +145,7 @@ template <typename S, int VEC> __device__ __forceinline__ raw_t<S, VEC> ldraw(co
         r.w[0] = *reinterpret_cast<const uint16_t *>(p);
         return r;
     } else {
-        return ld_stream<raw_t<S, VEC>>(p);
+        return ld_stream<raw_t<S, VEC>, alignof(S)>(p);
     }
 }
 template <typename S, typename E, int VEC> __device__ __forceinline__ Vec<E, VEC> cvtv(const raw_t<S, VEC> &raw)
@@ -144,13 +166,25 @@ template <typename S, typename E, int VEC> __device__ __forceinline__ Vec<E, VEC
 template <typename S, typename E, int VEC> __device__ __forceinline__ void stv(S *p, const Vec<E, VEC> &x)
 {
     if constexpr (std::is_same<S, E>::value) {
-        st_stream(p, x);
+        st_stream<Vec<E, VEC>, alignof(E)>(p, x);
     } else {
         Vec<S, VEC> raw;
 #pragma unroll
         for (int i = 0; i < VEC; ++i) raw.v[i] = (S)x.v[i];
-        st_stream(p, raw);
+        st_stream<Vec<S, VEC>, alignof(S)>(p, raw);
     }
+}
+
+// The carries (B,D): small, cached.
+template <typename E, int VEC> __device__ __forceinline__ Vec<E, VEC> ldc(const E *p)
+{
+    using W = typename StreamWord<sizeof(E) * VEC, alignof(E)>::type;
+    return __builtin_bit_cast(Vec<E, VEC>, W(*reinterpret_cast<const W *>(p)));
+}
+template <typename E, int VEC> __device__ __forceinline__ void stc(E *p, const Vec<E, VEC> &x)
+{
+    using W = typename StreamWord<sizeof(E) * VEC, alignof(E)>::type;
+    *reinterpret_cast<W *>(p) = __builtin_bit_cast(W, x);
 }
 
 // MinGRU in linear space.  The reference scans (log h, log decay) with logaddexp
@@ -199,13 +233,13 @@ struct MinGru {
     }
 };
 
-constexpr int TS = 8;  // time steps a wave holds in registers per super-step
+constexpr int TS_MIN = 8;  // time steps a wave holds in registers per super-step (template parameter TS of the kernels), at least
 
 // Forward.  grid = B * tiles workgroups, block = 64 * NW threads, NW <= MAXW (8, or 16 for the
 // one-vector-lane instances that small shapes take: with 16 waves of 8 steps a sequence of up to 128
 // steps is one super-step, every load of the workgroup in flight at once and a single barrier).
 // smem: sH[2][NW][64] Vec, sP[2][NW][64] Vec, sF[2][NW] int.
-template <typename E, int VEC, bool MG = false, int MAXW = 8, typename S = E>
+template <typename E, int VEC, bool MG = false, int MAXW = 8, typename S = E, int TS = TS_MIN>
 __global__ void __launch_bounds__(64 * MAXW)
 diag_scan_fwd_kernel(const S *__restrict__ a, const S *__restrict__ b,
                      const void *__restrict__ done, int done_f32,
@@ -217,22 +251,23 @@ diag_scan_fwd_kernel(const S *__restrict__ a, const S *__restrict__ b,
     using V = Vec<E, VEC>;
     using O = Ops<E>;
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    V *sH = reinterpret_cast<V *>(smem_raw);
-    V *sP = sH + 2 * NW * 64;
+    using L = LdsVec<E, VEC>;
+    L *sH = reinterpret_cast<L *>(smem_raw);
+    L *sP = sH + 2 * NW * 64;
     int *sF = reinterpret_cast<int *>(sP + 2 * NW * 64);
 
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int tile = blockIdx.x % tiles;
     const int64_t bi = blockIdx.x / tiles;
-    const int64_t col = ((int64_t)tile * 64 + lane) * VEC;
-    const bool act = col < D;
+    const bool act = ((int64_t)tile * 64 + lane) * VEC < D;
+    const int64_t col = first_col<VEC>((int64_t)tile * 64 + lane, D);
     const int64_t row0 = bi * T;
 
     V carry_h = vfill<E, VEC>(O::zero()), carry_p = vfill<E, VEC>(O::one());
     if (act) {
-        if (h0) carry_h = *reinterpret_cast<const V *>(h0 + bi * D + col);
-        if (P0) carry_p = *reinterpret_cast<const V *>(P0 + bi * D + col);
+        if (h0) carry_h = ldc<E, VEC>(h0 + bi * D + col);
+        if (P0) carry_p = ldc<E, VEC>(P0 + bi * D + col);
     }
 
     const int span = NW * TS;
@@ -304,8 +339,8 @@ diag_scan_fwd_kernel(const S *__restrict__ a, const S *__restrict__ b,
                 x[s] = hc;
                 p[s] = pc;
             }
-            sH[(buf * NW + w) * 64 + lane] = hc;
-            sP[(buf * NW + w) * 64 + lane] = pc;
+            sH[(buf * NW + w) * 64 + lane].x = hc;
+            sP[(buf * NW + w) * 64 + lane].x = pc;
             if (lane == 0) sF[buf * NW + w] = rmask != 0;
         }
         __syncthreads();
@@ -313,8 +348,8 @@ diag_scan_fwd_kernel(const S *__restrict__ a, const S *__restrict__ b,
         V cin_h = carry_h, cin_p = carry_p, my_h = carry_h;
         for (int j = 0; j < NW; ++j) {
             if (j == w) my_h = cin_h;
-            const V Hj = sH[(buf * NW + j) * 64 + lane];
-            const V Pj = sP[(buf * NW + j) * 64 + lane];
+            const V Hj = sH[(buf * NW + j) * 64 + lane].x;
+            const V Pj = sP[(buf * NW + j) * 64 + lane].x;
             const bool fj = sF[buf * NW + j] != 0;
 #pragma unroll
             for (int i = 0; i < VEC; ++i) {
@@ -341,15 +376,15 @@ diag_scan_fwd_kernel(const S *__restrict__ a, const S *__restrict__ b,
         buf ^= 1;
     }
     if (w == 0 && act) {
-        if (h_last) *reinterpret_cast<V *>(h_last + bi * D + col) = carry_h;
-        if (P_last) *reinterpret_cast<V *>(P_last + bi * D + col) = carry_p;
+        if (h_last) stc<E, VEC>(h_last + bi * D + col, carry_h);
+        if (P_last) stc<E, VEC>(P_last + bi * D + col, carry_p);
     }
 }
 
 // Backward: the same scan walked from t = T-1 down with coefficient conj(a_{t+1}),
 // cut where done_{t+1}; reversed index r = T-1-t runs forward.
 // MG: a holds z, hx holds x = h~; da receives dz and db receives dx.
-template <typename E, int VEC, bool MG = false, int MAXW = 8, typename S = E>
+template <typename E, int VEC, bool MG = false, int MAXW = 8, typename S = E, int TS = TS_MIN>
 __global__ void __launch_bounds__(64 * MAXW)
 diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S *__restrict__ hfw,
                      const void *__restrict__ done, int done_f32,
@@ -361,20 +396,21 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
     using V = Vec<E, VEC>;
     using O = Ops<E>;
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    V *sH = reinterpret_cast<V *>(smem_raw);
-    V *sP = sH + 2 * NW * 64;
+    using L = LdsVec<E, VEC>;
+    L *sH = reinterpret_cast<L *>(smem_raw);
+    L *sP = sH + 2 * NW * 64;
     int *sF = reinterpret_cast<int *>(sP + 2 * NW * 64);
 
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int tile = blockIdx.x % tiles;
     const int64_t bi = blockIdx.x / tiles;
-    const int64_t col = ((int64_t)tile * 64 + lane) * VEC;
-    const bool act = col < D;
+    const bool act = ((int64_t)tile * 64 + lane) * VEC < D;
+    const int64_t col = first_col<VEC>((int64_t)tile * 64 + lane, D);
     const int64_t row0 = bi * T;
 
     V carry = vfill<E, VEC>(O::zero());  // lam_{t+1} entering from the right
-    if (act && g_last) carry = *reinterpret_cast<const V *>(g_last + bi * D + col);
+    if (act && g_last) carry = ldc<E, VEC>(g_last + bi * D + col);
     // da_sum (time-invariant a): da is (B,D), the sum of the per-step terms over the sequence -- what the
     // gradient of a broadcast coefficient needs -- kept in registers instead of written per step
     V dsum = vfill<E, VEC>(O::zero());
@@ -418,7 +454,7 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
                     if (t > 0)
                         hp[s] = ldv<S, E, VEC>(hfw + off - D);
                     else if (h0)
-                        hp[s] = *reinterpret_cast<const V *>(h0 + bi * D + col);
+                        hp[s] = ldc<E, VEC>(h0 + bi * D + col);
                     if constexpr (MG) {
                         zt[s] = ldv<S, E, VEC>(a + off);
                         xt[s] = ldv<S, E, VEC>(hx + off);
@@ -429,7 +465,7 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
             // narrower storage: the values wait as stored and are widened once every load has been issued
             raw_t<S, VEC> rg[TS], ra[TS], rh[TS], rz[MG ? TS : 1], rxt[MG ? TS : 1];
             V h0v = vfill<E, VEC>(O::zero());  // h_{-1}: what step 0 multiplies its lam with
-            if (act && h0 && T - 1 - rs - (TS - 1) <= 0) h0v = *reinterpret_cast<const V *>(h0 + bi * D + col);
+            if (act && h0 && T - 1 - rs - (TS - 1) <= 0) h0v = ldc<E, VEC>(h0 + bi * D + col);
 #pragma unroll
             for (int s = 0; s < TS; ++s) {
                 const int t = T - 1 - (rs + s);
@@ -506,15 +542,15 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
                 x[s] = lc;
                 p[s] = pc;
             }
-            sH[(buf * NW + w) * 64 + lane] = lc;
-            sP[(buf * NW + w) * 64 + lane] = pc;
+            sH[(buf * NW + w) * 64 + lane].x = lc;
+            sP[(buf * NW + w) * 64 + lane].x = pc;
             if (lane == 0) sF[buf * NW + w] = cmask != 0;
             __syncthreads();
             V cin = carry;
             for (int j = 0; j < NW; ++j) {
                 if (j == w) my = cin;
-                const V Hj = sH[(buf * NW + j) * 64 + lane];
-                const V Pj = sP[(buf * NW + j) * 64 + lane];
+                const V Hj = sH[(buf * NW + j) * 64 + lane].x;
+                const V Pj = sP[(buf * NW + j) * 64 + lane].x;
                 const bool fj = sF[buf * NW + j] != 0;
 #pragma unroll
                 for (int i = 0; i < VEC; ++i) {
@@ -568,17 +604,17 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
     if (!MG && da_sum) {  // uniform over the workgroup
         if (NW > 1) {
             __syncthreads();  // the last fold has read sH
-            sH[w * 64 + lane] = dsum;
+            sH[w * 64 + lane].x = dsum;
             __syncthreads();
             if (w == 0) {
                 for (int j = 1; j < NW; ++j) {
-                    const V dj = sH[j * 64 + lane];
+                    const V dj = sH[j * 64 + lane].x;
 #pragma unroll
                     for (int i = 0; i < VEC; ++i) dsum.v[i] = O::madd(O::one(), dsum.v[i], dj.v[i]);
                 }
             }
         }
-        if (w == 0 && act) *reinterpret_cast<V *>(reinterpret_cast<E *>(da) + bi * D + col) = dsum;  // (B,D), arithmetic type
+        if (w == 0 && act) stc<E, VEC>(reinterpret_cast<E *>(da) + bi * D + col, dsum);  // (B,D), arithmetic type
     }
     if (w == 0 && act && dh0) {
         // carry = lam_0 ; dh0 = done_0 ? 0 : conj(a_0) lam_0
@@ -597,7 +633,7 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
             const E prod = O::mul(O::conj(a0.v[i]), carry.v[i]);
             o.v[i] = d0 ? O::zero() : prod;
         }
-        *reinterpret_cast<V *>(dh0 + bi * D + col) = o;
+        stc<E, VEC>(dh0 + bi * D + col, o);
     }
 }
 
@@ -623,12 +659,12 @@ diag_scan_fwd_stream_kernel(const S *__restrict__ a, const S *__restrict__ b,
     // one thread per VEC channels of one batch row
     const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t bi = gid / cols_per_row;
-    const int64_t col = (gid % cols_per_row) * VEC;
+    const int64_t col = first_col<VEC>(gid % cols_per_row, D);
     if (bi >= B) return;  // padding threads of the last workgroup (this kernel has no barriers)
     const int64_t row0 = bi * T;
     V ch = vfill<E, VEC>(O::zero()), cp = vfill<E, VEC>(O::one());
-    if (h0) ch = *reinterpret_cast<const V *>(h0 + bi * D + col);
-    if (P0) cp = *reinterpret_cast<const V *>(P0 + bi * D + col);
+    if (h0) ch = ldc<E, VEC>(h0 + bi * D + col);
+    if (P0) cp = ldc<E, VEC>(P0 + bi * D + col);
 
     using R = raw_t<S, VEC>;  // prefetched values stay as stored until they are consumed
     R xa[SG], xb[SG], na[SG], nb[SG];
@@ -671,8 +707,8 @@ diag_scan_fwd_stream_kernel(const S *__restrict__ a, const S *__restrict__ b,
 #pragma unroll
         for (int s = 0; s < SG; ++s) { xa[s] = na[s]; xb[s] = nb[s]; xd[s] = nd[s]; }
     }
-    if (h_last) *reinterpret_cast<V *>(h_last + bi * D + col) = ch;
-    if (P_last) *reinterpret_cast<V *>(P_last + bi * D + col) = cp;
+    if (h_last) stc<E, VEC>(h_last + bi * D + col, ch);
+    if (P_last) stc<E, VEC>(P_last + bi * D + col, cp);
 }
 
 // ---- final state only, decay shared by groups of channels ---------------------------
@@ -695,7 +731,7 @@ diag_scan_last_kernel(const E *__restrict__ a, const E *__restrict__ b, const vo
     if (bi >= B) return;  // padding threads of the last workgroup (this kernel has no barriers)
     const int64_t row0 = bi * T, Da = D / a_group, acol = col / a_group;  // VEC divides a_group
     V ch = vfill<E, VEC>(O::zero());
-    if (h0) ch = *reinterpret_cast<const V *>(h0 + bi * D + col);
+    if (h0) ch = ldc<E, VEC>(h0 + bi * D + col);
 
     E xa[SG], na[SG];
     V xb[SG], nb[SG];
@@ -707,7 +743,7 @@ diag_scan_last_kernel(const E *__restrict__ a, const E *__restrict__ b, const vo
             pd[s] = 0u;
             if (t < T) {
                 pa[s] = a[(row0 + t) * Da + acol];
-                pb[s] = *reinterpret_cast<const V *>(b + (row0 + t) * D + col);
+                pb[s] = ldc<E, VEC>(b + (row0 + t) * D + col);
                 pd[s] = done_raw(done, done_f32, row0 + t);
             }
         }
@@ -729,7 +765,7 @@ diag_scan_last_kernel(const E *__restrict__ a, const E *__restrict__ b, const vo
 #pragma unroll
         for (int s = 0; s < SG; ++s) { xa[s] = na[s]; xb[s] = nb[s]; xd[s] = nd[s]; }
     }
-    *reinterpret_cast<V *>(h_last + bi * D + col) = ch;
+    stc<E, VEC>(h_last + bi * D + col, ch);
 }
 
 // MG: a holds z, hx holds x = h~ (a fourth load per step); da receives dz and db receives dx.
@@ -755,12 +791,12 @@ diag_scan_bwd_stream_kernel(const S *__restrict__ a, const S *__restrict__ hx, c
     constexpr int done_f32 = DF;
     const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t bi = gid / cols_per_row;
-    const int64_t col = (gid % cols_per_row) * VEC;
+    const int64_t col = first_col<VEC>(gid % cols_per_row, D);
     if (bi >= B) return;
     const int64_t row0 = bi * T;
     V dsum = vfill<E, VEC>(O::zero());  // da_sum: the per-step terms summed over the sequence, da is (B,D)
     V lam = vfill<E, VEC>(O::zero());  // conj(abar_{t+1}) lam_{t+1} entering step t
-    if (g_last) lam = *reinterpret_cast<const V *>(g_last + bi * D + col);
+    if (g_last) lam = ldc<E, VEC>(g_last + bi * D + col);
 
     // step r (reversed index), t = T-1-r: needs g_t, a_t (for the carry to t-1), h_{t-1}, done_t
     using R = raw_t<S, VEC>;  // prefetched values stay as stored until they are consumed
@@ -770,7 +806,7 @@ diag_scan_bwd_stream_kernel(const S *__restrict__ a, const S *__restrict__ hx, c
     R xx[MG ? SG : 1], nx[MG ? SG : 1];
     uint32_t xd[SG], nd[SG];
     V h0v = vfill<E, VEC>(O::zero());  // h_{-1}: what step 0 multiplies its lam with
-    if (h0) h0v = *reinterpret_cast<const V *>(h0 + bi * D + col);
+    if (h0) h0v = ldc<E, VEC>(h0 + bi * D + col);
     auto load = [&](int r0, R *pg, R *pa, R *ph, R *px, uint32_t *pd) {
 #pragma unroll
         for (int s = 0; s < SG; ++s) {
@@ -865,13 +901,14 @@ diag_scan_bwd_stream_kernel(const S *__restrict__ a, const S *__restrict__ hx, c
             for (int s = 0; s < SG; ++s) xx[s] = nx[s];
         }
     }
-    if (!MG && da_sum) *reinterpret_cast<V *>(reinterpret_cast<E *>(da) + bi * D + col) = dsum;  // (B,D), arithmetic type
-    if (dh0) *reinterpret_cast<V *>(dh0 + bi * D + col) = lam;  // conj(abar_0) lam_0
+    if (!MG && da_sum) stc<E, VEC>(reinterpret_cast<E *>(da) + bi * D + col, dsum);  // (B,D), arithmetic type
+    if (dh0) stc<E, VEC>(dh0 + bi * D + col, lam);  // conj(abar_0) lam_0
 }
 
 struct ScanPlan {
     int vec, nw, tiles;
     bool stream;  // streaming kernel (no time split) instead of the wave-split kernel
+    int ts = TS_MIN;  // steps per wave and super-step of the wave-split kernel
 };
 
 // Which kernel, how many elements per lane and how many waves along time.  Two layers of rules: the first
@@ -894,19 +931,16 @@ struct ScanPlan {
 //    kernel runs whenever the columns alone give >= 2048 waves.  With the MinGRU map inside (a
 //    fourth stream and the map's arithmetic per element) the eight-wave split loses to streaming at
 //    1024x128x256 (202 vs 165 us; level at the large shape), so that case keeps the rule it had.
-ScanPlan plan_scan(int64_t B, int64_t T, int64_t D, size_t esize, bool al16, bool al8, bool bwd, bool mg = false,
-                   bool half_storage = false)
+ScanPlan plan_scan(int64_t B, int64_t T, int64_t D, size_t esize, bool bwd, bool mg, bool half_storage, bool a_ti)
 {
     const int maxvec = (int)(16 / esize);
     int vec = 1;
     for (int v = maxvec; v >= 1; v >>= 1) {
-        const size_t bytes = esize * v;
-        const bool ok_al = bytes == 16 ? al16 : (bytes == 8 ? al8 : true);
         // a vector so wide that the waves covering a row are less than three quarters full wastes the
         // idle lanes' share of every load (rows of 128 floats, backward: 0.87 -> 0.57 ms at 16384x64x128
         // with two floats per lane instead of four; rows of 64: 0.75 -> 0.36 ms)
         const int64_t covered = ((D + 64 * (int64_t)v - 1) / (64 * (int64_t)v)) * 64 * v;
-        if (D % v == 0 && ok_al && (v == 1 || 4 * D >= 3 * covered)) { vec = v; break; }
+        if (D >= v && (v == 1 || 4 * D >= 3 * covered)) { vec = v; break; }
     }
     auto ntiles = [&](int v) { return (D + 64 * (int64_t)v - 1) / (64 * (int64_t)v); };
     // ---- Sequences of 32 steps and more: rules from a sweep of every plan (vector 1/2/4 x streaming or
@@ -919,46 +953,67 @@ ScanPlan plan_scan(int64_t B, int64_t T, int64_t D, size_t esize, bool al16, boo
     // The sweep was repeated after the arrays' loads and stores had become non-temporal: two float32 rules
     // changed (marked below); against the new timings the rules stand at 1.03 / 1.02 (float32), 1.03 / 1.02
     // (MinGRU), 1.02 / 1.00 (bfloat16) and 1.02 / 1.01 (complex64).
-    if (T >= 4 * TS) {
+    // A third sweep, once rows of any width took vectors and the wave-split kernels could hold 16 steps per wave: eighteen shapes,
+    // half of them with ragged widths or few columns over long sequences.  What changed is marked (*); times in us, before -> now.
+    if (T >= 4 * TS_MIN) {
         auto cols = [&](int v) { return B * ntiles(v); };  // workgroups of the wave-split kernel
-        auto split = [&](int v, int n) { return ScanPlan{v, n, (int)ntiles(v), false}; };
+        auto split = [&](int v, int n, int ts = TS_MIN) { return ScanPlan{v, n, (int)ntiles(v), false, ts}; };
+        auto flow = [&](int v) { return ScanPlan{v, 1, (int)ntiles(v), true}; };
+        const bool ragged = D % 64 != 0 && D > 128;
+        const int64_t waves2 = B * D / 128;   // of the streaming kernels on two elements per lane
         int nw8 = 1;  // waves along time: up to eight, each with a whole group of steps to itself
-        while (nw8 < 8 && (int64_t)2 * nw8 * TS <= T) nw8 <<= 1;
-        // so few columns that eight waves along time leave most of the device idle: sixteen of one lane each
-        if (T >= 16 * TS && cols(1) <= 256) return split(1, 16);
+        while (nw8 < 8 && (int64_t)2 * nw8 * TS_MIN <= T) nw8 <<= 1;
+        // (*) bfloat16 backward: single elements are 2-byte loads, three or four arrays of them; two per lane and 16 steps
+        // per wave make up for half the waves (8 x 1000 x 64 66 -> 54, 57 x 2908 x 120 217 -> 166)
+        if (half_storage && bwd && !mg && D >= 2 && T >= 8 * TS_MIN && waves2 < 600) return split(2, 8, T >= 16 * TS_MIN ? 16 : 8);
+        // so few columns that eight waves along time leave most of the device idle: sixteen of one lane each; (*) forward with
+        // 16 steps each, half as many trips to memory (4 x 3000 x 512 101 -> 77, 75 x 679 x 64 29 -> 22)
+        if (T >= 16 * TS_MIN && cols(1) <= 256) return split(1, 16, !bwd && esize == 4 && T > 16 * TS_MIN ? 16 : 8);
         if (half_storage) {
             // (swept again once the bfloat16 values waited as stored bits: the wave-split kernels then lead
             // forward at every size; four elements per lane, backward, do not fit the wave-split kernel's
             // registers)
-            const int v = vec < 2 ? vec : 2;
-            if (!bwd) return split(v, cols(v) >= 1024 && nw8 > 4 ? 4 : nw8);
-            // the streaming kernels lay their threads flat over (row, column): a row need not fill whole waves
-            if (D % 2 == 0 && al8 && B * D / 128 >= 2048) return {2, 1, (int)ntiles(2), true};
-            return split(v, cols(v) >= 512 && nw8 > 4 ? 4 : nw8);
+            const int v = D <= 64 || (!bwd && cols(1) <= 256) ? 1 : 2;
+            // the streaming kernels lay their threads flat over (row, column): a row need not fill whole waves.
+            // (*) They lead as soon as they have 600 waves backward, and on ragged rows with a thousand (MinGRU 1800) forward
+            // (1500 x 300 x 165 240 -> 137 and 439 -> 231; 128 x 512 x 1000 122 -> 111 and 222 -> 169)
+            if (v == 2 && (bwd ? waves2 >= 600 : ragged && waves2 >= (mg ? 1800 : 1000))) return flow(2);
+            if (cols(v) >= (bwd ? 512 : 1024) && nw8 > 4) return split(v, 4);
+            return split(v, nw8, !bwd && T >= 64 * TS_MIN && nw8 == 8 ? 16 : 8);   // (*) 256 x 1024 x 96 63 -> 50
         }
         if (esize == 8 && !mg) {
-            if (!bwd && T <= 256) return split(1, nw8);
-            if (bwd && vec == 2 && (cols(2) >= 1024 || (cols(2) >= 256 && T >= 64 * TS))) return split(2, nw8);
+            // (*) ragged rows stream, and so do the backward that sums a broadcast decay's gradient (no da to write) and that of
+            // short sequences: 400 x 200 x 201 backward 208 -> 155, 300 x 64 x 645 broadcast 102 -> 77, 1024 x 128 x 256
+            // broadcast 182 -> 157, 583 x 38 x 576 130 -> 104
+            if (waves2 >= 600 && (ragged || (bwd && (a_ti || T <= 8 * TS_MIN)))) return flow(D < 2 ? 1 : 2);
+            if (!bwd && a_ti && vec == 2 && cols(2) >= 1024 && T >= 8 * TS_MIN) return split(2, nw8 > 4 ? 4 : nw8);   // (*) 124 -> 106
+            if (!bwd && (T <= 256 || cols(1) <= 1024)) return split(1, nw8);
+            if (bwd && vec == 2 && (cols(2) >= 1024 || (cols(2) >= 256 && T >= 64 * TS_MIN))) return split(2, nw8);
         }
         if (esize == 4) {
+            // (*) ragged rows take the widest vector although its last wave is half empty: the time goes with the number of
+            // load instructions (forward, backward: 1500 x 300 x 165 335 -> 182, 634 -> 344; 400 x 200 x 201 63 -> 48, 110 -> 89;
+            // MinGRU 345 -> 192, 618 -> 452), once there are columns enough (49 x 62 x 235 forward 9.5 -> 11.7)
+            if (ragged && nw8 == 8 && cols(4) >= 256) return split(4, bwd && !mg ? 8 : 4);
             if (!bwd) {
                 // (swept again once every array was loaded and stored non-temporally: two elements per lane
                 // then lead at the large shapes as well -- 512 x 1024 x 1024 forward 1067 -> 1009 us,
                 // 4096 x 128 x 256 291 -> 269 us -- where four used to)
-                return split(vec < 2 ? vec : 2, nw8);
+                if (D > 64 && D < 128 && cols(1) <= 512 && T >= 64 * TS_MIN) return split(1, 8, 16);   // (*) 256 x 1024 x 96 81 -> 68
+                return split(vec < 2 || cols(1) <= 256 ? 1 : 2, nw8);
             }
             if (mg) {
-                if (vec == 4 && cols(4) >= 2048 && T >= 8 * TS) return split(4, nw8 > 4 ? 4 : nw8);
+                if (vec == 4 && cols(4) >= 2048 && T >= 8 * TS_MIN) return split(4, nw8 > 4 ? 4 : nw8);
                 if (D <= 128 && cols(1) >= 2048) return split(1, nw8);
             } else {
                 if (D <= 128 && cols(1) >= 1024) return split(1, nw8);
-                if (T >= 8 * TS) {
+                if (T >= 8 * TS_MIN) {
                     for (int v = vec; v >= 1; v >>= 1) {
                         // rows of a single column tile take eight waves along time, wider rows four (the same
                         // sweep: 8192 x 128 x 256 backward 1007 -> 920 us, 256 x 128 x 1024 149 -> 132 us)
                         if (cols(v) >= 1024) return split(v, ntiles(v) == 1 ? 8 : 4);
                         if (cols(v) * 8 >= 4096) return split(v, 8);
-                        if (v <= 2 && cols(v) * 16 >= 4096 && T >= 16 * TS) return split(v, 16);
+                        if (v <= 2 && cols(v) * 16 >= 4096 && T >= 16 * TS_MIN) return split(v, 16);
                     }
                 }
             }
@@ -973,7 +1028,7 @@ ScanPlan plan_scan(int64_t B, int64_t T, int64_t D, size_t esize, bool al16, boo
         const int64_t cols = B * ntiles(vec);
         if (cols >= 1024) return {vec, 1, (int)ntiles(vec), true};
         int nw = 1;
-        while (nw < 8 && cols * nw < 2048 && (int64_t)nw * TS < T) nw <<= 1;
+        while (nw < 8 && cols * nw < 2048 && (int64_t)nw * TS_MIN < T) nw <<= 1;
         return {vec, nw, (int)ntiles(vec), nw == 1};
     }
     // complex64 (measured on 1024x128x{64,128,256}, 4096x128x64, 256x1024x{64,256}, 64x4096x256): one
@@ -988,7 +1043,7 @@ ScanPlan plan_scan(int64_t B, int64_t T, int64_t D, size_t esize, bool al16, boo
         while (v1 > 1 && B * ntiles(v1) < 2048) v1 >>= 1;
         const int64_t waves1 = B * ntiles(v1);
         if (v1 == 1 && waves1 >= (bwd ? 1024 : 2048)) return {1, 1, (int)ntiles(1), true};
-        if (vec == 2 && v1 == 1 && B * ntiles(2) * 8 >= 4096 && T >= 8 * TS) return {2, 8, (int)ntiles(2), false};
+        if (vec == 2 && v1 == 1 && B * ntiles(2) * 8 >= 4096 && T >= 8 * TS_MIN) return {2, 8, (int)ntiles(2), false};
     }
     // floats, backward: see above; rows of up to 128 floats first -- there a wave's loads in the
     // wave-split kernel are short pieces, and one column per lane in the streaming kernel is ahead
@@ -998,8 +1053,8 @@ ScanPlan plan_scan(int64_t B, int64_t T, int64_t D, size_t esize, bool al16, boo
     if (bwd && !mg && esize == 4) {
         for (int v = vec; v >= 1; v >>= 1) {
             const int64_t cols = B * ntiles(v);
-            if (cols * 8 >= 4096 && T >= 8 * TS) return {v, 8, (int)ntiles(v), false};
-            if (v <= 2 && cols * 16 >= 4096 && T >= 16 * TS) return {v, 16, (int)ntiles(v), false};
+            if (cols * 8 >= 4096 && T >= 8 * TS_MIN) return {v, 8, (int)ntiles(v), false};
+            if (v <= 2 && cols * 16 >= 4096 && T >= 16 * TS_MIN) return {v, 16, (int)ntiles(v), false};
         }
     }
     while (vec > 1 && B * ntiles(vec) < 2048) vec >>= 1;
@@ -1007,7 +1062,7 @@ ScanPlan plan_scan(int64_t B, int64_t T, int64_t D, size_t esize, bool al16, boo
     const int64_t waves = B * tiles;
     int nw = 1;
     const int maxw = vec == 1 ? 16 : 8;
-    while (nw < maxw && waves * nw < 8192 && (int64_t)nw * TS < T) nw <<= 1;
+    while (nw < maxw && waves * nw < 8192 && (int64_t)nw * TS_MIN < T) nw <<= 1;
     const bool stream = bwd ? waves >= 2048 : nw == 1;
     // MinGRU backward short of columns for that: one column per lane still streams ahead of the wave-split
     // kernel from 1024 waves (1024x128x64: 55 -> 45 us, 256x1024x256: 472 -> 332 us)
@@ -1033,6 +1088,28 @@ template <typename E, typename F> void vec_switch(int vec, F f)
     }
 }
 
+// The wave-split kernels that exist: f(VEC, MAXW, TS), each an integral constant.
+template <typename E, bool MG, bool BWD, bool HALF, typename F> void split_switch(const ScanPlan &pl, F f)
+{
+    using std::integral_constant;
+    auto with_steps = [&](auto vc, auto mw) {
+        constexpr int VEC = decltype(vc)::value, MAXW = decltype(mw)::value;
+        // 16 steps per wave, where plan_scan asks for it: 4-byte arithmetic forward, bfloat16 arrays backward
+        constexpr bool LONG = BWD ? HALF && !MG && VEC == 2 && MAXW == 8 : sizeof(E) == 4 && (VEC == 1 || (HALF && VEC == 2 && MAXW == 8));
+        if constexpr (LONG) {
+            if (pl.ts == 16) return f(vc, mw, integral_constant<int, 16>{});
+        }
+        f(vc, mw, integral_constant<int, TS_MIN>{});
+    };
+    vec_switch<E>(pl.vec, [&](auto vc) {
+        constexpr int VEC = decltype(vc)::value;
+        if constexpr (VEC == 1 || (BWD && VEC == 2 && sizeof(E) == 4 && !MG)) {
+            if (pl.nw == 16) return with_steps(vc, integral_constant<int, 16>{});
+        }
+        with_steps(vc, integral_constant<int, 8>{});
+    });
+}
+
 // MG (E = float): a and b hold the MinGRU projections z and h~.
 // S: storage type of the (B,T,D) arrays (E, or __bf16 with E = float).
 template <typename E, bool MG = false, typename S = E>
@@ -1040,14 +1117,10 @@ int launch_fwd(hipStream_t st, const void *a, const void *b, const void *done,
                int done_f32, const void *h0, const void *P0, void *h, void *h_last,
                void *P_last, int64_t B, int64_t T, int64_t D, int a_ti)
 {
-    const bool al16 = aligned(a, 16) && aligned(b, 16) && aligned(h, 16) && aligned(h0, 16) &&
-                      aligned(P0, 16) && aligned(h_last, 16) && aligned(P_last, 16);
-    const bool al8 = aligned(a, 8) && aligned(b, 8) && aligned(h, 8) && aligned(h0, 8) &&
-                     aligned(P0, 8) && aligned(h_last, 8) && aligned(P_last, 8);
-    const ScanPlan pl = plan_scan(B, T, D, sizeof(E), al16, al8, false, MG, !std::is_same<S, E>::value);
+    const ScanPlan pl = plan_scan(B, T, D, sizeof(E), false, MG, !std::is_same<S, E>::value, a_ti);
     int rc = MRX_ERR_LAUNCH;
     if (pl.stream) {
-        const int64_t cpr = D / pl.vec;
+        const int64_t cpr = (D + pl.vec - 1) / pl.vec;
         const dim3 grid((unsigned)((B * cpr + 255) / 256)), block(256);
         vec_switch<E>(pl.vec, [&](auto vc) {
             constexpr int VEC = decltype(vc)::value;
@@ -1062,19 +1135,10 @@ int launch_fwd(hipStream_t st, const void *a, const void *b, const void *done,
     } else {
         const dim3 grid((unsigned)(B * pl.tiles)), block(64 * pl.nw);
         const size_t smem = scan_smem(pl.nw, sizeof(E) * pl.vec);
-        vec_switch<E>(pl.vec, [&](auto vc) {
-            constexpr int VEC = decltype(vc)::value;
-            if constexpr (VEC == 1) {
-                if (pl.nw == 16) {
-                    rc = launch_kernel((diag_scan_fwd_kernel<E, 1, MG, 16, S>), grid, block, smem, st, (const S *)a,
-                                       (const S *)b, done, done_f32, (const E *)h0, (const E *)P0, (S *)h,
-                                       (E *)h_last, (E *)P_last, (int)T, D, pl.tiles, pl.nw, a_ti);
-                    return;
-                }
-            }
-            rc = launch_kernel((diag_scan_fwd_kernel<E, VEC, MG, 8, S>), grid, block, smem, st, (const S *)a,
-                               (const S *)b, done, done_f32, (const E *)h0, (const E *)P0, (S *)h,
-                               (E *)h_last, (E *)P_last, (int)T, D, pl.tiles, pl.nw, a_ti);
+        split_switch<E, MG, false, !std::is_same<S, E>::value>(pl, [&](auto vc, auto mw, auto ts) {
+            rc = launch_kernel((diag_scan_fwd_kernel<E, decltype(vc)::value, MG, decltype(mw)::value, S, decltype(ts)::value>), grid, block, smem,
+                               st, (const S *)a, (const S *)b, done, done_f32, (const E *)h0, (const E *)P0, (S *)h, (E *)h_last, (E *)P_last,
+                               (int)T, D, pl.tiles, pl.nw, a_ti);
         });
     }
     return rc;
@@ -1086,14 +1150,10 @@ int launch_bwd(hipStream_t st, const void *a, const void *hx, const void *h, con
                int done_f32, const void *h0, const void *g, const void *g_last, void *da,
                void *db, void *dh0, int64_t B, int64_t T, int64_t D, int a_ti, int da_sum = 0)
 {
-    const bool al16 = aligned(a, 16) && aligned(hx, 16) && aligned(h, 16) && aligned(g, 16) && aligned(h0, 16) &&
-                      aligned(g_last, 16) && aligned(da, 16) && aligned(db, 16) && aligned(dh0, 16);
-    const bool al8 = aligned(a, 8) && aligned(hx, 8) && aligned(h, 8) && aligned(g, 8) && aligned(h0, 8) &&
-                     aligned(g_last, 8) && aligned(da, 8) && aligned(db, 8) && aligned(dh0, 8);
-    const ScanPlan pl = plan_scan(B, T, D, sizeof(E), al16, al8, true, MG, !std::is_same<S, E>::value);
+    const ScanPlan pl = plan_scan(B, T, D, sizeof(E), true, MG, !std::is_same<S, E>::value, a_ti);
     int rc = MRX_ERR_LAUNCH;
     if (pl.stream) {
-        const int64_t cpr = D / pl.vec;
+        const int64_t cpr = (D + pl.vec - 1) / pl.vec;
         const dim3 grid((unsigned)((B * cpr + 255) / 256)), block(256);
         vec_switch<E>(pl.vec, [&](auto vc) {
             constexpr int VEC = decltype(vc)::value;
@@ -1120,21 +1180,10 @@ int launch_bwd(hipStream_t st, const void *a, const void *hx, const void *h, con
     } else {
         const dim3 grid((unsigned)(B * pl.tiles)), block(64 * pl.nw);
         const size_t smem = scan_smem(pl.nw, sizeof(E) * pl.vec);
-        vec_switch<E>(pl.vec, [&](auto vc) {
-            constexpr int VEC = decltype(vc)::value;
-            if constexpr (VEC == 1 || (VEC == 2 && sizeof(E) == 4 && !MG)) {
-                if (pl.nw == 16) {
-                    rc = launch_kernel((diag_scan_bwd_kernel<E, VEC, MG, 16, S>), grid, block, smem, st, (const S *)a,
-                                       (const S *)hx, (const S *)h, done, done_f32, (const E *)h0, (const S *)g,
-                                       (const E *)g_last, (S *)da, (S *)db, (E *)dh0, (int)T, D, pl.tiles,
-                                       pl.nw, a_ti, da_sum);
-                    return;
-                }
-            }
-            rc = launch_kernel((diag_scan_bwd_kernel<E, VEC, MG, 8, S>), grid, block, smem, st, (const S *)a,
-                               (const S *)hx, (const S *)h, done, done_f32, (const E *)h0, (const S *)g,
-                               (const E *)g_last, (S *)da, (S *)db, (E *)dh0, (int)T, D, pl.tiles,
-                               pl.nw, a_ti, da_sum);
+        split_switch<E, MG, true, !std::is_same<S, E>::value>(pl, [&](auto vc, auto mw, auto ts) {
+            rc = launch_kernel((diag_scan_bwd_kernel<E, decltype(vc)::value, MG, decltype(mw)::value, S, decltype(ts)::value>), grid, block, smem,
+                               st, (const S *)a, (const S *)hx, (const S *)h, done, done_f32, (const E *)h0, (const S *)g, (const E *)g_last,
+                               (S *)da, (S *)db, (E *)dh0, (int)T, D, pl.tiles, pl.nw, a_ti, da_sum);
         });
     }
     return rc;
@@ -1316,8 +1365,7 @@ __global__ void __launch_bounds__(256) mingru_step_kernel(const S *__restrict__ 
     if (at >= n) return;
     const bool reset = done_at(done, done_f32, at / D);
     const Vec<float, VEC> zv = cvtv<S, float, VEC>(ldraw<S, VEC>(z + at)), xv = cvtv<S, float, VEC>(ldraw<S, VEC>(x + at));
-    Vec<float, VEC> gv = vfill<float, VEC>(0.f), ls = *reinterpret_cast<const Vec<float, VEC> *>(log_state + at),
-                    ld = *reinterpret_cast<const Vec<float, VEC> *>(log_decay + at), out;
+    Vec<float, VEC> gv = vfill<float, VEC>(0.f), ls = ldc<float, VEC>(log_state + at), ld = ldc<float, VEC>(log_decay + at), out;
     if (gate) gv = cvtv<S, float, VEC>(ldraw<S, VEC>(gate + at));
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
@@ -1330,8 +1378,8 @@ __global__ void __launch_bounds__(256) mingru_step_kernel(const S *__restrict__ 
         const float hs = (float)(S)h, g = gv.v[i];   // the state as the cell hands it on
         out.v[i] = gate ? hs * g / (1.f + __expf(-g)) : hs;
     }
-    *reinterpret_cast<Vec<float, VEC> *>(log_state_out + at) = ls;
-    *reinterpret_cast<Vec<float, VEC> *>(log_decay_out + at) = ld;
+    stc<float, VEC>(log_state_out + at, ls);
+    stc<float, VEC>(log_decay_out + at, ld);
     stv<S, float, VEC>(y + at, out);
 }
 
