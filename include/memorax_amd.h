@@ -151,6 +151,22 @@ int mrx_linear_scan_bwd(void *stream, const void *a, const void *h,
                         int64_t B, int64_t T, int64_t D, int dtype,
                         int done_dtype, int a_time_invariant);
 
+/* Long sequences over few columns leave most of the device idle when one workgroup walks each of them.  Where
+ * mrx_scan_workspace gives a size (bytes; 0: the shape is not served this way), the _segmented forms -- same
+ * arguments, same results -- take a workspace of that size, 8-byte aligned and overwritten, and cut time into
+ * segments of workgroups of their own.  `what`: any of the three flags below. */
+#define MRX_SCAN_BACKWARD 1
+#define MRX_SCAN_MINGRU 2
+#define MRX_SCAN_SUM_DA 4   /* backward with MRX_A_TIME_INVARIANT_SUM_DA */
+int64_t mrx_scan_workspace(int64_t B, int64_t T, int64_t D, int dtype, int what);
+int mrx_linear_scan_fwd_segmented(void *stream, const void *a, const void *b, const void *done, const void *h0,
+                                  const void *P0, void *h, void *h_last, void *P_last, int64_t B, int64_t T,
+                                  int64_t D, int dtype, int done_dtype, int a_time_invariant, void *workspace);
+int mrx_linear_scan_bwd_segmented(void *stream, const void *a, const void *h, const void *done, const void *h0,
+                                  const void *g, const void *g_last, void *da, void *db, void *dh0, int64_t B,
+                                  int64_t T, int64_t D, int dtype, int done_dtype, int a_time_invariant,
+                                  void *workspace);
+
 /* ---- causal linear attention, chunked ---------------------------------------
  * Replaces LinearAttentionCell.__call__ / binary_operator / read numerator
  * (linear_attention.py:62-86,105) scanned by memoroid.py:60-91, without
@@ -464,6 +480,14 @@ int mrx_mingru_scan_bwd(void *stream, const void *z, const void *h_tilde, const 
                         const void *done, const void *h0, const void *g, const void *g_last,
                         void *dz, void *dh_tilde, void *dh0, int64_t B, int64_t T, int64_t D,
                         int dtype, int done_dtype);
+/* with a workspace (see mrx_scan_workspace) */
+int mrx_mingru_scan_fwd_segmented(void *stream, const void *z, const void *h_tilde, const void *done, const void *h0,
+                                  const void *P0, void *h, void *h_last, void *P_last, int64_t B, int64_t T,
+                                  int64_t D, int dtype, int done_dtype, void *workspace);
+int mrx_mingru_scan_bwd_segmented(void *stream, const void *z, const void *h_tilde, const void *h, const void *done,
+                                  const void *h0, const void *g, const void *g_last, void *dz, void *dh_tilde,
+                                  void *dh0, int64_t B, int64_t T, int64_t D, int dtype, int done_dtype,
+                                  void *workspace);
 
 /* ---- Gated linear attention: linear attention with a scalar decay per step and head ----
  * The Mamba cell's algebra (mamba.py:109-122: elements (h_t = (B_t dt_t) (x) x_t, decay_t =

@@ -33,6 +33,11 @@ SIGNATURES = {
     "mrx_delta_chunk_size": (_L, [_I]),
     "mrx_linear_scan_fwd": (_I, [_P] * 9 + [_L] * 3 + [_I] * 3),
     "mrx_linear_scan_bwd": (_I, [_P] * 10 + [_L] * 3 + [_I] * 3),
+    "mrx_scan_workspace": (_L, [_L] * 3 + [_I] * 2),
+    "mrx_linear_scan_fwd_segmented": (_I, [_P] * 9 + [_L] * 3 + [_I] * 3 + [_P]),
+    "mrx_linear_scan_bwd_segmented": (_I, [_P] * 10 + [_L] * 3 + [_I] * 3 + [_P]),
+    "mrx_mingru_scan_fwd_segmented": (_I, [_P] * 9 + [_L] * 3 + [_I] * 2 + [_P]),
+    "mrx_mingru_scan_bwd_segmented": (_I, [_P] * 11 + [_L] * 3 + [_I] * 2 + [_P]),
     "mrx_linear_attn_fwd": (_I, [_P] * 9 + [_L] * 5 + [_I] * 3),
     "mrx_linear_attn_bwd": (_I, [_P] * 13 + [_L] * 5 + [_I] * 3),
     "mrx_linear_attn_fwd_chunk_parallel": (_I, [_P] * 9 + [_L] * 5 + [_I] * 3),

@@ -37,8 +37,8 @@ using torch::autograd::variable_list;
 
 // ------------------------------------------------------------------------------------------------ entry points
 #define MRX_BOUND(X)                                                                                                 \
-    X(mrx_status_string) X(mrx_chunk_size) X(mrx_delta_chunk_size) X(mrx_linear_scan_fwd) X(mrx_linear_scan_bwd)     \
-    X(mrx_linear_scan_last) X(mrx_mingru_scan_fwd) X(mrx_mingru_scan_bwd) X(mrx_mlstm_gates_fwd)                     \
+    X(mrx_status_string) X(mrx_chunk_size) X(mrx_delta_chunk_size) X(mrx_scan_workspace) X(mrx_linear_scan_fwd_segmented) X(mrx_linear_scan_bwd_segmented)     \
+    X(mrx_linear_scan_last) X(mrx_mingru_scan_fwd_segmented) X(mrx_mingru_scan_bwd_segmented) X(mrx_mlstm_gates_fwd)                     \
     X(mrx_mlstm_gates_bwd) X(mrx_rms_norm_fwd) X(mrx_rms_norm_bwd) X(mrx_layer_norm_fwd) X(mrx_layer_norm_bwd)       \
     X(mrx_silu_gate_fwd) X(mrx_silu_gate_bwd) X(mrx_linear_attn_fwd) X(mrx_linear_attn_bwd)                          \
     X(mrx_linear_attn_fwd_chunk_parallel) X(mrx_linear_attn_bwd_chunk_parallel)                                      \
@@ -142,6 +142,13 @@ void chk_scan_dtype(ScalarType dt, bool complex, const char *what)
                       complex ? "complex64 and bfloat16" : "bfloat16");
 }
 
+// scratch for the scans that cut time into segments; undefined (a null pointer) where the shape is not served that way
+Tensor scan_workspace(const Tensor &x, int64_t B, int64_t T, int64_t D, ScalarType dt, int what)
+{
+    const int64_t bytes = lib.mrx_scan_workspace(B, T, D, code(dt), what);
+    return bytes ? fresh({bytes}, at::kByte, x) : Tensor();
+}
+
 ScanOut scan_fwd(const Tensor &a, const Tensor &b, const Tensor &done_, const OptTensor &h0, const OptTensor &P0, bool want_P)
 {
     TORCH_CHECK_VALUE(b.dim() == 3, "b must be (B,T,D)");
@@ -157,8 +164,9 @@ ScanOut scan_fwd(const Tensor &a, const Tensor &b, const Tensor &done_, const Op
     chk(P0, "P0", ct, {B, D});
     const Done done(done_, B, T);
     ScanOut r{fresh_like(b), fresh({B, D}, ct, b), want_P ? fresh({B, D}, ct, b) : Tensor()};
-    check(lib.mrx_linear_scan_fwd(stream(), ptr(a), ptr(b), done.p(), ptr(h0), ptr(P0), ptr(r.h), ptr(r.h_last), ptr(r.P_last), B, T, D,
-                                  code(dt), done.dtype, ti),
+    const Tensor workspace = scan_workspace(b, B, T, D, dt, 0);
+    check(lib.mrx_linear_scan_fwd_segmented(stream(), ptr(a), ptr(b), done.p(), ptr(h0), ptr(P0), ptr(r.h), ptr(r.h_last), ptr(r.P_last), B, T, D,
+                                  code(dt), done.dtype, ti, ptr(workspace)),
           "mrx_linear_scan_fwd");
     return r;
 }
@@ -185,8 +193,9 @@ ScanGrads scan_bwd(const Tensor &a, const Tensor &h, const Tensor &done_, const 
     const Done done(done_, B, T);
     TORCH_CHECK_VALUE(ti || !sum_da, "sum_da belongs to a time-invariant a");
     ScanGrads r{sum_da ? fresh({B, D}, ct, g) : fresh_like(g), fresh_like(g), fresh({B, D}, ct, g)};
-    check(lib.mrx_linear_scan_bwd(stream(), ptr(a), ptr(h), done.p(), ptr(h0), ptr(g), ptr(g_last), ptr(r.da), ptr(r.db), ptr(r.dh0), B, T, D,
-                                  code(dt), done.dtype, sum_da ? MRX_A_TIME_INVARIANT_SUM_DA : int(ti)),
+    const Tensor workspace = scan_workspace(g, B, T, D, dt, MRX_SCAN_BACKWARD | (sum_da ? MRX_SCAN_SUM_DA : 0));
+    check(lib.mrx_linear_scan_bwd_segmented(stream(), ptr(a), ptr(h), done.p(), ptr(h0), ptr(g), ptr(g_last), ptr(r.da), ptr(r.db), ptr(r.dh0), B, T, D,
+                                  code(dt), done.dtype, sum_da ? MRX_A_TIME_INVARIANT_SUM_DA : int(ti), ptr(workspace)),
           "mrx_linear_scan_bwd");
     return r;
 }
@@ -221,8 +230,9 @@ ScanOut mingru_fwd(const Tensor &z, const Tensor &x, const Tensor &done_, const 
     chk(P0, "P0", at::kFloat, {B, D});
     const Done done(done_, B, T);
     ScanOut r{fresh_like(z), fresh({B, D}, at::kFloat, z), want_P ? fresh({B, D}, at::kFloat, z) : Tensor()};
-    check(lib.mrx_mingru_scan_fwd(stream(), ptr(z), ptr(x), done.p(), fptr(h0), fptr(P0), ptr(r.h), fptr(r.h_last), fptr(r.P_last), B, T, D,
-                                  code(dt), done.dtype),
+    const Tensor workspace = scan_workspace(z, B, T, D, dt, MRX_SCAN_MINGRU);
+    check(lib.mrx_mingru_scan_fwd_segmented(stream(), ptr(z), ptr(x), done.p(), fptr(h0), fptr(P0), ptr(r.h), fptr(r.h_last), fptr(r.P_last), B, T, D,
+                                  code(dt), done.dtype, ptr(workspace)),
           "mrx_mingru_scan_fwd");
     return r;
 }
@@ -242,8 +252,9 @@ ScanGrads mingru_bwd(const Tensor &z, const Tensor &x, const Tensor &h, const Te
     chk(g_last, "g_last", at::kFloat, {B, D});
     const Done done(done_, B, T);
     ScanGrads r{fresh_like(g), fresh_like(g), fresh({B, D}, at::kFloat, g)};
-    check(lib.mrx_mingru_scan_bwd(stream(), ptr(z), ptr(x), ptr(h), done.p(), fptr(h0), ptr(g), fptr(g_last), ptr(r.da), ptr(r.db),
-                                  fptr(r.dh0), B, T, D, code(dt), done.dtype),
+    const Tensor workspace = scan_workspace(g, B, T, D, dt, MRX_SCAN_MINGRU | MRX_SCAN_BACKWARD);
+    check(lib.mrx_mingru_scan_bwd_segmented(stream(), ptr(z), ptr(x), ptr(h), done.p(), fptr(h0), ptr(g), fptr(g_last), ptr(r.da), ptr(r.db),
+                                  fptr(r.dh0), B, T, D, code(dt), done.dtype, ptr(workspace)),
           "mrx_mingru_scan_bwd");
     return r;
 }

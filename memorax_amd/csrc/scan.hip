@@ -235,18 +235,74 @@ struct MinGru {
 
 constexpr int TS_MIN = 8;  // time steps a wave holds in registers per super-step (template parameter TS of the kernels), at least
 
-// Forward.  grid = B * tiles workgroups, block = 64 * NW threads, NW <= MAXW (8, or 16 for the
+// Long sequences over few columns: time is cut into n segments of `steps` steps (a multiple of a super-step), each a workgroup
+// of its own.  A first launch (SEG = SUMMARISE) reads the two arrays the recurrence itself needs and leaves every segment's
+// composed step -- state from zero, product of the coefficients, "holds a reset" -- in the workspace; the second (SEG = APPLY)
+// composes those of the segments before its own into the state it starts from, and does the work.  Twice the reads of two
+// arrays, most of them from the last-level cache, against a chain of T / 128 trips to memory that leaves most of the device
+// idle.  Backward the same with time reversed.
+enum Segmented { WHOLE, SUMMARISE, APPLY };
+template <typename E> struct Segments {
+    int n, steps;
+    E *state, *product;  // (n, B, D)
+    int *cut;            // (n, B)
+    E *da_parts;         // (n, B, D): da_sum, a segment's share of it
+};
+
+// The summaries of the segments before `seg`, composed: each wave takes a contiguous share of them (its loads all in flight at
+// once) and leaves its result where a super-step's waves leave theirs, for fold_waves to carry the state through.
+template <typename E, int VEC, int MAXSEG>
+__device__ __forceinline__ void compose_segments(const Segments<E> &sg, int seg, int64_t bi, int64_t B, int64_t D, int64_t col, bool act, int w,
+                                                 int NW, Vec<E, VEC> &hc, Vec<E, VEC> &pc, bool &cut)
+{
+    using V = Vec<E, VEC>;
+    using O = Ops<E>;
+    constexpr int PER = MAXSEG / 8;  // NW is 8
+    const int per = (seg + NW - 1) / NW, j0 = w * per;
+    V hs[PER], ps[PER];
+    int fs[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        hs[i] = vfill<E, VEC>(O::zero());
+        ps[i] = vfill<E, VEC>(O::one());
+        fs[i] = 0;
+        if (i < per && j0 + i < seg && act) {
+            const int64_t row = (int64_t)(j0 + i) * B + bi;
+            hs[i] = ldc<E, VEC>(sg.state + row * D + col);
+            ps[i] = ldc<E, VEC>(sg.product + row * D + col);
+            fs[i] = sg.cut[row];
+        }
+    }
+    hc = vfill<E, VEC>(O::zero());
+    pc = vfill<E, VEC>(O::one());
+    cut = false;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const bool f = fs[i] != 0;
+        cut |= f;
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) {
+            const E hn = O::madd(ps[i].v[k], hc.v[k], hs[i].v[k]);
+            const E pn = O::mul(ps[i].v[k], pc.v[k]);
+            hc.v[k] = f ? hs[i].v[k] : hn;
+            pc.v[k] = f ? ps[i].v[k] : pn;
+        }
+    }
+}
+constexpr int MAX_SEGMENTS = 64;
+
+// Forward.  grid = B * tiles workgroups (times the segments), block = 64 * NW threads, NW <= MAXW (8, or 16 for the
 // one-vector-lane instances that small shapes take: with 16 waves of 8 steps a sequence of up to 128
 // steps is one super-step, every load of the workgroup in flight at once and a single barrier).
 // smem: sH[2][NW][64] Vec, sP[2][NW][64] Vec, sF[2][NW] int.
-template <typename E, int VEC, bool MG = false, int MAXW = 8, typename S = E, int TS = TS_MIN>
+template <typename E, int VEC, bool MG = false, int MAXW = 8, typename S = E, int TS = TS_MIN, int SEG = WHOLE>
 __global__ void __launch_bounds__(64 * MAXW)
 diag_scan_fwd_kernel(const S *__restrict__ a, const S *__restrict__ b,
                      const void *__restrict__ done, int done_f32,
                      const E *__restrict__ h0, const E *__restrict__ P0,
                      S *__restrict__ h, E *__restrict__ h_last,
                      E *__restrict__ P_last, int T, int64_t D, int tiles, int NW,
-                     int a_ti)
+                     int a_ti, Segments<E> sg)
 {
     using V = Vec<E, VEC>;
     using O = Ops<E>;
@@ -259,20 +315,46 @@ diag_scan_fwd_kernel(const S *__restrict__ a, const S *__restrict__ b,
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int tile = blockIdx.x % tiles;
-    const int64_t bi = blockIdx.x / tiles;
+    const int64_t bs = blockIdx.x / tiles;
+    const int64_t bi = SEG == WHOLE ? bs : bs / sg.n;
+    const int seg = SEG == WHOLE ? 0 : (int)(bs % sg.n);
+    [[maybe_unused]] const int64_t B = SEG == WHOLE ? 0 : (int64_t)gridDim.x / ((int64_t)tiles * sg.n);
+    const int t_begin = SEG == WHOLE ? 0 : seg * sg.steps, t_end = SEG == WHOLE || T - t_begin <= sg.steps ? T : t_begin + sg.steps;
     const bool act = ((int64_t)tile * 64 + lane) * VEC < D;
     const int64_t col = first_col<VEC>((int64_t)tile * 64 + lane, D);
     const int64_t row0 = bi * T;
 
     V carry_h = vfill<E, VEC>(O::zero()), carry_p = vfill<E, VEC>(O::one());
-    if (act) {
+    if (act && SEG != SUMMARISE) {
         if (h0) carry_h = ldc<E, VEC>(h0 + bi * D + col);
         if (P0) carry_p = ldc<E, VEC>(P0 + bi * D + col);
     }
 
-    const int span = NW * TS;
     int buf = 0;
-    for (int t0 = 0; t0 < T; t0 += span) {
+    [[maybe_unused]] bool seg_cut = false;
+    if constexpr (SEG == APPLY) {
+        V hc, pc;
+        bool cut;
+        compose_segments<E, VEC, MAX_SEGMENTS>(sg, seg, bi, B, D, col, act, w, NW, hc, pc, cut);
+        sH[w * 64 + lane].x = hc;
+        sP[w * 64 + lane].x = pc;
+        if (lane == 0) sF[w] = cut;
+        __syncthreads();
+        for (int j = 0; j < NW; ++j) {
+            const V Hj = sH[j * 64 + lane].x, Pj = sP[j * 64 + lane].x;
+            const bool fj = sF[j] != 0;
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) {
+                const E hn = O::madd(Pj.v[i], carry_h.v[i], Hj.v[i]);
+                const E pn = O::mul(Pj.v[i], carry_p.v[i]);
+                carry_h.v[i] = fj ? Hj.v[i] : hn;
+                carry_p.v[i] = fj ? Pj.v[i] : pn;
+            }
+        }
+        buf = 1;
+    }
+    const int span = NW * TS;
+    for (int t0 = t_begin; t0 < t_end; t0 += span) {
         const int ts = t0 + w * TS;
         V x[TS], p[TS];
         // reset flags of the wave's TS steps: lane s fetches the flag of step ts + s, one ballot makes the mask
@@ -351,6 +433,7 @@ diag_scan_fwd_kernel(const S *__restrict__ a, const S *__restrict__ b,
             const V Hj = sH[(buf * NW + j) * 64 + lane].x;
             const V Pj = sP[(buf * NW + j) * 64 + lane].x;
             const bool fj = sF[buf * NW + j] != 0;
+            if constexpr (SEG == SUMMARISE) seg_cut |= fj;
 #pragma unroll
             for (int i = 0; i < VEC; ++i) {
                 const E hn = O::madd(Pj.v[i], cin_h.v[i], Hj.v[i]);
@@ -370,12 +453,21 @@ diag_scan_fwd_kernel(const S *__restrict__ a, const S *__restrict__ b,
                 const E fx = O::madd(p[s].v[i], my_h.v[i], x[s].v[i]);
                 out.v[i] = seen ? x[s].v[i] : fx;
             }
-            if (ts + s < T && act)
+            if (SEG != SUMMARISE && ts + s < T && act)
                 stv<S, E, VEC>(h + (row0 + ts + s) * D + col, out);
         }
         buf ^= 1;
     }
-    if (w == 0 && act) {
+    if constexpr (SEG == SUMMARISE) {
+        if (w == 0 && act) {
+            const int64_t row = (int64_t)seg * B + bi;
+            stc<E, VEC>(sg.state + row * D + col, carry_h);
+            stc<E, VEC>(sg.product + row * D + col, carry_p);
+            if (lane == 0) sg.cut[row] = seg_cut;
+        }
+        return;
+    }
+    if (w == 0 && act && t_end == T) {
         if (h_last) stc<E, VEC>(h_last + bi * D + col, carry_h);
         if (P_last) stc<E, VEC>(P_last + bi * D + col, carry_p);
     }
@@ -384,14 +476,14 @@ diag_scan_fwd_kernel(const S *__restrict__ a, const S *__restrict__ b,
 // Backward: the same scan walked from t = T-1 down with coefficient conj(a_{t+1}),
 // cut where done_{t+1}; reversed index r = T-1-t runs forward.
 // MG: a holds z, hx holds x = h~; da receives dz and db receives dx.
-template <typename E, int VEC, bool MG = false, int MAXW = 8, typename S = E, int TS = TS_MIN>
+template <typename E, int VEC, bool MG = false, int MAXW = 8, typename S = E, int TS = TS_MIN, int SEG = WHOLE>
 __global__ void __launch_bounds__(64 * MAXW)
 diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S *__restrict__ hfw,
                      const void *__restrict__ done, int done_f32,
                      const E *__restrict__ h0, const S *__restrict__ g,
                      const E *__restrict__ g_last, S *__restrict__ da,
                      S *__restrict__ db, E *__restrict__ dh0, int T, int64_t D,
-                     int tiles, int NW, int a_ti, int da_sum)
+                     int tiles, int NW, int a_ti, int da_sum, Segments<E> sg)
 {
     using V = Vec<E, VEC>;
     using O = Ops<E>;
@@ -404,20 +496,45 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int tile = blockIdx.x % tiles;
-    const int64_t bi = blockIdx.x / tiles;
+    const int64_t bs = blockIdx.x / tiles;
+    const int64_t bi = SEG == WHOLE ? bs : bs / sg.n;
+    const int seg = SEG == WHOLE ? 0 : (int)(bs % sg.n);
+    [[maybe_unused]] const int64_t B = SEG == WHOLE ? 0 : (int64_t)gridDim.x / ((int64_t)tiles * sg.n);
+    const int r_begin = SEG == WHOLE ? 0 : seg * sg.steps, r_end = SEG == WHOLE || T - r_begin <= sg.steps ? T : r_begin + sg.steps;
     const bool act = ((int64_t)tile * 64 + lane) * VEC < D;
     const int64_t col = first_col<VEC>((int64_t)tile * 64 + lane, D);
     const int64_t row0 = bi * T;
 
     V carry = vfill<E, VEC>(O::zero());  // lam_{t+1} entering from the right
-    if (act && g_last) carry = ldc<E, VEC>(g_last + bi * D + col);
+    if (act && g_last && SEG != SUMMARISE) carry = ldc<E, VEC>(g_last + bi * D + col);
     // da_sum (time-invariant a): da is (B,D), the sum of the per-step terms over the sequence -- what the
     // gradient of a broadcast coefficient needs -- kept in registers instead of written per step
     V dsum = vfill<E, VEC>(O::zero());
 
-    const int span = NW * TS;
+    [[maybe_unused]] V seg_p = vfill<E, VEC>(O::one());
+    [[maybe_unused]] bool seg_cut = false;
     int buf = 0;
-    for (int r0 = 0; r0 < T; r0 += span) {
+    if constexpr (SEG == APPLY) {
+        V lc, pc;
+        bool cut;
+        compose_segments<E, VEC, MAX_SEGMENTS>(sg, seg, bi, B, D, col, act, w, NW, lc, pc, cut);
+        sH[w * 64 + lane].x = lc;
+        sP[w * 64 + lane].x = pc;
+        if (lane == 0) sF[w] = cut;
+        __syncthreads();
+        for (int j = 0; j < NW; ++j) {
+            const V Hj = sH[j * 64 + lane].x, Pj = sP[j * 64 + lane].x;
+            const bool fj = sF[j] != 0;
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) {
+                const E ln = O::madd(Pj.v[i], carry.v[i], Hj.v[i]);
+                carry.v[i] = fj ? Hj.v[i] : ln;
+            }
+        }
+        buf = 1;
+    }
+    const int span = NW * TS;
+    for (int r0 = r_begin; r0 < r_end; r0 += span) {
         const int rs = r0 + w * TS;
         // Everything the super-step reads is requested here, before the barrier: h_{t-1} (and the
         // MinGRU projections of step t) are only needed once lam_t is known, but a load issued after the
@@ -451,6 +568,7 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
 #pragma unroll
                         for (int i = 0; i < VEC; ++i) p[s].v[i] = MG ? av.v[i] : O::conj(av.v[i]);  // MG: z_{t+1} for now
                     }
+                    if (SEG == SUMMARISE) continue;
                     if (t > 0)
                         hp[s] = ldv<S, E, VEC>(hfw + off - D);
                     else if (h0)
@@ -465,7 +583,7 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
             // narrower storage: the values wait as stored and are widened once every load has been issued
             raw_t<S, VEC> rg[TS], ra[TS], rh[TS], rz[MG ? TS : 1], rxt[MG ? TS : 1];
             V h0v = vfill<E, VEC>(O::zero());  // h_{-1}: what step 0 multiplies its lam with
-            if (act && h0 && T - 1 - rs - (TS - 1) <= 0) h0v = ldc<E, VEC>(h0 + bi * D + col);
+            if (SEG != SUMMARISE && act && h0 && T - 1 - rs - (TS - 1) <= 0) h0v = ldc<E, VEC>(h0 + bi * D + col);
 #pragma unroll
             for (int s = 0; s < TS; ++s) {
                 const int t = T - 1 - (rs + s);
@@ -473,6 +591,7 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
                     const int64_t off = (row0 + t) * D + col;
                     rg[s] = ldraw<S, VEC>(g + off);
                     if (t + 1 < T) ra[s] = ldraw<S, VEC>(a + (a_ti ? col : off + D));
+                    if (SEG == SUMMARISE) continue;
                     if (t > 0) rh[s] = ldraw<S, VEC>(hfw + off - D);
                     if constexpr (MG) {
                         rz[s] = ldraw<S, VEC>(a + off);
@@ -493,6 +612,7 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
 #pragma unroll
                         for (int i = 0; i < VEC; ++i) p[s].v[i] = MG ? av.v[i] : O::conj(av.v[i]);  // MG: z_{t+1} for now
                     }
+                    if (SEG == SUMMARISE) continue;
                     if (t > 0) hp[s] = cvtv<S, E, VEC>(rh[s]);
                     else hp[s] = h0v;
                     if constexpr (MG) {
@@ -552,10 +672,15 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
                 const V Hj = sH[(buf * NW + j) * 64 + lane].x;
                 const V Pj = sP[(buf * NW + j) * 64 + lane].x;
                 const bool fj = sF[buf * NW + j] != 0;
+                if constexpr (SEG == SUMMARISE) seg_cut |= fj;
 #pragma unroll
                 for (int i = 0; i < VEC; ++i) {
                     const E ln = O::madd(Pj.v[i], cin.v[i], Hj.v[i]);
                     cin.v[i] = fj ? Hj.v[i] : ln;
+                    if constexpr (SEG == SUMMARISE) {
+                        const E pn = O::mul(Pj.v[i], seg_p.v[i]);
+                        seg_p.v[i] = fj ? Pj.v[i] : pn;
+                    }
                 }
             }
             carry = cin;
@@ -570,6 +695,7 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
             }
             buf ^= 1;
         }
+        if constexpr (SEG == SUMMARISE) continue;
         // x[s] = lam_t : emit db_t and da_t = done_t ? 0 : lam_t conj(h_{t-1})
 #pragma unroll
         for (int s = 0; s < TS; ++s) {
@@ -601,6 +727,15 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
             }
         }
     }
+    if constexpr (SEG == SUMMARISE) {
+        if (w == 0 && act) {
+            const int64_t row = (int64_t)seg * B + bi;
+            stc<E, VEC>(sg.state + row * D + col, carry);
+            stc<E, VEC>(sg.product + row * D + col, seg_p);
+            if (lane == 0) sg.cut[row] = seg_cut;
+        }
+        return;
+    }
     if (!MG && da_sum) {  // uniform over the workgroup
         if (NW > 1) {
             __syncthreads();  // the last fold has read sH
@@ -614,9 +749,10 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
                 }
             }
         }
-        if (w == 0 && act) stc<E, VEC>(reinterpret_cast<E *>(da) + bi * D + col, dsum);  // (B,D), arithmetic type
+        E *const sum = SEG == APPLY ? sg.da_parts + (int64_t)seg * B * D : reinterpret_cast<E *>(da);  // (B,D), arithmetic type
+        if (w == 0 && act) stc<E, VEC>(sum + bi * D + col, dsum);
     }
-    if (w == 0 && act && dh0) {
+    if (w == 0 && act && dh0 && r_end == T) {
         // carry = lam_0 ; dh0 = done_0 ? 0 : conj(a_0) lam_0
         const bool d0 = done_at(done, done_f32, row0);
         V a0 = ldv<S, E, VEC>(a + (a_ti ? col : row0 * D + col));
@@ -1070,6 +1206,71 @@ ScanPlan plan_scan(int64_t B, int64_t T, int64_t D, size_t esize, bool bwd, bool
     return {vec, stream ? 1 : nw, tiles, stream};
 }
 
+struct SegmentPlan {
+    int vec = 1, tiles = 0, n = 0, steps = 0, ts = TS_MIN;  // n = 0: not in segments
+};
+
+// When to cut time into segments, and how many: from a sweep over twenty shapes of 4..256 sequences x 250..4000 steps x 64..560
+// columns for every kind of scan.  One walk per column group costs a trip to memory per super-step, whatever the number of
+// columns; the segments cost a second launch (3 us) and the second reading.  So: few columns (in units of a wave, `cols`), and
+// steps enough per column unit -- the line T >= 9 cols forward and 4 cols backward, whose first pass reads two arrays of the
+// four or five.  Time in us, one walk -> segments, forward and backward: float32 8 x 1000 x 64 31 -> 14 and 57 -> 15, 16 x 4000 x 256
+// 114 -> 68 and 219 -> 90, 32 x 512 x 256 backward 34 -> 28, 57 x 2908 x 120 104 -> 110 (left out) and 194 -> 125; bfloat16 16 x 4000 x 256
+// 109 -> 50 and 210 -> 68, with the MinGRU map 320 -> 92 backward; complex64 16 x 2690 x 192 150 -> 73 and 260 -> 115.
+SegmentPlan plan_segments(int64_t B, int64_t T, int64_t D, size_t esize, bool bwd, bool mg, bool half_storage)
+{
+    SegmentPlan p;
+    auto tiles = [&](int64_t v) { return (D + 64 * v - 1) / (64 * v); };
+    const int64_t cols = B * tiles(1);
+    if (!bwd) {
+        const int64_t most = half_storage || esize == 8 ? 128 : 80;   // 57 x 2908 x 120 (cols 114): see above
+        if (cols > most || T < 9 * cols || T < (esize == 8 ? 256 : 384)) return p;
+    } else {
+        int64_t most = 192, per = 4;   // 20 x 1250 x 551 (cols 180) 120 -> 109, 49 x 1474 x 300 (245) 160 -> 162
+        if (esize == 8) most = 128, per = 5;               // 20 x 1250 x 551 188 -> 204
+        else if (half_storage && mg) most = 256;           // 49 x 1474 x 300 181 -> 159
+        else if (half_storage && D <= 64) per = 9;         // 128 x 1024 x 64 56 -> 60, 75 x 679 x 64 45 -> 32
+        else if (!half_storage && D <= 64) most = 128;     // 128 x 1024 x 64 62 -> 55, 189 x 1264 x 64 80 -> 92
+        if (cols > most || T < per * cols || T < 256) return p;
+    }
+    // two elements per lane where a row fills more than three quarters of its waves with them: bfloat16, and backward
+    // (57 x 2908 x 120 192 -> 125 us; rows of 192, three quarters, 57 -> 63 us)
+    if (D > 64 && (half_storage || (bwd && esize == 4 && 4 * D > 3 * 128 * tiles(2)))) p.vec = 2;
+    if (bwd && half_storage && !mg && p.vec == 2) p.ts = 16;
+    p.tiles = (int)tiles(p.vec);
+    const int64_t span = 8 * p.ts;
+    // a thousand workgroups in all, at most MAX_SEGMENTS per sequence
+    int64_t n = (1024 + B * p.tiles - 1) / (B * p.tiles);
+    n = n > MAX_SEGMENTS ? MAX_SEGMENTS : n;
+    const int64_t steps = ((T + n - 1) / n + span - 1) / span * span;
+    n = (T + steps - 1) / steps;
+    if (n < 2) return p;
+    p.n = (int)n;
+    p.steps = (int)steps;
+    return p;
+}
+
+template <typename E> size_t segment_bytes(const SegmentPlan &p, int64_t B, int64_t D, bool da_sum)
+{
+    return (size_t)p.n * B * (D * sizeof(E) * (da_sum ? 3 : 2) + sizeof(int));
+}
+template <typename E> Segments<E> segments_in(const SegmentPlan &p, int64_t B, int64_t D, bool da_sum, void *workspace)
+{
+    E *const w = reinterpret_cast<E *>(workspace);
+    const int64_t one = (int64_t)p.n * B * D;
+    return {p.n, p.steps, w, w + one, reinterpret_cast<int *>(w + (da_sum ? 3 : 2) * one), da_sum ? w + 2 * one : nullptr};
+}
+
+// The shares of the segments summed (da_sum): one thread per element of (B, D).
+template <typename E> __global__ void __launch_bounds__(256) segment_sum_kernel(const E *__restrict__ parts, E *__restrict__ out, int n, int64_t BD)
+{
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= BD) return;
+    E s = Ops<E>::zero();
+    for (int j = 0; j < n; ++j) s = Ops<E>::madd(Ops<E>::one(), s, parts[(int64_t)j * BD + i]);
+    out[i] = s;
+}
+
 size_t scan_smem(int nw, size_t vbytes)
 {
     return nw == 1 ? 0 : 2 * (size_t)nw * 64 * vbytes * 2 + 2 * (size_t)nw * sizeof(int);
@@ -1110,13 +1311,42 @@ template <typename E, bool MG, bool BWD, bool HALF, typename F> void split_switc
     });
 }
 
+// The kernels over segments that plan_segments asks for: f(VEC, TS); eight waves each.
+template <typename E, bool MG, bool BWD, bool HALF, typename F> void segment_switch(const SegmentPlan &pl, F f)
+{
+    using std::integral_constant;
+    if constexpr (HALF || (BWD && sizeof(E) == 4)) {
+        if (pl.vec == 2) return f(integral_constant<int, 2>{}, integral_constant<int, BWD && HALF && !MG ? 16 : TS_MIN>{});
+    }
+    f(integral_constant<int, 1>{}, integral_constant<int, TS_MIN>{});
+}
+
 // MG (E = float): a and b hold the MinGRU projections z and h~.
 // S: storage type of the (B,T,D) arrays (E, or __bf16 with E = float).
 template <typename E, bool MG = false, typename S = E>
 int launch_fwd(hipStream_t st, const void *a, const void *b, const void *done,
                int done_f32, const void *h0, const void *P0, void *h, void *h_last,
-               void *P_last, int64_t B, int64_t T, int64_t D, int a_ti)
+               void *P_last, int64_t B, int64_t T, int64_t D, int a_ti, void *workspace)
 {
+    if (const SegmentPlan sp = workspace ? plan_segments(B, T, D, sizeof(E), false, MG, !std::is_same<S, E>::value) : SegmentPlan{}; sp.n) {
+        Segments<E> sg = segments_in<E>(sp, B, D, false, workspace);
+        const dim3 block(512);
+        const size_t smem = scan_smem(8, sizeof(E) * sp.vec);
+        int rc = MRX_ERR_LAUNCH;
+        segment_switch<E, MG, false, !std::is_same<S, E>::value>(sp, [&](auto vc, auto ts) {
+            constexpr int VEC = decltype(vc)::value, TS = decltype(ts)::value;
+            sg.n = sp.n - 1;
+            rc = launch_kernel((diag_scan_fwd_kernel<E, VEC, MG, 8, S, TS, SUMMARISE>), dim3((unsigned)(B * sp.tiles * sg.n)), block, smem, st,
+                               (const S *)a, (const S *)b, done, done_f32, (const E *)nullptr, (const E *)nullptr, (S *)nullptr, (E *)nullptr,
+                               (E *)nullptr, (int)T, D, sp.tiles, 8, a_ti, sg);
+            if (rc != MRX_OK) return;
+            sg.n = sp.n;
+            rc = launch_kernel((diag_scan_fwd_kernel<E, VEC, MG, 8, S, TS, APPLY>), dim3((unsigned)(B * sp.tiles * sg.n)), block, smem, st,
+                               (const S *)a, (const S *)b, done, done_f32, (const E *)h0, (const E *)P0, (S *)h, (E *)h_last, (E *)P_last,
+                               (int)T, D, sp.tiles, 8, a_ti, sg);
+        });
+        return rc;
+    }
     const ScanPlan pl = plan_scan(B, T, D, sizeof(E), false, MG, !std::is_same<S, E>::value, a_ti);
     int rc = MRX_ERR_LAUNCH;
     if (pl.stream) {
@@ -1138,7 +1368,7 @@ int launch_fwd(hipStream_t st, const void *a, const void *b, const void *done,
         split_switch<E, MG, false, !std::is_same<S, E>::value>(pl, [&](auto vc, auto mw, auto ts) {
             rc = launch_kernel((diag_scan_fwd_kernel<E, decltype(vc)::value, MG, decltype(mw)::value, S, decltype(ts)::value>), grid, block, smem,
                                st, (const S *)a, (const S *)b, done, done_f32, (const E *)h0, (const E *)P0, (S *)h, (E *)h_last, (E *)P_last,
-                               (int)T, D, pl.tiles, pl.nw, a_ti);
+                               (int)T, D, pl.tiles, pl.nw, a_ti, Segments<E>{});
         });
     }
     return rc;
@@ -1148,8 +1378,30 @@ int launch_fwd(hipStream_t st, const void *a, const void *b, const void *done,
 template <typename E, bool MG = false, typename S = E>
 int launch_bwd(hipStream_t st, const void *a, const void *hx, const void *h, const void *done,
                int done_f32, const void *h0, const void *g, const void *g_last, void *da,
-               void *db, void *dh0, int64_t B, int64_t T, int64_t D, int a_ti, int da_sum = 0)
+               void *db, void *dh0, int64_t B, int64_t T, int64_t D, int a_ti, int da_sum, void *workspace)
 {
+    if (const SegmentPlan sp = workspace ? plan_segments(B, T, D, sizeof(E), true, MG, !std::is_same<S, E>::value) : SegmentPlan{}; sp.n) {
+        Segments<E> sg = segments_in<E>(sp, B, D, da_sum, workspace);
+        const dim3 block(512);
+        const size_t smem = scan_smem(8, sizeof(E) * sp.vec);
+        int rc = MRX_ERR_LAUNCH;
+        segment_switch<E, MG, true, !std::is_same<S, E>::value>(sp, [&](auto vc, auto ts) {
+            constexpr int VEC = decltype(vc)::value, TS = decltype(ts)::value;
+            sg.n = sp.n - 1;
+            rc = launch_kernel((diag_scan_bwd_kernel<E, VEC, MG, 8, S, TS, SUMMARISE>), dim3((unsigned)(B * sp.tiles * sg.n)), block, smem, st,
+                               (const S *)a, (const S *)nullptr, (const S *)nullptr, done, done_f32, (const E *)nullptr, (const S *)g,
+                               (const E *)nullptr, (S *)nullptr, (S *)nullptr, (E *)nullptr, (int)T, D, sp.tiles, 8, a_ti, 0, sg);
+            if (rc != MRX_OK) return;
+            sg.n = sp.n;
+            rc = launch_kernel((diag_scan_bwd_kernel<E, VEC, MG, 8, S, TS, APPLY>), dim3((unsigned)(B * sp.tiles * sg.n)), block, smem, st,
+                               (const S *)a, (const S *)hx, (const S *)h, done, done_f32, (const E *)h0, (const S *)g, (const E *)g_last,
+                               (S *)da, (S *)db, (E *)dh0, (int)T, D, sp.tiles, 8, a_ti, da_sum, sg);
+        });
+        if (rc == MRX_OK && da_sum)
+            rc = launch_kernel(segment_sum_kernel<E>, dim3((unsigned)((B * D + 255) / 256)), dim3(256), 0, st, (const E *)sg.da_parts, (E *)da,
+                               sp.n, B * D);
+        return rc;
+    }
     const ScanPlan pl = plan_scan(B, T, D, sizeof(E), true, MG, !std::is_same<S, E>::value, a_ti);
     int rc = MRX_ERR_LAUNCH;
     if (pl.stream) {
@@ -1183,7 +1435,7 @@ int launch_bwd(hipStream_t st, const void *a, const void *hx, const void *h, con
         split_switch<E, MG, true, !std::is_same<S, E>::value>(pl, [&](auto vc, auto mw, auto ts) {
             rc = launch_kernel((diag_scan_bwd_kernel<E, decltype(vc)::value, MG, decltype(mw)::value, S, decltype(ts)::value>), grid, block, smem,
                                st, (const S *)a, (const S *)hx, (const S *)h, done, done_f32, (const E *)h0, (const S *)g, (const E *)g_last,
-                               (S *)da, (S *)db, (E *)dh0, (int)T, D, pl.tiles, pl.nw, a_ti, da_sum);
+                               (S *)da, (S *)db, (E *)dh0, (int)T, D, pl.tiles, pl.nw, a_ti, da_sum, Segments<E>{});
         });
     }
     return rc;
@@ -1222,10 +1474,19 @@ bool scan_shape_ok(int64_t B, int64_t T, int64_t D)
 
 }  // namespace
 
-extern "C" int mrx_linear_scan_fwd(void *stream, const void *a, const void *b, const void *done,
-                                   const void *h0, const void *P0, void *h, void *h_last,
-                                   void *P_last, int64_t B, int64_t T, int64_t D, int dtype,
-                                   int done_dtype, int a_time_invariant)
+extern "C" int64_t mrx_scan_workspace(int64_t B, int64_t T, int64_t D, int dtype, int what)
+{
+    if (!scan_shape_ok(B, T, D) || dtype < MRX_F32 || dtype > MRX_C64) return 0;
+    const bool bwd = what & MRX_SCAN_BACKWARD, mg = what & MRX_SCAN_MINGRU, da_sum = what & MRX_SCAN_SUM_DA;
+    const SegmentPlan p = plan_segments(B, T, D, dtype == MRX_C64 ? 8 : 4, bwd, mg, dtype == MRX_BF16);
+    if (!p.n) return 0;
+    return (int64_t)(dtype == MRX_C64 ? segment_bytes<c64>(p, B, D, bwd && da_sum) : segment_bytes<float>(p, B, D, bwd && da_sum));
+}
+
+namespace {
+
+int linear_scan_fwd(void *stream, const void *a, const void *b, const void *done, const void *h0, const void *P0, void *h, void *h_last,
+                    void *P_last, int64_t B, int64_t T, int64_t D, int dtype, int done_dtype, int a_time_invariant, void *workspace)
 {
     if (!a || !b || !done || !h) return MRX_ERR_INVALID_ARG;
     if (!scan_shape_ok(B, T, D)) return MRX_ERR_INVALID_ARG;
@@ -1235,27 +1496,45 @@ extern "C" int mrx_linear_scan_fwd(void *stream, const void *a, const void *b, c
     const int ti = a_time_invariant != 0;
     if (dtype == MRX_F32) {
         if (!aligned(a, 4) || !aligned(b, 4) || !aligned(h, 4)) return MRX_ERR_INVALID_ARG;
-        return launch_fwd<float>(st, a, b, done, done_dtype, h0, P0, h, h_last, P_last, B, T, D, ti);
+        return launch_fwd<float>(st, a, b, done, done_dtype, h0, P0, h, h_last, P_last, B, T, D, ti, workspace);
     }
     if (dtype == MRX_C64) {
         if (!aligned(a, 8) || !aligned(b, 8) || !aligned(h, 8) || !aligned(h0, 8) ||
             !aligned(P0, 8) || !aligned(h_last, 8) || !aligned(P_last, 8))
             return MRX_ERR_INVALID_ARG;
-        return launch_fwd<c64>(st, a, b, done, done_dtype, h0, P0, h, h_last, P_last, B, T, D, ti);
+        return launch_fwd<c64>(st, a, b, done, done_dtype, h0, P0, h, h_last, P_last, B, T, D, ti, workspace);
     }
     if (dtype == MRX_BF16) {  // a, b, h in bfloat16; arithmetic and carries in float32
         if (!aligned(a, 2) || !aligned(b, 2) || !aligned(h, 2) || !aligned(h0, 4) || !aligned(P0, 4) ||
             !aligned(h_last, 4) || !aligned(P_last, 4))
             return MRX_ERR_INVALID_ARG;
-        return launch_fwd<float, false, __bf16>(st, a, b, done, done_dtype, h0, P0, h, h_last, P_last, B, T, D, ti);
+        return launch_fwd<float, false, __bf16>(st, a, b, done, done_dtype, h0, P0, h, h_last, P_last, B, T, D, ti, workspace);
     }
     return MRX_ERR_INVALID_ARG;
 }
 
-extern "C" int mrx_linear_scan_bwd(void *stream, const void *a, const void *h, const void *done,
-                                   const void *h0, const void *g, const void *g_last, void *da,
-                                   void *db, void *dh0, int64_t B, int64_t T, int64_t D,
-                                   int dtype, int done_dtype, int a_time_invariant)
+}  // namespace
+
+extern "C" int mrx_linear_scan_fwd(void *stream, const void *a, const void *b, const void *done, const void *h0, const void *P0, void *h,
+                                   void *h_last, void *P_last, int64_t B, int64_t T, int64_t D, int dtype, int done_dtype, int
+                                   a_time_invariant)
+{
+    return linear_scan_fwd(stream, a, b, done, h0, P0, h, h_last, P_last, B, T, D, dtype, done_dtype, a_time_invariant, nullptr);
+}
+
+extern "C" int mrx_linear_scan_fwd_segmented(void *stream, const void *a, const void *b, const void *done, const void *h0, const void *P0,
+                                             void *h, void *h_last, void *P_last, int64_t B, int64_t T, int64_t D, int dtype, int
+                                             done_dtype, int a_time_invariant, void *workspace)
+{
+    if (!aligned(workspace, 8)) return MRX_ERR_INVALID_ARG;
+    return linear_scan_fwd(stream, a, b, done, h0, P0, h, h_last, P_last, B, T, D, dtype, done_dtype, a_time_invariant, workspace);
+}
+
+namespace {
+
+int linear_scan_bwd(void *stream, const void *a, const void *h, const void *done, const void *h0, const void *g, const void *g_last, void
+                    *da, void *db, void *dh0, int64_t B, int64_t T, int64_t D, int dtype, int done_dtype, int a_time_invariant, void
+                    *workspace)
 {
     if (!a || !h || !done || !g || !da || !db) return MRX_ERR_INVALID_ARG;
     if (!scan_shape_ok(B, T, D)) return MRX_ERR_INVALID_ARG;
@@ -1268,22 +1547,39 @@ extern "C" int mrx_linear_scan_bwd(void *stream, const void *a, const void *h, c
     if (dtype == MRX_F32) {
         if (!aligned(a, 4) || !aligned(h, 4) || !aligned(g, 4) || !aligned(da, 4) || !aligned(db, 4))
             return MRX_ERR_INVALID_ARG;
-        return launch_bwd<float>(st, a, nullptr, h, done, done_dtype, h0, g, g_last, da, db, dh0, B, T, D, ti, da_sum);
+        return launch_bwd<float>(st, a, nullptr, h, done, done_dtype, h0, g, g_last, da, db, dh0, B, T, D, ti, da_sum, workspace);
     }
     if (dtype == MRX_C64) {
         if (!aligned(a, 8) || !aligned(h, 8) || !aligned(g, 8) || !aligned(da, 8) ||
             !aligned(db, 8) || !aligned(h0, 8) || !aligned(g_last, 8) || !aligned(dh0, 8))
             return MRX_ERR_INVALID_ARG;
-        return launch_bwd<c64>(st, a, nullptr, h, done, done_dtype, h0, g, g_last, da, db, dh0, B, T, D, ti, da_sum);
+        return launch_bwd<c64>(st, a, nullptr, h, done, done_dtype, h0, g, g_last, da, db, dh0, B, T, D, ti, da_sum, workspace);
     }
     if (dtype == MRX_BF16) {  // a, h, g, da (per step), db in bfloat16; carries and a summed da in float32
         if (!aligned(a, 2) || !aligned(h, 2) || !aligned(g, 2) || !aligned(da, da_sum ? 4 : 2) || !aligned(db, 2) ||
             !aligned(h0, 4) || !aligned(g_last, 4) || !aligned(dh0, 4))
             return MRX_ERR_INVALID_ARG;
         return launch_bwd<float, false, __bf16>(st, a, nullptr, h, done, done_dtype, h0, g, g_last, da, db, dh0, B, T, D,
-                                                ti, da_sum);
+                                                ti, da_sum, workspace);
     }
     return MRX_ERR_INVALID_ARG;
+}
+
+}  // namespace
+
+extern "C" int mrx_linear_scan_bwd(void *stream, const void *a, const void *h, const void *done, const void *h0, const void *g, const void
+                                   *g_last, void *da, void *db, void *dh0, int64_t B, int64_t T, int64_t D, int dtype, int done_dtype, int
+                                   a_time_invariant)
+{
+    return linear_scan_bwd(stream, a, h, done, h0, g, g_last, da, db, dh0, B, T, D, dtype, done_dtype, a_time_invariant, nullptr);
+}
+
+extern "C" int mrx_linear_scan_bwd_segmented(void *stream, const void *a, const void *h, const void *done, const void *h0, const void *g,
+                                             const void *g_last, void *da, void *db, void *dh0, int64_t B, int64_t T, int64_t D, int
+                                             dtype, int done_dtype, int a_time_invariant, void *workspace)
+{
+    if (!aligned(workspace, 8)) return MRX_ERR_INVALID_ARG;
+    return linear_scan_bwd(stream, a, h, done, h0, g, g_last, da, db, dh0, B, T, D, dtype, done_dtype, a_time_invariant, workspace);
 }
 
 extern "C" int mrx_linear_scan_last(void *stream, const void *a, const void *b, const void *done,
@@ -1307,9 +1603,10 @@ extern "C" int mrx_linear_scan_last(void *stream, const void *a, const void *b, 
     return dtype == MRX_BF16 ? MRX_ERR_UNSUPPORTED : MRX_ERR_INVALID_ARG;
 }
 
-extern "C" int mrx_mingru_scan_fwd(void *stream, const void *z, const void *h_tilde, const void *done,
-                                   const void *h0, const void *P0, void *h, void *h_last, void *P_last,
-                                   int64_t B, int64_t T, int64_t D, int dtype, int done_dtype)
+namespace {
+
+int mingru_scan_fwd(void *stream, const void *z, const void *h_tilde, const void *done, const void *h0, const void *P0, void *h, void
+                    *h_last, void *P_last, int64_t B, int64_t T, int64_t D, int dtype, int done_dtype, void *workspace)
 {
     if (!z || !h_tilde || !done || !h) return MRX_ERR_INVALID_ARG;
     if (!scan_shape_ok(B, T, D)) return MRX_ERR_INVALID_ARG;
@@ -1323,15 +1620,32 @@ extern "C" int mrx_mingru_scan_fwd(void *stream, const void *z, const void *h_ti
         if (!aligned(p, 4)) return MRX_ERR_INVALID_ARG;
     if (dtype == MRX_BF16)
         return launch_fwd<float, true, __bf16>((hipStream_t)stream, z, h_tilde, done, done_dtype, h0, P0, h, h_last,
-                                               P_last, B, T, D, 0);
+                                               P_last, B, T, D, 0, workspace);
     return launch_fwd<float, true>((hipStream_t)stream, z, h_tilde, done, done_dtype, h0, P0, h, h_last, P_last, B, T,
-                                   D, 0);
+                                   D, 0, workspace);
 }
 
-extern "C" int mrx_mingru_scan_bwd(void *stream, const void *z, const void *h_tilde, const void *h,
-                                   const void *done, const void *h0, const void *g, const void *g_last,
-                                   void *dz, void *dh_tilde, void *dh0, int64_t B, int64_t T, int64_t D,
-                                   int dtype, int done_dtype)
+}  // namespace
+
+extern "C" int mrx_mingru_scan_fwd(void *stream, const void *z, const void *h_tilde, const void *done, const void *h0, const void *P0,
+                                   void *h, void *h_last, void *P_last, int64_t B, int64_t T, int64_t D, int dtype, int done_dtype)
+{
+    return mingru_scan_fwd(stream, z, h_tilde, done, h0, P0, h, h_last, P_last, B, T, D, dtype, done_dtype, nullptr);
+}
+
+extern "C" int mrx_mingru_scan_fwd_segmented(void *stream, const void *z, const void *h_tilde, const void *done, const void *h0, const
+                                             void *P0, void *h, void *h_last, void *P_last, int64_t B, int64_t T, int64_t D, int dtype,
+                                             int done_dtype, void *workspace)
+{
+    if (!aligned(workspace, 8)) return MRX_ERR_INVALID_ARG;
+    return mingru_scan_fwd(stream, z, h_tilde, done, h0, P0, h, h_last, P_last, B, T, D, dtype, done_dtype, workspace);
+}
+
+namespace {
+
+int mingru_scan_bwd(void *stream, const void *z, const void *h_tilde, const void *h, const void *done, const void *h0, const void *g,
+                    const void *g_last, void *dz, void *dh_tilde, void *dh0, int64_t B, int64_t T, int64_t D, int dtype, int done_dtype,
+                    void *workspace)
 {
     if (!z || !h_tilde || !h || !done || !g || !dz || !dh_tilde) return MRX_ERR_INVALID_ARG;
     if (!scan_shape_ok(B, T, D)) return MRX_ERR_INVALID_ARG;
@@ -1345,9 +1659,26 @@ extern "C" int mrx_mingru_scan_bwd(void *stream, const void *z, const void *h_ti
         if (!aligned(p, 4)) return MRX_ERR_INVALID_ARG;
     if (dtype == MRX_BF16)
         return launch_bwd<float, true, __bf16>((hipStream_t)stream, z, h_tilde, h, done, done_dtype, h0, g, g_last, dz,
-                                               dh_tilde, dh0, B, T, D, 0);
+                                               dh_tilde, dh0, B, T, D, 0, 0, workspace);
     return launch_bwd<float, true>((hipStream_t)stream, z, h_tilde, h, done, done_dtype, h0, g, g_last, dz, dh_tilde,
-                                   dh0, B, T, D, 0);
+                                   dh0, B, T, D, 0, 0, workspace);
+}
+
+}  // namespace
+
+extern "C" int mrx_mingru_scan_bwd(void *stream, const void *z, const void *h_tilde, const void *h, const void *done, const void *h0,
+                                   const void *g, const void *g_last, void *dz, void *dh_tilde, void *dh0, int64_t B, int64_t T, int64_t
+                                   D, int dtype, int done_dtype)
+{
+    return mingru_scan_bwd(stream, z, h_tilde, h, done, h0, g, g_last, dz, dh_tilde, dh0, B, T, D, dtype, done_dtype, nullptr);
+}
+
+extern "C" int mrx_mingru_scan_bwd_segmented(void *stream, const void *z, const void *h_tilde, const void *h, const void *done, const void
+                                             *h0, const void *g, const void *g_last, void *dz, void *dh_tilde, void *dh0, int64_t B,
+                                             int64_t T, int64_t D, int dtype, int done_dtype, void *workspace)
+{
+    if (!aligned(workspace, 8)) return MRX_ERR_INVALID_ARG;
+    return mingru_scan_bwd(stream, z, h_tilde, h, done, h0, g, g_last, dz, dh_tilde, dh0, B, T, D, dtype, done_dtype, workspace);
 }
 
 namespace {

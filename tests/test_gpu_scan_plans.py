@@ -1,5 +1,5 @@
 """The diagonal scans where the plan changes: rows that are no whole number of vectors (also narrower than one), super-steps of
-16 steps per wave and their remainders, streaming kernels on ragged rows; every kind of array, forward and backward, against a
+16 steps per wave and their remainders, streaming kernels on ragged rows, time in segments; every kind of array, forward and backward, against a
 sequential reference in double precision."""
 import pytest
 import torch
@@ -12,7 +12,8 @@ SHAPES = [
     (2, 513, 65), (5, 272, 130),
     (300, 520, 70),                               # eight waves of 16 steps
     (1101, 33, 131), (601, 65, 257),              # streaming on ragged rows
-    (1, 1200, 512),
+    (1, 385, 2), (1, 513, 65), (12, 450, 130), (1, 1200, 512),   # time in segments, the last one partly filled
+    (1, 4096, 70),                                # as many segments as there can be
 ]
 
 
