@@ -585,6 +585,19 @@ int mrx_row_dense(void *stream, const void *x, const float *scale, const float *
                   int layers, const float *residual, int64_t rows, int64_t K, int x_dtype, int w_dtype, int b_dtype,
                   int y_dtype, int product_dtype, float eps);
 
+/* ---- Gradients of dense layers that read the same rows ----
+ * For layers l = 0 .. layers - 1 (at most MRX_DENSE_LAYERS) with y_l = x W_l^T + b_l, of dy_l (rows, n_out[l]):
+ *   dx (nullable): (rows, K) in dx_dtype, sum_l dy_l W_l;
+ *   params (nullable): float32, [dW_0 (n_out[0], K) | dW_1 | ...] and then db_l (n_out[l]) of the layers whose bit is set in
+ *     bias_mask; padded to a multiple of four floats.
+ * x, dy_l and W_l (n_out[l], K) in `dtype`, MRX_F32 or MRX_BF16, sums in float32; K a multiple of 8.  x may be NULL without
+ * params, weights without dx.  workspace: mrx_dense_grads_workspace(...) floats, overwritten (NULL where that is 0). */
+#define MRX_DENSE_LAYERS 8
+int64_t mrx_dense_grads_workspace(int64_t rows, int64_t K, const int64_t *n_out, int layers, int dtype, unsigned bias_mask);
+int mrx_dense_grads(void *stream, const void *x, const void *const *dys, const void *const *weights, const int64_t *n_out,
+                    int layers, void *dx, float *params, float *workspace, int64_t rows, int64_t K, int dtype, int dx_dtype,
+                    unsigned bias_mask);
+
 #ifdef __cplusplus
 }
 #endif

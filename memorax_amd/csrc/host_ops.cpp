@@ -47,7 +47,7 @@ using torch::autograd::variable_list;
     X(mrx_delta_rule_fwd_noalloc) X(mrx_deltanet_fwd) X(mrx_deltanet_bwd) X(mrx_linear_attn_step)                    \
     X(mrx_gated_linear_attn_step) X(mrx_delta_rule_step) X(mrx_causal_conv_silu_fwd) X(mrx_causal_conv_silu_bwd)     \
     X(mrx_mamba_elements_fwd) X(mrx_mamba_elements_bwd) X(mrx_decay_last) X(mrx_mamba_readout_fwd)                   \
-    X(mrx_mamba_readout_bwd) X(mrx_deltanet_step) X(mrx_mingru_step) X(mrx_row_dense)
+    X(mrx_mamba_readout_bwd) X(mrx_deltanet_step) X(mrx_mingru_step) X(mrx_row_dense) X(mrx_dense_grads) X(mrx_dense_grads_workspace)
 struct {
 #define MRX_MEMBER(name) decltype(&::name) name = nullptr;
     MRX_BOUND(MRX_MEMBER)
@@ -1221,11 +1221,65 @@ Tensor weight_gradient(const Tensor &dy, const Tensor &x)
     return (half(dy.scalar_type()) ? at::bmm(a, b, at::kFloat) : at::bmm(a, b)).sum(0);
 }
 
+// Gradients of dense layers that read the rows x (rows, K), of dys[l] (rows, n_l): the input's (undefined unless wanted), then
+// each layer's weight and bias gradients (views of one float32 block; undefined unless wanted / without a bias).
+std::vector<Tensor> dense_grads(const Tensor &x, const std::vector<Tensor> &dys, const std::vector<Tensor> &weights, const std::vector<bool> &has_bias,
+                                bool want_dx, ScalarType dx_dtype, bool want_params)
+{
+    const size_t L = dys.size();
+    TORCH_CHECK_VALUE(L >= 1 && L <= MRX_DENSE_LAYERS && weights.size() == L && has_bias.size() == L, "dense_grads takes 1 to ", MRX_DENSE_LAYERS, " layers");
+    const int64_t rows = x.size(0), K = x.size(1);
+    const auto dt = x.scalar_type();
+    chk(x, "x");
+    std::array<const void *, MRX_DENSE_LAYERS> dy{}, w{};
+    std::array<int64_t, MRX_DENSE_LAYERS> n{};
+    unsigned bias = 0;
+    int64_t total = 0;
+    for (size_t l = 0; l < L; ++l) {
+        n[l] = weights[l].size(0);
+        chk(dys[l], "dy", dt, {rows, n[l]});
+        chk(weights[l], "weight", dt, {n[l], K});
+        dy[l] = ptr(dys[l]), w[l] = ptr(weights[l]);
+        total += n[l] * (K + has_bias[l]);
+        if (has_bias[l]) bias |= 1u << l;
+    }
+    const Tensor dx = want_dx ? fresh({rows, K}, dx_dtype, x) : Tensor();
+    Tensor params, work;
+    if (want_params) {
+        params = fresh({(total + 3) / 4 * 4}, at::kFloat, x);
+        if (const int64_t floats = lib.mrx_dense_grads_workspace(rows, K, n.data(), (int)L, code(dt), bias)) work = fresh({floats}, at::kFloat, x);
+    }
+    check(lib.mrx_dense_grads(stream(), ptr(x), dy.data(), w.data(), n.data(), (int)L, ptr(dx), fptr(params), fptr(work), rows, K, code(dt),
+                              code(dx_dtype), bias),
+          "mrx_dense_grads");
+    std::vector<Tensor> out(1 + 2 * L);
+    out[0] = dx;
+    if (want_params) {
+        int64_t at = 0;
+        for (size_t l = 0; l < L; ++l, at += n[l - 1] * K) out[1 + l] = params.narrow(0, at, n[l] * K).view({n[l], K});
+        for (size_t l = 0; l < L; ++l)
+            if (has_bias[l]) out[1 + L + l] = params.narrow(0, at, n[l]), at += n[l];
+    }
+    return out;
+}
+
 // The dtype the array library's autocast would run a product on x in.
 std::optional<ScalarType> autocast_dtype(const Tensor &x)
 {
     if (x.is_cuda() && x.is_floating_point() && at::autocast::is_autocast_enabled(at::kCUDA)) return at::autocast::get_autocast_dtype(at::kCUDA);
     return std::nullopt;
+}
+
+// Which of a group's gradients the library's kernels form.  Parameters: while they are bound by reading the rows, i.e. up to widths
+// where the array library's larger tiles take over (us, here / there: bfloat16 131072 x 256 -> 3 x 256 105 / 277, 11455 x 128 ->
+// 3 x 256 26 / 225, 32768 x 1024 -> 1024 148 / 121; float32 131072 x 256 -> 256 188 / 181, 23100 x 64 -> 256 26 / 99, 131072 x 512 ->
+// 3 x 512 2080 / 1740).  The input: several layers at once, as narrow (68200 x 128 -> 3 x 64 + 2 25 / 69, 131072 x 256 -> 3 x 256 + 4
+// 118 / 150; float32 68 / 93, but 131072 x 256 -> 3 x 256 536 / 454), or few rows, where the host's calls are what it costs.
+bool params_suit(ScalarType dt, int64_t K, int64_t widest) { return K * widest <= (dt == at::kBFloat16 ? 512 * 512 : 256 * 256); }
+bool input_suits(ScalarType dt, int64_t rows, int64_t K, int64_t widest, size_t layers)
+{
+    const int64_t most = dt == at::kBFloat16 ? 256 : 128;
+    return layers > 1 && ((K <= most && widest <= most) || (rows <= 4096 && K * widest <= 512 * 512));
 }
 
 // Several dense layers on one input: one cast of it, and the gradients with respect to it accumulated by the products
@@ -1241,16 +1295,42 @@ struct DenseOp {
         c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
         const Tensor &x = s[0], x2 = x.reshape({-1, x.size(-1)});
         const size_t n = weights.size();
+        const auto dt = x.scalar_type();
         variable_list out(1 + 2 * n);
+        std::vector<Tensor> dys, ws;   // of the layers whose outputs were used: the others cost no products
+        std::vector<size_t> used;
+        std::vector<bool> bias;
+        int64_t widest = 0;
+        bool want_params = false, regular = x.is_cuda() && (dt == at::kFloat || dt == at::kBFloat16) && x2.size(1) % 8 == 0 && x2.numel() > 0;
         for (size_t l = 0; l < n; ++l) {
-            if (!grads[l].defined()) continue;   // an output nobody used costs no products
-            const Tensor w = weights[l].unpack(), dy = grads[l].to(x.scalar_type()).reshape({-1, w.size(0)});
-            if (node.wants(0)) {
-                if (out[0].defined()) out[0].addmm_(dy, w);
-                else out[0] = at::mm(dy, w);
+            if (!grads[l].defined()) continue;
+            ws.push_back(weights[l].unpack());
+            dys.push_back(grads[l].to(dt).reshape({-1, ws.back().size(0)}).contiguous());
+            used.push_back(l);
+            bias.push_back(has_bias[l] && node.wants(1 + n + l));
+            widest = std::max(widest, ws.back().size(0));
+            want_params = want_params || node.wants(1 + l) || bias.back();
+            regular = regular && ws.back().is_contiguous() && ws.back().size(0) > 0 && reinterpret_cast<uintptr_t>(ws.back().data_ptr()) % 16 == 0;
+        }
+        if (used.empty()) return out;
+        regular = regular && used.size() <= MRX_DENSE_LAYERS && x2.is_contiguous() && reinterpret_cast<uintptr_t>(x2.data_ptr()) % 16 == 0;
+        const bool own_params = want_params && regular && params_suit(dt, x2.size(1), widest),
+                   own_dx = node.wants(0) && regular && (x_dtype == at::kFloat || x_dtype == at::kBFloat16) &&
+                            input_suits(dt, x2.size(0), x2.size(1), widest, used.size());
+        if (own_params || own_dx) {
+            auto r = dense_grads(x2, dys, ws, bias, own_dx, x_dtype, own_params);
+            out[0] = r[0];
+            for (size_t i = 0; i < used.size(); ++i) out[1 + used[i]] = r[1 + i], out[1 + n + used[i]] = r[1 + used.size() + i];
+        }
+        for (size_t i = 0; i < used.size(); ++i) {
+            const size_t l = used[i];
+            if (node.wants(0) && !own_dx) {
+                if (i > 0) out[0].addmm_(dys[i], ws[i]);
+                else out[0] = at::mm(dys[i], ws[i]);
             }
-            if (node.wants(1 + l)) out[1 + l] = weight_gradient(dy, x2);
-            if (has_bias[l] && node.wants(1 + n + l)) out[1 + n + l] = dy.sum({0}, false, wide(dy.scalar_type()));
+            if (own_params) continue;
+            if (node.wants(1 + l)) out[1 + l] = weight_gradient(dys[i], x2);
+            if (bias[i]) out[1 + n + l] = dys[i].sum({0}, false, wide(dt));
         }
         if (out[0].defined()) out[0] = out[0].view(x.sizes()).to(x_dtype);
         return out;
@@ -1590,6 +1670,7 @@ PYBIND11_MODULE(_native, m)
     def("silu_gate", &silu_gate);
     def("norm", &norm);
     def("dense_group", &dense_group);
+    def("dense_grads", &dense_grads);
     def("weight_gradient", &weight_gradient);
     def("weight_gradient_slices", &weight_gradient_slices);
     def("causal_conv_silu", &causal_conv_silu);

@@ -1,13 +1,15 @@
 """Dense layers of the host-side mirror (flax.linen.Dense in the reference's cells and blocks,
 e.g. linear_attention.py:62-80, min_gru.py:49-62, blocks/ffn.py:11-123).
 
-The products stay the array library's; what this module changes is their shape.  A rollout batch
+The forward products stay the array library's; the gradients are the library's own kernels
+(csrc/dense_grads.hip) up to the widths where those of the array library take over, and there what this
+module changes is their shape.  A rollout batch
 has a hundred thousand rows and a few hundred features, so the weight gradient ``dy^T x`` is a
 product with a tiny result and an enormous inner dimension, which the library's GEMM runs on as
 many workgroups as the result has tiles (sixteen for 256 x 256: 330 us where the forward product
-of the same operands takes 32 us).  ``dense`` cuts the rows into slices, multiplies them as one
-batched product with float32 partial results and sums those (41 us); ``dense_group`` runs the
-layers that share an input on one cast of it and lets their products add up the input gradient.
+of the same operands takes 32 us).  Where the library's kernels do not serve a layer, ``dense`` cuts the rows
+into slices, multiplies them as one batched product with float32 partial results and sums those (41 us);
+``dense_group`` runs the layers that share an input on one cast of it, and their gradients as one operation.
 Without gradients and on few rows (acting) the layers are one launch of the library's row kernel.  The nodes
 are native (csrc/host_ops.cpp): a layer of a small update is bound by what the host does around its products.
 """

@@ -1,0 +1,40 @@
+"""The gradients of grouped dense layers (mrx_dense_grads) against double precision: widths around the kernels' tiles, layers of a
+few outputs whose rows are no whole 16-byte segments, one row to several slices of rows."""
+import pytest
+import torch
+
+from memorax_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    (1, 8, [1]), (63, 64, [3, 64]), (64, 72, [64, 65, 2]), (257, 128, [129, 7, 128, 4]), (1000, 256, [256]),
+    (513, 264, [100, 16]), (9001, 64, [8] * 8), (70000, 128, [64, 64, 64, 2]),
+]
+
+
+@pytest.mark.parametrize("rows,K,outs", CASES)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dx_dtype", [torch.float32, torch.bfloat16])
+def test_dense_grads(rows, K, outs, dtype, dx_dtype):
+    gen = torch.Generator(device="cuda").manual_seed(rows + K)
+    rnd = lambda *s: torch.randn(*s, generator=gen, device="cuda").to(dtype)
+    x, dys, ws = rnd(rows, K), [rnd(rows, n) for n in outs], [rnd(n, K) for n in outs]
+    bias = [l % 2 == 0 for l in range(len(outs))]
+    print(f"case dense grads rows={rows} K={K} outs={outs} {dtype} {dx_dtype}", flush=True)
+    dx, *params = _lib.native().dense_grads(x, dys, ws, bias, True, dx_dtype, True)
+    tol = 2e-5
+
+    def check(got, want, t=tol):
+        assert (got.double() - want).abs().max() <= t * want.abs().max().clamp_min(1e-30)
+
+    assert dx.dtype == dx_dtype
+    check(dx, sum(d.double() @ w.double() for d, w in zip(dys, ws)), 1e-2 if dx_dtype == torch.bfloat16 else tol)
+    for l, d in enumerate(dys):
+        check(params[l], d.double().t() @ x.double())
+        if bias[l]:
+            check(params[len(outs) + l], d.double().sum(0))
+        else:
+            assert params[len(outs) + l] is None or not params[len(outs) + l].numel()
+    only = _lib.native().dense_grads(x, dys, ws, bias, False, dx_dtype, True)
+    assert all(torch.equal(a, b) for a, b in zip(only[1:], params) if b is not None)
