@@ -578,12 +578,30 @@ int mrx_mingru_step(void *stream, const void *z, const void *h_tilde, const void
  * in w_dtype; b_l: (n_out[l]) in b_dtype or NULL; y_l: (rows,n_out[l]) in y_dtype.  product_dtype: MRX_BF16 rounds the
  * normalised rows, weights, biases and results to bfloat16 (float32 sums), MRX_F32 multiplies in float32; round_norm: the
  * normalised rows pass through bfloat16 in either case.  weights, biases, outs, n_out: HOST arrays of `layers` entries.
- * K a multiple of 8, at most 2048; x, W and the norm's vectors 16-byte aligned. */
+ * K a multiple of 8, at most 2048; x, W and the norm's vectors 16-byte aligned.
+ * weights2 (nullable, one layer): W_0 lies in two arrays, (n_out, k1) and (n_out, K - k1), k1 a multiple of 8.
+ * skip, skip_out (both or neither): skip_out (rows,K) float32 = x + skip * norm(x), skip (K). */
 #define MRX_ROW_DENSE_LAYERS 4
 int mrx_row_dense(void *stream, const void *x, const float *scale, const float *norm_bias, int norm, int round_norm,
                   const void *const *weights, const void *const *biases, void *const *outs, const int64_t *n_out,
                   int layers, const float *residual, int64_t rows, int64_t K, int x_dtype, int w_dtype, int b_dtype,
-                  int y_dtype, int product_dtype, float eps);
+                  int y_dtype, int product_dtype, float eps, const void *weights2, int64_t k1, const float *skip,
+                  float *skip_out);
+
+/* What lies between the dense layers of an acting step (all float32).
+ * LRU cell (lru.py:76-108): from the rows u = norm(x) [B_re | B_im]^T (each (B,N)), lambda = exp(-exp(nu_log) + i exp(theta_log)),
+ *   h' = (done ? 0 : lambda h) + exp(gamma_log) u,  P' = (done ? 1 : P) lambda  (complex64, (B,N)); row: (B,2N) [Re h' | -Im h'].
+ * mLSTM cell (mlstm.py:31-240): from up = (B,2 H D) [x | z], the convolution's last tap, the block-diagonal maps wq, wk, wv (H,D,D),
+ *   the gates wi, wf (H,3 H D), bi, bf (H), the carry C (B,H,D,D), log_f, m (B,H), n (B,H,D): the carry after the step and
+ *   y (B,H D), the normalised and gated read-out before the output projection.  D 16, 32 or 64, H at most 8, H D at most 256. */
+int mrx_lru_step(void *stream, const float *u_re, const float *u_im, const float *nu_log, const float *theta_log,
+                 const float *gamma_log, const void *done, const void *h, const void *P, void *h_out, void *P_out,
+                 float *row, int64_t B, int64_t N, int done_dtype);
+int mrx_mlstm_step(void *stream, const float *up, const float *conv_w, const float *conv_b, const float *wq, const float *wk,
+                   const float *wv, const float *wi, const float *bi, const float *wf, const float *bf,
+                   const float *norm_w, const float *skip, const void *done, const float *C, const float *lf,
+                   const float *n, const float *m, float *C_out, float *lf_out, float *n_out, float *m_out, float *y,
+                   int64_t B, int64_t H, int64_t D, int64_t conv_k, int done_dtype, float g_floor);
 
 /* ---- Gradients of dense layers that read the same rows ----
  * For layers l = 0 .. layers - 1 (at most MRX_DENSE_LAYERS) with y_l = x W_l^T + b_l, of dy_l (rows, n_out[l]):

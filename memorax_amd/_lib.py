@@ -59,7 +59,9 @@ SIGNATURES = {
     "mrx_delta_rule_step": (_I, [_P] * 9 + [_L] * 4 + [_I] * 2),
     "mrx_deltanet_step": (_I, [_P] * 9 + [_L] * 4 + [_I] * 2),
     "mrx_mingru_step": (_I, [_P] * 10 + [_L] * 2 + [_I] * 2),
-    "mrx_row_dense": (_I, [_P] * 4 + [_I] * 2 + [_P] * 4 + [_I, _P] + [_L] * 2 + [_I] * 5 + [ctypes.c_float]),
+    "mrx_row_dense": (_I, [_P] * 4 + [_I] * 2 + [_P] * 4 + [_I, _P] + [_L] * 2 + [_I] * 5 + [ctypes.c_float, _P, _L, _P, _P]),
+    "mrx_lru_step": (_I, [_P] * 12 + [_L] * 2 + [_I]),
+    "mrx_mlstm_step": (_I, [_P] * 23 + [_L] * 4 + [_I, ctypes.c_float]),
     "mrx_dense_grads_workspace": (_L, [_L] * 2 + [_P] + [_I] * 2 + [ctypes.c_uint]),
     "mrx_dense_grads": (_I, [_P] * 5 + [_I] + [_P] * 3 + [_L] * 2 + [_I] * 2 + [ctypes.c_uint]),
     "mrx_gated_linear_attn_step": (_I, [_P] * 9 + [_L] * 4 + [_I] * 3),

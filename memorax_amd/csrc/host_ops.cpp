@@ -47,7 +47,8 @@ using torch::autograd::variable_list;
     X(mrx_delta_rule_fwd_noalloc) X(mrx_deltanet_fwd) X(mrx_deltanet_bwd) X(mrx_linear_attn_step)                    \
     X(mrx_gated_linear_attn_step) X(mrx_delta_rule_step) X(mrx_causal_conv_silu_fwd) X(mrx_causal_conv_silu_bwd)     \
     X(mrx_mamba_elements_fwd) X(mrx_mamba_elements_bwd) X(mrx_decay_last) X(mrx_mamba_readout_fwd)                   \
-    X(mrx_mamba_readout_bwd) X(mrx_deltanet_step) X(mrx_mingru_step) X(mrx_row_dense) X(mrx_dense_grads) X(mrx_dense_grads_workspace)
+    X(mrx_mamba_readout_bwd) X(mrx_deltanet_step) X(mrx_mingru_step) X(mrx_row_dense) X(mrx_dense_grads) X(mrx_dense_grads_workspace)                  \
+    X(mrx_lru_step) X(mrx_mlstm_step)
 struct {
 #define MRX_MEMBER(name) decltype(&::name) name = nullptr;
     MRX_BOUND(MRX_MEMBER)
@@ -708,7 +709,8 @@ StepOut delta_rule_step(const Tensor &q, const Tensor &k, const Tensor &v, const
 // layer's result.
 std::vector<Tensor> row_dense(const Tensor &x, int norm, const OptTensor &scale, const OptTensor &nbias, double eps, bool round_norm,
                               const std::vector<Tensor> &weights, const std::vector<OptTensor> &biases, ScalarType product, ScalarType out_dtype,
-                              const OptTensor &residual)
+                              const OptTensor &residual, const OptTensor &weight2 = std::nullopt, const OptTensor &skip = std::nullopt,
+                              Tensor *skip_out = nullptr)
 {
     TORCH_CHECK_VALUE(x.dim() >= 2 && !weights.empty() && weights.size() <= MRX_ROW_DENSE_LAYERS && biases.size() == weights.size(),
                       "row_dense takes rows and 1 to ", MRX_ROW_DENSE_LAYERS, " layers");
@@ -727,7 +729,7 @@ std::vector<Tensor> row_dense(const Tensor &x, int norm, const OptTensor &scale,
     bool first_bias = true;
     for (size_t l = 0; l < weights.size(); ++l) {
         n[l] = weights[l].size(0);
-        chk(weights[l], "weight", wd, {n[l], K});
+        chk(weights[l], "weight", wd, {n[l], weight2.has_value() ? K - weight2->size(1) : K});
         if (biases[l].has_value()) {
             if (std::exchange(first_bias, false)) bd = biases[l]->scalar_type();
             chk(*biases[l], "bias", bd, {n[l]});
@@ -737,11 +739,66 @@ std::vector<Tensor> row_dense(const Tensor &x, int norm, const OptTensor &scale,
         w[l] = ptr(weights[l]), b[l] = ptr(biases[l]), y[l] = ptr(out[l]);
     }
     chk(residual, "residual", at::kFloat, out[0].sizes());
+    if (weight2.has_value()) chk(*weight2, "weight2", wd, {n[0], weight2->size(1)});
+    chk(skip, "skip", at::kFloat, {K});
+    if (skip.has_value()) *skip_out = fresh(x.sizes(), at::kFloat, x);
     check(lib.mrx_row_dense(stream(), ptr(x), fptr(scale), fptr(nbias), norm, round_norm, w.data(), b.data(), y.data(), n.data(),
                             (int)weights.size(), fptr(residual), rows, K, code(x.scalar_type()), code(wd), code(bd), code(out_dtype),
-                            code(product), (float)eps),
+                            code(product), (float)eps, ptr(weight2), weight2.has_value() ? weights[0].size(1) : 0, fptr(skip),
+                            skip_out ? fptr(*skip_out) : nullptr),
           "mrx_row_dense");
     return out;
+}
+
+// A pre-norm residual block around an LRU cell, one acting step: x (B,1,F) float32, the carry's leaves (B,1,N) complex64
+// -> y, h, P.  params: nu_log, theta_log, gamma_log, B_real, B_imag, C_real, C_imag, D.
+std::tuple<Tensor, Tensor, Tensor> lru_act(const Tensor &x, int norm, const OptTensor &scale, const OptTensor &nbias, double eps,
+                                           const std::vector<Tensor> &params, const Tensor &done_, const Tensor &h_, const Tensor &P_)
+{
+    TORCH_CHECK_VALUE(x.dim() == 3 && x.size(1) == 1 && params.size() == 8, "lru_act takes one time step");
+    const int64_t B = x.size(0), F = x.size(2), N = params[0].size(0);
+    for (int i = 0; i < 3; ++i) chk(params[i], "parameter", at::kFloat, {N});
+    const Tensor h = h_.contiguous(), P = P_.contiguous();
+    chk(h, "h", at::kComplexFloat, {B, 1, N});
+    chk(P, "P", at::kComplexFloat, {B, 1, N});
+    const Done done(done_, B, 1);
+    Tensor skip;
+    const auto u = row_dense(x, norm, scale, nbias, eps, false, {params[3], params[4]}, {std::nullopt, std::nullopt}, at::kFloat, at::kFloat,
+                             std::nullopt, std::nullopt, params[7], &skip);
+    const Tensor hn = fresh_like(h), Pn = fresh_like(P), row = fresh({B, 1, 2 * N}, at::kFloat, x);
+    check(lib.mrx_lru_step(stream(), fptr(u[0]), fptr(u[1]), fptr(params[0]), fptr(params[1]), fptr(params[2]), done.p(), ptr(h), ptr(P), ptr(hn),
+                           ptr(Pn), fptr(row), B, N, done.dtype),
+          "mrx_lru_step");
+    return {row_dense(row, 0, std::nullopt, std::nullopt, 0.0, false, {params[5]}, {std::nullopt}, at::kFloat, at::kFloat, skip, params[6])[0], hn, Pn};
+}
+
+// The same around an mLSTM cell; params: up, conv weight and bias, query, key, value, i_gate and f_gate (weight, bias), norm_weight,
+// learnable_skip, output projection; the carry's leaves C (B,1,H,D,D), log_f, n (B,1,H,D,1), m.
+std::vector<Tensor> mlstm_act(const Tensor &x, int norm, const OptTensor &scale, const OptTensor &nbias, double eps, const std::vector<Tensor> &p,
+                              const Tensor &done_, const std::vector<Tensor> &carry, double g_floor)
+{
+    TORCH_CHECK_VALUE(x.dim() == 3 && x.size(1) == 1 && p.size() == 13 && carry.size() == 4, "mlstm_act takes one time step");
+    const int64_t B = x.size(0), H = p[3].size(0), D = p[3].size(1), W = H * D, K = p[1].size(2);
+    chk(p[1], "conv weight", at::kFloat, {W, 1, K});
+    chk(p[2], "conv bias", at::kFloat, {W});
+    for (int i = 3; i < 6; ++i) chk(p[i], "block-diagonal map", at::kFloat, {H, D, D});
+    for (int i : {6, 8}) chk(p[i], "gate weight", at::kFloat, {H, 3 * W}), chk(p[i + 1], "gate bias", at::kFloat, {H});
+    chk(p[10], "norm_weight", at::kFloat, {H, D});
+    chk(p[11], "learnable_skip", at::kFloat, {W});
+    const Tensor C = carry[0].contiguous(), lf = carry[1].contiguous(), n = carry[2].contiguous(), m = carry[3].contiguous();
+    chk(C, "C", at::kFloat, {B, 1, H, D, D});
+    chk(n, "n", at::kFloat, {B, 1, H, D, 1});
+    chk(lf, "log_f", at::kFloat, {B, 1, H, 1, 1});
+    chk(m, "m", at::kFloat, {B, 1, H, 1, 1});
+    const Done done(done_, B, 1);
+    const auto up = row_dense(x, norm, scale, nbias, eps, false, {p[0]}, {std::nullopt}, at::kFloat, at::kFloat, std::nullopt)[0];
+    const Tensor Co = fresh_like(C), lfo = fresh_like(lf), no = fresh_like(n), mo = fresh_like(m), y = fresh({B, 1, W}, at::kFloat, x);
+    TORCH_CHECK_VALUE(up.size(2) == 2 * W, "up projection");
+    check(lib.mrx_mlstm_step(stream(), fptr(up), fptr(p[1]), fptr(p[2]), fptr(p[3]), fptr(p[4]), fptr(p[5]), fptr(p[6]), fptr(p[7]), fptr(p[8]),
+                             fptr(p[9]), fptr(p[10]), fptr(p[11]), done.p(), fptr(C), fptr(lf), fptr(n), fptr(m), fptr(Co), fptr(lfo), fptr(no),
+                             fptr(mo), fptr(y), B, H, D, K, done.dtype, (float)g_floor),
+          "mrx_mlstm_step");
+    return {row_dense(y, 0, std::nullopt, std::nullopt, 0.0, false, {p[12]}, {std::nullopt}, at::kFloat, at::kFloat, x)[0], Co, lfo, no, mo};
 }
 
 constexpr int64_t ROW_DENSE_ROWS = 16384;   // up to here one launch beats the array library's products and casts
@@ -1657,7 +1714,13 @@ PYBIND11_MODULE(_native, m)
         auto r = delta_rule_step(q, k, v, beta, done, S, inplace, false);
         return std::make_tuple(r.o, r.S);
     });
-    def("row_dense", &row_dense);
+    def("row_dense", [](const Tensor &x, int norm, const OptTensor &scale, const OptTensor &nbias, double eps, bool round_norm,
+                        const std::vector<Tensor> &weights, const std::vector<OptTensor> &biases, ScalarType product, ScalarType out_dtype,
+                        const OptTensor &residual) {
+        return row_dense(x, norm, scale, nbias, eps, round_norm, weights, biases, product, out_dtype, residual);
+    });
+    def("lru_act", &lru_act);
+    def("mlstm_act", &mlstm_act);
     def("mingru_step", &mingru_step);
     // differentiable operators (memorax_amd/functional.py)
     def("linear_scan", &linear_scan);

@@ -25,6 +25,10 @@ constexpr int RD_MAX_K = 2048;
 struct RowDenseArgs {
     const void *x;
     const float *scale, *nbias, *residual;
+    const float *skip;      // K factors: skip_out = x + skip * norm(x), for the residual branch of a cell with a feed-through term
+    float *skip_out;
+    const void *w2;         // a single layer whose weights lie in two arrays: columns k1 .. K
+    int k1;
     const void *w[MRX_ROW_DENSE_LAYERS], *b[MRX_ROW_DENSE_LAYERS];
     void *y[MRX_ROW_DENSE_LAYERS];
     int n[MRX_ROW_DENSE_LAYERS], first_tile[MRX_ROW_DENSE_LAYERS + 1];   // columns of a layer, its first 64-column tile
@@ -132,7 +136,11 @@ __global__ void __launch_bounds__(RD_THREADS) row_dense_kernel(RowDenseArgs a)
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct) {
                 const int k = (s0 + s) * KB + KP * g, row = n0 + ct * 16 + i16;   // K is a multiple of KP
-                if (row < N && k < a.K) next[s][ct] = weight_raw<T, WBF>(w, (int64_t)row * a.K + k);
+                if (row < N && k < a.K) {
+                    const bool second = a.w2 && k >= a.k1;
+                    const int wide = a.w2 ? (second ? a.K - a.k1 : a.k1) : a.K;
+                    next[s][ct] = weight_raw<T, WBF>(second ? a.w2 : w, (int64_t)row * wide + (second ? k - a.k1 : k));
+                }
                 else next[s][ct] = RawFrag<T, WBF>{};
             }
     };
@@ -192,6 +200,12 @@ __global__ void __launch_bounds__(RD_THREADS) row_dense_kernel(RowDenseArgs a)
                         o.v[e] = o.v[e] * rstd * sc[i].v[e] + nb[i].v[e];
                         if (a.round_norm) o.v[e] = (float)(__bf16)o.v[e];
                     }
+                if (a.skip_out && tile == 0 && r0 + wv * RPW + j < a.rows && c < a.K) {
+                    const int64_t at = (r0 + wv * RPW + j) * a.K + c;
+                    const Quad x = a.x_bf16 ? quad_of<true>(a.x, at) : quad_of<false>(a.x, at), d = quad_of<false>(a.skip, c);
+                    *reinterpret_cast<f32x4 *>(a.skip_out + at) =
+                        f32x4{x.v[0] + d.v[0] * o.v[0], x.v[1] + d.v[1] * o.v[1], x.v[2] + d.v[2] * o.v[2], x.v[3] + d.v[3] * o.v[3]};
+                }
                 *reinterpret_cast<typename TT<T>::pack4 *>(sx + (wv * RPW + j) * ld + c) = TT<T>::pack(o.v[0], o.v[1], o.v[2], o.v[3]);
             }
         }
@@ -323,7 +337,7 @@ const KernelRegistrar registrars[] = {
 extern "C" int mrx_row_dense(void *stream, const void *x, const float *scale, const float *norm_bias, int norm, int round_norm,
                              const void *const *weights, const void *const *biases, void *const *outs, const int64_t *n_out, int layers,
                              const float *residual, int64_t rows, int64_t K, int x_dtype, int w_dtype, int b_dtype, int y_dtype,
-                             int product_dtype, float eps)
+                             int product_dtype, float eps, const void *weights2, int64_t k1, const float *skip, float *skip_out)
 {
     using namespace mrx;
     auto known = [](int dt) { return dt == MRX_F32 || dt == MRX_BF16; };
@@ -333,7 +347,10 @@ extern "C" int mrx_row_dense(void *stream, const void *x, const float *scale, co
         return MRX_ERR_INVALID_ARG;
     if (residual && (layers != 1 || y_dtype != MRX_F32)) return MRX_ERR_INVALID_ARG;
     if (K % 8 != 0 || K > RD_MAX_K) return MRX_ERR_UNSUPPORTED;
+    if (weights2 && (layers != 1 || k1 <= 0 || k1 >= K || k1 % 8 != 0 || !aligned(weights2, 16))) return MRX_ERR_INVALID_ARG;
+    if ((skip == nullptr) != (skip_out == nullptr) || !aligned(skip, 16) || !aligned(skip_out, 16)) return MRX_ERR_INVALID_ARG;
     RowDenseArgs a{};
+    a.w2 = weights2, a.k1 = (int)k1, a.skip = skip, a.skip_out = skip_out;
     a.x = x, a.scale = scale, a.nbias = norm_bias, a.residual = residual;
     a.layers = layers, a.K = (int)K, a.norm = norm, a.rows = rows, a.eps = eps, a.inv_K = 1.f / (float)K;
     a.x_bf16 = x_dtype == MRX_BF16, a.w_bf16 = w_dtype == MRX_BF16, a.b_bf16 = b_dtype == MRX_BF16, a.y_bf16 = y_dtype == MRX_BF16;

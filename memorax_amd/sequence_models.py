@@ -243,6 +243,14 @@ class LRUCell(_DiagonalCell):
     def read(self, h, x, **kwargs):
         return _real_read_out(h[0], torch.stack([self.C_real, -self.C_imag], -1)) + self.D * x
 
+    def acting(self, x, norm, done, carry):
+        params = [self.nu_log, self.theta_log, self.gamma_log, self.B_real, self.B_imag, self.C_real, self.C_imag, self.D]
+        if not (_as_written(self, LRUCell) and autocast_dtype(x) is None and self.hidden_dim % 8 == 0 and 2 * self.hidden_dim <= _RMS_NORM_MAX_D
+                and all(p.dtype is torch.float32 for p in params)):
+            return None
+        y, *carry = native().lru_act(x, *_norm_of(norm), params, done, *carry)
+        return tuple(carry), y
+
     def initialize_carry(self, key, input_shape):
         *batch, _ = input_shape
         dev = self.nu_log.device
@@ -455,13 +463,17 @@ def _row_layers(x, layers):
                                and (m.bias is None or m.bias.dtype in (torch.float32, torch.bfloat16)) for m in layers)
 
 
+def _norm_of(norm):
+    """A norm as the row kernels take it: kind, scale, bias, eps."""
+    if norm is None:
+        return 0, None, None, 0.0
+    return (1, norm.scale, None, norm.eps) if type(norm) is _RMSNorm else (2, norm.weight, norm.bias, norm.eps)
+
+
 def _rows(x, norm, layers, product, out_dtype, residual=None):
     """norm(x) through the layers in one launch, as _RMSNorm / _LayerNorm / Dense would compute it; residual: added to the one result."""
-    rms = type(norm) is _RMSNorm
-    kind = 0 if norm is None else 1 if rms else 2
-    scale = None if norm is None else norm.scale if rms else norm.weight
-    return native().row_dense(x, kind, scale, None if norm is None or rms else norm.bias, 0.0 if norm is None else norm.eps,
-                              x.dtype == torch.bfloat16, [m.weight for m in layers], [m.bias for m in layers], product, out_dtype, residual)
+    return native().row_dense(x, *_norm_of(norm), x.dtype == torch.bfloat16, [m.weight for m in layers], [m.bias for m in layers], product,
+                              out_dtype, residual)
 
 
 def _as_written(cell, cls):
@@ -859,6 +871,17 @@ class mLSTMCell(MemoroidCellBase):
         q, k, v, z, u = self._project(x)
         h, carry = self.scan(self._elements(q, k, v), initial_carry, done)
         return carry, self._read_out(h, x, z, u)
+
+    def acting(self, x, norm, done, carry):
+        H, d = self.num_heads, self.hidden_dim // self.num_heads
+        params = [self.up_projection.weight, self.causal_conv.weight, self.causal_conv.bias, self.query.kernel, self.key.kernel, self.value.kernel,
+                  self.i_gate.weight, self.i_gate.bias, self.f_gate.weight, self.f_gate.bias, self.norm_weight, self.learnable_skip,
+                  self.output_projection.weight]
+        if not (_as_written(self, mLSTMCell) and autocast_dtype(x) is None and d in (16, 32, 64) and H <= 8 and H * d <= 256
+                and all(p.dtype is torch.float32 for p in params)):
+            return None
+        y, *carry = native().mlstm_act(x, *_norm_of(norm), params, done, list(carry), self._G_FLOOR)
+        return tuple(carry), y
 
     def binary_operator(self, a, b):
         C_a, log_f_a, n_a, m_a = a

@@ -97,3 +97,33 @@ def test_acting_blocks_equal_their_composition(d, autocast):
                 for a, b in zip(carry, ref):
                     assert a.shape == b.shape and a.dtype == b.dtype and relerr(a, _np(b)) <= tol, (name, relerr(a, _np(b)))
                 ref = tuple(c.detach() for c in ref)
+
+
+@pytest.mark.parametrize("cell", ["lru 8", "lru 136", "mlstm 1 16", "mlstm 3 16", "mlstm 8 32", "mlstm 2 64", "mlstm 4 64"])
+@pytest.mark.parametrize("B", [1, 45])
+def test_acting_lru_and_mlstm_blocks_equal_their_composition(cell, B):
+    from memorax_amd import sequence_models as sm
+    torch.manual_seed(B)
+    Fe = 72
+    kind, *sizes = cell.split()
+    sizes = [int(s) for s in sizes]
+    make = (lambda: sm.LRUCell(Fe, *sizes)) if kind == "lru" else (lambda: sm.mLSTMCell(Fe, hidden_dim=sizes[0] * sizes[1], num_heads=sizes[0]))
+    for norm in (sm.RMSNorm, sm.LayerNorm):
+        block = sm.Residual(sm.PreNorm(sm.Memoroid(make()), Fe, norm=norm)).cuda()
+        with torch.no_grad():   # initial zeros would hide a wrong index
+            for p in block.parameters():
+                p.add_(0.1 * torch.randn_like(p))
+        if kind == "lru":
+            block.module.module.cell.gamma_log.data.clamp_(max=0.3)
+        carry = ref = block.initialize_carry(None, (B, Fe))
+        for t in range(4):
+            x, done = torch.randn(B, 1, Fe, device="cuda"), torch.rand(B, 1, device="cuda") < 0.3
+            ref, want = block(x, done, ref)
+            with torch.no_grad():
+                carry, y = block(x, done, carry)
+            assert y.dtype == want.dtype and relerr(y, _np(want)) <= 1e-4, (t, relerr(y, _np(want)))
+            for a, b in zip(carry, ref):
+                assert a.shape == b.shape and a.dtype == b.dtype
+                a, b = (torch.view_as_real(v.detach().contiguous()) if v.is_complex() else v.detach() for v in (a, b))
+                assert relerr(a, _np(b)) <= 1e-4, (t, relerr(a, _np(b)))
+            ref = tuple(c.detach() for c in ref)
