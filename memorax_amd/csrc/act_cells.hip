@@ -5,6 +5,8 @@
 // forty-eight; a step of an agent is bound by their number, on the host as on the device.
 #include <math.h>
 
+#include <type_traits>
+
 #include "common.h"
 
 namespace mrx {
@@ -60,6 +62,19 @@ struct MlstmStepArgs {
     float g_floor;
 };
 __device__ __forceinline__ float silu(float x) { return x / (1.f + __expf(-x)); }
+// Sum over groups of 4, 8 or 16 lanes, in every one of them: DPP moves.
+template <int LANES> __device__ __forceinline__ float lanes_total(float x)
+{
+    auto add = [&](auto ctrl) {
+        const int moved = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, true);
+        x += __builtin_bit_cast(float, moved);
+    };
+    add(std::integral_constant<int, 0xB1>{});    // quad_perm [1,0,3,2]
+    add(std::integral_constant<int, 0x4E>{});    // quad_perm [2,3,0,1]
+    if constexpr (LANES >= 8) add(std::integral_constant<int, 0x141>{});    // row_half_mirror
+    if constexpr (LANES >= 16) add(std::integral_constant<int, 0x140>{});   // row_mirror
+    return x;
+}
 template <int D> __device__ __forceinline__ float head_total(float x)   // over the D lanes that hold a head's values
 {
 #pragma unroll
@@ -96,18 +111,28 @@ template <int D> __global__ void __launch_bounds__(256) mlstm_step_kernel(MlstmS
         su[t] = u;
     }
     __syncthreads();
-    float q = 0.f, k = 0.f, v = 0.f;
-    if (own) {
-        const f32x4 *rq = reinterpret_cast<const f32x4 *>(a.wq) + t * (D / 4), *rk = reinterpret_cast<const f32x4 *>(a.wk) + t * (D / 4),
-                    *rv = reinterpret_cast<const f32x4 *>(a.wv) + t * (D / 4);
+    // the block-diagonal maps: D / 4 lanes read a row together and sum over themselves (a row per lane touches a cache line per
+    // lane and load: 877 environments with four heads of 64 65 -> 32 us, where the state's way in and out is 19)
+    {
+        constexpr int LPR = D / 4, RPI = 64 / LPR;
+        const int j = lane % LPR;
 #pragma unroll
-        for (int j = 0; j < D / 4; ++j) {
-            const f32x4 uj = *reinterpret_cast<const f32x4 *>(su + h * D + 4 * j), xj = *reinterpret_cast<const f32x4 *>(sx + h * D + 4 * j);
-            const f32x4 a0 = rq[j], a1 = rk[j], a2 = rv[j];
+        for (int p = 0; p < LPR; ++p) {
+            const int r = w * 64 + p * RPI + lane / LPR, at = r / D * D + 4 * j;
+            if (w * 64 + p * RPI >= W) break;   // W is a multiple of the rows of an instruction
+            const f32x4 uj = *reinterpret_cast<const f32x4 *>(su + at), xj = *reinterpret_cast<const f32x4 *>(sx + at);
+            const f32x4 a0 = reinterpret_cast<const f32x4 *>(a.wq)[r * LPR + j], a1 = reinterpret_cast<const f32x4 *>(a.wk)[r * LPR + j],
+                        a2 = reinterpret_cast<const f32x4 *>(a.wv)[r * LPR + j];
+            float q = 0.f, k = 0.f, v = 0.f;
 #pragma unroll
             for (int e = 0; e < 4; ++e) q += a0[e] * uj[e], k += a1[e] * uj[e], v += a2[e] * xj[e];
+            q = lanes_total<LPR>(q), k = lanes_total<LPR>(k), v = lanes_total<LPR>(v);
+            if (j == 0) sq[r] = q, sk[r] = k, sv[r] = v;
         }
     }
+    __syncthreads();
+    float q = 0.f, k = 0.f, v = 0.f;
+    if (own) q = sq[t], k = sk[t], v = sv[t];
     // the gates of every head read all of (q | k | v), head by head
     for (int g = 0; g < 2 * H; ++g) {
         const float *row = (g < H ? a.wi + (int64_t)g * 3 * W : a.wf + (int64_t)(g - H) * 3 * W) + h * 3 * D + o;
@@ -135,7 +160,7 @@ template <int D> __global__ void __launch_bounds__(256) mlstm_step_kernel(MlstmS
             k *= weight[h];
             n = reset ? k : decay[h] * n_prev + k;
             a.n_out[b * W + t] = n;
-            sq[t] = q, sk[t] = k, sv[t] = v;
+            sk[t] = k;
         }
         const float qn = head_total<D>(own ? q * n : 0.f);
         if (own) den = fmaxf(fabsf(qn), floor_m[h]) + 1e-6f;
