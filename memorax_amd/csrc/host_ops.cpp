@@ -16,6 +16,7 @@
 #include <ATen/hip/HIPContextLight.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/utils/pybind.h>
@@ -104,6 +105,15 @@ void chk(const OptTensor &t, const char *name, ScalarType dt, IntArrayRef shape)
 {
     if (t.has_value() && t->defined()) chk(*t, name, dt, shape);
 }
+
+// contiguous and on a 16-byte boundary; the tensor itself where it is that already (a parameter may be a view into a flat vector)
+Tensor dense16(const Tensor &t)
+{
+    if (!t.defined()) return t;
+    const Tensor c = t.contiguous();
+    return reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 == 0 ? c : c.clone();
+}
+Tensor dense16(const OptTensor &t) { return t.has_value() ? dense16(*t) : Tensor(); }
 
 Tensor fresh(IntArrayRef shape, ScalarType dt, const Tensor &like)
 {
@@ -705,19 +715,26 @@ StepOut delta_rule_step(const Tensor &q, const Tensor &k, const Tensor &v, const
 }
 
 // ---- acting: dense layers on few rows, the MinGRU cell's step
+Tensor norm_param(const OptTensor &t) { return t.has_value() ? dense16(t->to(at::kFloat)) : Tensor(); }
+
 // norm: 0 none, 1 RMS, 2 layer norm.  The results keep x's leading axes; residual (float32, x's leading axes): added to the one
 // layer's result.
-std::vector<Tensor> row_dense(const Tensor &x, int norm, const OptTensor &scale, const OptTensor &nbias, double eps, bool round_norm,
-                              const std::vector<Tensor> &weights, const std::vector<OptTensor> &biases, ScalarType product, ScalarType out_dtype,
-                              const OptTensor &residual, const OptTensor &weight2 = std::nullopt, const OptTensor &skip = std::nullopt,
+std::vector<Tensor> row_dense(const Tensor &x_, int norm, const OptTensor &scale_, const OptTensor &nbias_, double eps, bool round_norm,
+                              std::vector<Tensor> weights, std::vector<OptTensor> biases, ScalarType product, ScalarType out_dtype,
+                              const OptTensor &residual_, const OptTensor &weight2_ = std::nullopt, const OptTensor &skip_ = std::nullopt,
                               Tensor *skip_out = nullptr)
 {
+    const Tensor x = dense16(x_), scale = norm_param(scale_), nbias = norm_param(nbias_), weight2 = dense16(weight2_), skip = dense16(skip_),
+                 residual = residual_.has_value() ? residual_->contiguous() : Tensor();
+    for (Tensor &w : weights) w = dense16(w);
+    for (OptTensor &b : biases)
+        if (b.has_value()) b = b->contiguous();
     TORCH_CHECK_VALUE(x.dim() >= 2 && !weights.empty() && weights.size() <= MRX_ROW_DENSE_LAYERS && biases.size() == weights.size(),
                       "row_dense takes rows and 1 to ", MRX_ROW_DENSE_LAYERS, " layers");
     const int64_t K = x.size(-1), rows = x.numel() / K;
     chk(x, "x");
-    chk(scale, "scale", at::kFloat, {K});
-    chk(nbias, "bias of the norm", at::kFloat, {K});
+    if (scale.defined()) chk(scale, "scale", at::kFloat, {K});
+    if (nbias.defined()) chk(nbias, "bias of the norm", at::kFloat, {K});
     const auto wd = weights[0].scalar_type();
     auto bd = at::kFloat;
     std::array<const void *, MRX_ROW_DENSE_LAYERS> w{}, b{};
@@ -729,7 +746,7 @@ std::vector<Tensor> row_dense(const Tensor &x, int norm, const OptTensor &scale,
     bool first_bias = true;
     for (size_t l = 0; l < weights.size(); ++l) {
         n[l] = weights[l].size(0);
-        chk(weights[l], "weight", wd, {n[l], weight2.has_value() ? K - weight2->size(1) : K});
+        chk(weights[l], "weight", wd, {n[l], weight2.defined() ? K - weight2.size(1) : K});
         if (biases[l].has_value()) {
             if (std::exchange(first_bias, false)) bd = biases[l]->scalar_type();
             chk(*biases[l], "bias", bd, {n[l]});
@@ -738,13 +755,13 @@ std::vector<Tensor> row_dense(const Tensor &x, int norm, const OptTensor &scale,
         out.push_back(fresh(shape, out_dtype, x));
         w[l] = ptr(weights[l]), b[l] = ptr(biases[l]), y[l] = ptr(out[l]);
     }
-    chk(residual, "residual", at::kFloat, out[0].sizes());
-    if (weight2.has_value()) chk(*weight2, "weight2", wd, {n[0], weight2->size(1)});
-    chk(skip, "skip", at::kFloat, {K});
-    if (skip.has_value()) *skip_out = fresh(x.sizes(), at::kFloat, x);
+    if (residual.defined()) chk(residual, "residual", at::kFloat, out[0].sizes());
+    if (weight2.defined()) chk(weight2, "weight2", wd, {n[0], weight2.size(1)});
+    if (skip.defined()) chk(skip, "skip", at::kFloat, {K});
+    if (skip.defined()) *skip_out = fresh(x.sizes(), at::kFloat, x);
     check(lib.mrx_row_dense(stream(), ptr(x), fptr(scale), fptr(nbias), norm, round_norm, w.data(), b.data(), y.data(), n.data(),
                             (int)weights.size(), fptr(residual), rows, K, code(x.scalar_type()), code(wd), code(bd), code(out_dtype),
-                            code(product), (float)eps, ptr(weight2), weight2.has_value() ? weights[0].size(1) : 0, fptr(skip),
+                            code(product), (float)eps, ptr(weight2), weight2.defined() ? weights[0].size(1) : 0, fptr(skip),
                             skip_out ? fptr(*skip_out) : nullptr),
           "mrx_row_dense");
     return out;
@@ -753,10 +770,11 @@ std::vector<Tensor> row_dense(const Tensor &x, int norm, const OptTensor &scale,
 // A pre-norm residual block around an LRU cell, one acting step: x (B,1,F) float32, the carry's leaves (B,1,N) complex64
 // -> y, h, P.  params: nu_log, theta_log, gamma_log, B_real, B_imag, C_real, C_imag, D.
 std::tuple<Tensor, Tensor, Tensor> lru_act(const Tensor &x, int norm, const OptTensor &scale, const OptTensor &nbias, double eps,
-                                           const std::vector<Tensor> &params, const Tensor &done_, const Tensor &h_, const Tensor &P_)
+                                           std::vector<Tensor> params, const Tensor &done_, const Tensor &h_, const Tensor &P_)
 {
     TORCH_CHECK_VALUE(x.dim() == 3 && x.size(1) == 1 && params.size() == 8, "lru_act takes one time step");
-    const int64_t B = x.size(0), F = x.size(2), N = params[0].size(0);
+    const int64_t B = x.size(0), N = params[0].size(0);
+    for (Tensor &t : params) t = dense16(t);
     for (int i = 0; i < 3; ++i) chk(params[i], "parameter", at::kFloat, {N});
     const Tensor h = h_.contiguous(), P = P_.contiguous();
     chk(h, "h", at::kComplexFloat, {B, 1, N});
@@ -774,18 +792,19 @@ std::tuple<Tensor, Tensor, Tensor> lru_act(const Tensor &x, int norm, const OptT
 
 // The same around an mLSTM cell; params: up, conv weight and bias, query, key, value, i_gate and f_gate (weight, bias), norm_weight,
 // learnable_skip, output projection; the carry's leaves C (B,1,H,D,D), log_f, n (B,1,H,D,1), m.
-std::vector<Tensor> mlstm_act(const Tensor &x, int norm, const OptTensor &scale, const OptTensor &nbias, double eps, const std::vector<Tensor> &p,
+std::vector<Tensor> mlstm_act(const Tensor &x, int norm, const OptTensor &scale, const OptTensor &nbias, double eps, std::vector<Tensor> p,
                               const Tensor &done_, const std::vector<Tensor> &carry, double g_floor)
 {
     TORCH_CHECK_VALUE(x.dim() == 3 && x.size(1) == 1 && p.size() == 13 && carry.size() == 4, "mlstm_act takes one time step");
     const int64_t B = x.size(0), H = p[3].size(0), D = p[3].size(1), W = H * D, K = p[1].size(2);
+    for (Tensor &t : p) t = dense16(t);
     chk(p[1], "conv weight", at::kFloat, {W, 1, K});
     chk(p[2], "conv bias", at::kFloat, {W});
     for (int i = 3; i < 6; ++i) chk(p[i], "block-diagonal map", at::kFloat, {H, D, D});
     for (int i : {6, 8}) chk(p[i], "gate weight", at::kFloat, {H, 3 * W}), chk(p[i + 1], "gate bias", at::kFloat, {H});
     chk(p[10], "norm_weight", at::kFloat, {H, D});
     chk(p[11], "learnable_skip", at::kFloat, {W});
-    const Tensor C = carry[0].contiguous(), lf = carry[1].contiguous(), n = carry[2].contiguous(), m = carry[3].contiguous();
+    const Tensor C = dense16(carry[0]), lf = carry[1].contiguous(), n = carry[2].contiguous(), m = carry[3].contiguous();
     chk(C, "C", at::kFloat, {B, 1, H, D, D});
     chk(n, "n", at::kFloat, {B, 1, H, D, 1});
     chk(lf, "log_f", at::kFloat, {B, 1, H, 1, 1});
@@ -825,9 +844,43 @@ std::tuple<Tensor, Tensor, Tensor> mingru_step(const Tensor &z, const Tensor &x,
 }
 
 // ------------------------------------------------------------------------------------------------ autograd nodes
+bool differentiable(const Tensor &t) { return t.defined() && t.requires_grad(); }
+bool differentiable(const OptTensor &t) { return t.has_value() && differentiable(*t); }
+
+// The nodes know no forward mode: an input with a tangent is refused, as an autograd function without a jvp refuses it.
+void refuse_tangent(const Tensor &t)
+{
+    TORCH_CHECK_NOT_IMPLEMENTED(!t.defined() || !t._fw_grad(0).defined(), "memorax_amd operators have no forward-mode derivative");
+}
+void refuse_tangent(const OptTensor &t)
+{
+    if (t.has_value()) refuse_tangent(*t);
+}
+template <typename... Ts> bool need_grad(const Ts &...ts)
+{
+    (refuse_tangent(ts), ...);
+    return at::GradMode::is_enabled() && (differentiable(ts) || ...);
+}
+
+// Gradients that say so when they are differentiated again, instead of passing for constants.
+variable_list refuse_second(variable_list &&grads)
+{
+    variable_list defined;
+    for (Tensor &g : grads)
+        if (g.defined()) defined.push_back(g.detach().set_requires_grad(true));
+    const auto error = std::make_shared<torch::autograd::DelayedError>(
+        "trying to differentiate twice a function that is differentiable once", (int64_t)defined.size());
+    defined = (*error)(std::move(defined));
+    size_t i = 0;
+    for (Tensor &g : grads)
+        if (g.defined()) g = defined[i++];
+    return std::move(grads);
+}
+
 // One node type for every operator: Op holds what is no tensor of the graph (flags, scalars, the reset flags) and
 //     static constexpr int SAVED          how many tensors the backward reads
 //     static const char *name()
+//     static constexpr bool ONCE          (where it is declared) differentiating the gradients again is an error
 //     variable_list backward(node, saved, grads)
 template <class Op> struct OpNode final : torch::autograd::Node {
     Op op;
@@ -844,8 +897,15 @@ template <class Op> struct OpNode final : torch::autograd::Node {
         std::lock_guard<std::mutex> lock(mutex_);
         std::array<Tensor, Op::SAVED> s;
         for (int i = 0; i < Op::SAVED; ++i) s[i] = saved[i].unpack(output[i] ? shared_from_this() : nullptr);
-        at::AutoDispatchBelowADInplaceOrView below;
-        return op.backward(*this, s, grads);
+        variable_list out;
+        {
+            at::AutoDispatchBelowADInplaceOrView below;
+            out = op.backward(*this, s, grads);
+        }
+        if constexpr (requires { Op::ONCE; })
+            if (at::GradMode::is_enabled() && std::any_of(grads.begin(), grads.end(), [](const Tensor &g) { return differentiable(g); }))
+                return refuse_second(std::move(out));
+        return out;
     }
     void release_variables() override
     {
@@ -865,9 +925,6 @@ template <class Op, typename... Ts> std::shared_ptr<OpNode<Op>> record(Op &&op, 
     return node;
 }
 
-bool differentiable(const Tensor &t) { return t.defined() && t.requires_grad(); }
-bool differentiable(const OptTensor &t) { return t.has_value() && differentiable(*t); }
-template <typename... Ts> bool need_grad(const Ts &...ts) { return at::GradMode::is_enabled() && (differentiable(ts) || ...); }
 
 Tensor unwrap(const OptTensor &t) { return t.has_value() ? *t : Tensor(); }
 OptTensor some(const Tensor &t) { return t.defined() ? OptTensor(t) : std::nullopt; }
@@ -1178,6 +1235,7 @@ std::tuple<Tensor, Tensor, Tensor> mlstm_gates(const Tensor &log_i, const Tensor
 
 struct SiluGateOp {
     static constexpr int SAVED = 2;   // h, g
+    static constexpr bool ONCE = true;
     static const char *name() { return "MemoraxSiluGateBackward"; }
     variable_list backward(OpNode<SiluGateOp> &, std::array<Tensor, 2> &s, variable_list &grads)
     {
@@ -1210,6 +1268,7 @@ Tensor silu_gate(const Tensor &h, const Tensor &g)
 // gradients of both meet in the norm's backward kernel instead of in a pass of their own.
 struct NormOp {
     static constexpr int SAVED = 2;   // x, scale
+    static constexpr bool ONCE = true;
     static const char *name() { return "MemoraxNormBackward"; }
     double eps;
     bool center, fork;
@@ -1343,6 +1402,7 @@ bool input_suits(ScalarType dt, int64_t rows, int64_t K, int64_t widest, size_t 
 // themselves (each adds onto the sum so far) instead of by a pass per layer.
 struct DenseOp {
     static constexpr int SAVED = 1;   // x as the products read it; the weights follow in `weights`
+    static constexpr bool ONCE = true;
     static const char *name() { return "MemoraxDenseBackward"; }
     std::vector<SavedVariable> weights;
     std::vector<bool> has_bias;
@@ -1458,6 +1518,7 @@ std::vector<Tensor> dense_group(const Tensor &x, const std::vector<Tensor> &weig
 // ---- causal depthwise convolution over time with silu behind it (conv_cells.hip)
 struct ConvSiluOp {
     static constexpr int SAVED = 3;   // x, weight, bias
+    static constexpr bool ONCE = true;
     static const char *name() { return "MemoraxCausalConvSiluBackward"; }
     variable_list backward(OpNode<ConvSiluOp> &, std::array<Tensor, 3> &s, variable_list &grads)
     {
@@ -1474,23 +1535,24 @@ struct ConvSiluOp {
 };
 
 // x (B,T,C) float32, dense or the leading columns of wider rows; weight (C,1,K), bias (C).
-Tensor causal_conv_silu(const Tensor &x_, const Tensor &weight, const Tensor &bias)
+Tensor causal_conv_silu(const Tensor &x_, const Tensor &weight_, const Tensor &bias_)
 {
-    TORCH_CHECK_VALUE(x_.dim() == 3 && weight.dim() == 3 && x_.is_cuda() && x_.scalar_type() == at::kFloat,
+    TORCH_CHECK_VALUE(x_.dim() == 3 && weight_.dim() == 3 && x_.is_cuda() && x_.scalar_type() == at::kFloat,
                       "causal_conv_silu takes (B,T,C) float32 arrays on the GPU");
-    const int64_t B = x_.size(0), T = x_.size(1), C = x_.size(2), K = weight.size(2);
-    chk(weight, "weight", at::kFloat, {C, 1, K});
-    chk(bias, "bias", at::kFloat, {C});
-    Tensor x, y;
+    const int64_t B = x_.size(0), T = x_.size(1), C = x_.size(2), K = weight_.size(2);
+    Tensor x, y, weight, bias;
     {
         at::AutoDispatchBelowADInplaceOrView below;
+        weight = dense16(weight_), bias = dense16(bias_);
+        chk(weight, "weight", at::kFloat, {C, 1, K});
+        chk(bias, "bias", at::kFloat, {C});
         const bool rows = x_.stride(2) == 1 && x_.stride(1) % 4 == 0 && x_.stride(0) == T * x_.stride(1) && ((uintptr_t)x_.data_ptr()) % 16 == 0;
-        x = rows ? x_ : x_.contiguous();
+        x = rows ? x_ : dense16(x_);
         y = fresh({B, T, C}, at::kFloat, x);
         check(lib.mrx_causal_conv_silu_fwd(stream(), fptr(x), x.stride(1), fptr(weight), fptr(bias), fptr(y), B, T, C, K), "mrx_causal_conv_silu_fwd");
     }
-    if (need_grad(x_, weight, bias)) {
-        auto node = record(ConvSiluOp{}, x_, weight, bias);
+    if (need_grad(x_, weight_, bias_)) {
+        auto node = record(ConvSiluOp{}, x_, weight_, bias_);
         torch::autograd::set_history(y, node);
         node->keep(0, x);
         node->keep(1, weight);
@@ -1506,6 +1568,7 @@ struct MambaSizes {
 
 struct MambaOp {
     enum { UP, BIN, CIN, DTIN, CONVW, CONVB, DTB, ALOG, D_, SCALE, V, K_, Q, G, O, SCHK, SLAST, SAVED };
+    static constexpr bool ONCE = true;
     static const char *name() { return "MemoraxMambaBackward"; }
     Tensor done;
     MambaSizes n;
@@ -1544,14 +1607,21 @@ struct MambaOp {
 
 // up (B,T,2HP), b_in, c_in (B,T,HN), dt_in (B,T,H) and the cell's parameters, all float32 -> y (B,T,HP) before the output
 // projection, S_last (B,H,P,N), decay_last (B,H).  Acting (one step, no gradients) runs the single-step kernel.
-std::tuple<Tensor, Tensor, Tensor> mamba_mix(const Tensor &up, const Tensor &b_in, const Tensor &c_in, const Tensor &dt_in, const Tensor &conv_w,
-                                             const Tensor &conv_b, const Tensor &dt_bias, const Tensor &A_log, const Tensor &D,
-                                             const Tensor &scale, const Tensor &done_, const Tensor &S0, const Tensor &decay0, double eps,
+std::tuple<Tensor, Tensor, Tensor> mamba_mix(const Tensor &up, const Tensor &b_in, const Tensor &c_in, const Tensor &dt_in, const Tensor &conv_w_,
+                                             const Tensor &conv_b_, const Tensor &dt_bias_, const Tensor &A_log_, const Tensor &D_,
+                                             const Tensor &scale_, const Tensor &done_, const Tensor &S0, const Tensor &decay0, double eps,
                                              bool in_place)
 {
-    TORCH_CHECK_VALUE(up.dim() == 3 && S0.dim() == 4 && conv_w.dim() == 3, "mamba_mix: up (B,T,2HP), S0 (B,H,P,N), conv_w (C,1,K)");
-    MambaSizes n{up.size(0), up.size(1), S0.size(1), S0.size(2), S0.size(3), conv_w.size(2), S0.size(1) * S0.size(2)};
+    TORCH_CHECK_VALUE(up.dim() == 3 && S0.dim() == 4 && conv_w_.dim() == 3, "mamba_mix: up (B,T,2HP), S0 (B,H,P,N), conv_w (C,1,K)");
+    MambaSizes n{up.size(0), up.size(1), S0.size(1), S0.size(2), S0.size(3), conv_w_.size(2), S0.size(1) * S0.size(2)};
     const int64_t C = n.W + 2 * n.H * n.N;
+    const bool need = need_grad(up, b_in, c_in, dt_in, conv_w_, conv_b_, dt_bias_, A_log_, D_, scale_, S0, decay0);
+    Tensor conv_w, conv_b, dt_bias, A_log, D, scale;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        conv_w = dense16(conv_w_), conv_b = dense16(conv_b_), dt_bias = dense16(dt_bias_), A_log = dense16(A_log_), D = dense16(D_),
+        scale = dense16(scale_);
+    }
     chk(up, "up", at::kFloat, {n.B, n.T, 2 * n.W});
     chk(b_in, "b_in", at::kFloat, {n.B, n.T, n.H * n.N});
     chk(c_in, "c_in", at::kFloat, {n.B, n.T, n.H * n.N});
@@ -1562,7 +1632,6 @@ std::tuple<Tensor, Tensor, Tensor> mamba_mix(const Tensor &up, const Tensor &b_i
     chk(A_log, "A_log", at::kFloat, {n.H});
     chk(D, "D", at::kFloat, {n.H});
     chk(scale, "scale", at::kFloat, {n.W});
-    const bool need = need_grad(up, b_in, c_in, dt_in, conv_w, conv_b, dt_bias, A_log, D, scale, S0, decay0);
     Tensor v, k, q, g, o, S_chk, S_last, y, decay0_, decay_last;
     {
         at::AutoDispatchBelowADInplaceOrView below;
@@ -1590,7 +1659,7 @@ std::tuple<Tensor, Tensor, Tensor> mamba_mix(const Tensor &up, const Tensor &b_i
         check(lib.mrx_decay_last(stream(), fptr(g), done.p(), fptr(decay0_), fptr(decay_last), n.B, n.T, n.H, done.dtype), "mrx_decay_last");
     }
     if (need) {
-        auto node = record(MambaOp{done_, n, eps, decay0_}, up, b_in, c_in, dt_in, conv_w, conv_b, dt_bias, A_log, D, scale, S0, decay0);
+        auto node = record(MambaOp{done_, n, eps, decay0_}, up, b_in, c_in, dt_in, conv_w_, conv_b_, dt_bias_, A_log_, D_, scale_, S0, decay0);
         torch::autograd::set_history(y, node);
         torch::autograd::set_history(S_last, node);
         torch::autograd::set_history(decay_last, node);

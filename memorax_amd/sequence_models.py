@@ -29,6 +29,8 @@ import torch.nn.functional as F
 
 from typing import NamedTuple
 
+from torch.nn.modules.module import _has_any_global_hook as _any_global_hook
+
 from ._lib import native
 from .dense import Dense, Weights, autocast_dtype, dense, dense_group
 from .functional import (deltanet, gated_linear_attention, linear_attention, linear_scan, mingru_scan, mlstm_gates,
@@ -162,7 +164,7 @@ class Memoroid(SequenceModel):
     def forward(self, inputs, done, initial_carry=None, **kwargs):
         if initial_carry is None:
             initial_carry = self.cell.initialize_carry(None, get_input_shape(inputs))
-        whole = self.cell.whole(inputs, done, initial_carry)
+        whole = None if kwargs or _hooked(self.cell) else self.cell.whole(inputs, done, initial_carry)
         if whole is not None:
             return whole
         z = self.cell(inputs, **kwargs)
@@ -459,8 +461,23 @@ def _row_layers(x, layers):
     """Whether the row kernels multiply with these layers' weights as they are (under autocast: whatever dtype the products run in)."""
     wd = layers[0].weight.dtype
     plain = (torch.float32,) if autocast_dtype(x) is None else (torch.float32, torch.bfloat16)
-    return wd in plain and all(m.weight.dtype == wd and m.weight.shape[1] % 8 == 0 and m.weight.shape[1] <= _RMS_NORM_MAX_D
+    return wd in plain and all(_plain(m) and m.weight.dtype == wd and m.weight.shape[1] % 8 == 0 and m.weight.shape[1] <= _RMS_NORM_MAX_D
                                and (m.bias is None or m.bias.dtype in (torch.float32, torch.bfloat16)) for m in layers)
+
+
+def _hooked(module):
+    """Whether a hook waits in this module or below, or for every module: fused operations do not run the modules they stand for."""
+    return _any_global_hook() or _any_hook(module)
+
+
+def _any_hook(m):
+    return bool(m._forward_pre_hooks or m._forward_hooks or m._backward_hooks or m._backward_pre_hooks
+                or any(c is not None and _any_hook(c) for c in m._modules.values()))
+
+
+def _plain(layer):
+    """A layer that a product with its weight stands for."""
+    return type(layer) in (Dense, nn.Linear)
 
 
 def _norm_of(norm):
@@ -566,7 +583,7 @@ class LinearAttentionCell(MemoroidCellBase):
 
     def acting(self, x, norm, done, carry):
         layers = [self.value, self.key, self.query]
-        if not (_as_written(self, LinearAttentionCell) and _row_layers(x, [*layers, self.output_projection])):
+        if not (type(self.norm) is _RMSNorm and _as_written(self, LinearAttentionCell) and _row_layers(x, [*layers, self.output_projection])):
             return None
         product = autocast_dtype(x) or x.dtype
         z = tuple(self._heads(t) for t in _rows(x, norm, layers, product, product))
@@ -633,7 +650,7 @@ class DeltaNetCell(MemoroidCellBase):
 
     def acting(self, x, norm, done, carry):
         layers = [self.query, self.key, self.value, self.beta]
-        if not (_as_written(self, DeltaNetCell) and self.dtype in (torch.float32, torch.bfloat16)
+        if not (type(self.norm) is _RMSNorm and _as_written(self, DeltaNetCell) and self.dtype in (torch.float32, torch.bfloat16)
                 and _row_layers(x, [*layers, self.output_projection])):
             return None
         product = autocast_dtype(x) or x.dtype
@@ -651,7 +668,7 @@ def _causal_conv_silu(x, conv):
     """silu of a depthwise convolution over time that sees the steps up to its own and nothing before the call's first
     (mamba.py:88-106): the library's kernel where it takes the arrays, else the array library's operations."""
     K = conv.kernel_size[0]
-    if (x.is_cuda and x.dtype == torch.float32 and conv.weight.dtype == torch.float32 and autocast_dtype(x) is None and K <= 4
+    if (not _hooked(conv) and x.is_cuda and x.dtype == torch.float32 and conv.weight.dtype == torch.float32 and autocast_dtype(x) is None and K <= 4
             and x.shape[2] % 4 == 0 and x.numel() > 0):
         return native().causal_conv_silu(x, conv.weight, conv.bias)
     return F.silu(conv(F.pad(x.transpose(1, 2), (K - 1, 0)))).transpose(1, 2)
@@ -733,7 +750,9 @@ class MambaCell(MemoroidCellBase):
 
     def _native_sizes(self):
         P = self.head_dim
-        return (P % 4 == 0 and P <= 64 and self.state_dim in (4, 8, 16, 32, 64) and self.conv_dim <= 4
+        return (type(self.norm) is _RMSNorm and self.norm.scale.dtype == torch.float32 and _plain(self.output_projection)
+                and type(self.conv) is nn.Conv1d and self.conv.bias is not None
+                and P % 4 == 0 and P <= 64 and self.state_dim in (4, 8, 16, 32, 64) and self.conv_dim <= 4
                 and self.num_heads * P <= _RMS_NORM_MAX_D and self.conv.weight.dtype == torch.float32)
 
     def _mix(self, projections, done, carry):
@@ -845,7 +864,8 @@ class mLSTMCell(MemoroidCellBase):
     def _heads_as_one(self, x):
         """Heads of up to 64 features go through one product with the block-diagonal matrix: a batched product of such narrow
         blocks, its permutations and its weight gradients over every row cost several times the zeros' arithmetic."""
-        return x.is_cuda and autocast_dtype(x) is None and self.hidden_dim // self.num_heads <= 64 and self.num_heads <= 8
+        return (x.is_cuda and autocast_dtype(x) is None and self.hidden_dim // self.num_heads <= 64 and self.num_heads <= 8
+                and all(type(m) is _BlockDiagonalDense and not _hooked(m) for m in (self.query, self.key, self.value)))
 
     def forward(self, x, **kwargs):
         """Elements in kernel form: (k / sqrt(d), v, log_i, log_f, q)."""
@@ -864,6 +884,12 @@ class mLSTMCell(MemoroidCellBase):
         log_f = F.logsigmoid(f_pre.float())
         return (k / math.sqrt(d), v, log_i, log_f, q)
 
+    def _parts_as_written(self):
+        blocks, dense = (self.query, self.key, self.value), (self.up_projection, self.i_gate, self.f_gate, self.output_projection)
+        return (all(type(m) is _BlockDiagonalDense for m in blocks) and all(map(_plain, dense)) and type(self.causal_conv) is nn.Conv1d
+                and self.up_projection.bias is None and self.output_projection.bias is None
+                and all(m.bias is not None for m in (self.causal_conv, self.i_gate, self.f_gate)))
+
     def whole(self, x, done, initial_carry):
         """The composition below with the projections formed once (``read`` forms them again)."""
         if not (x.is_cuda and x.dim() == 3 and _as_written(self, mLSTMCell)):
@@ -877,7 +903,7 @@ class mLSTMCell(MemoroidCellBase):
         params = [self.up_projection.weight, self.causal_conv.weight, self.causal_conv.bias, self.query.kernel, self.key.kernel, self.value.kernel,
                   self.i_gate.weight, self.i_gate.bias, self.f_gate.weight, self.f_gate.bias, self.norm_weight, self.learnable_skip,
                   self.output_projection.weight]
-        if not (_as_written(self, mLSTMCell) and autocast_dtype(x) is None and d in (16, 32, 64) and H <= 8 and H * d <= 256
+        if not (_as_written(self, mLSTMCell) and self._parts_as_written() and autocast_dtype(x) is None and d in (16, 32, 64) and H <= 8 and H * d <= 256
                 and all(p.dtype is torch.float32 for p in params)):
             return None
         y, *carry = native().mlstm_act(x, *_norm_of(norm), params, done, list(carry), self._G_FLOOR)
@@ -1012,7 +1038,8 @@ class Residual(nn.Module):
 
     def forward(self, inputs, done=None, initial_carry=None, **kwargs):
         inner = self.module
-        if type(inner) is PreNorm and not kwargs and hasattr(inner.module, "acting") and _acts(inputs, done, inner.norm):
+        if (type(inner) is PreNorm and not kwargs and hasattr(inner.module, "acting") and _acts(inputs, done, inner.norm)
+                and not _hooked(inner)):
             acted = inner.module.acting(inputs, inner.norm, done, initial_carry)
             if acted is not None:
                 return acted

@@ -1,0 +1,50 @@
+"""Acting steps on parameters and inputs as programs have them: views into flat vectors, hooks, second names."""
+import pytest
+import torch
+
+from memorax_amd import sequence_models as sm
+
+pytestmark = pytest.mark.gpu
+
+CELLS = {"lru": lambda: sm.LRUCell(64, 64), "mamba": lambda: sm.MambaCell(64, num_heads=2, head_dim=16, state_dim=16),
+         "mlstm": lambda: sm.mLSTMCell(64, hidden_dim=64, num_heads=2), "linear_attention": lambda: sm.LinearAttentionCell(64, 16, 2),
+         "delta": lambda: sm.DeltaNetCell(64, 16, 2)}
+
+
+def _block(cell):
+    torch.manual_seed(0)
+    with torch.device("cuda"):
+        return sm.Residual(sm.PreNorm(sm.Memoroid(CELLS[cell]()), 64)).cuda()
+
+
+@pytest.mark.parametrize("T", [1, 5])
+@pytest.mark.parametrize("cell", sorted(CELLS))
+def test_parameters_off_their_boundaries(cell, T):
+    """Parameters that are views into a vector at odd offsets, a misaligned input: the same numbers."""
+    block = _block(cell)
+    x, done = torch.randn(6, T, 64, device="cuda"), torch.zeros(6, T, dtype=torch.bool, device="cuda")
+    with torch.no_grad():
+        want = block(x, done)[1]
+        for name, p in block.named_parameters():
+            if T > 1 and "norm" in name:   # the norm kernels over whole rollouts take aligned parameters only
+                continue
+            flat = torch.empty(p.numel() + 1, device="cuda", dtype=p.dtype)
+            flat[1:] = p.flatten()
+            p.data = flat[1:].view(p.shape)
+        if T == 1:
+            flat = torch.empty(x.numel() + 1, device="cuda")
+            flat[1:] = x.flatten()
+            x = flat[1:].view(x.shape)
+        got = block(x, done)[1]
+    # the same kernels or the array library's products in another order of summation: float32 sums of 64 terms, bfloat16 for delta
+    torch.testing.assert_close(got, want, rtol=0, atol=2e-2 if cell == "delta" else 1e-5 * float(want.abs().max()))
+
+
+@pytest.mark.parametrize("cell", sorted(CELLS))
+def test_a_hook_runs(cell):
+    block = _block(cell)
+    seen = []
+    block.module.module.cell.register_forward_hook(lambda m, i, o: seen.append(1))
+    with torch.no_grad():
+        block(torch.randn(6, 1, 64, device="cuda"), torch.zeros(6, 1, dtype=torch.bool, device="cuda"))
+    assert seen
