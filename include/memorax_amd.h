@@ -489,6 +489,30 @@ int mrx_mingru_scan_bwd_segmented(void *stream, const void *z, const void *h_til
                                   void *dh0, int64_t B, int64_t T, int64_t D, int dtype, int done_dtype,
                                   void *workspace);
 
+/* ---- the normalised and the gated form on grids that do not fill the device -----------------
+ * As mrx_linear_attn_*_chunk_parallel (the rule of mrx_linear_attn_chunk_parallel_pays holds for them too): S_chk (required) is
+ * float32 and dense, and so is z_chk (required); the calls of a pair must be of the same kind.
+ * normalised: workspace (B,H,ceil(T/chunk)) x (dv dk + dk) float32.  gated: dec (B,H,ceil(T/chunk)) float32 scratch of the
+ * forward call; workspace (B,H,ceil(T/chunk)) x (dv dk + 1) float32; S_last is required. */
+int mrx_linear_attn_norm_fwd_chunk_parallel(void *stream, const void *q, const void *k, const void
+    *v, const void *done, const void *S0, const float *z0, void *o, float *den, float *ss, void
+    *S_last, float *z_last, float *S_chk, float *z_chk, int64_t B, int64_t T, int64_t H, int64_t dk,
+    int64_t dv, int dtype, int done_dtype, int feature_map, float eps);
+int mrx_linear_attn_norm_bwd_chunk_parallel(void *stream, const void *q, const void *k, const void
+    *v, const void *done, const float *S_chk, const float *z_chk, const void *o, const float *den,
+    const void *dout, const float *d_ss, const void *dS_last, const float *dz_last, void *dq, void
+    *dk_out, void *dv_out, void *dS0, float *dz0, float *workspace, int64_t B, int64_t T, int64_t H,
+    int64_t dk, int64_t dv, int dtype, int done_dtype, int feature_map, float eps);
+int mrx_gated_linear_attn_fwd_chunk_parallel(void *stream, const void *q, const void *k, const void
+    *v, const float *g, const void *done, const void *S0, void *o, void *S_last, float *S_chk, float
+    *dec, int64_t B, int64_t T, int64_t H, int64_t dk, int64_t dv, int dtype, int done_dtype, int
+    feature_map);
+int mrx_gated_linear_attn_bwd_chunk_parallel(void *stream, const void *q, const void *k, const void
+    *v, const float *g, const void *done, const float *S_chk, const float *S_last, const void *dout,
+    const void *dS_last, void *dq, void *dk_out, void *dv_out, float *dg, void *dS0, float
+    *workspace, int64_t B, int64_t T, int64_t H, int64_t dk, int64_t dv, int dtype, int done_dtype,
+    int feature_map);
+
 /* ---- Gated linear attention: linear attention with a scalar decay per step and head ----
  * The Mamba cell's algebra (mamba.py:109-122: elements (h_t = (B_t dt_t) (x) x_t, decay_t =
  * exp(dt_t A)), binary_operator (decay_j h_i + h_j, decay_j decay_i), read y_t = C_t . h_t), scanned

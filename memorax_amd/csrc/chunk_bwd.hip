@@ -84,10 +84,11 @@ struct NormBwdArgs {
 // walks the chunks and their episodes from the end anyway, so wave 0 carries that running sum in
 // a register (a reverse cumulative sum over the chunk's rows by lane shuffles, cut at resets) and
 // writes dg itself.
-// PAR (plain linear attention): one workgroup per chunk (grid.y = chunk).  Slot c of S_chk holds, in
-// fp32, the state entering chunk c and slot c of dS_last -- then a (B,H,NC,64,64) array -- the gradient
+// PAR: one workgroup per chunk (grid.y = chunk).  Slot c of S_chk (z_chk) holds, in
+// fp32, the state entering chunk c and slot c of dS_last (dz_last) -- then a (B,H,NC,64,64) array -- the gradient
 // of the state leaving it (la_states.h); the workgroup forms the chunk's dQ, dK, dV from them and neither
-// walks the state nor accumulates its gradient.
+// walks the state nor accumulates its gradient.  Gated: the running sum behind dg enters a chunk as <S, dS> of the state that
+// leaves it, which is what the sum over the later steps of the episode comes to.
 // NARROW: narrow heads, as in the forward kernel: q, k and their gradients are dka wide in memory, v, dout, o and
 // dv dva, states [dva][dka], z [dka]; tiles keep the build's width, zero beyond, and only the rows' own
 // width is ever stored.
@@ -100,7 +101,6 @@ la_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restr
               float *__restrict__ dS0, int Tlen, int H, NormBwdArgs na, int dka, int dva)
 {
     static_assert(!(GATED && NORM), "the normalised read-out belongs to plain linear attention");
-    static_assert(!PAR || (!GATED && !NORM), "one workgroup per chunk: plain linear attention only");
     constexpr int NW = 4, NTHR = 64 * NW;
     using L = LaBwdSmem<T, C, GATED, NORM>;
     using Frag = typename TT<T>::frag;
@@ -159,8 +159,9 @@ la_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restr
         const int dkt = TMS::mt(w, mi * TMS::NBW) * 16;
         dzacc[mi] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (NORM && na.dz_last) {
-            if (VN) { if (!NARROW || dkt + li < dkw) dzacc[mi][0] = na.dz_last[(int64_t)bh * dkw + dkt + li]; }
-            else if (!NARROW || dkt + 4 * lg < dkw) dzacc[mi] = *reinterpret_cast<const f32x4 *>(na.dz_last + (int64_t)bh * dkw + dkt + 4 * lg);
+            const float *dz_in = na.dz_last + (PAR ? (int64_t)bh * NC + c_hi : (int64_t)bh) * dkw;
+            if (VN) { if (!NARROW || dkt + li < dkw) dzacc[mi][0] = dz_in[dkt + li]; }
+            else if (!NARROW || dkt + 4 * lg < dkw) dzacc[mi] = *reinterpret_cast<const f32x4 *>(dz_in + dkt + 4 * lg);
         }
     }
 
@@ -170,7 +171,7 @@ la_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restr
     // only where the walk cannot pass -- chunks with resets -- and at every walk_anchor()-th chunk, where it
     // starts afresh from the exact state: the chunks the forward call writes then.
     // Gated: every chunk has a checkpoint in the I/O type, staged row-wise.
-    constexpr bool WALK = !GATED;
+    constexpr bool WALK = !GATED || PAR;  // PAR: the one state it needs waits in fp32 likewise
     constexpr int NSA = WALK ? TMS::TPW : 1;
     f32x4 Sacc[NSA];
     zero_acc<NSA>(Sacc);
@@ -186,13 +187,16 @@ la_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restr
 
     // gated: the running sum behind dg, held by wave 0; it starts from <S_last, dS_last>
     float dg_carry = 0.f;
-    if (GATED && dS_last && S_last) {
+    const float *S_out = PAR && c_hi + 1 < NC ? reinterpret_cast<const float *>(S_chk) + (slot + dvw) * dkw  // the state leaving the walk's first chunk
+                         : S_last             ? S_last + (int64_t)bh * dvw * dkw
+                                              : nullptr;
+    if (GATED && dS_last && S_out) {
         float part = 0.f;
 #pragma unroll
         for (int j = 0; j < TMS::TPW; ++j) {
             const int dk0 = TMS::mt(w, j) * 16 + 4 * lg, dvv = TMS::nt(w, j) * 16 + li;
             if (!in_state(dvv, dk0)) continue;
-            const f32x4 sl = *reinterpret_cast<const f32x4 *>(S_last + ((int64_t)bh * dvw + dvv) * dkw + dk0);
+            const f32x4 sl = *reinterpret_cast<const f32x4 *>(S_out + (int64_t)dvv * dkw + dk0);
             part += dSacc[j][0] * sl[0] + dSacc[j][1] * sl[1] + dSacc[j][2] * sl[2] + dSacc[j][3] * sl[3];
         }
 #pragma unroll
@@ -1405,6 +1409,78 @@ MRX_EXPORT int MRX_API(mrx_linear_attn_bwd_chunk_parallel)(void *stream, const v
                   : launch_la<__bf16, LA_BF16_CHUNK, false, false, false, true>(MRX_ARGS);
     return fm ? launch_la<float, 32, true, false, false, true>(MRX_ARGS)
               : launch_la<float, 32, false, false, false, true>(MRX_ARGS);
+#undef MRX_ARGS
+}
+
+// The same for the gated and the normalised form.
+MRX_EXPORT int MRX_API(mrx_gated_linear_attn_bwd_chunk_parallel)(void *stream, const void *q, const void *k, const void *v, const float *g,
+                                                        const void *done, const float *S_chk, const float *S_last, const void *dout,
+                                                        const void *dS_last, void *dq, void *dk_out, void *dv_out, float *dg, void *dS0,
+                                                        float *workspace, int64_t B, int64_t T, int64_t H, int64_t dk, int64_t dv,
+                                                        int dtype, int done_dtype, int feature_map)
+{
+#if MRX_HD == 64
+    if (dk <= 32 && dv <= 32) return mrx_gated_linear_attn_bwd_chunk_parallel_hd32(stream, q, k, v, g, done, S_chk, S_last, dout, dS_last, dq, dk_out, dv_out, dg, dS0, workspace, B, T, H, dk, dv, dtype, done_dtype, feature_map);
+#endif
+    const int rc = check_bwd(q, k, v, done, S_chk, dout, dS_last, dq, dk_out, dv_out, dS0, B, T, H, dk,
+                             dv, dtype, done_dtype, true);
+    if (rc != MRX_OK) return rc;
+    if (!g || !dg || !aligned(g, 4) || !aligned(dg, 4) || !S_last || !aligned(S_last, 16)) return MRX_ERR_INVALID_ARG;
+    if (!workspace || !aligned(workspace, 16)) return MRX_ERR_INVALID_ARG;
+    if (feature_map != MRX_FMAP_NONE && feature_map != MRX_FMAP_ELU1) return MRX_ERR_INVALID_ARG;
+    hipStream_t st = (hipStream_t)stream;
+    const bool fm = feature_map == MRX_FMAP_ELU1;
+    const int C = (int)mrx_chunk_size(dtype);
+    const int64_t NC = (T + C - 1) / C;
+    if (NC > 65535) return MRX_ERR_INVALID_ARG;
+    LaStateArgs a;
+    a.glog = g, a.dec = workspace + B * H * NC * dk * dv;
+    int rc2 = launch_la_chunk_states(st, q, dout, done, done_dtype, workspace, B, T, H, dtype, fm, true, dk, dv, a);
+    if (rc2 != MRX_OK) return rc2;
+    rc2 = launch_la_state_scan(st, workspace, (const float *)dS_last, (float *)dS0, done, done_dtype, B, T, H, C, true, dk, dv, a);
+    if (rc2 != MRX_OK) return rc2;
+#define MRX_ARGS st, q, k, v, done, done_dtype, S_chk, S_last, dout, workspace, dq, dk_out, dv_out, nullptr, B, T, H, g, dg, NormBwdArgs{}, dk, dv
+    if (dtype == MRX_BF16)
+        return fm ? launch_la<__bf16, LA_BF16_CHUNK, true, true, false, true>(MRX_ARGS)
+                  : launch_la<__bf16, LA_BF16_CHUNK, false, true, false, true>(MRX_ARGS);
+    return fm ? launch_la<float, 32, true, true, false, true>(MRX_ARGS) : launch_la<float, 32, false, true, false, true>(MRX_ARGS);
+#undef MRX_ARGS
+}
+
+MRX_EXPORT int MRX_API(mrx_linear_attn_norm_bwd_chunk_parallel)(void *stream, const void *q, const void *k, const void *v, const void *done,
+                                                       const float *S_chk, const float *z_chk, const void *o, const float *den,
+                                                       const void *dout, const float *d_ss, const void *dS_last, const float *dz_last,
+                                                       void *dq, void *dk_out, void *dv_out, void *dS0, float *dz0, float *workspace,
+                                                       int64_t B, int64_t T, int64_t H, int64_t dk, int64_t dv, int dtype,
+                                                       int done_dtype, int feature_map, float eps)
+{
+#if MRX_HD == 64
+    if (dk <= 32 && dv <= 32) return mrx_linear_attn_norm_bwd_chunk_parallel_hd32(stream, q, k, v, done, S_chk, z_chk, o, den, dout, d_ss, dS_last, dz_last, dq, dk_out, dv_out, dS0, dz0, workspace, B, T, H, dk, dv, dtype, done_dtype, feature_map, eps);
+#endif
+    const int rc = check_bwd(q, k, v, done, S_chk, dout, dS_last, dq, dk_out, dv_out, dS0, B, T, H, dk,
+                             dv, dtype, done_dtype, true);
+    if (rc != MRX_OK) return rc;
+    if (!z_chk || !o || !den || !workspace || !aligned(workspace, 16)) return MRX_ERR_INVALID_ARG;
+    if (!aligned(z_chk, 16) || !aligned(o, 16) || !aligned(den, 4) || !aligned(d_ss, 4) || !aligned(dz_last, 16) || !aligned(dz0, 16))
+        return MRX_ERR_INVALID_ARG;
+    if (feature_map != MRX_FMAP_NONE && feature_map != MRX_FMAP_ELU1) return MRX_ERR_INVALID_ARG;
+    hipStream_t st = (hipStream_t)stream;
+    const bool fm = feature_map == MRX_FMAP_ELU1;
+    const int C = (int)mrx_chunk_size(dtype);
+    const int64_t NC = (T + C - 1) / C;
+    if (NC > 65535) return MRX_ERR_INVALID_ARG;
+    LaStateArgs a;
+    a.z = workspace + B * H * NC * dk * dv, a.o = o, a.den = den, a.d_ss = d_ss, a.eps = eps, a.z_init = dz_last, a.z_fin = dz0;
+    int rc2 = launch_la_chunk_states(st, q, dout, done, done_dtype, workspace, B, T, H, dtype, fm, true, dk, dv, a);
+    if (rc2 != MRX_OK) return rc2;
+    rc2 = launch_la_state_scan(st, workspace, (const float *)dS_last, (float *)dS0, done, done_dtype, B, T, H, C, true, dk, dv, a);
+    if (rc2 != MRX_OK) return rc2;
+    const NormBwdArgs na{o, den, z_chk, a.z, nullptr, eps, d_ss};
+#define MRX_ARGS st, q, k, v, done, done_dtype, S_chk, nullptr, dout, workspace, dq, dk_out, dv_out, nullptr, B, T, H, nullptr, nullptr, na, dk, dv
+    if (dtype == MRX_BF16)
+        return fm ? launch_la<__bf16, LA_BF16_CHUNK, true, false, true, true>(MRX_ARGS)
+                  : launch_la<__bf16, LA_BF16_CHUNK, false, false, true, true>(MRX_ARGS);
+    return fm ? launch_la<float, 32, true, false, true, true>(MRX_ARGS) : launch_la<float, 32, false, false, true, true>(MRX_ARGS);
 #undef MRX_ARGS
 }
 

@@ -74,8 +74,8 @@ struct NormArgs {
 // TMIN (delta rule): the triangular factors have been computed by delta_tm_kernel and are read from
 // Tm_chk like any other input; the kernel then has neither the K K^T product nor the inverse and
 // a chunk costs four barriers.  Without it (no Tm_chk buffer given) the inverse runs in here.
-// PAR (plain linear attention): one workgroup per chunk (grid.y = chunk) instead of one per sequence.
-// S_chk then is an input: slot c holds, in fp32, the state entering chunk c (la_states.h); the
+// PAR (linear attention, its gated and normalised forms): one workgroup per chunk (grid.y = chunk) instead of one per
+// sequence.  S_chk (and z_chk) then is an input: slot c holds, in fp32, the state entering chunk c (la_states.h); the
 // workgroup forms the chunk's outputs from it and neither updates nor writes any state.
 // NARROW (every variant): narrow heads.  Keys and queries are dka wide in memory, values
 // and outputs dva (both at most the head dim of the build, whole 16-byte segments), and so are the
@@ -104,7 +104,7 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
     static_assert(!NORM || (!DELTA && !GATED), "the normalised read-out belongs to plain linear attention");
     static_assert(!PRO || DELTA, "the prologue belongs to the delta rule");
     static_assert(!TMIN || (DELTA && C == 32), "precomputed factors belong to the delta rule's 32-row chunks");
-    static_assert(!PAR || (!DELTA && !GATED && !NORM), "one workgroup per chunk: plain linear attention only");
+    static_assert(!PAR || !DELTA, "one workgroup per chunk: linear attention only");
     static_assert(!MERGE || (TMIN && !NARROW), "merged episodes: the delta rule on precomputed factors, full-width heads");
     using IOT = TileIO<T, C, NTHR, C>;  // the [C][C] triangular factor
     using L = FwdSmem<T, C, DELTA, GATED, NORM>;
@@ -172,9 +172,10 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
     for (int mi = 0; mi < TMS::MBW; ++mi) {
         const int dkt = TMS::mt(w, mi * TMS::NBW) * 16;
         zacc[mi] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (NORM && na.z0) {
-            if (VN) { if (!NARROW || dkt + li < dkw) zacc[mi][0] = na.z0[(int64_t)bh * dkw + dkt + li]; }
-            else if (!NARROW || dkt + 4 * lg < dkw) zacc[mi] = *reinterpret_cast<const f32x4 *>(na.z0 + (int64_t)bh * dkw + dkt + 4 * lg);
+        const float *z_in = PAR ? na.z_chk + ((int64_t)bh * NC + c_first) * dkw : na.z0 ? na.z0 + (int64_t)bh * dkw : nullptr;
+        if (NORM && z_in) {
+            if (VN) { if (!NARROW || dkt + li < dkw) zacc[mi][0] = z_in[dkt + li]; }
+            else if (!NARROW || dkt + 4 * lg < dkw) zacc[mi] = *reinterpret_cast<const f32x4 *>(z_in + dkt + 4 * lg);
         }
     }
     const Frag ones = TT<T>::ones();
@@ -371,7 +372,7 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
 #pragma unroll
                     for (int mi = 0; mi < TMS::MBW; ++mi) {
                         const int dkt = TMS::mt(w, mi * TMS::NBW) * 16;
-                        float *zc = (na.z_chk && pass == 0) ? na.z_chk + ((int64_t)bh * NC + c) * dkw + dkt : nullptr;
+                        float *zc = (!PAR && na.z_chk && pass == 0) ? na.z_chk + ((int64_t)bh * NC + c) * dkw + dkt : nullptr;
                         if (VN) {
                             sZ[dkt + li] = (T)zacc[mi][0];
                             if (zc && (!NARROW || dkt + li < dkw)) zc[li] = zacc[mi][0];
@@ -858,6 +859,71 @@ MRX_EXPORT int MRX_API(mrx_linear_attn_fwd_chunk_parallel)(void *stream, const v
                   : launch<__bf16, LA_BF16_CHUNK, false, false, false, false, false, false, true>(MRX_ARGS);
     return fm ? launch<float, 32, false, true, false, false, false, false, true>(MRX_ARGS)
               : launch<float, 32, false, false, false, false, false, false, true>(MRX_ARGS);
+#undef MRX_ARGS
+}
+
+// The same for the gated and the normalised form.
+MRX_EXPORT int MRX_API(mrx_gated_linear_attn_fwd_chunk_parallel)(void *stream, const void *q, const void *k, const void *v, const float *g,
+                                                        const void *done, const void *S0, void *o, void *S_last, float *S_chk,
+                                                        float *dec, int64_t B, int64_t T, int64_t H, int64_t dk, int64_t dv, int dtype,
+                                                        int done_dtype, int feature_map)
+{
+#if MRX_HD == 64
+    if (dk <= 32 && dv <= 32) return mrx_gated_linear_attn_fwd_chunk_parallel_hd32(stream, q, k, v, g, done, S0, o, S_last, S_chk, dec, B, T, H, dk, dv, dtype, done_dtype, feature_map);
+#endif
+    const int rc = check_common(q, k, v, done, o, S0, S_last, S_chk, B, T, H, dk, dv, dtype, done_dtype, true);
+    if (rc != MRX_OK) return rc;
+    if (!S_chk || !dec || !g || !aligned(g, 4) || !aligned(dec, 4)) return MRX_ERR_INVALID_ARG;
+    if (feature_map != MRX_FMAP_NONE && feature_map != MRX_FMAP_ELU1) return MRX_ERR_INVALID_ARG;
+    hipStream_t st = (hipStream_t)stream;
+    const bool fm = feature_map == MRX_FMAP_ELU1;
+    const int C = (int)mrx_chunk_size(dtype);
+    if ((T + C - 1) / C > 65535) return MRX_ERR_INVALID_ARG;
+    LaStateArgs a;
+    a.glog = g, a.dec = dec;
+    int rc2 = launch_la_chunk_states(st, k, v, done, done_dtype, S_chk, B, T, H, dtype, fm, false, dk, dv, a);
+    if (rc2 != MRX_OK) return rc2;
+    rc2 = launch_la_state_scan(st, S_chk, (const float *)S0, (float *)S_last, done, done_dtype, B, T, H, C, false, dk, dv, a);
+    if (rc2 != MRX_OK) return rc2;
+#define MRX_ARGS st, q, k, v, nullptr, done, done_dtype, nullptr, o, nullptr, S_chk, nullptr, B, T, H, g, NormArgs{}, dk, dv
+    if (dtype == MRX_BF16)
+        return fm ? launch<__bf16, LA_BF16_CHUNK, false, true, true, false, false, false, true>(MRX_ARGS)
+                  : launch<__bf16, LA_BF16_CHUNK, false, false, true, false, false, false, true>(MRX_ARGS);
+    return fm ? launch<float, 32, false, true, true, false, false, false, true>(MRX_ARGS)
+              : launch<float, 32, false, false, true, false, false, false, true>(MRX_ARGS);
+#undef MRX_ARGS
+}
+
+MRX_EXPORT int MRX_API(mrx_linear_attn_norm_fwd_chunk_parallel)(void *stream, const void *q, const void *k, const void *v, const void *done,
+                                                       const void *S0, const float *z0, void *o, float *den, float *ss, void *S_last,
+                                                       float *z_last, float *S_chk, float *z_chk, int64_t B, int64_t T, int64_t H,
+                                                       int64_t dk, int64_t dv, int dtype, int done_dtype, int feature_map, float eps)
+{
+#if MRX_HD == 64
+    if (dk <= 32 && dv <= 32) return mrx_linear_attn_norm_fwd_chunk_parallel_hd32(stream, q, k, v, done, S0, z0, o, den, ss, S_last, z_last, S_chk, z_chk, B, T, H, dk, dv, dtype, done_dtype, feature_map, eps);
+#endif
+    const int rc = check_common(q, k, v, done, o, S0, S_last, S_chk, B, T, H, dk, dv, dtype, done_dtype, true);
+    if (rc != MRX_OK) return rc;
+    if (!S_chk || !z_chk || !den || !aligned(den, 4) || !aligned(ss, 4) || !aligned(z0, 16) || !aligned(z_last, 16) || !aligned(z_chk, 16))
+        return MRX_ERR_INVALID_ARG;
+    if (feature_map != MRX_FMAP_NONE && feature_map != MRX_FMAP_ELU1) return MRX_ERR_INVALID_ARG;
+    hipStream_t st = (hipStream_t)stream;
+    const bool fm = feature_map == MRX_FMAP_ELU1;
+    const int C = (int)mrx_chunk_size(dtype);
+    if ((T + C - 1) / C > 65535) return MRX_ERR_INVALID_ARG;
+    LaStateArgs a;
+    a.z = z_chk, a.z_init = z0, a.z_fin = z_last;
+    int rc2 = launch_la_chunk_states(st, k, v, done, done_dtype, S_chk, B, T, H, dtype, fm, false, dk, dv, a);
+    if (rc2 != MRX_OK) return rc2;
+    rc2 = launch_la_state_scan(st, S_chk, (const float *)S0, (float *)S_last, done, done_dtype, B, T, H, C, false, dk, dv, a);
+    if (rc2 != MRX_OK) return rc2;
+    const NormArgs na{nullptr, den, nullptr, z_chk, eps, ss};
+#define MRX_ARGS st, q, k, v, nullptr, done, done_dtype, nullptr, o, nullptr, S_chk, nullptr, B, T, H, nullptr, na, dk, dv
+    if (dtype == MRX_BF16)
+        return fm ? launch<__bf16, LA_BF16_CHUNK, false, true, false, true, false, false, true>(MRX_ARGS)
+                  : launch<__bf16, LA_BF16_CHUNK, false, false, false, true, false, false, true>(MRX_ARGS);
+    return fm ? launch<float, 32, false, true, false, true, false, false, true>(MRX_ARGS)
+              : launch<float, 32, false, false, false, true, false, false, true>(MRX_ARGS);
 #undef MRX_ARGS
 }
 

@@ -49,7 +49,8 @@ using torch::autograd::variable_list;
     X(mrx_gated_linear_attn_step) X(mrx_delta_rule_step) X(mrx_causal_conv_silu_fwd) X(mrx_causal_conv_silu_bwd)     \
     X(mrx_mamba_elements_fwd) X(mrx_mamba_elements_bwd) X(mrx_decay_last) X(mrx_mamba_readout_fwd)                   \
     X(mrx_mamba_readout_bwd) X(mrx_deltanet_step) X(mrx_mingru_step) X(mrx_row_dense) X(mrx_dense_grads) X(mrx_dense_grads_workspace)                  \
-    X(mrx_lru_step) X(mrx_mlstm_step)
+    X(mrx_lru_step) X(mrx_mlstm_step) X(mrx_linear_attn_norm_fwd_chunk_parallel) X(mrx_linear_attn_norm_bwd_chunk_parallel) \
+    X(mrx_gated_linear_attn_fwd_chunk_parallel) X(mrx_gated_linear_attn_bwd_chunk_parallel)
 struct {
 #define MRX_MEMBER(name) decltype(&::name) name = nullptr;
     MRX_BOUND(MRX_MEMBER)
@@ -441,6 +442,16 @@ AttnOut linear_attn_fwd(const Tensor &q, const Tensor &k, const Tensor &v, const
     return r;
 }
 
+// Whether the gated or the normalised form cuts the work along time, a workgroup per chunk: the library's rule, and on heads of up to
+// 32 features more than twelve chunks.  The six launches of a forward and backward pair take the host 82 us, two take it 70; a
+// sequential pair's chain costs 12 us a chunk in bfloat16 (64 features), 7 us up to 32 features (bfloat16, 32 sequences: 8 chunks 100
+// -> 81 and 65 -> 83 us, 16 chunks 180 -> 81 and 112 -> 83 us, 32 chunks 334 -> 87 and 219 -> 82 us; float32 of 64 features, 128
+// sequences of 64 chunks 736 -> 505 us, 192 of 8 to 64 chunks level).
+bool chunk_parallel_pays(const Shape &s)
+{
+    return lib.mrx_linear_attn_chunk_parallel_pays(s.B, s.T, s.H, code(s.dt)) != 0 && (std::max(s.dk, s.dv) > 32 || s.chunks() > 12);
+}
+
 struct AttnGrads {
     Tensor dq, dk, dv, extra, dS0, dz0;   // extra: the gradient of the gate (gated: dg, delta rule: dbeta)
 };
@@ -471,35 +482,44 @@ AttnGrads linear_attn_bwd(const Tensor &q, const Tensor &k, const Tensor &v, con
 
 struct NormAttnOut {
     Tensor o, den, S_last, z_last, S_chk, z_chk, ss;
+    bool parallel;   // as in AttnOut
 };
 
 NormAttnOut linear_attn_norm_fwd(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &done_, const OptTensor &S0,
-                                 const OptTensor &z0, int fmap, double eps, bool save_chk, bool want_ss)
+                                 const OptTensor &z0, int fmap, double eps, bool save_chk, bool want_ss, bool chunk_parallel = false)
 {
     const Shape s(q, k, v);
     chk(S0, "S0", at::kFloat, s.state());
     chk(z0, "z0", at::kFloat, {s.B, s.H, s.dk});
     const Done done(done_, s.B, s.T);
     NormAttnOut r;
+    r.parallel = chunk_parallel && chunk_parallel_pays(s);
     r.o = fresh_like(v);
     r.den = fresh({s.B, s.H, s.T}, at::kFloat, q);
     r.S_last = fresh(s.state(), at::kFloat, q);
     r.z_last = fresh({s.B, s.H, s.dk}, at::kFloat, q);
-    if (save_chk) {
+    if (save_chk || r.parallel) {
         r.S_chk = fresh({s.B, s.H, s.chunks(), s.dv, s.dk}, at::kFloat, q);
         r.z_chk = fresh({s.B, s.H, s.chunks(), s.dk}, at::kFloat, q);
     }
     if (want_ss) r.ss = fresh({s.B, s.H, s.T}, at::kFloat, q);
-    check(lib.mrx_linear_attn_norm_fwd(stream(), ptr(q), ptr(k), ptr(v), done.p(), fptr(S0), fptr(z0), ptr(r.o), fptr(r.den), fptr(r.ss),
-                                       fptr(r.S_last), fptr(r.z_last), fptr(r.S_chk), fptr(r.z_chk), s.B, s.T, s.H, s.dk, s.dv, code(s.dt),
-                                       done.dtype, fmap, (float)eps),
-          "mrx_linear_attn_norm_fwd");
+    if (r.parallel)
+        check(lib.mrx_linear_attn_norm_fwd_chunk_parallel(stream(), ptr(q), ptr(k), ptr(v), done.p(), fptr(S0), fptr(z0), ptr(r.o), fptr(r.den),
+                                                          fptr(r.ss), fptr(r.S_last), fptr(r.z_last), fptr(r.S_chk), fptr(r.z_chk), s.B, s.T,
+                                                          s.H, s.dk, s.dv, code(s.dt), done.dtype, fmap, (float)eps),
+              "mrx_linear_attn_norm_fwd_chunk_parallel");
+    else
+        check(lib.mrx_linear_attn_norm_fwd(stream(), ptr(q), ptr(k), ptr(v), done.p(), fptr(S0), fptr(z0), ptr(r.o), fptr(r.den), fptr(r.ss),
+                                           fptr(r.S_last), fptr(r.z_last), fptr(r.S_chk), fptr(r.z_chk), s.B, s.T, s.H, s.dk, s.dv,
+                                           code(s.dt), done.dtype, fmap, (float)eps),
+              "mrx_linear_attn_norm_fwd");
     return r;
 }
 
 AttnGrads linear_attn_norm_bwd(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &done_, const Tensor &S_chk,
                                const Tensor &z_chk, const Tensor &S_last, const Tensor &o, const Tensor &den, const Tensor &dout,
-                               const OptTensor &dS_last, const OptTensor &dz_last, int fmap, double eps, bool want_d0, const OptTensor &d_ss)
+                               const OptTensor &dS_last, const OptTensor &dz_last, int fmap, double eps, bool want_d0, const OptTensor &d_ss,
+                               bool parallel = false)
 {
     const Shape s(q, k, v);
     chk(S_last, "S_last", at::kFloat, s.state());
@@ -514,6 +534,15 @@ AttnGrads linear_attn_norm_bwd(const Tensor &q, const Tensor &k, const Tensor &v
     const Done done(done_, s.B, s.T);
     AttnGrads r{fresh_like(q), fresh_like(k), fresh_like(v), {}, want_d0 ? fresh(s.state(), at::kFloat, q) : Tensor(),
                 want_d0 ? fresh({s.B, s.H, s.dk}, at::kFloat, q) : Tensor()};
+    if (parallel) {
+        const Tensor ws = fresh({s.B, s.H, s.chunks(), s.dv + 1, s.dk}, at::kFloat, q);
+        check(lib.mrx_linear_attn_norm_bwd_chunk_parallel(stream(), ptr(q), ptr(k), ptr(v), done.p(), fptr(S_chk), fptr(z_chk), ptr(o), fptr(den),
+                                                          ptr(dout), fptr(d_ss), fptr(dS_last), fptr(dz_last), ptr(r.dq), ptr(r.dk), ptr(r.dv),
+                                                          fptr(r.dS0), fptr(r.dz0), fptr(ws), s.B, s.T, s.H, s.dk, s.dv, code(s.dt), done.dtype,
+                                                          fmap, (float)eps),
+              "mrx_linear_attn_norm_bwd_chunk_parallel");
+        return r;
+    }
     check(lib.mrx_linear_attn_norm_bwd(stream(), ptr(q), ptr(k), ptr(v), done.p(), fptr(S_chk), fptr(S_last), fptr(z_chk), ptr(o), fptr(den),
                                        ptr(dout), fptr(d_ss), fptr(dS_last), fptr(dz_last), ptr(r.dq), ptr(r.dk), ptr(r.dv), fptr(r.dS0),
                                        fptr(r.dz0), s.B, s.T, s.H, s.dk, s.dv, code(s.dt), done.dtype, fmap, (float)eps),
@@ -522,14 +551,21 @@ AttnGrads linear_attn_norm_bwd(const Tensor &q, const Tensor &k, const Tensor &v
 }
 
 AttnOut gated_linear_attn_fwd(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &g, const Tensor &done_, const OptTensor &S0,
-                              int fmap, bool save_chk)
+                              int fmap, bool save_chk, bool chunk_parallel = false)
 {
     const Shape s(q, k, v);
     chk(g, "g", at::kFloat, {s.B, s.T, s.H});
     chk(S0, "S0", at::kFloat, s.state());
     const Done done(done_, s.B, s.T);
-    AttnOut r{fresh_like(v), fresh(s.state(), at::kFloat, q), {}, false};
-    if (save_chk) r.S_chk = fresh({s.B, s.H, s.chunks(), s.dv, s.dk}, s.dt, q);
+    AttnOut r{fresh_like(v), fresh(s.state(), at::kFloat, q), {}, chunk_parallel && chunk_parallel_pays(s)};
+    if (save_chk || r.parallel) r.S_chk = fresh({s.B, s.H, s.chunks(), s.dv, s.dk}, r.parallel ? at::kFloat : s.dt, q);
+    if (r.parallel) {
+        const Tensor dec = fresh({s.B, s.H, s.chunks()}, at::kFloat, q);
+        check(lib.mrx_gated_linear_attn_fwd_chunk_parallel(stream(), ptr(q), ptr(k), ptr(v), fptr(g), done.p(), fptr(S0), ptr(r.o), fptr(r.S_last),
+                                                           fptr(r.S_chk), fptr(dec), s.B, s.T, s.H, s.dk, s.dv, code(s.dt), done.dtype, fmap),
+              "mrx_gated_linear_attn_fwd_chunk_parallel");
+        return r;
+    }
     check(lib.mrx_gated_linear_attn_fwd(stream(), ptr(q), ptr(k), ptr(v), fptr(g), done.p(), fptr(S0), ptr(r.o), fptr(r.S_last), ptr(r.S_chk),
                                         s.B, s.T, s.H, s.dk, s.dv, code(s.dt), done.dtype, fmap),
           "mrx_gated_linear_attn_fwd");
@@ -537,17 +573,26 @@ AttnOut gated_linear_attn_fwd(const Tensor &q, const Tensor &k, const Tensor &v,
 }
 
 AttnGrads gated_linear_attn_bwd(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &g, const Tensor &done_, const Tensor &S_chk,
-                                const Tensor &dout, const OptTensor &dS_last, int fmap, bool want_dS0, const OptTensor &S_last)
+                                const Tensor &dout, const OptTensor &dS_last, int fmap, bool want_dS0, const OptTensor &S_last,
+                                bool parallel = false)
 {
     const Shape s(q, k, v);
     chk(g, "g", at::kFloat, {s.B, s.T, s.H});
     chk(dout, "do", s.dt, v.sizes());
-    chk(S_chk, "S_chk", s.dt, {s.B, s.H, s.chunks(), s.dv, s.dk});
+    chk(S_chk, "S_chk", parallel ? at::kFloat : s.dt, {s.B, s.H, s.chunks(), s.dv, s.dk});
     chk(dS_last, "dS_last", at::kFloat, s.state());
     chk(S_last, "S_last", at::kFloat, s.state());
     TORCH_CHECK_VALUE(!ptr(dS_last) || ptr(S_last), "S_last is required with dS_last");
     const Done done(done_, s.B, s.T);
     AttnGrads r{fresh_like(q), fresh_like(k), fresh_like(v), fresh_like(g), want_dS0 ? fresh(s.state(), at::kFloat, q) : Tensor(), {}};
+    if (parallel) {
+        const Tensor ws = fresh({s.B * s.H * s.chunks() * (s.dv * s.dk + 1)}, at::kFloat, q);
+        check(lib.mrx_gated_linear_attn_bwd_chunk_parallel(stream(), ptr(q), ptr(k), ptr(v), fptr(g), done.p(), fptr(S_chk), fptr(S_last), ptr(dout),
+                                                           fptr(dS_last), ptr(r.dq), ptr(r.dk), ptr(r.dv), fptr(r.extra), fptr(r.dS0), fptr(ws),
+                                                           s.B, s.T, s.H, s.dk, s.dv, code(s.dt), done.dtype, fmap),
+              "mrx_gated_linear_attn_bwd_chunk_parallel");
+        return r;
+    }
     check(lib.mrx_gated_linear_attn_bwd(stream(), ptr(q), ptr(k), ptr(v), fptr(g), done.p(), ptr(S_chk), fptr(S_last), ptr(dout),
                                         fptr(dS_last), ptr(r.dq), ptr(r.dk), ptr(r.dv), fptr(r.extra), fptr(r.dS0), s.B, s.T, s.H, s.dk, s.dv,
                                         code(s.dt), done.dtype, fmap),
@@ -1061,12 +1106,12 @@ struct NormalisedOp {
     Tensor done;
     int fmap;
     double eps;
-    bool has_ss;
+    bool has_ss, parallel;
     variable_list backward(OpNode<NormalisedOp> &node, std::array<Tensor, 8> &s, variable_list &grads)
     {
         auto r = linear_attn_norm_bwd(s[0], s[1], s[2], done, s[5], s[6], s[7], s[3], s[4], grad_or_zeros(grads[0], s[2]),
                                       some(as(grads[1], at::kFloat)), some(as(grads[2], at::kFloat)), fmap, eps, node.wants(3) || node.wants(4),
-                                      has_ss ? some(as(grads[3], at::kFloat)) : std::nullopt);
+                                      has_ss ? some(as(grads[3], at::kFloat)) : std::nullopt, parallel);
         return {r.dq, r.dk, r.dv, unless(!node.wants(3), r.dS0), unless(!node.wants(4), r.dz0)};
     }
 };
@@ -1090,10 +1135,10 @@ std::tuple<Tensor, Tensor, Tensor, OptTensor> normalised_linear_attention(const 
             if (want_ss) ss = st.o.to(at::kFloat).square().sum(-1).unsqueeze(-1);   // (B,H,1)
             return {st.o.unsqueeze(1), st.S, st.z, ss};
         }
-        r = linear_attn_norm_fwd(q_, k_, v_, done, some(S0_), some(z0_), fmap, eps, need, want_ss);
+        r = linear_attn_norm_fwd(q_, k_, v_, done, some(S0_), some(z0_), fmap, eps, need, want_ss, true);
     }
     if (need) {
-        auto node = record(NormalisedOp{done, fmap, eps, want_ss}, q, k, v, unwrap(S0), unwrap(z0));
+        auto node = record(NormalisedOp{done, fmap, eps, want_ss, r.parallel}, q, k, v, unwrap(S0), unwrap(z0));
         torch::autograd::set_history(r.o, node);
         torch::autograd::set_history(r.S_last, node);
         torch::autograd::set_history(r.z_last, node);
@@ -1115,10 +1160,11 @@ struct GatedOp {
     static const char *name() { return "MemoraxGatedLinearAttentionBackward"; }
     Tensor done;
     int fmap;
+    bool parallel;
     variable_list backward(OpNode<GatedOp> &node, std::array<Tensor, 6> &s, variable_list &grads)
     {
         auto r = gated_linear_attn_bwd(s[0], s[1], s[2], s[3], done, s[4], grad_or_zeros(grads[0], s[2]), some(as(grads[1], at::kFloat)), fmap,
-                                       node.wants(4), some(s[5]));
+                                       node.wants(4), some(s[5]), parallel);
         return {r.dq, r.dk, r.dv, r.extra, r.dS0};
     }
 };
@@ -1138,10 +1184,10 @@ std::tuple<Tensor, Tensor> gated_linear_attention(const Tensor &q, const Tensor 
                                              in_place && S0.has_value() && S0_.is_same(*S0));
             return {st.o.unsqueeze(1), st.S};
         }
-        r = gated_linear_attn_fwd(q_, k_, v_, g_, done, some(S0_), fmap, need);
+        r = gated_linear_attn_fwd(q_, k_, v_, g_, done, some(S0_), fmap, need, true);
     }
     if (need) {
-        auto node = record(GatedOp{done, fmap}, q, k, v, g, unwrap(S0));
+        auto node = record(GatedOp{done, fmap, r.parallel}, q, k, v, g, unwrap(S0));
         torch::autograd::set_history(r.o, node);
         torch::autograd::set_history(r.S_last, node);
         node->keep(0, q_);
@@ -1581,7 +1627,7 @@ struct MambaOp {
         check(lib.mrx_mamba_readout_bwd(stream(), fptr(s[O]), fptr(s[V]), fptr(up) + n.W, 2 * n.W, fptr(s[D_]), fptr(s[SCALE]), fptr(dy),
                                         fptr(d_o), fptr(d_up) + n.W, 2 * n.W, fptr(dscale), fptr(work), n.B * n.T, n.H, n.P, (float)eps),
               "mrx_mamba_readout_bwd");
-        auto r = gated_linear_attn_bwd(s[Q], s[K_], s[V], s[G], done, s[SCHK], d_o, some(as(grads[1], at::kFloat)), 0, node.wants(10), s[SLAST]);
+        auto r = gated_linear_attn_bwd(s[Q], s[K_], s[V], s[G], done, s[SCHK], d_o, some(as(grads[1], at::kFloat)), 0, node.wants(10), s[SLAST], parallel);
         Tensor ddecay0;
         if (grads[2].defined()) {   // the decay leaf handed on: it depends on every g from the last reset on
             const Tensor behind = done.ne(0).to(at::kInt).flip(1).cumsum(1).flip(1);   // resets at or after each step
@@ -1603,6 +1649,7 @@ struct MambaOp {
         return {d_up, db_in, dc_in, ddt, dw, dcb, ddtb, dA, dD, dscale, r.dS0, ddecay0};
     }
     Tensor decay0;
+    bool parallel;
 };
 
 // up (B,T,2HP), b_in, c_in (B,T,HN), dt_in (B,T,H) and the cell's parameters, all float32 -> y (B,T,HP) before the output
@@ -1633,6 +1680,7 @@ std::tuple<Tensor, Tensor, Tensor> mamba_mix(const Tensor &up, const Tensor &b_i
     chk(D, "D", at::kFloat, {n.H});
     chk(scale, "scale", at::kFloat, {n.W});
     Tensor v, k, q, g, o, S_chk, S_last, y, decay0_, decay_last;
+    bool parallel = false;
     {
         at::AutoDispatchBelowADInplaceOrView below;
         const Tensor S0_ = as(S0, at::kFloat);
@@ -1648,7 +1696,8 @@ std::tuple<Tensor, Tensor, Tensor> mamba_mix(const Tensor &up, const Tensor &b_i
                                              in_place && S0_.is_same(S0));
             o = st.o, S_last = st.S;
         } else {
-            auto r = gated_linear_attn_fwd(q, k, v, g, done.t, S0_, 0, need);
+            auto r = gated_linear_attn_fwd(q, k, v, g, done.t, S0_, 0, need, true);
+            parallel = r.parallel;
             o = r.o, S_last = r.S_last, S_chk = r.S_chk;
         }
         y = fresh({n.B, n.T, n.W}, at::kFloat, up);
@@ -1659,7 +1708,7 @@ std::tuple<Tensor, Tensor, Tensor> mamba_mix(const Tensor &up, const Tensor &b_i
         check(lib.mrx_decay_last(stream(), fptr(g), done.p(), fptr(decay0_), fptr(decay_last), n.B, n.T, n.H, done.dtype), "mrx_decay_last");
     }
     if (need) {
-        auto node = record(MambaOp{done_, n, eps, decay0_}, up, b_in, c_in, dt_in, conv_w_, conv_b_, dt_bias_, A_log_, D_, scale_, S0, decay0);
+        auto node = record(MambaOp{done_, n, eps, decay0_, parallel}, up, b_in, c_in, dt_in, conv_w_, conv_b_, dt_bias_, A_log_, D_, scale_, S0, decay0);
         torch::autograd::set_history(y, node);
         torch::autograd::set_history(S_last, node);
         torch::autograd::set_history(decay_last, node);

@@ -1,6 +1,8 @@
 // The kernels declared in la_states.h.
 #include "la_states.h"
 
+#include <type_traits>
+
 #include "chunk_common.h"
 
 namespace mrx {
@@ -13,16 +15,19 @@ namespace {
 // first episode (backward: what it adds to the gradient of the state that enters it).
 // NARROW: narrow heads -- x rows are dka wide in memory, y rows dva, a slot is [dva][dka]; the tiles keep the
 // build's width with zeros beyond (after the feature map).
-template <typename T, int C, bool FMAP, bool BWD, bool NARROW>
+// GATED, NORM: as in the chunk kernels; kept rows are weighted in fp32 before they are rounded to the tiles' type.
+template <typename T, int C, bool FMAP, bool BWD, bool NARROW, bool GATED, bool NORM>
 __global__ void __launch_bounds__(256)
 la_chunk_state_kernel(const T *__restrict__ x, const T *__restrict__ y, const void *__restrict__ done, int done_f32,
-                      float *__restrict__ slots, int Tlen, int H, int NC, int dka, int dva)
+                      float *__restrict__ slots, int Tlen, int H, int NC, int dka, int dva, LaStateArgs a)
 {
     constexpr int NW = 4, NTHR = 64 * NW, LDD = HD + pad_of<T>();
     using IO = TileIO<T, C, NTHR>;
     using TMS = TileMap<HD, HD, NW>;
     __shared__ __align__(16) T sX[C * LDD];
     __shared__ __align__(16) T sY[C * LDD];
+    __shared__ float sDd[NORM && BWD ? C : 1];           // dden of the kept rows
+    __shared__ float sPart[NORM ? NTHR : 1];             // partial column sums
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4;
@@ -36,20 +41,93 @@ la_chunk_state_kernel(const T *__restrict__ x, const T *__restrict__ y, const vo
     IO::zero(ry);
     if (segx) IO::load(rx, x + ((int64_t)b * Tlen * H + h) * dkw, (int64_t)H * dkw, t0, Tlen, tid);
     if (segy) IO::load(ry, y + ((int64_t)b * Tlen * H + h) * dvw, (int64_t)H * dvw, t0, Tlen, tid);
+    typename IO::Regs ro;
+    if (NORM && BWD) {
+        IO::zero(ro);
+        if (segy) IO::load(ro, static_cast<const T *>(a.o) + ((int64_t)b * Tlen * H + h) * dvw, (int64_t)H * dvw, t0, Tlen, tid);
+    }
+    float rg = 0.f;
+    if (GATED && lane < C && t0 + lane < Tlen) rg = a.glog[((int64_t)b * Tlen + t0 + lane) * H + h];
     const bool dn = lane < C && t0 + lane < Tlen && done_at(done, done_f32, (int64_t)b * Tlen + t0 + lane);
     const unsigned long long dmask = __ballot(dn);
     const int nres = __popcll(dmask);
     if (segx) IO::template fmap<FMAP>(rx);  // columns beyond a narrow head's width stay zero
+    const int ep = BWD ? 0 : nres;
+    auto keep = [&](int r) { return nres == 0 || episode_of(dmask, r) == ep; };
     if (nres != 0) {  // rows of other episodes leave by select: what they hold must not meet a zero in a product
-        const int ep = BWD ? 0 : nres;
-        auto keep = [&](int r) { return episode_of(dmask, r) == ep; };
         IO::mask_rows(rx, tid, keep);
         IO::mask_rows(ry, tid, keep);
+        if (NORM && BWD) IO::mask_rows(ro, tid, keep);
+    }
+    if (GATED) {
+        // G_i = sum of the log-decays of the kept episode up to row i, without its first step's (chunk kernels)
+        float G = lane < C && keep(lane) && !((dmask >> lane) & 1ull) ? rg : 0.f;
+#pragma unroll
+        for (int off = 1; off < C; off <<= 1) {
+            const float up = __shfl_up(G, off);
+            if (lane >= off) G += up;
+        }
+        const float Glast = __shfl(G, C - 1);
+        const float E = __expf(BWD ? G : Glast - G);
+        float f[IO::PASSES];
+#pragma unroll
+        for (int p = 0; p < IO::PASSES; ++p) f[p] = __shfl(E, IO::row_of(tid, p) % C);
+        IO::scale_rows(rx, f);
+        if (tid == 0) a.dec[(int64_t)bh * NC + c] = __expf(Glast);
+    }
+    if (NORM && !BWD && t0 + C > Tlen) IO::mask_rows(rx, tid, [&](int r) { return t0 + r < Tlen; });  // phi(0) = 1 must not count towards z
+    if (NORM && BWD) {
+        // dnum_i = dout_i / den_i in the place of dout_i, dden_i = -(dout_i . o_i) / den_i (chunk kernels)
+        float inv[IO::PASSES];
+#pragma unroll
+        for (int p = 0; p < IO::PASSES; ++p) {
+            const int r = IO::row_of(tid, p);
+            const bool on = (IO::FULL || r < C) && t0 + r < Tlen && keep(r);
+            const int64_t at = (int64_t)bh * Tlen + t0 + r;
+            const float den = on ? a.den[at] : 1.f;
+            if (a.d_ss) {  // dout_i + 2 d_ss_i o_i takes the place of dout_i
+                const float two = on ? 2.f * a.d_ss[at] : 0.f;
+                float dot = 0.f, oo = 0.f;
+#pragma unroll
+                for (int e = 0; e < IO::KP; ++e) {
+                    const float of = (float)ro.v[p][e], yf = (float)ry.v[p][e];
+                    dot += yf * of, oo += of * of;
+                    ry.v[p][e] = (T)((yf + two * of) / den);
+                }
+                inv[p] = seg_sum<IO::SEGS>(dot) + two * seg_sum<IO::SEGS>(oo);
+            } else {
+                float dot = 0.f;
+#pragma unroll
+                for (int e = 0; e < IO::KP; ++e) dot += (float)ry.v[p][e] * (float)ro.v[p][e];
+                inv[p] = seg_sum<IO::SEGS>(dot);
+            }
+            if (tid % IO::SEGS == 0 && (IO::FULL || r < C)) sDd[r] = on && den > a.eps ? -inv[p] / den : 0.f;
+            inv[p] = 1.f / den;
+        }
+        if (!a.d_ss) IO::scale_rows(ry, inv);
     }
     // rows past the end of the sequence: y is zero there, and phi(0) = 1 in x is finite
     IO::to_lds(rx, sX, LDD, tid);
     IO::to_lds(ry, sY, LDD, tid);
     sync_lds();
+    if (NORM) {  // column sums of the keys (of the queries, weighted by dden): the chunk's part of z (of its gradient)
+        constexpr int G = NTHR / HD;
+        const int col = tid % HD;
+        float part = 0.f;
+#pragma unroll
+        for (int i = 0; i < C / G; ++i) {
+            const int r = i * G + tid / HD;
+            part += (float)sX[r * LDD + col] * (BWD ? sDd[BWD ? r : 0] : 1.f);
+        }
+        sPart[tid] = part;
+        sync_lds();
+        if (tid < HD && tid < dkw) {
+            float z = 0.f;
+#pragma unroll
+            for (int i = 0; i < G; ++i) z += sPart[i * HD + tid];
+            a.z[((int64_t)bh * NC + c) * dkw + tid] = z;
+        }
+    }
     f32x4 acc[TMS::TPW];  // S^T: m = dk, n = dv
     zero_acc<TMS::TPW>(acc);
     gemm<T, HD, HD, C, KROW, KROW, NW>(acc, sX, LDD, sY, LDD, w, lane);
@@ -61,22 +139,27 @@ la_chunk_state_kernel(const T *__restrict__ x, const T *__restrict__ y, const vo
     }
 }
 
-// grid (B * H, d * d / 1024): each thread carries four of the d x d state elements through the chunks.  Only the
+// grid (B * H, d * d / 1024, plus one where z is scanned too): each thread carries four of the d x d state elements through the chunks.  Only the
 // additions are sequential: the slots (and the reset flags) of the next group of eight chunks are
 // requested before the current group is summed and written back, so that one trip to memory is exposed
 // per sequence, not one per group.
 // NARROW: narrow heads, the state's size is a run-time value.
-template <bool NARROW>
+// DECAY: the sum so far enters a chunk without resets times dec[chunk].  Z: the last block of the grid's second axis
+// carries the dk elements of z instead.
+template <bool NARROW, bool DECAY, bool Z>
 __global__ void __launch_bounds__(256)
 la_state_scan_kernel(float *__restrict__ slots, const float *__restrict__ init, float *__restrict__ fin,
-                     const void *__restrict__ done, int done_f32, int Tlen, int H, int NC, int C, int backward, int Qn)
+                     const void *__restrict__ done, int done_f32, int Tlen, int H, int NC, int C, int backward, int Qn,
+                     const float *__restrict__ dec, float *__restrict__ zslots, const float *__restrict__ zinit, float *__restrict__ zfin, int zq)
 {
-    const int Q = NARROW ? Qn : HD * HD / 4;  // f32x4 per state (d_v * d_k / 4)
+    const bool zpart = Z && blockIdx.y == gridDim.y - 1;
+    const int Q = zpart ? zq : NARROW ? Qn : HD * HD / 4;  // f32x4 per state (d_v * d_k / 4)
+    if (zpart) slots = zslots, init = zinit, fin = zfin;
     constexpr int G = 8;            // chunks per group
     const int tid = threadIdx.x, lane = tid & 63;
     const int bh = blockIdx.x, b = bh / H;
-    const int idx = blockIdx.y * 256 + tid;
-    const bool act = !NARROW || idx < Q;  // a narrow state has fewer elements than the workgroup has threads; the idle lanes
+    const int idx = (zpart ? 0 : blockIdx.y * 256) + tid;
+    const bool act = !(NARROW || Z) || idx < Q;  // a narrow state has fewer elements than the workgroup has threads; the idle lanes
                                        // still bring their reset flags to the ballots
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     f32x4 S = init && act ? reinterpret_cast<const f32x4 *>(init)[(int64_t)bh * Q + idx] : zero;
@@ -84,14 +167,17 @@ la_state_scan_kernel(float *__restrict__ slots, const float *__restrict__ init, 
     auto chunk_of = [&](int s) { return backward ? NC - 1 - s : s; };
     f32x4 nt[G];
     uint32_t nd[G];  // raw reset flag of chunk row `lane`
+    float ne[G];     // the chunk's decay
     auto fetch = [&](int s0) {
 #pragma unroll
         for (int u = 0; u < G; ++u) {
             const int s = s0 + u, c = chunk_of(s);
             nt[u] = zero;
             nd[u] = 0u;
+            ne[u] = 1.f;
             if (s < NC) {  // uniform over the workgroup
                 if (act) nt[u] = p[(int64_t)c * Q];
+                if (DECAY) ne[u] = dec[(int64_t)bh * NC + c];
                 const int tt = c * C + lane;
                 if (lane < C && tt < Tlen) nd[u] = done_raw(done, done_f32, (int64_t)b * Tlen + tt);
             }
@@ -101,9 +187,11 @@ la_state_scan_kernel(float *__restrict__ slots, const float *__restrict__ init, 
     for (int s0 = 0; s0 < NC; s0 += G) {
         f32x4 t[G];
         bool cut[G];
+        float e[G];
 #pragma unroll
         for (int u = 0; u < G; ++u) {
             t[u] = nt[u];
+            e[u] = ne[u];
             cut[u] = __ballot(done_test(nd[u], done_f32)) != 0ull;
         }
         if (s0 + G < NC) fetch(s0 + G);
@@ -112,7 +200,7 @@ la_state_scan_kernel(float *__restrict__ slots, const float *__restrict__ init, 
             const int s = s0 + u;
             if (s < NC) {
                 if (act) p[(int64_t)chunk_of(s) * Q] = S;
-                S = cut[u] ? t[u] : S + t[u];
+                S = cut[u] ? t[u] : DECAY ? e[u] * S + t[u] : S + t[u];
             }
         }
     }
@@ -121,45 +209,57 @@ la_state_scan_kernel(float *__restrict__ slots, const float *__restrict__ init, 
 
 template <typename T, int C>
 int launch_states(hipStream_t st, const void *x, const void *y, const void *done, int done_f32, float *slots, int64_t B,
-                  int64_t Tlen, int64_t H, bool fmap, bool backward, int64_t dk, int64_t dv)
+                  int64_t Tlen, int64_t H, bool fmap, bool backward, int64_t dk, int64_t dv, const LaStateArgs &a)
 {
     const int64_t NC = (Tlen + C - 1) / C;
     if (B * H > 0x7fffffffLL || NC > 65535) return MRX_ERR_INVALID_ARG;
-    const dim3 grid((unsigned)(B * H), (unsigned)NC), block(256);
-#define MRX_LAUNCH(FM, BW, RG)                                                                                         \
-    launch_kernel((la_chunk_state_kernel<T, C, FM, BW, RG>), grid, block, 0, st, (const T *)x, (const T *)y, done,       \
-                  done_f32, slots, (int)Tlen, (int)H, (int)NC, (int)dk, (int)dv)
-    if (dk != HD || dv != HD) {  // narrow heads
-        if (fmap) return backward ? MRX_LAUNCH(true, true, true) : MRX_LAUNCH(true, false, true);
-        return backward ? MRX_LAUNCH(false, true, true) : MRX_LAUNCH(false, false, true);
-    }
-    if (fmap) return backward ? MRX_LAUNCH(true, true, false) : MRX_LAUNCH(true, false, false);
-    return backward ? MRX_LAUNCH(false, true, false) : MRX_LAUNCH(false, false, false);
-#undef MRX_LAUNCH
+    auto go = [&](auto fm, auto bw, auto narrow, auto gated, auto norm) {
+        return launch_kernel(la_chunk_state_kernel<T, C, decltype(fm)::value, decltype(bw)::value, decltype(narrow)::value,
+                                                   decltype(gated)::value, decltype(norm)::value>,
+                             dim3((unsigned)(B * H), (unsigned)NC), dim3(256), 0, st, (const T *)x, (const T *)y, done, done_f32, slots,
+                             (int)Tlen, (int)H, (int)NC, (int)dk, (int)dv, a);
+    };
+    using Y = std::true_type;
+    using N = std::false_type;
+    auto variant = [&](auto fm, auto bw, auto narrow) {
+        if (a.glog) return go(fm, bw, narrow, Y{}, N{});
+        if (a.z) return go(fm, bw, narrow, N{}, Y{});
+        return go(fm, bw, narrow, N{}, N{});
+    };
+    auto sized = [&](auto fm, auto bw) { return dk != HD || dv != HD ? variant(fm, bw, Y{}) : variant(fm, bw, N{}); };
+    if (fmap) return backward ? sized(Y{}, Y{}) : sized(Y{}, N{});
+    return backward ? sized(N{}, Y{}) : sized(N{}, N{});
 }
 
 }  // namespace
 
 int launch_la_chunk_states(hipStream_t st, const void *x, const void *y, const void *done, int done_f32, float *slots,
-                           int64_t B, int64_t Tlen, int64_t H, int dtype, bool fmap, bool backward, int64_t dk, int64_t dv)
+                           int64_t B, int64_t Tlen, int64_t H, int dtype, bool fmap, bool backward, int64_t dk, int64_t dv,
+                           const LaStateArgs &a)
 {
     if (dtype == MRX_BF16)
-        return launch_states<__bf16, LA_BF16_CHUNK>(st, x, y, done, done_f32, slots, B, Tlen, H, fmap, backward, dk, dv);
-    return launch_states<float, 32>(st, x, y, done, done_f32, slots, B, Tlen, H, fmap, backward, dk, dv);
+        return launch_states<__bf16, LA_BF16_CHUNK>(st, x, y, done, done_f32, slots, B, Tlen, H, fmap, backward, dk, dv, a);
+    return launch_states<float, 32>(st, x, y, done, done_f32, slots, B, Tlen, H, fmap, backward, dk, dv, a);
 }
 
 int launch_la_state_scan(hipStream_t st, float *slots, const float *init, float *fin, const void *done, int done_f32,
-                         int64_t B, int64_t Tlen, int64_t H, int C, bool backward, int64_t dk, int64_t dv)
+                         int64_t B, int64_t Tlen, int64_t H, int C, bool backward, int64_t dk, int64_t dv, const LaStateArgs &a)
 {
     const int64_t NC = (Tlen + C - 1) / C;
     if (B * H > 0x7fffffffLL) return MRX_ERR_INVALID_ARG;
     const int Q = (int)(dk * dv / 4);
-    const dim3 grid((unsigned)(B * H), (unsigned)((Q + 255) / 256));
-    if (dk != HD || dv != HD)
-        return launch_kernel(la_state_scan_kernel<true>, grid, dim3(256), 0, st, slots, init, fin, done, done_f32, (int)Tlen,
-                             (int)H, (int)NC, C, backward ? 1 : 0, Q);
-    return launch_kernel(la_state_scan_kernel<false>, grid, dim3(256), 0, st, slots, init, fin, done, done_f32, (int)Tlen,
-                         (int)H, (int)NC, C, backward ? 1 : 0, Q);
+    const dim3 grid((unsigned)(B * H), (unsigned)((Q + 255) / 256 + (a.z ? 1 : 0)));
+    auto go = [&](auto narrow, auto decay, auto z) {
+        return launch_kernel(la_state_scan_kernel<decltype(narrow)::value, decltype(decay)::value, decltype(z)::value>, grid, dim3(256), 0, st,
+                             slots, init, fin, done, done_f32, (int)Tlen, (int)H, (int)NC, C, backward ? 1 : 0, Q, (const float *)a.dec, a.z,
+                             a.z_init, a.z_fin, (int)(dk / 4));
+    };
+    auto variant = [&](auto narrow) {
+        if (a.dec) return go(narrow, std::true_type{}, std::false_type{});
+        if (a.z) return go(narrow, std::false_type{}, std::true_type{});
+        return go(narrow, std::false_type{}, std::false_type{});
+    };
+    return dk != HD || dv != HD ? variant(std::true_type{}) : variant(std::false_type{});
 }
 
 }  // namespace MRX_HD_NS
