@@ -443,13 +443,13 @@ AttnOut linear_attn_fwd(const Tensor &q, const Tensor &k, const Tensor &v, const
 }
 
 // Whether the gated or the normalised form cuts the work along time, a workgroup per chunk: the library's rule, and on heads of up to
-// 32 features more than twelve chunks.  The six launches of a forward and backward pair take the host 82 us, two take it 70; a
-// sequential pair's chain costs 12 us a chunk in bfloat16 (64 features), 7 us up to 32 features (bfloat16, 32 sequences: 8 chunks 100
-// -> 81 and 65 -> 83 us, 16 chunks 180 -> 81 and 112 -> 83 us, 32 chunks 334 -> 87 and 219 -> 82 us; float32 of 64 features, 128
-// sequences of 64 chunks 736 -> 505 us, 192 of 8 to 64 chunks level).
+// 32 features ten chunks or more.  Six launches instead of two for a forward and backward pair cost the host 12 us (82 and 70 us
+// from a slow host, 44 and 35 from a fast one); a sequential pair's chain costs 12 us a chunk in bfloat16 (64 features), 7 us up to 32
+// features (slow host, bfloat16, 32 sequences: 8 chunks 100 -> 81 and 65 -> 83 us, 16 chunks 180 -> 81 and 112 -> 83 us, 32 chunks
+// 334 -> 87 and 219 -> 82 us; float32 of 64 features, 128 sequences of 64 chunks 736 -> 505 us, 192 of 8 to 64 chunks level).
 bool chunk_parallel_pays(const Shape &s)
 {
-    return lib.mrx_linear_attn_chunk_parallel_pays(s.B, s.T, s.H, code(s.dt)) != 0 && (std::max(s.dk, s.dv) > 32 || s.chunks() > 12);
+    return lib.mrx_linear_attn_chunk_parallel_pays(s.B, s.T, s.H, code(s.dt)) != 0 && (std::max(s.dk, s.dv) > 32 || s.chunks() >= 10);
 }
 
 struct AttnGrads {
