@@ -385,6 +385,9 @@ int mrx_silu_gate_fwd(void *stream, const void *h, const void *g, void *y, int64
 int mrx_silu_gate_bwd(void *stream, const void *h, const void *g, const void *dy, void *dh, void *dg,
                       int64_t n, int dtype);
 
+/* The residual sum around a block (residual.py:23-26) of a float32 stream and a bfloat16 branch: y_i = x_i + branch_i, float32. */
+int mrx_residual_add(void *stream, const float *x, const void *branch, float *y, int64_t n);
+
 /* ---- Mamba and mLSTM cells: the passes around their recurrence -----------------
  * The causal depthwise convolution over time with silu behind it (mamba.py:88-106, mlstm.py:110-125):
  *     s_t = bias + sum_j w_j x_{t-K+1+j} ,  y_t = silu(s_t)     (x = 0 before the call's first step; resets do not cut it)

@@ -73,6 +73,7 @@ SIGNATURES = {
     "mrx_mlstm_gates_bwd": (_I, [_P] * 12 + [_L] * 3 + [_I, ctypes.c_float]),
     "mrx_layer_norm_fwd": (_I, [_P] * 5 + [_L] * 2 + [_I, _I, ctypes.c_float]),
     "mrx_layer_norm_bwd": (_I, [_P] * 9 + [_L] * 2 + [_I, _I, ctypes.c_float]),
+    "mrx_residual_add": (_I, [_P] * 4 + [_L]),
     "mrx_silu_gate_fwd": (_I, [_P] * 4 + [_L, _I]),
     "mrx_silu_gate_bwd": (_I, [_P] * 6 + [_L, _I]),
     "mrx_causal_conv_silu_fwd": (_I, [_P, _P, _L, _P, _P, _P] + [_L] * 4),

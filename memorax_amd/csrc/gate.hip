@@ -89,6 +89,28 @@ __global__ void __launch_bounds__(GT_THREADS) silu_gate_bwd_kernel(const T *__re
     }
 }
 
+// The residual sum of a float32 stream and a bfloat16 branch.  The array library's sum of two types gives a workgroup 16384
+// elements, so a rollout of a few hundred thousand is a few dozen workgroups of strided loads; here eight elements make a thread
+// (690 k elements 100 -> 6.4 us, 8.7 M 104 -> 27 us, 34 M 86 -> 84 us, with other traffic between the launches).
+__global__ void __launch_bounds__(GT_THREADS) residual_add_kernel(const float *__restrict__ x, const __bf16 *__restrict__ b,
+                                                                  float *__restrict__ y, int64_t n)
+{
+    const int64_t stride = (int64_t)gridDim.x * GT_THREADS * 8;
+    for (int64_t i = ((int64_t)blockIdx.x * GT_THREADS + threadIdx.x) * 8; i < n; i += stride) {
+        if (i + 8 <= n) {
+            const Pack<float> lo = *reinterpret_cast<const Pack<float> *>(x + i), hi = *reinterpret_cast<const Pack<float> *>(x + i + 4);
+            const Pack<__bf16> bv = *reinterpret_cast<const Pack<__bf16> *>(b + i);
+            Pack<float> a, c;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a.v[e] = lo.v[e] + (float)bv.v[e], c.v[e] = hi.v[e] + (float)bv.v[4 + e];
+            *reinterpret_cast<Pack<float> *>(y + i) = a;
+            *reinterpret_cast<Pack<float> *>(y + i + 4) = c;
+        } else {
+            for (int64_t j = i; j < n; ++j) y[j] = x[j] + (float)b[j];
+        }
+    }
+}
+
 unsigned gate_grid(int64_t n, int per_thread)
 {
     const int64_t wgs = (n + (int64_t)GT_THREADS * per_thread - 1) / ((int64_t)GT_THREADS * per_thread);
@@ -136,4 +158,14 @@ extern "C" int mrx_silu_gate_bwd(void *stream, const void *h, const void *g, con
     return launch_kernel(silu_gate_bwd_kernel<__bf16>, dim3(gate_grid(n, 8)), dim3(GT_THREADS), 0, s, static_cast<const __bf16 *>(h),
                          static_cast<const __bf16 *>(g), static_cast<const __bf16 *>(dy), static_cast<__bf16 *>(dh),
                          static_cast<__bf16 *>(dg), n);
+}
+
+extern "C" int mrx_residual_add(void *stream, const float *x, const void *branch, float *y, int64_t n)
+{
+    using namespace mrx;
+    int rc;
+    if (!gate_args_ok({x, branch, y}, n, MRX_BF16, &rc)) return rc;
+    if (const int st = prepare_device(); st != MRX_OK) return st;
+    return launch_kernel(residual_add_kernel, dim3(gate_grid(n, 8)), dim3(GT_THREADS), 0, static_cast<hipStream_t>(stream), x,
+                         static_cast<const __bf16 *>(branch), y, n);
 }

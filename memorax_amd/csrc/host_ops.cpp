@@ -18,6 +18,7 @@
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/generated/Functions.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/utils/pybind.h>
 
@@ -41,7 +42,7 @@ using torch::autograd::variable_list;
     X(mrx_status_string) X(mrx_chunk_size) X(mrx_delta_chunk_size) X(mrx_scan_workspace) X(mrx_linear_scan_fwd_segmented) X(mrx_linear_scan_bwd_segmented)     \
     X(mrx_linear_scan_last) X(mrx_mingru_scan_fwd_segmented) X(mrx_mingru_scan_bwd_segmented) X(mrx_mlstm_gates_fwd)                     \
     X(mrx_mlstm_gates_bwd) X(mrx_rms_norm_fwd) X(mrx_rms_norm_bwd) X(mrx_layer_norm_fwd) X(mrx_layer_norm_bwd)       \
-    X(mrx_silu_gate_fwd) X(mrx_silu_gate_bwd) X(mrx_linear_attn_fwd) X(mrx_linear_attn_bwd)                          \
+    X(mrx_silu_gate_fwd) X(mrx_silu_gate_bwd) X(mrx_residual_add) X(mrx_linear_attn_fwd) X(mrx_linear_attn_bwd)                          \
     X(mrx_linear_attn_fwd_chunk_parallel) X(mrx_linear_attn_bwd_chunk_parallel)                                      \
     X(mrx_linear_attn_chunk_parallel_pays) X(mrx_linear_attn_norm_fwd) X(mrx_linear_attn_norm_bwd)                   \
     X(mrx_gated_linear_attn_fwd) X(mrx_gated_linear_attn_bwd) X(mrx_delta_rule_fwd) X(mrx_delta_rule_bwd)            \
@@ -1310,6 +1311,32 @@ Tensor silu_gate(const Tensor &h, const Tensor &g)
     return y;
 }
 
+// x + branch for a float32 stream and a bfloat16 branch; the node is the array library's own, so derivatives of any order are what
+// its sum's are, and so is everything the kernel does not take.
+Tensor residual_add(const Tensor &x, const Tensor &branch)
+{
+    auto plain = [](const Tensor &t) {
+        return t.is_cuda() && t.is_contiguous() && t.has_storage() && !t.is_neg() && !t._fw_grad(0).defined() &&
+               !t.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::FuncTorchBatched})) &&
+               reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+    };
+    if (x.scalar_type() != at::kFloat || branch.scalar_type() != at::kBFloat16 || x.sizes() != branch.sizes() || x.numel() == 0 ||
+        x.device() != branch.device() || !plain(x) || !plain(branch))
+        return at::add(x, branch);
+    const Tensor y = fresh_like(x);
+    check(lib.mrx_residual_add(stream(), fptr(x), ptr(branch), fptr(y), x.numel()), "mrx_residual_add");
+    if (at::GradMode::is_enabled() && (differentiable(x) || differentiable(branch))) {
+        auto node = std::shared_ptr<torch::autograd::generated::AddBackward0>(new torch::autograd::generated::AddBackward0(),
+                                                                              torch::autograd::deleteNode);
+        node->set_next_edges(torch::autograd::collect_next_edges(x, branch));
+        node->alpha = 1;
+        node->self_scalar_type = at::kFloat;
+        node->other_scalar_type = at::kBFloat16;
+        torch::autograd::set_history(y, node);
+    }
+    return y;
+}
+
 // RMS norm (center false) or layer norm; fork: the input is handed on beside its norm -- (x, norm(x)) -- so that the
 // gradients of both meet in the norm's backward kernel instead of in a pass of their own.
 struct NormOp {
@@ -1849,6 +1876,7 @@ PYBIND11_MODULE(_native, m)
     def("delta_rule", &delta_rule);
     def("mlstm_gates", &mlstm_gates);
     def("silu_gate", &silu_gate);
+    def("residual_add", &residual_add);
     def("norm", &norm);
     def("dense_group", &dense_group);
     def("dense_grads", &dense_grads);

@@ -1048,6 +1048,8 @@ class Residual(nn.Module):
             carry, y = inner.module(normed, done, initial_carry, **kwargs)
         else:
             carry, y = inner(inputs, done, initial_carry, **kwargs)
+        if inputs.is_cuda and inputs.dtype is torch.float32 and y.dtype is torch.bfloat16:   # a mixed-precision block on a float32 stream
+            return carry, native().residual_add(inputs, y)
         return carry, inputs + y
 
     def initialize_carry(self, key, input_shape):
