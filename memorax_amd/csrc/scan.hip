@@ -1100,8 +1100,9 @@ ScanPlan plan_scan(int64_t B, int64_t T, int64_t D, size_t esize, bool bwd, bool
         int nw8 = 1;  // waves along time: up to eight, each with a whole group of steps to itself
         while (nw8 < 8 && (int64_t)2 * nw8 * TS_MIN <= T) nw8 <<= 1;
         // (*) bfloat16 backward: single elements are 2-byte loads, three or four arrays of them; two per lane and 16 steps
-        // per wave make up for half the waves (8 x 1000 x 64 66 -> 54, 57 x 2908 x 120 217 -> 166)
-        if (half_storage && bwd && !mg && D >= 2 && T >= 8 * TS_MIN && waves2 < 600) return split(2, 8, T >= 16 * TS_MIN ? 16 : 8);
+        // per wave make up for half the waves (8 x 1000 x 64 66 -> 54, 57 x 2908 x 120 217 -> 166), while a workgroup per compute
+        // unit is all there is
+        if (half_storage && bwd && !mg && D >= 2 && T >= 8 * TS_MIN && waves2 < 600 && (cols(2) <= 256 || D <= 64)) return split(2, 8, T >= 16 * TS_MIN ? 16 : 8);
         // so few columns that eight waves along time leave most of the device idle: sixteen of one lane each; (*) forward with
         // 16 steps each, half as many trips to memory (4 x 3000 x 512 101 -> 77, 75 x 679 x 64 29 -> 22)
         if (T >= 16 * TS_MIN && cols(1) <= 256) return split(1, 16, !bwd && esize == 4 && T > 16 * TS_MIN ? 16 : 8);
@@ -1113,9 +1114,16 @@ ScanPlan plan_scan(int64_t B, int64_t T, int64_t D, size_t esize, bool bwd, bool
             // the streaming kernels lay their threads flat over (row, column): a row need not fill whole waves.
             // (*) They lead as soon as they have 600 waves backward, and on ragged rows with a thousand (MinGRU 1800) forward
             // (1500 x 300 x 165 240 -> 137 and 439 -> 231; 128 x 512 x 1000 122 -> 111 and 222 -> 169)
+            // (**) A last sweep, twenty shapes of 256 to 800 workgroups: eight waves of 16 steps fill a compute unit's registers, of 8
+            // steps half of them, four waves a third, so beyond 256 workgroups of the first or 512 of the second a few left over
+            // cost a whole round.  Forward 256 to 512 workgroups 8 steps, above four waves (79 x 808 x 391 117 -> 89 with the MinGRU
+            // map and 94 -> 74 without, 85 x 1500 x 391 203 -> 156, 150 x 600 x 512 117 -> 92); backward four waves above 256
+            // (205 -> 173 and 138 -> 118, 373 -> 314), also where whole rows would stream with up to 768 (221 -> 205 and 146 -> 112,
+            // 200 x 1200 x 384 495 -> 391; ragged ones not: 200 x 400 x 391 122 -> 147)
+            if (v == 2 && bwd && nw8 > 4 && cols(2) > 256 && (waves2 < 600 || (!ragged && waves2 < 768))) return split(2, 4);
             if (v == 2 && (bwd ? waves2 >= 600 : ragged && waves2 >= (mg ? 1800 : 1000))) return flow(2);
-            if (cols(v) >= (bwd ? 512 : 1024) && nw8 > 4) return split(v, 4);
-            return split(v, nw8, !bwd && T >= 64 * TS_MIN && nw8 == 8 ? 16 : 8);   // (*) 256 x 1024 x 96 63 -> 50
+            if ((bwd ? cols(v) >= 512 : cols(v) >= (v == 2 ? 513 : 1024)) && nw8 > 4) return split(v, 4);
+            return split(v, nw8, !bwd && T >= 64 * TS_MIN && nw8 == 8 && (v == 1 || cols(v) <= 256) ? 16 : 8);   // (*) 256 x 1024 x 96 63 -> 50
         }
         if (esize == 8 && !mg) {
             // (*) ragged rows stream, and so do the backward that sums a broadcast decay's gradient (no da to write) and that of

@@ -12,6 +12,7 @@ SHAPES = [
     (2, 513, 65), (5, 272, 130),
     (300, 520, 70),                               # eight waves of 16 steps
     (1101, 33, 131), (601, 65, 257),              # streaming on ragged rows
+    (135, 515, 200), (300, 70, 256),              # bfloat16: more workgroups than one or two per compute unit
     (1, 385, 2), (1, 513, 65), (12, 450, 130), (1, 1200, 512),   # time in segments, the last one partly filled
     (1, 4096, 70),                                # as many segments as there can be
 ]
