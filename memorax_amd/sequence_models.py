@@ -467,12 +467,7 @@ def _row_layers(x, layers):
 
 def _hooked(module):
     """Whether a hook waits in this module or below, or for every module: fused operations do not run the modules they stand for."""
-    return _any_global_hook() or _any_hook(module)
-
-
-def _any_hook(m):
-    return bool(m._forward_pre_hooks or m._forward_hooks or m._backward_hooks or m._backward_pre_hooks
-                or any(c is not None and _any_hook(c) for c in m._modules.values()))
+    return _any_global_hook() or native().any_hook(module)
 
 
 def _plain(layer):
