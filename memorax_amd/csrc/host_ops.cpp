@@ -1464,7 +1464,16 @@ std::optional<ScalarType> autocast_dtype(const Tensor &x)
 // 3 x 256 26 / 225, 32768 x 1024 -> 1024 148 / 121; float32 131072 x 256 -> 256 188 / 181, 23100 x 64 -> 256 26 / 99, 131072 x 512 ->
 // 3 x 512 2080 / 1740).  The input: several layers at once, as narrow (68200 x 128 -> 3 x 64 + 2 25 / 69, 131072 x 256 -> 3 x 256 + 4
 // 118 / 150; float32 68 / 93, but 131072 x 256 -> 3 x 256 536 / 454), or few rows, where the host's calls are what it costs.
-bool params_suit(ScalarType dt, int64_t K, int64_t widest) { return K * widest <= (dt == at::kBFloat16 ? 512 * 512 : 256 * 256); }
+// In float32 the array library's slices also lead where they are whole and many and few layers have a bias, which it sums in a launch
+// of 50 us each (three layers without / with biases, here / there: 131072 x 256 -> 256 481 / 393 and 547 / 570, 32768 rows 145 / 129 and
+// 157 / 212; 131072 x 128 -> 256 252 / 221 and 285 / 391, 32768 rows 86 / 87 and 93 / 170; 131072 x 128 -> 128 143 / 147).
+bool params_suit(ScalarType dt, int64_t rows, int64_t K, int64_t widest, size_t layers, size_t biases)
+{
+    if (dt == at::kBFloat16) return K * widest <= 512 * 512;
+    if (K * widest > 256 * 256) return false;
+    const bool wide = K * widest == 256 * 256;
+    return 2 * biases >= layers || K * widest < 128 * 256 || weight_gradient_slices(rows, widest, K) < (wide ? 16 : 32);
+}
 bool input_suits(ScalarType dt, int64_t rows, int64_t K, int64_t widest, size_t layers)
 {
     const int64_t most = dt == at::kBFloat16 ? 256 : 128;
@@ -1504,7 +1513,7 @@ struct DenseOp {
         }
         if (used.empty()) return out;
         regular = regular && used.size() <= MRX_DENSE_LAYERS && x2.is_contiguous() && reinterpret_cast<uintptr_t>(x2.data_ptr()) % 16 == 0;
-        const bool own_params = want_params && regular && params_suit(dt, x2.size(1), widest),
+        const bool own_params = want_params && regular && params_suit(dt, x2.size(0), x2.size(1), widest, used.size(), std::count(bias.begin(), bias.end(), true)),
                    own_dx = node.wants(0) && regular && (x_dtype == at::kFloat || x_dtype == at::kBFloat16) &&
                             input_suits(dt, x2.size(0), x2.size(1), widest, used.size());
         if (own_params || own_dx) {

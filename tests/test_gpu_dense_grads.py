@@ -38,3 +38,22 @@ def test_dense_grads(rows, K, outs, dtype, dx_dtype):
             assert params[len(outs) + l] is None or not params[len(outs) + l].numel()
     only = _lib.native().dense_grads(x, dys, ws, bias, False, dx_dtype, True)
     assert all(torch.equal(a, b) for a, b in zip(only[1:], params) if b is not None)
+
+
+@pytest.mark.parametrize("rows,K,n,biases", [(32768, 256, 256, 0), (32768, 256, 256, 2), (16384, 256, 256, 0), (65536, 128, 256, 1), (65536, 128, 248, 0)])
+def test_float32_groups_on_either_side_of_the_rule(rows, K, n, biases):
+    """The library's kernels or the array library's slices: float32 sums over the rows, in error against float64 a random walk of
+    rounding errors (sqrt(rows) eps of the terms' root mean square), times eight for the longest walk among the elements."""
+    import torch
+    from memorax_amd.dense import Weights, dense_group
+    g = torch.Generator(device="cuda").manual_seed(rows + K + n + biases)
+    x = torch.randn(rows, K, device="cuda", generator=g)
+    ws = [torch.randn(n, K, device="cuda", generator=g).requires_grad_() for _ in range(3)]
+    bs = [torch.randn(n, device="cuda", generator=g).requires_grad_() if i < biases else None for i in range(3)]
+    dy = [torch.randn(rows, n, device="cuda", generator=g) for _ in range(3)]
+    torch.autograd.backward(dense_group(x, [Weights(w, b) for w, b in zip(ws, bs)]), dy)
+    for w, b, d in zip(ws, bs, dy):
+        tol = 8 * rows ** 0.5 * 2.0 ** -24 * rows ** 0.5
+        assert float((w.grad.double() - d.double().t() @ x.double()).abs().max()) <= tol
+        if b is not None:
+            assert float((b.grad.double() - d.double().sum(0)).abs().max()) <= tol
