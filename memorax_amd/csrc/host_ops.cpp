@@ -902,9 +902,24 @@ void refuse_tangent(const OptTensor &t)
 {
     if (t.has_value()) refuse_tangent(*t);
 }
+// Nor do they know functorch's transforms: a history set on the wrapper of a batched tensor is lost when vmap unwraps it.
+bool transformed(const Tensor &t)
+{
+    return t.defined() && t.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::FuncTorchBatched}));
+}
+bool transformed(const OptTensor &t) { return t.has_value() && transformed(*t); }
+void refuse(const Tensor &t)
+{
+    refuse_tangent(t);
+    TORCH_CHECK(!transformed(t), "memorax_amd operators do not run under functorch's transforms (vmap, grad, vjp, ...)");
+}
+void refuse(const OptTensor &t)
+{
+    if (t.has_value()) refuse(*t);
+}
 template <typename... Ts> bool need_grad(const Ts &...ts)
 {
-    (refuse_tangent(ts), ...);
+    (refuse(ts), ...);
     return at::GradMode::is_enabled() && (differentiable(ts) || ...);
 }
 
@@ -1294,6 +1309,7 @@ struct SiluGateOp {
 
 Tensor silu_gate(const Tensor &h, const Tensor &g)
 {
+    const bool need = need_grad(h, g);
     Tensor hc, gc, y;
     {
         at::AutoDispatchBelowADInplaceOrView below;
@@ -1302,7 +1318,7 @@ Tensor silu_gate(const Tensor &h, const Tensor &g)
         hc = as(h, dt), gc = as(g, dt);
         y = silu_gate_fwd(hc, gc);
     }
-    if (need_grad(h, g)) {
+    if (need) {
         auto node = record(SiluGateOp{}, h, g);
         torch::autograd::set_history(y, node);
         node->keep(0, hc);
@@ -1317,7 +1333,7 @@ Tensor residual_add(const Tensor &x, const Tensor &branch)
 {
     auto plain = [](const Tensor &t) {
         return t.is_cuda() && t.is_contiguous() && t.has_storage() && !t.is_neg() && !t._fw_grad(0).defined() &&
-               !t.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::FuncTorchBatched})) &&
+               !transformed(t) && !t.key_set().has(c10::DispatchKey::Python) &&
                reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
     };
     if (x.scalar_type() != at::kFloat || branch.scalar_type() != at::kBFloat16 || x.sizes() != branch.sizes() || x.numel() == 0 ||
@@ -1358,6 +1374,7 @@ struct NormOp {
 std::tuple<Tensor, Tensor> norm(const Tensor &x, const OptTensor &scale, const OptTensor &bias, double eps, std::optional<ScalarType> out_dtype,
                                 bool center, bool fork)
 {
+    const bool need = need_grad(x, scale, bias);
     Tensor xc, sc, y, res;
     {
         at::AutoDispatchBelowADInplaceOrView below;
@@ -1369,7 +1386,7 @@ std::tuple<Tensor, Tensor> norm(const Tensor &x, const OptTensor &scale, const O
                       ? xc.to(x.scalar_type())
                       : Tensor(xc.unsafeGetTensorImpl()->shallow_copy_and_detach(torch::autograd::impl::version_counter(xc), false));
     }
-    if (need_grad(x, scale, bias)) {
+    if (need) {
         auto node = record(NormOp{eps, center, fork}, x, unwrap(scale), unwrap(bias));
         if (fork) torch::autograd::set_history(res, node);
         torch::autograd::set_history(y, node);
@@ -1560,12 +1577,22 @@ bool rows_suit(const Tensor &x, const std::vector<Tensor> &weights, const std::v
 std::vector<Tensor> dense_group(const Tensor &x, const std::vector<Tensor> &weights, const std::vector<OptTensor> &biases)
 {
     TORCH_CHECK_VALUE(!weights.empty() && biases.size() == weights.size(), "dense_group takes one bias (or None) per weight");
+    std::vector<Tensor> out;
+    out.reserve(weights.size());
+    bool others = transformed(x);
+    for (size_t l = 0; l < weights.size(); ++l) others = others || transformed(weights[l]) || transformed(biases[l]);
+    if (others) {   // the array library's layers, which vmap and the functional gradients know
+        refuse_tangent(x);
+        for (size_t l = 0; l < weights.size(); ++l) {
+            refuse_tangent(weights[l]), refuse_tangent(biases[l]);
+            out.push_back(at::linear(x, weights[l], biases[l]));
+        }
+        return out;
+    }
     const auto cast = autocast_dtype(x);
     bool need = need_grad(x);
     for (size_t l = 0; l < weights.size(); ++l) need = need || need_grad(weights[l], biases[l]);
     c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
-    std::vector<Tensor> out;
-    out.reserve(weights.size());
     std::vector<Tensor> ws;
     Tensor xc;
     {
@@ -1622,6 +1649,7 @@ Tensor causal_conv_silu(const Tensor &x_, const Tensor &weight_, const Tensor &b
     TORCH_CHECK_VALUE(x_.dim() == 3 && weight_.dim() == 3 && x_.is_cuda() && x_.scalar_type() == at::kFloat,
                       "causal_conv_silu takes (B,T,C) float32 arrays on the GPU");
     const int64_t B = x_.size(0), T = x_.size(1), C = x_.size(2), K = weight_.size(2);
+    const bool need = need_grad(x_, weight_, bias_);
     Tensor x, y, weight, bias;
     {
         at::AutoDispatchBelowADInplaceOrView below;
@@ -1633,7 +1661,7 @@ Tensor causal_conv_silu(const Tensor &x_, const Tensor &weight_, const Tensor &b
         y = fresh({B, T, C}, at::kFloat, x);
         check(lib.mrx_causal_conv_silu_fwd(stream(), fptr(x), x.stride(1), fptr(weight), fptr(bias), fptr(y), B, T, C, K), "mrx_causal_conv_silu_fwd");
     }
-    if (need_grad(x_, weight_, bias_)) {
+    if (need) {
         auto node = record(ConvSiluOp{}, x_, weight_, bias_);
         torch::autograd::set_history(y, node);
         node->keep(0, x);

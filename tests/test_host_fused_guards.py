@@ -1,10 +1,12 @@
-"""What the fused host paths must not pass by: hooks and replaced parts of a module, second derivatives, forward mode."""
+"""What the fused host paths must not pass by: hooks and replaced parts of a module, second derivatives, forward mode, functorch."""
 import pytest
 import torch
 import torch.nn as nn
 
+from memorax_amd import functional as Fn
 from memorax_amd import sequence_models as sm
-from memorax_amd.dense import Dense, dense
+from memorax_amd._lib import native
+from memorax_amd.dense import Dense, dense, dense_group
 
 
 def test_gradients_refuse_a_second_derivative():
@@ -48,3 +50,48 @@ def test_a_replaced_part_is_no_row_layer():
     assert cell._parts_as_written()
     cell.up_projection = Dense(8, 64)
     assert not cell._parts_as_written()
+
+
+@pytest.mark.parametrize("bias", [False, True])
+def test_a_mapped_dense_layer_keeps_its_gradients(bias):
+    """As torch.nn.functional.linear: the mapped input, the parameters closed over, and a second path through them."""
+    lin, x = nn.Linear(8, 3, bias=bias).double(), torch.randn(5, 4, 8, dtype=torch.float64, requires_grad=True)
+    params = [x, *lin.parameters()]
+
+    def loss(layer):
+        return (torch.vmap(layer)(x) ** 2).sum() + (lin.weight ** 3).sum()
+
+    got = torch.autograd.grad(loss(lambda t: dense(t, lin.weight, lin.bias)), params)
+    grouped = torch.autograd.grad(loss(lambda t: dense_group(t, [lin, lin])[1]), params)
+    for g, h, want in zip(got, grouped, torch.autograd.grad(loss(lin), params)):
+        torch.testing.assert_close(g, want, rtol=1e-12, atol=1e-12)
+        torch.testing.assert_close(h, want, rtol=1e-12, atol=1e-12)
+    f = lambda layer: torch.func.grad(lambda w: layer(x.detach()[0], w).pow(2).sum())(lin.weight.detach())  # noqa: E731
+    torch.testing.assert_close(f(dense), f(nn.functional.linear), rtol=1e-12, atol=1e-12)
+
+
+def _operators():
+    """Every operator that records a node, of one tensor that all its floating arguments are made of."""
+    done, s = torch.zeros(2, 3), torch.ones(4)
+    heads = lambda t: t.view(2, 3, 1, 4)  # noqa: E731
+    return {
+        "linear_scan": lambda t: Fn.linear_scan(t, t, done),
+        "mingru_scan": lambda t: Fn.mingru_scan(t, t, done),
+        "linear_attention": lambda t: native().linear_attention(heads(t), heads(t), heads(t), done, None, 0, False),
+        "normalised": lambda t: native().normalised_linear_attention(heads(t), heads(t), heads(t), done, None, None, 0, 1e-6, False, False),
+        "gated": lambda t: native().gated_linear_attention(heads(t), heads(t), heads(t), t[..., :1], done, None, 0, False),
+        "delta_rule": lambda t: native().delta_rule(heads(t), heads(t), heads(t), t[..., :1], done, None, False, 0, False),
+        "mlstm_gates": lambda t: Fn.mlstm_gates(t, t, done),
+        "rms_norm": lambda t: Fn.rms_norm(t, s),
+        "layer_norm": lambda t: Fn.layer_norm_fork(t, s, s)[1],
+        "silu_gate": lambda t: Fn.silu_gate(t, t),
+        "mamba_mix": lambda t: native().mamba_mix(t, t, t, t[..., :1], torch.ones(10, 1, 4), torch.ones(10), s[:1], s[:1], s[:1], s[:2], done,
+                                                  torch.zeros(2, 1, 2, 4), torch.ones(2, 1), 1e-6, False),
+    }
+
+
+@pytest.mark.parametrize("name", sorted(_operators()))
+def test_functorch_is_refused_by_name(name):
+    f = _operators()[name]
+    with pytest.raises(RuntimeError, match="functorch"):
+        torch.vmap(f)(torch.randn(5, 2, 3, 4))
