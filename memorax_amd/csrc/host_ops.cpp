@@ -763,6 +763,44 @@ StepOut delta_rule_step(const Tensor &q, const Tensor &k, const Tensor &v, const
 // ---- acting: dense layers on few rows, the MinGRU cell's step
 Tensor norm_param(const OptTensor &t) { return t.has_value() ? dense16(t->to(at::kFloat)) : Tensor(); }
 
+// The operators know no forward mode: an input with a tangent is refused, as an autograd function without a jvp refuses it (also where
+// gradients are switched off: no_grad leaves tangents on).
+void refuse_tangent(const Tensor &t)
+{
+    TORCH_CHECK_NOT_IMPLEMENTED(!t.defined() || !t._fw_grad(0).defined(), "memorax_amd operators have no forward-mode derivative");
+}
+void refuse_tangent(const OptTensor &t)
+{
+    if (t.has_value()) refuse_tangent(*t);
+}
+// Nor do they know functorch's transforms: a history set on the wrapper of a batched tensor is lost when vmap unwraps it.
+bool transformed(const Tensor &t)
+{
+    return t.defined() && t.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::FuncTorchBatched}));
+}
+bool transformed(const OptTensor &t) { return t.has_value() && transformed(*t); }
+void refuse(const Tensor &t)
+{
+    refuse_tangent(t);
+    TORCH_CHECK(!transformed(t), "memorax_amd operators do not run under functorch's transforms (vmap, grad, vjp, ...)");
+}
+void refuse(const OptTensor &t)
+{
+    if (t.has_value()) refuse(*t);
+}
+void refuse(const std::vector<Tensor> &ts)
+{
+    for (const Tensor &t : ts) refuse(t);
+}
+void refuse(const std::vector<OptTensor> &ts)
+{
+    for (const OptTensor &t : ts) refuse(t);
+}
+template <typename... Ts> void refuse(const Ts &...ts) requires(sizeof...(Ts) > 1)
+{
+    (refuse(ts), ...);
+}
+
 // norm: 0 none, 1 RMS, 2 layer norm.  The results keep x's leading axes; residual (float32, x's leading axes): added to the one
 // layer's result.
 std::vector<Tensor> row_dense(const Tensor &x_, int norm, const OptTensor &scale_, const OptTensor &nbias_, double eps, bool round_norm,
@@ -770,6 +808,7 @@ std::vector<Tensor> row_dense(const Tensor &x_, int norm, const OptTensor &scale
                               const OptTensor &residual_, const OptTensor &weight2_ = std::nullopt, const OptTensor &skip_ = std::nullopt,
                               Tensor *skip_out = nullptr)
 {
+    refuse(x_, scale_, nbias_, weights, biases, residual_, weight2_, skip_);
     const Tensor x = dense16(x_), scale = norm_param(scale_), nbias = norm_param(nbias_), weight2 = dense16(weight2_), skip = dense16(skip_),
                  residual = residual_.has_value() ? residual_->contiguous() : Tensor();
     for (Tensor &w : weights) w = dense16(w);
@@ -819,6 +858,7 @@ std::tuple<Tensor, Tensor, Tensor> lru_act(const Tensor &x, int norm, const OptT
                                            std::vector<Tensor> params, const Tensor &done_, const Tensor &h_, const Tensor &P_)
 {
     TORCH_CHECK_VALUE(x.dim() == 3 && x.size(1) == 1 && params.size() == 8, "lru_act takes one time step");
+    refuse(x, scale, nbias, params, done_, h_, P_);
     const int64_t B = x.size(0), N = params[0].size(0);
     for (Tensor &t : params) t = dense16(t);
     for (int i = 0; i < 3; ++i) chk(params[i], "parameter", at::kFloat, {N});
@@ -842,6 +882,7 @@ std::vector<Tensor> mlstm_act(const Tensor &x, int norm, const OptTensor &scale,
                               const Tensor &done_, const std::vector<Tensor> &carry, double g_floor)
 {
     TORCH_CHECK_VALUE(x.dim() == 3 && x.size(1) == 1 && p.size() == 13 && carry.size() == 4, "mlstm_act takes one time step");
+    refuse(x, scale, nbias, p, done_, carry);
     const int64_t B = x.size(0), H = p[3].size(0), D = p[3].size(1), W = H * D, K = p[1].size(2);
     for (Tensor &t : p) t = dense16(t);
     chk(p[1], "conv weight", at::kFloat, {W, 1, K});
@@ -873,6 +914,7 @@ std::tuple<Tensor, Tensor, Tensor> mingru_step(const Tensor &z, const Tensor &x,
                                                const Tensor &log_state, const Tensor &log_decay, bool in_place)
 {
     TORCH_CHECK_VALUE(z.dim() == 3 && z.size(1) == 1, "mingru_step takes one time step");
+    refuse(z, x, gate, done_, log_state, log_decay);
     const int64_t B = z.size(0), D = z.size(2);
     const auto dt = z.scalar_type();
     chk_scan_dtype(dt, false, "mingru_step");
@@ -893,30 +935,6 @@ std::tuple<Tensor, Tensor, Tensor> mingru_step(const Tensor &z, const Tensor &x,
 bool differentiable(const Tensor &t) { return t.defined() && t.requires_grad(); }
 bool differentiable(const OptTensor &t) { return t.has_value() && differentiable(*t); }
 
-// The nodes know no forward mode: an input with a tangent is refused, as an autograd function without a jvp refuses it.
-void refuse_tangent(const Tensor &t)
-{
-    TORCH_CHECK_NOT_IMPLEMENTED(!t.defined() || !t._fw_grad(0).defined(), "memorax_amd operators have no forward-mode derivative");
-}
-void refuse_tangent(const OptTensor &t)
-{
-    if (t.has_value()) refuse_tangent(*t);
-}
-// Nor do they know functorch's transforms: a history set on the wrapper of a batched tensor is lost when vmap unwraps it.
-bool transformed(const Tensor &t)
-{
-    return t.defined() && t.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::FuncTorchBatched}));
-}
-bool transformed(const OptTensor &t) { return t.has_value() && transformed(*t); }
-void refuse(const Tensor &t)
-{
-    refuse_tangent(t);
-    TORCH_CHECK(!transformed(t), "memorax_amd operators do not run under functorch's transforms (vmap, grad, vjp, ...)");
-}
-void refuse(const OptTensor &t)
-{
-    if (t.has_value()) refuse(*t);
-}
 template <typename... Ts> bool need_grad(const Ts &...ts)
 {
     (refuse(ts), ...);
@@ -1012,6 +1030,7 @@ struct LinearScanOp {
 
 std::tuple<Tensor, Tensor, Tensor> linear_scan(const Tensor &a, const Tensor &b, const Tensor &done, const OptTensor &h0, const OptTensor &P0)
 {
+    refuse(done, P0);
     const bool need = need_grad(a, b, h0);
     Tensor a_, h0_;
     ScanOut r;
@@ -1048,6 +1067,7 @@ struct MinGruOp {
 
 std::tuple<Tensor, Tensor, Tensor> mingru_scan(const Tensor &z, const Tensor &x, const Tensor &done, const OptTensor &h0, const OptTensor &P0)
 {
+    refuse(done, P0);
     const bool need = need_grad(z, x, h0);
     Tensor z_, x_, h0_;
     ScanOut r;
@@ -1089,6 +1109,7 @@ struct LinearAttentionOp {
 std::tuple<Tensor, Tensor> linear_attention(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &done, const OptTensor &S0, int fmap,
                                             bool in_place)
 {
+    refuse(done);
     const bool need = need_grad(q, k, v, S0);
     Tensor q_, k_, v_, S0_;
     AttnOut r;
@@ -1136,6 +1157,7 @@ std::tuple<Tensor, Tensor, Tensor, OptTensor> normalised_linear_attention(const 
                                                                           const OptTensor &S0, const OptTensor &z0, int fmap, double eps,
                                                                           bool want_ss, bool in_place)
 {
+    refuse(done);
     const bool need = need_grad(q, k, v, S0, z0);
     Tensor q_, k_, v_;
     NormAttnOut r;
@@ -1188,6 +1210,7 @@ struct GatedOp {
 std::tuple<Tensor, Tensor> gated_linear_attention(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &g, const Tensor &done,
                                                   const OptTensor &S0, int fmap, bool in_place)
 {
+    refuse(done);
     const bool need = need_grad(q, k, v, g, S0);
     Tensor q_, k_, v_, g_;
     AttnOut r;
@@ -1233,6 +1256,7 @@ struct DeltaOp {
 std::tuple<Tensor, Tensor> delta_rule(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &beta, const Tensor &done,
                                       const OptTensor &S0, bool prologue, int resets, bool in_place)
 {
+    refuse(done);
     const bool need = need_grad(q, k, v, beta, S0);
     Tensor q_, k_, v_, b_;
     DeltaOut r;
@@ -1276,6 +1300,7 @@ struct MlstmGatesOp {
 
 std::tuple<Tensor, Tensor, Tensor> mlstm_gates(const Tensor &log_i, const Tensor &log_f, const Tensor &done, const OptTensor &m0, double g_floor)
 {
+    refuse(done);
     const bool need = need_grad(log_i, log_f, m0);
     Tensor li, lf, m0_;
     std::array<Tensor, 3> r;
@@ -1591,7 +1616,7 @@ std::vector<Tensor> dense_group(const Tensor &x, const std::vector<Tensor> &weig
     }
     const auto cast = autocast_dtype(x);
     bool need = need_grad(x);
-    for (size_t l = 0; l < weights.size(); ++l) need = need || need_grad(weights[l], biases[l]);
+    for (size_t l = 0; l < weights.size(); ++l) need = need_grad(weights[l], biases[l]) || need;   // every one is looked at
     c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
     std::vector<Tensor> ws;
     Tensor xc;
@@ -1726,6 +1751,7 @@ std::tuple<Tensor, Tensor, Tensor> mamba_mix(const Tensor &up, const Tensor &b_i
     TORCH_CHECK_VALUE(up.dim() == 3 && S0.dim() == 4 && conv_w_.dim() == 3, "mamba_mix: up (B,T,2HP), S0 (B,H,P,N), conv_w (C,1,K)");
     MambaSizes n{up.size(0), up.size(1), S0.size(1), S0.size(2), S0.size(3), conv_w_.size(2), S0.size(1) * S0.size(2)};
     const int64_t C = n.W + 2 * n.H * n.N;
+    refuse(done_);
     const bool need = need_grad(up, b_in, c_in, dt_in, conv_w_, conv_b_, dt_bias_, A_log_, D_, scale_, S0, decay0);
     Tensor conv_w, conv_b, dt_bias, A_log, D, scale;
     {

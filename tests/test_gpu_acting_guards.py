@@ -48,3 +48,23 @@ def test_a_hook_runs(cell):
     with torch.no_grad():
         block(torch.randn(6, 1, 64, device="cuda"), torch.zeros(6, 1, dtype=torch.bool, device="cuda"))
     assert seen
+
+
+@pytest.mark.parametrize("dual", ["input", "parameter", "carry"])
+@pytest.mark.parametrize("cell", [*sorted(CELLS), "recurrence"])
+def test_an_acting_block_refuses_tangents(cell, dual):
+    block = _block(cell) if cell in CELLS else sm.Residual(sm.PreNorm(sm.GatedLinearRecurrence(64), 64)).cuda()
+    x, done = torch.randn(6, 1, 64, device="cuda"), torch.zeros(6, 1, dtype=torch.bool, device="cuda")
+    carry = block.initialize_carry(None, (6, 64))
+    make = lambda t: torch.autograd.forward_ad.make_dual(t, torch.ones_like(t))  # noqa: E731
+    with torch.no_grad(), torch.autograd.forward_ad.dual_level():
+        params = {}
+        if dual == "input":
+            x = make(x)
+        elif dual == "carry":
+            carry = (make(carry[0]), *carry[1:])
+        else:
+            name, p = next((n, p) for n, p in block.named_parameters() if p.dim() == 2)
+            params[name] = make(p.detach())
+        with pytest.raises(NotImplementedError, match="forward-mode"):
+            torch.func.functional_call(block, params, (x, done, carry))

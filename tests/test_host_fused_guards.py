@@ -23,6 +23,52 @@ def test_a_tangent_is_refused():
             dense(torch.autograd.forward_ad.make_dual(x, torch.ones_like(x)), w)
 
 
+@pytest.mark.parametrize("at", ["weight", "bias", "second weight"])
+def test_a_parameter_s_tangent_is_refused_beside_an_input_that_requires_gradients(at):
+    dual = lambda t: torch.autograd.forward_ad.make_dual(t, torch.ones_like(t))  # noqa: E731
+    x, w, v, b = torch.randn(4, 8, requires_grad=True), torch.randn(3, 8), torch.randn(3, 8), torch.randn(3)
+    with torch.autograd.forward_ad.dual_level():
+        w, v, b = dual(w) if at == "weight" else w, dual(v) if at == "second weight" else v, dual(b) if at == "bias" else b
+        with pytest.raises(NotImplementedError, match="forward-mode"):
+            native().dense_group(x, [w, v], [b, None])
+
+
+def _acting():
+    """The acting entries, with the argument that carries a tangent handed in (named as in the entry)."""
+    N, done, ones = 8, torch.zeros(4, 1), torch.ones
+    x, state = ones(4, 1, N), ones(4, 1, N, dtype=torch.complex64)
+    lru = [ones(N), ones(N), ones(N), ones(N, N), ones(N, N), ones(N, N), ones(N, N), ones(N)]
+    mlstm = [ones(2 * N, N), ones(N, 1, 4), ones(N), *[ones(2, 4, 4)] * 3, *[ones(2, 3 * N), ones(2)] * 2, ones(2, 4), ones(N), ones(N, N)]
+    carry = [ones(4, 1, 2, 4, 4), ones(4, 1, 2, 1, 1), ones(4, 1, 2, 4, 1), ones(4, 1, 2, 1, 1)]
+    put = lambda lst, i, t: [*lst[:i], t, *lst[i + 1:]]  # noqa: E731
+    return {
+        "row_dense x": (x, lambda t: native().row_dense(t, 0, None, None, 0.0, False, [ones(N, N)], [None], torch.float32, torch.float32, None)),
+        "row_dense scale": (ones(N), lambda t: native().row_dense(x, 1, t, None, 0.0, False, [ones(N, N)], [None], torch.float32, torch.float32, None)),
+        "row_dense weight": (ones(N, N), lambda t: native().row_dense(x, 0, None, None, 0.0, False, [ones(N, N), t], [None, None], torch.float32,
+                                                                      torch.float32, None)),
+        "row_dense bias": (ones(N), lambda t: native().row_dense(x, 0, None, None, 0.0, False, [ones(N, N)], [t], torch.float32, torch.float32, None)),
+        "row_dense residual": (x, lambda t: native().row_dense(x, 0, None, None, 0.0, False, [ones(N, N)], [None], torch.float32, torch.float32, t)),
+        "lru_act x": (x, lambda t: native().lru_act(t, 0, None, None, 0.0, lru, done, state, state)),
+        "lru_act parameter": (ones(N), lambda t: native().lru_act(x, 0, None, None, 0.0, put(lru, 1, t), done, state, state)),
+        "lru_act carry": (state, lambda t: native().lru_act(x, 0, None, None, 0.0, lru, done, state, t)),
+        "mlstm_act x": (x, lambda t: native().mlstm_act(t, 0, None, None, 0.0, mlstm, done, carry, -60.0)),
+        "mlstm_act parameter": (ones(2, 4, 4), lambda t: native().mlstm_act(x, 0, None, None, 0.0, put(mlstm, 4, t), done, carry, -60.0)),
+        "mlstm_act carry": (carry[2], lambda t: native().mlstm_act(x, 0, None, None, 0.0, mlstm, done, put(carry, 2, t), -60.0)),
+        "mingru_step z": (x, lambda t: native().mingru_step(t, x, None, done, x, x, False)),
+        "mingru_step gate": (x, lambda t: native().mingru_step(x, x, t, done, x, x, False)),
+        "mingru_step carry": (x, lambda t: native().mingru_step(x, x, None, done, x, t, False)),
+    }
+
+
+@pytest.mark.parametrize("name", sorted(_acting()))
+def test_acting_refuses_a_tangent(name):
+    """Switching gradients off leaves tangents on: the acting entries, which run without gradients, look for them."""
+    t, call = _acting()[name]
+    with torch.no_grad(), torch.autograd.forward_ad.dual_level():
+        with pytest.raises(NotImplementedError, match="forward-mode"):
+            call(torch.autograd.forward_ad.make_dual(t, torch.ones_like(t)))
+
+
 @pytest.mark.parametrize("kind", ["forward", "pre", "backward", "backward_pre"])
 def test_hooks_are_seen_at_any_depth(kind):
     block = sm.PreNorm(sm.Memoroid(sm.LRUCell(8, 8)), 8)
