@@ -1702,7 +1702,7 @@ struct MambaSizes {
 };
 
 struct MambaOp {
-    enum { UP, BIN, CIN, DTIN, CONVW, CONVB, DTB, ALOG, D_, SCALE, V, K_, Q, G, O, SCHK, SLAST, SAVED };
+    enum { UP, BIN, CIN, DTIN, CONVW, CONVB, DTB, ALOG, D_, SCALE, V, K_, Q, G, O, SCHK, DECAY0, SLAST, SAVED };
     static constexpr bool ONCE = true;
     static const char *name() { return "MemoraxMambaBackward"; }
     Tensor done;
@@ -1717,6 +1717,7 @@ struct MambaOp {
                                         fptr(d_o), fptr(d_up) + n.W, 2 * n.W, fptr(dscale), fptr(work), n.B * n.T, n.H, n.P, (float)eps),
               "mrx_mamba_readout_bwd");
         auto r = gated_linear_attn_bwd(s[Q], s[K_], s[V], s[G], done, s[SCHK], d_o, some(as(grads[1], at::kFloat)), 0, node.wants(10), s[SLAST], parallel);
+        const Tensor &decay0 = s[DECAY0];
         Tensor ddecay0;
         if (grads[2].defined()) {   // the decay leaf handed on: it depends on every g from the last reset on
             const Tensor behind = done.ne(0).to(at::kInt).flip(1).cumsum(1).flip(1);   // resets at or after each step
@@ -1737,7 +1738,6 @@ struct MambaOp {
         const Tensor dw = part(C * n.K).view({C, 1, n.K}), dcb = part(C), ddtb = part(n.H), dA = part(n.H), dD = part(n.W / 4).view({n.H, n.P / 4}).sum(1);
         return {d_up, db_in, dc_in, ddt, dw, dcb, ddtb, dA, dD, dscale, r.dS0, ddecay0};
     }
-    Tensor decay0;
     bool parallel;
 };
 
@@ -1798,11 +1798,11 @@ std::tuple<Tensor, Tensor, Tensor> mamba_mix(const Tensor &up, const Tensor &b_i
         check(lib.mrx_decay_last(stream(), fptr(g), done.p(), fptr(decay0_), fptr(decay_last), n.B, n.T, n.H, done.dtype), "mrx_decay_last");
     }
     if (need) {
-        auto node = record(MambaOp{done_, n, eps, decay0_, parallel}, up, b_in, c_in, dt_in, conv_w_, conv_b_, dt_bias_, A_log_, D_, scale_, S0, decay0);
+        auto node = record(MambaOp{done_, n, eps, parallel}, up, b_in, c_in, dt_in, conv_w_, conv_b_, dt_bias_, A_log_, D_, scale_, S0, decay0);
         torch::autograd::set_history(y, node);
         torch::autograd::set_history(S_last, node);
         torch::autograd::set_history(decay_last, node);
-        const Tensor *kept[] = {&up, &b_in, &c_in, &dt_in, &conv_w, &conv_b, &dt_bias, &A_log, &D, &scale, &v, &k, &q, &g, &o, &S_chk};
+        const Tensor *kept[] = {&up, &b_in, &c_in, &dt_in, &conv_w, &conv_b, &dt_bias, &A_log, &D, &scale, &v, &k, &q, &g, &o, &S_chk, &decay0_};
         for (int i = 0; i < MambaOp::SLAST; ++i) node->keep(i, *kept[i]);
         node->keep(MambaOp::SLAST, S_last, true);
     }

@@ -66,3 +66,16 @@ def test_mamba_cell_acting_equals_its_composition():
             assert relerr(y, _np(cell.read(h, x))) <= 1e-4
             for a, b in zip(carry, ref):
                 assert a.shape == b.shape and relerr(a, _np(b)) <= 1e-4
+
+
+def test_mamba_cell_notices_a_carry_overwritten_before_the_backward():
+    """The decay leaf is read by the backward: a rollout that reuses its buffer in between must not pass in silence."""
+    from memorax_amd import sequence_models as sm
+    torch.manual_seed(5)
+    cell = sm.MambaCell(16, num_heads=2, head_dim=32, state_dim=32).cuda()
+    carry = (torch.zeros(3, 1, 2, 32, 32, device="cuda"), torch.full((3, 1, 2, 1, 1), 0.5, device="cuda"))
+    nxt, y = cell.whole(torch.randn(3, 5, 16, device="cuda"), torch.zeros(3, 5, dtype=torch.bool, device="cuda"), carry)
+    loss = y.sum() + nxt[1].sum()
+    carry[1].mul_(2.0)
+    with pytest.raises(RuntimeError, match="inplace operation"):
+        loss.backward()
