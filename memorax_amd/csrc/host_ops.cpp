@@ -907,8 +907,6 @@ std::vector<Tensor> mlstm_act(const Tensor &x, int norm, const OptTensor &scale,
     return {row_dense(y, 0, std::nullopt, std::nullopt, 0.0, false, {p[12]}, {std::nullopt}, at::kFloat, at::kFloat, x)[0], Co, lfo, no, mo};
 }
 
-constexpr int64_t ROW_DENSE_ROWS = 16384;   // up to here one launch beats the array library's products and casts
-
 // z, h~, gate (B,1,D), done (B,1), the carry's leaves (B,1,D) float32 -> y, log_state, log_decay
 std::tuple<Tensor, Tensor, Tensor> mingru_step(const Tensor &z, const Tensor &x, const OptTensor &gate, const Tensor &done_,
                                                const Tensor &log_state, const Tensor &log_decay, bool in_place)
@@ -1582,6 +1580,40 @@ struct DenseOp {
     }
 };
 
+// Whether the row kernel beats the array library's products on rows of (at most) K features, for layers whose weights hold `weights`
+// elements together.  It reads every weight once per 16 or 32 rows, so beyond a few hundred MFLOP a layer the library's larger tiles take
+// over, and above 512 features its tiles are the small ones whatever the rows.  Plain layers, device time here / the library's (which costs
+// the host 19 us a layer, 30 under autocast, against 5-7 for one launch): rows x K x n, float32 1024 x 256 x 256 6.5 / 5.8 us, 4096 x 256 x
+// 256 12 / 10, 16384 x 256 x 256 34 / 22, 4096 x 512 x 1024 63 / 36, 256 x 1024 x 256 15 / 5.6, 16384 x 1024 x 4096 2227 / 966; bfloat16
+// products of float32 rows and weights 4096 x 256 x 256 7 / 9, 16384 x 256 x 256 15 / 16, 4096 x 512 x 1024 33 / 15, 16384 x 1024 x 4096
+// 1208 / 131.
+// fused: an acting block, whose composition has a norm, casts, a sum and a dozen calls more.  Whole blocks in a graph / host-issued, fused
+// over composed (gated recurrence, float32): 1024 x 512 62 / 76 and 61 / 74, 2048 x 512 96 / 80 and 91 / 134, 4096 x 512 153 / 129 and
+// 147 / 135, 64 x 1024 38 / 47 and 39 / 135, 256 x 1024 65 / 60 and 62 / 134, 1024 x 1024 194 / 109 and 182 / 133, 32 x 2048 67 / 57 and
+// 64 / 136; bfloat16 4096 x 512 110 / 87, 1024 x 1024 166 / 75, 32 x 2048 65 / 76.
+constexpr int64_t ROW_DENSE_ROWS = 16384, ROW_DENSE_K = 512;
+bool rows_pay(int64_t rows, int64_t K, int64_t weights, int64_t layers, bool fused, bool bf16)
+{
+    if (rows > ROW_DENSE_ROWS) return false;
+    if (K <= ROW_DENSE_K) return rows * weights <= layers << 28;
+    return fused && K <= (bf16 ? 2048 : 1024) && rows * weights <= layers << 27;
+}
+
+// The layers of an acting block: what the row kernel multiplies with as it is (half: bfloat16 products, under autocast), where that pays.
+bool row_layers_suit(int64_t rows, const std::vector<Tensor> &weights, const std::vector<OptTensor> &biases, bool half)
+{
+    auto suits = [](const Tensor &t) { return t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16; };
+    int64_t widest = 0, elements = 0;
+    for (const Tensor &w : weights) {
+        if (w.scalar_type() != weights[0].scalar_type() || !(half ? suits(w) : w.scalar_type() == at::kFloat) || w.dim() != 2 || w.size(1) % 8 != 0)
+            return false;
+        widest = std::max(widest, w.size(1)), elements += w.numel();
+    }
+    for (const OptTensor &b : biases)
+        if (b.has_value() && !suits(*b)) return false;
+    return rows_pay(rows, widest, elements, (int64_t)weights.size(), true, half);   // (which takes no more features than the kernel does)
+}
+
 // Few rows without gradients: the layers as one launch of the row kernel, where it takes the arrays as they are.
 bool rows_suit(const Tensor &x, const std::vector<Tensor> &weights, const std::vector<OptTensor> &biases, std::optional<ScalarType> cast)
 {
@@ -1589,8 +1621,10 @@ bool rows_suit(const Tensor &x, const std::vector<Tensor> &weights, const std::v
     auto suits = [](ScalarType dt) { return dt == at::kFloat || dt == at::kBFloat16; };
     auto fits = [](const Tensor &t) { return t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
     const auto wd = weights[0].scalar_type();
-    if (!x.is_cuda() || x.dim() < 2 || x.numel() == 0 || weights.size() > MRX_ROW_DENSE_LAYERS || K % 8 != 0 || K > 2048) return false;
-    if (x.numel() / K > ROW_DENSE_ROWS || !suits(x.scalar_type()) || !suits(wd) || !fits(x)) return false;
+    if (!x.is_cuda() || x.dim() < 2 || x.numel() == 0 || weights.size() > MRX_ROW_DENSE_LAYERS || K % 8 != 0) return false;
+    int64_t elements = 0;
+    for (const Tensor &w : weights) elements += w.numel();
+    if (!rows_pay(x.numel() / K, K, elements, (int64_t)weights.size(), false, cast.has_value() || wd == at::kBFloat16) || !suits(x.scalar_type()) || !suits(wd) || !fits(x)) return false;
     if (cast.has_value() ? *cast != at::kBFloat16 : wd != x.scalar_type()) return false;
     for (size_t l = 0; l < weights.size(); ++l) {
         if (weights[l].scalar_type() != wd || weights[l].dim() != 2 || weights[l].size(1) != K || weights[l].size(0) == 0 || !fits(weights[l])) return false;
@@ -1949,6 +1983,8 @@ PYBIND11_MODULE(_native, m)
                         const OptTensor &residual) {
         return row_dense(x, norm, scale, nbias, eps, round_norm, weights, biases, product, out_dtype, residual);
     });
+    def("rows_pay", &rows_pay);
+    def("row_layers_suit", &row_layers_suit);
     def("lru_act", &lru_act);
     def("mlstm_act", &mlstm_act);
     def("mingru_step", &mingru_step);

@@ -247,8 +247,10 @@ class LRUCell(_DiagonalCell):
 
     def acting(self, x, norm, done, carry):
         params = [self.nu_log, self.theta_log, self.gamma_log, self.B_real, self.B_imag, self.C_real, self.C_imag, self.D]
+        # fused / composed, in a graph and host-issued (us, features = hidden width): 1024 x 512 64 / 75 and 61 / 146, 4096 x 512 190 / 142 and
+        # 180 / 147, 256 x 1024 66 / 78 and 64 / 146, 1024 x 1024 227 / 133 and 213 / 145
         if not (_as_written(self, LRUCell) and autocast_dtype(x) is None and self.hidden_dim % 8 == 0 and 2 * self.hidden_dim <= _RMS_NORM_MAX_D
-                and all(p.dtype is torch.float32 for p in params)):
+                and x.shape[0] * self.features * self.hidden_dim <= 1 << 28 and all(p.dtype is torch.float32 for p in params)):
             return None
         y, *carry = native().lru_act(x, *_norm_of(norm), params, done, *carry)
         return tuple(carry), y
@@ -447,7 +449,7 @@ class GatedLinearRecurrence(SequenceModel):
 # ----------------------------------------------------------------------------------
 # acting: one time step without gradients (ppo.py:105-143), rows = environments
 # ----------------------------------------------------------------------------------
-_ACTING_ROWS = 16384   # as in csrc/host_ops.cpp: up to here one launch beats the array library's products and casts
+_ACTING_ROWS = 16384   # the most rows that csrc/host_ops.cpp (rows_pay) gives to the row kernels
 
 
 def _acts(x, done, norm):
@@ -458,11 +460,10 @@ def _acts(x, done, norm):
 
 
 def _row_layers(x, layers):
-    """Whether the row kernels multiply with these layers' weights as they are (under autocast: whatever dtype the products run in)."""
-    wd = layers[0].weight.dtype
-    plain = (torch.float32,) if autocast_dtype(x) is None else (torch.float32, torch.bfloat16)
-    return wd in plain and all(_plain(m) and m.weight.dtype == wd and m.weight.shape[1] % 8 == 0 and m.weight.shape[1] <= _RMS_NORM_MAX_D
-                               and (m.bias is None or m.bias.dtype in (torch.float32, torch.bfloat16)) for m in layers)
+    """Whether the row kernels multiply with these layers' weights as they are (under autocast: whatever dtype the products run in), in
+    less time than the array library."""
+    return (all(map(_plain, layers))
+            and native().row_layers_suit(x.shape[0], [m.weight for m in layers], [m.bias for m in layers], autocast_dtype(x) is not None))
 
 
 def _hooked(module):

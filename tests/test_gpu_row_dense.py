@@ -127,3 +127,47 @@ def test_acting_lru_and_mlstm_blocks_equal_their_composition(cell, B):
                 a, b = (torch.view_as_real(v.detach().contiguous()) if v.is_complex() else v.detach() for v in (a, b))
                 assert relerr(a, _np(b)) <= 1e-4, (t, relerr(a, _np(b)))
             ref = tuple(c.detach() for c in ref)
+
+
+@pytest.mark.parametrize("autocast", [False, True])
+@pytest.mark.parametrize("rows,K,n,own", [(1024, 512, 512, True), (1025, 512, 512, False), (4096, 256, 256, True), (4097, 256, 256, False),
+                                          (16384, 64, 256, True), (16385, 64, 64, False), (9, 520, 16, False), (16384, 1024, 512, False),
+                                          (256, 2048, 64, False)])
+def test_dense_layers_take_the_row_kernel_up_to_its_line(rows, K, n, own, autocast):
+    """Beyond the line the array library's products, bit for bit; up to it one launch, whose sums run in another order."""
+    from memorax_amd.dense import Weights, dense_group
+    from memorax_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    x = torch.randn(rows, K, device="cuda", generator=g)
+    layers = [Weights(torch.randn(n, K, device="cuda", generator=g) / K ** 0.5, torch.randn(n, device="cuda", generator=g) if i else None)
+              for i in range(2)]
+    assert _lib.native().rows_pay(rows, K, 2 * n * K, 2, False, autocast) == own
+    with torch.no_grad(), torch.autocast("cuda", dtype=BF, enabled=autocast):
+        got = dense_group(x, layers)
+        want = [F.linear(x, w, b) for w, b in layers]
+    for y, w, (weight, bias) in zip(got, want, layers):
+        assert y.dtype == w.dtype
+        if not own:
+            assert torch.equal(y, w)
+        else:
+            ops = [t.to(BF).double() if autocast else t.double() for t in (x, weight)]
+            ref = F.linear(*ops, None if bias is None else bias.to(BF).double() if autocast else bias.double())
+            assert relerr(y, _np(ref)) <= (2e-2 if autocast else 1e-5)
+
+
+@pytest.mark.parametrize("autocast", [False, True])
+@pytest.mark.parametrize("rows,Fe,own", [(1024, 512, True), (1025, 512, False), (128, 1024, True), (129, 1024, False), (32, 2048, None), (33, 2048, False)])
+def test_acting_blocks_around_their_line(rows, Fe, own, autocast):
+    from memorax_amd import sequence_models as sm
+    torch.manual_seed(rows)
+    own = autocast if own is None else own   # rows of 2048 features: bfloat16 products only
+    block = sm.Residual(sm.PreNorm(sm.GatedLinearRecurrence(Fe), Fe)).cuda()
+    x, done = torch.randn(rows, 1, Fe, device="cuda"), torch.rand(rows, 1, device="cuda") < 0.3
+    with torch.autocast("cuda", dtype=BF, enabled=autocast):
+        with torch.no_grad():
+            assert (block.module.module.acting(x, block.module.norm, done, None) is not None) == own
+            carry, y = block(x, done)
+        ref, want = block(x, done)
+    assert y.dtype == want.dtype
+    for a, b in zip([y, *carry], [want, *ref]):
+        assert relerr(a, _np(b)) <= (2e-2 if autocast else 1e-4)
