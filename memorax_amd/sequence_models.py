@@ -455,7 +455,7 @@ _ACTING_ROWS = 16384   # the most rows that csrc/host_ops.cpp (rows_pay) gives t
 def _acts(x, done, norm):
     """Whether a pre-norm residual block on ``x`` is an acting step that the row kernels take."""
     return (not torch.is_grad_enabled() and x.dim() == 3 and x.shape[1] == 1 and 0 < x.shape[0] <= _ACTING_ROWS and x.is_cuda
-            and x.dtype == torch.float32 and x.shape[2] % 8 == 0 and x.is_contiguous() and autocast_dtype(x) in (None, torch.bfloat16)
+            and x.dtype == torch.float32 and x.shape[2] % 8 == 0 and x.shape[2] <= _RMS_NORM_MAX_D and x.is_contiguous() and autocast_dtype(x) in (None, torch.bfloat16)
             and (type(norm) is _RMSNorm or (type(norm) is _LayerNorm and norm.elementwise_affine)))
 
 

@@ -68,3 +68,17 @@ def test_an_acting_block_refuses_tangents(cell, dual):
             params[name] = make(p.detach())
         with pytest.raises(NotImplementedError, match="forward-mode"):
             torch.func.functional_call(block, params, (x, done, carry))
+
+
+@pytest.mark.parametrize("cell", ["lru", "mlstm", "recurrence"])
+def test_blocks_wider_than_the_row_kernel_act_on_their_composition(cell):
+    Fe = 2056
+    torch.manual_seed(1)
+    make = {"lru": lambda: sm.Memoroid(sm.LRUCell(Fe, 16)), "mlstm": lambda: sm.Memoroid(sm.mLSTMCell(Fe, hidden_dim=32, num_heads=2)),
+            "recurrence": lambda: sm.GatedLinearRecurrence(Fe, 16)}[cell]
+    block = sm.Residual(sm.PreNorm(make(), Fe, norm=sm.RMSNorm)).cuda()
+    x, done = torch.randn(3, 1, Fe, device="cuda"), torch.zeros(3, 1, dtype=torch.bool, device="cuda")
+    with torch.no_grad():
+        y = block(x, done)[1]
+    want = block(x, done)[1]
+    torch.testing.assert_close(y, want, rtol=0, atol=1e-5 * float(want.detach().abs().max()))
