@@ -61,7 +61,7 @@ struct MlstmStepArgs {
     int conv_k, H, done_f32;
     float g_floor;
 };
-__device__ __forceinline__ float silu(float x) { return x / (1.f + __expf(-x)); }
+__device__ __forceinline__ float silu(float x) { return x / (1.f + expf(-x)); }
 // Sum over groups of 4, 8 or 16 lanes, in every one of them: DPP moves.
 template <int LANES> __device__ __forceinline__ float lanes_total(float x)
 {

@@ -81,9 +81,9 @@ step_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restric
         }
     }
     if (PRO) {
-        const float inv = 1.f / fmaxf(sqrtf(reduce_row(dot4(k4, k4))), 1e-12f);
+        const float norm = fmaxf(sqrtf(reduce_row(dot4(k4, k4))), 1e-12f), inv = 1.f / norm;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) k4[e] = (float)(T)(k4[e] * inv);
+        for (int e = 0; e < 4; ++e) k4[e] = std::is_same<T, float>::value ? k4[e] / norm : (float)(T)(k4[e] * inv);   // bfloat16 hides the second rounding
     }
     const float *Sp = S_in ? S_in + bh * dvw * dkw : nullptr;
     const float decay = (!DELTA && glog) ? __expf(glog[bh]) : 1.f;  // gated linear attention: the carried state decays first
@@ -102,7 +102,7 @@ step_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restric
     for (int p = 0; p < NP; ++p) s[p] = reset ? zero4 : s[p] * decay;
     if (DELTA) {
         float bb = (float)beta[bh];
-        if (PRO) bb = (float)(T)(1.f / (1.f + __expf(-bb)));
+        if (PRO) bb = (float)(T)(1.f / (1.f + expf(-bb)));
 #pragma unroll
         for (int p = 0; p < NP; ++p) u[p] = bb * (u[p] - reduce_row(dot4(s[p], k4)));
     }
