@@ -1451,12 +1451,13 @@ Tensor weight_gradient(const Tensor &dy, const Tensor &x)
 }
 
 // Gradients of dense layers that read the rows x (rows, K), of dys[l] (rows, n_l): the input's (undefined unless wanted), then
-// each layer's weight and bias gradients (views of one float32 block; undefined unless wanted / without a bias).
+// each layer's weight and bias gradients (views of one float32 block; undefined unless wanted / without a bias).  The weights are read
+// for the input's gradient only.
 std::vector<Tensor> dense_grads(const Tensor &x, const std::vector<Tensor> &dys, const std::vector<Tensor> &weights, const std::vector<bool> &has_bias,
                                 bool want_dx, ScalarType dx_dtype, bool want_params)
 {
     const size_t L = dys.size();
-    TORCH_CHECK_VALUE(L >= 1 && L <= MRX_DENSE_LAYERS && weights.size() == L && has_bias.size() == L, "dense_grads takes 1 to ", MRX_DENSE_LAYERS, " layers");
+    TORCH_CHECK_VALUE(L >= 1 && L <= MRX_DENSE_LAYERS && (weights.size() == L || !want_dx) && has_bias.size() == L, "dense_grads takes 1 to ", MRX_DENSE_LAYERS, " layers");
     const int64_t rows = x.size(0), K = x.size(1);
     const auto dt = x.scalar_type();
     chk(x, "x");
@@ -1465,10 +1466,11 @@ std::vector<Tensor> dense_grads(const Tensor &x, const std::vector<Tensor> &dys,
     unsigned bias = 0;
     int64_t total = 0;
     for (size_t l = 0; l < L; ++l) {
-        n[l] = weights[l].size(0);
+        TORCH_CHECK_VALUE(dys[l].dim() == 2, "dy must be (rows, n)");
+        n[l] = dys[l].size(1);
         chk(dys[l], "dy", dt, {rows, n[l]});
-        chk(weights[l], "weight", dt, {n[l], K});
-        dy[l] = ptr(dys[l]), w[l] = ptr(weights[l]);
+        if (want_dx) chk(weights[l], "weight", dt, {n[l], K});
+        dy[l] = ptr(dys[l]), w[l] = want_dx ? ptr(weights[l]) : nullptr;
         total += n[l] * (K + has_bias[l]);
         if (has_bias[l]) bias |= 1u << l;
     }
@@ -1612,6 +1614,95 @@ bool row_layers_suit(int64_t rows, const std::vector<Tensor> &weights, const std
     for (const OptTensor &b : biases)
         if (b.has_value() && !suits(*b)) return false;
     return rows_pay(rows, widest, elements, (int64_t)weights.size(), true, half);   // (which takes no more features than the kernel does)
+}
+
+// Dense maps of one input head by head (block-diagonal matrices given by their blocks (H, o, d)): x (..., H d) -> (..., H o) each.
+// Batched products over strided views in both directions, so that a head's values -- infinities and NaN among them -- meet its own block
+// alone; the weights' gradients are the diagonal blocks of the whole dy^T x, an element of which reads one feature of each side.  As the array
+// library's einsum forms them (a batched product over every row for a result of 16 to 64 features a side, permutations around it) forward
+// and backward of three maps on 32768 rows take 312 us (four heads of 16) to 531 us (four of 64) and the host 390 us; here 106 to 282 and
+// 170.  (One product with the whole matrix, zeros included, takes 100 to 411 and 213, and lets heads see each other.)
+struct HeadMapsOp {
+    static constexpr int SAVED = 1;   // x; the maps follow in `maps`
+    static constexpr bool ONCE = true;
+    static const char *name() { return "MemoraxHeadMapsBackward"; }
+    std::vector<SavedVariable> maps;
+    variable_list backward(OpNode<HeadMapsOp> &node, std::array<Tensor, 1> &s, variable_list &grads)
+    {
+        c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
+        const Tensor &x = s[0];
+        variable_list out(1 + maps.size());
+        std::vector<Tensor> dys;
+        std::vector<size_t> wanted;
+        for (size_t l = 0; l < maps.size(); ++l) {
+            if (!grads[l].defined()) continue;
+            const Tensor map = maps[l].unpack();
+            const int64_t H = map.size(0), o = map.size(1), d = map.size(2);
+            const Tensor dy = grads[l].reshape({-1, H * o}).contiguous(), heads = dy.view({-1, H, o}).transpose(0, 1);
+            if (node.wants(0)) {
+                const bool first = !out[0].defined();
+                if (first) out[0] = fresh(x.sizes(), x.scalar_type(), x);
+                Tensor dx = out[0].view({-1, H, d}).transpose(0, 1);
+                if (first) at::bmm_out(dx, heads, map);
+                else dx.baddbmm_(heads, map);
+            }
+            if (node.wants(1 + l)) dys.push_back(dy), wanted.push_back(l);
+        }
+        if (wanted.empty()) return out;
+        const Tensor x2 = x.reshape({-1, x.size(-1)}).contiguous();
+        int64_t widest = 0;
+        for (const Tensor &dy : dys) widest = std::max(widest, dy.size(1));
+        std::vector<Tensor> whole;
+        if (x2.size(1) % 8 == 0 && dys.size() <= MRX_DENSE_LAYERS && reinterpret_cast<uintptr_t>(x2.data_ptr()) % 16 == 0 &&
+            params_suit(x2.scalar_type(), x2.size(0), x2.size(1), widest, dys.size(), 0)) {
+            whole = dense_grads(x2, dys, {}, std::vector<bool>(dys.size(), false), false, x2.scalar_type(), true);
+            whole.erase(whole.begin());
+        } else {
+            for (const Tensor &dy : dys) whole.push_back(weight_gradient(dy, x2));
+        }
+        for (size_t i = 0; i < wanted.size(); ++i) {
+            const auto map = maps[wanted[i]].unpack();
+            const int64_t H = map.size(0);
+            out[1 + wanted[i]] = whole[i].view({H, map.size(1), H, map.size(2)}).diagonal(0, 0, 2).permute({2, 0, 1}).contiguous();
+        }
+        return out;
+    }
+    void release()
+    {
+        for (auto &m : maps) m.reset_data();
+    }
+};
+
+std::vector<Tensor> head_maps(const Tensor &x, const std::vector<Tensor> &maps)
+{
+    bool need = need_grad(x);
+    for (const Tensor &m : maps) need = need_grad(m) || need;
+    TORCH_CHECK_VALUE(x.is_cuda() && x.dim() >= 2 && x.scalar_type() == at::kFloat && x.numel() > 0, "head_maps takes float32 rows on the GPU");
+    c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
+    std::vector<Tensor> out;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        for (const Tensor &m : maps) {
+            TORCH_CHECK_VALUE(m.dim() == 3 && m.scalar_type() == at::kFloat && m.size(0) * m.size(2) == x.size(-1), "a map must be float32 (H, o, d) with H d = ",
+                              x.size(-1), ", got ", m.sizes());
+            const int64_t H = m.size(0), o = m.size(1), d = m.size(2);
+            c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
+            shape.back() = H * o;
+            out.push_back(fresh(shape, at::kFloat, x));
+            Tensor y = out.back().view({-1, H, o}).transpose(0, 1);
+            at::bmm_out(y, x.reshape({-1, H, d}).transpose(0, 1), m.transpose(1, 2));
+        }
+    }
+    if (need) {
+        auto node = std::shared_ptr<OpNode<HeadMapsOp>>(new OpNode<HeadMapsOp>(), torch::autograd::deleteNode);
+        torch::autograd::edge_list edges = torch::autograd::collect_next_edges(x);
+        for (const Tensor &m : maps) edges.push_back(torch::autograd::impl::gradient_edge(m));
+        node->set_next_edges(std::move(edges));
+        for (Tensor &y : out) torch::autograd::set_history(y, node);
+        node->keep(0, x);
+        for (const Tensor &m : maps) node->op.maps.emplace_back(m, false);
+    }
+    return out;
 }
 
 // Few rows without gradients: the layers as one launch of the row kernel, where it takes the arrays as they are.
@@ -2000,6 +2091,7 @@ PYBIND11_MODULE(_native, m)
     def("residual_add", &residual_add);
     def("norm", &norm);
     def("dense_group", &dense_group);
+    def("head_maps", &head_maps);
     def("dense_grads", &dense_grads);
     def("weight_gradient", &weight_gradient);
     def("weight_gradient_slices", &weight_gradient_slices);

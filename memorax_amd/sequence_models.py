@@ -795,12 +795,6 @@ class _BlockDiagonalDense(nn.Module):
         bs = features // num_heads
         self.num_heads = num_heads
         self.kernel = nn.Parameter(torch.randn(num_heads, bs, bs) * math.sqrt(2.0 / (5.0 * bs)))
-        self.register_buffer("_eye", torch.eye(num_heads), persistent=False)
-
-    def whole_weight(self):
-        """The map as one (features, features) matrix, zero off the diagonal blocks."""
-        h, o, d = self.kernel.shape
-        return (self.kernel[:, :, None, :] * self._eye.to(self.kernel.dtype)[:, None, :, None]).reshape(h * o, h * d)
 
     def forward(self, x):
         *batch, f = x.shape
@@ -850,18 +844,22 @@ class mLSTMCell(MemoroidCellBase):
         x_mlstm, z = self.up_projection(x).chunk(2, dim=-1)
         u = _causal_conv_silu(x_mlstm, self.causal_conv)
         heads = lambda t: t.reshape(Bn, T, self.num_heads, d)  # noqa: E731
-        if self._heads_as_one(x):
-            q, k = dense_group(u, [Weights(self.query.whole_weight()), Weights(self.key.whole_weight())])
-            v = dense(x_mlstm.contiguous(), self.value.whole_weight())
+        if self._maps_native(u):
+            q, k = native().head_maps(u, [self.query.kernel, self.key.kernel])
+            (v,) = native().head_maps(x_mlstm, [self.value.kernel])
         else:
             q, k, v = self.query(u), self.key(u), self.value(x_mlstm)
         return heads(q), heads(k), heads(v), z, u
 
-    def _heads_as_one(self, x):
-        """Heads of up to 64 features go through one product with the block-diagonal matrix: a batched product of such narrow
-        blocks, its permutations and its weight gradients over every row cost several times the zeros' arithmetic."""
-        return (x.is_cuda and autocast_dtype(x) is None and self.hidden_dim // self.num_heads <= 64 and self.num_heads <= 8
-                and all(type(m) is _BlockDiagonalDense and not _hooked(m) for m in (self.query, self.key, self.value)))
+    def _maps_native(self, u):
+        """Whether the block-diagonal maps run as one operation each way (csrc/host_ops.cpp): float32 on the device, heads of up to 64
+        features, where a batched product's permutations and its weight gradients over every row cost several times its arithmetic."""
+        maps = (self.query, self.key, self.value)
+        return (self._few_narrow_heads(u) and u.dtype == torch.float32 and u.numel() > 0
+                and all(type(m) is _BlockDiagonalDense and not _hooked(m) and m.kernel.dtype == torch.float32 for m in maps))
+
+    def _few_narrow_heads(self, x):
+        return x.is_cuda and autocast_dtype(x) is None and self.hidden_dim // self.num_heads <= 64 and self.num_heads <= 8
 
     def forward(self, x, **kwargs):
         """Elements in kernel form: (k / sqrt(d), v, log_i, log_f, q)."""
@@ -869,7 +867,7 @@ class mLSTMCell(MemoroidCellBase):
 
     def _elements(self, q, k, v):
         Bn, T, H, d = q.shape
-        if self._heads_as_one(q):   # the gates read (q | k | v) head by head: three products that add up instead of that array
+        if self._few_narrow_heads(q):   # the gates read (q | k | v) head by head: three products that add up instead of that array
             w = torch.cat([self.i_gate.weight, self.f_gate.weight]).view(2 * H, H, 3, d)
             parts = [dense(t.reshape(Bn, T, H * d), w[:, :, i].reshape(2 * H, H * d)) for i, t in enumerate((q, k, v))]
             i_pre, f_pre = (parts[0] + parts[1] + parts[2] + torch.cat([self.i_gate.bias, self.f_gate.bias])).chunk(2, dim=-1)
