@@ -870,7 +870,8 @@ class mLSTMCell(MemoroidCellBase):
         if self._few_narrow_heads(q):   # the gates read (q | k | v) head by head: three products that add up instead of that array
             w = torch.cat([self.i_gate.weight, self.f_gate.weight]).view(2 * H, H, 3, d)
             parts = [dense(t.reshape(Bn, T, H * d), w[:, :, i].reshape(2 * H, H * d)) for i, t in enumerate((q, k, v))]
-            i_pre, f_pre = (parts[0] + parts[1] + parts[2] + torch.cat([self.i_gate.bias, self.f_gate.bias])).chunk(2, dim=-1)
+            i_pre, f_pre = (parts[0] + parts[1] + parts[2]).chunk(2, dim=-1)
+            i_pre, f_pre = (t if gate.bias is None else t + gate.bias for t, gate in ((i_pre, self.i_gate), (f_pre, self.f_gate)))
         else:
             gate_input = torch.cat([q, k, v], dim=-1).reshape(Bn, T, -1)
             i_pre, f_pre = dense_group(gate_input, [self.i_gate, self.f_gate])

@@ -65,3 +65,26 @@ def test_the_cell_keeps_its_heads_apart():
         q, k, v, _, _ = cell._project(torch.randn(2, 9, 16, device="cuda"))
     for t, finite in ((q, [True, False, True, True]), (k, [True, False, True, True]), (v, [True] * 4)):
         assert torch.isfinite(t).all(3).all(1).all(0).tolist() == finite
+
+
+@pytest.mark.parametrize("i_bias,f_bias", [(False, True), (True, False), (False, False)])
+@pytest.mark.parametrize("T", [1, 6])
+def test_gates_without_a_bias(i_bias, f_bias, T):
+    """A gate whose bias is taken away is a gate with a bias of zero."""
+    torch.manual_seed(2)
+    block = sm.Residual(sm.PreNorm(sm.Memoroid(sm.mLSTMCell(16, hidden_dim=64, num_heads=2)), 16)).cuda()
+    cell = block.module.module.cell
+    x, done = torch.randn(3, T, 16, device="cuda"), torch.zeros(3, T, dtype=torch.bool, device="cuda")
+    for gate, has in ((cell.i_gate, i_bias), (cell.f_gate, f_bias)):
+        if not has:
+            gate.bias.data.zero_()
+    with torch.no_grad():
+        want = block(x, done)[1]
+    for gate, has in ((cell.i_gate, i_bias), (cell.f_gate, f_bias)):
+        if not has:
+            gate.bias = None
+    with torch.no_grad():
+        y = block(x, done)[1]
+    assert relerr(y, want.cpu().numpy()) <= 1e-5
+    block(x, done)[1].sum().backward()
+    assert all(torch.isfinite(p.grad).all() for p in cell.parameters() if p.grad is not None)
