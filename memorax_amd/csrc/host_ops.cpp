@@ -20,6 +20,7 @@
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/generated/Functions.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/csrc/utils/pybind.h>
 
 #include <array>
@@ -788,6 +789,10 @@ void refuse(const OptTensor &t)
 {
     if (t.has_value()) refuse(*t);
 }
+// A traced graph (torch.jit.trace) would hold a kernel's results as constants: what is a composition of array operations is traced as
+// that, the rest refused.
+bool tracing() { return torch::jit::tracer::isTracing(); }
+void refuse_tracing() { TORCH_CHECK(!tracing(), "memorax_amd operators cannot be traced by torch.jit.trace"); }
 void refuse(const std::vector<Tensor> &ts)
 {
     for (const Tensor &t : ts) refuse(t);
@@ -798,6 +803,7 @@ void refuse(const std::vector<OptTensor> &ts)
 }
 template <typename... Ts> void refuse(const Ts &...ts) requires(sizeof...(Ts) > 1)
 {
+    refuse_tracing();
     (refuse(ts), ...);
 }
 
@@ -935,6 +941,7 @@ bool differentiable(const OptTensor &t) { return t.has_value() && differentiable
 
 template <typename... Ts> bool need_grad(const Ts &...ts)
 {
+    refuse_tracing();
     (refuse(ts), ...);
     return at::GradMode::is_enabled() && (differentiable(ts) || ...);
 }
@@ -1332,6 +1339,11 @@ struct SiluGateOp {
 
 Tensor silu_gate(const Tensor &h, const Tensor &g)
 {
+    if (tracing()) {
+        refuse_tangent(h), refuse_tangent(g);
+        const auto dt = c10::promoteTypes(h.scalar_type(), g.scalar_type());
+        return (h.to(at::kFloat) * at::silu(g.to(at::kFloat))).to(dt == at::kBFloat16 ? dt : at::kFloat);
+    }
     const bool need = need_grad(h, g);
     Tensor hc, gc, y;
     {
@@ -1359,7 +1371,7 @@ Tensor residual_add(const Tensor &x, const Tensor &branch)
                !transformed(t) && !t.key_set().has(c10::DispatchKey::Python) &&
                reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
     };
-    if (x.scalar_type() != at::kFloat || branch.scalar_type() != at::kBFloat16 || x.sizes() != branch.sizes() || x.numel() == 0 ||
+    if (tracing() || x.scalar_type() != at::kFloat || branch.scalar_type() != at::kBFloat16 || x.sizes() != branch.sizes() || x.numel() == 0 ||
         x.device() != branch.device() || !plain(x) || !plain(branch))
         return at::add(x, branch);
     const Tensor y = fresh_like(x);
@@ -1397,6 +1409,13 @@ struct NormOp {
 std::tuple<Tensor, Tensor> norm(const Tensor &x, const OptTensor &scale, const OptTensor &bias, double eps, std::optional<ScalarType> out_dtype,
                                 bool center, bool fork)
 {
+    if (tracing()) {
+        refuse_tangent(x), refuse_tangent(scale), refuse_tangent(bias);
+        const Tensor xf = x.to(at::kFloat), w = scale.has_value() ? scale->to(at::kFloat) : Tensor(), b = bias.has_value() ? bias->to(at::kFloat) : Tensor();
+        const Tensor y = center ? at::layer_norm(xf, x.sizes().slice(x.dim() - 1), some(w), some(b), eps)
+                                : at::rms_norm(xf, x.sizes().slice(x.dim() - 1), some(w), eps);
+        return {x, y.to(out_dtype.value_or(x.scalar_type() == at::kBFloat16 ? at::kBFloat16 : at::kFloat))};
+    }
     const bool need = need_grad(x, scale, bias);
     Tensor xc, sc, y, res;
     {
@@ -1729,9 +1748,9 @@ std::vector<Tensor> dense_group(const Tensor &x, const std::vector<Tensor> &weig
     TORCH_CHECK_VALUE(!weights.empty() && biases.size() == weights.size(), "dense_group takes one bias (or None) per weight");
     std::vector<Tensor> out;
     out.reserve(weights.size());
-    bool others = transformed(x);
+    bool others = tracing() || transformed(x);
     for (size_t l = 0; l < weights.size(); ++l) others = others || transformed(weights[l]) || transformed(biases[l]);
-    if (others) {   // the array library's layers, which vmap and the functional gradients know
+    if (others) {   // the array library's layers, which vmap, the functional gradients and the tracer know
         refuse_tangent(x);
         for (size_t l = 0; l < weights.size(); ++l) {
             refuse_tangent(weights[l]), refuse_tangent(biases[l]);
