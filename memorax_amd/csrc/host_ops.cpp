@@ -1526,14 +1526,16 @@ std::optional<ScalarType> autocast_dtype(const Tensor &x)
 // 3 x 512 2080 / 1740).  The input: several layers at once, as narrow (68200 x 128 -> 3 x 64 + 2 25 / 69, 131072 x 256 -> 3 x 256 + 4
 // 118 / 150; float32 68 / 93, but 131072 x 256 -> 3 x 256 536 / 454), or few rows, where the host's calls are what it costs.
 // In float32 the array library's slices also lead where they are whole and many and few layers have a bias, which it sums in a launch
-// of 50 us each (three layers without / with biases, here / there: 131072 x 256 -> 256 481 / 393 and 547 / 570, 32768 rows 145 / 129 and
-// 157 / 212; 131072 x 128 -> 256 252 / 221 and 285 / 391, 32768 rows 86 / 87 and 93 / 170; 131072 x 128 -> 128 143 / 147).
+// of 50 us each (131072 rows, three layers without / with biases, here / there: 256 -> 256 481 / 393 and 547 / 570, 128 -> 256 252 / 221 and
+// 285 / 391).  From how many slices on, by width (three layers without biases, here / there): 128 -> 128 16 slices 52 / 63, 32 82 / 82,
+// 64 138 / 130; 128 -> 192 16 slices 79 / 100, 32 135 / 109; 160 -> 256 8 slices 77 / 96, 16 133 / 104; 192 -> 256 80 / 97 and 135 / 106;
+// 256 -> 256 81 / 75 and 136 / 122 (and four slices 53 / 58).
 bool params_suit(ScalarType dt, int64_t rows, int64_t K, int64_t widest, size_t layers, size_t biases)
 {
     if (dt == at::kBFloat16) return K * widest <= 512 * 512;
     if (K * widest > 256 * 256) return false;
-    const bool wide = K * widest == 256 * 256;
-    return 2 * biases >= layers || K * widest < 128 * 256 || weight_gradient_slices(rows, widest, K) < (wide ? 16 : 32);
+    if (2 * biases >= layers || K * widest < 128 * 192) return true;
+    return weight_gradient_slices(rows, widest, K) < (K * widest < 128 * 256 ? 32 : 16);
 }
 bool input_suits(ScalarType dt, int64_t rows, int64_t K, int64_t widest, size_t layers)
 {
@@ -2112,6 +2114,7 @@ PYBIND11_MODULE(_native, m)
     def("dense_group", &dense_group);
     def("head_maps", &head_maps);
     def("dense_grads", &dense_grads);
+    def("params_suit", &params_suit);
     def("weight_gradient", &weight_gradient);
     def("weight_gradient_slices", &weight_gradient_slices);
     def("causal_conv_silu", &causal_conv_silu);

@@ -117,3 +117,16 @@ def test_dense_group_on_the_device_under_autocast():
     for m, g in zip(layers, gs):
         dw = g.bfloat16().double().reshape(-1, m.out_features).t() @ xe
         assert (m.weight.grad.double() - dw).abs().max().item() <= 1e-4 * dw.abs().max().item()
+
+
+@pytest.mark.parametrize("rows", [8192, 16384, 32768, 50000, 65536, 131072])
+def test_the_choice_of_the_parameter_kernels_has_no_place_for_one_width(rows):
+    """Layers a little narrower than 256 x 256 and 128 x 256 take the route of those widths; no narrower layer is refused what a wider
+    one gets."""
+    from memorax_amd._lib import native
+    suits = lambda K, n, biases=0: native().params_suit(torch.float32, rows, K, n, 3, biases)  # noqa: E731
+    assert suits(256, 256) == suits(256, 248) == suits(248, 256) == suits(200, 256)
+    routes = [suits(K, n) for K, n in sorted([(64, 64), (128, 128), (128, 184), (128, 200), (160, 200), (160, 256), (224, 256), (256, 256), (256, 264)],
+                                             key=lambda s: s[0] * s[1])]
+    assert routes == sorted(routes, reverse=True)
+    assert suits(256, 256, 2) and suits(128, 128) and not suits(256, 264, 3)
