@@ -16,31 +16,36 @@ from __future__ import annotations
 
 import contextlib
 import functools
+import threading
 
 import torch
 
 from . import _lib
 from . import kernels as K
 
-_step_in_place = False
+class _PerThread(threading.local):
+    step_in_place = False   # a thread that captures a step must not have another's acting steps overwrite their carries
+
+
+_here = _PerThread()
 
 
 @contextlib.contextmanager
 def step_in_place():
     """Inside this context the acting paths (one time step, no gradients) update the carried state where it
     lies instead of writing a new array: the state handed in is overwritten and handed back.  For a caller that
-    owns the carry's buffers (rollout.GraphedStep); elsewhere the carry a caller passes stays untouched."""
-    global _step_in_place
-    before, _step_in_place = _step_in_place, True
+    owns the carry's buffers (rollout.GraphedStep); elsewhere, and on other threads, the carry a caller passes
+    stays untouched."""
+    before, _here.step_in_place = _here.step_in_place, True
     try:
         yield
     finally:
-        _step_in_place = before
+        _here.step_in_place = before
 
 
 def stepping_in_place():
     """Whether the caller has allowed it (step_in_place)."""
-    return _step_in_place
+    return _here.step_in_place
 
 
 _FMAP = {None: 0, "none": 0, 0: 0, "elu1": 1, 1: 1}
@@ -215,9 +220,9 @@ def linear_attention(q, k, v, done, S0=None, feature_map="none"):
     if _no_steps(q):
         return _attention_without_steps(q, v, S0)
     if _native_heads(q, v):
-        return _lib.native().linear_attention(q, k, v, done, S0, _FMAP[feature_map], _step_in_place)
+        return _lib.native().linear_attention(q, k, v, done, S0, _FMAP[feature_map], _here.step_in_place)
     hd = _Heads(q, v, _FMAP[feature_map], narrow=True, split_k=True)
-    o, S_last = _lib.native().linear_attention(hd.qk(q), hd.qk(k), hd.v(v), done, hd.state_in(S0), hd.fmap, _step_in_place)
+    o, S_last = _lib.native().linear_attention(hd.qk(q), hd.qk(k), hd.v(v), done, hd.state_in(S0), hd.fmap, _here.step_in_place)
     return hd.out(o), hd.state_out(S_last)
 
 
@@ -236,7 +241,7 @@ def normalised_linear_attention(q, k, v, done, S0=None, z0=None, feature_map="el
         return (*out, q.new_zeros((B, T, H), dtype=torch.float32)) if return_ss else out
     hd = _Heads(q, v, _FMAP[feature_map], narrow=True)
     o, S_last, z_last, ss = _lib.native().normalised_linear_attention(hd.qk(q), hd.qk(k), hd.v(v), done, hd.state_in(S0),
-                                                                      hd.z_in(z0), hd.fmap, eps, return_ss, _step_in_place)
+                                                                      hd.z_in(z0), hd.fmap, eps, return_ss, _here.step_in_place)
     out = (hd.out(o), hd.state_out(S_last), hd.z_out(z_last))
     if not return_ss:
         return out
@@ -252,10 +257,10 @@ def gated_linear_attention(q, k, v, g, done, S0=None, feature_map="none"):
     if _no_steps(q):
         return _attention_without_steps(q, v, S0)
     if _native_heads(q, v):
-        return _lib.native().gated_linear_attention(q, k, v, g, done, S0, _FMAP[feature_map], _step_in_place)
+        return _lib.native().gated_linear_attention(q, k, v, g, done, S0, _FMAP[feature_map], _here.step_in_place)
     hd = _Heads(q, v, _FMAP[feature_map], narrow=True, split_k=True)
     o, S_last = _lib.native().gated_linear_attention(hd.qk(q), hd.qk(k), hd.v(v), hd.per_head(g), done, hd.state_in(S0),
-                                                     hd.fmap, _step_in_place)
+                                                     hd.fmap, _here.step_in_place)
     return hd.out(o), hd.state_out(S_last)
 
 
@@ -268,10 +273,10 @@ def delta_rule(q, k, v, beta, done, S0=None, resets=None):
     if _no_steps(q):
         return _attention_without_steps(q, v, S0)
     if _native_heads(q, v):
-        return _lib.native().delta_rule(q, k, v, beta, done, S0, False, K._RESETS[resets], _step_in_place)
+        return _lib.native().delta_rule(q, k, v, beta, done, S0, False, K._RESETS[resets], _here.step_in_place)
     hd = _Heads(q, v, narrow=True)
     o, S_last = _lib.native().delta_rule(hd.qk(q), hd.qk(k), hd.v(v), hd.per_head(beta), done, hd.state_in(S0), False,
-                                         K._RESETS[resets], _step_in_place)
+                                         K._RESETS[resets], _here.step_in_place)
     return hd.out(o), hd.state_out(S_last)
 
 
@@ -283,10 +288,10 @@ def deltanet(q, k, v, beta_raw, done, S0=None, resets=None):
     if _no_steps(q):
         return _attention_without_steps(q, v, S0)
     if _native_heads(q, v):
-        return _lib.native().delta_rule(q, k, v, beta_raw, done, S0, True, K._RESETS[resets], _step_in_place)
+        return _lib.native().delta_rule(q, k, v, beta_raw, done, S0, True, K._RESETS[resets], _here.step_in_place)
     hd = _Heads(q, v, narrow=True)   # where keys are padded: zeros leave their norm unchanged
     o, S_last = _lib.native().delta_rule(hd.qk(q), hd.qk(k), hd.v(v), hd.per_head(beta_raw), done, hd.state_in(S0), True,
-                                         K._RESETS[resets], _step_in_place)
+                                         K._RESETS[resets], _here.step_in_place)
     return hd.out(o), hd.state_out(S_last)
 
 

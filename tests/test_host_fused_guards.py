@@ -1,4 +1,6 @@
 """What the fused host paths must not pass by: hooks and replaced parts of a module, second derivatives, forward mode, functorch."""
+import threading
+
 import pytest
 import torch
 import torch.nn as nn
@@ -141,3 +143,14 @@ def test_functorch_is_refused_by_name(name):
     f = _operators()[name]
     with pytest.raises(RuntimeError, match="functorch"):
         torch.vmap(f)(torch.randn(5, 2, 3, 4))
+
+
+def test_stepping_in_place_is_a_thread_s_own():
+    """A thread that captures a step in place leaves the carries of the others' steps alone."""
+    seen = {}
+    with Fn.step_in_place():
+        t = threading.Thread(target=lambda: seen.update(other=Fn.stepping_in_place()))
+        t.start()
+        t.join()
+        seen["own"] = Fn.stepping_in_place()
+    assert seen == {"other": False, "own": True} and not Fn.stepping_in_place()
