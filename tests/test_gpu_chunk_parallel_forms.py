@@ -2,9 +2,10 @@
 sequential pair of kernels.py: values, carries and every gradient, from the smallest number of chunks the rule takes to a ragged
 end, whole and narrow heads, few and many resets, with and without carries.
 
-Both are measured against the masked products over the whole sequence in float64 on the same (rounded) inputs.  The two splits
-differ in the order of float32 sums and in where a bfloat16 operand is rounded, so the error of a result may be twice the
-sequential pair's (two roundings of one size, independent), plus 2e-6, what float32 sums show where the other happens to be exact."""
+Both are measured against the masked products over the whole sequence in float64 on the same (rounded) inputs.  No result's error is
+larger than the sequential pair's: over all cases below the mean ratio is 0.4 to 1.01, and 1.02 at most for any one, but for the
+three results that the two splits sum in another order (dg, z, dz0: means of 0.6 to 1.01, single cases up to 1.35, two roundings
+of one size).  1e-7 on top is float32's own rounding of a result, for where the other happens to be exact."""
 import pytest
 import torch
 
@@ -40,7 +41,7 @@ def _distance(a, b):
 def _compare(got, own, yard):
     for name in yard:
         far, near = _distance(got[name], yard[name]), _distance(own[name], yard[name])
-        assert far <= 2 * near + 2e-6, (name, far, near)
+        assert far <= (1.5 if name in ("dg", "z", "dz0") else 1.05) * near + 1e-7, (name, far, near)
 
 
 def _exact(q, k, v, gate, done, S0, z0, fmap, normalise):
