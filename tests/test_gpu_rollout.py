@@ -77,3 +77,28 @@ def test_graphed_step_equals_the_eager_step(autocast):
     for a, b in zip(_flat(mid, []), before):
         assert torch.equal(a, b)
 
+
+
+@pytest.mark.parametrize("autocast", [None, torch.bfloat16])
+@pytest.mark.parametrize("B,Fe", [(200, 1024), (1100, 512)])
+def test_graphed_step_of_wide_blocks(B, Fe, autocast):
+    """Blocks past the row kernel's line: their composition, the array library's products among it, replayed and checked every time."""
+    from memorax_amd import sequence_models as sm
+    from memorax_amd.rollout import GraphedStep
+    torso = _torso(sm, Fe, 64, 2)
+    g = torch.Generator(device="cuda").manual_seed(6)
+    with torch.no_grad():
+        assert torso.blocks[1].module.module.acting(torch.zeros(B, 1, Fe, device="cuda"), torso.blocks[1].module.norm,
+                                                    torch.zeros(B, 1, device="cuda"), None) is None
+    act = GraphedStep(torso, B, Fe, autocast=autocast)
+    carry = torso.initialize_carry(None, (B, Fe))
+    for i in range(5):
+        x, done = torch.randn(B, 1, Fe, device="cuda", generator=g), torch.rand(B, 1, device="cuda", generator=g) < 0.3
+        with torch.no_grad(), torch.autocast("cuda", dtype=autocast or torch.bfloat16, enabled=autocast is not None):
+            carry, want = torso(x, done, carry)
+        y = act(x, done)
+        torch.cuda.synchronize()
+        assert torch.equal(y, want), i
+        for got, ref in zip(_flat(act.carry, []), _flat(carry, [])):
+            assert torch.equal(got, ref), i
+        _ = (torch.randn(256, 256, device="cuda") @ torch.randn(256, 256, device="cuda")).sum().item()   # eager work between replays
