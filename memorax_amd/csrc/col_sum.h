@@ -27,10 +27,14 @@ __global__ void __launch_bounds__(64 * CS_GROUPS) column_sum_kernel(const float 
     red[g][c] = (s[0] + s[1]) + (s[2] + s[3]);
     __syncthreads();
     if (g == 0 && col < D) {
-        float t = 0.f;
+        float t[CS_GROUPS];   // in pairs: a running sum would round the whole total sixteen times
 #pragma unroll
-        for (int j = 0; j < CS_GROUPS; ++j) t += red[j][c];
-        out[col] = t;
+        for (int j = 0; j < CS_GROUPS; ++j) t[j] = red[j][c];
+#pragma unroll
+        for (int half = CS_GROUPS / 2; half > 0; half /= 2)
+#pragma unroll
+            for (int j = 0; j < half; ++j) t[j] += t[j + half];
+        out[col] = t[0];
     }
 }
 

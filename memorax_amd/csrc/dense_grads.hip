@@ -128,11 +128,24 @@ __global__ void __launch_bounds__(DG_THREADS, 2) dense_weight_grad_kernel(DenseG
     f32x4 acc[TM::TPW], accb[NBW];
     zero_acc<TM::TPW>(acc);
     zero_acc<NBW>(accb);
+    // the bias gradient, in float32 a step's sum at a time with what its additions round off (131072 x 4: 1.6e-7 -> 4e-8)
+    float bias_sum[NBW], bias_low[NBW];
+#pragma unroll
+    for (int j = 0; j < NBW; ++j) bias_sum[j] = bias_low[j] = 0.f;
     TileX tx;
     TileY ty;
     tx.load(x, r0, r1, a.rows, k0, a.K, tid);
     ty.load(dy, r0, r1, a.rows, n0, N, tid);
     int buf = 0;
+    auto sum_bias = [&]() {
+#pragma unroll
+        for (int j = 0; j < NBW; ++j) {
+            const float y = accb[j][0] - bias_low[j], s = bias_sum[j] + y;
+            bias_low[j] = (s - bias_sum[j]) - y;
+            bias_sum[j] = s;
+        }
+        zero_acc<NBW>(accb);
+    };
     for (int64_t r = r0; r < r1; r += RC, buf ^= 1) {
         T *const sx = lds + buf * BUF, *const sy = sx + RC * TileX::LD;
         tx.to_lds(sx, tid);
@@ -141,6 +154,7 @@ __global__ void __launch_bounds__(DG_THREADS, 2) dense_weight_grad_kernel(DenseG
             tx.load(x, r + RC, r1, a.rows, k0, a.K, tid);
             ty.load(dy, r + RC, r1, a.rows, n0, N, tid);
         }
+        if (sizeof(T) == 4 && bias) sum_bias();   // of the step before: its products are done
         sync_lds();   // the buffer two steps back has been read by every wave that reaches the barrier
         gemm<T, TK, TN, RC, KROW, KROW, DG_WAVES, MBW>(acc, sx, TileX::LD, sy, TileY::LD, w, lane, NoHook(),
                                                        [&](int ni, int, typename TT<T>::frag &f) {
@@ -153,11 +167,12 @@ __global__ void __launch_bounds__(DG_THREADS, 2) dense_weight_grad_kernel(DenseG
         const int k = k0 + TM::mt(w, j) * 16 + 4 * g, n = n0 + TM::nt(w, j) * 16 + i16;
         if (k < a.K && n < N) *reinterpret_cast<f32x4 *>(out + a.w_at[l] + (int64_t)n * a.K + k) = acc[j];
     }
+    if (bias) sum_bias();
     if (bias && g == 0) {
 #pragma unroll
         for (int j = 0; j < NBW; ++j) {
             const int n = n0 + TM::nt(w, j) * 16 + i16;
-            if (n < N) out[a.b_at[l] + n] = accb[j][0];
+            if (n < N) out[a.b_at[l] + n] = bias_sum[j];
         }
     }
 }
@@ -177,8 +192,13 @@ __global__ void __launch_bounds__(DG_THREADS, 2) dense_input_grad_kernel(DenseGr
     if (task < 0) return;
     const int64_t r0 = task / a.ktiles * TM_;
     const int k0 = (int)(task % a.ktiles) * TK;
-    f32x4 acc[TM::TPW];
+    // float32: a layer's share is summed by itself, as products one after another would sum it (three layers of 128: 3.5e-7 -> 2.1e-7, the
+    // array library's error; 131072 x 128 138 -> 142 us).  bfloat16 operands hide the difference.
+    constexpr bool BY_LAYER = sizeof(T) == 4;
+    f32x4 acc[TM::TPW], total[BY_LAYER ? TM::TPW : 1];
     zero_acc<TM::TPW>(acc);
+    zero_acc<(BY_LAYER ? TM::TPW : 1)>(total);
+    bool last[2] = {false, false};   // of its layer
     TileW tw[2];   // the steps on their way: two, so that a trip to memory spans two products
     TileY ty[2];
     int l = 0, n0 = 0, steps = 0;   // where the next fetch reads; steps fetched and not yet multiplied
@@ -187,7 +207,8 @@ __global__ void __launch_bounds__(DG_THREADS, 2) dense_input_grad_kernel(DenseGr
         tw[i].load(static_cast<const T *>(a.w[l]), n0, a.n[l], a.n[l], k0, a.K, tid);
         ty[i].load(static_cast<const T *>(a.dy[l]), r0, a.rows, a.rows, n0, a.n[l], tid);
         n0 += NC;
-        if (n0 >= a.n[l]) ++l, n0 = 0;
+        last[i] = n0 >= a.n[l];
+        if (last[i]) ++l, n0 = 0;
         ++steps;
     };
     fetch(0);
@@ -197,9 +218,15 @@ __global__ void __launch_bounds__(DG_THREADS, 2) dense_input_grad_kernel(DenseGr
         tw[i].to_lds(sw, tid);
         ty[i].to_lds(sy, tid);
         --steps;
+        const bool ends = last[i];
         fetch(i);
         sync_lds();
         gemm<T, TK, TM_, NC, KROW, ROWK, DG_WAVES, MBW>(acc, sw, TileW::LD, sy, TileY::LD, w, lane);
+        if (BY_LAYER && ends) {
+#pragma unroll
+            for (int j = 0; j < TM::TPW; ++j) total[j] += acc[j];
+            zero_acc<TM::TPW>(acc);
+        }
     };
     while (steps > 0) {
         step(0);
@@ -211,8 +238,9 @@ __global__ void __launch_bounds__(DG_THREADS, 2) dense_input_grad_kernel(DenseGr
         const int64_t r = r0 + TM::nt(w, j) * 16 + i16;
         if (k >= a.K || r >= a.rows) continue;
         const int64_t at = r * a.K + k;
-        if (a.dx_bf16) *reinterpret_cast<bf16x4 *>(static_cast<__bf16 *>(a.dx) + at) = TT<__bf16>::pack(acc[j][0], acc[j][1], acc[j][2], acc[j][3]);
-        else *reinterpret_cast<f32x4 *>(static_cast<float *>(a.dx) + at) = acc[j];
+        const f32x4 y = BY_LAYER ? total[BY_LAYER ? j : 0] : acc[j];
+        if (a.dx_bf16) *reinterpret_cast<bf16x4 *>(static_cast<__bf16 *>(a.dx) + at) = TT<__bf16>::pack(y[0], y[1], y[2], y[3]);
+        else *reinterpret_cast<f32x4 *>(static_cast<float *>(a.dx) + at) = y;
     }
 }
 
@@ -226,7 +254,11 @@ struct WeightPlan {
     int64_t slice_rows, total;
 };
 // 128 x 128 tiles, 64 where the layers are narrower; the rows cut so that five hundred workgroups run (two per compute unit), but no
-// shorter than four steps of a workgroup.
+// shorter than four steps of a workgroup, and a whole number of such rounds where a slice would have more than CHAIN rows: a running
+// sum in float32 errs in proportion to its length.  131072 rows, three layers of 256 x 256 and one of 256 x 4, error of the weights against
+// float64: bfloat16 (3648 rows a slice) 8.4e-8 -> 4.5e-8, where the array library's slices have 5.2e-8, 132 -> 134 us; float32 1.6e-7 -> 4.4e-8
+// (library 9.3e-8), 576 -> 618 us.
+constexpr int64_t CHAIN_BF16 = 2048, CHAIN_F32 = 512;
 WeightPlan plan_weights(int64_t rows, int64_t K, const int64_t *n, int layers, bool bf16, unsigned bias_mask)
 {
     WeightPlan p{};
@@ -245,6 +277,8 @@ WeightPlan plan_weights(int64_t rows, int64_t K, const int64_t *n, int layers, b
     const int64_t most = (rows + 4 * rc - 1) / (4 * rc);
     int64_t s = tiles >= 512 ? 1 : 512 / tiles;
     s = s > most ? most : s;
+    const int64_t chain = bf16 ? CHAIN_BF16 : CHAIN_F32;
+    if (tiles < 512 && rows > s * chain) s = (rows + s * chain - 1) / (s * chain) * 512 / tiles;
     p.slice_rows = ((rows + s - 1) / s + rc - 1) / rc * rc;
     p.slices = (int)((rows + p.slice_rows - 1) / p.slice_rows);
     p.tiles = (int)tiles;

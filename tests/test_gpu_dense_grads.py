@@ -57,3 +57,27 @@ def test_float32_groups_on_either_side_of_the_rule(rows, K, n, biases):
         assert float((w.grad.double() - d.double().t() @ x.double()).abs().max()) <= tol
         if b is not None:
             assert float((b.grad.double() - d.double().sum(0)).abs().max()) <= tol
+
+
+@pytest.mark.parametrize("rows,K,outs", [(131072, 256, [256, 256, 256, 4]), (32768, 256, [256, 256, 256, 4]), (1000, 64, [128, 128, 128]), (100, 256, [256, 256])])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_long_sums_keep_float32_s_precision(rows, K, outs, dtype):
+    """Rows with a mean, whose sums grow steadily: the parameters' gradients are within 7e-8 of float64 (2-norm; 2^-24 = 6e-8 is one
+    rounding of the result, and the partial sums' errors average out over the slices; 1.5e-7 where one slice is all there is, a chain
+    of a hundred additions), the input's no further than the array library's products that add up layer by layer."""
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    rnd = lambda n: (torch.randn(rows, n, generator=gen, device="cuda") + torch.randn(n, generator=gen, device="cuda")).to(dtype)  # noqa: E731
+    x, dys = rnd(K), [rnd(n) for n in outs]
+    ws = [(torch.randn(n, K, generator=gen, device="cuda") * K ** -0.5).to(dtype) for n in outs]
+    err = lambda got, want: float((got.double() - want).norm() / want.norm())  # noqa: E731
+    dx, *params = _lib.native().dense_grads(x, dys, ws, [True] * len(outs), True, torch.float32, True)
+    bound = 7e-8 if rows > 100 else 1.6e-7
+    for l, d in enumerate(dys):
+        assert err(params[l], d.double().t() @ x.double()) <= bound, l
+        assert err(params[len(outs) + l], d.double().sum(0)) <= 1.5 * bound, l   # a handful of values: a mean over fewer roundings
+    if dtype == torch.float32:
+        exact = sum(d.double() @ w.double() for d, w in zip(dys, ws))
+        lib = dys[0] @ ws[0]
+        for d, w in zip(dys[1:], ws[1:]):
+            lib.addmm_(d, w)
+        assert err(dx, exact) <= 1.1 * err(lib, exact)
