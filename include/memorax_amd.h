@@ -643,6 +643,31 @@ int mrx_dense_grads(void *stream, const void *x, const void *const *dys, const v
                     int layers, void *dx, float *params, float *workspace, int64_t rows, int64_t K, int dtype, int dx_dtype,
                     unsigned bias_mask);
 
+/* ---- Dense layers over many rows in bfloat16, their weights held in registers ----
+ * Up to three layers of n outputs (64 or more) and one of at most eight, on the same rows (rows, K).
+ * mrx_dense_rows_suit: which of the calls below take these sizes -- a mask of
+ *   MRX_DENSE_ROWS_FORWARD   mrx_dense_rows without residual (K 64, 128 or 256; n a multiple of 8),
+ *   MRX_DENSE_ROWS_RESIDUAL  mrx_dense_rows with residual (one layer; K and n 64, 128 or 256),
+ *   MRX_DENSE_ROWS_INPUT     mrx_dense_rows_input_grad (n 64, 128 or 256; K 64 to 1024, a multiple of 8; the narrow layer beside three
+ *                            wide ones and of an even number of outputs).
+ * mrx_dense_pack: for weights W_l (n_out[l], K) in w_dtype (MRX_F32, MRX_BF16) their bfloat16 copies (`copies`, or single entries
+ *   of it, may be NULL) and, unless NULL, `transposed`: bfloat16 (K, sum of n_out[l] over the layers of more than eight outputs), the W_l^T side by side.
+ * mrx_dense_rows: y_l = x W_l^T + b_l, everything bfloat16, sums in float32; biases in b_dtype (entries may be NULL; rounded to bfloat16).
+ *   residual (rows, n) float32, nullable: the one layer's y is float32, residual + (x W^T + b) without a rounding between.
+ * mrx_dense_rows_input_grad: dx (rows, K) bfloat16 = sum_l dy_l W_l from `transposed`; narrow_weights: the narrow layer's W (n_out, K) in
+ *   bfloat16.  dy_dtype MRX_F32 (one layer): dy is rounded to bfloat16 first, and written so to dy_copy unless that is NULL.
+ * Rows, weights and results of wide layers on 16-byte boundaries, a narrow layer's dy on 4. */
+#define MRX_DENSE_ROWS_FORWARD 1
+#define MRX_DENSE_ROWS_RESIDUAL 2
+#define MRX_DENSE_ROWS_INPUT 4
+int mrx_dense_rows_suit(int64_t rows, int64_t K, const int64_t *n_out, int layers);
+int mrx_dense_pack(void *stream, const void *const *weights, const int64_t *n_out, int layers, int64_t K, int w_dtype,
+                   void *const *copies, void *transposed);
+int mrx_dense_rows(void *stream, const void *x, const void *const *weights, const void *const *biases, void *const *outs,
+                   const int64_t *n_out, int layers, const float *residual, int64_t rows, int64_t K, int b_dtype);
+int mrx_dense_rows_input_grad(void *stream, const void *const *dys, const int64_t *n_out, int layers, const void *transposed,
+                              const void *narrow_weights, void *dx, void *dy_copy, int64_t rows, int64_t K, int dy_dtype);
+
 #ifdef __cplusplus
 }
 #endif

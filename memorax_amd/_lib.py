@@ -68,6 +68,10 @@ SIGNATURES = {
     "mrx_mlstm_step": (_I, [_P] * 23 + [_L] * 4 + [_I, ctypes.c_float]),
     "mrx_dense_grads_workspace": (_L, [_L] * 2 + [_P] + [_I] * 2 + [ctypes.c_uint]),
     "mrx_dense_grads": (_I, [_P] * 5 + [_I] + [_P] * 3 + [_L] * 2 + [_I] * 2 + [ctypes.c_uint]),
+    "mrx_dense_rows_suit": (_I, [_L] * 2 + [_P, _I]),
+    "mrx_dense_pack": (_I, [_P] * 3 + [_I, _L, _I] + [_P] * 2),
+    "mrx_dense_rows": (_I, [_P] * 6 + [_I, _P] + [_L] * 2 + [_I]),
+    "mrx_dense_rows_input_grad": (_I, [_P] * 3 + [_I] + [_P] * 4 + [_L] * 2 + [_I]),
     "mrx_gated_linear_attn_step": (_I, [_P] * 9 + [_L] * 4 + [_I] * 3),
     "mrx_mlstm_gates_fwd": (_I, [_P] * 8 + [_L] * 3 + [_I, ctypes.c_float]),
     "mrx_mlstm_gates_bwd": (_I, [_P] * 12 + [_L] * 3 + [_I, ctypes.c_float]),

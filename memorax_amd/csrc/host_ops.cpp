@@ -51,6 +51,7 @@ using torch::autograd::variable_list;
     X(mrx_gated_linear_attn_step) X(mrx_delta_rule_step) X(mrx_causal_conv_silu_fwd) X(mrx_causal_conv_silu_bwd)     \
     X(mrx_mamba_elements_fwd) X(mrx_mamba_elements_bwd) X(mrx_decay_last) X(mrx_mamba_readout_fwd)                   \
     X(mrx_mamba_readout_bwd) X(mrx_deltanet_step) X(mrx_mingru_step) X(mrx_row_dense) X(mrx_dense_grads) X(mrx_dense_grads_workspace)                  \
+    X(mrx_dense_rows_suit) X(mrx_dense_pack) X(mrx_dense_rows) X(mrx_dense_rows_input_grad)                          \
     X(mrx_lru_step) X(mrx_mlstm_step) X(mrx_linear_attn_norm_fwd_chunk_parallel) X(mrx_linear_attn_norm_bwd_chunk_parallel) \
     X(mrx_gated_linear_attn_fwd_chunk_parallel) X(mrx_gated_linear_attn_bwd_chunk_parallel)
 struct {
@@ -1543,6 +1544,88 @@ bool input_suits(ScalarType dt, int64_t rows, int64_t K, int64_t widest, size_t 
     return layers > 1 && ((K <= most && widest <= most) || (rows <= 4096 && K * widest <= 512 * 512));
 }
 
+// Layers in bfloat16 whose weights fit the registers of a compute unit: the rows pass all of them once, in either direction (dense_rows.hip).
+struct RowLayers {
+    int suit = 0;                  // MRX_DENSE_ROWS_*
+    std::vector<Tensor> weights;   // bfloat16, as the products read them
+    Tensor transposed;             // (K, outputs of the wide layers): what the gradient of the input reads
+};
+
+// Whether these layers on x -- the rows in bfloat16 -- are such; their weights are not looked at beyond type, shape and place.
+int row_layers(const Tensor &x, const std::vector<Tensor> &weights, const std::vector<OptTensor> &biases, bool cast)
+{
+    auto plain = [&](const Tensor &t) {
+        return t.device() == x.device() && t.has_storage() && !t.is_neg() && !t.key_set().has(c10::DispatchKey::Python);
+    };
+    auto suits = [&](ScalarType dt) { return dt == at::kBFloat16 || (cast && dt == at::kFloat); };
+    if (!x.is_cuda() || !plain(x) || x.scalar_type() != at::kBFloat16 || x.dim() < 2 || x.numel() == 0 || weights.size() > MRX_DENSE_LAYERS) return 0;
+    const int64_t K = x.size(-1);
+    const auto wd = weights[0].scalar_type();
+    std::array<int64_t, MRX_DENSE_LAYERS> n{};
+    std::optional<ScalarType> bd;
+    for (size_t l = 0; l < weights.size(); ++l) {
+        const Tensor &w = weights[l];
+        if (!plain(w) || w.scalar_type() != wd || !suits(wd) || w.dim() != 2 || w.size(1) != K || !w.is_contiguous() ||
+            reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 != 0)
+            return 0;
+        n[l] = w.size(0);
+        if (!biases[l].has_value()) continue;
+        if (!plain(*biases[l]) || !biases[l]->is_contiguous() || biases[l]->dim() != 1 || biases[l]->numel() != n[l] || !suits(biases[l]->scalar_type())) return 0;
+        if (bd.value_or(biases[l]->scalar_type()) != biases[l]->scalar_type()) return 0;
+        bd = biases[l]->scalar_type();
+    }
+    return lib.mrx_dense_rows_suit(x.numel() / K, K, n.data(), (int)weights.size());
+}
+
+// The weights of such layers for the products: cast, and transposed where the input's gradient will be wanted.
+RowLayers pack_layers(int suit, const std::vector<Tensor> &weights, bool transpose)
+{
+    RowLayers r;
+    r.suit = suit, r.weights = weights;
+    const int64_t K = weights[0].size(1);
+    const bool cast = weights[0].scalar_type() != at::kBFloat16;
+    transpose = transpose && (suit & MRX_DENSE_ROWS_INPUT);
+    if (!cast && !transpose) return r;
+    std::array<const void *, MRX_DENSE_LAYERS> w{};
+    std::array<void *, MRX_DENSE_LAYERS> copies{};
+    std::array<int64_t, MRX_DENSE_LAYERS> n{};
+    int64_t total = 0, wide = 0;
+    for (size_t l = 0; l < weights.size(); ++l) {
+        n[l] = weights[l].size(0), total += n[l] * K, w[l] = ptr(weights[l]);
+        if (n[l] > 8) wide += n[l];
+    }
+    if (cast) {
+        const Tensor all = fresh({total}, at::kBFloat16, weights[0]);
+        int64_t at = 0;
+        for (size_t l = 0; l < weights.size(); ++l, at += n[l - 1] * K) r.weights[l] = all.narrow(0, at, n[l] * K).view({n[l], K}), copies[l] = ptr(r.weights[l]);
+    }
+    if (transpose) r.transposed = fresh({K, wide}, at::kBFloat16, weights[0]);
+    check(lib.mrx_dense_pack(stream(), w.data(), n.data(), (int)weights.size(), K, code(weights[0].scalar_type()), copies.data(), ptr(r.transposed)),
+          "mrx_dense_pack");
+    return r;
+}
+
+// The outputs of such layers on the rows x (bfloat16, dense); residual: the one layer's result added to it, in float32.
+std::vector<Tensor> dense_rows(const Tensor &x, const RowLayers &layers, const std::vector<OptTensor> &biases, const Tensor &residual)
+{
+    std::vector<Tensor> out;
+    std::array<const void *, MRX_DENSE_LAYERS> w{}, b{};
+    std::array<void *, MRX_DENSE_LAYERS> y{};
+    std::array<int64_t, MRX_DENSE_LAYERS> n{};
+    auto bd = at::kFloat;
+    c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
+    for (size_t l = 0; l < layers.weights.size(); ++l) {
+        shape.back() = n[l] = layers.weights[l].size(0);
+        out.push_back(fresh(shape, residual.defined() ? at::kFloat : at::kBFloat16, x));
+        w[l] = ptr(layers.weights[l]), b[l] = ptr(biases[l]), y[l] = ptr(out[l]);
+        if (biases[l].has_value()) bd = biases[l]->scalar_type();
+    }
+    check(lib.mrx_dense_rows(stream(), ptr(x), w.data(), b.data(), y.data(), n.data(), (int)out.size(), fptr(residual), x.numel() / x.size(-1),
+                             x.size(-1), code(bd)),
+          "mrx_dense_rows");
+    return out;
+}
+
 // Several dense layers on one input: one cast of it, and the gradients with respect to it accumulated by the products
 // themselves (each adds onto the sum so far) instead of by a pass per layer.
 struct DenseOp {
@@ -1550,6 +1633,7 @@ struct DenseOp {
     static constexpr bool ONCE = true;
     static const char *name() { return "MemoraxDenseBackward"; }
     std::vector<SavedVariable> weights;
+    Tensor transposed;   // of a group whose input's gradient is mrx_dense_rows_input_grad's
     std::vector<bool> has_bias;
     ScalarType x_dtype;
     variable_list backward(OpNode<DenseOp> &node, std::array<Tensor, 1> &s, variable_list &grads)
@@ -1576,17 +1660,18 @@ struct DenseOp {
         }
         if (used.empty()) return out;
         regular = regular && used.size() <= MRX_DENSE_LAYERS && x2.is_contiguous() && reinterpret_cast<uintptr_t>(x2.data_ptr()) % 16 == 0;
+        const bool rows_dx = node.wants(0) && transposed.defined() && used.size() == n && regular && input_from_rows(dys, ws, x2.size(1), out);
         const bool own_params = want_params && regular && params_suit(dt, x2.size(0), x2.size(1), widest, used.size(), std::count(bias.begin(), bias.end(), true)),
-                   own_dx = node.wants(0) && regular && (x_dtype == at::kFloat || x_dtype == at::kBFloat16) &&
+                   own_dx = node.wants(0) && !rows_dx && regular && (x_dtype == at::kFloat || x_dtype == at::kBFloat16) &&
                             input_suits(dt, x2.size(0), x2.size(1), widest, used.size());
         if (own_params || own_dx) {
             auto r = dense_grads(x2, dys, ws, bias, own_dx, x_dtype, own_params);
-            out[0] = r[0];
+            if (own_dx) out[0] = r[0];
             for (size_t i = 0; i < used.size(); ++i) out[1 + used[i]] = r[1 + i], out[1 + n + used[i]] = r[1 + used.size() + i];
         }
         for (size_t i = 0; i < used.size(); ++i) {
             const size_t l = used[i];
-            if (node.wants(0) && !own_dx) {
+            if (node.wants(0) && !own_dx && !rows_dx) {
                 if (i > 0) out[0].addmm_(dys[i], ws[i]);
                 else out[0] = at::mm(dys[i], ws[i]);
             }
@@ -1597,9 +1682,27 @@ struct DenseOp {
         if (out[0].defined()) out[0] = out[0].view(x.sizes()).to(x_dtype);
         return out;
     }
+    // The input's gradient as the rows' way past the transposed weights.
+    bool input_from_rows(const std::vector<Tensor> &dys, const std::vector<Tensor> &ws, int64_t K, variable_list &out) const
+    {
+        std::array<const void *, MRX_DENSE_LAYERS> dy{};
+        std::array<int64_t, MRX_DENSE_LAYERS> n{};
+        const void *narrow = nullptr;
+        for (size_t l = 0; l < dys.size(); ++l) {
+            n[l] = ws[l].size(0), dy[l] = ptr(dys[l]);
+            if (reinterpret_cast<uintptr_t>(dy[l]) % 16) return false;
+            if (n[l] <= 8) narrow = ptr(ws[l]);
+        }
+        out[0] = fresh({dys[0].size(0), K}, at::kBFloat16, dys[0]);
+        check(lib.mrx_dense_rows_input_grad(stream(), dy.data(), n.data(), (int)dys.size(), ptr(transposed), narrow, ptr(out[0]), nullptr,
+                                            dys[0].size(0), K, MRX_BF16),
+              "mrx_dense_rows_input_grad");
+        return true;
+    }
     void release()
     {
         for (auto &w : weights) w.reset_data();
+        transposed.reset();
     }
 };
 
@@ -1765,7 +1868,7 @@ std::vector<Tensor> dense_group(const Tensor &x, const std::vector<Tensor> &weig
     for (size_t l = 0; l < weights.size(); ++l) need = need_grad(weights[l], biases[l]) || need;   // every one is looked at
     c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
     std::vector<Tensor> ws;
-    Tensor xc;
+    Tensor xc, transposed;
     {
         at::AutoDispatchBelowADInplaceOrView below;
         if (!need && rows_suit(x, weights, biases, cast)) {
@@ -1773,9 +1876,17 @@ std::vector<Tensor> dense_group(const Tensor &x, const std::vector<Tensor> &weig
             return row_dense(x, 0, std::nullopt, std::nullopt, 0.0, false, weights, biases, product, product, std::nullopt);
         }
         xc = cast.has_value() ? x.to(*cast) : x;
-        for (size_t l = 0; l < weights.size(); ++l) {
-            ws.push_back(cast.has_value() ? weights[l].to(*cast) : weights[l]);
-            out.push_back(at::linear(xc, ws[l], biases[l].has_value() && cast.has_value() ? OptTensor(biases[l]->to(*cast)) : biases[l]));
+        const int suit = row_layers(xc, weights, biases, cast.has_value());
+        if (suit & MRX_DENSE_ROWS_FORWARD) {
+            xc = dense16(xc);
+            auto layers = pack_layers(suit, weights, need_grad(x) && x.scalar_type() == at::kBFloat16);
+            out = dense_rows(xc, layers, biases, Tensor());
+            ws = std::move(layers.weights), transposed = layers.transposed;
+        } else {
+            for (size_t l = 0; l < weights.size(); ++l) {
+                ws.push_back(cast.has_value() ? weights[l].to(*cast) : weights[l]);
+                out.push_back(at::linear(xc, ws[l], biases[l].has_value() && cast.has_value() ? OptTensor(biases[l]->to(*cast)) : biases[l]));
+            }
         }
     }
     if (need) {
@@ -1785,6 +1896,7 @@ std::vector<Tensor> dense_group(const Tensor &x, const std::vector<Tensor> &weig
         for (const OptTensor &b : biases) edges.push_back(b.has_value() ? torch::autograd::impl::gradient_edge(*b) : torch::autograd::Edge());
         node->set_next_edges(std::move(edges));
         node->op.x_dtype = x.scalar_type();
+        node->op.transposed = transposed;
         for (Tensor &y : out) torch::autograd::set_history(y, node);
         node->keep(0, xc);
         for (size_t l = 0; l < ws.size(); ++l) {

@@ -1,0 +1,87 @@
+"""Dense layers whose weights wait in registers (mrx_dense_rows, mrx_dense_rows_input_grad) against double precision: rows around the
+tiles and the ring of tiles, each width and number of layers, the narrow layer, the closing layer of a residual branch."""
+import ctypes
+
+import pytest
+import torch
+
+from memorax_amd import _lib
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+ROWS = [1, 15, 33, 64, 700, 20011]
+
+
+def _ptrs(ts):
+    return (ctypes.c_void_p * 8)(*[None if t is None else t.data_ptr() for t in ts])
+
+
+def _stream():
+    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+
+def _rounded(got, exact, terms, eps=2.0 ** -8):
+    """One rounding of the result (eps: bfloat16's half unit and a margin of two) and the float32 sums' own (2^-24 of the terms' sum
+    of magnitudes an addition)."""
+    assert ((got.double() - exact).abs() <= eps * exact.abs() + terms).all()
+
+
+@pytest.mark.parametrize("rows", ROWS)
+@pytest.mark.parametrize("K,outs,bias", [(64, [64], True), (64, [72, 72, 72, 2], False), (128, [128, 128, 128, 4], True), (128, [256, 256], False),
+                                         (256, [256, 256, 256, 3], True), (256, [64, 64, 64, 8], False), (256, [1000], True)])
+def test_forward_and_input_gradient(rows, K, outs, bias):
+    lib = _lib.load()
+    print(f"case dense rows {rows} {K} {outs} {bias}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(rows + K)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    n = (ctypes.c_int64 * 8)(*outs)
+    suit = lib.mrx_dense_rows_suit(rows, K, n, len(outs))
+    assert suit & 1
+    x, params = rnd(rows, K).to(BF), [rnd(o, K) * K ** -0.5 for o in outs]
+    bs = [rnd(o) if bias else None for o in outs]
+    ws = [torch.empty_like(w, dtype=BF) for w in params]
+    wide = sum(o for o in outs if o > 8)
+    wt = torch.empty(K, wide, device="cuda", dtype=BF)
+    assert lib.mrx_dense_pack(_stream(), _ptrs(params), n, len(outs), K, _lib.MRX_F32, _ptrs(ws), wt.data_ptr()) == 0
+    assert all(torch.equal(w, p.to(BF)) for w, p in zip(ws, params))
+    assert torch.equal(wt, torch.cat([w.t() for w, o in zip(ws, outs) if o > 8], 1))
+    ys = [torch.full((rows + 3, o), 7.0, device="cuda", dtype=BF) for o in outs]   # rows past the last stay as they are
+    assert lib.mrx_dense_rows(_stream(), x.data_ptr(), _ptrs(ws), _ptrs(bs), _ptrs(ys), n, len(outs), None, rows, K, _lib.MRX_F32) == 0
+    for y, w, b in zip(ys, ws, bs):
+        b16 = 0.0 if b is None else b.to(BF).double()
+        _rounded(y[:rows], x.double() @ w.double().t() + b16, (K + 1) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t() + abs(b16)))
+        assert (y[rows:] == 7.0).all()
+    if not suit & 4:
+        assert lib.mrx_dense_rows_input_grad(_stream(), _ptrs(ys), n, len(outs), wt.data_ptr(), None, ys[0].data_ptr(), None, rows, K, _lib.MRX_BF16) == -2
+        return
+    dys = [rnd(rows, o).to(BF) for o in outs]
+    dx = torch.full((rows + 3, K), 7.0, device="cuda", dtype=BF)
+    narrow = next((w.data_ptr() for w, o in zip(ws, outs) if o <= 8), None)
+    assert lib.mrx_dense_rows_input_grad(_stream(), _ptrs(dys), n, len(outs), wt.data_ptr(), narrow, dx.data_ptr(), None, rows, K, _lib.MRX_BF16) == 0
+    _rounded(dx[:rows], sum(d.double() @ w.double() for d, w in zip(dys, ws)),
+             sum(outs) * 2.0 ** -24 * sum(d.double().abs() @ w.double().abs() for d, w in zip(dys, ws)))
+    assert (dx[rows:] == 7.0).all()
+
+
+@pytest.mark.parametrize("rows", ROWS)
+@pytest.mark.parametrize("K", [64, 128, 256])
+@pytest.mark.parametrize("n", [64, 128, 256])
+def test_the_layer_that_closes_a_residual_branch(rows, K, n):
+    lib = _lib.load()
+    print(f"case closing layer {rows} {K} {n}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(rows + K + n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    x, w, b, res = rnd(rows, K).to(BF), (rnd(n, K) * K ** -0.5).to(BF), rnd(n).to(BF), rnd(rows, n)
+    ns = (ctypes.c_int64 * 8)(n)
+    y = torch.full((rows + 3, n), 7.0, device="cuda")
+    assert lib.mrx_dense_rows(_stream(), x.data_ptr(), _ptrs([w]), _ptrs([b]), _ptrs([y]), ns, 1, res.data_ptr(), rows, K, _lib.MRX_BF16) == 0
+    terms = (K + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t() + b.double().abs() + res.double().abs())
+    _rounded(y[:rows], res.double() + x.double() @ w.double().t() + b.double(), terms, 2.0 ** -23)
+    assert (y[rows:] == 7.0).all()
+    # backward: the stream's gradient is float32, its rounded copy what the products read
+    dy, wt = rnd(rows, n), w.t().contiguous()
+    dx, copy = torch.full((rows + 3, K), 7.0, device="cuda", dtype=BF), torch.full((rows + 3, n), 7.0, device="cuda", dtype=BF)
+    assert lib.mrx_dense_rows_input_grad(_stream(), _ptrs([dy]), ns, 1, wt.data_ptr(), None, dx.data_ptr(), copy.data_ptr(), rows, K, _lib.MRX_F32) == 0
+    assert torch.equal(copy[:rows], dy.to(BF)) and (copy[rows:] == 7.0).all() and (dx[rows:] == 7.0).all()
+    d = dy.to(BF).double()
+    _rounded(dx[:rows], d @ w.double(), n * 2.0 ** -24 * (d.abs() @ w.double().abs()))
