@@ -1636,13 +1636,15 @@ struct DenseOp {
     Tensor transposed;   // of a group whose input's gradient is mrx_dense_rows_input_grad's
     std::vector<bool> has_bias;
     ScalarType x_dtype;
+    bool onto = false;   // the one layer's result was added to a float32 residual, whose gradient follows the others
     variable_list backward(OpNode<DenseOp> &node, std::array<Tensor, 1> &s, variable_list &grads)
     {
         c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
         const Tensor &x = s[0], x2 = x.reshape({-1, x.size(-1)});
         const size_t n = weights.size();
         const auto dt = x.scalar_type();
-        variable_list out(1 + 2 * n);
+        variable_list out(1 + 2 * n + onto);
+        if (onto) out.back() = grads[0];
         std::vector<Tensor> dys, ws;   // of the layers whose outputs were used: the others cost no products
         std::vector<size_t> used;
         std::vector<bool> bias;
@@ -1651,7 +1653,7 @@ struct DenseOp {
         for (size_t l = 0; l < n; ++l) {
             if (!grads[l].defined()) continue;
             ws.push_back(weights[l].unpack());
-            dys.push_back(grads[l].to(dt).reshape({-1, ws.back().size(0)}).contiguous());
+            dys.push_back((onto && transposed.defined() && grads[l].scalar_type() == at::kFloat ? grads[l] : grads[l].to(dt)).reshape({-1, ws.back().size(0)}).contiguous());
             used.push_back(l);
             bias.push_back(has_bias[l] && node.wants(1 + n + l));
             widest = std::max(widest, ws.back().size(0));
@@ -1660,7 +1662,8 @@ struct DenseOp {
         }
         if (used.empty()) return out;
         regular = regular && used.size() <= MRX_DENSE_LAYERS && x2.is_contiguous() && reinterpret_cast<uintptr_t>(x2.data_ptr()) % 16 == 0;
-        const bool rows_dx = node.wants(0) && transposed.defined() && used.size() == n && regular && input_from_rows(dys, ws, x2.size(1), out);
+        const bool rows_dx = node.wants(0) && transposed.defined() && used.size() == n && regular && input_from_rows(dys, ws, x2.size(1), want_params, out);
+        for (Tensor &dy : dys) dy = dy.to(dt);   // (a residual stream's gradient: unless that has left its rounded copy)
         const bool own_params = want_params && regular && params_suit(dt, x2.size(0), x2.size(1), widest, used.size(), std::count(bias.begin(), bias.end(), true)),
                    own_dx = node.wants(0) && !rows_dx && regular && (x_dtype == at::kFloat || x_dtype == at::kBFloat16) &&
                             input_suits(dt, x2.size(0), x2.size(1), widest, used.size());
@@ -1682,8 +1685,8 @@ struct DenseOp {
         if (out[0].defined()) out[0] = out[0].view(x.sizes()).to(x_dtype);
         return out;
     }
-    // The input's gradient as the rows' way past the transposed weights.
-    bool input_from_rows(const std::vector<Tensor> &dys, const std::vector<Tensor> &ws, int64_t K, variable_list &out) const
+    // The input's gradient as the rows' way past the transposed weights; a float32 dy is left rounded where the parameters want it.
+    bool input_from_rows(std::vector<Tensor> &dys, const std::vector<Tensor> &ws, int64_t K, bool want_params, variable_list &out) const
     {
         std::array<const void *, MRX_DENSE_LAYERS> dy{};
         std::array<int64_t, MRX_DENSE_LAYERS> n{};
@@ -1693,10 +1696,13 @@ struct DenseOp {
             if (reinterpret_cast<uintptr_t>(dy[l]) % 16) return false;
             if (n[l] <= 8) narrow = ptr(ws[l]);
         }
+        const auto dt = dys[0].scalar_type();
+        const Tensor copy = dt == at::kFloat && want_params ? fresh(dys[0].sizes(), at::kBFloat16, dys[0]) : Tensor();
         out[0] = fresh({dys[0].size(0), K}, at::kBFloat16, dys[0]);
-        check(lib.mrx_dense_rows_input_grad(stream(), dy.data(), n.data(), (int)dys.size(), ptr(transposed), narrow, ptr(out[0]), nullptr,
-                                            dys[0].size(0), K, MRX_BF16),
+        check(lib.mrx_dense_rows_input_grad(stream(), dy.data(), n.data(), (int)dys.size(), ptr(transposed), narrow, ptr(out[0]), ptr(copy),
+                                            dys[0].size(0), K, code(dt)),
               "mrx_dense_rows_input_grad");
+        if (copy.defined()) dys[0] = copy;
         return true;
     }
     void release()
@@ -1848,6 +1854,27 @@ bool rows_suit(const Tensor &x, const std::vector<Tensor> &weights, const std::v
     return true;
 }
 
+// Records the node of layers on x, which went into the products as xc with the weights ws.
+void record_dense(const Tensor &x, const Tensor &xc, const std::vector<Tensor> &weights, const std::vector<OptTensor> &biases,
+                  const std::vector<Tensor> &ws, const Tensor &transposed, const OptTensor &residual, std::vector<Tensor> &out)
+{
+    auto node = std::shared_ptr<OpNode<DenseOp>>(new OpNode<DenseOp>(), torch::autograd::deleteNode);
+    torch::autograd::edge_list edges = torch::autograd::collect_next_edges(x);
+    for (const Tensor &w : weights) edges.push_back(torch::autograd::impl::gradient_edge(w));
+    for (const OptTensor &b : biases) edges.push_back(b.has_value() ? torch::autograd::impl::gradient_edge(*b) : torch::autograd::Edge());
+    if (residual.has_value()) edges.push_back(torch::autograd::impl::gradient_edge(*residual));
+    node->set_next_edges(std::move(edges));
+    node->op.x_dtype = x.scalar_type();
+    node->op.transposed = transposed;
+    node->op.onto = residual.has_value();
+    for (Tensor &y : out) torch::autograd::set_history(y, node);
+    node->keep(0, xc);
+    for (size_t l = 0; l < ws.size(); ++l) {
+        node->op.weights.emplace_back(ws[l], false);
+        node->op.has_bias.push_back(biases[l].has_value());
+    }
+}
+
 std::vector<Tensor> dense_group(const Tensor &x, const std::vector<Tensor> &weights, const std::vector<OptTensor> &biases)
 {
     TORCH_CHECK_VALUE(!weights.empty() && biases.size() == weights.size(), "dense_group takes one bias (or None) per weight");
@@ -1889,22 +1916,46 @@ std::vector<Tensor> dense_group(const Tensor &x, const std::vector<Tensor> &weig
             }
         }
     }
-    if (need) {
-        auto node = std::shared_ptr<OpNode<DenseOp>>(new OpNode<DenseOp>(), torch::autograd::deleteNode);
-        torch::autograd::edge_list edges = torch::autograd::collect_next_edges(x);
-        for (const Tensor &w : weights) edges.push_back(torch::autograd::impl::gradient_edge(w));
-        for (const OptTensor &b : biases) edges.push_back(b.has_value() ? torch::autograd::impl::gradient_edge(*b) : torch::autograd::Edge());
-        node->set_next_edges(std::move(edges));
-        node->op.x_dtype = x.scalar_type();
-        node->op.transposed = transposed;
-        for (Tensor &y : out) torch::autograd::set_history(y, node);
-        node->keep(0, xc);
-        for (size_t l = 0; l < ws.size(); ++l) {
-            node->op.weights.emplace_back(ws[l], false);
-            node->op.has_bias.push_back(biases[l].has_value());
+    if (need) record_dense(x, xc, weights, biases, ws, transposed, OptTensor(), out);
+    return out;
+}
+
+// residual + dense(x): the layer that closes a residual branch of a float32 stream, under autocast or in bfloat16 as one launch, the sum
+// in float32 and unrounded between; the array library's sum of a layer's output otherwise.
+Tensor dense_onto(const Tensor &residual, const Tensor &x, const Tensor &weight, const OptTensor &bias)
+{
+    auto composed = [&]() {
+        const Tensor y = dense_group(x, {weight}, {bias})[0];
+        return residual.is_cuda() && residual.scalar_type() == at::kFloat && y.scalar_type() == at::kBFloat16 ? residual_add(residual, y) : at::add(residual, y);
+    };
+    if (tracing() || transformed(x) || transformed(weight) || transformed(bias) || transformed(residual) || x.dim() < 2 || weight.dim() != 2 ||
+        residual.scalar_type() != at::kFloat || residual._fw_grad(0).defined() || !residual.has_storage() || residual.is_neg() ||
+        residual.key_set().has(c10::DispatchKey::Python) || residual.device() != x.device() || !residual.is_contiguous() ||
+        reinterpret_cast<uintptr_t>(residual.data_ptr()) % 16 != 0)
+        return composed();
+    c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
+    shape.back() = weight.size(0);
+    const auto cast = autocast_dtype(x);
+    if (residual.sizes() != IntArrayRef(shape) || (cast.has_value() ? *cast : x.scalar_type()) != at::kBFloat16) return composed();
+    const bool need_x = need_grad(x), need_params = need_grad(weight, bias);
+    const bool need = (at::GradMode::is_enabled() && differentiable(residual)) || need_x || need_params;
+    RowLayers layers;
+    Tensor xc;
+    std::vector<Tensor> out;
+    {
+        c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
+        at::AutoDispatchBelowADInplaceOrView below;
+        xc = x.to(at::kBFloat16);
+        const int suit = row_layers(xc, {weight}, {bias}, cast.has_value());
+        if (suit & MRX_DENSE_ROWS_RESIDUAL) {
+            xc = dense16(xc);
+            layers = pack_layers(suit, {weight}, need_x && x.scalar_type() == at::kBFloat16);
+            out = dense_rows(xc, layers, {bias}, residual);
         }
     }
-    return out;
+    if (out.empty()) return composed();
+    if (need) record_dense(x, xc, {weight}, {bias}, layers.weights, layers.transposed, residual, out);
+    return out[0];
 }
 
 // ---- causal depthwise convolution over time with silu behind it (conv_cells.hip)
@@ -2224,6 +2275,7 @@ PYBIND11_MODULE(_native, m)
     def("residual_add", &residual_add);
     def("norm", &norm);
     def("dense_group", &dense_group);
+    def("dense_onto", &dense_onto);
     def("head_maps", &head_maps);
     def("dense_grads", &dense_grads);
     def("params_suit", &params_suit);

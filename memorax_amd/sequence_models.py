@@ -68,6 +68,10 @@ class SequenceModel(nn.Module):
         """The pre-norm residual block around this model for one acting step; see MemoroidCellBase.acting."""
         return None
 
+    def onto(self, residual, inputs, done, carry):
+        """(next_carry, residual + y) where the model's last layer takes the sum with it; else None."""
+        return None
+
 
 class MemoroidCellBase(nn.Module):
     """memoroid.py:20-33 plus the kernel hook ``scan``."""
@@ -92,6 +96,14 @@ class MemoroidCellBase(nn.Module):
         """(next_carry, x + read(scan(self(norm(x))))) for one time step without gradients (``_acts``), where a cell has its
         launches fused for these arrays; else None."""
         return None
+
+    def closes(self):
+        """Whether ``closing`` stands for this cell's read-out."""
+        return False
+
+    def closing(self, h, x):
+        """(layer, rows): read(h, x) is the dense layer ``layer`` on ``rows``."""
+        raise NotImplementedError
 
     def scan(self, z, initial_carry, done):
         """Reset-aware inclusive scan of the cell's algebra over time, carry-in
@@ -171,6 +183,15 @@ class Memoroid(SequenceModel):
         h, next_carry = self.cell.scan(z, initial_carry, done)
         y = self.cell.read(h, inputs, **kwargs)
         return next_carry, y
+
+    def onto(self, residual, inputs, done, carry):
+        if not (type(self).forward is Memoroid.forward and type(self.cell).whole is MemoroidCellBase.whole and self.cell.closes()):
+            return None
+        if carry is None:
+            carry = self.cell.initialize_carry(None, get_input_shape(inputs))
+        h, next_carry = self.cell.scan(self.cell(inputs), carry, done)
+        layer, rows = self.cell.closing(h, inputs)
+        return next_carry, native().dense_onto(residual, rows, layer.weight, layer.bias)
 
     def acting(self, x, norm, done, carry):
         return self.cell.acting(x, norm, done, self.cell.initialize_carry(None, get_input_shape(x)) if carry is None else carry)
@@ -426,9 +447,21 @@ class GatedLinearRecurrence(SequenceModel):
     def forward(self, inputs, done, initial_carry=None, **kwargs):
         if initial_carry is None:
             initial_carry = self.cell.initialize_carry(None, get_input_shape(inputs))
+        rows, next_carry = self._gated_states(inputs, done, initial_carry)
+        return next_carry, self.out(rows)
+
+    def _gated_states(self, inputs, done, carry):
         z, h_tilde, gate = dense_group(inputs, [self.cell.z, self.cell.h, self.gate])
-        h, next_carry = self.cell.scan(self.cell.elements(z, h_tilde), initial_carry, done)
-        return next_carry, self.out(_gated(h[0], gate))
+        h, next_carry = self.cell.scan(self.cell.elements(z, h_tilde), carry, done)
+        return _gated(h[0], gate), next_carry
+
+    def onto(self, residual, inputs, done, carry):
+        if not (type(self).forward is GatedLinearRecurrence.forward and _plain(self.out)):
+            return None
+        if carry is None:
+            carry = self.cell.initialize_carry(None, get_input_shape(inputs))
+        rows, next_carry = self._gated_states(inputs, done, carry)
+        return next_carry, native().dense_onto(residual, rows, self.out.weight, self.out.bias)
 
     def acting(self, x, norm, done, carry):
         layers = [self.cell.z, self.cell.h, self.gate]
@@ -575,7 +608,14 @@ class LinearAttentionCell(MemoroidCellBase):
         operations here that rescale and its gradient cost more passes than the norm kernel, which gets the
         row's statistic from the row it reads anyway: 1.72 -> 1.20 ms for this cell's forward and backward at
         1024 x 128 x 4 x 64.)"""
-        return self.output_projection(self.norm(h.reshape(*x.shape[:2], -1)).to(x.dtype))
+        layer, rows = LinearAttentionCell.closing(self, h, x)
+        return layer(rows)
+
+    def closes(self):
+        return _as_written(self, LinearAttentionCell) and _plain(self.output_projection)
+
+    def closing(self, h, x):
+        return self.output_projection, self.norm(h.reshape(*x.shape[:2], -1)).to(x.dtype)
 
     def acting(self, x, norm, done, carry):
         layers = [self.value, self.key, self.query]
@@ -641,8 +681,14 @@ class DeltaNetCell(MemoroidCellBase):
         return o, (S_last[:, None],)
 
     def read(self, h, x, **kwargs):
-        out = h.reshape(*x.shape[:2], -1)
-        return self.output_projection(self.norm(out).to(x.dtype))
+        layer, rows = DeltaNetCell.closing(self, h, x)
+        return layer(rows)
+
+    def closes(self):
+        return _as_written(self, DeltaNetCell) and _plain(self.output_projection)
+
+    def closing(self, h, x):
+        return self.output_projection, self.norm(h.reshape(*x.shape[:2], -1)).to(x.dtype)
 
     def acting(self, x, norm, done, carry):
         layers = [self.query, self.key, self.value, self.beta]
@@ -1040,6 +1086,11 @@ class Residual(nn.Module):
                 return acted
         if isinstance(inner, PreNorm) and hasattr(inner.norm, "fork"):   # x + f(norm(x)): one kernel takes both gradients of x
             inputs, normed = inner.norm.fork(inputs)
+            if (isinstance(inner.module, SequenceModel) and not kwargs and inputs.is_cuda and inputs.dtype is torch.float32
+                    and normed.dtype is torch.bfloat16 and not _hooked(inner.module)):   # a mixed-precision block on a float32 stream
+                summed = inner.module.onto(inputs, normed, done, initial_carry)
+                if summed is not None:
+                    return summed
             carry, y = inner.module(normed, done, initial_carry, **kwargs)
         else:
             carry, y = inner(inputs, done, initial_carry, **kwargs)

@@ -85,3 +85,57 @@ def test_the_layer_that_closes_a_residual_branch(rows, K, n):
     assert torch.equal(copy[:rows], dy.to(BF)) and (copy[rows:] == 7.0).all() and (dx[rows:] == 7.0).all()
     d = dy.to(BF).double()
     _rounded(dx[:rows], d @ w.double(), n * 2.0 ** -24 * (d.abs() @ w.double().abs()))
+
+
+def _block(kind, F, H, d):
+    from memorax_amd import sequence_models as sm
+    model = {"delta": lambda: sm.Memoroid(sm.DeltaNetCell(F, d, H)), "attention": lambda: sm.Memoroid(sm.LinearAttentionCell(F, d, H)),
+             "recurrence": lambda: sm.GatedLinearRecurrence(F)}[kind]()
+    return sm.Residual(sm.PreNorm(model, F, norm=sm.RMSNorm)).cuda()
+
+
+@pytest.mark.parametrize("kind", ["delta", "attention", "recurrence"])
+@pytest.mark.parametrize("B,T,F,H,d", [(3, 7, 64, 2, 32), (5, 40, 128, 2, 64), (2, 33, 256, 4, 64), (2, 20, 96, 2, 16)])
+def test_residual_blocks_close_with_their_sum(kind, B, T, F, H, d):
+    """The block with its last layer and the residual sum as one operation, against the composition (which a hook brings back): the
+    branch is rounded to bfloat16 once less, 2^-8 of it, in the result and in each gradient; 96 features take the composition."""
+    torch.manual_seed(F)
+    print(f"case block {kind} {B} {T} {F}", flush=True)
+    block = _block(kind, F, H, d)
+    x, done, gy = torch.randn(B, T, F, device="cuda"), torch.rand(B, T, device="cuda") < 0.05, torch.randn(B, T, F, device="cuda")
+
+    def run():
+        xs = x.clone().requires_grad_()
+        block.zero_grad()
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            carry, y = block(xs, done, block.initialize_carry(None, (B, F)))
+        name = type(y.grad_fn).__name__
+        y.backward(gy)
+        return name, [y.detach(), xs.grad, *[p.grad.clone() for p in block.parameters()], *carry]
+
+    name, got = run()
+    handle = block.module.module.register_forward_hook(lambda *a: None)
+    plain, want = run()
+    handle.remove()
+    assert plain != name or F == 96
+    assert got[0].dtype == torch.float32
+    for a, b in zip(got, want):
+        assert a.dtype == b.dtype and float((a.float() - b.float()).detach().norm()) <= 2e-2 * float(b.detach().float().norm())
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        _, y = block(x, done, block.initialize_carry(None, (B, F)))
+    assert float((y - got[0]).norm()) <= 1e-2 * float(got[0].norm())
+
+
+def test_the_sum_falls_back_to_the_array_library():
+    n = _lib.native()
+    x, w, b, res = torch.randn(4, 5, 64, device="cuda"), torch.randn(64, 64, device="cuda"), torch.randn(64, device="cuda"), torch.randn(4, 5, 64, device="cuda")
+    want = res + torch.nn.functional.linear(x, w, b)
+    torch.testing.assert_close(n.dense_onto(res, x, w, b), want)                                # float32 products
+    torch.testing.assert_close(n.dense_onto(res[:1], x, w, b), res[:1] + torch.nn.functional.linear(x, w, b))   # a sum that broadcasts
+    torch.testing.assert_close(n.dense_onto(res.transpose(0, 1).contiguous().transpose(0, 1), x, w, b), want)
+    half = n.dense_onto(res.to(BF), x.to(BF), w.to(BF), b.to(BF))
+    assert half.dtype == BF
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(res.to(BF).float(), torch.ones_like(res))
+        out = n.dense_onto(dual, x.to(BF), w.to(BF), b.to(BF))
+        assert torch.equal(torch.autograd.forward_ad.unpack_dual(out).tangent, torch.ones_like(res))
