@@ -650,7 +650,7 @@ int mrx_dense_grads(void *stream, const void *x, const void *const *dys, const v
  *   MRX_DENSE_ROWS_RESIDUAL  mrx_dense_rows with residual (one layer; K and n 64, 128 or 256),
  *   MRX_DENSE_ROWS_INPUT     mrx_dense_rows_input_grad (n 64, 128 or 256; K 64 to 1024, a multiple of 8; the narrow layer beside three
  *                            wide ones and of an even number of outputs).
- * mrx_dense_pack: for weights W_l (n_out[l], K) in w_dtype (MRX_F32, MRX_BF16) their bfloat16 copies (`copies`, or single entries
+ * mrx_dense_pack: for weights W_l (n_out[l], K; K a multiple of 4) in w_dtype (MRX_F32, MRX_BF16) their bfloat16 copies (`copies`, or single entries
  *   of it, may be NULL) and, unless NULL, `transposed`: bfloat16 (K, sum of n_out[l] over the layers of more than eight outputs), the W_l^T side by side.
  * mrx_dense_rows: y_l = x W_l^T + b_l, everything bfloat16, sums in float32; biases in b_dtype (entries may be NULL; rounded to bfloat16).
  *   residual (rows, n) float32, nullable: the one layer's y is float32, residual + (x W^T + b) without a rounding between.

@@ -17,6 +17,7 @@
 // 131072 rows x 256, us: three layers forward 96 -> 60 (with one of 4 beside them 113 -> 63), dx of three 110 -> 60, closing layer and sum
 // 89 -> 60, its dx with the cast 70 -> 48: 4.5 to 5.6 TB/s.
 #include "chunk_common.h"
+#include "row_dma.h"
 
 namespace mrx {
 namespace {
@@ -52,19 +53,6 @@ template <int SEGS, int KBS, bool XF32, int RC, bool XN> struct RowsTile {
     static_assert(STAGES >= 2, "a tile in use and one on its way");
 };
 
-// All but the last N vector memory operations of this wave are done (they end in order).
-template <int N> __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N < 63 ? N : 63) : "memory"); }
-// 16 (4) bytes for each lane from base + off to LDS, lane by lane from `lds` on.  The compiler does not see these, or it would wait for
-// all of them before every read of LDS.
-__device__ __forceinline__ void dma16(const void *base, uint32_t off, uint32_t lds)
-{
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
-}
-__device__ __forceinline__ void dma4(const void *base, uint32_t off, uint32_t lds)
-{
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
-}
-
 // Where the 16-byte piece q of row r lies in a tile of SPR pieces a row: at q ^ swz(r).
 template <int SPR> __device__ __forceinline__ int swz(int r) { return SPR >= 16 ? r & 15 : r / (16 / SPR) & (SPR - 1); }
 
@@ -85,7 +73,7 @@ __global__ void __launch_bounds__(DR_THREADS, 1) dense_rows_kernel(DenseRowsArgs
     const int l = group / a.groups_per_layer, g0 = group % a.groups_per_layer * (128 * NT), c0 = g0 + wv * 16 * NT;
     const int64_t tiles = (a.rows + TR - 1) / TR;
     if (worker >= tiles) return;
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
+    const uint32_t lds0 = lds_address(smem);
 
     // every request of a tile is made whatever exists of it: rows past the last are the last one, tiles past the last are the last one
     auto request = [&](int64_t t, int stage) {
@@ -223,7 +211,7 @@ __global__ void __launch_bounds__(DR_THREADS, 1) dense_rows_kernel(DenseRowsArgs
                 for (int j = 0; j < NT; ++j) {
                     const int q = (wv * 16 * NT + 4 * NT * g) / 4 + j;
                     const f32x4 x = *reinterpret_cast<const f32x4 *>(tile + SEGS * Tile::SEG + (16 * m + i) * (RC * 4) + (q ^ swz<RSPR>(16 * m + i)) * 16);
-                    __builtin_nontemporal_store(x + (acc[m][j] + bias[j]), reinterpret_cast<f32x4 *>(static_cast<float *>(a.y[l]) + r * a.n + col + 4 * j));
+                    *reinterpret_cast<f32x4 *>(static_cast<float *>(a.y[l]) + r * a.n + col + 4 * j) = x + (acc[m][j] + bias[j]);
                 }
             } else {
                 bf16x4 p[NT];
@@ -349,19 +337,35 @@ __global__ void __launch_bounds__(256) dense_pack_kernel(PackArgs a)
     int l = 0;
     while (b >= a.first[l + 1]) ++l;
     const int n0 = (b - a.first[l]) / kt * 64, k0 = (b - a.first[l]) % kt * 64, N = a.n[l];
-    for (int e = tid; e < 64 * 64; e += 256) {
-        const int r = n0 + e / 64, c = k0 + e % 64;
-        if (r >= N || c >= a.K) continue;
-        const int64_t at = (int64_t)r * a.K + c;
-        const __bf16 v = a.w_bf16 ? static_cast<const __bf16 *>(a.w[l])[at] : (__bf16)static_cast<const float *>(a.w[l])[at];
-        if (a.copy[l]) a.copy[l][at] = v;
-        tile[e / 64][e % 64] = v;
+    // four columns of four rows a thread, all of them requested before the first is used; K and thus a row's quads are whole
+    const int c = tid % 16 * 4;
+    bf16x4 v[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        const int r = n0 + tid / 16 + 16 * p;
+        v[p] = bf16x4{};
+        if (r >= N || k0 + c >= a.K) continue;
+        const int64_t at = (int64_t)r * a.K + k0 + c;
+        if (a.w_bf16) {
+            v[p] = *reinterpret_cast<const bf16x4 *>(static_cast<const __bf16 *>(a.w[l]) + at);
+        } else {
+            const f32x4 x = *reinterpret_cast<const f32x4 *>(static_cast<const float *>(a.w[l]) + at);
+            v[p] = TT<__bf16>::pack(x[0], x[1], x[2], x[3]);
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        const int r = tid / 16 + 16 * p;
+        if (a.copy[l] && n0 + r < N && k0 + c < a.K) *reinterpret_cast<bf16x4 *>(a.copy[l] + (int64_t)(n0 + r) * a.K + k0 + c) = v[p];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) tile[r][c + e] = v[p][e];
     }
     if (!a.transposed || a.at[l] < 0) return;
     __syncthreads();
-    for (int e = tid; e < 64 * 64; e += 256) {
-        const int c = k0 + e / 64, r = n0 + e % 64;
-        if (r < N && c < a.K) a.transposed[(int64_t)c * a.wide + a.at[l] + r] = tile[e % 64][e / 64];
+#pragma unroll
+    for (int p = 0; p < 16; ++p) {
+        const int k = tid / 64 + 4 * p, r = tid % 64;
+        if (n0 + r < N && k0 + k < a.K) a.transposed[(int64_t)(k0 + k) * a.wide + a.at[l] + n0 + r] = tile[r][k];
     }
 }
 
@@ -381,12 +385,12 @@ extern "C" int mrx_dense_pack(void *stream, const void *const *weights, const in
                               void *const *copies, void *transposed)
 {
     using namespace mrx;
-    if (!weights || !n_out || layers < 1 || layers > MRX_DENSE_LAYERS || K <= 0 || K > (1 << 16) || (w_dtype != MRX_F32 && w_dtype != MRX_BF16))
+    if (!weights || !n_out || layers < 1 || layers > MRX_DENSE_LAYERS || K <= 0 || K % 4 != 0 || K > (1 << 16) || (w_dtype != MRX_F32 && w_dtype != MRX_BF16))
         return MRX_ERR_INVALID_ARG;
     PackArgs a{};
     a.layers = layers, a.K = (int)K, a.w_bf16 = w_dtype == MRX_BF16, a.transposed = static_cast<__bf16 *>(transposed);
     for (int l = 0; l < layers; ++l) {
-        if (!weights[l] || n_out[l] <= 0 || n_out[l] > (1 << 16)) return MRX_ERR_INVALID_ARG;
+        if (!weights[l] || n_out[l] <= 0 || n_out[l] > (1 << 16) || !aligned(weights[l], 16) || (copies && !aligned(copies[l], 8))) return MRX_ERR_INVALID_ARG;
         a.w[l] = weights[l], a.copy[l] = copies ? static_cast<__bf16 *>(copies[l]) : nullptr, a.n[l] = (int)n_out[l];
         a.first[l + 1] = a.first[l] + (int)((n_out[l] + 63) / 64 * ((K + 63) / 64));
         a.at[l] = n_out[l] <= DR_NARROW ? -1 : a.wide;
