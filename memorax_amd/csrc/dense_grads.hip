@@ -18,6 +18,7 @@
 // of both operands instead: a second step there costs the registers those need, 123 -> 147 us).
 #include "chunk_common.h"
 #include "col_sum.h"
+#include "row_dma.h"
 
 #include <type_traits>
 
@@ -177,6 +178,157 @@ __global__ void __launch_bounds__(DG_THREADS, 2) dense_weight_grad_kernel(DenseG
     }
 }
 
+// ---- weight gradients in bfloat16 on tiles of 256 x 256
+// Four times the tile of the kernel above reads the rows half as often, and a ring of row tiles that go from memory to LDS directly
+// (row_dma.h) keeps three or four steps on their way where registers held one: one workgroup of eight waves on a compute unit, one
+// barrier a step of 32 rows.  Granules of 32 bytes are exchanged within a row (`granule`), so that the transposing reads, which take 32
+// bytes of sixteen rows at once, spread over the banks.  131072 rows x 256, with the partial results' sum, us: three layers of 256
+// 131 -> 98-103, with one of 4 beside them 146 -> 109.
+constexpr int WT_WAVES = 8, WT_THREADS = 64 * WT_WAVES, WT_ROWS = 32, WT_NARROW = 8, WT_SLOTS = 256;
+
+struct WideGradArgs {
+    const __bf16 *x, *dy[MRX_DENSE_LAYERS], *dyn;   // dyn: of a layer of nn outputs beside the wide ones
+    float *out;                                     // (slices, total)
+    int64_t w_at[MRX_DENSE_LAYERS], b_at[MRX_DENSE_LAYERS], wn_at, bn_at;
+    int n[MRX_DENSE_LAYERS], first_tile[MRX_DENSE_LAYERS + 1];
+    int layers, nn, K, ktiles, tiles, slices;
+    int64_t rows, slice_rows, total;
+};
+
+// Granule c of row r of a tile lies at c ^ granule(r): the rows that one transposing read takes (four and, eight further on, four more, by
+// each half wave) in eight different places.
+__device__ __forceinline__ int granule(int r) { return (r & 3) | (r >> 3 & 1) << 2; }
+__device__ __forceinline__ bf16x8 transposed_fragment(const unsigned char *p, int four_rows)
+{
+    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+    union {
+        s16x4 h[2];
+        bf16x8 f;
+    } u;
+    u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)p);
+    u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(p + four_rows));
+    return u.f;
+}
+
+template <bool NARROW> struct WideTile {
+    static constexpr int W = 256, WN = 2, WK = WT_WAVES / WN;        // outputs and features; waves across the outputs, across the features
+    static constexpr int NT = W / 16 / WN, KT = W / 16 / WK;         // 16 x 16 tiles of a wave
+    static constexpr int XB = WT_ROWS * W * 2, YB = XB, NB = NARROW ? WT_ROWS * WT_NARROW * 2 : 0, STAGE = XB + YB + NB;
+    static constexpr int OPS = (XB + YB) / 1024 / WT_WAVES, STAGES = 160 * 1024 / STAGE;
+    static_assert((XB + YB) % (1024 * WT_WAVES) == 0 && NT % WK == 0 && KT % WN == 0, "whole requests and tiles");
+};
+
+template <bool NARROW>   // a layer of nn outputs beside the wide ones
+__global__ void __launch_bounds__(WT_THREADS, 1) wide_weight_grad_kernel(WideGradArgs a)
+{
+    using T = WideTile<NARROW>;
+    constexpr int RBX = T::W * 2, RBY = RBX, NT = T::NT, KT = T::KT, STAGES = T::STAGES;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), i = lane & 15, g = lane >> 4;
+    const int64_t task = task_of((int64_t)a.tiles * a.slices);
+    if (task < 0) return;
+    const int slice = (int)(task / a.tiles), tile = (int)(task % a.tiles);
+    const int kt = tile % a.ktiles, nt = tile / a.ktiles;
+    int l = 0;
+    while (nt >= a.first_tile[l + 1]) ++l;
+    const int n0 = (nt - a.first_tile[l]) * T::W, k0 = kt * T::W, N = a.n[l];
+    const int64_t r0 = slice * a.slice_rows, r1 = r0 + a.slice_rows < a.rows ? r0 + a.slice_rows : a.rows;
+    const int steps = (int)((r1 - r0 + WT_ROWS - 1) / WT_ROWS);
+    const bool narrow = NARROW && nt == 0;                        // the narrow layer's gradient is these workgroups' too
+    const bool bias = a.b_at[l] >= 0 && kt == 0, bias_n = narrow && a.bn_at >= 0 && kt == 0 && wv == 0;
+    const bool requests_n = narrow && wv < T::NB / 256;
+    const uint32_t lds0 = lds_address(smem);
+
+    // every request of a step is made whatever exists of it: rows past the last are the last one, steps past the last are the last one
+    auto request = [&](int step, int stage) {
+        if (step >= steps) step = steps - 1;
+        const int64_t r = r0 + (int64_t)step * WT_ROWS;
+        const int last = (int)(a.rows - 1 - r < WT_ROWS - 1 ? a.rows - 1 - r : WT_ROWS - 1);
+        const uint32_t at = lds0 + stage * T::STAGE;
+#pragma unroll
+        for (int p = 0; p < T::OPS; ++p) {
+            const int op = wv * T::OPS + p;
+            const bool of_x = op < T::XB / 1024;
+            const int o = of_x ? op : op - T::XB / 1024, row = o * 2 + lane / 32, q = lane % 32 ^ granule(row) << 1;
+            const uint32_t wide = of_x ? a.K : N;
+            const __bf16 *base = of_x ? a.x + r * a.K + k0 : a.dy[l] + r * N + n0;
+            dma16(base, (uint32_t)(row < last ? row : last) * wide * 2 + q * 16, at + op * 1024);
+        }
+        if (requests_n) {
+            const uint32_t off = wv * 256 + lane * 4, end = (uint32_t)((last + 1) * a.nn * 2 - 4);
+            dma4(a.dyn + r * a.nn, off < end ? off : end, at + T::XB + T::YB + wv * 256);
+        }
+    };
+#pragma unroll
+    for (int s = 0; s < STAGES - 1; ++s) request(s, s);
+
+    const int wn = wv / T::WK, wk = wv % T::WK;
+    constexpr int BT = NT / T::WK, ST = KT / T::WN;   // of the bias and of the narrow layer: each wave its share
+    f32x4 acc[KT][NT], accb[BT], accn[ST], accbn = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < KT; ++k) zero_acc<NT>(acc[k]);
+    zero_acc<BT>(accb);
+    zero_acc<ST>(accn);
+    const int row = 8 * g + (i >> 2), sw = granule(row);
+    int stage = 0;
+    for (int step = 0; step < steps; ++step) {
+        if (requests_n) wait_vm<(STAGES - 2) * (T::OPS + 1)>();
+        else wait_vm<(STAGES - 2) * T::OPS>();
+        sync_lds();   // every wave has its part, and is done with the step before, whose place the next request takes
+        request(step + STAGES - 1, stage == 0 ? STAGES - 1 : stage - 1);
+        unsigned char *const sx = smem + stage * T::STAGE, *const sy = sx + T::XB, *const sn = sy + T::YB;
+        const int have = (int)(r1 - r0 - (int64_t)step * WT_ROWS);
+        if (have < WT_ROWS) {   // of the last step: rows that are not there count nothing
+            for (int e = tid; e < (WT_ROWS - have) * (RBX / 4); e += WT_THREADS) reinterpret_cast<uint32_t *>(sx + have * RBX)[e] = 0u;
+            for (int e = tid; e < (WT_ROWS - have) * (RBY / 4); e += WT_THREADS) reinterpret_cast<uint32_t *>(sy + have * RBY)[e] = 0u;
+            if (narrow)
+                for (int e = tid; e < (WT_ROWS - have) * a.nn / 2; e += WT_THREADS) reinterpret_cast<uint32_t *>(sn + have * a.nn * 2)[e] = 0u;
+            sync_lds();
+        }
+        const unsigned char *px = sx + row * RBX + (i & 3) * 8, *py = sy + row * RBY + (i & 3) * 8;
+        bf16x8 fx[KT];
+#pragma unroll
+        for (int k = 0; k < KT; ++k) fx[k] = transposed_fragment(px + ((wk * KT + k) ^ sw) * 32, 4 * RBX);
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            const bf16x8 fy = transposed_fragment(py + ((wn * NT + n) ^ sw) * 32, 4 * RBY);
+#pragma unroll
+            for (int k = 0; k < KT; ++k) acc[k][n] = TT<__bf16>::mma(fx[k], fy, acc[k][n]);
+        }
+        if (bias)
+#pragma unroll
+            for (int j = 0; j < BT; ++j)
+                accb[j] = TT<__bf16>::mma(TT<__bf16>::ones(), transposed_fragment(py + ((wn * NT + wk * BT + j) ^ sw) * 32, 4 * RBY), accb[j]);
+        if (narrow) {
+            bf16x8 fy = {};
+            if (i < a.nn)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) fy[e] = reinterpret_cast<const __bf16 *>(sn)[(8 * g + e) * a.nn + i];
+#pragma unroll
+            for (int j = 0; j < ST; ++j)
+                accn[j] = TT<__bf16>::mma(transposed_fragment(px + ((wk * KT + wn * ST + j) ^ sw) * 32, 4 * RBX), fy, accn[j]);
+            if (bias_n) accbn = TT<__bf16>::mma(TT<__bf16>::ones(), fy, accbn);
+        }
+        stage = stage == STAGES - 1 ? 0 : stage + 1;
+    }
+    wait_vm<0>();
+    float *const out = a.out + slice * a.total;
+#pragma unroll
+    for (int k = 0; k < KT; ++k)
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+            *reinterpret_cast<f32x4 *>(out + a.w_at[l] + (int64_t)(n0 + (wn * NT + n) * 16 + i) * a.K + k0 + (wk * KT + k) * 16 + 4 * g) = acc[k][n];
+    if (bias && g == 0)
+#pragma unroll
+        for (int j = 0; j < BT; ++j) out[a.b_at[l] + n0 + (wn * NT + wk * BT + j) * 16 + i] = accb[j][0];
+    if (narrow && i < a.nn) {
+#pragma unroll
+        for (int j = 0; j < ST; ++j)
+            *reinterpret_cast<f32x4 *>(out + a.wn_at + (int64_t)i * a.K + k0 + (wk * KT + wn * ST + j) * 16 + 4 * g) = accn[j];
+        if (bias_n && g == 0) out[a.bn_at + i] = accbn[0];
+    }
+}
+
 template <typename T, int TM_, int TK>
 __global__ void __launch_bounds__(DG_THREADS, 2) dense_input_grad_kernel(DenseGradArgs a)
 {
@@ -250,8 +402,9 @@ template <typename T, int R1, int W1, int R2, int W2, OpMode M2> constexpr size_
 }
 
 struct WeightPlan {
-    int tn, tk, tiles, slices;
+    int tn, tk, tiles, slices, narrow;   // narrow: the layer that rides along, -1
     int64_t slice_rows, total;
+    bool wide;                           // wide_weight_grad_kernel
 };
 // 128 x 128 tiles, 64 where the layers are narrower; the rows cut so that five hundred workgroups run (two per compute unit), but no
 // shorter than four steps of a workgroup, and a whole number of such rounds where a slice would have more than CHAIN rows: a running
@@ -259,7 +412,35 @@ struct WeightPlan {
 // float64: bfloat16 (3648 rows a slice) 8.4e-8 -> 4.5e-8, where the array library's slices have 5.2e-8, 132 -> 134 us; float32 1.6e-7 -> 4.4e-8
 // (library 9.3e-8), 576 -> 618 us.
 constexpr int64_t CHAIN_BF16 = 2048, CHAIN_F32 = 512;
-WeightPlan plan_weights(int64_t rows, int64_t K, const int64_t *n, int layers, bool bf16, unsigned bias_mask)
+
+constexpr int64_t WIDE_WORK = 3 << 16;
+// The plan on wide tiles, for bfloat16 layers whose sizes are whole tiles (one of two, four, six or eight outputs may ride along): one round of
+// workgroups, or whole rounds where a slice would be longer than CHAIN.  Its partial results are 64 MB whatever the rows, so it needs rows
+// times tiles (us, here / the plan below): three layers of 256 x 256 16384 rows 35 / 31, 49152 53 / 53, 65536 61 / 63, 100000 80 / 101,
+// 131072 98-103 / 131 and with one of 4 beside them 109 / 146; one of 512 x 512 32768 rows 48 / 47, 65536 68 / 77, 131072 118 / 151; two
+// of 256 x 256 65536 rows 49 / 46, 100000 63 / 64, 131072 72 / 77.  Tiles of half the size gained 8 % at 131072 rows and lost below 65536.
+bool plan_wide(WeightPlan &p, int64_t rows, int64_t K, const int64_t *n, int layers)
+{
+    if (K % 256 != 0) return false;
+    p.narrow = -1;
+    int64_t columns = 0;
+    for (int l = 0; l < layers; ++l) {
+        if (n[l] <= WT_NARROW && n[l] % 2 == 0 && p.narrow < 0) {
+            p.narrow = l;
+            continue;
+        }
+        if (n[l] % 256 != 0) return false;
+        columns += n[l];
+    }
+    const int64_t tiles = columns / 256 * (K / 256);
+    if (tiles < 2 || tiles > WT_SLOTS || rows * tiles < WIDE_WORK) return false;
+    const int64_t s = WT_SLOTS / tiles, rounds = (rows + s * CHAIN_BF16 - 1) / (s * CHAIN_BF16);
+    p.tiles = (int)tiles;
+    p.slice_rows = ((rows + rounds * s - 1) / (rounds * s) + WT_ROWS - 1) / WT_ROWS * WT_ROWS;
+    p.slices = (int)((rows + p.slice_rows - 1) / p.slice_rows);
+    return true;
+}
+WeightPlan plan_weights(int64_t rows, int64_t K, const int64_t *n, int layers, bool bf16, unsigned bias_mask, bool wide)
 {
     WeightPlan p{};
     int64_t widest = 0;
@@ -274,6 +455,10 @@ WeightPlan plan_weights(int64_t rows, int64_t K, const int64_t *n, int layers, b
     for (int l = 0; l < layers; ++l)
         if (bias_mask >> l & 1) p.total += n[l];
     p.total = (p.total + 3) / 4 * 4;   // rows of partial results start on 16-byte boundaries
+    if (wide && bf16 && plan_wide(p, rows, K, n, layers)) {
+        p.wide = true;
+        return p;
+    }
     const int64_t most = (rows + 4 * rc - 1) / (4 * rc);
     int64_t s = tiles >= 512 ? 1 : 512 / tiles;
     s = s > most ? most : s;
@@ -299,6 +484,24 @@ template <typename T, int TM, int TK> int launch_input_grad(hipStream_t st, Dens
                          dg_lds<T, dg_rows<T>(), TK, TM, dg_rows<T>(), ROWK>(), st, a);
 }
 
+template <bool NARROW> int launch_wide(hipStream_t st, const DenseGradArgs &a, const WeightPlan &p)
+{
+    using T = WideTile<NARROW>;
+    WideGradArgs w{};
+    w.x = static_cast<const __bf16 *>(a.x), w.out = a.out, w.K = a.K, w.ktiles = a.K / T::W, w.tiles = p.tiles, w.slices = p.slices, w.rows = a.rows;
+    w.slice_rows = p.slice_rows, w.total = p.total;
+    for (int l = 0; l < a.layers; ++l) {
+        if (l == p.narrow) {
+            w.dyn = static_cast<const __bf16 *>(a.dy[l]), w.nn = a.n[l], w.wn_at = a.w_at[l], w.bn_at = a.b_at[l];
+            continue;
+        }
+        const int j = w.layers++;
+        w.dy[j] = static_cast<const __bf16 *>(a.dy[l]), w.n[j] = a.n[l], w.w_at[j] = a.w_at[l], w.b_at[j] = a.b_at[l];
+        w.first_tile[j + 1] = w.first_tile[j] + a.n[l] / T::W;
+    }
+    return launch_kernel(wide_weight_grad_kernel<NARROW>, dim3(grid_of((int64_t)p.tiles * p.slices)), dim3(WT_THREADS), T::STAGES * T::STAGE, st, w);
+}
+
 template <typename T> int launch_grads(hipStream_t st, DenseGradArgs &a, const WeightPlan &p, float *params, float *workspace)
 {
     if (a.dx) {
@@ -312,7 +515,8 @@ template <typename T> int launch_grads(hipStream_t st, DenseGradArgs &a, const W
     if (!params) return MRX_OK;
     a.slices = p.slices, a.slice_rows = p.slice_rows, a.total = p.total;
     a.out = p.slices == 1 ? params : workspace;
-    const int rc = p.tn == 64 ? (p.tk == 64 ? launch_weight_grads<T, 64, 64>(st, a, p) : launch_weight_grads<T, 64, 128>(st, a, p))
+    const int rc = p.wide ? (p.narrow >= 0 ? launch_wide<true>(st, a, p) : launch_wide<false>(st, a, p))
+                   : p.tn == 64 ? (p.tk == 64 ? launch_weight_grads<T, 64, 64>(st, a, p) : launch_weight_grads<T, 64, 128>(st, a, p))
                               : (p.tk == 64 ? launch_weight_grads<T, 128, 64>(st, a, p) : launch_weight_grads<T, 128, 128>(st, a, p));
     if (rc != MRX_OK || p.slices == 1) return rc;
     return launch_column_sum(st, workspace, params, nullptr, p.slices, (int)p.total);
@@ -324,6 +528,8 @@ const KernelRegistrar registrars[] = {
     {reinterpret_cast<const void *>(dense_weight_grad_kernel<float, 128, 128>), big_lds<__bf16>},
     {reinterpret_cast<const void *>(dense_input_grad_kernel<__bf16, 128, 128>), big_lds<__bf16>},
     {reinterpret_cast<const void *>(dense_input_grad_kernel<float, 128, 128>), big_lds<__bf16>},
+    {reinterpret_cast<const void *>(wide_weight_grad_kernel<false>), WideTile<false>::STAGES *WideTile<false>::STAGE},
+    {reinterpret_cast<const void *>(wide_weight_grad_kernel<true>), WideTile<true>::STAGES *WideTile<true>::STAGE},
 };
 
 bool dense_shape_ok(int64_t rows, int64_t K, const int64_t *n, int layers)
@@ -341,8 +547,12 @@ extern "C" int64_t mrx_dense_grads_workspace(int64_t rows, int64_t K, const int6
 {
     using namespace mrx;
     if (!dense_shape_ok(rows, K, n_out, layers)) return 0;
-    const WeightPlan p = plan_weights(rows, K, n_out, layers, dtype == MRX_BF16, bias_mask);
-    return p.slices == 1 ? 0 : p.slices * p.total;
+    int64_t floats = 0;   // enough for either plan: which of them it is depends on where the rows lie
+    for (bool wide : {false, true}) {
+        const WeightPlan p = plan_weights(rows, K, n_out, layers, dtype == MRX_BF16, bias_mask, wide);
+        if (p.slices > 1) floats = p.slices * p.total > floats ? p.slices * p.total : floats;
+    }
+    return floats;
 }
 
 extern "C" int mrx_dense_grads(void *stream, const void *x, const void *const *dys, const void *const *weights, const int64_t *n_out,
@@ -368,7 +578,9 @@ extern "C" int mrx_dense_grads(void *stream, const void *x, const void *const *d
         a.b_at[l] = -1;
         if (bias_mask >> l & 1) a.b_at[l] = at, at += n_out[l];
     }
-    const WeightPlan p = plan_weights(rows, K, n_out, layers, bf, bias_mask);
+    bool wide = true;   // rows on the boundaries of whole requests
+    for (int l = 0; l < layers; ++l) wide = wide && aligned(dys[l], n_out[l] <= WT_NARROW ? 4 : 16);
+    const WeightPlan p = plan_weights(rows, K, n_out, layers, bf, bias_mask, wide);
     if (params && p.slices > 1 && (!workspace || !aligned(workspace, 16))) return MRX_ERR_INVALID_ARG;
     if ((int64_t)p.tiles * p.slices >= (1ll << 31) || p.total >= (1ll << 31) || (rows + 63) / 64 * ((K + 63) / 64) >= (1ll << 31))
         return MRX_ERR_INVALID_ARG;

@@ -81,3 +81,26 @@ def test_long_sums_keep_float32_s_precision(rows, K, outs, dtype):
         for d, w in zip(dys[1:], ws[1:]):
             lib.addmm_(d, w)
         assert err(dx, exact) <= 1.1 * err(lib, exact)
+
+
+@pytest.mark.parametrize("rows,K,outs,bias", [(98304, 256, [256, 256], True), (98309, 256, [256, 8, 256], True), (65567, 256, [256, 256, 2, 256], False),
+                                              (49171, 512, [512], True), (262400, 256, [6, 256, 256, 256], False), (25000, 512, [512, 512], True)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_wide_tiles(rows, K, outs, bias, shift):
+    """Bfloat16 parameters' gradients on 256 x 256 tiles: rows that end inside a step, one and several rounds, the narrow layer in every
+    place, and (shift) a gradient off the boundaries of whole requests, which takes the other kernel.  Bounds as above."""
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    print(f"case wide tiles rows={rows} K={K} outs={outs} bias={bias} shift={shift}", flush=True)
+    rnd = lambda n: (torch.randn(rows, n, generator=gen, device="cuda") + torch.randn(n, generator=gen, device="cuda")).to(torch.bfloat16)  # noqa: E731
+    x, dys = rnd(K), [rnd(n) for n in outs]
+    if shift:
+        at = next(l for l, n in enumerate(outs) if n > 8)
+        flat = torch.empty(dys[at].numel() + 4, device="cuda", dtype=torch.bfloat16)
+        flat[4:] = dys[at].flatten()
+        dys[at] = flat[4:].view(rows, -1)
+    _, *params = _lib.native().dense_grads(x, dys, [], [bias] * len(outs), False, torch.bfloat16, True)
+    err = lambda got, want: float((got.double() - want).norm() / want.norm())  # noqa: E731
+    for l, d in enumerate(dys):
+        assert err(params[l], d.double().t() @ x.double()) <= 7e-8, l
+        if bias:
+            assert err(params[len(outs) + l], d.double().sum(0)) <= 1.05e-7, l
