@@ -30,22 +30,11 @@ constexpr int LPR = HD / 4;    // lanes per row of the state
 constexpr int RPP = 256 / LPR;  // rows the workgroup covers at a time
 constexpr int NP = HD / RPP;    // times it does so
 
-__device__ __forceinline__ float reduce_row(float x)
-{
-    x += __shfl_xor(x, 1);
-    x += __shfl_xor(x, 2);
-    x += __shfl_xor(x, 4);
-    if (LPR == 16) x += __shfl_xor(x, 8);
-    return x;
-}
+__device__ __forceinline__ float reduce_row(float x) { return seg_sum<LPR>(x); }
 
-template <typename T> __device__ __forceinline__ f32x4 load4(const T *p);
-template <> __device__ __forceinline__ f32x4 load4<float>(const float *p) { return *reinterpret_cast<const f32x4 *>(p); }
-template <> __device__ __forceinline__ f32x4 load4<__bf16>(const __bf16 *p)
-{
-    const bf16x4 x = *reinterpret_cast<const bf16x4 *>(p);
-    return f32x4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]};
-}
+// Four elements as they lie in memory, and their values.
+template <typename T> using Raw4 = typename TT<T>::pack4;
+template <typename T> __device__ __forceinline__ f32x4 floats_of(const Raw4<T> &x) { return f32x4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]}; }
 
 __device__ __forceinline__ float dot4(const f32x4 &a, const f32x4 &b)
 {
@@ -65,14 +54,33 @@ step_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restric
 {
     const int tid = threadIdx.x, c4 = tid % LPR, r0 = tid / LPR;
     const int64_t bh = blockIdx.x;
-    const int b = (int)(bh / H);
-    const bool reset = done_at(done, done_f32, b);
+    const int b = (int)(blockIdx.x / (unsigned)H);
     const int dkw = NARROW ? dka : HD, dvw = NARROW ? dva : HD;
     const bool cin = !NARROW || 4 * c4 < dkw;  // this lane's four dk lie inside a row
     const T *qp = q + bh * dkw, *kp = k + bh * dkw, *vp = v + bh * dvw;
-
     const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
-    f32x4 k4 = cin ? load4<T>(kp + 4 * c4) : zero4, q4 = cin ? load4<T>(qp + 4 * c4) : zero4;
+
+    // Everything is requested before anything is used, and without branches between: a use, or the merge of a branch's values, would wait
+    // there -- flag, keys, state and values one after another are four trips to memory where this is one.  So the carried state is
+    // loaded whether or not the flag says reset, and where there is none what lies in S_out is loaded; both are dropped by select.
+    Raw4<T> kr = {}, qr = {};
+    if (cin) kr = *reinterpret_cast<const Raw4<T> *>(kp + 4 * c4), qr = *reinterpret_cast<const Raw4<T> *>(qp + 4 * c4);
+    uint32_t vr[NP], br = 0;
+#pragma unroll
+    for (int p = 0; p < NP; ++p) vr[p] = (!NARROW || r0 + RPP * p < dvw) ? load_raw<T>(vp + r0 + RPP * p) : 0u;
+    if (DELTA) br = load_raw<T>(beta + bh);
+    const float *Sp = (S_in ? S_in : S_out) + bh * dvw * dkw, *zp = z_in ? z_in : z_out;
+    f32x4 s[NP], z4 = zero4;
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        const int row = r0 + RPP * p;
+        s[p] = (cin && (!NARROW || row < dvw)) ? *reinterpret_cast<const f32x4 *>(Sp + row * dkw + 4 * c4) : zero4;
+    }
+    if (!DELTA && z_out && cin) z4 = *reinterpret_cast<const f32x4 *>(zp + bh * dkw + 4 * c4);
+    const float graw = (!DELTA && glog) ? glog[bh] : 0.f;
+    const uint32_t flag = done_raw(done, done_f32, b);
+
+    f32x4 k4 = floats_of<T>(kr), q4 = floats_of<T>(qr);
     if (FMAP && cin) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -85,23 +93,15 @@ step_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restric
 #pragma unroll
         for (int e = 0; e < 4; ++e) k4[e] = std::is_same<T, float>::value ? k4[e] / norm : (float)(T)(k4[e] * inv);   // bfloat16 hides the second rounding
     }
-    const float *Sp = S_in ? S_in + bh * dvw * dkw : nullptr;
-    const float decay = (!DELTA && glog) ? __expf(glog[bh]) : 1.f;  // gated linear attention: the carried state decays first
-    f32x4 s[NP];
-#pragma unroll
-    for (int p = 0; p < NP; ++p) {
-        const int row = r0 + RPP * p;
-        // the carried state is loaded whether or not the flag says reset, and dropped by select below: a load
-        // that waits for the flag would be a second trip to memory behind the first
-        s[p] = (Sp && cin && (!NARROW || row < dvw)) ? *reinterpret_cast<const f32x4 *>(Sp + row * dkw + 4 * c4) : zero4;
-    }
+    const bool reset = done_test(flag, done_f32);
+    const float decay = (!DELTA && glog) ? __expf(graw) : 1.f;  // gated linear attention: the carried state decays first
     float u[NP];
 #pragma unroll
-    for (int p = 0; p < NP; ++p) u[p] = (!NARROW || r0 + RPP * p < dvw) ? (float)vp[r0 + RPP * p] : 0.f;
+    for (int p = 0; p < NP; ++p) u[p] = raw_to_float<T>(vr[p]);
 #pragma unroll
-    for (int p = 0; p < NP; ++p) s[p] = reset ? zero4 : s[p] * decay;
+    for (int p = 0; p < NP; ++p) s[p] = reset || !S_in ? zero4 : s[p] * decay;
     if (DELTA) {
-        float bb = (float)beta[bh];
+        float bb = raw_to_float<T>(br);
         if (PRO) bb = (float)(T)(1.f / (1.f + expf(-bb)));
 #pragma unroll
         for (int p = 0; p < NP; ++p) u[p] = bb * (u[p] - reduce_row(dot4(s[p], k4)));
@@ -109,8 +109,7 @@ step_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restric
     float den = 1.f;
     if (!DELTA && z_out) {
         // every row's lanes recompute the normaliser of the sequence; row 0 stores it
-        f32x4 z4 = (z_in && cin) ? *reinterpret_cast<const f32x4 *>(z_in + bh * dkw + 4 * c4) : zero4;
-        if (reset) z4 = zero4;
+        if (reset || !z_in) z4 = zero4;
         z4 += k4;
         // updated in place, z_out is z_in: every row's lanes must hold the carried z before row 0 overwrites it
         // (a row that read it afterwards would add k a second time and divide by the wrong normaliser)
