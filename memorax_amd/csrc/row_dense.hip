@@ -12,9 +12,7 @@
 //
 // Rounding follows the composition it stands for: with bfloat16 products the normalised rows, the weights and the biases are
 // rounded to bfloat16, sums are float32, and a result is rounded to bfloat16 before the residual is added.
-#include <type_traits>
-
-#include "chunk_common.h"
+#include "row_parts.h"
 
 namespace mrx {
 namespace {
@@ -23,8 +21,8 @@ constexpr int RD_WAVES = 4, RD_THREADS = 64 * RD_WAVES;
 constexpr int RD_MAX_K = 2048;
 
 struct RowDenseArgs {
-    const void *x;
-    const float *scale, *nbias, *residual;
+    RowInput in;
+    const float *residual;
     const float *skip;      // K factors: skip_out = x + skip * norm(x), for the residual branch of a cell with a feed-through term
     float *skip_out;
     const void *w2;         // a single layer whose weights lie in two arrays: columns k1 .. K
@@ -32,86 +30,13 @@ struct RowDenseArgs {
     const void *w[MRX_ROW_DENSE_LAYERS], *b[MRX_ROW_DENSE_LAYERS];
     void *y[MRX_ROW_DENSE_LAYERS];
     int n[MRX_ROW_DENSE_LAYERS], first_tile[MRX_ROW_DENSE_LAYERS + 1];   // columns of a layer, its first 64-column tile
-    int layers, K, norm;          // norm: 0 none, 1 RMS, 2 layer norm
-    int64_t rows;
-    float eps, inv_K;
-    bool x_bf16, w_bf16, b_bf16, y_bf16, round_norm;   // round_norm: the normalised rows pass through bfloat16 (float32 products)
+    int layers;
+    bool x_bf16, w_bf16, b_bf16, y_bf16;
 };
 
-struct Quad {
-    float v[4];
-};
-template <bool BF> __device__ __forceinline__ Quad quad_of(const void *p, int64_t at)
-{
-    Quad q;
-    if (BF) {
-        const bf16x4 x = *reinterpret_cast<const bf16x4 *>(static_cast<const __bf16 *>(p) + at);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) q.v[e] = (float)x[e];
-    } else {
-        const f32x4 x = *reinterpret_cast<const f32x4 *>(static_cast<const float *>(p) + at);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) q.v[e] = x[e];
-    }
-    return q;
-}
-
-// Sum over a wave, in every lane: within rows of sixteen lanes by DPP moves (one instruction each, where a shuffle is a trip to
-// LDS), the four rows by shuffles.
-__device__ __forceinline__ float wave_total(float x)
-{
-    auto add = [&](auto ctrl) {
-        const int moved = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, true);
-        x += __builtin_bit_cast(float, moved);
-    };
-    add(std::integral_constant<int, 0xB1>{});    // quad_perm [1,0,3,2]
-    add(std::integral_constant<int, 0x4E>{});    // quad_perm [2,3,0,1]
-    add(std::integral_constant<int, 0x141>{});   // row_half_mirror
-    add(std::integral_constant<int, 0x140>{});   // row_mirror
-    x += __shfl_xor(x, 16);
-    x += __shfl_xor(x, 32);
-    return x;
-}
-
-// A weight fragment as it waits in registers: KP consecutive k of one row, stored bits.
-template <typename T, bool WBF> struct RawFrag {
-    static constexpr int WORDS = TT<T>::KP * (WBF ? 2 : 4) / 8;   // 8-byte words
-    uint64_t w[WORDS];
-};
-template <typename T, bool WBF> __device__ __forceinline__ RawFrag<T, WBF> weight_raw(const void *w, int64_t at)
-{
-    RawFrag<T, WBF> r;
-    const char *p = static_cast<const char *>(w) + at * (WBF ? 2 : 4);
-#pragma unroll
-    for (int i = 0; i < RawFrag<T, WBF>::WORDS; ++i) r.w[i] = reinterpret_cast<const uint64_t *>(p)[i];
-    return r;
-}
-template <typename T, bool WBF> __device__ __forceinline__ typename TT<T>::frag weight_frag(const RawFrag<T, WBF> &r)
-{
-    typename TT<T>::frag f;
-    if constexpr (std::is_same<T, __bf16>::value && WBF) {
-        f = __builtin_bit_cast(bf16x8, r);
-    } else if constexpr (std::is_same<T, __bf16>::value) {
-        struct F8 {
-            float v[8];
-        };
-        const F8 x = __builtin_bit_cast(F8, r);
-        const bf16x4 lo = TT<__bf16>::pack(x.v[0], x.v[1], x.v[2], x.v[3]), hi = TT<__bf16>::pack(x.v[4], x.v[5], x.v[6], x.v[7]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) f[e] = lo[e], f[4 + e] = hi[e];
-    } else if constexpr (WBF) {
-        const bf16x4 x = __builtin_bit_cast(bf16x4, r);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) f[e] = (float)x[e];
-    } else {
-        f = __builtin_bit_cast(f32x4, r);
-    }
-    return f;
-}
-
-// T: the products' type; MT: rows per workgroup (16 or 32); NV: 256-feature groups a lane holds of a row (K <= 256 NV);
-// CT: 16-column tiles per wave.
-template <typename T, bool WBF, int MT, int NV, int CT>
+// T: the products' type; WBF, XBF: bfloat16 weights, rows; MT: rows per workgroup (16 or 32); NV: 256-feature groups a lane holds of a row
+// (K <= 256 NV); CT: 16-column tiles per wave; EXTRA: weights in two arrays, the feed-through term.
+template <typename T, bool WBF, bool XBF, int MT, int NV, int CT, bool EXTRA>
 __global__ void __launch_bounds__(RD_THREADS) row_dense_kernel(RowDenseArgs a)
 {
     using F = typename TT<T>::frag;
@@ -119,98 +44,64 @@ __global__ void __launch_bounds__(RD_THREADS) row_dense_kernel(RowDenseArgs a)
     constexpr int AHEAD = 8 / CT;   // k steps whose weight fragments are requested at once
     extern __shared__ __align__(16) unsigned char smem[];
     T *sx = reinterpret_cast<T *>(smem);
-    const int kpad = (a.K + KB - 1) / KB * KB, ld = kpad + pad_of<T>(), steps = kpad / KB;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, i16 = lane & 15, g = lane >> 4;
+    const int K = a.in.K, kpad = (K + KB - 1) / KB * KB, ld = kpad + pad_of<T>(), steps = kpad / KB;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), i16 = lane & 15, g = lane >> 4;
     const int tiles = a.first_tile[a.layers];
     const int tile = (int)(blockIdx.x % (unsigned)tiles);
-    const int64_t r0 = (int64_t)(blockIdx.x / (unsigned)tiles) * MT;
+    const int64_t r0 = (int64_t)(blockIdx.x / (unsigned)tiles) * MT, rows = a.in.rows;
     int l = 0;
-    while (tile >= a.first_tile[l + 1]) ++l;
+#pragma unroll
+    for (int j = 1; j < MRX_ROW_DENSE_LAYERS; ++j) l += j < a.layers && tile >= a.first_tile[j];
     const int n0 = ((tile - a.first_tile[l]) * RD_WAVES + wv) * 16 * CT, N = a.n[l];
-    const void *w = a.w[l];
+    const void *w = a.w[l], *b = a.b[l], *out = a.y[l];
 
+    RowPanel<XBF, RPW, NV> panel;
+    panel.load(a.in, r0 + wv * RPW, lane);
     RawFrag<T, WBF> next[AHEAD][CT];
     auto fetch = [&](int s0) {
 #pragma unroll
         for (int s = 0; s < AHEAD; ++s)
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct) {
-                const int k = (s0 + s) * KB + KP * g, row = n0 + ct * 16 + i16;   // K is a multiple of KP
-                if (row < N && k < a.K) {
-                    const bool second = a.w2 && k >= a.k1;
-                    const int wide = a.w2 ? (second ? a.K - a.k1 : a.k1) : a.K;
-                    next[s][ct] = weight_raw<T, WBF>(second ? a.w2 : w, (int64_t)row * wide + (second ? k - a.k1 : k));
-                }
-                else next[s][ct] = RawFrag<T, WBF>{};
+                const int k = weight_k<T>((s0 + s) * KB + KP * g, K), c = n0 + ct * 16 + i16, row = c < N ? c : N - 1;
+                const bool second = EXTRA && a.w2 && k >= a.k1;
+                const int wide = EXTRA && a.w2 ? (second ? K - a.k1 : a.k1) : K;
+                next[s][ct] = weight_raw<T, WBF>(second ? a.w2 : w, (int64_t)row * wide + (second ? k - a.k1 : k));
             }
     };
     fetch(0);
-
-    {   // rows -> norm -> LDS; a wave takes RPW rows, all of them requested before the first is used
-        Quad xv[RPW][NV];
+    panel.load_norm(a.in, lane);
+    // lane (i16, g) ends up with columns c0 .. c0 + 3 of row i16 of each row tile: one load or store where rows are whole quads
+    const bool quads = N % 4 == 0;
+    uint32_t bias_raw[CT][4];
+    f32x4 res[RT][CT];
 #pragma unroll
-        for (int j = 0; j < RPW; ++j)
+    for (int ct = 0; ct < CT; ++ct) {
+        const int c0 = n0 + ct * 16 + 4 * g;
 #pragma unroll
-            for (int i = 0; i < NV; ++i) {
-                const int c = (i * 64 + lane) * 4;
-                const int64_t r = r0 + wv * RPW + j;
-                if (r < a.rows && c < a.K) xv[j][i] = a.x_bf16 ? quad_of<true>(a.x, r * a.K + c) : quad_of<false>(a.x, r * a.K + c);
-                else xv[j][i] = Quad{{0.f, 0.f, 0.f, 0.f}};
+        for (int e = 0; e < 4; ++e) bias_raw[ct][e] = 0u;
+        if (b) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int c = c0 + e < N ? c0 + e : N - 1;
+                if (a.b_bf16) bias_raw[ct][e] = static_cast<const uint16_t *>(b)[c];
+                else bias_raw[ct][e] = static_cast<const uint32_t *>(b)[c];
             }
-        Quad sc[NV], nb[NV];
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            const int c = (i * 64 + lane) * 4;
-            const bool in = a.norm && c < a.K;
-            sc[i] = in && a.scale ? quad_of<false>(a.scale, c) : Quad{{1.f, 1.f, 1.f, 1.f}};
-            nb[i] = in && a.nbias ? quad_of<false>(a.nbias, c) : Quad{{0.f, 0.f, 0.f, 0.f}};
         }
 #pragma unroll
-        for (int j = 0; j < RPW; ++j) {
-            float rstd = 1.f;
-            if (a.norm) {
-                if (a.norm == 2) {
-                    float s = 0.f;
-#pragma unroll
-                    for (int i = 0; i < NV; ++i)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) s += xv[j][i].v[e];
-                    const float mu = wave_total(s) * a.inv_K;
-#pragma unroll
-                    for (int i = 0; i < NV; ++i)
-                        if ((i * 64 + lane) * 4 < a.K)
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) xv[j][i].v[e] -= mu;
-                }
-                float ss = 0.f;
-#pragma unroll
-                for (int i = 0; i < NV; ++i)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) ss += xv[j][i].v[e] * xv[j][i].v[e];
-                rstd = rsqrtf(wave_total(ss) * a.inv_K + a.eps);
-            }
-#pragma unroll
-            for (int i = 0; i < NV; ++i) {
-                const int c = (i * 64 + lane) * 4;
-                if (c >= kpad) continue;   // columns K .. kpad hold zeros
-                Quad o = xv[j][i];
-                if (a.norm && c < a.K)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        o.v[e] = o.v[e] * rstd * sc[i].v[e] + nb[i].v[e];
-                        if (a.round_norm) o.v[e] = (float)(__bf16)o.v[e];
-                    }
-                if (a.skip_out && tile == 0 && r0 + wv * RPW + j < a.rows && c < a.K) {
-                    const int64_t at = (r0 + wv * RPW + j) * a.K + c;
-                    const Quad x = a.x_bf16 ? quad_of<true>(a.x, at) : quad_of<false>(a.x, at), d = quad_of<false>(a.skip, c);
-                    *reinterpret_cast<f32x4 *>(a.skip_out + at) =
-                        f32x4{x.v[0] + d.v[0] * o.v[0], x.v[1] + d.v[1] * o.v[1], x.v[2] + d.v[2] * o.v[2], x.v[3] + d.v[3] * o.v[3]};
-                }
-                *reinterpret_cast<typename TT<T>::pack4 *>(sx + (wv * RPW + j) * ld + c) = TT<T>::pack(o.v[0], o.v[1], o.v[2], o.v[3]);
-            }
+        for (int rt = 0; rt < RT; ++rt) {
+            res[rt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+            const int64_t r = r0 + rt * 16 + i16 < rows ? r0 + rt * 16 + i16 : rows - 1;
+            if (a.residual && quads) res[rt][ct] = *reinterpret_cast<const f32x4 *>(a.residual + r * N + (c0 < N ? c0 : 0));
         }
     }
-    __syncthreads();
+
+    panel.template finish<T>(a.in, sx + wv * RPW * ld, ld, kpad, lane, [&](int j, int i, int c, const f32x4 &y) {
+        const int64_t r = r0 + wv * RPW + j;
+        if (EXTRA && a.skip_out && tile == 0 && r < rows && c < K)
+            *reinterpret_cast<f32x4 *>(a.skip_out + r * K + c) = panel.floats(panel.x[j][i]) + *reinterpret_cast<const f32x4 *>(a.skip + c) * y;
+    });
+    sync_lds();   // (the weights may still be on their way)
 
     f32x4 acc[RT][CT];
 #pragma unroll
@@ -229,7 +120,10 @@ __global__ void __launch_bounds__(RD_THREADS) row_dense_kernel(RowDenseArgs a)
             if (s0 + s >= steps) break;
             F wf[CT];
 #pragma unroll
-            for (int ct = 0; ct < CT; ++ct) wf[ct] = weight_frag<T, WBF>(cur[s][ct]);
+            for (int ct = 0; ct < CT; ++ct) {
+                wf[ct] = weight_frag<T, WBF>(cur[s][ct]);
+                if (kpad != K && (s0 + s) * KB + KP * g >= K) wf[ct] = F{};
+            }
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt) {
                 const F xf = TT<T>::template load<ROWK>(sx, ld, rt * 16, (s0 + s) * KB, lane);
@@ -239,33 +133,30 @@ __global__ void __launch_bounds__(RD_THREADS) row_dense_kernel(RowDenseArgs a)
         }
     }
 
-    // lane (i16, g) holds columns c0 .. c0 + 3 of row i16 of each row tile: one store where rows are whole quads
-    const bool quads = N % 4 == 0;
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
         const int c0 = n0 + ct * 16 + 4 * g;
         if (c0 >= N) continue;
-        float bias[4] = {0.f, 0.f, 0.f, 0.f};
+        float bias[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (a.b[l] && c0 + e < N) {
-                bias[e] = a.b_bf16 ? (float)static_cast<const __bf16 *>(a.b[l])[c0 + e] : static_cast<const float *>(a.b[l])[c0 + e];
-                if (std::is_same<T, __bf16>::value) bias[e] = (float)(__bf16)bias[e];
-            }
+        for (int e = 0; e < 4; ++e) {
+            bias[e] = a.b_bf16 ? raw_to_float<__bf16>(bias_raw[ct][e]) : raw_to_float<float>(bias_raw[ct][e]);
+            if (std::is_same<T, __bf16>::value) bias[e] = (float)(__bf16)bias[e];
+        }
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
             const int64_t r = r0 + rt * 16 + i16, at = r * N + c0;
-            if (r >= a.rows) continue;
+            if (r >= rows) continue;
             f32x4 y;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 y[e] = acc[rt][ct][e] + bias[e];
                 if (std::is_same<T, __bf16>::value) y[e] = (float)(__bf16)y[e];
             }
-            float *yf = static_cast<float *>(a.y[l]) + at;
-            __bf16 *yb = static_cast<__bf16 *>(a.y[l]) + at;
+            float *yf = static_cast<float *>(const_cast<void *>(out)) + at;
+            __bf16 *yb = static_cast<__bf16 *>(const_cast<void *>(out)) + at;
             if (quads) {
-                if (a.residual) y += *reinterpret_cast<const f32x4 *>(a.residual + at);
+                y += res[rt][ct];
                 if (a.y_bf16) *reinterpret_cast<bf16x4 *>(yb) = TT<__bf16>::pack(y[0], y[1], y[2], y[3]);
                 else *reinterpret_cast<f32x4 *>(yf) = y;
                 continue;
@@ -281,20 +172,32 @@ __global__ void __launch_bounds__(RD_THREADS) row_dense_kernel(RowDenseArgs a)
     }
 }
 
-template <typename T, bool WBF, int MT, int CT> int launch_rows(hipStream_t st, RowDenseArgs &a)
+// A kernel that needs more than the default 64 KB of dynamic LDS (float32 rows of more than 500 features at 32 rows, 1 000 at 16)
+// announces it.
+template <typename T, bool WBF, bool XBF, int MT, int NV, int CT, bool EXTRA> struct RowKernel {
+    static constexpr auto fn = row_dense_kernel<T, WBF, XBF, MT, NV, CT, EXTRA>;
+    static constexpr int most_lds = MT * (256 * NV + pad_of<T>()) * (int)sizeof(T);
+    static inline const KernelRegistrar registrar{reinterpret_cast<const void *>(fn), most_lds};
+    static auto get()
+    {
+        if constexpr (most_lds > 64 * 1024) (void)&registrar;
+        return fn;
+    }
+};
+template <typename T, bool WBF, bool XBF, int MT, int CT, bool EXTRA = false> int launch_rows(hipStream_t st, RowDenseArgs &a)
 {
     constexpr int KB = TT<T>::KB, COLS = 16 * CT * RD_WAVES;
     for (int l = 0; l < a.layers; ++l) a.first_tile[l + 1] = a.first_tile[l] + (a.n[l] + COLS - 1) / COLS;
-    const size_t lds = (size_t)MT * ((a.K + KB - 1) / KB * KB + pad_of<T>()) * sizeof(T);
-    const int64_t grid = (a.rows + MT - 1) / MT * a.first_tile[a.layers];
+    const size_t lds = (size_t)MT * ((a.in.K + KB - 1) / KB * KB + pad_of<T>()) * sizeof(T);
+    const int64_t grid = (a.in.rows + MT - 1) / MT * a.first_tile[a.layers];
     if (grid >= (1ll << 31)) return MRX_ERR_INVALID_ARG;
     auto go = [&](auto nv) {
-        return launch_kernel(row_dense_kernel<T, WBF, MT, decltype(nv)::value, CT>, dim3((unsigned)grid), dim3(RD_THREADS), lds, st, a);
+        return launch_kernel(RowKernel<T, WBF, XBF, MT, decltype(nv)::value, CT, EXTRA>::get(), dim3((unsigned)grid), dim3(RD_THREADS), lds, st, a);
     };
-    if (a.K <= 256) return go(std::integral_constant<int, 1>{});
+    if (a.in.K <= 256) return go(std::integral_constant<int, 1>{});
     if constexpr (MT == 16) {
-        if (a.K > 1024) return go(std::integral_constant<int, 8>{});
-        if (a.K > 512) return go(std::integral_constant<int, 4>{});
+        if (a.in.K > 1024) return go(std::integral_constant<int, 8>{});
+        if (a.in.K > 512) return go(std::integral_constant<int, 4>{});
     }
     return go(std::integral_constant<int, 2>{});
 }
@@ -304,32 +207,21 @@ template <typename T, bool WBF, int MT, int CT> int launch_rows(hipStream_t st, 
 // 32 x 128, of 2 048 12.0 / 10.9 / 9.6, of 4 096 19.4 / 17.4 / 14.2; a single 256-column layer 5.3 / 7.3 / 9.0 at 1 024 rows,
 // 6.3 / 7.5 / 9.3 at 2 048, 9.2 / 8.8 / 9.4 at 4 096.  (The library's products alone, without the norm: 14.8, 15.8, 19.7 for the
 // first three.)  Wide rows stay at 16: their registers and LDS would not fit otherwise.
-template <typename T, bool WBF> int by_shape(hipStream_t st, RowDenseArgs &a)
+template <typename T, bool WBF, bool XBF> int by_shape(hipStream_t st, RowDenseArgs &a)
 {
+    if (a.w2 || a.skip_out) return launch_rows<T, WBF, XBF, 16, 1, true>(st, a);
     int64_t small = 0;
     for (int l = 0; l < a.layers; ++l) small += (a.n[l] + 63) / 64;
-    small *= (a.rows + 15) / 16;
-    if (small <= 512 || a.K > 512) return launch_rows<T, WBF, 16, 1>(st, a);
-    if (small <= 1024) return launch_rows<T, WBF, 32, 1>(st, a);
-    return launch_rows<T, WBF, 32, 2>(st, a);
+    small *= (a.in.rows + 15) / 16;
+    if (small <= 512 || a.in.K > 512) return launch_rows<T, WBF, XBF, 16, 1>(st, a);
+    if (small <= 1024) return launch_rows<T, WBF, XBF, 32, 1>(st, a);
+    return launch_rows<T, WBF, XBF, 32, 2>(st, a);
 }
-
-// Dynamic LDS beyond the default limit of 64 KB: float32 rows of more than 500 (32 rows) or 1 000 features (16 rows).
-constexpr int RD_MAX_LDS = 16 * (RD_MAX_K + 4) * 4;
-const KernelRegistrar registrars[] = {
-    {reinterpret_cast<const void *>(row_dense_kernel<float, false, 16, 8, 1>), RD_MAX_LDS},
-    {reinterpret_cast<const void *>(row_dense_kernel<float, true, 16, 8, 1>), RD_MAX_LDS},
-    {reinterpret_cast<const void *>(row_dense_kernel<float, false, 16, 4, 1>), RD_MAX_LDS},
-    {reinterpret_cast<const void *>(row_dense_kernel<float, true, 16, 4, 1>), RD_MAX_LDS},
-    {reinterpret_cast<const void *>(row_dense_kernel<float, false, 32, 2, 1>), RD_MAX_LDS},
-    {reinterpret_cast<const void *>(row_dense_kernel<float, true, 32, 2, 1>), RD_MAX_LDS},
-    {reinterpret_cast<const void *>(row_dense_kernel<float, false, 32, 2, 2>), RD_MAX_LDS},
-    {reinterpret_cast<const void *>(row_dense_kernel<float, true, 32, 2, 2>), RD_MAX_LDS},
-    {reinterpret_cast<const void *>(row_dense_kernel<__bf16, false, 16, 8, 1>), RD_MAX_LDS},
-    {reinterpret_cast<const void *>(row_dense_kernel<__bf16, true, 16, 8, 1>), RD_MAX_LDS},
-    {reinterpret_cast<const void *>(row_dense_kernel<__bf16, false, 16, 4, 1>), RD_MAX_LDS},
-    {reinterpret_cast<const void *>(row_dense_kernel<__bf16, true, 16, 4, 1>), RD_MAX_LDS},
-};
+template <typename T> int by_type(hipStream_t st, RowDenseArgs &a)
+{
+    if (a.x_bf16) return a.w_bf16 ? by_shape<T, true, true>(st, a) : by_shape<T, false, true>(st, a);
+    return a.w_bf16 ? by_shape<T, true, false>(st, a) : by_shape<T, false, false>(st, a);
+}
 
 }  // namespace
 }  // namespace mrx
@@ -351,10 +243,9 @@ extern "C" int mrx_row_dense(void *stream, const void *x, const float *scale, co
     if ((skip == nullptr) != (skip_out == nullptr) || !aligned(skip, 16) || !aligned(skip_out, 16)) return MRX_ERR_INVALID_ARG;
     RowDenseArgs a{};
     a.w2 = weights2, a.k1 = (int)k1, a.skip = skip, a.skip_out = skip_out;
-    a.x = x, a.scale = scale, a.nbias = norm_bias, a.residual = residual;
-    a.layers = layers, a.K = (int)K, a.norm = norm, a.rows = rows, a.eps = eps, a.inv_K = 1.f / (float)K;
+    a.in = RowInput{x, scale, norm_bias, rows, (int)K, norm, eps, 1.f / (float)K, round_norm != 0};
+    a.residual = residual, a.layers = layers;
     a.x_bf16 = x_dtype == MRX_BF16, a.w_bf16 = w_dtype == MRX_BF16, a.b_bf16 = b_dtype == MRX_BF16, a.y_bf16 = y_dtype == MRX_BF16;
-    a.round_norm = round_norm != 0;
     if (!aligned(x, 16) || !aligned(scale, 16) || !aligned(norm_bias, 16) || !aligned(residual, 4)) return MRX_ERR_INVALID_ARG;
     for (int l = 0; l < layers; ++l) {
         if (!weights[l] || !outs[l] || !aligned(weights[l], 16) || !aligned(outs[l], 4)) return MRX_ERR_INVALID_ARG;
@@ -363,7 +254,5 @@ extern "C" int mrx_row_dense(void *stream, const void *x, const float *scale, co
     }
     if (const int rc = prepare_device(); rc != MRX_OK) return rc;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const bool bf = product_dtype == MRX_BF16;
-    if (bf) return a.w_bf16 ? by_shape<__bf16, true>(st, a) : by_shape<__bf16, false>(st, a);
-    return a.w_bf16 ? by_shape<float, true>(st, a) : by_shape<float, false>(st, a);
+    return product_dtype == MRX_BF16 ? by_type<__bf16>(st, a) : by_type<float>(st, a);
 }
