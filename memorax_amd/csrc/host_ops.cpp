@@ -51,6 +51,7 @@ using torch::autograd::variable_list;
     X(mrx_gated_linear_attn_step) X(mrx_delta_rule_step) X(mrx_causal_conv_silu_fwd) X(mrx_causal_conv_silu_bwd)     \
     X(mrx_mamba_elements_fwd) X(mrx_mamba_elements_bwd) X(mrx_decay_last) X(mrx_mamba_readout_fwd)                   \
     X(mrx_mamba_readout_bwd) X(mrx_deltanet_step) X(mrx_mingru_step) X(mrx_row_dense) X(mrx_dense_grads) X(mrx_dense_grads_workspace)                  \
+    X(mrx_gated_recurrence_act) X(mrx_state_act)                                                                      \
     X(mrx_dense_rows_suit) X(mrx_dense_pack) X(mrx_dense_rows) X(mrx_dense_rows_input_grad)                          \
     X(mrx_lru_step) X(mrx_mlstm_step) X(mrx_linear_attn_norm_fwd_chunk_parallel) X(mrx_linear_attn_norm_bwd_chunk_parallel) \
     X(mrx_gated_linear_attn_fwd_chunk_parallel) X(mrx_gated_linear_attn_bwd_chunk_parallel)
@@ -934,6 +935,80 @@ std::tuple<Tensor, Tensor, Tensor> mingru_step(const Tensor &z, const Tensor &x,
                               code(dt), done.dtype),
           "mrx_mingru_step");
     return {y, ls, ld};
+}
+
+// The acting steps of whole recurrences (act_blocks.hip): x (B,1,K) float32 through norm, bias-free layers and the recurrence's step.  An
+// undefined result says that the sizes are not theirs: the launches they stand for take them.
+struct ActInput {
+    Tensor x, scale, nbias;
+    std::vector<Tensor> w;
+    int64_t B, K;
+    bool ok;
+    ActInput(const Tensor &x_, const OptTensor &scale_, const OptTensor &nbias_, const std::vector<Tensor> &weights, ScalarType product, int64_t most)
+    {
+        x = dense16(x_), scale = norm_param(scale_), nbias = norm_param(nbias_), B = x.size(0), K = x.size(2);
+        const auto wd = weights[0].scalar_type();
+        ok = K % 8 == 0 && K <= most && (product == at::kBFloat16 || (product == at::kFloat && wd == at::kFloat)) && (wd == at::kFloat || wd == at::kBFloat16);
+        chk(x, "x", at::kFloat);
+        if (scale.defined()) chk(scale, "scale", at::kFloat, {K});
+        if (nbias.defined()) chk(nbias, "bias of the norm", at::kFloat, {K});
+        for (const Tensor &t : weights) {
+            w.push_back(dense16(t));
+            TORCH_CHECK_VALUE(t.dim() == 2 && t.size(1) == K, "a weight must be (n, ", K, "), got ", t.sizes());
+            chk(w.back(), "weight", wd);
+        }
+    }
+};
+
+// weights of z, h~ and gate, the carry's leaves (B,1,N) -> z, y, log_state, log_decay
+std::vector<Tensor> gated_recurrence_act(const Tensor &x, int norm, const OptTensor &scale, const OptTensor &nbias, double eps,
+                                         const std::vector<Tensor> &weights, ScalarType product, const Tensor &done_, const Tensor &log_state,
+                                         const Tensor &log_decay, bool in_place)
+{
+    TORCH_CHECK_VALUE(x.dim() == 3 && x.size(1) == 1 && weights.size() == 3, "gated_recurrence_act takes one time step");
+    refuse(x, scale, nbias, weights, done_, log_state, log_decay);
+    const ActInput in(x, scale, nbias, weights, product, 512);
+    const int64_t N = weights[0].size(0);
+    for (const Tensor &w : in.w) chk(w, "weight", w.scalar_type(), {N, in.K});
+    auto place = [](const Tensor &t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+    chk(log_state, "log_state", at::kFloat, {in.B, 1, N});
+    chk(log_decay, "log_decay", at::kFloat, {in.B, 1, N});
+    if (!in.ok || N % 4 != 0 || N == 0 || in.B == 0 || !place(log_state) || !place(log_decay)) return {};
+    const Done done(done_, in.B, 1);
+    const Tensor z = fresh({in.B, 1, N}, product, x), y = fresh({in.B, 1, N}, product, x), ls = in_place ? log_state : fresh_like(log_state),
+                 ld = in_place ? log_decay : fresh_like(log_decay);
+    check(lib.mrx_gated_recurrence_act(stream(), fptr(in.x), fptr(in.scale), fptr(in.nbias), norm, ptr(in.w[0]), ptr(in.w[1]), ptr(in.w[2]), done.p(),
+                                       fptr(log_state), fptr(log_decay), ptr(z), ptr(y), fptr(ls), fptr(ld), in.B, in.K, N, code(in.w[0].scalar_type()),
+                                       code(product), done.dtype, (float)eps),
+          "mrx_gated_recurrence_act");
+    return {z, y, ls, ld};
+}
+
+// weights of q, k, v (H D, K) and, for the delta rule, beta (H, K); S (B,1,H,D,D), for linear attention z (B,1,H,D) -> o (B,1,H D), S, z
+std::vector<Tensor> state_act(const Tensor &x, int norm, const OptTensor &scale, const OptTensor &nbias, double eps, const std::vector<Tensor> &weights,
+                              ScalarType product, ScalarType o_dtype, const Tensor &done_, const Tensor &S, const OptTensor &z, double den_eps, bool in_place)
+{
+    TORCH_CHECK_VALUE(x.dim() == 3 && x.size(1) == 1 && weights.size() == (z.has_value() ? 3u : 4u) && S.dim() == 5, "state_act takes one time step");
+    refuse(x, scale, nbias, weights, done_, S, z);
+    const ActInput in(x, scale, nbias, weights, product, 256);
+    const int64_t H = S.size(2), D = S.size(3);
+    if (S.scalar_type() != at::kFloat || (z.has_value() && z->scalar_type() != at::kFloat)) return {};
+    const Tensor S_ = dense16(S), z_ = z.has_value() ? dense16(*z) : Tensor();
+    chk(S_, "S", at::kFloat, {in.B, 1, H, D, D});
+    if (z_.defined()) chk(z_, "z", at::kFloat, {in.B, 1, H, D});
+    for (int i = 0; i < 3; ++i) chk(in.w[i], "weight", in.w[i].scalar_type(), {H * D, in.K});
+    if (!z.has_value()) chk(in.w[3], "weight of beta", in.w[3].scalar_type(), {H, in.K});
+    if (!in.ok || (D != 16 && D != 32 && D != 64) || in.B * H == 0 || in.B * H >= (1ll << 29)) return {};
+    const Done done(done_, in.B, 1);
+    const Tensor o = fresh({in.B, 1, H * D}, o_dtype, x), So = in_place && S_.is_same(S) ? S : fresh(S.sizes(), at::kFloat, x),
+                 zo = z_.defined() ? (in_place && z_.is_same(*z) && S_.is_same(S) ? *z : fresh(z->sizes(), at::kFloat, x)) : Tensor();
+    check(lib.mrx_state_act(stream(), fptr(in.x), fptr(in.scale), fptr(in.nbias), norm, ptr(in.w[0]), ptr(in.w[1]), ptr(in.w[2]),
+                            z.has_value() ? nullptr : ptr(in.w[3]), done.p(), fptr(S_), fptr(z_), ptr(o), fptr(So), fptr(zo), in.B, in.K, H, D,
+                            code(in.w[0].scalar_type()), code(product), code(o_dtype), done.dtype, (float)eps, (float)den_eps),
+          "mrx_state_act");
+    std::vector<Tensor> out{o, So};
+    if (zo.defined()) out.push_back(zo);
+    return out;
 }
 
 // ------------------------------------------------------------------------------------------------ autograd nodes
@@ -2263,6 +2338,8 @@ PYBIND11_MODULE(_native, m)
     def("lru_act", &lru_act);
     def("mlstm_act", &mlstm_act);
     def("mingru_step", &mingru_step);
+    def("gated_recurrence_act", &gated_recurrence_act);
+    def("state_act", &state_act);
     // differentiable operators (memorax_amd/functional.py)
     def("linear_scan", &linear_scan);
     def("mingru_scan", &mingru_scan);

@@ -470,6 +470,12 @@ class GatedLinearRecurrence(SequenceModel):
         if carry is None:
             carry = self.cell.initialize_carry(None, get_input_shape(x))
         product = autocast_dtype(x) or x.dtype
+        if all(m.bias is None for m in layers):
+            acted = native().gated_recurrence_act(x, *_norm_of(norm), [m.weight for m in layers], product, done, *carry, stepping_in_place())
+            if acted:   # (sizes that it takes)
+                z, y, *carry = acted
+                self.cell.intermediates.sow("gate", lambda z=z: z.float().mean())
+                return tuple(carry), _rows(y, None, [self.out], product, x.dtype, x)[0]
         z, h_tilde, gate = _rows(x, norm, layers, product, product)
         self.cell.intermediates.sow("gate", lambda z=z: z.float().mean())
         y, *carry = native().mingru_step(z, h_tilde, gate, done, *carry, stepping_in_place())
@@ -622,6 +628,12 @@ class LinearAttentionCell(MemoroidCellBase):
         if not (type(self.norm) is _RMSNorm and _as_written(self, LinearAttentionCell) and _row_layers(x, [*layers, self.output_projection])):
             return None
         product = autocast_dtype(x) or x.dtype
+        if all(m.bias is None for m in layers):
+            acted = native().state_act(x, *_norm_of(norm), [m.weight for m in (self.query, self.key, self.value)], product, product, done, *carry, self.eps,
+                                       stepping_in_place())
+            if acted:   # (sizes that it takes)
+                o, *carry = acted
+                return tuple(carry), _rows(o, self.norm, [self.output_projection], product, x.dtype, x)[0]
         z = tuple(self._heads(t) for t in _rows(x, norm, layers, product, product))
         h, carry = self.scan(z, carry, done)
         return carry, _rows(h.reshape(*x.shape[:2], -1), self.norm, [self.output_projection], product, x.dtype, x)[0]
@@ -696,6 +708,11 @@ class DeltaNetCell(MemoroidCellBase):
                 and _row_layers(x, [*layers, self.output_projection])):
             return None
         product = autocast_dtype(x) or x.dtype
+        if all(m.bias is None for m in layers):
+            acted = native().state_act(x, *_norm_of(norm), [m.weight for m in layers], product, self.dtype, done, carry[0], None, 0.0, stepping_in_place())
+            if acted:   # (sizes that it takes)
+                o, S = acted
+                return (S,), _rows(o, self.norm, [self.output_projection], product, x.dtype, x)[0]
         q, k, v, beta = _rows(x, norm, layers, product, self.dtype)
         h, carry = self.scan((self._heads(q), self._heads(k), self._heads(v), beta), carry, done)
         return carry, _rows(h.reshape(*x.shape[:2], -1), self.norm, [self.output_projection], product, x.dtype, x)[0]
