@@ -643,22 +643,15 @@ int mrx_dense_grads(void *stream, const void *x, const void *const *dys, const v
                     int layers, void *dx, float *params, float *workspace, int64_t rows, int64_t K, int dtype, int dx_dtype,
                     unsigned bias_mask);
 
-/* ---- Acting steps of whole recurrences: a pre-norm block's step up to what its closing layer reads ----
- * x (rows, K) float32, normalised as mrx_row_dense does (norm 0, 1, 2; K a multiple of 8); weights without biases in w_dtype; products in
- * product_dtype (float32 products: float32 weights), each result rounded to it.  done (rows).  Arrays on 16-byte boundaries.
- * mrx_gated_recurrence_act: z, h~ and gate (N features, a multiple of 4; K up to 512), then mrx_mingru_step on them; z and y (rows, N)
- *   in product_dtype, the carry (rows, N) float32 and possibly updated in place.
- * mrx_state_act: q, k, v (H heads of D = 16, 32 or 64; K up to 256) and, unless w_beta is NULL, beta (H), each rounded to o_dtype too; then
- *   with beta mrx_deltanet_step, without it mrx_linear_attn_step with the elu + 1 map and the normaliser z (rows, H, D).  o (rows, H D) in
- *   o_dtype; S (rows, H, D, D) and z float32 and possibly updated in place. */
+/* ---- The acting step of a gated recurrence up to what its closing layer reads ----
+ * x (rows, K) float32, normalised as mrx_row_dense does (norm 0, 1, 2; K a multiple of 8 up to 512); weights (N, K) without biases in w_dtype;
+ * products in product_dtype (float32 products: float32 weights), each result rounded to it; then mrx_mingru_step on z, h~ and the gate (N
+ * a multiple of 4).  z and y (rows, N) in product_dtype; the carry (rows, N) float32 and possibly updated in place; done (rows).  Arrays
+ * on 16-byte boundaries. */
 int mrx_gated_recurrence_act(void *stream, const float *x, const float *scale, const float *norm_bias, int norm, const void *w_z,
                              const void *w_h, const void *w_gate, const void *done, const float *log_state, const float *log_decay,
                              void *z, void *y, float *log_state_out, float *log_decay_out, int64_t rows, int64_t K, int64_t N, int w_dtype,
                              int product_dtype, int done_dtype, float eps);
-int mrx_state_act(void *stream, const float *x, const float *scale, const float *norm_bias, int norm, const void *w_q, const void *w_k,
-                  const void *w_v, const void *w_beta, const void *done, const float *S_in, const float *z_in, void *o, float *S_out,
-                  float *z_out, int64_t rows, int64_t K, int64_t H, int64_t D, int w_dtype, int product_dtype, int o_dtype, int done_dtype,
-                  float eps, float den_eps);
 
 /* ---- Dense layers over many rows in bfloat16, their weights held in registers ----
  * Up to three layers of n outputs (64 or more) and one of at most eight, on the same rows (rows, K).

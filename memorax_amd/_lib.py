@@ -65,7 +65,6 @@ SIGNATURES = {
     "mrx_mingru_step": (_I, [_P] * 10 + [_L] * 2 + [_I] * 2),
     "mrx_row_dense": (_I, [_P] * 4 + [_I] * 2 + [_P] * 4 + [_I, _P] + [_L] * 2 + [_I] * 5 + [ctypes.c_float, _P, _L, _P, _P]),
     "mrx_gated_recurrence_act": (_I, [_P] * 4 + [_I] + [_P] * 10 + [_L] * 3 + [_I] * 3 + [ctypes.c_float]),
-    "mrx_state_act": (_I, [_P] * 4 + [_I] + [_P] * 10 + [_L] * 4 + [_I] * 4 + [ctypes.c_float] * 2),
     "mrx_lru_step": (_I, [_P] * 12 + [_L] * 2 + [_I]),
     "mrx_mlstm_step": (_I, [_P] * 23 + [_L] * 4 + [_I, ctypes.c_float]),
     "mrx_dense_grads_workspace": (_L, [_L] * 2 + [_P] + [_I] * 2 + [ctypes.c_uint]),

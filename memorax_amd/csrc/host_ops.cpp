@@ -51,7 +51,7 @@ using torch::autograd::variable_list;
     X(mrx_gated_linear_attn_step) X(mrx_delta_rule_step) X(mrx_causal_conv_silu_fwd) X(mrx_causal_conv_silu_bwd)     \
     X(mrx_mamba_elements_fwd) X(mrx_mamba_elements_bwd) X(mrx_decay_last) X(mrx_mamba_readout_fwd)                   \
     X(mrx_mamba_readout_bwd) X(mrx_deltanet_step) X(mrx_mingru_step) X(mrx_row_dense) X(mrx_dense_grads) X(mrx_dense_grads_workspace)                  \
-    X(mrx_gated_recurrence_act) X(mrx_state_act)                                                                      \
+    X(mrx_gated_recurrence_act)                                                                                       \
     X(mrx_dense_rows_suit) X(mrx_dense_pack) X(mrx_dense_rows) X(mrx_dense_rows_input_grad)                          \
     X(mrx_lru_step) X(mrx_mlstm_step) X(mrx_linear_attn_norm_fwd_chunk_parallel) X(mrx_linear_attn_norm_bwd_chunk_parallel) \
     X(mrx_gated_linear_attn_fwd_chunk_parallel) X(mrx_gated_linear_attn_bwd_chunk_parallel)
@@ -937,78 +937,70 @@ std::tuple<Tensor, Tensor, Tensor> mingru_step(const Tensor &z, const Tensor &x,
     return {y, ls, ld};
 }
 
-// The acting steps of whole recurrences (act_blocks.hip): x (B,1,K) float32 through norm, bias-free layers and the recurrence's step.  An
-// undefined result says that the sizes are not theirs: the launches they stand for take them.
-struct ActInput {
-    Tensor x, scale, nbias;
-    std::vector<Tensor> w;
-    int64_t B, K;
-    bool ok;
-    ActInput(const Tensor &x_, const OptTensor &scale_, const OptTensor &nbias_, const std::vector<Tensor> &weights, ScalarType product, int64_t most)
-    {
-        x = dense16(x_), scale = norm_param(scale_), nbias = norm_param(nbias_), B = x.size(0), K = x.size(2);
-        const auto wd = weights[0].scalar_type();
-        ok = K % 8 == 0 && K <= most && (product == at::kBFloat16 || (product == at::kFloat && wd == at::kFloat)) && (wd == at::kFloat || wd == at::kBFloat16);
-        chk(x, "x", at::kFloat);
-        if (scale.defined()) chk(scale, "scale", at::kFloat, {K});
-        if (nbias.defined()) chk(nbias, "bias of the norm", at::kFloat, {K});
-        for (const Tensor &t : weights) {
-            w.push_back(dense16(t));
-            TORCH_CHECK_VALUE(t.dim() == 2 && t.size(1) == K, "a weight must be (n, ", K, "), got ", t.sizes());
-            chk(w.back(), "weight", wd);
-        }
-    }
-};
-
-// weights of z, h~ and gate, the carry's leaves (B,1,N) -> z, y, log_state, log_decay
-std::vector<Tensor> gated_recurrence_act(const Tensor &x, int norm, const OptTensor &scale, const OptTensor &nbias, double eps,
-                                         const std::vector<Tensor> &weights, ScalarType product, const Tensor &done_, const Tensor &log_state,
-                                         const Tensor &log_decay, bool in_place)
+// Pre-norm residual blocks, one acting step each: x (B,1,K) float32 -> x + block(norm(x)) and what the cell carries on.  One call from Python
+// instead of one for each launch, with a dozen checks and views between them.
+// A gated recurrence: weights and biases of z, h~, gate and the closing layer, the carry's leaves (B,1,N) -> y, z, log_state, log_decay
+std::tuple<Tensor, Tensor, Tensor, Tensor> gated_act(const Tensor &x, int norm, const OptTensor &scale, const OptTensor &nbias, double eps,
+                                                     const std::vector<Tensor> &weights, const std::vector<OptTensor> &biases, ScalarType product,
+                                                     const Tensor &done_, const Tensor &log_state, const Tensor &log_decay, bool in_place)
 {
-    TORCH_CHECK_VALUE(x.dim() == 3 && x.size(1) == 1 && weights.size() == 3, "gated_recurrence_act takes one time step");
-    refuse(x, scale, nbias, weights, done_, log_state, log_decay);
-    const ActInput in(x, scale, nbias, weights, product, 512);
-    const int64_t N = weights[0].size(0);
-    for (const Tensor &w : in.w) chk(w, "weight", w.scalar_type(), {N, in.K});
-    auto place = [](const Tensor &t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
-    chk(log_state, "log_state", at::kFloat, {in.B, 1, N});
-    chk(log_decay, "log_decay", at::kFloat, {in.B, 1, N});
-    if (!in.ok || N % 4 != 0 || N == 0 || in.B == 0 || !place(log_state) || !place(log_decay)) return {};
-    const Done done(done_, in.B, 1);
-    const Tensor z = fresh({in.B, 1, N}, product, x), y = fresh({in.B, 1, N}, product, x), ls = in_place ? log_state : fresh_like(log_state),
-                 ld = in_place ? log_decay : fresh_like(log_decay);
-    check(lib.mrx_gated_recurrence_act(stream(), fptr(in.x), fptr(in.scale), fptr(in.nbias), norm, ptr(in.w[0]), ptr(in.w[1]), ptr(in.w[2]), done.p(),
-                                       fptr(log_state), fptr(log_decay), ptr(z), ptr(y), fptr(ls), fptr(ld), in.B, in.K, N, code(in.w[0].scalar_type()),
-                                       code(product), done.dtype, (float)eps),
-          "mrx_gated_recurrence_act");
-    return {z, y, ls, ld};
+    TORCH_CHECK_VALUE(x.dim() == 3 && x.size(1) == 1 && weights.size() == 4 && biases.size() == 4, "gated_act takes one time step");
+    refuse(x, scale, nbias, weights, biases, done_, log_state, log_decay);
+    const int64_t B = x.size(0), K = x.size(2), N = weights[0].size(0);
+    auto fits = [](const Tensor &t) { return t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+    const auto wd = weights[0].scalar_type();
+    bool whole = K % 8 == 0 && K <= 512 && N % 4 == 0 && B > 0 && fits(x) && fits(log_state) && fits(log_decay) &&
+                 (product == at::kBFloat16 ? wd == at::kFloat || wd == at::kBFloat16 : wd == at::kFloat);
+    for (int l = 0; l < 3; ++l)
+        whole = whole && !biases[l].has_value() && weights[l].scalar_type() == wd && fits(weights[l]) && weights[l].sizes() == IntArrayRef({N, K});
+    Tensor z, y, ls, ld;
+    if (whole) {
+        const Tensor sc = norm_param(scale), nb = norm_param(nbias);
+        chk(x, "x", at::kFloat);
+        if (sc.defined()) chk(sc, "scale", at::kFloat, {K});
+        if (nb.defined()) chk(nb, "bias of the norm", at::kFloat, {K});
+        chk(log_state, "log_state", at::kFloat, {B, 1, N});
+        chk(log_decay, "log_decay", at::kFloat, {B, 1, N});
+        const Done done(done_, B, 1);
+        z = fresh({B, 1, N}, product, x), y = fresh({B, 1, N}, product, x);
+        ls = in_place ? log_state : fresh_like(log_state), ld = in_place ? log_decay : fresh_like(log_decay);
+        check(lib.mrx_gated_recurrence_act(stream(), fptr(x), fptr(sc), fptr(nb), norm, ptr(weights[0]), ptr(weights[1]), ptr(weights[2]), done.p(),
+                                           fptr(log_state), fptr(log_decay), ptr(z), ptr(y), fptr(ls), fptr(ld), B, K, N, code(wd), code(product),
+                                           done.dtype, (float)eps),
+              "mrx_gated_recurrence_act");
+    } else {
+        auto u = row_dense(x, norm, scale, nbias, eps, false, {weights[0], weights[1], weights[2]}, {biases[0], biases[1], biases[2]}, product, product,
+                           std::nullopt);
+        z = u[0];
+        std::tie(y, ls, ld) = mingru_step(z, u[1], u[2], done_, log_state, log_decay, in_place);
+    }
+    return {row_dense(y, 0, std::nullopt, std::nullopt, 0.0, false, {weights[3]}, {biases[3]}, product, at::kFloat, x)[0], z, ls, ld};
 }
 
-// weights of q, k, v (H D, K) and, for the delta rule, beta (H, K); S (B,1,H,D,D), for linear attention z (B,1,H,D) -> o (B,1,H D), S, z
-std::vector<Tensor> state_act(const Tensor &x, int norm, const OptTensor &scale, const OptTensor &nbias, double eps, const std::vector<Tensor> &weights,
-                              ScalarType product, ScalarType o_dtype, const Tensor &done_, const Tensor &S, const OptTensor &z, double den_eps, bool in_place)
+// A matrix state: weights and biases of q, k, v (, beta: the delta rule with its prologue; without it linear attention with the elu + 1 map and
+// its normaliser z (B,1,H,D)) and of the closing layer, behind the RMS norm of the read-out; projections handed on in `dtype`;
+// S (B,1,H,D,D) -> y, S, z
+std::tuple<Tensor, Tensor, OptTensor> state_act(const Tensor &x, int norm, const OptTensor &scale, const OptTensor &nbias, double eps,
+                                                std::vector<Tensor> weights, std::vector<OptTensor> biases, const Tensor &out_scale, double out_eps,
+                                                ScalarType product, ScalarType dtype, const Tensor &done, const Tensor &S, const OptTensor &z, double den_eps,
+                                                bool in_place)
 {
-    TORCH_CHECK_VALUE(x.dim() == 3 && x.size(1) == 1 && weights.size() == (z.has_value() ? 3u : 4u) && S.dim() == 5, "state_act takes one time step");
-    refuse(x, scale, nbias, weights, done_, S, z);
-    const ActInput in(x, scale, nbias, weights, product, 256);
-    const int64_t H = S.size(2), D = S.size(3);
-    if (S.scalar_type() != at::kFloat || (z.has_value() && z->scalar_type() != at::kFloat)) return {};
-    const Tensor S_ = dense16(S), z_ = z.has_value() ? dense16(*z) : Tensor();
-    chk(S_, "S", at::kFloat, {in.B, 1, H, D, D});
-    if (z_.defined()) chk(z_, "z", at::kFloat, {in.B, 1, H, D});
-    for (int i = 0; i < 3; ++i) chk(in.w[i], "weight", in.w[i].scalar_type(), {H * D, in.K});
-    if (!z.has_value()) chk(in.w[3], "weight of beta", in.w[3].scalar_type(), {H, in.K});
-    if (!in.ok || (D != 16 && D != 32 && D != 64) || in.B * H == 0 || in.B * H >= (1ll << 29)) return {};
-    const Done done(done_, in.B, 1);
-    const Tensor o = fresh({in.B, 1, H * D}, o_dtype, x), So = in_place && S_.is_same(S) ? S : fresh(S.sizes(), at::kFloat, x),
-                 zo = z_.defined() ? (in_place && z_.is_same(*z) && S_.is_same(S) ? *z : fresh(z->sizes(), at::kFloat, x)) : Tensor();
-    check(lib.mrx_state_act(stream(), fptr(in.x), fptr(in.scale), fptr(in.nbias), norm, ptr(in.w[0]), ptr(in.w[1]), ptr(in.w[2]),
-                            z.has_value() ? nullptr : ptr(in.w[3]), done.p(), fptr(S_), fptr(z_), ptr(o), fptr(So), fptr(zo), in.B, in.K, H, D,
-                            code(in.w[0].scalar_type()), code(product), code(o_dtype), done.dtype, (float)eps, (float)den_eps),
-          "mrx_state_act");
-    std::vector<Tensor> out{o, So};
-    if (zo.defined()) out.push_back(zo);
-    return out;
+    TORCH_CHECK_VALUE(x.dim() == 3 && x.size(1) == 1 && weights.size() == (z.has_value() ? 4u : 5u) && biases.size() == weights.size() && S.dim() == 5,
+                      "state_act takes one time step");
+    refuse(x, scale, nbias, weights, biases, out_scale, done, S, z);
+    const int64_t B = x.size(0), H = S.size(2), D = S.size(3);
+    const Tensor out_w = weights.back();
+    const OptTensor out_b = biases.back();
+    weights.pop_back(), biases.pop_back();
+    auto u = row_dense(x, norm, scale, nbias, eps, false, weights, biases, product, dtype, std::nullopt);
+    for (int i = 0; i < 3; ++i) u[i] = u[i].view({B, H, D});
+    auto carried = [](const Tensor &t) { return t.select(1, 0).to(at::kFloat).contiguous(); };
+    const bool own = in_place && S.scalar_type() == at::kFloat && S.is_contiguous() && (!z.has_value() || (z->scalar_type() == at::kFloat && z->is_contiguous()));
+    const Tensor S_ = carried(S);
+    StepOut r = z.has_value() ? linear_attn_step(u[0], u[1], u[2], done, S_, carried(*z), MRX_FMAP_ELU1, true, den_eps, own)
+                              : delta_rule_step(u[0], u[1], u[2], u[3].view({B, H}), done, S_, own, true);
+    const Tensor y = row_dense(r.o.view({B, 1, H * D}), 1, out_scale, std::nullopt, out_eps, dtype == at::kBFloat16, {out_w}, {out_b}, product, at::kFloat, x)[0];
+    return {y, own ? S : r.S.unsqueeze(1), own ? z : z.has_value() ? OptTensor(r.z.unsqueeze(1)) : std::nullopt};
 }
 
 // ------------------------------------------------------------------------------------------------ autograd nodes
@@ -2338,7 +2330,7 @@ PYBIND11_MODULE(_native, m)
     def("lru_act", &lru_act);
     def("mlstm_act", &mlstm_act);
     def("mingru_step", &mingru_step);
-    def("gated_recurrence_act", &gated_recurrence_act);
+    def("gated_act", &gated_act);
     def("state_act", &state_act);
     // differentiable operators (memorax_amd/functional.py)
     def("linear_scan", &linear_scan);

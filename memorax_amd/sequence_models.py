@@ -470,16 +470,11 @@ class GatedLinearRecurrence(SequenceModel):
         if carry is None:
             carry = self.cell.initialize_carry(None, get_input_shape(x))
         product = autocast_dtype(x) or x.dtype
-        if all(m.bias is None for m in layers):
-            acted = native().gated_recurrence_act(x, *_norm_of(norm), [m.weight for m in layers], product, done, *carry, stepping_in_place())
-            if acted:   # (sizes that it takes)
-                z, y, *carry = acted
-                self.cell.intermediates.sow("gate", lambda z=z: z.float().mean())
-                return tuple(carry), _rows(y, None, [self.out], product, x.dtype, x)[0]
-        z, h_tilde, gate = _rows(x, norm, layers, product, product)
+        layers.append(self.out)
+        y, z, *carry = native().gated_act(x, *_norm_of(norm), [m.weight for m in layers], [m.bias for m in layers], product, done, *carry,
+                                          stepping_in_place())
         self.cell.intermediates.sow("gate", lambda z=z: z.float().mean())
-        y, *carry = native().mingru_step(z, h_tilde, gate, done, *carry, stepping_in_place())
-        return tuple(carry), _rows(y, None, [self.out], product, x.dtype, x)[0]
+        return tuple(carry), y
 
     def initialize_carry(self, key, input_shape):
         return self.cell.initialize_carry(key, input_shape)
@@ -513,6 +508,11 @@ def _hooked(module):
 def _plain(layer):
     """A layer that a product with its weight stands for."""
     return type(layer) in (Dense, nn.Linear)
+
+
+def _state_acts(head_dim, dtype):
+    """Whether the step kernels take heads of this width as they are."""
+    return head_dim <= 64 and head_dim % (16 // dtype.itemsize) == 0
 
 
 def _norm_of(norm):
@@ -628,12 +628,11 @@ class LinearAttentionCell(MemoroidCellBase):
         if not (type(self.norm) is _RMSNorm and _as_written(self, LinearAttentionCell) and _row_layers(x, [*layers, self.output_projection])):
             return None
         product = autocast_dtype(x) or x.dtype
-        if all(m.bias is None for m in layers):
-            acted = native().state_act(x, *_norm_of(norm), [m.weight for m in (self.query, self.key, self.value)], product, product, done, *carry, self.eps,
-                                       stepping_in_place())
-            if acted:   # (sizes that it takes)
-                o, *carry = acted
-                return tuple(carry), _rows(o, self.norm, [self.output_projection], product, x.dtype, x)[0]
+        if _state_acts(self.head_dim, product):
+            layers = [self.query, self.key, self.value, self.output_projection]
+            y, *carry = native().state_act(x, *_norm_of(norm), [m.weight for m in layers], [m.bias for m in layers], self.norm.scale, self.norm.eps,
+                                           product, product, done, *carry, self.eps, stepping_in_place())
+            return tuple(carry), y
         z = tuple(self._heads(t) for t in _rows(x, norm, layers, product, product))
         h, carry = self.scan(z, carry, done)
         return carry, _rows(h.reshape(*x.shape[:2], -1), self.norm, [self.output_projection], product, x.dtype, x)[0]
@@ -708,11 +707,11 @@ class DeltaNetCell(MemoroidCellBase):
                 and _row_layers(x, [*layers, self.output_projection])):
             return None
         product = autocast_dtype(x) or x.dtype
-        if all(m.bias is None for m in layers):
-            acted = native().state_act(x, *_norm_of(norm), [m.weight for m in layers], product, self.dtype, done, carry[0], None, 0.0, stepping_in_place())
-            if acted:   # (sizes that it takes)
-                o, S = acted
-                return (S,), _rows(o, self.norm, [self.output_projection], product, x.dtype, x)[0]
+        if _state_acts(self.head_dim, self.dtype):
+            layers.append(self.output_projection)
+            y, S, _ = native().state_act(x, *_norm_of(norm), [m.weight for m in layers], [m.bias for m in layers], self.norm.scale, self.norm.eps,
+                                         product, self.dtype, done, carry[0], None, 0.0, stepping_in_place())
+            return (S,), y
         q, k, v, beta = _rows(x, norm, layers, product, self.dtype)
         h, carry = self.scan((self._heads(q), self._heads(k), self._heads(v), beta), carry, done)
         return carry, _rows(h.reshape(*x.shape[:2], -1), self.norm, [self.output_projection], product, x.dtype, x)[0]
