@@ -194,6 +194,27 @@ template <typename E, int VEC> __device__ __forceinline__ void stc(E *p, const V
 // The kernels below take z and x in place of a and b when MG is set, so the coefficients never
 // exist in memory; the backward kernels then emit dz and dx instead of da and db.
 
+// Workgroup barrier that orders LDS traffic only.  __syncthreads() waits for every store of the super-step before and every load on its way,
+// which nothing behind the barrier needs.
+// PACED: with it, and each super-step's flags waited for before the rest is requested, one step after the other: where half a gigabyte and
+// more of float32 streams past, requests that come in a burst from every wave cost the memory more than the waits did (512 x 1024 x 1024 forward
+// 1025 paced, 1080 not, backward 1704 and 1744 us; 1024 x 512 x 512 501 and 522).  From 2^27 elements on, and on two or four of them a lane;
+// below it costs (200 x 150 x 800 70 and 66 us, 800 x 100 x 600 133 and 127; 1024 x 128 x 256 75 and 76).
+template <bool PACED> __device__ __forceinline__ void step_barrier()
+{
+    if constexpr (PACED) __syncthreads();
+    else asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+constexpr int64_t PACED_ELEMENTS = 1ll << 27;
+
+// A row's start, the same for the whole wave, plus a lane's place in it: what one memory instruction adds by itself (plan_scan sees to it
+// that a row is less than 4 GB).
+template <typename S> __device__ __forceinline__ S *at_bytes(S *row, uint32_t bytes)
+{
+    using C = typename std::conditional<std::is_const<S>::value, const char, char>::type;
+    return reinterpret_cast<S *>(reinterpret_cast<C *>(row) + bytes);
+}
+
 constexpr int TS_MIN = 8;  // time steps a wave holds in registers per super-step (template parameter TS of the kernels), at least
 
 // Long sequences over few columns: time is cut into n segments of `steps` steps (a multiple of a super-step), each a workgroup
@@ -256,8 +277,8 @@ constexpr int MAX_SEGMENTS = 64;
 // one-vector-lane instances that small shapes take: with 16 waves of 8 steps a sequence of up to 128
 // steps is one super-step, every load of the workgroup in flight at once and a single barrier).
 // smem: sH[2][NW][64] Vec, sP[2][NW][64] Vec, sF[2][NW] int.
-template <typename E, int VEC, bool MG = false, int MAXW = 8, typename S = E, int TS = TS_MIN, int SEG = WHOLE>
-__global__ void __launch_bounds__(64 * MAXW)
+template <typename E, int VEC, bool MG = false, int MAXW = 8, typename S = E, int TS = TS_MIN, int SEG = WHOLE, bool ATI = false, bool PACED = false>
+__global__ void __launch_bounds__(64 * MAXW, sizeof(E) == 8 && VEC == 1 ? 4 : 1)   // (two eight-wave workgroups of single complex elements a compute unit)
 diag_scan_fwd_kernel(const S *__restrict__ a, const S *__restrict__ b,
                      const void *__restrict__ done, int done_f32,
                      const E *__restrict__ h0, const E *__restrict__ P0,
@@ -284,6 +305,8 @@ diag_scan_fwd_kernel(const S *__restrict__ a, const S *__restrict__ b,
     const bool act = ((int64_t)tile * 64 + lane) * VEC < D;
     const int64_t col = first_col<VEC>((int64_t)tile * 64 + lane, D);
     const int64_t row0 = bi * T;
+    const uint32_t col_bytes = (uint32_t)col * (uint32_t)sizeof(S);
+    constexpr bool SKIP = std::is_same<S, E>::value && (SEG == WHOLE || sizeof(E) == 8);   // (narrower storage: the branch costs a quarter more registers)
 
     V carry_h = vfill<E, VEC>(O::zero()), carry_p = vfill<E, VEC>(O::one());
     if (act && SEG != SUMMARISE) {
@@ -300,7 +323,7 @@ diag_scan_fwd_kernel(const S *__restrict__ a, const S *__restrict__ b,
         sH[w * 64 + lane].x = hc;
         sP[w * 64 + lane].x = pc;
         if (lane == 0) sF[w] = cut;
-        __syncthreads();
+        step_barrier<PACED>();
         for (int j = 0; j < NW; ++j) {
             const V Hj = sH[j * 64 + lane].x, Pj = sP[j * 64 + lane].x;
             const bool fj = sF[j] != 0;
@@ -314,30 +337,64 @@ diag_scan_fwd_kernel(const S *__restrict__ a, const S *__restrict__ b,
         }
         buf = 1;
     }
+    [[maybe_unused]] V p_all;   // a broadcast coefficient
+    if constexpr (ATI) p_all = ldv<S, E, VEC>(a + col);
     const int span = NW * TS;
     for (int t0 = t_begin; t0 < t_end; t0 += span) {
         const int ts = t0 + w * TS;
         V x[TS], p[TS];
-        // reset flags of the wave's TS steps: lane s fetches the flag of step ts + s, one ballot makes the mask
-        const unsigned rmask = (unsigned)__ballot(lane < TS && ts + lane < T && done_at(done, done_f32, row0 + ts + lane));
-        raw_t<S, VEC> rp[TS], rx[TS];  // as stored; converted once every load of the super-step has been issued
+        // Everything is requested before anything is used, without branches: steps past the last read the last, lanes past the row its
+        // last channels.  Reset flags of the wave's TS steps: lane s fetches the flag of step ts + s, one ballot makes the mask.
+        uint32_t flag = 0;
+        auto row_of = [&](int s) { return row0 + (ts + s < T ? ts + s : T - 1); };
+        auto a_at = [&](int s) { return at_bytes(a + (a_ti ? 0 : row_of(s) * D), col_bytes); };
+        auto b_at = [&](int s) { return at_bytes(b + row_of(s) * D, col_bytes); };
+        unsigned rmask = 0;
+        auto form_mask = [&]() { rmask = (unsigned)__ballot(lane < TS && ts + lane < T && done_test(flag, done_f32)); };
+        if constexpr (PACED) {
+            flag = done_raw(done, done_f32, row_of(lane & (TS - 1)));
+            form_mask();
+            raw_t<S, VEC> rp[TS], rx[TS];   // (loads into registers of their own: into p and x the 512 x 1024 x 1024 call took 1045 us instead of 1027)
 #pragma unroll
-        for (int s = 0; s < TS; ++s) {
-            const int t = ts + s;
-            if (t < T && act) {
-                const int64_t off = (row0 + t) * D + col;
-                rp[s] = ldraw<S, VEC>(a + (a_ti ? col : off));
-                rx[s] = ldraw<S, VEC>(b + off);
+            for (int s = 0; s < TS; ++s) {
+                if (ts + s < T && act) {
+                    const int64_t off = (row0 + ts + s) * D + col;
+                    rp[s] = ldraw<S, VEC>(a + (a_ti ? col : off));
+                    rx[s] = ldraw<S, VEC>(b + off);
+                }
             }
-        }
 #pragma unroll
-        for (int s = 0; s < TS; ++s) {
-            if (ts + s < T && act) {
-                p[s] = cvtv<S, E, VEC>(rp[s]);
-                x[s] = cvtv<S, E, VEC>(rx[s]);
-            } else {
-                p[s] = vfill<E, VEC>(O::one());
-                x[s] = vfill<E, VEC>(O::zero());
+            for (int s = 0; s < TS; ++s) {
+                const bool in = ts + s < T && act;
+                p[s] = in ? cvtv<S, E, VEC>(rp[s]) : vfill<E, VEC>(O::one());
+                x[s] = in ? cvtv<S, E, VEC>(rx[s]) : vfill<E, VEC>(O::zero());
+            }
+        } else {
+            if (ts < T || !SKIP) {   // (a wave past the end requests nothing)
+                flag = done_raw(done, done_f32, row_of(lane));   // with those of the super-steps to come in tow
+                if constexpr (std::is_same<S, E>::value) {
+#pragma unroll
+                    for (int s = 0; s < TS; ++s) {
+                        if constexpr (ATI) p[s] = p_all;
+                        else p[s] = ldv<S, E, VEC>(a_at(s));
+                        x[s] = ldv<S, E, VEC>(b_at(s));
+                    }
+                } else {
+                    raw_t<S, VEC> rp[TS], rx[TS];  // as stored; converted once every load of the super-step has been issued
+#pragma unroll
+                    for (int s = 0; s < TS; ++s) {
+                        rp[s] = ldraw<S, VEC>(a_at(s));
+                        rx[s] = ldraw<S, VEC>(b_at(s));
+                    }
+#pragma unroll
+                    for (int s = 0; s < TS; ++s) p[s] = cvtv<S, E, VEC>(rp[s]), x[s] = cvtv<S, E, VEC>(rx[s]);
+                }
+            }
+            form_mask();
+            if (ts + TS > T) {
+#pragma unroll
+                for (int s = 0; s < TS; ++s)
+                    if (ts + s >= T) p[s] = vfill<E, VEC>(O::one()), x[s] = vfill<E, VEC>(O::zero());
             }
         }
         if constexpr (MG) {  // after every load of the super-step has been issued
@@ -362,7 +419,7 @@ diag_scan_fwd_kernel(const S *__restrict__ a, const S *__restrict__ b,
                     carry_p.v[i] = r ? p[s].v[i] : pn;
                 }
                 if (ts + s < T && act)
-                    stv<S, E, VEC>(h + (row0 + ts + s) * D + col, carry_h);
+                    stv<S, E, VEC>(at_bytes(h + (row0 + ts + s) * D, col_bytes), carry_h);
             }
             continue;
         }
@@ -386,7 +443,7 @@ diag_scan_fwd_kernel(const S *__restrict__ a, const S *__restrict__ b,
             sP[(buf * NW + w) * 64 + lane].x = pc;
             if (lane == 0) sF[buf * NW + w] = rmask != 0;
         }
-        __syncthreads();
+        step_barrier<PACED>();
         // fold the summaries: carry-in of this wave, then the workgroup carry
         V cin_h = carry_h, cin_p = carry_p, my_h = carry_h;
         for (int j = 0; j < NW; ++j) {
@@ -415,7 +472,7 @@ diag_scan_fwd_kernel(const S *__restrict__ a, const S *__restrict__ b,
                 out.v[i] = seen ? x[s].v[i] : fx;
             }
             if (SEG != SUMMARISE && ts + s < T && act)
-                stv<S, E, VEC>(h + (row0 + ts + s) * D + col, out);
+                stv<S, E, VEC>(at_bytes(h + (row0 + ts + s) * D, col_bytes), out);
         }
         buf ^= 1;
     }
@@ -437,7 +494,7 @@ diag_scan_fwd_kernel(const S *__restrict__ a, const S *__restrict__ b,
 // Backward: the same scan walked from t = T-1 down with coefficient conj(a_{t+1}),
 // cut where done_{t+1}; reversed index r = T-1-t runs forward.
 // MG: a holds z, hx holds x = h~; da receives dz and db receives dx.
-template <typename E, int VEC, bool MG = false, int MAXW = 8, typename S = E, int TS = TS_MIN, int SEG = WHOLE>
+template <typename E, int VEC, bool MG = false, int MAXW = 8, typename S = E, int TS = TS_MIN, int SEG = WHOLE, bool ATI = false, bool PACED = false>
 __global__ void __launch_bounds__(64 * MAXW)
 diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S *__restrict__ hfw,
                      const void *__restrict__ done, int done_f32,
@@ -465,6 +522,8 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
     const bool act = ((int64_t)tile * 64 + lane) * VEC < D;
     const int64_t col = first_col<VEC>((int64_t)tile * 64 + lane, D);
     const int64_t row0 = bi * T;
+    const uint32_t col_bytes = (uint32_t)col * (uint32_t)sizeof(S);
+    constexpr bool SKIP = std::is_same<S, E>::value && (SEG == WHOLE || sizeof(E) == 8);
 
     V carry = vfill<E, VEC>(O::zero());  // lam_{t+1} entering from the right
     if (act && g_last && SEG != SUMMARISE) carry = ldc<E, VEC>(g_last + bi * D + col);
@@ -482,7 +541,7 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
         sH[w * 64 + lane].x = lc;
         sP[w * 64 + lane].x = pc;
         if (lane == 0) sF[w] = cut;
-        __syncthreads();
+        step_barrier<PACED>();
         for (int j = 0; j < NW; ++j) {
             const V Hj = sH[j * 64 + lane].x, Pj = sP[j * 64 + lane].x;
             const bool fj = sF[j] != 0;
@@ -494,6 +553,14 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
         }
         buf = 1;
     }
+    [[maybe_unused]] V h0v = vfill<E, VEC>(O::zero());   // h_{-1}: what step 0 multiplies its lam with
+    if (SEG != SUMMARISE && h0) h0v = ldc<E, VEC>(h0 + bi * D + col);
+    [[maybe_unused]] V p_all;                            // a broadcast coefficient
+    if constexpr (ATI) {
+        p_all = ldv<S, E, VEC>(a + col);
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) p_all.v[i] = O::conj(p_all.v[i]);
+    }
     const int span = NW * TS;
     for (int r0 = r_begin; r0 < r_end; r0 += span) {
         const int rs = r0 + w * TS;
@@ -502,84 +569,87 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
         // barrier would be a second trip to memory on the critical path.
         V x[TS], p[TS], hp[TS];
         V zt[MG ? TS : 1], xt[MG ? TS : 1];
-        // reset flags: step s of the wave is t_s = T - 1 - (rs + s); lane l fetches done at T - rs - l, i.e.
+        // Steps before the sequence's first read the first, as lanes past the row read its last channels: no branch between the requests.
+        // Reset flags: step s of the wave is t_s = T - 1 - (rs + s); lane l fetches done at T - rs - l, i.e.
         // done_{t_0 + 1}, done_{t_0}, done_{t_1}, ..., and one ballot serves both masks (steps before the
         // sequence's first, t_s < 0, take no bit: a cut there would drop the carry on its way to dh0)
-        unsigned cmask, dmask;  // bit s: chain cut between step t_s and t_s + 1 (done_{t_s + 1}) / done_{t_s}
-        {
-            const int tt = T - rs - lane;
-            const unsigned fl = (unsigned)__ballot(lane <= TS && tt >= 0 && tt < T && done_at(done, done_f32, row0 + tt));
+        auto t_of = [&](int s) { return T - 1 - (rs + s); };
+        auto row_of = [&](int t) { return (row0 + (t < 0 ? 0 : t >= T ? T - 1 : t)) * D; };
+        const int tt = T - rs - (PACED && lane > TS ? TS : lane);
+        const uint32_t flag = done_raw(done, done_f32, row0 + (tt < 0 ? 0 : tt >= T ? T - 1 : tt));
+        unsigned cmask = 0, dmask = 0;  // bit s: chain cut between step t_s and t_s + 1 (done_{t_s + 1}) / done_{t_s}
+        auto form_masks = [&]() {
+            const unsigned fl = (unsigned)__ballot(lane <= TS && tt >= 0 && tt < T && done_test(flag, done_f32));
             const int nv = T - rs < TS ? (T - rs < 0 ? 0 : T - rs) : TS;  // steps of the wave inside the sequence
             const unsigned vm = (1u << nv) - 1u;
             cmask = fl & vm;
             dmask = (fl >> 1) & vm;
-        }
-        if constexpr (std::is_same<S, E>::value) {
+        };
+        if (PACED) form_masks();
+        if (rs < T || !SKIP) {   // (a wave past the end requests nothing)
+            if constexpr (std::is_same<S, E>::value) {
 #pragma unroll
-            for (int s = 0; s < TS; ++s) {
-                const int t = T - 1 - (rs + s);
-                p[s] = vfill<E, VEC>(O::one());
-                x[s] = vfill<E, VEC>(O::zero());
-                hp[s] = vfill<E, VEC>(O::zero());
-                if (t >= 0 && act) {
-                    const int64_t off = (row0 + t) * D + col;
-                    x[s] = ldv<S, E, VEC>(g + off);
-                    if (t + 1 < T) {
-                        V av = ldv<S, E, VEC>(a + (a_ti ? col : off + D));
-#pragma unroll
-                        for (int i = 0; i < VEC; ++i) p[s].v[i] = MG ? av.v[i] : O::conj(av.v[i]);  // MG: z_{t+1} for now
-                    }
-                    if (SEG == SUMMARISE) continue;
-                    if (t > 0)
-                        hp[s] = ldv<S, E, VEC>(hfw + off - D);
-                    else if (h0)
-                        hp[s] = ldc<E, VEC>(h0 + bi * D + col);
-                    if constexpr (MG) {
-                        zt[s] = ldv<S, E, VEC>(a + off);
-                        xt[s] = ldv<S, E, VEC>(hx + off);
+                for (int s = 0; s < TS; ++s) {
+                    const int t = t_of(s);
+                    if (PACED && !(t >= 0 && act)) continue;
+                    x[s] = ldv<S, E, VEC>(at_bytes(g + row_of(t), col_bytes));
+                    if constexpr (ATI) p[s] = p_all;
+                    else p[s] = ldv<S, E, VEC>(at_bytes(a + (a_ti ? 0 : row_of(t + 1)), col_bytes));
+                    if constexpr (SEG != SUMMARISE) {
+                        hp[s] = ldv<S, E, VEC>(at_bytes(hfw + row_of(t - 1), col_bytes));
+                        if constexpr (MG) {
+                            zt[s] = ldv<S, E, VEC>(at_bytes(a + row_of(t), col_bytes));
+                            xt[s] = ldv<S, E, VEC>(at_bytes(hx + row_of(t), col_bytes));
+                        }
                     }
                 }
-            }
-        } else {
-            // narrower storage: the values wait as stored and are widened once every load has been issued
-            raw_t<S, VEC> rg[TS], ra[TS], rh[TS], rz[MG ? TS : 1], rxt[MG ? TS : 1];
-            V h0v = vfill<E, VEC>(O::zero());  // h_{-1}: what step 0 multiplies its lam with
-            if (SEG != SUMMARISE && act && h0 && T - 1 - rs - (TS - 1) <= 0) h0v = ldc<E, VEC>(h0 + bi * D + col);
+            } else {
+                // narrower storage: the values wait as stored and are widened once every load has been issued
+                raw_t<S, VEC> rg[TS], ra[TS], rh[TS], rz[MG ? TS : 1], rxt[MG ? TS : 1];
 #pragma unroll
-            for (int s = 0; s < TS; ++s) {
-                const int t = T - 1 - (rs + s);
-                if (t >= 0 && act) {
-                    const int64_t off = (row0 + t) * D + col;
-                    rg[s] = ldraw<S, VEC>(g + off);
-                    if (t + 1 < T) ra[s] = ldraw<S, VEC>(a + (a_ti ? col : off + D));
-                    if (SEG == SUMMARISE) continue;
-                    if (t > 0) rh[s] = ldraw<S, VEC>(hfw + off - D);
-                    if constexpr (MG) {
-                        rz[s] = ldraw<S, VEC>(a + off);
-                        rxt[s] = ldraw<S, VEC>(hx + off);
+                for (int s = 0; s < TS; ++s) {
+                    const int t = t_of(s);
+                    rg[s] = ldraw<S, VEC>(at_bytes(g + row_of(t), col_bytes));
+                    ra[s] = ldraw<S, VEC>(at_bytes(a + (a_ti ? 0 : row_of(t + 1)), col_bytes));
+                    if constexpr (SEG != SUMMARISE) {
+                        rh[s] = ldraw<S, VEC>(at_bytes(hfw + row_of(t - 1), col_bytes));
+                        if constexpr (MG) {
+                            rz[s] = ldraw<S, VEC>(at_bytes(a + row_of(t), col_bytes));
+                            rxt[s] = ldraw<S, VEC>(at_bytes(hx + row_of(t), col_bytes));
+                        }
                     }
                 }
-            }
 #pragma unroll
-            for (int s = 0; s < TS; ++s) {
-                const int t = T - 1 - (rs + s);
-                p[s] = vfill<E, VEC>(O::one());
-                x[s] = vfill<E, VEC>(O::zero());
-                hp[s] = vfill<E, VEC>(O::zero());
-                if (t >= 0 && act) {
+                for (int s = 0; s < TS; ++s) {
                     x[s] = cvtv<S, E, VEC>(rg[s]);
-                    if (t + 1 < T) {
-                        const V av = cvtv<S, E, VEC>(ra[s]);
+                    p[s] = cvtv<S, E, VEC>(ra[s]);
+                    if constexpr (SEG != SUMMARISE) {
+                        hp[s] = cvtv<S, E, VEC>(rh[s]);
+                        if constexpr (MG) {
+                            zt[s] = cvtv<S, E, VEC>(rz[s]);
+                            xt[s] = cvtv<S, E, VEC>(rxt[s]);
+                        }
+                    }
+                }
+            }
+        }
+        if (!PACED) form_masks();
+        if constexpr (!MG && !ATI) {
 #pragma unroll
-                        for (int i = 0; i < VEC; ++i) p[s].v[i] = MG ? av.v[i] : O::conj(av.v[i]);  // MG: z_{t+1} for now
-                    }
-                    if (SEG == SUMMARISE) continue;
-                    if (t > 0) hp[s] = cvtv<S, E, VEC>(rh[s]);
-                    else hp[s] = h0v;
-                    if constexpr (MG) {
-                        zt[s] = cvtv<S, E, VEC>(rz[s]);
-                        xt[s] = cvtv<S, E, VEC>(rxt[s]);
-                    }
+            for (int s = 0; s < TS; ++s)
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) p[s].v[i] = O::conj(p[s].v[i]);   // MG: z_{t+1} for now
+        }
+        if (rs == 0) p[0] = vfill<E, VEC>(O::one());   // nothing follows the last step
+        if (rs + TS >= T) {   // the sequence's first step, and what would come before it
+#pragma unroll
+            for (int s = 0; s < TS; ++s) {
+                const int t = t_of(s);
+                if (t == 0 && SEG != SUMMARISE) hp[s] = h0v;
+                if (t < 0) {
+                    p[s] = vfill<E, VEC>(O::one());
+                    x[s] = vfill<E, VEC>(O::zero());
+                    hp[s] = vfill<E, VEC>(O::zero());
                 }
             }
         }
@@ -626,7 +696,7 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
             sH[(buf * NW + w) * 64 + lane].x = lc;
             sP[(buf * NW + w) * 64 + lane].x = pc;
             if (lane == 0) sF[buf * NW + w] = cmask != 0;
-            __syncthreads();
+            step_barrier<PACED>();
             V cin = carry;
             for (int j = 0; j < NW; ++j) {
                 if (j == w) my = cin;
@@ -699,9 +769,9 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
     }
     if (!MG && da_sum) {  // uniform over the workgroup
         if (NW > 1) {
-            __syncthreads();  // the last fold has read sH
+            step_barrier<PACED>();  // the last fold has read sH
             sH[w * 64 + lane].x = dsum;
-            __syncthreads();
+            step_barrier<PACED>();
             if (w == 0) {
                 for (int j = 1; j < NW; ++j) {
                     const V dj = sH[j * 64 + lane].x;
@@ -1032,6 +1102,7 @@ ScanPlan plan_scan(int64_t B, int64_t T, int64_t D, size_t esize, bool bwd, bool
 {
     const int maxvec = (int)(16 / esize);
     int vec = 1;
+    if (D >= (1ll << 28)) return {1, 1, (int)((D + 63) / 64), true};   // the wave-split kernels count a row's bytes in 32 bits
     for (int v = maxvec; v >= 1; v >>= 1) {
         // a vector so wide that the waves covering a row are less than three quarters full wastes the
         // idle lanes' share of every load (rows of 128 floats, backward: 0.87 -> 0.57 ms at 16384x64x128
@@ -1060,6 +1131,11 @@ ScanPlan plan_scan(int64_t B, int64_t T, int64_t D, size_t esize, bool bwd, bool
         const int64_t waves2 = B * D / 128;   // of the streaming kernels on two elements per lane
         int nw8 = 1;  // waves along time: up to eight, each with a whole group of steps to itself
         while (nw8 < 8 && (int64_t)2 * nw8 * TS_MIN <= T) nw8 <<= 1;
+        // (***) A fourth sweep, once the wave-split kernels requested everything of a super-step at once, waited for no store at their barriers and
+        // read a broadcast coefficient once: twenty-six shapes of each kind, `full`: four elements per lane leave few lanes idle.  Four waves
+        // along time on wide vectors gained most -- a workgroup's registers then leave room for others beside it.  us, before -> now.
+        const int64_t covered4 = 256 * ntiles(4);
+        const bool full = ntiles(4) == 1 ? D >= 176 : 10 * D >= 9 * covered4;
         // (*) bfloat16 backward: single elements are 2-byte loads, three or four arrays of them; two per lane and 16 steps
         // per wave make up for half the waves (8 x 1000 x 64 66 -> 54, 57 x 2908 x 120 217 -> 166), while a workgroup per compute
         // unit is all there is
@@ -1067,6 +1143,20 @@ ScanPlan plan_scan(int64_t B, int64_t T, int64_t D, size_t esize, bool bwd, bool
         // so few columns that eight waves along time leave most of the device idle: sixteen of one lane each; (*) forward with
         // 16 steps each, half as many trips to memory (4 x 3000 x 512 101 -> 77, 75 x 679 x 64 29 -> 22)
         if (T >= 16 * TS_MIN && cols(1) <= 256) return split(1, 16, !bwd && esize == 4 && T > 16 * TS_MIN ? 16 : 8);
+        if (half_storage && T >= 8 * TS_MIN) {
+            // (***) bfloat16, forward and backward: 512 x 1024 x 1024 661 -> 527 and 1066 -> 848, 400 x 200 x 201 43 -> 32 and 67 -> 52, 1024 x 512 x 512 332
+            // -> 287 and 536 -> 489, 500 x 64 x 200 16 -> 14 and 28 -> 20; backward also with more lanes idle (984 x 378 x 448 362 -> 342), but not
+            // where a thousand columns of ragged rows make few workgroups (128 x 512 x 1000 176 / 191)
+            if (!mg && cols(4) >= 400 && (full || (bwd && !a_ti && 100 * D >= 68 * covered4)) && !(bwd && a_ti && T < 16 * TS_MIN) && !(bwd && ragged && ntiles(4) > 1 && cols(4) < 1024)) return split(4, 4);
+            // MinGRU backward: with columns enough whole rows stream on four elements per lane (1510 x 943 x 165 966 -> 857, 4096 x 64 x 256 165 -> 144,
+            // 300 x 700 x 1000 863 -> 751), with fewer the split (256 x 2048 x 512 891 -> 663, 128 x 1024 x 1024 437 -> 323, 500 x 64 x 200 35 -> 27;
+            // forward 300 x 700 x 1000 430 -> 372, 256 x 2048 x 512 397 -> 360)
+            if (mg && bwd && B * D >= 256 * 1100) return flow(4);
+            if (mg && bwd && cols(4) >= 400 && cols(4) < 640 && full) return split(4, 4);
+            if (mg && !bwd && ragged && cols(4) >= 400 && full) return split(4, 4);
+            if (mg && bwd && D > 64 && D <= 128 && cols(2) >= 512) return split(2, 4);   // 1000 x 500 x 128 222 -> 175
+            if (mg && !bwd && !ragged && D % 64 == 0 && cols(2) >= 1024) return split(2, 4);   // 256 x 2048 x 512 397 -> 347
+        }
         if (half_storage) {
             // (swept again once the bfloat16 values waited as stored bits: the wave-split kernels then lead
             // forward at every size; four elements per lane, backward, do not fit the wave-split kernel's
@@ -1085,6 +1175,12 @@ ScanPlan plan_scan(int64_t B, int64_t T, int64_t D, size_t esize, bool bwd, bool
             if (v == 2 && (bwd ? waves2 >= 600 : ragged && waves2 >= (mg ? 1800 : 1000))) return flow(2);
             if ((bwd ? cols(v) >= 512 : cols(v) >= (v == 2 ? 513 : 1024)) && nw8 > 4) return split(v, 4);
             return split(v, nw8, !bwd && T >= 64 * TS_MIN && nw8 == 8 && (v == 1 || cols(v) <= 256) ? 16 : 8);   // (*) 256 x 1024 x 96 63 -> 50
+        }
+        if (esize == 8 && !mg && a_ti && T >= 8 * TS_MIN) {
+            // (***) complex64 with a broadcast decay, forward and backward: 300 x 700 x 500 486 -> 381 and 684 -> 554, 500 x 200 x 184 98 -> 68 and 123 ->
+            // 103, 192 x 250 x 184 42 -> 40 and 66 -> 56, 100 x 600 x 512 102 -> 89 and 148 -> 134, 1024 x 64 x 256 53 -> 48 and 81 -> 71
+            if (T >= 12 * TS_MIN ? cols(2) >= 400 : (cols(2) >= 512 && D % 64 != 0)) return split(2, 4);
+            if (cols(1) >= 512) return split(1, 4);
         }
         if (esize == 8 && !mg) {
             // (*) ragged rows stream, and so do the backward that sums a broadcast decay's gradient (no da to write) and that of
@@ -1108,6 +1204,8 @@ ScanPlan plan_scan(int64_t B, int64_t T, int64_t D, size_t esize, bool bwd, bool
                 return split(vec < 2 || cols(1) <= 256 ? 1 : 2, nw8);
             }
             if (mg) {
+                // (***) 1024 x 512 x 512 1137 -> 1037, 800 x 100 x 600 284 -> 254, 4096 x 64 x 256 306 -> 252
+                if (T >= 8 * TS_MIN && D > 128 && waves2 >= 3000) return flow(2);
                 if (vec == 4 && cols(4) >= 2048 && T >= 8 * TS_MIN) return split(4, nw8 > 4 ? 4 : nw8);
                 if (D <= 128 && cols(1) >= 2048) return split(1, nw8);
             } else {
@@ -1335,9 +1433,18 @@ int launch_fwd(hipStream_t st, const void *a, const void *b, const void *done,
         const dim3 grid((unsigned)(B * pl.tiles)), block(64 * pl.nw);
         const size_t smem = scan_smem(pl.nw, sizeof(E) * pl.vec);
         split_switch<E, MG, false, !std::is_same<S, E>::value>(pl, [&](auto vc, auto mw, auto ts) {
-            rc = launch_kernel((diag_scan_fwd_kernel<E, decltype(vc)::value, MG, decltype(mw)::value, S, decltype(ts)::value>), grid, block, smem,
-                               st, (const S *)a, (const S *)b, done, done_f32, (const E *)h0, (const E *)P0, (S *)h, (E *)h_last, (E *)P_last,
-                               (int)T, D, pl.tiles, pl.nw, a_ti, Segments<E>{});
+            auto go = [&](auto ti, auto paced) {
+                rc = launch_kernel((diag_scan_fwd_kernel<E, decltype(vc)::value, MG, decltype(mw)::value, S, decltype(ts)::value, WHOLE, decltype(ti)::value, decltype(paced)::value>),
+                                   grid, block, smem, st, (const S *)a, (const S *)b, done, done_f32, (const E *)h0, (const E *)P0, (S *)h, (E *)h_last,
+                                   (E *)P_last, (int)T, D, pl.tiles, pl.nw, a_ti, Segments<E>{});
+            };
+            if constexpr (!MG && std::is_same<S, E>::value) {   // a broadcast coefficient is read once
+                if (a_ti) return go(std::true_type{}, std::false_type{});
+            }
+            if constexpr (std::is_same<S, float>::value && decltype(vc)::value >= 2 && decltype(mw)::value == 8 && decltype(ts)::value == TS_MIN) {
+                if (B * T * D >= PACED_ELEMENTS) return go(std::false_type{}, std::true_type{});
+            }
+            go(std::false_type{}, std::false_type{});
         });
     }
     return rc;
@@ -1402,9 +1509,18 @@ int launch_bwd(hipStream_t st, const void *a, const void *hx, const void *h, con
         const dim3 grid((unsigned)(B * pl.tiles)), block(64 * pl.nw);
         const size_t smem = scan_smem(pl.nw, sizeof(E) * pl.vec);
         split_switch<E, MG, true, !std::is_same<S, E>::value>(pl, [&](auto vc, auto mw, auto ts) {
-            rc = launch_kernel((diag_scan_bwd_kernel<E, decltype(vc)::value, MG, decltype(mw)::value, S, decltype(ts)::value>), grid, block, smem,
-                               st, (const S *)a, (const S *)hx, (const S *)h, done, done_f32, (const E *)h0, (const S *)g, (const E *)g_last,
-                               (S *)da, (S *)db, (E *)dh0, (int)T, D, pl.tiles, pl.nw, a_ti, da_sum, Segments<E>{});
+            auto go = [&](auto ti, auto paced) {
+                rc = launch_kernel((diag_scan_bwd_kernel<E, decltype(vc)::value, MG, decltype(mw)::value, S, decltype(ts)::value, WHOLE, decltype(ti)::value, decltype(paced)::value>),
+                                   grid, block, smem, st, (const S *)a, (const S *)hx, (const S *)h, done, done_f32, (const E *)h0, (const S *)g,
+                                   (const E *)g_last, (S *)da, (S *)db, (E *)dh0, (int)T, D, pl.tiles, pl.nw, a_ti, da_sum, Segments<E>{});
+            };
+            if constexpr (!MG && std::is_same<S, E>::value) {
+                if (a_ti) return go(std::true_type{}, std::false_type{});
+            }
+            if constexpr (std::is_same<S, float>::value && decltype(vc)::value >= 2 && decltype(mw)::value == 8 && decltype(ts)::value == TS_MIN) {
+                if (B * T * D >= PACED_ELEMENTS) return go(std::false_type{}, std::true_type{});
+            }
+            go(std::false_type{}, std::false_type{});
         });
     }
     return rc;

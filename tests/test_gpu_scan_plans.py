@@ -65,3 +65,20 @@ def test_scan_plans(kind, shape):
                                (2e-2, 1e-4, 2e-2, 2e-2, 2e-2) if half else (1e-4,) * 5):
         err = float((x.to(r.dtype) - r).abs().max() / r.abs().max().clamp_min(1e-30))
         assert err <= tol, (name, err)
+
+
+WIDE = [
+    (405, 66, 176), (403, 67, 200), (410, 65, 201),      # four waves on wide vectors: whole and ragged rows, spans partly filled
+    (1100, 64, 256), (1101, 70, 257),                    # whole rows streaming on wide vectors (MinGRU, bfloat16)
+    (520, 70, 100), (520, 72, 256), (260, 80, 128),      # two elements and single ones per lane, four waves
+    (405, 97, 67), (134, 101, 515),                      # a lane of the last tile
+    (1025, 513, 256), (130, 1009, 1024), (260, 520, 1000),   # large float32 calls (2^27 elements and more)
+]
+
+
+@pytest.mark.parametrize("shape", WIDE)
+@pytest.mark.parametrize("kind", ["f32", "f32 broadcast", "bf16", "bf16 broadcast", "c64", "c64 broadcast", "mingru", "mingru bf16"])
+def test_wide_splits(kind, shape):
+    if shape[0] * shape[1] * shape[2] >= 1 << 27 and kind not in ("f32", "mingru"):
+        pytest.skip("float32 storage with coefficients of every step only")
+    test_scan_plans(kind, shape)
