@@ -9,10 +9,13 @@
 //             dt = softplus(dt_in + dt_bias),  g = -dt exp(A_log)
 //   read-out  y = rms_norm(o + D hidden) * scale * silu(z)
 //
-// All are bound by HBM.  Layout: a wave is 64 lanes x 4 consecutive channels of one time tile and walks its steps with the
-// last K inputs in registers, so a row of an array is read once per tile (plus K - 1 rows that the neighbouring tile of the
-// same workgroup has just brought in), four rows requested ahead of their use.
+// Layout: a wave is 64 lanes x 4 consecutive channels of one time tile and walks its steps with the last K inputs in registers, so a row of an
+// array is read once per tile (plus K - 1 rows that the neighbouring tile of the same workgroup has just brought in), four rows requested ahead
+// of their use.  256 x 128 steps x 1536 channels: the elements 84 us forward and 143 backward (402 and 670 MB: 63 and 105 us at what a copy
+// reaches), bound by HBM and the exponentials' arithmetic about alike; with a branch at every load, a division per sigmoid and a head's gate formed
+// by each of its lanes at each step they took 93 and 184.  Two channels per lane -- twice the waves in flight -- read the same (86 and 143).
 #include <initializer_list>
+#include <type_traits>
 
 #include "col_sum.h"
 #include "common.h"
@@ -32,7 +35,13 @@ __device__ __forceinline__ F4 load4(const float *p) { return *reinterpret_cast<c
 __device__ __forceinline__ void store4(float *p, const F4 &x) { *reinterpret_cast<F4 *>(p) = x; }
 
 // The library exponential: the hardware's errs by |x| / 2 ulp, which silu keeps as a relative error, and the passes are bound by HBM.
-__device__ __forceinline__ float sigmoidf(float x) { return 1.f / (1.f + expf(-x)); }
+// The quotient by one Newton step on the hardware's reciprocal (the remainder formed exactly: as good as a division's own steps, a third as many;
+// the fix-up restores 0 and NaN).
+__device__ __forceinline__ float sigmoidf(float x)
+{
+    const float d = 1.f + expf(-x), r = __builtin_amdgcn_rcpf(d);
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, r, 1.f), r, r), d, 1.f);
+}
 __device__ __forceinline__ float softplusf(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 
 // One run of channels of a convolution: where its rows lie and what becomes of them.
@@ -83,81 +92,250 @@ template <int K> __device__ __forceinline__ void load_taps(const ConvArgs &a, co
         for (int j = 0; j < K; ++j) w[j].v[e] = a.w[(int64_t)(sg.w0 + c + e) * K + j];
 }
 
-template <int K> __global__ void __launch_bounds__(CV_THREADS) conv_fwd_kernel(ConvArgs a)
+// A value of lane I of the lane's group of four, and that of the lane whose number differs in the bits of M.
+template <int I> __device__ __forceinline__ float of_lane(float x)
 {
-    int ntiles = 0;
-    for (int s = 0; s < a.nseg; ++s) ntiles += a.tiles[s];
-    int tile = (int)(blockIdx.x % (unsigned)ntiles);
-    const int64_t item = (int64_t)(blockIdx.x / (unsigned)ntiles) * CV_WAVES + (threadIdx.x >> 6);
-    if (item >= a.items) return;
-    const bool first = tile == 0;
-    const int lane = threadIdx.x & 63;
-    const Segment &sg = a.seg[segment_of(a, tile)];
-    const int c = (tile * 64 + lane) * 4;
-    const bool act = c < sg.C;
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), I * 0x55, 0xf, 0xf, true));
+}
+template <int M> __device__ __forceinline__ float other_lane(float x)
+{
+    constexpr int ctrl = (0 ^ M) | (1 ^ M) << 2 | (2 ^ M) << 4 | (3 ^ M) << 6;
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), ctrl, 0xf, 0xf, true));
+}
+// Four values of every lane, added up over the lane's group of four: lane l is left with the sum of the value l & 3.
+__device__ __forceinline__ float sum_of_four(const float (&x)[4], int lane)
+{
+    const bool odd = lane & 1, high = lane & 2;
+    const float s01 = (odd ? x[1] : x[0]) + other_lane<1>(odd ? x[0] : x[1]), s23 = (odd ? x[3] : x[2]) + other_lane<1>(odd ? x[2] : x[3]);
+    return (high ? s23 : s01) + other_lane<2>(high ? s01 : s23);
+}
+
+// What the kinds of channels differ in: PLAIN, GATED (y times dt of the head), SKIP (a second gradient, backward only).
+enum Kind { PLAIN, GATED, SKIP };
+
+// Rows are requested four at a time and four ahead of their use, without a branch: rows past the sequence read its last one, lanes past the
+// channels the first ones.  A head's gate at the four steps is formed once, by the four lanes of each group of four (a head of sixteen features
+// is four lanes; narrower ones form all four in every lane).
+template <int K, int KIND> __device__ __forceinline__ void conv_fwd_walk(const ConvArgs &a, const Segment &sg, int c, bool act, int64_t item)
+{
+    const int lane = threadIdx.x & 63, cc = act ? c : 0;
     const int64_t b = item / a.tiles_t;
     const int t0 = (int)(item % a.tiles_t) * a.tile_t, t1 = min(a.T, t0 + a.tile_t);
     const int64_t row0 = b * a.T;
-
-    if (first && a.g) {   // the log-decay, beside the first tile's work
-        const int n = (t1 - t0) * a.H;
-        for (int i = lane; i < n; i += 64) {
-            const int h = i % a.H;
-            const int64_t at = (row0 + t0) * a.H + i;
-            a.g[at] = softplusf(a.dt_in[at] + a.dt_bias[h]) * -expf(a.A_log[h]);
-        }
-    }
     F4 w[K], bias, win[K];
     load_taps<K>(a, sg, c, act, w, bias);
-    const float *x = sg.x + row0 * sg.ld + c;
-    float *y = sg.y + row0 * sg.C + c;
-    const int h = sg.gated && act ? c / a.N : 0;
-    const float dtb = sg.gated ? a.dt_bias[h] : 0.f;
+    const float *x = sg.x + row0 * sg.ld;
+    float *y = sg.y + row0 * sg.C;
+    const int h = KIND == GATED ? cc / a.N : 0;
+    const bool four = a.N >= 16;
+    const float dtb = KIND == GATED ? a.dt_bias[h] : 0.f;
+    auto row = [&](int t) { return t < a.T ? t : a.T - 1; };
 #pragma unroll
     for (int j = 0; j < K - 1; ++j) {
         const int t = t0 - (K - 1) + j;
-        win[j + 1] = act && t >= 0 ? load4(x + t * sg.ld) : F4_ZERO;
+        win[j + 1] = load4(x + (t < 0 ? 0 : t) * sg.ld + cc);
+        if (t < 0) win[j + 1] = F4_ZERO;
     }
     F4 next[CV_AHEAD];
-    float dt_next[CV_AHEAD];
+    float dt_next = 0.f;
     auto fetch = [&](int t) {
 #pragma unroll
-        for (int i = 0; i < CV_AHEAD; ++i) {
-            const bool in = act && t + i < t1;
-            next[i] = in ? load4(x + (t + i) * sg.ld) : F4_ZERO;
-            dt_next[i] = in && sg.gated ? a.dt_in[(row0 + t + i) * a.H + h] : 0.f;
-        }
+        for (int i = 0; i < CV_AHEAD; ++i) next[i] = load4(x + row(t + i) * sg.ld + cc);
+        if (KIND == GATED && four) dt_next = a.dt_in[(row0 + row(t + (lane & 3))) * a.H + h];
     };
     fetch(t0);
     for (int t = t0; t < t1; t += CV_AHEAD) {
         F4 cur[CV_AHEAD];
-        float dt[CV_AHEAD];
 #pragma unroll
-        for (int i = 0; i < CV_AHEAD; ++i) cur[i] = next[i], dt[i] = dt_next[i];
-        fetch(t + CV_AHEAD);
+        for (int i = 0; i < CV_AHEAD; ++i) cur[i] = next[i];
+        float gate[CV_AHEAD] = {1.f, 1.f, 1.f, 1.f};
+        const float dt = dt_next;
+        if (t + CV_AHEAD < t1) fetch(t + CV_AHEAD);
+        if (KIND == GATED) {
+            if (four) {
+                const float g = softplusf(dt + dtb);
+                gate[0] = of_lane<0>(g), gate[1] = of_lane<1>(g), gate[2] = of_lane<2>(g), gate[3] = of_lane<3>(g);
+            } else {
+#pragma unroll
+                for (int i = 0; i < CV_AHEAD; ++i) gate[i] = softplusf(a.dt_in[(row0 + row(t + i)) * a.H + h] + dtb);
+            }
+        }
 #pragma unroll
         for (int i = 0; i < CV_AHEAD; ++i) {
 #pragma unroll
             for (int j = 0; j + 1 < K; ++j) win[j] = win[j + 1];
             win[K - 1] = cur[i];
-            const float gate = sg.gated ? softplusf(dt[i] + dtb) : 1.f;
             F4 o;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 float s = bias.v[e];
 #pragma unroll
                 for (int j = 0; j < K; ++j) s += w[j].v[e] * win[j].v[e];
-                o.v[e] = s * sigmoidf(s) * gate;
+                o.v[e] = s * sigmoidf(s);
+                if (KIND == GATED) o.v[e] *= gate[i];
             }
-            if (act && t + i < t1) store4(y + (int64_t)(t + i) * sg.C, o);
+            if (act && t + i < t1) store4(y + (int64_t)(t + i) * sg.C + c, o);
         }
     }
 }
+
+template <int K> __global__ void __launch_bounds__(CV_THREADS) conv_fwd_kernel(ConvArgs a)
+{
+    int ntiles = 0;
+    for (int s = 0; s < a.nseg; ++s) ntiles += a.tiles[s];
+    int tile = (int)(blockIdx.x % (unsigned)ntiles);
+    const int64_t item = (int64_t)(blockIdx.x / (unsigned)ntiles) * CV_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (item >= a.items) return;
+    const int lane = threadIdx.x & 63;
+    if (tile == 0 && a.g) {   // the log-decay, beside the first tile's work
+        const int t0 = (int)(item % a.tiles_t) * a.tile_t, n = (min(a.T, t0 + a.tile_t) - t0) * a.H;
+        const int64_t first = (item / a.tiles_t * a.T + t0) * a.H;
+        for (int i = lane; i < n; i += 64) {
+            const int h = i % a.H;
+            a.g[first + i] = softplusf(a.dt_in[first + i] + a.dt_bias[h]) * -expf(a.A_log[h]);
+        }
+    }
+    const Segment &sg = a.seg[segment_of(a, tile)];
+    const int c = (tile * 64 + lane) * 4;
+    if (sg.gated) conv_fwd_walk<K, GATED>(a, sg, c, c < sg.C, item);
+    else conv_fwd_walk<K, PLAIN>(a, sg, c, c < sg.C, item);
+}
+
+// A wave's share of the parameters' gradients.
+template <int K> struct ConvSums {
+    F4 dw[K], dbias;
+    float dtb, A, D;
+};
 
 // Backward: the pre-activations are formed again from the inputs; a step's gradient ds_t = dy_t silu'(s_t) reaches the inputs
 // t-K+1 .. t, so dx_{t-K+1} is complete once ds_t is known, and a tile walks K - 1 steps past its end for its last rows.
 // The parameters' gradients stay in registers over all tiles of a wave (workgroup column p takes the items p, p + nparts, ...)
 // and leave as one row of partial sums per workgroup.
+template <int K, int KIND> __device__ __forceinline__ void conv_bwd_walk(const ConvArgs &a, const Segment &sg, int c, bool act, int64_t first, ConvSums<K> &sum)
+{
+    const int lane = threadIdx.x & 63, cc = act ? c : 0;
+    F4 w[K], bias;
+    load_taps<K>(a, sg, c, act, w, bias);
+    const int h = KIND == GATED ? cc / a.N : KIND == SKIP ? cc / a.P : 0;
+    const bool four = a.N >= 16;
+    const float dtb = KIND == GATED ? a.dt_bias[h] : 0.f, A = KIND == GATED ? -expf(a.A_log[h]) : 0.f;
+    const float skip_scale = KIND == SKIP ? a.D[h] : 0.f;
+    const bool heads_lane = KIND == GATED && act && cc % a.N < (four ? 16 : 4);   // the lanes that write what is one number per head and step
+
+    for (int64_t item = first; item < a.items; item += (int64_t)a.nparts * CV_WAVES) {
+        const int64_t b = item / a.tiles_t;
+        const int t0 = (int)(item % a.tiles_t) * a.tile_t, t1 = min(a.T, t0 + a.tile_t);
+        const int64_t row0 = b * a.T;
+        const float *x = sg.x + row0 * sg.ld, *dy = sg.dy + row0 * sg.C, *skip = KIND == SKIP ? sg.skip + row0 * sg.C : nullptr;
+        float *dx = sg.dx + row0 * sg.ld_dx;
+        auto row = [&](int t) { return t < a.T ? t : a.T - 1; };
+        F4 win[K], dwin[K];
+#pragma unroll
+        for (int j = 0; j < K; ++j) dwin[j] = F4_ZERO;
+#pragma unroll
+        for (int j = 0; j < K - 1; ++j) {
+            const int t = t0 - (K - 1) + j;
+            win[j + 1] = load4(x + (t < 0 ? 0 : t) * sg.ld + cc);
+            if (t < 0) win[j + 1] = F4_ZERO;
+        }
+        F4 xn[CV_AHEAD], yn[CV_AHEAD], kn[KIND == SKIP ? CV_AHEAD : 1];
+        float dtn = 0.f, dgn = 0.f;
+        auto fetch = [&](int t) {
+#pragma unroll
+            for (int i = 0; i < CV_AHEAD; ++i) {
+                const int64_t r = row(t + i);
+                xn[i] = load4(x + r * sg.ld + cc);
+                yn[i] = load4(dy + r * sg.C + cc);
+                if constexpr (KIND == SKIP) kn[i] = load4(skip + r * sg.C + cc);
+            }
+            if (KIND == GATED && four) {
+                const int64_t at = (row0 + row(t + (lane & 3))) * a.H + h;
+                dtn = a.dt_in[at], dgn = a.dg[at];
+            }
+        };
+        // Four steps; whole: all of them in the tile.
+        auto steps = [&](int t, auto whole) {
+            F4 xc[CV_AHEAD], yc[CV_AHEAD], kc[KIND == SKIP ? CV_AHEAD : 1];
+#pragma unroll
+            for (int i = 0; i < CV_AHEAD; ++i) {
+                xc[i] = xn[i], yc[i] = yn[i];
+                if constexpr (KIND == SKIP) kc[i] = kn[i];
+                if (!decltype(whole)::value && t + i >= a.T) {   // rows past the sequence hold zeros
+                    xc[i] = yc[i] = F4_ZERO;
+                    if constexpr (KIND == SKIP) kc[i] = F4_ZERO;
+                }
+            }
+            const float dt = dtn, dg = dgn;
+            if (t + CV_AHEAD < t1 + K - 1) fetch(t + CV_AHEAD);
+            float gate[CV_AHEAD], ddt[CV_AHEAD] = {0.f, 0.f, 0.f, 0.f};
+            const float pre = dt + dtb, gate4 = KIND == GATED ? softplusf(pre) : 1.f;
+            if (KIND == GATED) {
+                if (four) {
+                    gate[0] = of_lane<0>(gate4), gate[1] = of_lane<1>(gate4), gate[2] = of_lane<2>(gate4), gate[3] = of_lane<3>(gate4);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < CV_AHEAD; ++i) gate[i] = softplusf(a.dt_in[(row0 + row(t + i)) * a.H + h] + dtb);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < CV_AHEAD; ++i) {
+                const int ti = t + i;
+                const bool own = decltype(whole)::value || ti < t1;   // counts towards the parameters here; later steps count in their own tile
+#pragma unroll
+                for (int j = 0; j + 1 < K; ++j) win[j] = win[j + 1], dwin[j] = dwin[j + 1];
+                win[K - 1] = xc[i];
+                dwin[K - 1] = F4_ZERO;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float s = bias.v[e];
+#pragma unroll
+                    for (int j = 0; j < K; ++j) s += w[j].v[e] * win[j].v[e];
+                    const float sg1 = sigmoidf(s), y = s * sg1;
+                    float up = yc[i].v[e];   // gradient of y
+                    if (KIND == GATED) up *= gate[i], ddt[i] += yc[i].v[e] * y;
+                    if constexpr (KIND == SKIP) up += kc[i].v[e] * skip_scale;
+                    const float ds = up * sg1 * (1.f + s * (1.f - sg1));
+                    if (own) {
+                        if constexpr (KIND == SKIP) sum.D += kc[i].v[e] * y;
+                        sum.dbias.v[e] += ds;
+#pragma unroll
+                        for (int j = 0; j < K; ++j) sum.dw[j].v[e] += ds * win[j].v[e];
+                    }
+#pragma unroll
+                    for (int j = 0; j < K; ++j) dwin[j].v[e] += w[j].v[e] * ds;
+                }
+                const int tx = ti - (K - 1);
+                if (act && tx >= t0 && tx < t1) store4(dx + tx * sg.ld_dx + c, dwin[0]);
+            }
+            if (KIND != GATED) return;
+            auto leaves = [&](int ti, float total, float pre_t, float gate_t, float dg_t) {   // a head's gradient at one step
+                if (!heads_lane || ti >= t1) return;
+                const float dpre = (total + dg_t * A) * (pre_t > 20.f ? 1.f : sigmoidf(pre_t));
+                a.ddt_in[(row0 + ti) * a.H + h] = dpre;
+                sum.dtb += dpre;
+                sum.A += dg_t * gate_t * A;   // dg/dA_log = g
+            };
+            if (four) {   // lane l sees to step l & 3
+                float total = sum_of_four(ddt, lane);
+                for (int off = 4; off < a.N / 4; off <<= 1) total += __shfl_xor(total, off);
+                leaves(t + (lane & 3), total, pre, gate4, dg);
+            } else {
+                for (int i = 0; i < CV_AHEAD; ++i) {
+                    float total = i == 0 ? ddt[0] : i == 1 ? ddt[1] : i == 2 ? ddt[2] : ddt[3];
+                    if (a.N == 8) total += __shfl_xor(total, 1);
+                    const int64_t at = (row0 + row(t + i)) * a.H + h;
+                    const float p = a.dt_in[at] + dtb;
+                    leaves(t + i, total, p, softplusf(p), a.dg[at]);
+                }
+            }
+        };
+        fetch(t0);
+        int t = t0;
+        for (; t + CV_AHEAD <= t1; t += CV_AHEAD) steps(t, std::true_type{});
+        for (; t < t1 + K - 1; t += CV_AHEAD) steps(t, std::false_type{});
+    }
+}
+
 template <int K> __global__ void __launch_bounds__(CV_THREADS) conv_bwd_kernel(ConvArgs a)
 {
     __shared__ F4 red[CV_WAVES][K + 1][64];
@@ -166,106 +344,23 @@ template <int K> __global__ void __launch_bounds__(CV_THREADS) conv_bwd_kernel(C
     for (int s = 0; s < a.nseg; ++s) ntiles += a.tiles[s];
     int tile = (int)(blockIdx.x % (unsigned)ntiles);
     const int part = (int)(blockIdx.x / (unsigned)ntiles);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int si = segment_of(a, tile);
     const Segment &sg = a.seg[si];
     const int c = (tile * 64 + lane) * 4;
     const bool act = c < sg.C;
-    F4 w[K], bias, dw[K], dbias = F4_ZERO;
-    load_taps<K>(a, sg, c, act, w, bias);
-#pragma unroll
-    for (int j = 0; j < K; ++j) dw[j] = F4_ZERO;
-    const int h = act ? (sg.gated ? c / a.N : sg.skip ? c / a.P : 0) : 0;
-    const float dtb = sg.gated ? a.dt_bias[h] : 0.f, A = sg.gated ? -expf(a.A_log[h]) : 0.f;
-    const float skip_scale = sg.skip ? a.D[h] : 0.f;
-    float acc_dtb = 0.f, acc_A = 0.f, acc_D = 0.f;
-
-    for (int64_t item = (int64_t)part * CV_WAVES + wv; item < a.items; item += (int64_t)a.nparts * CV_WAVES) {
-        const int64_t b = item / a.tiles_t;
-        const int t0 = (int)(item % a.tiles_t) * a.tile_t, t1 = min(a.T, t0 + a.tile_t);
-        const int t2 = min(a.T, t1 + K - 1);   // steps whose ds reaches a row of this tile
-        const int64_t row0 = b * a.T;
-        const float *x = sg.x + row0 * sg.ld + c, *dy = sg.dy + row0 * sg.C + c;
-        const float *skip = sg.skip ? sg.skip + row0 * sg.C + c : nullptr;
-        float *dx = sg.dx + row0 * sg.ld_dx + c;
-        F4 win[K], dwin[K];
-#pragma unroll
-        for (int j = 0; j < K; ++j) dwin[j] = F4_ZERO;
-#pragma unroll
-        for (int j = 0; j < K - 1; ++j) {
-            const int t = t0 - (K - 1) + j;
-            win[j + 1] = act && t >= 0 ? load4(x + t * sg.ld) : F4_ZERO;
-        }
-        F4 xn[CV_AHEAD], yn[CV_AHEAD], kn[CV_AHEAD];
-        float dtn[CV_AHEAD], dgn[CV_AHEAD];
-        auto fetch = [&](int t) {
-#pragma unroll
-            for (int i = 0; i < CV_AHEAD; ++i) {
-                const bool in = act && t + i < t2;
-                xn[i] = in ? load4(x + (t + i) * sg.ld) : F4_ZERO;
-                yn[i] = in ? load4(dy + (int64_t)(t + i) * sg.C) : F4_ZERO;
-                kn[i] = in && skip ? load4(skip + (int64_t)(t + i) * sg.C) : F4_ZERO;
-                const int64_t at = (row0 + t + i) * a.H + h;
-                dtn[i] = in && sg.gated ? a.dt_in[at] : 0.f;
-                dgn[i] = in && sg.gated ? a.dg[at] : 0.f;
-            }
-        };
-        fetch(t0);
-        for (int t = t0; t < t1 + K - 1; t += CV_AHEAD) {
-            F4 xc[CV_AHEAD], yc[CV_AHEAD], kc[CV_AHEAD];
-            float dtc[CV_AHEAD], dgc[CV_AHEAD];
-#pragma unroll
-            for (int i = 0; i < CV_AHEAD; ++i) xc[i] = xn[i], yc[i] = yn[i], kc[i] = kn[i], dtc[i] = dtn[i], dgc[i] = dgn[i];
-            fetch(t + CV_AHEAD);
-#pragma unroll
-            for (int i = 0; i < CV_AHEAD; ++i) {
-                const int ti = t + i;
-                const bool own = ti < t1;   // counts towards the parameters here; later steps count in their own tile
-#pragma unroll
-                for (int j = 0; j + 1 < K; ++j) win[j] = win[j + 1], dwin[j] = dwin[j + 1];
-                win[K - 1] = xc[i];
-                dwin[K - 1] = F4_ZERO;
-                const float pre = dtc[i] + dtb, gate = sg.gated ? softplusf(pre) : 1.f;
-                float ddt = 0.f;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float s = bias.v[e];
-#pragma unroll
-                    for (int j = 0; j < K; ++j) s += w[j].v[e] * win[j].v[e];
-                    const float sg1 = sigmoidf(s), y = s * sg1;
-                    const float up = yc[i].v[e] * gate + kc[i].v[e] * skip_scale;   // gradient of y (rows past the sequence hold zeros)
-                    const float ds = up * sg1 * (1.f + s * (1.f - sg1));
-                    ddt += yc[i].v[e] * y;
-                    if (own) {
-                        acc_D += kc[i].v[e] * y;
-                        dbias.v[e] += ds;
-#pragma unroll
-                        for (int j = 0; j < K; ++j) dw[j].v[e] += ds * win[j].v[e];
-                    }
-#pragma unroll
-                    for (int j = 0; j < K; ++j) dwin[j].v[e] += w[j].v[e] * ds;
-                }
-                if (sg.gated) {   // one head = N / 4 neighbouring lanes
-                    for (int off = a.N / 8; off > 0; off >>= 1) ddt += __shfl_xor(ddt, off);
-                    const float dpre = (ddt + dgc[i] * A) * (pre > 20.f ? 1.f : sigmoidf(pre));
-                    if (own && act && (c % a.N) == 0) {
-                        a.ddt_in[(row0 + ti) * a.H + h] = dpre;
-                        acc_dtb += dpre;
-                        acc_A += dgc[i] * gate * A;   // dg/dA_log = g
-                    }
-                }
-                const int tx = ti - (K - 1);
-                if (act && tx >= t0 && tx < t1) store4(dx + tx * sg.ld_dx, dwin[0]);
-            }
-        }
-    }
+    ConvSums<K> sum{};
+    const int64_t first = (int64_t)part * CV_WAVES + wv;
+    if (sg.gated) conv_bwd_walk<K, GATED>(a, sg, c, act, first, sum);
+    else if (sg.skip) conv_bwd_walk<K, SKIP>(a, sg, c, act, first, sum);
+    else conv_bwd_walk<K, PLAIN>(a, sg, c, act, first, sum);
     // the workgroup's share of the parameters' gradients
 #pragma unroll
-    for (int j = 0; j < K; ++j) red[wv][j][lane] = dw[j];
-    red[wv][K][lane] = dbias;
-    red_h[wv][0][lane] = acc_dtb;
-    red_h[wv][1][lane] = acc_A;
-    red_h[wv][2][lane] = acc_D;
+    for (int j = 0; j < K; ++j) red[wv][j][lane] = sum.dw[j];
+    red[wv][K][lane] = sum.dbias;
+    red_h[wv][0][lane] = sum.dtb;
+    red_h[wv][1][lane] = sum.A;
+    red_h[wv][2][lane] = sum.D;
     __syncthreads();
     if (wv != 0 || !act) return;
     float *out = a.parts + (int64_t)part * a.columns;
@@ -280,13 +375,16 @@ template <int K> __global__ void __launch_bounds__(CV_THREADS) conv_bwd_kernel(C
         }
     if (!a.dt_in) return;
     float s[3] = {0.f, 0.f, 0.f};
-    for (int u = 0; u < CV_WAVES; ++u)
-        for (int m = 0; m < 3; ++m) s[m] += red_h[u][m][lane];
     float *out_h = out + a.C_total * (K + 1);
-    if (sg.gated && (c % a.N) == 0) {
-        out_h[h] = s[0];
-        out_h[a.H + h] = s[1];
+    if (sg.gated && c % a.N == 0) {
+        const int lanes = a.N >= 16 ? 4 : 1;   // of a head that saw to steps
+        for (int u = 0; u < CV_WAVES; ++u)
+            for (int l = lane; l < lane + lanes; ++l)
+                for (int m = 0; m < 2; ++m) s[m] += red_h[u][m][l];
+        out_h[c / a.N] = s[0];
+        out_h[a.H + c / a.N] = s[1];
     }
+    for (int u = 0; u < CV_WAVES; ++u) s[2] += red_h[u][2][lane];
     if (si == 0) out_h[2 * a.H + c / 4] = s[2];
 }
 

@@ -52,6 +52,12 @@ def test_mamba_cell_whole_equals_its_composition(B, T, H, P, N, K):
         assert relerr(a, _np(b)) <= 2e-4, (n, relerr(a, _np(b)))
 
 
+@pytest.mark.parametrize("B,T,H,P,N,K", [(3, 37, 3, 20, 8, 4), (9, 67, 9, 32, 8, 3), (2, 3, 5, 8, 4, 2), (260, 35, 5, 52, 16, 4)])
+def test_mamba_cell_narrow_heads_and_tails(B, T, H, P, N, K):
+    """Heads narrower than the four lanes that share a step's gates, and tiles that end inside a group of four steps."""
+    test_mamba_cell_whole_equals_its_composition(B, T, H, P, N, K)
+
+
 def test_mamba_cell_acting_equals_its_composition():
     from memorax_amd import sequence_models as sm
     torch.manual_seed(3)
