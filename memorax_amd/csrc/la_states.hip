@@ -140,13 +140,15 @@ la_chunk_state_kernel(const T *__restrict__ x, const T *__restrict__ y, const vo
 }
 
 // grid (B * H, d * d / 1024, plus one where z is scanned too): each thread carries four of the d x d state elements through the chunks.  Only the
-// additions are sequential: the slots (and the reset flags) of the next group of eight chunks are
-// requested before the current group is summed and written back, so that one trip to memory is exposed
-// per sequence, not one per group.
+// additions are sequential, so all there is to it is trips to memory: up to 32 slots are on their way at once, each requested as the one 32 before
+// it has been used, and resets and decays of 64 chunks are fetched together -- the flags by all threads, a row each, and kept as one bit per chunk.
+// (32 sequences of 24 chunks of 32 x 32: 7.6 us a scan with groups of eight slots and their flags on their way, 5.5 now; 4 of 512 chunks 62 and 32;
+// 64 of 64 chunks of 64 x 64 26 and 24.)
 // NARROW: narrow heads, the state's size is a run-time value.
 // DECAY: the sum so far enters a chunk without resets times dec[chunk].  Z: the last block of the grid's second axis
 // carries the dk elements of z instead.
-template <bool NARROW, bool DECAY, bool Z>
+// SLOTS: on their way at once, 32 or, where the workgroups already fill the device, 8 (launch_la_state_scan).
+template <bool NARROW, bool DECAY, bool Z, int SLOTS>
 __global__ void __launch_bounds__(256)
 la_state_scan_kernel(float *__restrict__ slots, const float *__restrict__ init, float *__restrict__ fin,
                      const void *__restrict__ done, int done_f32, int Tlen, int H, int NC, int C, int backward, int Qn,
@@ -155,53 +157,72 @@ la_state_scan_kernel(float *__restrict__ slots, const float *__restrict__ init, 
     const bool zpart = Z && blockIdx.y == gridDim.y - 1;
     const int Q = zpart ? zq : NARROW ? Qn : HD * HD / 4;  // f32x4 per state (d_v * d_k / 4)
     if (zpart) slots = zslots, init = zinit, fin = zfin;
-    constexpr int G = 8;            // chunks per group
+    constexpr int G = SLOTS, WINDOW = 64;   // (WINDOW: chunks whose flags are fetched together)
+    __shared__ int sCut[WINDOW];
     const int tid = threadIdx.x, lane = tid & 63;
     const int bh = blockIdx.x, b = bh / H;
     const int idx = (zpart ? 0 : blockIdx.y * 256) + tid;
     const bool act = !(NARROW || Z) || idx < Q;  // a narrow state has fewer elements than the workgroup has threads; the idle lanes
-                                       // still bring their reset flags to the ballots
+                                       // still see to their share of the flags
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    f32x4 S = init && act ? reinterpret_cast<const f32x4 *>(init)[(int64_t)bh * Q + idx] : zero;
-    f32x4 *p = reinterpret_cast<f32x4 *>(slots) + (int64_t)bh * NC * Q + idx;
+    f32x4 *p = reinterpret_cast<f32x4 *>(slots) + (int64_t)bh * NC * Q + (act ? idx : 0);
     auto chunk_of = [&](int s) { return backward ? NC - 1 - s : s; };
-    f32x4 nt[G];
-    uint32_t nd[G];  // raw reset flag of chunk row `lane`
-    float ne[G];     // the chunk's decay
-    auto fetch = [&](int s0) {
+    f32x4 t[G];
+    auto fetch = [&](int u, int s) { t[u] = p[(int64_t)chunk_of(s) * Q]; };
 #pragma unroll
-        for (int u = 0; u < G; ++u) {
-            const int s = s0 + u, c = chunk_of(s);
-            nt[u] = zero;
-            nd[u] = 0u;
-            ne[u] = 1.f;
-            if (s < NC) {  // uniform over the workgroup
-                if (act) nt[u] = p[(int64_t)c * Q];
-                if (DECAY) ne[u] = dec[(int64_t)bh * NC + c];
-                const int tt = c * C + lane;
-                if (lane < C && tt < Tlen) nd[u] = done_raw(done, done_f32, (int64_t)b * Tlen + tt);
-            }
-        }
-    };
-    fetch(0);
+    for (int u = 0; u < G; ++u)
+        if (u < NC) fetch(u, u);
+    f32x4 S = init && act ? reinterpret_cast<const f32x4 *>(init)[(int64_t)bh * Q + idx] : zero;
+    const int shift = 31 - __builtin_clz(C);   // (chunks are powers of two)
+    uint64_t cuts = 0;   // of the window's chunks, by the order they are walked in
+    float decays = 0.f;  // lane l: that of the window's chunk l
     for (int s0 = 0; s0 < NC; s0 += G) {
-        f32x4 t[G];
-        bool cut[G];
-        float e[G];
+        if (s0 % WINDOW == 0) {
+            const int n = NC - s0 < WINDOW ? NC - s0 : WINDOW;   // chunks of the window, from its first row on
+            const int row0 = (backward ? NC - s0 - n : s0) * C, row1 = row0 + n * C < Tlen ? row0 + n * C : Tlen;
+            if constexpr (DECAY) decays = dec[(int64_t)bh * NC + chunk_of(s0 + (lane < n ? lane : n - 1))];
+            if (s0) __syncthreads();   // (the window before has been read)
+            if (tid < WINDOW) sCut[tid] = 0;
+            __syncthreads();
+            for (int r0 = row0 + tid; r0 < row1; r0 += 8 * 256) {
+                uint32_t flag[8];
+                if (done_f32) {
 #pragma unroll
-        for (int u = 0; u < G; ++u) {
-            t[u] = nt[u];
-            e[u] = ne[u];
-            cut[u] = __ballot(done_test(nd[u], done_f32)) != 0ull;
-        }
-        if (s0 + G < NC) fetch(s0 + G);
+                    for (int i = 0; i < 8; ++i) flag[i] = done_raw(done, 1, (int64_t)b * Tlen + (r0 + i * 256 < row1 ? r0 + i * 256 : r0));
+                } else {
 #pragma unroll
-        for (int u = 0; u < G; ++u) {
-            const int s = s0 + u;
-            if (s < NC) {
-                if (act) p[(int64_t)chunk_of(s) * Q] = S;
-                S = cut[u] ? t[u] : DECAY ? e[u] * S + t[u] : S + t[u];
+                    for (int i = 0; i < 8; ++i) flag[i] = done_raw(done, 0, (int64_t)b * Tlen + (r0 + i * 256 < row1 ? r0 + i * 256 : r0));
+                }
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const int r = r0 + i * 256 < row1 ? r0 + i * 256 : r0, c = (r - row0) >> shift;
+                    if (done_test(flag[i], done_f32)) sCut[backward ? n - 1 - c : c] = 1;
+                }
             }
+            __syncthreads();
+            cuts = __ballot(sCut[lane] != 0);
+        }
+        auto step = [&](int u) {
+            const int s = s0 + u;
+            if (act) p[(int64_t)chunk_of(s) * Q] = S;
+            float e = 1.f;
+            if constexpr (DECAY) e = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, decays), s % WINDOW));
+            const uint32_t cut = -(uint32_t)(cuts >> (s % WINDOW) & 1);
+            S = DECAY ? e * S + t[u] : S + t[u];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)   // (selected by bits: a branch per chunk costs more than the sum)
+                S[i] = __builtin_bit_cast(float, (__builtin_bit_cast(uint32_t, (float)t[u][i]) & cut) | (__builtin_bit_cast(uint32_t, (float)S[i]) & ~cut));
+        };
+        if (s0 + G <= NC) {
+#pragma unroll
+            for (int u = 0; u < G; ++u) {
+                step(u);
+                fetch(u, s0 + G + u < NC ? s0 + G + u : NC - 1);
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < G; ++u)
+                if (s0 + u < NC) step(u);
         }
     }
     if (fin && act) reinterpret_cast<f32x4 *>(fin)[(int64_t)bh * Q + idx] = S;
@@ -242,6 +263,9 @@ int launch_la_chunk_states(hipStream_t st, const void *x, const void *y, const v
     return launch_states<float, 32>(st, x, y, done, done_f32, slots, B, Tlen, H, fmap, backward, dk, dv, a);
 }
 
+// 32 slots on their way take a compute unit's registers for one workgroup: up to one of those per compute unit (16 sequences x 8 heads x 16 chunks
+// of 64 x 64, 512 workgroups: 14 us with 32, 11 with 8), and from 16 chunks on (10 chunks: 4.5 and 4.3 us).
+constexpr int64_t SCAN_FEW = 256, SCAN_LONG = 16;
 int launch_la_state_scan(hipStream_t st, float *slots, const float *init, float *fin, const void *done, int done_f32,
                          int64_t B, int64_t Tlen, int64_t H, int C, bool backward, int64_t dk, int64_t dv, const LaStateArgs &a)
 {
@@ -249,10 +273,14 @@ int launch_la_state_scan(hipStream_t st, float *slots, const float *init, float 
     if (B * H > 0x7fffffffLL) return MRX_ERR_INVALID_ARG;
     const int Q = (int)(dk * dv / 4);
     const dim3 grid((unsigned)(B * H), (unsigned)((Q + 255) / 256 + (a.z ? 1 : 0)));
+    auto scan = [&](auto narrow, auto decay, auto z, auto slots_ahead) {
+        return launch_kernel(la_state_scan_kernel<decltype(narrow)::value, decltype(decay)::value, decltype(z)::value, decltype(slots_ahead)::value>,
+                             grid, dim3(256), 0, st, slots, init, fin, done, done_f32, (int)Tlen, (int)H, (int)NC, C, backward ? 1 : 0, Q,
+                             (const float *)a.dec, a.z, a.z_init, a.z_fin, (int)(dk / 4));
+    };
     auto go = [&](auto narrow, auto decay, auto z) {
-        return launch_kernel(la_state_scan_kernel<decltype(narrow)::value, decltype(decay)::value, decltype(z)::value>, grid, dim3(256), 0, st,
-                             slots, init, fin, done, done_f32, (int)Tlen, (int)H, (int)NC, C, backward ? 1 : 0, Q, (const float *)a.dec, a.z,
-                             a.z_init, a.z_fin, (int)(dk / 4));
+        return (int64_t)grid.x * grid.y <= SCAN_FEW && NC >= SCAN_LONG ? scan(narrow, decay, z, std::integral_constant<int, 32>{})
+                                                    : scan(narrow, decay, z, std::integral_constant<int, 8>{});
     };
     auto variant = [&](auto narrow) {
         if (a.dec) return go(narrow, std::true_type{}, std::false_type{});

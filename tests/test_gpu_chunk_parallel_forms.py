@@ -125,6 +125,33 @@ def test_normalised(shape, dtype, ss, p, carries):
     _compare(got, own, yard)
 
 
+LONG = [(2, 1, 32, 64, 16.0), (1, 2, 64, 64, 31.6), (1, 1, 48, 32, 33.0), (2, 1, 64, 64, 64.0), (1, 2, 32, 32, 65.1), (1, 1, 64, 48, 129.4),
+        (16, 8, 64, 64, 16.5)]
+
+
+@pytest.mark.parametrize("p", [0.0, 0.002])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("shape", LONG)
+def test_long_scans_of_the_state(shape, dtype, p):
+    """As many chunks as slots are on their way (32, and 8 where there are many sequences) or share their flags (64), and a few more.  A slot
+    or a flag of the wrong chunk errs by the size of the result; bfloat16 operands of up to three products in a row (2^-9 each, of either sign)
+    and float32 sums of up to 4200 terms (2^-24 sqrt(4200) = 4e-6) by less than the bounds.  (The normalised dq is a difference of nearly equal
+    sums, which bfloat16's rounding has no such bound for.)"""
+    print(f"case long scans {shape} {dtype} {p}", flush=True)
+    q, k, v, gate, do, done, S0, z0, dS, dz, _ = _inputs(shape, dtype, p, True, 9)
+    for normalise in (False, True) if dtype == "f32" else (False,):
+        leaves = [t.detach().requires_grad_() for t in ((q, k, v, S0, z0) if normalise else (q, k, v, gate, S0))]
+        cotangents = (do, dS, dz) if normalise else (do, dS)
+        if normalise:
+            yard = _exact_with_gradients((q, k, v, None, S0, z0), done, "elu1", True, cotangents)
+            out = Fn.normalised_linear_attention(*leaves[:3], done, *leaves[3:], "elu1")[:3]
+        else:
+            yard = _exact_with_gradients((q, k, v, gate, S0, None), done, "elu1", False, cotangents)
+            out = Fn.gated_linear_attention(*leaves[:4], done, leaves[4], "elu1")
+        for x, y in zip((*out, *torch.autograd.grad(out, leaves, cotangents)), sum(yard, [])):
+            assert _distance(x, y) <= (1e-2 if dtype == "bf16" else 1e-5), (normalise, tuple(x.shape), _distance(x, y))
+
+
 @pytest.mark.parametrize("form", ["gated", "normalised"])
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 def test_what_lies_before_a_reset_reaches_nothing_after_it(form, dtype):
