@@ -1,7 +1,7 @@
 // Dense layers over many rows in bfloat16, forward and with respect to their input:
 //
 //     y_l = x W_l^T + b_l          up to three layers of one width that read the same rows, and one of up to eight outputs beside them
-//     y   = x_res + (x W^T + b)    the layer that closes a residual branch of a float32 stream, its sum unrounded
+//     y   = x_res + (x W^T + b)    the layer that closes a residual branch of a float32 stream; its own result is rounded first, as by itself
 //     dx  = sum_l dy_l W_l         of such a group, or of one layer whose gradient is float32 (the stream's; its rounded copy, which the
 //                                  parameters' gradients read, is a by-product)
 //
@@ -211,7 +211,9 @@ __global__ void __launch_bounds__(DR_THREADS, 1) dense_rows_kernel(DenseRowsArgs
                 for (int j = 0; j < NT; ++j) {
                     const int q = (wv * 16 * NT + 4 * NT * g) / 4 + j;
                     const f32x4 x = *reinterpret_cast<const f32x4 *>(tile + SEGS * Tile::SEG + (16 * m + i) * (RC * 4) + (q ^ swz<RSPR>(16 * m + i)) * 16);
-                    *reinterpret_cast<f32x4 *>(static_cast<float *>(a.y[l]) + r * a.n + col + 4 * j) = x + (acc[m][j] + bias[j]);
+                    const f32x4 z = acc[m][j] + bias[j];
+                    const bf16x4 y = TT<__bf16>::pack(z[0], z[1], z[2], z[3]);
+                    *reinterpret_cast<f32x4 *>(static_cast<float *>(a.y[l]) + r * a.n + col + 4 * j) = x + f32x4{(float)y[0], (float)y[1], (float)y[2], (float)y[3]};
                 }
             } else {
                 bf16x4 p[NT];

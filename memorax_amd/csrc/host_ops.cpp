@@ -1987,8 +1987,8 @@ std::vector<Tensor> dense_group(const Tensor &x, const std::vector<Tensor> &weig
     return out;
 }
 
-// residual + dense(x): the layer that closes a residual branch of a float32 stream, under autocast or in bfloat16 as one launch, the sum
-// in float32 and unrounded between; the array library's sum of a layer's output otherwise.
+// residual + dense(x): the layer that closes a residual branch of a float32 stream, under autocast or in bfloat16 as one launch: the
+// layer's own result rounded to bfloat16, the sum in float32, as one after the other; the array library's sum of a layer's output otherwise.
 Tensor dense_onto(const Tensor &residual, const Tensor &x, const Tensor &weight, const OptTensor &bias)
 {
     auto composed = [&]() {

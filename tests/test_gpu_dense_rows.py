@@ -76,7 +76,8 @@ def test_the_layer_that_closes_a_residual_branch(rows, K, n):
     y = torch.full((rows + 3, n), 7.0, device="cuda")
     assert lib.mrx_dense_rows(_stream(), x.data_ptr(), _ptrs([w]), _ptrs([b]), _ptrs([y]), ns, 1, res.data_ptr(), rows, K, _lib.MRX_BF16) == 0
     terms = (K + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t() + b.double().abs() + res.double().abs())
-    _rounded(y[:rows], res.double() + x.double() @ w.double().t() + b.double(), terms, 2.0 ** -23)
+    branch = x.double() @ w.double().t() + b.double()
+    _rounded(y[:rows], res.double() + branch, terms + 2.0 ** -8 * branch.abs(), 2.0 ** -23)   # (the branch's result is bfloat16)
     assert (y[rows:] == 7.0).all()
     # backward: the stream's gradient is float32, its rounded copy what the products read
     dy, wt = rnd(rows, n), w.t().contiguous()
@@ -97,8 +98,8 @@ def _block(kind, F, H, d):
 @pytest.mark.parametrize("kind", ["delta", "attention", "recurrence"])
 @pytest.mark.parametrize("B,T,F,H,d", [(3, 7, 64, 2, 32), (5, 40, 128, 2, 64), (2, 33, 256, 4, 64), (2, 20, 96, 2, 16)])
 def test_residual_blocks_close_with_their_sum(kind, B, T, F, H, d):
-    """The block with its last layer and the residual sum as one operation, against the composition (which a hook brings back): the
-    branch is rounded to bfloat16 once less, 2^-8 of it, in the result and in each gradient; 96 features take the composition."""
+    """The block with its last layer and the residual sum as one operation, against the composition (which a hook brings back): another
+    order of the products' sums, which bfloat16 rounds 2^-8 apart, in the result and in each gradient; 96 features take the composition."""
     torch.manual_seed(F)
     print(f"case block {kind} {B} {T} {F}", flush=True)
     block = _block(kind, F, H, d)
