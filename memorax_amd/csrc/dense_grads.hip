@@ -7,8 +7,8 @@
 // library runs them as a product per layer and direction -- with the rows cut into slices by hand, a reduction per layer over
 // those, a reduction per bias, and the sum of the input gradients rounded and read back between the layers -- most of them at a
 // fraction of the bandwidth (131072 rows, three layers of 256 x 256 and one of 256 x 4 in bfloat16: 330 us for the parameters and 150 us
-// for the input; 11455 rows, three of 128 x 256: 225 and 23 us).  Here they are two launches and one reduction: 134 and 118 us, 24 and
-// 16 us.  At 256 features a compute unit is short of loads in flight rather than of bandwidth: LDS holds two steps of two workgroups.
+// for the input; 11455 rows, three of 128 x 256: 225 and 23 us).  Here they are two launches and one reduction: 104 (on wide tiles, below; 134 on the others) and
+// 118 us, 24 and 16 us; the input's gradient in bfloat16 over wide rows is dense_rows.hip's (60 us), the kernel here serves the rest.  At 256 features a compute unit is short of loads in flight rather than of bandwidth: LDS holds two steps of two workgroups.
 //
 // Weight gradients: a workgroup of four waves owns a TN x TK tile of one layer's result and a slice of the rows, 64 (float32: 32)
 // of which wait in LDS while the next are on their way; both operands are contracted over their rows, which the transposing

@@ -1,8 +1,8 @@
 """Dense layers of the host-side mirror (flax.linen.Dense in the reference's cells and blocks,
 e.g. linear_attention.py:62-80, min_gru.py:49-62, blocks/ffn.py:11-123).
 
-The forward products stay the array library's; the gradients are the library's own kernels
-(csrc/dense_grads.hip) up to the widths where those of the array library take over, and there what this
+In bfloat16 over many rows the products are the library's own kernels (csrc/dense_rows.hip), and so are the
+gradients (csrc/dense_grads.hip) up to the widths where those of the array library take over; there what this
 module changes is their shape.  A rollout batch
 has a hundred thousand rows and a few hundred features, so the weight gradient ``dy^T x`` is a
 product with a tiny result and an enormous inner dimension, which the library's GEMM runs on as
