@@ -151,6 +151,10 @@ int mrx_linear_scan_bwd(void *stream, const void *a, const void *h,
                         int64_t B, int64_t T, int64_t D, int dtype,
                         int done_dtype, int a_time_invariant);
 
+/* out[c] = sum over the rows of x (rows, columns), float32, in a fixed order: what is left to do for the gradient of a
+ * broadcast coefficient (a complex one as two columns). */
+int mrx_column_sum(void *stream, const float *x, float *out, int64_t rows, int64_t columns);
+
 /* Long sequences over few columns leave most of the device idle when one workgroup walks each of them.  Where
  * mrx_scan_workspace gives a size (bytes; 0: the shape is not served this way), the _segmented forms -- same
  * arguments, same results -- take a workspace of that size, 8-byte aligned and overwritten, and cut time into

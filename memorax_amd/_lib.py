@@ -33,6 +33,7 @@ SIGNATURES = {
     "mrx_delta_chunk_size": (_L, [_I]),
     "mrx_linear_scan_fwd": (_I, [_P] * 9 + [_L] * 3 + [_I] * 3),
     "mrx_linear_scan_bwd": (_I, [_P] * 10 + [_L] * 3 + [_I] * 3),
+    "mrx_column_sum": (_I, [_P] * 3 + [_L] * 2),
     "mrx_scan_workspace": (_L, [_L] * 3 + [_I] * 2),
     "mrx_linear_scan_fwd_segmented": (_I, [_P] * 9 + [_L] * 3 + [_I] * 3 + [_P]),
     "mrx_linear_scan_bwd_segmented": (_I, [_P] * 10 + [_L] * 3 + [_I] * 3 + [_P]),

@@ -40,7 +40,7 @@ using torch::autograd::variable_list;
 
 // ------------------------------------------------------------------------------------------------ entry points
 #define MRX_BOUND(X)                                                                                                 \
-    X(mrx_status_string) X(mrx_chunk_size) X(mrx_delta_chunk_size) X(mrx_scan_workspace) X(mrx_linear_scan_fwd_segmented) X(mrx_linear_scan_bwd_segmented)     \
+    X(mrx_status_string) X(mrx_chunk_size) X(mrx_delta_chunk_size) X(mrx_scan_workspace) X(mrx_column_sum) X(mrx_linear_scan_fwd_segmented) X(mrx_linear_scan_bwd_segmented)     \
     X(mrx_linear_scan_last) X(mrx_mingru_scan_fwd_segmented) X(mrx_mingru_scan_bwd_segmented) X(mrx_mlstm_gates_fwd)                     \
     X(mrx_mlstm_gates_bwd) X(mrx_rms_norm_fwd) X(mrx_rms_norm_bwd) X(mrx_layer_norm_fwd) X(mrx_layer_norm_bwd)       \
     X(mrx_silu_gate_fwd) X(mrx_silu_gate_bwd) X(mrx_residual_add) X(mrx_linear_attn_fwd) X(mrx_linear_attn_bwd)                          \
@@ -1085,6 +1085,20 @@ Tensor as(const Tensor &t, ScalarType dt) { return t.defined() ? t.to(dt).contig
 Tensor grad_or_zeros(const Tensor &g, const Tensor &like) { return g.defined() ? g.contiguous() : at::zeros_like(like); }
 Tensor unless(bool skip, const Tensor &t) { return skip ? Tensor() : t; }
 
+// The sum over the rows of a (B,D) float32 or complex64 array: one launch of the library's column sum up to 512 rows (64 x 184 4.1 and 1.9 us, complex64
+// 192 x 184 5.6 and 2.1, 512 x 256 8.4 and 2.8).  Beyond, its chains of sums grow longer than the array library's: 2048 x 64 errs by 1.4e-7
+// and 1.1e-7 against float64, 512 x 64 by 0.9e-7 and 1.0e-7.
+constexpr int64_t SUM_ROWS = 512;
+Tensor sum_rows(const Tensor &x)
+{
+    const bool complex = x.scalar_type() == at::kComplexFloat;
+    if ((!complex && x.scalar_type() != at::kFloat) || x.numel() == 0 || x.size(0) > SUM_ROWS) return x.sum(0);
+    const Tensor out = fresh({x.size(1)}, x.scalar_type(), x);
+    check(lib.mrx_column_sum(stream(), static_cast<const float *>(ptr(x)), static_cast<float *>(ptr(out)), x.size(0), x.size(1) * (complex ? 2 : 1)),
+          "mrx_column_sum");
+    return out;
+}
+
 struct LinearScanOp {
     static constexpr int SAVED = 3;   // a, h, h0
     static const char *name() { return "MemoraxLinearScanBackward"; }
@@ -1095,7 +1109,7 @@ struct LinearScanOp {
         const bool ti = a.dim() == 1;   // a broadcast coefficient: the kernel sums its gradient over time, the rest is (B,D)
         auto r = scan_bwd(a, h, done, some(s[2]), grad_or_zeros(grads[0], h), some(as(grads[1], s[2].defined() ? s[2].scalar_type() : carry(h))),
                           ti);
-        if (ti && node.wants(0)) r.da = r.da.sum(0).to(a.scalar_type());
+        if (ti && node.wants(0)) r.da = sum_rows(r.da).to(a.scalar_type());
         return {unless(!node.wants(0), r.da), unless(!node.wants(1), r.db), unless(!node.wants(2), r.dh0)};
     }
     static ScalarType carry(const Tensor &h) { return h.scalar_type() == at::kBFloat16 ? at::kFloat : h.scalar_type(); }

@@ -13,6 +13,7 @@
 #include <initializer_list>
 #include <type_traits>
 
+#include "col_sum.h"
 #include "common.h"
 #include "mingru.h"
 
@@ -1826,4 +1827,12 @@ extern "C" int mrx_mingru_step(void *stream, const void *z, const void *h_tilde,
     using Four = std::integral_constant<int, 4>;
     if (dtype == MRX_BF16) return quads ? go(__bf16(), Four{}) : go(__bf16(), One{});
     return quads ? go(float(), Four{}) : go(float(), One{});
+}
+
+extern "C" int mrx_column_sum(void *stream, const float *x, float *out, int64_t rows, int64_t columns)
+{
+    using namespace mrx;
+    if (!x || !out || rows <= 0 || columns <= 0 || rows >= (1ll << 31) || columns >= (1ll << 31)) return MRX_ERR_INVALID_ARG;
+    if (const int rc = prepare_device(); rc != MRX_OK) return rc;
+    return launch_column_sum((hipStream_t)stream, x, out, nullptr, (int)rows, (int)columns);
 }
