@@ -88,6 +88,25 @@ def test_the_layer_that_closes_a_residual_branch(rows, K, n):
     _rounded(dx[:rows], d @ w.double(), n * 2.0 ** -24 * (d.abs() @ w.double().abs()))
 
 
+def _rows_past_the_counted_wait():
+    """A workgroup's first tiles wait for its requests alone; from the tile on that reuses the ring's first place (the eighth of at most 64
+    rows) its stores are counted among them.  Every workgroup -- one a compute unit -- gets so far, some of them two tiles farther."""
+    return 64 * 8 * torch.cuda.get_device_properties(0).multi_processor_count + 64 * 300 + 37
+
+
+@pytest.mark.parametrize("K", [64, 128, 256])
+@pytest.mark.parametrize("n", [64, 128, 256])
+@pytest.mark.parametrize("wide,narrow", [(1, 0), (2, 0), (3, 0), (3, 4)])
+def test_every_forward_and_input_gradient_past_the_counted_wait(K, n, wide, narrow):
+    test_forward_and_input_gradient(_rows_past_the_counted_wait(), K, [n] * wide + [narrow] * (narrow > 0), True)
+
+
+@pytest.mark.parametrize("K", [64, 128, 256])
+@pytest.mark.parametrize("n", [64, 128, 256])
+def test_every_closing_layer_past_the_counted_wait(K, n):
+    test_the_layer_that_closes_a_residual_branch(_rows_past_the_counted_wait(), K, n)
+
+
 def _block(kind, F, H, d):
     from memorax_amd import sequence_models as sm
     model = {"delta": lambda: sm.Memoroid(sm.DeltaNetCell(F, d, H)), "attention": lambda: sm.Memoroid(sm.LinearAttentionCell(F, d, H)),
