@@ -809,6 +809,27 @@ template <typename... Ts> void refuse(const Ts &...ts) requires(sizeof...(Ts) > 
     (refuse(ts), ...);
 }
 
+// What an acting call reads and writes lies on the GPU of its rows: a layer left on the host, or on another GPU, is an error and no address.
+void chk_beside(const Tensor &x, const Tensor &t)
+{
+    if (!t.defined()) return;
+    TORCH_CHECK_VALUE(t.is_cuda(), "parameters and carries must live on the GPU (memorax_amd has no CPU path)");
+    TORCH_CHECK_VALUE(t.device() == x.device(), "parameters and carries must live on the GPU of the rows, ", x.device(), ", got ", t.device());
+}
+void chk_beside(const Tensor &x, const OptTensor &t)
+{
+    if (t.has_value()) chk_beside(x, *t);
+}
+template <typename T> void chk_beside(const Tensor &x, const std::vector<T> &ts)
+{
+    for (const T &t : ts) chk_beside(x, t);
+}
+template <typename... Ts> void chk_beside(const Tensor &x, const Ts &...ts) requires(sizeof...(Ts) > 1)
+{
+    TORCH_CHECK_VALUE(x.is_cuda(), "x must live on the GPU (memorax_amd has no CPU path)");
+    (chk_beside(x, ts), ...);
+}
+
 // norm: 0 none, 1 RMS, 2 layer norm.  The results keep x's leading axes; residual (float32, x's leading axes): added to the one
 // layer's result.
 std::vector<Tensor> row_dense(const Tensor &x_, int norm, const OptTensor &scale_, const OptTensor &nbias_, double eps, bool round_norm,
@@ -817,6 +838,7 @@ std::vector<Tensor> row_dense(const Tensor &x_, int norm, const OptTensor &scale
                               Tensor *skip_out = nullptr)
 {
     refuse(x_, scale_, nbias_, weights, biases, residual_, weight2_, skip_);
+    chk_beside(x_, scale_, nbias_, weights, biases, residual_, weight2_, skip_);
     const Tensor x = dense16(x_), scale = norm_param(scale_), nbias = norm_param(nbias_), weight2 = dense16(weight2_), skip = dense16(skip_),
                  residual = residual_.has_value() ? residual_->contiguous() : Tensor();
     for (Tensor &w : weights) w = dense16(w);
@@ -867,6 +889,7 @@ std::tuple<Tensor, Tensor, Tensor> lru_act(const Tensor &x, int norm, const OptT
 {
     TORCH_CHECK_VALUE(x.dim() == 3 && x.size(1) == 1 && params.size() == 8, "lru_act takes one time step");
     refuse(x, scale, nbias, params, done_, h_, P_);
+    chk_beside(x, scale, nbias, params, done_, h_, P_);
     const int64_t B = x.size(0), N = params[0].size(0);
     for (Tensor &t : params) t = dense16(t);
     for (int i = 0; i < 3; ++i) chk(params[i], "parameter", at::kFloat, {N});
@@ -891,6 +914,7 @@ std::vector<Tensor> mlstm_act(const Tensor &x, int norm, const OptTensor &scale,
 {
     TORCH_CHECK_VALUE(x.dim() == 3 && x.size(1) == 1 && p.size() == 13 && carry.size() == 4, "mlstm_act takes one time step");
     refuse(x, scale, nbias, p, done_, carry);
+    chk_beside(x, scale, nbias, p, done_, carry);
     const int64_t B = x.size(0), H = p[3].size(0), D = p[3].size(1), W = H * D, K = p[1].size(2);
     for (Tensor &t : p) t = dense16(t);
     chk(p[1], "conv weight", at::kFloat, {W, 1, K});
@@ -921,6 +945,7 @@ std::tuple<Tensor, Tensor, Tensor> mingru_step(const Tensor &z, const Tensor &x,
 {
     TORCH_CHECK_VALUE(z.dim() == 3 && z.size(1) == 1, "mingru_step takes one time step");
     refuse(z, x, gate, done_, log_state, log_decay);
+    chk_beside(z, x, gate, done_, log_state, log_decay);
     const int64_t B = z.size(0), D = z.size(2);
     const auto dt = z.scalar_type();
     chk_scan_dtype(dt, false, "mingru_step");
@@ -946,6 +971,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> gated_act(const Tensor &x, int norm, 
 {
     TORCH_CHECK_VALUE(x.dim() == 3 && x.size(1) == 1 && weights.size() == 4 && biases.size() == 4, "gated_act takes one time step");
     refuse(x, scale, nbias, weights, biases, done_, log_state, log_decay);
+    chk_beside(x, scale, nbias, weights, biases, done_, log_state, log_decay);
     const int64_t B = x.size(0), K = x.size(2), N = weights[0].size(0);
     auto fits = [](const Tensor &t) { return t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
     const auto wd = weights[0].scalar_type();
@@ -988,6 +1014,7 @@ std::tuple<Tensor, Tensor, OptTensor> state_act(const Tensor &x, int norm, const
     TORCH_CHECK_VALUE(x.dim() == 3 && x.size(1) == 1 && weights.size() == (z.has_value() ? 4u : 5u) && biases.size() == weights.size() && S.dim() == 5,
                       "state_act takes one time step");
     refuse(x, scale, nbias, weights, biases, out_scale, done, S, z);
+    chk_beside(x, scale, nbias, weights, biases, out_scale, done, S, z);
     const int64_t B = x.size(0), H = S.size(2), D = S.size(3);
     const Tensor out_w = weights.back();
     const OptTensor out_b = biases.back();

@@ -3,6 +3,7 @@ import pytest
 import torch
 
 from memorax_amd import sequence_models as sm
+from memorax_amd._lib import native
 
 pytestmark = pytest.mark.gpu
 
@@ -82,3 +83,27 @@ def test_blocks_wider_than_the_row_kernel_act_on_their_composition(cell):
         y = block(x, done)[1]
     want = block(x, done)[1]
     torch.testing.assert_close(y, want, rtol=0, atol=1e-5 * float(want.detach().abs().max()))
+
+
+@pytest.mark.parametrize("part", ["cell.z", "cell.h", "gate", "out"])
+@pytest.mark.parametrize("first", [False, True])
+@pytest.mark.parametrize("autocast", [False, True])
+def test_a_layer_left_on_the_host_is_an_error(part, first, autocast):
+    """Before a launch has its address; the first step (no carry yet) and one that carries on."""
+    block = sm.Residual(sm.PreNorm(sm.GatedLinearRecurrence(64), 64)).cuda()
+    carry = None if first else block.initialize_carry(None, (6, 64))
+    block.module.module.get_submodule(part).cpu()
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+        with pytest.raises(ValueError, match="must live on the GPU"):
+            block(torch.randn(6, 1, 64, device="cuda"), torch.zeros(6, 1, dtype=torch.bool, device="cuda"), carry)
+
+
+@pytest.mark.parametrize("at", ["scale", "weight", "closing weight", "bias", "done", "log_state", "log_decay"])
+def test_whatever_a_gated_step_reads_is_on_its_gpu(at):
+    x, done, ones = torch.randn(6, 1, 64, device="cuda"), torch.zeros(6, 1, device="cuda"), torch.ones(64, device="cuda")
+    ws, bs, state = [torch.randn(64, 64, device="cuda") for _ in range(4)], [None] * 4, torch.zeros(6, 1, 64, device="cuda")
+    host = lambda t, name: t.cpu() if at == name else t  # noqa: E731
+    ws[1], ws[3], bs[0] = host(ws[1], "weight"), host(ws[3], "closing weight"), ones.cpu() if at == "bias" else None
+    with torch.no_grad(), pytest.raises(ValueError, match="must live on the GPU"):
+        native().gated_act(x, 1, host(ones, "scale"), None, 1e-6, ws, bs, torch.float32, host(done, "done"), host(state, "log_state"),
+                           host(state.clone(), "log_decay"), False)
