@@ -2226,12 +2226,15 @@ std::tuple<Tensor, Tensor, Tensor> mamba_mix(const Tensor &up, const Tensor &b_i
     return {y, S_last, decay_last};
 }
 
-// Whether a hook waits in a torch module or below it.  An acting step asks on every call: from Python the walk over the eighteen
-// modules of a small block pair takes 7 us of a step of 88.
+// Whether a hook waits in a torch module or below it, or one of the methods that fused operations stand for was replaced on an instance (as
+// adapters and accelerators do).  An acting step asks on every call: from Python the walk over the eighteen modules of a small block pair
+// takes 7 us of a step of 88.
 bool any_hook(PyObject *module)
 {
     static PyObject *const hooks[] = {PyUnicode_InternFromString("_forward_hooks"), PyUnicode_InternFromString("_forward_pre_hooks"),
                                       PyUnicode_InternFromString("_backward_hooks"), PyUnicode_InternFromString("_backward_pre_hooks")};
+    static PyObject *const methods[] = {PyUnicode_InternFromString("forward"), PyUnicode_InternFromString("scan"),
+                                        PyUnicode_InternFromString("read"), PyUnicode_InternFromString("elements")};
     static PyObject *const children = PyUnicode_InternFromString("_modules");
     PyObject **const at = _PyObject_GetDictPtr(module);
     if (!at || !*at) return false;   // None, or no torch module
@@ -2239,6 +2242,8 @@ bool any_hook(PyObject *module)
         PyObject *const held = PyDict_GetItem(*at, name);
         if (held && PyDict_Check(held) && PyDict_Size(held) > 0) return true;
     }
+    for (PyObject *name : methods)
+        if (PyDict_GetItem(*at, name)) return true;
     PyObject *const below = PyDict_GetItem(*at, children);
     if (!below || !PyDict_Check(below)) return false;
     PyObject *key, *child;

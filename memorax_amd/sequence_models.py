@@ -501,7 +501,8 @@ def _row_layers(x, layers):
 
 
 def _hooked(module):
-    """Whether a hook waits in this module or below, or for every module: fused operations do not run the modules they stand for."""
+    """Whether a hook waits in this module or below, or for every module, or an instance has a ``forward`` (``scan``, ``read``,
+    ``elements``) of its own: fused operations do not run the modules they stand for."""
     return _any_global_hook() or native().any_hook(module)
 
 

@@ -51,6 +51,24 @@ def test_a_hook_runs(cell):
     assert seen
 
 
+PARTS = {"lru": ["", "cell"], "mamba": ["", "cell", "cell.output_projection"], "mlstm": ["", "cell", "cell.output_projection"],
+         "linear_attention": ["", "cell.norm", "cell.output_projection"], "delta": ["", "cell.output_projection"], "recurrence": ["", "out"]}
+
+
+@pytest.mark.parametrize("T,grad", [(1, False), (5, False), (5, True)])
+@pytest.mark.parametrize("cell,part,autocast", [(c, p, a) for c in sorted(PARTS) for p in PARTS[c] for a in (False, True)
+                                                if not (a and c == "mamba")])   # (float32 only)
+def test_a_forward_set_on_an_instance_runs(cell, part, autocast, T, grad):
+    """As adapters and accelerators set it: on a layer, a cell or the sequence model, acting and over sequences."""
+    block = _block(cell) if cell in CELLS else sm.Residual(sm.PreNorm(sm.GatedLinearRecurrence(64), 64)).cuda()
+    m, seen = block.module.module.get_submodule(part), []
+    own = m.forward
+    m.forward = lambda *a, **k: seen.append(1) or own(*a, **k)
+    with torch.set_grad_enabled(grad), torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+        block(torch.randn(6, T, 64, device="cuda"), torch.zeros(6, T, dtype=torch.bool, device="cuda"))
+    assert seen
+
+
 @pytest.mark.parametrize("dual", ["input", "parameter", "carry"])
 @pytest.mark.parametrize("cell", [*sorted(CELLS), "recurrence"])
 def test_an_acting_block_refuses_tangents(cell, dual):

@@ -86,6 +86,18 @@ def test_hooks_are_seen_at_any_depth(kind):
     handle.remove()
 
 
+@pytest.mark.parametrize("part,method", [("", "forward"), ("module", "forward"), ("norm", "forward"), ("module.cell", "forward"), ("module.cell", "scan"),
+                                         ("module.cell", "read"), ("module.cell.output_projection", "forward")])
+def test_a_method_set_on_an_instance_is_seen_at_any_depth(part, method):
+    block = sm.PreNorm(sm.Memoroid(sm.LinearAttentionCell(8, 4, 2)), 8)
+    assert not sm._hooked(block)
+    m = block.get_submodule(part)
+    setattr(m, method, getattr(m, method))
+    assert sm._hooked(block)
+    delattr(m, method)
+    assert not sm._hooked(block)
+
+
 def test_a_replaced_part_is_no_row_layer():
     class Wrapped(Dense):
         def forward(self, x):
