@@ -194,6 +194,8 @@ class Memoroid(SequenceModel):
         return next_carry, native().dense_onto(residual, rows, layer.weight, layer.bias)
 
     def acting(self, x, norm, done, carry):
+        if type(self).forward is not Memoroid.forward:
+            return None
         return self.cell.acting(x, norm, done, self.cell.initialize_carry(None, get_input_shape(x)) if carry is None else carry)
 
     def initialize_carry(self, key, input_shape):
@@ -465,7 +467,8 @@ class GatedLinearRecurrence(SequenceModel):
 
     def acting(self, x, norm, done, carry):
         layers = [self.cell.z, self.cell.h, self.gate]
-        if not (type(self).forward is GatedLinearRecurrence.forward and self.cell.fused and _row_layers(x, [*layers, self.out])):
+        if not (type(self).forward is GatedLinearRecurrence.forward and _as_written(self.cell, MinGRUCell, "scan", "elements") and self.cell.fused
+                and _row_layers(x, [*layers, self.out])):
             return None
         if carry is None:
             carry = self.cell.initialize_carry(None, get_input_shape(x))
@@ -529,9 +532,9 @@ def _rows(x, norm, layers, product, out_dtype, residual=None):
                               out_dtype, residual)
 
 
-def _as_written(cell, cls):
-    """A subclass that overrides what the whole-cell operations stand for runs its own composition."""
-    return type(cell) is cls or all(getattr(type(cell), n) is getattr(cls, n) for n in ("forward", "scan", "read"))
+def _as_written(cell, cls, *methods):
+    """A subclass that overrides what the whole-cell operations stand for (``methods``; forward, scan and read) runs its own composition."""
+    return type(cell) is cls or all(getattr(type(cell), n, None) is getattr(cls, n) for n in methods or ("forward", "scan", "read"))
 
 
 # ----------------------------------------------------------------------------------
@@ -723,11 +726,17 @@ class DeltaNetCell(MemoroidCellBase):
         return (torch.zeros(*batch, 1, self.num_heads, self.head_dim, self.head_dim, device=dev),)
 
 
+def _depthwise(conv):
+    """A convolution that the library's causal kernel stands for: one filter a channel, with a bias, every step, nothing padded."""
+    return (type(conv) is nn.Conv1d and conv.bias is not None and conv.groups == conv.in_channels == conv.out_channels
+            and conv.stride == conv.dilation == (1,) and conv.padding == (0,))
+
+
 def _causal_conv_silu(x, conv):
     """silu of a depthwise convolution over time that sees the steps up to its own and nothing before the call's first
     (mamba.py:88-106): the library's kernel where it takes the arrays, else the array library's operations."""
     K = conv.kernel_size[0]
-    if (not _hooked(conv) and x.is_cuda and x.dtype == torch.float32 and conv.weight.dtype == torch.float32 and autocast_dtype(x) is None and K <= 4
+    if (_depthwise(conv) and not _hooked(conv) and x.is_cuda and x.dtype == torch.float32 and conv.weight.dtype == torch.float32 and autocast_dtype(x) is None and K <= 4
             and x.shape[2] % 4 == 0 and x.numel() > 0):
         return native().causal_conv_silu(x, conv.weight, conv.bias)
     return F.silu(conv(F.pad(x.transpose(1, 2), (K - 1, 0)))).transpose(1, 2)
@@ -810,7 +819,7 @@ class MambaCell(MemoroidCellBase):
     def _native_sizes(self):
         P = self.head_dim
         return (type(self.norm) is _RMSNorm and self.norm.scale.dtype == torch.float32 and _plain(self.output_projection)
-                and type(self.conv) is nn.Conv1d and self.conv.bias is not None
+                and _depthwise(self.conv)
                 and P % 4 == 0 and P <= 64 and self.state_dim in (4, 8, 16, 32, 64) and self.conv_dim <= 4
                 and self.num_heads * P <= _RMS_NORM_MAX_D and self.conv.weight.dtype == torch.float32)
 
@@ -944,9 +953,9 @@ class mLSTMCell(MemoroidCellBase):
 
     def _parts_as_written(self):
         blocks, dense = (self.query, self.key, self.value), (self.up_projection, self.i_gate, self.f_gate, self.output_projection)
-        return (all(type(m) is _BlockDiagonalDense for m in blocks) and all(map(_plain, dense)) and type(self.causal_conv) is nn.Conv1d
+        return (all(type(m) is _BlockDiagonalDense for m in blocks) and all(map(_plain, dense)) and _depthwise(self.causal_conv)
                 and self.up_projection.bias is None and self.output_projection.bias is None
-                and all(m.bias is not None for m in (self.causal_conv, self.i_gate, self.f_gate)))
+                and all(m.bias is not None for m in (self.i_gate, self.f_gate)))
 
     def whole(self, x, done, initial_carry):
         """The composition below with the projections formed once (``read`` forms them again)."""

@@ -125,3 +125,50 @@ def test_whatever_a_gated_step_reads_is_on_its_gpu(at):
     with torch.no_grad(), pytest.raises(ValueError, match="must live on the GPU"):
         native().gated_act(x, 1, host(ones, "scale"), None, 1e-6, ws, bs, torch.float32, host(done, "done"), host(state, "log_state"),
                            host(state.clone(), "log_decay"), False)
+
+
+def _counting(cls, method, seen):
+    """A subclass of ``cls`` that notes each call of ``method``."""
+    def run(self, *a, **k):
+        seen.append(1)
+        return getattr(cls, method)(self, *a, **k)
+    return type("Own" + cls.__name__, (cls,), {method: run})
+
+
+@pytest.mark.parametrize("T", [1, 5])
+@pytest.mark.parametrize("replaced", ["memoroid", "recurrence cell scan", "recurrence cell elements", "mamba conv", "mlstm conv"])
+def test_a_subclass_runs_what_it_overrides(replaced, T):
+    seen = []
+    if replaced == "memoroid":
+        model = _counting(sm.Memoroid, "forward", seen)(sm.LinearAttentionCell(64, 16, 2))
+    elif "conv" in replaced:
+        cell = CELLS[replaced.split()[0]]()
+        name = "conv" if replaced.startswith("mamba") else "causal_conv"
+        old = getattr(cell, name)
+        setattr(cell, name, _counting(torch.nn.Conv1d, "forward", seen)(old.in_channels, old.out_channels, 4, groups=old.groups))
+        model = sm.Memoroid(cell)
+    else:
+        model = sm.GatedLinearRecurrence(64)
+        model.cell = _counting(sm.MinGRUCell, replaced.split()[-1], seen)(64)
+    block = sm.Residual(sm.PreNorm(model, 64)).cuda()
+    with torch.no_grad():
+        block(torch.randn(6, T, 64, device="cuda"), torch.zeros(6, T, dtype=torch.bool, device="cuda"))
+    assert seen
+
+
+@pytest.mark.parametrize("T", [1, 5])
+@pytest.mark.parametrize("cell,make", [("mamba", lambda c: torch.nn.Conv1d(c, c, 4, groups=c, bias=False)), ("mlstm", lambda c: torch.nn.Conv1d(c, c, 4)),
+                                       ("mlstm", lambda c: torch.nn.Conv1d(c, c, 4, groups=c, bias=False))])
+def test_convolutions_that_are_no_causal_kernel_s(cell, make, T):
+    """Without a bias, or over every channel: the array library's, in both directions."""
+    block = _block(cell)
+    inner = block.module.module.cell
+    name = "conv" if cell == "mamba" else "causal_conv"
+    setattr(inner, name, make(getattr(inner, name).in_channels).cuda())
+    x, done = torch.randn(6, T, 64, device="cuda"), torch.zeros(6, T, dtype=torch.bool, device="cuda")
+    with torch.no_grad():
+        got = block(x, done)[1]
+    want = block(x, done)[1]
+    want.sum().backward()
+    assert getattr(inner, name).weight.grad is not None
+    torch.testing.assert_close(got, want, rtol=0, atol=1e-5 * float(want.detach().abs().max()))
