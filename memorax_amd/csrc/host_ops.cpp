@@ -2228,8 +2228,8 @@ std::tuple<Tensor, Tensor, Tensor> mamba_mix(const Tensor &up, const Tensor &b_i
 
 // Whether a hook waits in a torch module or below it, or one of the methods that fused operations stand for was replaced on an instance (as
 // adapters and accelerators do).  An acting step asks on every call: from Python the walk over the eighteen modules of a small block pair
-// takes 7 us of a step of 88.
-bool any_hook(PyObject *module)
+// takes 7 us of a step of 88.  deep: below it too.
+bool any_hook(PyObject *module, bool deep)
 {
     static PyObject *const hooks[] = {PyUnicode_InternFromString("_forward_hooks"), PyUnicode_InternFromString("_forward_pre_hooks"),
                                       PyUnicode_InternFromString("_backward_hooks"), PyUnicode_InternFromString("_backward_pre_hooks")};
@@ -2244,11 +2244,12 @@ bool any_hook(PyObject *module)
     }
     for (PyObject *name : methods)
         if (PyDict_GetItem(*at, name)) return true;
+    if (!deep) return false;
     PyObject *const below = PyDict_GetItem(*at, children);
     if (!below || !PyDict_Check(below)) return false;
     PyObject *key, *child;
     for (Py_ssize_t pos = 0; PyDict_Next(below, &pos, &key, &child);)
-        if (any_hook(child)) return true;
+        if (any_hook(child, true)) return true;
     return false;
 }
 
@@ -2257,7 +2258,7 @@ bool any_hook(PyObject *module)
 PYBIND11_MODULE(_native, m)
 {
     m.def("bind", &bind);
-    m.def("any_hook", [](py::handle module) { return any_hook(module.ptr()); });
+    m.def("any_hook", [](py::handle module, bool deep) { return any_hook(module.ptr(), deep); });
     // the other calls touch no Python object: they run without the interpreter's lock
     auto def = [&](const char *name, auto f) { m.def(name, f, py::call_guard<py::gil_scoped_release>()); };
     def("chunk_size", &chunk_size);

@@ -503,10 +503,10 @@ def _row_layers(x, layers):
             and native().row_layers_suit(x.shape[0], [m.weight for m in layers], [m.bias for m in layers], autocast_dtype(x) is not None))
 
 
-def _hooked(module):
-    """Whether a hook waits in this module or below, or for every module, or an instance has a ``forward`` (``scan``, ``read``,
+def _hooked(module, deep=True):
+    """Whether a hook waits in this module or (deep) below, or for every module, or an instance has a ``forward`` (``scan``, ``read``,
     ``elements``) of its own: fused operations do not run the modules they stand for."""
-    return _any_global_hook() or native().any_hook(module)
+    return _any_global_hook() or native().any_hook(module, deep)
 
 
 def _plain(layer):
@@ -1096,6 +1096,15 @@ class PostNorm(nn.Module):
         return self.module.initialize_carry(key, input_shape)
 
 
+def _forks(block):
+    """Whether ``block`` is a pre-norm block that its norm's ``fork`` and its model stand for."""
+    if not (isinstance(block, PreNorm) and type(block).forward is PreNorm.forward and hasattr(block.norm, "fork")):
+        return False
+    norm = type(block.norm)
+    return (all(getattr(norm, "fork", None) is not c.fork or norm.forward is c.forward for c in (_RMSNorm, _LayerNorm))
+            and not _hooked(block, deep=False) and not _hooked(block.norm))
+
+
 class Residual(nn.Module):
     """residual.py:10-30: x + module(x)."""
 
@@ -1110,7 +1119,7 @@ class Residual(nn.Module):
             acted = inner.module.acting(inputs, inner.norm, done, initial_carry)
             if acted is not None:
                 return acted
-        if isinstance(inner, PreNorm) and hasattr(inner.norm, "fork"):   # x + f(norm(x)): one kernel takes both gradients of x
+        if inputs.is_cuda and _forks(inner):   # x + f(norm(x)): one kernel takes both gradients of x
             inputs, normed = inner.norm.fork(inputs)
             if (isinstance(inner.module, SequenceModel) and not kwargs and inputs.is_cuda and inputs.dtype is torch.float32
                     and normed.dtype is torch.bfloat16 and not _hooked(inner.module)):   # a mixed-precision block on a float32 stream

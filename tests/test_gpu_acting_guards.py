@@ -172,3 +172,27 @@ def test_convolutions_that_are_no_causal_kernel_s(cell, make, T):
     want.sum().backward()
     assert getattr(inner, name).weight.grad is not None
     torch.testing.assert_close(got, want, rtol=0, atol=1e-5 * float(want.detach().abs().max()))
+
+
+@pytest.mark.parametrize("T,grad", [(1, False), (5, False), (5, True)])
+@pytest.mark.parametrize("norm", [sm.RMSNorm, sm.LayerNorm])
+@pytest.mark.parametrize("way", ["hook", "instance", "subclass"])
+@pytest.mark.parametrize("part", ["block", "norm"])
+def test_a_pre_norm_block_around_the_fork_runs_what_was_put_in(part, way, norm, T, grad):
+    """x + f(norm(x)) through the norm's two results passes neither the norm nor the block around it by."""
+    seen = []
+    block = sm.PreNorm(sm.GatedLinearRecurrence(64), 64, norm=norm)
+    if way == "subclass" and part == "norm":
+        cls = type(block.norm)
+        block.norm = _counting(cls, "forward", seen)(64)
+    elif way == "subclass":
+        block = _counting(sm.PreNorm, "forward", seen)(block.module, 64, norm=norm)
+    m = block if part == "block" else block.norm
+    if way == "hook":
+        m.register_forward_hook(lambda *a: seen.append(1))
+    elif way == "instance":
+        own = m.forward
+        m.forward = lambda *a, **k: seen.append(1) or own(*a, **k)
+    with torch.set_grad_enabled(grad), torch.autocast("cuda", dtype=torch.bfloat16):
+        sm.Residual(block).cuda()(torch.randn(6, T, 64, device="cuda"), torch.zeros(6, T, dtype=torch.bool, device="cuda"))
+    assert seen
