@@ -1741,14 +1741,14 @@ struct DenseOp {
     static constexpr bool ONCE = true;
     static const char *name() { return "MemoraxDenseBackward"; }
     std::vector<SavedVariable> weights;
-    Tensor transposed;   // of a group whose input's gradient is mrx_dense_rows_input_grad's
+    SavedVariable transposed;   // of a group whose input's gradient is mrx_dense_rows_input_grad's; else undefined
     std::vector<bool> has_bias;
     ScalarType x_dtype;
     bool onto = false;   // the one layer's result was added to a float32 residual, whose gradient follows the others
     variable_list backward(OpNode<DenseOp> &node, std::array<Tensor, 1> &s, variable_list &grads)
     {
         c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
-        const Tensor &x = s[0], x2 = x.reshape({-1, x.size(-1)});
+        const Tensor &x = s[0], x2 = x.reshape({-1, x.size(-1)}), across = node.wants(0) ? transposed.unpack() : Tensor();
         const size_t n = weights.size();
         const auto dt = x.scalar_type();
         variable_list out(1 + 2 * n + onto);
@@ -1761,7 +1761,7 @@ struct DenseOp {
         for (size_t l = 0; l < n; ++l) {
             if (!grads[l].defined()) continue;
             ws.push_back(weights[l].unpack());
-            dys.push_back((onto && transposed.defined() && grads[l].scalar_type() == at::kFloat ? grads[l] : grads[l].to(dt)).reshape({-1, ws.back().size(0)}).contiguous());
+            dys.push_back((onto && across.defined() && grads[l].scalar_type() == at::kFloat ? grads[l] : grads[l].to(dt)).reshape({-1, ws.back().size(0)}).contiguous());
             used.push_back(l);
             bias.push_back(has_bias[l] && node.wants(1 + n + l));
             widest = std::max(widest, ws.back().size(0));
@@ -1770,7 +1770,7 @@ struct DenseOp {
         }
         if (used.empty()) return out;
         regular = regular && used.size() <= MRX_DENSE_LAYERS && x2.is_contiguous() && reinterpret_cast<uintptr_t>(x2.data_ptr()) % 16 == 0;
-        const bool rows_dx = node.wants(0) && transposed.defined() && used.size() == n && regular && input_from_rows(dys, ws, x2.size(1), want_params, out);
+        const bool rows_dx = across.defined() && used.size() == n && regular && input_from_rows(dys, ws, across, x2.size(1), want_params, out);
         for (Tensor &dy : dys) dy = dy.to(dt);   // (a residual stream's gradient: unless that has left its rounded copy)
         const bool own_params = want_params && regular && params_suit(dt, x2.size(0), x2.size(1), widest, used.size(), std::count(bias.begin(), bias.end(), true)),
                    own_dx = node.wants(0) && !rows_dx && regular && (x_dtype == at::kFloat || x_dtype == at::kBFloat16) &&
@@ -1793,9 +1793,15 @@ struct DenseOp {
         if (out[0].defined()) out[0] = out[0].view(x.sizes()).to(x_dtype);
         return out;
     }
-    // The input's gradient as the rows' way past the transposed weights; a float32 dy is left rounded where the parameters want it.
-    bool input_from_rows(std::vector<Tensor> &dys, const std::vector<Tensor> &ws, int64_t K, bool want_params, variable_list &out) const
+    // The input's gradient as the rows' way past the transposed weights `across`, where those are what the forward has saved (a hook on saved
+    // tensors may hand on others); a float32 dy is left rounded where the parameters want it.
+    static bool input_from_rows(std::vector<Tensor> &dys, const std::vector<Tensor> &ws, const Tensor &across, int64_t K, bool want_params, variable_list &out)
     {
+        int64_t wide = 0;
+        for (const Tensor &w : ws) wide += w.size(0) > 8 ? w.size(0) : 0;
+        if (across.device() != dys[0].device() || across.scalar_type() != at::kBFloat16 || across.sizes() != IntArrayRef({K, wide}) || !across.is_contiguous() ||
+            reinterpret_cast<uintptr_t>(across.data_ptr()) % 16)
+            return false;
         std::array<const void *, MRX_DENSE_LAYERS> dy{};
         std::array<int64_t, MRX_DENSE_LAYERS> n{};
         const void *narrow = nullptr;
@@ -1807,7 +1813,7 @@ struct DenseOp {
         const auto dt = dys[0].scalar_type();
         const Tensor copy = dt == at::kFloat && want_params ? fresh(dys[0].sizes(), at::kBFloat16, dys[0]) : Tensor();
         out[0] = fresh({dys[0].size(0), K}, at::kBFloat16, dys[0]);
-        check(lib.mrx_dense_rows_input_grad(stream(), dy.data(), n.data(), (int)dys.size(), ptr(transposed), narrow, ptr(out[0]), ptr(copy),
+        check(lib.mrx_dense_rows_input_grad(stream(), dy.data(), n.data(), (int)dys.size(), ptr(across), narrow, ptr(out[0]), ptr(copy),
                                             dys[0].size(0), K, code(dt)),
               "mrx_dense_rows_input_grad");
         if (copy.defined()) dys[0] = copy;
@@ -1816,7 +1822,7 @@ struct DenseOp {
     void release()
     {
         for (auto &w : weights) w.reset_data();
-        transposed.reset();
+        transposed.reset_data();
     }
 };
 
@@ -1973,7 +1979,7 @@ void record_dense(const Tensor &x, const Tensor &xc, const std::vector<Tensor> &
     if (residual.has_value()) edges.push_back(torch::autograd::impl::gradient_edge(*residual));
     node->set_next_edges(std::move(edges));
     node->op.x_dtype = x.scalar_type();
-    node->op.transposed = transposed;
+    if (transposed.defined()) node->op.transposed = SavedVariable(transposed, false);
     node->op.onto = residual.has_value();
     for (Tensor &y : out) torch::autograd::set_history(y, node);
     node->keep(0, xc);

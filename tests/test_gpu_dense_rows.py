@@ -159,3 +159,33 @@ def test_the_sum_falls_back_to_the_array_library():
         dual = torch.autograd.forward_ad.make_dual(res.to(BF).float(), torch.ones_like(res))
         out = n.dense_onto(dual, x.to(BF), w.to(BF), b.to(BF))
         assert torch.equal(torch.autograd.forward_ad.unpack_dual(out).tangent, torch.ones_like(res))
+
+
+@pytest.mark.parametrize("onto", [False, True])
+@pytest.mark.parametrize("unpacked", ["as saved", "another layout"])
+def test_hooks_on_saved_tensors_see_the_transposed_weights(onto, unpacked):
+    """Everything the node keeps for its backward passes torch's hooks (offloading, checkpoints); what they hand back in another layout is
+    read as it is."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    w, b, x0, res, gy = (rnd(64, 128) / 11).requires_grad_(), rnd(64).requires_grad_(), rnd(700, 128).to(BF), rnd(700, 64), rnd(700, 64)
+    shapes = []
+
+    def run(hooks):
+        x = x0.clone().requires_grad_()
+        with torch.autocast("cuda", dtype=BF), hooks:
+            y = _lib.native().dense_onto(res, x, w, b) if onto else _lib.native().dense_group(x, [w], [b])[0]
+        return torch.autograd.grad(y, [x, w, b], gy.to(y.dtype))
+
+    def pack(t):
+        shapes.append(tuple(t.shape))
+        return t.cpu()
+
+    def unpack(t):
+        t = t.cuda()
+        return t if unpacked == "as saved" else t.t().contiguous().t()
+
+    want, got = run(torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t)), run(torch.autograd.graph.saved_tensors_hooks(pack, unpack))
+    assert sorted(shapes) == [(64, 128), (128, 64), (700, 128)]   # the weights, the same transposed, the rows
+    for a, b in zip(got, want):   # the same kernels, or the array library's sums of 64 and 700 products in another order, rounded to bfloat16
+        assert torch.equal(a, b) if unpacked == "as saved" else float((a - b).norm()) <= 2.0 ** -7 * float(b.norm())
