@@ -667,7 +667,8 @@ int mrx_gated_recurrence_act(void *stream, const float *x, const float *scale, c
  * mrx_dense_pack: for weights W_l (n_out[l], K; K a multiple of 4) in w_dtype (MRX_F32, MRX_BF16) their bfloat16 copies (`copies`, or single entries
  *   of it, may be NULL) and, unless NULL, `transposed`: bfloat16 (K, sum of n_out[l] over the layers of more than eight outputs), the W_l^T side by side.
  * mrx_dense_rows: y_l = x W_l^T + b_l, everything bfloat16, sums in float32; biases in b_dtype (entries may be NULL; rounded to bfloat16).
- *   residual (rows, n) float32, nullable: the one layer's y is float32, residual + (x W^T + b) without a rounding between.
+ *   residual (rows, n) float32, nullable: the one layer's y is float32, residual + bf16(x W^T + b) -- the layer's own result is rounded as by itself,
+ *   the sum with the residual is float32.
  * mrx_dense_rows_input_grad: dx (rows, K) bfloat16 = sum_l dy_l W_l from `transposed`; narrow_weights: the narrow layer's W (n_out, K) in
  *   bfloat16.  dy_dtype MRX_F32 (one layer): dy is rounded to bfloat16 first, and written so to dy_copy unless that is NULL.
  * Rows, weights and results of wide layers on 16-byte boundaries, a narrow layer's dy on 4. */

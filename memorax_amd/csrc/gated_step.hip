@@ -5,7 +5,7 @@
 // states have pushed the weights out of L2: 10.2 us, as two launches 9.0 + 5.4.  (The same for a matrix state -- projections of a head and
 // its step in one launch, the states on their way meanwhile -- gains nothing: whole rows of states are 256 KB a workgroup, one
 // workgroup a compute unit, and the slowest of them ends 40 % after the mean: 31 us, as two launches 31; few rows 9.2 / 7.7.)
-// Rounding follows the launches it stands for (row_dense.hip, mingru_step_kernel).
+// Rounding follows the launches it stands for (row_dense.hip, mingru_step_kernel); 1024 rows x 256 come out with the same bits.
 #include "mingru.h"
 #include "row_parts.h"
 
