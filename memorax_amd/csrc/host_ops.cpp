@@ -1766,7 +1766,7 @@ struct DenseOp {
             bias.push_back(has_bias[l] && node.wants(1 + n + l));
             widest = std::max(widest, ws.back().size(0));
             want_params = want_params || node.wants(1 + l) || bias.back();
-            regular = regular && ws.back().is_contiguous() && ws.back().size(0) > 0 && reinterpret_cast<uintptr_t>(ws.back().data_ptr()) % 16 == 0;
+            regular = regular && ws.back().device() == x.device() && ws.back().scalar_type() == dt && ws.back().is_contiguous() && ws.back().size(0) > 0 && reinterpret_cast<uintptr_t>(ws.back().data_ptr()) % 16 == 0;
         }
         if (used.empty()) return out;
         regular = regular && used.size() <= MRX_DENSE_LAYERS && x2.is_contiguous() && reinterpret_cast<uintptr_t>(x2.data_ptr()) % 16 == 0;
@@ -2073,6 +2073,14 @@ Tensor dense_onto(const Tensor &residual, const Tensor &x, const Tensor &weight,
 }
 
 // ---- causal depthwise convolution over time with silu behind it (conv_cells.hip)
+// x (B,T,C) as the kernels walk it: its own rows where they are dense or the leading columns of wider ones
+Tensor as_rows(const Tensor &x)
+{
+    TORCH_CHECK_VALUE(x.dim() == 3 && x.is_cuda() && x.scalar_type() == at::kFloat, "causal_conv_silu takes (B,T,C) float32 arrays on the GPU");
+    const bool rows = x.stride(2) == 1 && x.stride(1) % 4 == 0 && x.stride(0) == x.size(1) * x.stride(1) && ((uintptr_t)x.data_ptr()) % 16 == 0;
+    return rows ? x : dense16(x);
+}
+
 struct ConvSiluOp {
     static constexpr int SAVED = 3;   // x, weight, bias
     static constexpr bool ONCE = true;
@@ -2080,11 +2088,12 @@ struct ConvSiluOp {
     variable_list backward(OpNode<ConvSiluOp> &, std::array<Tensor, 3> &s, variable_list &grads)
     {
         if (!grads[0].defined()) return {Tensor(), Tensor(), Tensor()};
-        const Tensor &x = s[0];
-        const int64_t B = x.size(0), T = x.size(1), C = x.size(2), K = s[1].size(2);
+        const Tensor x = as_rows(s[0]), weight = dense16(s[1]), bias = dense16(s[2]);   // a hook may hand them on in another layout
+        chk(weight, "weight", at::kFloat), chk(bias, "bias", at::kFloat);
+        const int64_t B = x.size(0), T = x.size(1), C = x.size(2), K = weight.size(2);
         const Tensor dy = grads[0].contiguous(), dx = fresh(x.sizes(), at::kFloat, x), params = fresh({C * (K + 1)}, at::kFloat, x),
                      work = fresh({MRX_CONV_PARTS, C * (K + 1)}, at::kFloat, x);
-        check(lib.mrx_causal_conv_silu_bwd(stream(), fptr(x), x.stride(1), fptr(s[1]), fptr(s[2]), fptr(dy), fptr(dx), C, fptr(params),
+        check(lib.mrx_causal_conv_silu_bwd(stream(), fptr(x), x.stride(1), fptr(weight), fptr(bias), fptr(dy), fptr(dx), C, fptr(params),
                                            fptr(work), B, T, C, K),
               "mrx_causal_conv_silu_bwd");
         return {dx, params.narrow(0, 0, C * K).view({C, 1, K}), params.narrow(0, C * K, C)};
@@ -2104,8 +2113,7 @@ Tensor causal_conv_silu(const Tensor &x_, const Tensor &weight_, const Tensor &b
         weight = dense16(weight_), bias = dense16(bias_);
         chk(weight, "weight", at::kFloat, {C, 1, K});
         chk(bias, "bias", at::kFloat, {C});
-        const bool rows = x_.stride(2) == 1 && x_.stride(1) % 4 == 0 && x_.stride(0) == T * x_.stride(1) && ((uintptr_t)x_.data_ptr()) % 16 == 0;
-        x = rows ? x_ : dense16(x_);
+        x = as_rows(x_);
         y = fresh({B, T, C}, at::kFloat, x);
         check(lib.mrx_causal_conv_silu_fwd(stream(), fptr(x), x.stride(1), fptr(weight), fptr(bias), fptr(y), B, T, C, K), "mrx_causal_conv_silu_fwd");
     }
@@ -2133,6 +2141,10 @@ struct MambaOp {
     double eps;
     variable_list backward(OpNode<MambaOp> &node, std::array<Tensor, SAVED> &s, variable_list &grads)
     {
+        for (Tensor &t : s) {   // a hook on saved tensors may hand them on in another layout
+            t = dense16(t);
+            if (t.defined()) chk(t, "saved tensor", at::kFloat);
+        }
         const Tensor dy = grad_or_zeros(grads[0], s[V].view({n.B, n.T, n.W})), &up = s[UP];
         const Tensor d_up = fresh_like(up), d_o = fresh_like(s[O]), dscale = fresh({n.W}, at::kFloat, up);
         Tensor work = fresh({MRX_RMS_NORM_PARTS, n.W}, at::kFloat, up);

@@ -85,3 +85,33 @@ def test_mamba_cell_notices_a_carry_overwritten_before_the_backward():
     carry[1].mul_(2.0)
     with pytest.raises(RuntimeError, match="inplace operation"):
         loss.backward()
+
+
+@pytest.mark.parametrize("what", ["conv", "mamba"])
+def test_saved_tensors_that_a_hook_hands_back_in_another_layout(what):
+    """Torch's hooks on saved tensors may hand on copies whose elements lie elsewhere: they are read by their strides."""
+    from memorax_amd import _lib, sequence_models as sm
+    torch.manual_seed(7)
+    if what == "conv":
+        x, w, b = torch.randn(3, 9, 16, device="cuda"), torch.randn(16, 1, 4, device="cuda"), torch.randn(16, device="cuda")
+        leaves = [t.requires_grad_() for t in (x, w, b)]
+        run = lambda: _lib.native().causal_conv_silu(x, w, b)  # noqa: E731
+    else:
+        cell = sm.MambaCell(16, num_heads=2, head_dim=32, state_dim=32).cuda()
+        x, done = torch.randn(3, 9, 16, device="cuda", requires_grad=True), torch.rand(3, 9, device="cuda") < 0.1
+        carry = cell.initialize_carry(None, (3, 16))
+        leaves = [x, *cell.parameters()]
+        run = lambda: cell.whole(x, done, carry)[1]  # noqa: E731
+    seen = []
+
+    def unpack(t):
+        seen.append(t.dim() > 1)
+        return t.transpose(0, -1).contiguous().transpose(0, -1) if t.dim() > 1 else t
+
+    want = torch.autograd.grad(run().square().sum(), leaves)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        loss = run().square().sum()
+    got = torch.autograd.grad(loss, leaves)
+    assert any(seen)
+    for a, b in zip(got, want):   # the same kernels on the same numbers; the projections around Mamba's in another order of their sums
+        assert float((a - b).norm()) <= (0.0 if what == "conv" else 1e-5) * float(b.norm())
