@@ -640,12 +640,22 @@ int mrx_mlstm_step(void *stream, const float *up, const float *conv_w, const flo
  *   params (nullable): float32, [dW_0 (n_out[0], K) | dW_1 | ...] and then db_l (n_out[l]) of the layers whose bit is set in
  *     bias_mask; padded to a multiple of four floats.
  * x, dy_l and W_l (n_out[l], K) in `dtype`, MRX_F32 or MRX_BF16, sums in float32; K a multiple of 8.  x may be NULL without
- * params, weights without dx.  workspace: mrx_dense_grads_workspace(...) floats, overwritten (NULL where that is 0). */
+ * params, weights without dx.  workspace: mrx_dense_grads_workspace(...) floats, overwritten (NULL where that is 0).  float32: products as
+ * those of mrx_dense_f32. */
 #define MRX_DENSE_LAYERS 8
 int64_t mrx_dense_grads_workspace(int64_t rows, int64_t K, const int64_t *n_out, int layers, int dtype, unsigned bias_mask);
 int mrx_dense_grads(void *stream, const void *x, const void *const *dys, const void *const *weights, const int64_t *n_out,
                     int layers, void *dx, float *params, float *workspace, int64_t rows, int64_t K, int dtype, int dx_dtype,
                     unsigned bias_mask);
+
+/* ---- Dense layers over rows in float32 ----
+ * y_l (rows, n_out[l]) = x W_l^T + b_l of up to MRX_DENSE_LAYERS layers on the rows x (rows, K), everything float32 (entries of `biases` may be NULL);
+ * residual (rows, n), nullable: added to the one layer's result.  K a multiple of 8.  Products on the float16 matrix units, every value as the sum of
+ * two scaled float16 ones (22 bits and a sign, 2^-39 of its row's or column's largest value); infinities and NaN as float32 has them.
+ * workspace: mrx_dense_f32_workspace(...) floats (0: sizes that are not served), overwritten.  x, weights, results and workspace on 16-byte boundaries. */
+int64_t mrx_dense_f32_workspace(const int64_t *n_out, int layers, int64_t K);
+int mrx_dense_f32(void *stream, const float *x, const void *const *weights, const void *const *biases, void *const *outs,
+                  const int64_t *n_out, int layers, const float *residual, int64_t rows, int64_t K, float *workspace);
 
 /* ---- The acting step of a gated recurrence up to what its closing layer reads ----
  * x (rows, K) float32, normalised as mrx_row_dense does (norm 0, 1, 2; K a multiple of 8 up to 512); weights (N, K) without biases in w_dtype;

@@ -8,9 +8,9 @@
 // those, a reduction per bias, and the sum of the input gradients rounded and read back between the layers -- most of them at a
 // fraction of the bandwidth (131072 rows, three layers of 256 x 256 and one of 256 x 4 in bfloat16: 330 us for the parameters and 150 us
 // for the input; 11455 rows, three of 128 x 256: 225 and 23 us).  Here they are two launches and one reduction: 104 (on wide tiles, below; 134 on the others) and
-// 118 us, 24 and 16 us; the input's gradient in bfloat16 over wide rows is dense_rows.hip's (60 us), the kernel here serves the rest.  At 256 features a compute unit is short of loads in flight rather than of bandwidth: LDS holds two steps of two workgroups.
+// 118 us, 24 and 16 us; the input's gradient in bfloat16 over wide rows is dense_rows.hip's (60 us), in float32 dense_split.hip's, the kernel here serves the rest.  At 256 features a compute unit is short of loads in flight rather than of bandwidth: LDS holds two steps of two workgroups.
 //
-// Weight gradients: a workgroup of four waves owns a TN x TK tile of one layer's result and a slice of the rows, 64 (float32: 32)
+// Weight gradients: a workgroup of four waves owns a TN x TK tile of one layer's result and a slice of the rows, 64 (float32: 32, below)
 // of which wait in LDS while the next are on their way; both operands are contracted over their rows, which the transposing
 // LDS reads serve without a copy.  The slices' partial results are summed in a fixed order (col_sum.h).
 // Input gradient: a workgroup owns TM rows and TK features and walks the layers' outputs, two steps ahead in registers (one step: 120
@@ -18,7 +18,9 @@
 // of both operands instead: a second step there costs the registers those need, 123 -> 147 us).
 #include "chunk_common.h"
 #include "col_sum.h"
+#include "dense_split.h"
 #include "row_dma.h"
+#include "split_f16.h"
 
 #include <type_traits>
 
@@ -92,7 +94,7 @@ template <typename T, int R, int W, OpMode MODE> struct RowTile {
     }
 };
 
-template <typename T> constexpr int dg_rows() { return sizeof(T) == 2 ? 64 : 32; }   // rows (weight gradients) or outputs (dx) per step
+constexpr int DG_STEP = 64, SG_STEP = 32;   // rows (weight gradients) or outputs (dx) of a step, in bfloat16 and in float32
 
 // Workgroups are dealt to the eight dies in turn, and tasks that read the same rows follow each other: each die takes a contiguous
 // share of them, and its L2 serves the second reader.  -1: none left.
@@ -103,10 +105,11 @@ __device__ __forceinline__ int64_t task_of(int64_t tasks)
 }
 inline unsigned grid_of(int64_t tasks) { return (unsigned)((tasks + 7) / 8 * 8); }
 
-template <typename T, int TN, int TK>
+template <int TN, int TK>
 __global__ void __launch_bounds__(DG_THREADS, 2) dense_weight_grad_kernel(DenseGradArgs a)
 {
-    constexpr int RC = dg_rows<T>(), MBW = TK / 32, NBW = TN / 32;
+    using T = __bf16;
+    constexpr int RC = DG_STEP, MBW = TK / 32, NBW = TN / 32;
     using TileX = RowTile<T, RC, TK, KROW>;
     using TileY = RowTile<T, RC, TN, KROW>;
     using TM = TileMap<TK, TN, DG_WAVES, MBW>;
@@ -129,24 +132,11 @@ __global__ void __launch_bounds__(DG_THREADS, 2) dense_weight_grad_kernel(DenseG
     f32x4 acc[TM::TPW], accb[NBW];
     zero_acc<TM::TPW>(acc);
     zero_acc<NBW>(accb);
-    // the bias gradient, in float32 a step's sum at a time with what its additions round off (131072 x 4: 1.6e-7 -> 4e-8)
-    float bias_sum[NBW], bias_low[NBW];
-#pragma unroll
-    for (int j = 0; j < NBW; ++j) bias_sum[j] = bias_low[j] = 0.f;
     TileX tx;
     TileY ty;
     tx.load(x, r0, r1, a.rows, k0, a.K, tid);
     ty.load(dy, r0, r1, a.rows, n0, N, tid);
     int buf = 0;
-    auto sum_bias = [&]() {
-#pragma unroll
-        for (int j = 0; j < NBW; ++j) {
-            const float y = accb[j][0] - bias_low[j], s = bias_sum[j] + y;
-            bias_low[j] = (s - bias_sum[j]) - y;
-            bias_sum[j] = s;
-        }
-        zero_acc<NBW>(accb);
-    };
     for (int64_t r = r0; r < r1; r += RC, buf ^= 1) {
         T *const sx = lds + buf * BUF, *const sy = sx + RC * TileX::LD;
         tx.to_lds(sx, tid);
@@ -155,7 +145,6 @@ __global__ void __launch_bounds__(DG_THREADS, 2) dense_weight_grad_kernel(DenseG
             tx.load(x, r + RC, r1, a.rows, k0, a.K, tid);
             ty.load(dy, r + RC, r1, a.rows, n0, N, tid);
         }
-        if (sizeof(T) == 4 && bias) sum_bias();   // of the step before: its products are done
         sync_lds();   // the buffer two steps back has been read by every wave that reaches the barrier
         gemm<T, TK, TN, RC, KROW, KROW, DG_WAVES, MBW>(acc, sx, TileX::LD, sy, TileY::LD, w, lane, NoHook(),
                                                        [&](int ni, int, typename TT<T>::frag &f) {
@@ -168,12 +157,226 @@ __global__ void __launch_bounds__(DG_THREADS, 2) dense_weight_grad_kernel(DenseG
         const int k = k0 + TM::mt(w, j) * 16 + 4 * g, n = n0 + TM::nt(w, j) * 16 + i16;
         if (k < a.K && n < N) *reinterpret_cast<f32x4 *>(out + a.w_at[l] + (int64_t)n * a.K + k) = acc[j];
     }
-    if (bias) sum_bias();
     if (bias && g == 0) {
 #pragma unroll
         for (int j = 0; j < NBW; ++j) {
             const int n = n0 + TM::nt(w, j) * 16 + i16;
-            if (n < N) out[a.b_at[l] + n] = bias_sum[j];
+            if (n < N) out[a.b_at[l] + n] = accb[j][0];
+        }
+    }
+}
+
+// ---- weight gradients in float32 on the float16 matrix units (split_f16.h)
+// The same tiles, slices and steps; a step's rows are split into two float16 tiles each on their way into LDS, every column with a power of two
+// of its own.  A column's scale leaves room for values 16 times the largest so far: where a step goes beyond, the workgroup finds the columns'
+// largest values again, brings the running sums to the new scales and splits the step once more (the first step does).
+// us, here / on float32 products before: 32768 x 256 -> 1024 + 512 + 512 + 8 199 / 305 (the array library), 131072 x 256 -> 3 x 256 + 4 315 / 576, 4096 x 256 ->
+// 3 x 256 35 / 53.  Without the products the first takes 170, without the splitting 165, without the loads 145: two workgroups of a compute
+// unit in turn, each a trip to L2, the split, a barrier and the products a step.  Three (half the LDS, a second barrier) spill.
+template <int W> __device__ __forceinline__ f16x8 split_fragment(const _Float16 *tile, int c0, int lane)
+{
+    constexpr int LD = W + 16;   // as RowTile::LD
+    const int i = lane & 15, g = lane >> 4;
+    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+    const _Float16 *p = tile + (8 * g + (i >> 2)) * LD + c0 + 4 * (i & 3);
+    union {
+        s16x4 h[2];
+        f16x8 f;
+    } u;
+    u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)p);
+    u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(p + 4 * LD));
+    return u.f;
+}
+
+// One operand's step: 32 rows x W columns in registers, and the scales of this thread's four columns.
+template <int W> struct SplitTile {
+    using Rows = RowTile<float, 32, W, KROW>;
+    static constexpr int LD = W + 16, HALF = 32 * LD;   // float16 between rows; of the high, then of the low parts
+    static constexpr int COLS = W / 4;                  // threads across
+    Rows rows;
+    float scale[4];
+    // columns past the last count nothing
+    __device__ __forceinline__ void mask(int tid)
+    {
+        const int have = rows.cols - tid % COLS * 4;
+        if (have < 4)
+#pragma unroll
+            for (int p = 0; p < Rows::PASSES; ++p)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (q >= have) rows.v[p][q] = 0u;
+    }
+    // the largest scaled value of this thread's part; in (hi, lo) tiles
+    __device__ __forceinline__ float to_lds(_Float16 *dst, int tid)
+    {
+        float m = 0.f;
+        const sf32x4 s = {scale[0], scale[1], scale[2], scale[3]};
+#pragma unroll
+        for (int p = 0; p < Rows::PASSES; ++p) {
+            const sf32x4 x = __builtin_bit_cast(sf32x4, rows.v[p]) * s;
+            m = max4(m, x);
+            const Split4 y = split4(x, 1.f);
+            const int at = (tid / COLS + p * (DG_THREADS / COLS)) * LD + tid % COLS * 4;
+            *reinterpret_cast<f16x4 *>(dst + at) = y.hi;
+            *reinterpret_cast<f16x4 *>(dst + HALF + at) = y.lo;
+        }
+        return m;
+    }
+    __device__ __forceinline__ void peaks(int *top, int tid) const   // of each of this thread's columns
+    {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            float m = 0.f;
+#pragma unroll
+            for (int p = 0; p < Rows::PASSES; ++p) m = fmaxf(m, fabsf(__uint_as_float(rows.v[p][q])));
+            atomicMax(&top[tid % COLS * 4 + q], (int)(__float_as_uint(m) & 0x7fffffffu));
+        }
+    }
+    __device__ __forceinline__ void rescale(const int *log_scale, int tid)
+    {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) scale[q] = power_of_two(log_scale[tid % COLS * 4 + q]);
+    }
+};
+constexpr int SG_TOP = 10;            // the largest of a column so far lies in [2^10, 2^11) when its scale is chosen
+constexpr float SG_LIMIT = 32768.f;
+
+template <int TN, int TK> constexpr size_t split_lds() { return 2 * 2 * (SplitTile<TN>::HALF + SplitTile<TK>::HALF) * sizeof(_Float16); }
+
+template <int TN, int TK> __global__ void __launch_bounds__(DG_THREADS, 2) split_weight_grad_kernel(DenseGradArgs a)
+{
+    constexpr int RC = SG_STEP, MBW = TK / 32, NBW = TN / 32;
+    using TM = TileMap<TK, TN, DG_WAVES, MBW>;
+    constexpr int BUF = 2 * (SplitTile<TK>::HALF + SplitTile<TN>::HALF);
+    static_assert(RC == 32, "one block of the contraction a step");
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ int top[TK + TN], log_scale[TK + TN], change[TK + TN], beyond[2], infinite;
+    _Float16 *const lds = reinterpret_cast<_Float16 *>(smem);
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), i16 = lane & 15, g = lane >> 4;
+    const int tiles = a.first_tile[a.layers] * a.ktiles;
+    const int64_t task = task_of((int64_t)tiles * a.slices);
+    if (task < 0) return;
+    const int slice = (int)(task / tiles), tile = (int)(task % tiles);
+    const int kt = tile % a.ktiles, nt = tile / a.ktiles;
+    int l = 0;
+    while (nt >= a.first_tile[l + 1]) ++l;
+    const int N = a.n[l], n0 = (nt - a.first_tile[l]) * TN, k0 = kt * TK;
+    const int64_t r0 = slice * a.slice_rows, r1 = r0 + a.slice_rows < a.rows ? r0 + a.slice_rows : a.rows;
+    const float *x = static_cast<const float *>(a.x), *dy = static_cast<const float *>(a.dy[l]);
+    const bool bias = a.b_at[l] >= 0 && kt == 0;
+    if (tid < TK + TN) top[tid] = 0, log_scale[tid] = 126;
+    if (tid == 0) beyond[0] = beyond[1] = infinite = 0;
+
+    f32x4 acc[TM::TPW];
+    zero_acc<TM::TPW>(acc);
+    // the bias gradient, a step's sum at a time with what its additions round off
+    sf32x4 bias_sum = {0.f, 0.f, 0.f, 0.f}, bias_low = bias_sum;
+    SplitTile<TK> tx;
+    SplitTile<TN> ty;
+    sync_lds();
+    tx.rescale(log_scale, tid);
+    ty.rescale(log_scale + TK, tid);
+    auto load = [&](int64_t r) {
+        tx.rows.load(x, r, r1, a.rows, k0, a.K, tid);
+        ty.rows.load(dy, r, r1, a.rows, n0, N, tid);
+    };
+    load(r0);
+    int buf = 0, step = 0;
+    for (int64_t r = r0; r < r1; r += RC, buf ^= 1) {
+        _Float16 *const sx = lds + buf * BUF, *const sy = sx + 2 * SplitTile<TK>::HALF;
+        ++step;
+        tx.mask(tid);
+        ty.mask(tid);
+        if (fmaxf(tx.to_lds(sx, tid), ty.to_lds(sy, tid)) >= SG_LIMIT) beyond[buf] = step;
+        if (bias) {
+            sf32x4 part = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int p = 0; p < SplitTile<TN>::Rows::PASSES; ++p) part += __builtin_bit_cast(sf32x4, ty.rows.v[p]);
+            const sf32x4 y = part - bias_low, s = bias_sum + y;
+            bias_low = (s - bias_sum) - y, bias_sum = s;
+        }
+        sync_lds();   // the buffer two steps back has been read by every wave that reaches the barrier
+        if (beyond[buf] == step) {
+            tx.peaks(top, tid);
+            ty.peaks(top + TK, tid);
+            sync_lds();
+            if (tid < TK + TN) {
+                const int e = exponent(__uint_as_float((uint32_t)top[tid])), was = log_scale[tid];
+                int now = SG_TOP - e;
+                now = now < was ? now : was;
+                now = now < -126 ? -126 : now;
+                change[tid] = now - was, log_scale[tid] = now;
+                if (e == 128) infinite = 1;
+            }
+            sync_lds();
+#pragma unroll
+            for (int j = 0; j < TM::TPW; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    acc[j][v] = __builtin_ldexpf(acc[j][v], change[TM::mt(w, j) * 16 + 4 * g + v] + change[TK + TM::nt(w, j) * 16 + i16]);
+            tx.rescale(log_scale, tid);
+            ty.rescale(log_scale + TK, tid);
+            tx.to_lds(sx, tid);
+            ty.to_lds(sy, tid);
+            sync_lds();
+        }
+        if (r + RC < r1) load(r + RC);
+        f16x8 fx[MBW][2];
+#pragma unroll
+        for (int m = 0; m < MBW; ++m)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) fx[m][h] = split_fragment<TK>(sx + h * SplitTile<TK>::HALF, TM::mt(w, m * TM::NBW) * 16, lane);
+#pragma unroll
+        for (int n = 0; n < NBW; ++n) {
+            f16x8 fy[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) fy[h] = split_fragment<TN>(sy + h * SplitTile<TN>::HALF, TM::nt(w, n) * 16, lane);
+            // the small products by themselves first: two roundings of the running sum a step instead of three
+            f32x4 low[MBW];
+#pragma unroll
+            for (int m = 0; m < MBW; ++m) low[m] = mma_f16(fx[m][1], fy[0], f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+            for (int m = 0; m < MBW; ++m) low[m] = mma_f16(fx[m][0], fy[1], low[m]);
+#pragma unroll
+            for (int m = 0; m < MBW; ++m) acc[m * TM::NBW + n] = mma_f16(fx[m][0], fy[0], acc[m * TM::NBW + n]);
+#pragma unroll
+            for (int m = 0; m < MBW; ++m) acc[m * TM::NBW + n] += low[m];
+        }
+    }
+    float *const out = a.out + slice * a.total;
+    if (infinite) {   // sums one by one: what an infinity makes of them is float32's
+        for (int e = tid; e < TN * TK; e += DG_THREADS) {
+            const int n = n0 + e / TK, k = k0 + e % TK;
+            if (n >= N || k >= a.K) continue;
+            float sum = 0.f;
+            for (int64_t r = r0; r < r1; ++r) sum = fmaf(dy[r * N + n], x[r * a.K + k], sum);
+            out[a.w_at[l] + (int64_t)n * a.K + k] = sum;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < TM::TPW; ++j) {
+            const int ki = TM::mt(w, j) * 16 + 4 * g, ni = TM::nt(w, j) * 16 + i16;
+            if (k0 + ki >= a.K || n0 + ni >= N) continue;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[j][v] = __builtin_ldexpf(acc[j][v], -(log_scale[ki + v] + log_scale[TK + ni]));
+            *reinterpret_cast<f32x4 *>(out + a.w_at[l] + (int64_t)(n0 + ni) * a.K + k0 + ki) = acc[j];
+        }
+    }
+    if (bias) {   // the threads' shares of a column, in pairs
+        constexpr int SHARES = DG_THREADS / SplitTile<TN>::COLS;
+        float *const part = reinterpret_cast<float *>(smem);
+        sync_lds();
+        *reinterpret_cast<sf32x4 *>(part + tid / SplitTile<TN>::COLS * TN + tid % SplitTile<TN>::COLS * 4) = bias_sum;
+        sync_lds();
+        if (tid < TN && n0 + tid < N) {
+            float t[SHARES];
+#pragma unroll
+            for (int s = 0; s < SHARES; ++s) t[s] = part[s * TN + tid];
+#pragma unroll
+            for (int half = SHARES / 2; half > 0; half /= 2)
+#pragma unroll
+                for (int s = 0; s < half; ++s) t[s] += t[s + half];
+            out[a.b_at[l] + n0 + tid] = t[0];
         }
     }
 }
@@ -329,10 +532,11 @@ __global__ void __launch_bounds__(WT_THREADS, 1) wide_weight_grad_kernel(WideGra
     }
 }
 
-template <typename T, int TM_, int TK>
+template <int TM_, int TK>
 __global__ void __launch_bounds__(DG_THREADS, 2) dense_input_grad_kernel(DenseGradArgs a)
 {
-    constexpr int NC = dg_rows<T>(), MBW = TK / 32;
+    using T = __bf16;
+    constexpr int NC = DG_STEP, MBW = TK / 32;
     using TileW = RowTile<T, NC, TK, KROW>;
     using TileY = RowTile<T, TM_, NC, ROWK>;
     using TM = TileMap<TK, TM_, DG_WAVES, MBW>;
@@ -344,13 +548,8 @@ __global__ void __launch_bounds__(DG_THREADS, 2) dense_input_grad_kernel(DenseGr
     if (task < 0) return;
     const int64_t r0 = task / a.ktiles * TM_;
     const int k0 = (int)(task % a.ktiles) * TK;
-    // float32: a layer's share is summed by itself, as products one after another would sum it (three layers of 128: 3.5e-7 -> 2.1e-7, the
-    // array library's error; 131072 x 128 138 -> 142 us).  bfloat16 operands hide the difference.
-    constexpr bool BY_LAYER = sizeof(T) == 4;
-    f32x4 acc[TM::TPW], total[BY_LAYER ? TM::TPW : 1];
+    f32x4 acc[TM::TPW];
     zero_acc<TM::TPW>(acc);
-    zero_acc<(BY_LAYER ? TM::TPW : 1)>(total);
-    bool last[2] = {false, false};   // of its layer
     TileW tw[2];   // the steps on their way: two, so that a trip to memory spans two products
     TileY ty[2];
     int l = 0, n0 = 0, steps = 0;   // where the next fetch reads; steps fetched and not yet multiplied
@@ -359,8 +558,7 @@ __global__ void __launch_bounds__(DG_THREADS, 2) dense_input_grad_kernel(DenseGr
         tw[i].load(static_cast<const T *>(a.w[l]), n0, a.n[l], a.n[l], k0, a.K, tid);
         ty[i].load(static_cast<const T *>(a.dy[l]), r0, a.rows, a.rows, n0, a.n[l], tid);
         n0 += NC;
-        last[i] = n0 >= a.n[l];
-        if (last[i]) ++l, n0 = 0;
+        if (n0 >= a.n[l]) ++l, n0 = 0;
         ++steps;
     };
     fetch(0);
@@ -370,15 +568,9 @@ __global__ void __launch_bounds__(DG_THREADS, 2) dense_input_grad_kernel(DenseGr
         tw[i].to_lds(sw, tid);
         ty[i].to_lds(sy, tid);
         --steps;
-        const bool ends = last[i];
         fetch(i);
         sync_lds();
         gemm<T, TK, TM_, NC, KROW, ROWK, DG_WAVES, MBW>(acc, sw, TileW::LD, sy, TileY::LD, w, lane);
-        if (BY_LAYER && ends) {
-#pragma unroll
-            for (int j = 0; j < TM::TPW; ++j) total[j] += acc[j];
-            zero_acc<TM::TPW>(acc);
-        }
     };
     while (steps > 0) {
         step(0);
@@ -390,15 +582,15 @@ __global__ void __launch_bounds__(DG_THREADS, 2) dense_input_grad_kernel(DenseGr
         const int64_t r = r0 + TM::nt(w, j) * 16 + i16;
         if (k >= a.K || r >= a.rows) continue;
         const int64_t at = r * a.K + k;
-        const f32x4 y = BY_LAYER ? total[BY_LAYER ? j : 0] : acc[j];
+        const f32x4 y = acc[j];
         if (a.dx_bf16) *reinterpret_cast<bf16x4 *>(static_cast<__bf16 *>(a.dx) + at) = TT<__bf16>::pack(y[0], y[1], y[2], y[3]);
         else *reinterpret_cast<f32x4 *>(static_cast<float *>(a.dx) + at) = y;
     }
 }
 
-template <typename T, int R1, int W1, int R2, int W2, OpMode M2> constexpr size_t dg_lds()
+template <int R1, int W1, int R2, int W2, OpMode M2> constexpr size_t dg_lds()
 {
-    return 2 * sizeof(T) * (R1 * RowTile<T, R1, W1, KROW>::LD + R2 * RowTile<T, R2, W2, M2>::LD);
+    return 2 * sizeof(__bf16) * (R1 * RowTile<__bf16, R1, W1, KROW>::LD + R2 * RowTile<__bf16, R2, W2, M2>::LD);
 }
 
 struct WeightPlan {
@@ -409,9 +601,9 @@ struct WeightPlan {
 // 128 x 128 tiles, 64 where the layers are narrower; the rows cut so that five hundred workgroups run (two per compute unit), but no
 // shorter than four steps of a workgroup, and a whole number of such rounds where a slice would have more than CHAIN rows: a running
 // sum in float32 errs in proportion to its length.  131072 rows, three layers of 256 x 256 and one of 256 x 4, error of the weights against
-// float64: bfloat16 (3648 rows a slice) 8.4e-8 -> 4.5e-8, where the array library's slices have 5.2e-8, 132 -> 134 us; float32 1.6e-7 -> 4.4e-8
-// (library 9.3e-8), 576 -> 618 us.
-constexpr int64_t CHAIN_BF16 = 2048, CHAIN_F32 = 512;
+// float64: bfloat16 (3648 rows a slice) 8.4e-8 -> 4.5e-8, where the array library's slices have 5.2e-8, 132 -> 134 us.  A float32 slice may be longer
+// than on float32 products (512), with a quarter of their roundings: 32768 x 256 -> 2056 outputs 512 rows a slice 2.7e-7 and 220 us, 1152 2.6e-7 and 199 us.
+constexpr int64_t CHAIN_BF16 = 2048, CHAIN_F32 = 1152;
 
 constexpr int64_t WIDE_WORK = 3 << 16;
 // The plan on wide tiles, for bfloat16 layers whose sizes are whole tiles (one of two, four, six or eight outputs may ride along): one round of
@@ -470,18 +662,19 @@ WeightPlan plan_weights(int64_t rows, int64_t K, const int64_t *n, int layers, b
     return p;
 }
 
-template <typename T, int TN, int TK> int launch_weight_grads(hipStream_t st, DenseGradArgs &a, const WeightPlan &p)
+template <int TN, int TK> int launch_weight_grads(hipStream_t st, DenseGradArgs &a, const WeightPlan &p, bool bf16)
 {
     for (int l = 0; l < a.layers; ++l) a.first_tile[l + 1] = a.first_tile[l] + (a.n[l] + TN - 1) / TN;
     a.ktiles = (a.K + TK - 1) / TK;
-    return launch_kernel(dense_weight_grad_kernel<T, TN, TK>, dim3(grid_of((int64_t)p.tiles * p.slices)), dim3(DG_THREADS),
-                         dg_lds<T, dg_rows<T>(), TK, dg_rows<T>(), TN, KROW>(), st, a);
+    const dim3 grid(grid_of((int64_t)p.tiles * p.slices));
+    return bf16 ? launch_kernel(dense_weight_grad_kernel<TN, TK>, grid, dim3(DG_THREADS), dg_lds<DG_STEP, TK, DG_STEP, TN, KROW>(), st, a)
+                : launch_kernel(split_weight_grad_kernel<TN, TK>, grid, dim3(DG_THREADS), split_lds<TN, TK>(), st, a);
 }
-template <typename T, int TM, int TK> int launch_input_grad(hipStream_t st, DenseGradArgs &a)
+template <int TM, int TK> int launch_input_grad(hipStream_t st, DenseGradArgs &a)
 {
     a.ktiles = (a.K + TK - 1) / TK;
-    return launch_kernel(dense_input_grad_kernel<T, TM, TK>, dim3(grid_of((a.rows + TM - 1) / TM * a.ktiles)), dim3(DG_THREADS),
-                         dg_lds<T, dg_rows<T>(), TK, TM, dg_rows<T>(), ROWK>(), st, a);
+    return launch_kernel(dense_input_grad_kernel<TM, TK>, dim3(grid_of((a.rows + TM - 1) / TM * a.ktiles)), dim3(DG_THREADS),
+                         dg_lds<DG_STEP, TK, TM, DG_STEP, ROWK>(), st, a);
 }
 
 template <bool NARROW> int launch_wide(hipStream_t st, const DenseGradArgs &a, const WeightPlan &p)
@@ -502,32 +695,31 @@ template <bool NARROW> int launch_wide(hipStream_t st, const DenseGradArgs &a, c
     return launch_kernel(wide_weight_grad_kernel<NARROW>, dim3(grid_of((int64_t)p.tiles * p.slices)), dim3(WT_THREADS), T::STAGES * T::STAGE, st, w);
 }
 
-template <typename T> int launch_grads(hipStream_t st, DenseGradArgs &a, const WeightPlan &p, float *params, float *workspace)
+int launch_grads(hipStream_t st, DenseGradArgs &a, const WeightPlan &p, bool bf16, float *params, float *workspace)
 {
-    if (a.dx) {
+    if (a.dx && bf16) {
         // rows and features per workgroup: large tiles read dy and the weights less often, small ones fill the device
         const int64_t large = (a.rows + 127) / 128 * ((a.K + 127) / 128);
-        const int rc = a.K <= 64 ? (a.rows >= 128 * 512 ? launch_input_grad<T, 128, 64>(st, a) : launch_input_grad<T, 64, 64>(st, a))
-                       : large >= 512 ? launch_input_grad<T, 128, 128>(st, a)
-                                      : launch_input_grad<T, 64, 64>(st, a);
+        const int rc = a.K <= 64 ? (a.rows >= 128 * 512 ? launch_input_grad<128, 64>(st, a) : launch_input_grad<64, 64>(st, a))
+                       : large >= 512 ? launch_input_grad<128, 128>(st, a)
+                                      : launch_input_grad<64, 64>(st, a);
         if (rc != MRX_OK) return rc;
     }
     if (!params) return MRX_OK;
     a.slices = p.slices, a.slice_rows = p.slice_rows, a.total = p.total;
     a.out = p.slices == 1 ? params : workspace;
     const int rc = p.wide ? (p.narrow >= 0 ? launch_wide<true>(st, a, p) : launch_wide<false>(st, a, p))
-                   : p.tn == 64 ? (p.tk == 64 ? launch_weight_grads<T, 64, 64>(st, a, p) : launch_weight_grads<T, 64, 128>(st, a, p))
-                              : (p.tk == 64 ? launch_weight_grads<T, 128, 64>(st, a, p) : launch_weight_grads<T, 128, 128>(st, a, p));
+                   : p.tn == 64 ? (p.tk == 64 ? launch_weight_grads<64, 64>(st, a, p, bf16) : launch_weight_grads<64, 128>(st, a, p, bf16))
+                                : (p.tk == 64 ? launch_weight_grads<128, 64>(st, a, p, bf16) : launch_weight_grads<128, 128>(st, a, p, bf16));
     if (rc != MRX_OK || p.slices == 1) return rc;
     return launch_column_sum(st, workspace, params, nullptr, p.slices, (int)p.total);
 }
 
-template <typename T> constexpr int big_lds = (int)dg_lds<T, 128, 128, 128, 128, KROW>();
+constexpr int big_lds = (int)dg_lds<128, 128, 128, 128, KROW>();
 const KernelRegistrar registrars[] = {
-    {reinterpret_cast<const void *>(dense_weight_grad_kernel<__bf16, 128, 128>), big_lds<__bf16>},
-    {reinterpret_cast<const void *>(dense_weight_grad_kernel<float, 128, 128>), big_lds<__bf16>},
-    {reinterpret_cast<const void *>(dense_input_grad_kernel<__bf16, 128, 128>), big_lds<__bf16>},
-    {reinterpret_cast<const void *>(dense_input_grad_kernel<float, 128, 128>), big_lds<__bf16>},
+    {reinterpret_cast<const void *>(dense_weight_grad_kernel<128, 128>), big_lds},
+    {reinterpret_cast<const void *>(split_weight_grad_kernel<128, 128>), (int)split_lds<128, 128>()},
+    {reinterpret_cast<const void *>(dense_input_grad_kernel<128, 128>), big_lds},
     {reinterpret_cast<const void *>(wide_weight_grad_kernel<false>), WideTile<false>::STAGES *WideTile<false>::STAGE},
     {reinterpret_cast<const void *>(wide_weight_grad_kernel<true>), WideTile<true>::STAGES *WideTile<true>::STAGE},
 };
@@ -552,7 +744,7 @@ extern "C" int64_t mrx_dense_grads_workspace(int64_t rows, int64_t K, const int6
         const WeightPlan p = plan_weights(rows, K, n_out, layers, dtype == MRX_BF16, bias_mask, wide);
         if (p.slices > 1) floats = p.slices * p.total > floats ? p.slices * p.total : floats;
     }
-    return floats;
+    return floats + (dtype == MRX_F32 ? split_pack_floats(n_out, layers, K, true) : 0);   // and the weights behind them
 }
 
 extern "C" int mrx_dense_grads(void *stream, const void *x, const void *const *dys, const void *const *weights, const int64_t *n_out,
@@ -581,10 +773,16 @@ extern "C" int mrx_dense_grads(void *stream, const void *x, const void *const *d
     bool wide = true;   // rows on the boundaries of whole requests
     for (int l = 0; l < layers; ++l) wide = wide && aligned(dys[l], n_out[l] <= WT_NARROW ? 4 : 16);
     const WeightPlan p = plan_weights(rows, K, n_out, layers, bf, bias_mask, wide);
-    if (params && p.slices > 1 && (!workspace || !aligned(workspace, 16))) return MRX_ERR_INVALID_ARG;
+    if (((params && p.slices > 1) || (dx && !bf)) && (!workspace || !aligned(workspace, 16))) return MRX_ERR_INVALID_ARG;
     if ((int64_t)p.tiles * p.slices >= (1ll << 31) || p.total >= (1ll << 31) || (rows + 63) / 64 * ((K + 63) / 64) >= (1ll << 31))
         return MRX_ERR_INVALID_ARG;
     if (const int rc = prepare_device(); rc != MRX_OK) return rc;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    return bf ? launch_grads<__bf16>(st, a, p, params, workspace) : launch_grads<float>(st, a, p, params, workspace);
+    if (dx && !bf) {
+        SplitCall c;
+        c.dys = dys, c.weights = weights, c.n_out = n_out, c.layers = layers, c.dx = dx, c.dx_bf16 = a.dx_bf16, c.rows = rows, c.K = K;
+        c.workspace = workspace + (p.slices > 1 ? p.slices * p.total : 0);
+        if (const int rc = split_rows(st, c); rc != MRX_OK) return rc;
+    }
+    return launch_grads(st, a, p, bf, params, workspace);
 }

@@ -52,7 +52,7 @@ using torch::autograd::variable_list;
     X(mrx_mamba_elements_fwd) X(mrx_mamba_elements_bwd) X(mrx_decay_last) X(mrx_mamba_readout_fwd)                   \
     X(mrx_mamba_readout_bwd) X(mrx_deltanet_step) X(mrx_mingru_step) X(mrx_row_dense) X(mrx_dense_grads) X(mrx_dense_grads_workspace)                  \
     X(mrx_gated_recurrence_act)                                                                                       \
-    X(mrx_dense_rows_suit) X(mrx_dense_pack) X(mrx_dense_rows) X(mrx_dense_rows_input_grad)                          \
+    X(mrx_dense_f32_workspace) X(mrx_dense_f32) X(mrx_dense_rows_suit) X(mrx_dense_pack) X(mrx_dense_rows) X(mrx_dense_rows_input_grad)                          \
     X(mrx_lru_step) X(mrx_mlstm_step) X(mrx_linear_attn_norm_fwd_chunk_parallel) X(mrx_linear_attn_norm_bwd_chunk_parallel) \
     X(mrx_gated_linear_attn_fwd_chunk_parallel) X(mrx_gated_linear_attn_bwd_chunk_parallel)
 struct {
@@ -1606,8 +1606,9 @@ std::vector<Tensor> dense_grads(const Tensor &x, const std::vector<Tensor> &dys,
     Tensor params, work;
     if (want_params) {
         params = fresh({(total + 3) / 4 * 4}, at::kFloat, x);
-        if (const int64_t floats = lib.mrx_dense_grads_workspace(rows, K, n.data(), (int)L, code(dt), bias)) work = fresh({floats}, at::kFloat, x);
     }
+    if (want_params || dt == at::kFloat)   // (where a float32 input gradient has its weights)
+        if (const int64_t floats = lib.mrx_dense_grads_workspace(rows, K, n.data(), (int)L, code(dt), bias)) work = fresh({floats}, at::kFloat, x);
     check(lib.mrx_dense_grads(stream(), ptr(x), dy.data(), w.data(), n.data(), (int)L, ptr(dx), fptr(params), fptr(work), rows, K, code(dt),
                               code(dx_dtype), bias),
           "mrx_dense_grads");
@@ -1629,27 +1630,31 @@ std::optional<ScalarType> autocast_dtype(const Tensor &x)
     return std::nullopt;
 }
 
-// Which of a group's gradients the library's kernels form.  Parameters: while they are bound by reading the rows, i.e. up to widths
-// where the array library's larger tiles take over (us, here / there: bfloat16 131072 x 256 -> 3 x 256 105 / 277, 11455 x 128 ->
-// 3 x 256 26 / 225, 32768 x 1024 -> 1024 148 / 121; float32 131072 x 256 -> 256 188 / 181, 23100 x 64 -> 256 26 / 99, 131072 x 512 ->
-// 3 x 512 2080 / 1740).  The input: several layers at once, as narrow (68200 x 128 -> 3 x 64 + 2 25 / 69, 131072 x 256 -> 3 x 256 + 4
-// 118 / 150; float32 68 / 93, but 131072 x 256 -> 3 x 256 536 / 454), or few rows, where the host's calls are what it costs.
-// In float32 the array library's slices also lead where they are whole and many and few layers have a bias, which it sums in a launch
-// of 50 us each (131072 rows, three layers without / with biases, here / there: 256 -> 256 481 / 393 and 547 / 570, 128 -> 256 252 / 221 and
-// 285 / 391).  From how many slices on, by width (three layers without biases, here / there): 128 -> 128 16 slices 52 / 63, 32 82 / 82,
-// 64 138 / 130; 128 -> 192 16 slices 79 / 100, 32 135 / 109; 160 -> 256 8 slices 77 / 96, 16 133 / 104; 192 -> 256 80 / 97 and 135 / 106;
-// 256 -> 256 81 / 75 and 136 / 122 (and four slices 53 / 58).
-bool params_suit(ScalarType dt, int64_t rows, int64_t K, int64_t widest, size_t layers, size_t biases)
+// Which of a group's gradients the library's kernels form.
+// bfloat16.  Parameters: while they are bound by reading the rows, i.e. up to widths where the array library's larger tiles take over (us,
+// here / there: 131072 x 256 -> 3 x 256 105 / 277, 11455 x 128 -> 3 x 256 26 / 225, 32768 x 1024 -> 1024 148 / 121).  The input: several layers at
+// once, as narrow (68200 x 128 -> 3 x 64 + 2 25 / 69, 131072 x 256 -> 3 x 256 + 4 118 / 150), or few rows, where the host's calls are what it costs.
+// float32, on the float16 matrix units (split_f16.h), in graphs and thus without the 20 us of the host that a product of the array library costs:
+// parameters 4096 x 128 -> 3 x 128 23 / 78, 4096 x 256 -> 3 x 256 35 / 79, 32768 x 256 -> 256 39 / 49, 131072 x 256 -> 3 x 256 + 4 315 / 425.  Wider
+// layers 256 x 512 -> 512 25 / 14, 1024 x 512 -> 512 29 / 15, 4096 x 512 -> 512 38 / 32, 4096 x 512 -> 3 x 512 65 / 83, 4096 x 1024 -> 1024 78 / 74, 16384 x
+// 1024 -> 1024 189 / 252, 32768 x 1024 -> 1024 357 / 504.  The input 4096 x 128 -> 3 x 128 26 / 22, 4096 x 256 -> 3 x 256 30 / 33, 131072 x 256 -> 3 x 256 +
+// 4 261 / 520; one layer 256 x 512 -> 512 24 / 15, 1024 x 512 -> 512 24 / 15, 4096 x 512 -> 512 26 / 27, 4096 x 1024 -> 1024 53 / 75, 32768 x 512 -> 256 47 / 83.
+// Sums of fewer than SPLIT_TERMS products stay float32's, whose error is that of their few additions: 64 terms 1.0e-7 here, 1.4e-7 there, 8 terms
+// 1.0e-7 and 0.3e-7.
+constexpr int64_t SPLIT_TERMS = 64, SPLIT_WIDEST = 1 << 20;
+bool params_suit(ScalarType dt, int64_t rows, int64_t K, int64_t widest, size_t, size_t)
 {
-    if (dt == at::kBFloat16) return K * widest <= 512 * 512;
-    if (K * widest > 256 * 256) return false;
-    if (2 * biases >= layers || K * widest < 128 * 192) return true;
-    return weight_gradient_slices(rows, widest, K) < (K * widest < 128 * 256 ? 32 : 16);
+    return dt == at::kBFloat16 ? K * widest <= 512 * 512 : rows >= SPLIT_TERMS && K * widest <= 256 * 256;
 }
-bool input_suits(ScalarType dt, int64_t rows, int64_t K, int64_t widest, size_t layers)
+// The same for float32 layers beyond that: results of many tiles, which the array library needs many rows to be slower at.
+bool wide_params_suit(ScalarType dt, int64_t rows, int64_t K, int64_t widest)
 {
-    const int64_t most = dt == at::kBFloat16 ? 256 : 128;
-    return layers > 1 && ((K <= most && widest <= most) || (rows <= 4096 && K * widest <= 512 * 512));
+    return dt == at::kFloat && K * widest > 256 * 256 && K * widest <= SPLIT_WIDEST && (rows >= 4096 || (rows >= SPLIT_TERMS && K * widest <= 256 * 1024));
+}
+bool input_suits(ScalarType dt, int64_t rows, int64_t K, int64_t widest, int64_t outputs, size_t layers)
+{
+    if (dt == at::kFloat) return outputs >= SPLIT_TERMS && K * widest <= SPLIT_WIDEST && (layers > 1 || rows >= 4096 || K * widest <= 256 * 512);
+    return layers > 1 && ((K <= 256 && widest <= 256) || (rows <= 4096 && K * widest <= 512 * 512));
 }
 
 // Layers in bfloat16 whose weights fit the registers of a compute unit: the rows pass all of them once, in either direction (dense_rows.hip).
@@ -1659,30 +1664,60 @@ struct RowLayers {
     Tensor transposed;             // (K, outputs of the wide layers): what the gradient of the input reads
 };
 
-// Whether these layers on x -- the rows in bfloat16 -- are such; their weights are not looked at beyond type, shape and place.
-int row_layers(const Tensor &x, const std::vector<Tensor> &weights, const std::vector<OptTensor> &biases, bool cast)
+// Outputs of layers whose parameters the kernels read where they lie -- dense, of the types that `suits` names, beside x -- or nothing.
+template <typename Suits>
+bool plain_layers(const Tensor &x, const std::vector<Tensor> &weights, const std::vector<OptTensor> &biases, Suits suits, std::array<int64_t, MRX_DENSE_LAYERS> &n)
 {
     auto plain = [&](const Tensor &t) {
         return t.device() == x.device() && t.has_storage() && !t.is_neg() && !t.key_set().has(c10::DispatchKey::Python);
     };
-    auto suits = [&](ScalarType dt) { return dt == at::kBFloat16 || (cast && dt == at::kFloat); };
-    if (!x.is_cuda() || !plain(x) || x.scalar_type() != at::kBFloat16 || x.dim() < 2 || x.numel() == 0 || weights.size() > MRX_DENSE_LAYERS) return 0;
+    if (!x.is_cuda() || !plain(x) || x.dim() < 2 || x.numel() == 0 || weights.size() > MRX_DENSE_LAYERS) return false;
     const int64_t K = x.size(-1);
     const auto wd = weights[0].scalar_type();
-    std::array<int64_t, MRX_DENSE_LAYERS> n{};
     std::optional<ScalarType> bd;
     for (size_t l = 0; l < weights.size(); ++l) {
         const Tensor &w = weights[l];
         if (!plain(w) || w.scalar_type() != wd || !suits(wd) || w.dim() != 2 || w.size(1) != K || !w.is_contiguous() ||
             reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 != 0)
-            return 0;
+            return false;
         n[l] = w.size(0);
         if (!biases[l].has_value()) continue;
-        if (!plain(*biases[l]) || !biases[l]->is_contiguous() || biases[l]->dim() != 1 || biases[l]->numel() != n[l] || !suits(biases[l]->scalar_type())) return 0;
-        if (bd.value_or(biases[l]->scalar_type()) != biases[l]->scalar_type()) return 0;
+        if (!plain(*biases[l]) || !biases[l]->is_contiguous() || biases[l]->dim() != 1 || biases[l]->numel() != n[l] || !suits(biases[l]->scalar_type())) return false;
+        if (bd.value_or(biases[l]->scalar_type()) != biases[l]->scalar_type()) return false;
         bd = biases[l]->scalar_type();
     }
-    return lib.mrx_dense_rows_suit(x.numel() / K, K, n.data(), (int)weights.size());
+    return true;
+}
+
+// Whether these layers on x -- the rows in bfloat16 -- are such; their weights are not looked at beyond type, shape and place.
+int row_layers(const Tensor &x, const std::vector<Tensor> &weights, const std::vector<OptTensor> &biases, bool cast)
+{
+    std::array<int64_t, MRX_DENSE_LAYERS> n{};
+    if (x.scalar_type() != at::kBFloat16 ||
+        !plain_layers(x, weights, biases, [&](ScalarType dt) { return dt == at::kBFloat16 || (cast && dt == at::kFloat); }, n))
+        return 0;
+    return lib.mrx_dense_rows_suit(x.numel() / x.size(-1), x.size(-1), n.data(), (int)weights.size());
+}
+
+// The outputs of float32 layers on float32 rows (dense_split.hip), residual: added to the one layer's; nothing where the library does not serve them.
+std::vector<Tensor> dense_f32(const Tensor &x_, const std::vector<Tensor> &weights, const std::vector<OptTensor> &biases, const Tensor &residual)
+{
+    std::vector<Tensor> out;
+    std::array<int64_t, MRX_DENSE_LAYERS> n{};
+    if (x_.scalar_type() != at::kFloat || !plain_layers(x_, weights, biases, [](ScalarType dt) { return dt == at::kFloat; }, n)) return out;
+    const int64_t K = x_.size(-1), rows = x_.numel() / K, floats = lib.mrx_dense_f32_workspace(n.data(), (int)weights.size(), K);
+    if (!floats || rows >= (1ll << 31) || K < SPLIT_TERMS || K * *std::max_element(n.begin(), n.end()) > SPLIT_WIDEST) return out;
+    const Tensor x = dense16(x_), work = fresh({floats}, at::kFloat, x);
+    std::array<const void *, MRX_DENSE_LAYERS> w{}, b{};
+    std::array<void *, MRX_DENSE_LAYERS> y{};
+    c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
+    for (size_t l = 0; l < weights.size(); ++l) {
+        shape.back() = n[l];
+        out.push_back(fresh(shape, at::kFloat, x));
+        w[l] = ptr(weights[l]), b[l] = ptr(biases[l]), y[l] = ptr(out[l]);
+    }
+    check(lib.mrx_dense_f32(stream(), fptr(x), w.data(), b.data(), y.data(), n.data(), (int)out.size(), fptr(residual), rows, K, fptr(work)), "mrx_dense_f32");
+    return out;
 }
 
 // The weights of such layers for the products: cast, and transposed where the input's gradient will be wanted.
@@ -1756,7 +1791,7 @@ struct DenseOp {
         std::vector<Tensor> dys, ws;   // of the layers whose outputs were used: the others cost no products
         std::vector<size_t> used;
         std::vector<bool> bias;
-        int64_t widest = 0;
+        int64_t widest = 0, outputs = 0;
         bool want_params = false, regular = x.is_cuda() && (dt == at::kFloat || dt == at::kBFloat16) && x2.size(1) % 8 == 0 && x2.numel() > 0;
         for (size_t l = 0; l < n; ++l) {
             if (!grads[l].defined()) continue;
@@ -1764,7 +1799,7 @@ struct DenseOp {
             dys.push_back((onto && across.defined() && grads[l].scalar_type() == at::kFloat ? grads[l] : grads[l].to(dt)).reshape({-1, ws.back().size(0)}).contiguous());
             used.push_back(l);
             bias.push_back(has_bias[l] && node.wants(1 + n + l));
-            widest = std::max(widest, ws.back().size(0));
+            widest = std::max(widest, ws.back().size(0)), outputs += ws.back().size(0);
             want_params = want_params || node.wants(1 + l) || bias.back();
             regular = regular && ws.back().device() == x.device() && ws.back().scalar_type() == dt && ws.back().is_contiguous() && ws.back().size(0) > 0 && reinterpret_cast<uintptr_t>(ws.back().data_ptr()) % 16 == 0;
         }
@@ -1772,9 +1807,11 @@ struct DenseOp {
         regular = regular && used.size() <= MRX_DENSE_LAYERS && x2.is_contiguous() && reinterpret_cast<uintptr_t>(x2.data_ptr()) % 16 == 0;
         const bool rows_dx = across.defined() && used.size() == n && regular && input_from_rows(dys, ws, across, x2.size(1), want_params, out);
         for (Tensor &dy : dys) dy = dy.to(dt);   // (a residual stream's gradient: unless that has left its rounded copy)
-        const bool own_params = want_params && regular && params_suit(dt, x2.size(0), x2.size(1), widest, used.size(), std::count(bias.begin(), bias.end(), true)),
+        const bool own_params = want_params && regular &&
+                                (params_suit(dt, x2.size(0), x2.size(1), widest, used.size(), std::count(bias.begin(), bias.end(), true)) ||
+                                 wide_params_suit(dt, x2.size(0), x2.size(1), widest)),
                    own_dx = node.wants(0) && !rows_dx && regular && (x_dtype == at::kFloat || x_dtype == at::kBFloat16) &&
-                            input_suits(dt, x2.size(0), x2.size(1), widest, used.size());
+                            input_suits(dt, x2.size(0), x2.size(1), widest, outputs, used.size());
         if (own_params || own_dx) {
             auto r = dense_grads(x2, dys, ws, bias, own_dx, x_dtype, own_params);
             if (own_dx) out[0] = r[0];
@@ -2023,6 +2060,8 @@ std::vector<Tensor> dense_group(const Tensor &x, const std::vector<Tensor> &weig
             auto layers = pack_layers(suit, weights, need_grad(x) && x.scalar_type() == at::kBFloat16);
             out = dense_rows(xc, layers, biases, Tensor());
             ws = std::move(layers.weights), transposed = layers.transposed;
+        } else if (need && weights.size() > 1 && (out = dense_f32(xc, weights, biases, Tensor()), !out.empty())) {
+            ws = weights;   // (a layer by itself has torch.nn.Linear's results bit for bit, and so has any without gradients)
         } else {
             for (size_t l = 0; l < weights.size(); ++l) {
                 ws.push_back(cast.has_value() ? weights[l].to(*cast) : weights[l]);

@@ -1,0 +1,131 @@
+"""Float32 dense layers on the float16 matrix units (csrc/dense_split.hip, the float32 kernels of csrc/dense_grads.hip) against double
+precision: sizes around their tiles and steps, rows and columns of very different magnitudes, infinities and NaN."""
+import pytest
+import torch
+
+from memorax_amd import _lib
+from memorax_amd.dense import Weights, dense_group
+
+pytestmark = pytest.mark.gpu
+
+EPS = 2.0 ** -24
+
+
+def _case(rows, K, outs, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(rows + K + len(outs) + seed)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    return rnd(rows, K), [rnd(n, K) for n in outs], [rnd(n) if i % 2 else None for i, n in enumerate(outs)], [rnd(rows, n) for n in outs]
+
+
+def _run(x, ws, bs, dys):
+    x, ws = x.clone().requires_grad_(), [w.clone().requires_grad_() for w in ws]
+    ys = dense_group(x, [Weights(w, b) for w, b in zip(ws, bs)])
+    torch.autograd.backward(ys, dys)
+    return [y.detach() for y in ys], x.grad, [w.grad for w in ws]
+
+
+def _close(got, a, b, add=None):
+    """got = a b (+ add) with a (m, k), b (k, n): an element is out by what splitting leaves of each product (2^-22) and by the roundings of
+    its running sum, together within 16 eps of the products' 2-norm -- eight times what they are on average."""
+    want = a.double() @ b.double()
+    size = (a.double().abs() ** 2 @ b.double().abs() ** 2).sqrt()
+    if add is not None:
+        want, size = want + add.double(), size + add.double().abs()
+    assert ((got.double() - want).abs() <= 16 * EPS * a.shape[1] ** 0.25 * size + 1e-38).all(), float(((got.double() - want).abs() / size.clamp_min(1e-30)).max() / EPS)
+
+
+@pytest.mark.parametrize("rows,K,outs", [(1, 64, [64, 3]), (63, 64, [1, 16, 17]), (65, 72, [130, 256]), (128, 256, [64, 64, 64, 2]), (129, 264, [48, 260]),
+                                         (300, 520, [16, 5, 16]), (4097, 256, [512, 256, 8]), (9000, 128, [128] * 8)])
+def test_sizes(rows, K, outs):
+    x, ws, bs, dys = _case(rows, K, outs)
+    print(f"case dense split rows={rows} K={K} outs={outs}", flush=True)
+    ys, dx, dws = _run(x, ws, bs, dys)
+    for y, w, b in zip(ys, ws, bs):
+        _close(y, x, w.t(), b)
+    _close(dx, torch.cat(dys, 1), torch.cat(ws))
+    for dw, dy in zip(dws, dys):
+        _close(dw, dy.t(), x)
+
+
+def test_magnitudes():
+    """Every row, and every column of the weights, has its own scale; a step of a longer contraction may be far larger or smaller than the one before."""
+    x, ws, bs, dys = _case(500, 520, [300, 16])
+    rows, feats = (torch.randint(-40, 40, (n,), generator=torch.Generator().manual_seed(n)).cuda() for n in (500, 300))
+    x = torch.ldexp(x, rows[:, None])
+    x[:, 256:] = torch.ldexp(x[:, 256:], torch.tensor(-18, device="cuda"))
+    x[7], x[8, 256:], x[9, :256] = 0., 0., 0.
+    ws[0] = torch.ldexp(ws[0], (feats[:, None] // 4))
+    ws[0][3] = 0.
+    dys[0][:, :256] = torch.ldexp(dys[0][:, :256], torch.tensor(30, device="cuda"))   # far above what follows it
+    ys, dx, dws = _run(x, ws, bs, dys)
+    for y, w, b in zip(ys, ws, bs):
+        _close(y, x, w.t(), b)
+    _close(dx, torch.cat(dys, 1), torch.cat(ws))
+
+
+@pytest.mark.parametrize("late", [False, True])
+def test_columns_that_grow_along_the_rows(late):
+    """The parameters' gradients rescale a column when a later step goes beyond the earlier ones, zeros first among them."""
+    x, ws, bs, dys = _case(2000, 64, [64, 8])
+    x[:, 5], dys[0][:, 9] = 0., 0.
+    at = slice(700, None) if late else slice(0, 40)
+    x[at, 3] = torch.ldexp(x[at, 3], torch.tensor(30, device="cuda"))
+    x[at, 5] = 1e-30
+    dys[0][at, 9] = 1e20
+    dys[1][at] = torch.ldexp(dys[1][at], torch.tensor(12, device="cuda"))
+    _, _, dws = _run(x, ws, bs, dys)
+    for dw, dy in zip(dws, dys):
+        _close(dw, dy.t(), x)
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+def test_what_is_not_finite(bad):
+    """What float32 makes of it: infinite or NaN where the operand has a part in the sum, everything else as without it."""
+    x, ws, bs, dys = _case(200, 128, [64, 72])
+    clean = _run(x, ws, bs, dys)
+    x1, w1, dy1 = x.clone(), [w.clone() for w in ws], [d.clone() for d in dys]
+    x1[70, 5] = bad
+    w1[1][9, 3] = bad
+    ys, _, dws = _run(x1, w1, bs, dys)
+    for l, y in enumerate(ys):
+        want = x1.double() @ w1[l].double().t() + (0 if bs[l] is None else bs[l].double())
+        assert torch.equal(torch.isnan(y), torch.isnan(want)) and torch.equal(torch.isposinf(y), torch.isposinf(want))
+        fine = torch.isfinite(want)
+        assert (y.double() - want)[fine].abs().max() <= 64 * EPS * 128
+    for l, dw in enumerate(dws):
+        fine = torch.ones(128, dtype=torch.bool, device="cuda")
+        fine[5] = False
+        assert not torch.isfinite(dw[:, 5]).any() and (dw - clean[2][l])[:, fine].abs().max() <= 64 * EPS * 200
+    dy1[0][70, 9] = bad
+    _, dx, dws = _run(x, ws, bs, dy1)
+    want = sum(d.double() @ w.double() for d, w in zip(dy1, ws))
+    assert torch.equal(torch.isnan(dx), torch.isnan(want)) and torch.equal(torch.isneginf(dx), torch.isneginf(want))
+    assert not torch.isfinite(dws[0][9]).any() and torch.isfinite(dws[1]).all() and torch.isfinite(dws[0][:9]).all()
+
+
+def test_residual_and_bfloat16_results():
+    """The C entry's residual sum, and an input gradient that is asked for in bfloat16."""
+    x, ws, _, dys = _case(1000, 128, [96])
+    got = _lib.native().dense_grads(x, dys, ws, [False], True, torch.bfloat16, False)[0]
+    want = dys[0].double() @ ws[0].double()
+    assert got.dtype == torch.bfloat16 and ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all()
+
+
+def test_graph_replays():
+    """Two launches and no memset: a captured call gives the eager result on every replay."""
+    x, ws, bs, dys = _case(700, 128, [64, 64])
+    ws = [w.requires_grad_() for w in ws]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        dense_group(x, [Weights(w, b) for w, b in zip(ws, bs)])
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ys = dense_group(x, [Weights(w, b) for w, b in zip(ws, bs)])
+    for k in range(3):
+        x.copy_(torch.randn(x.shape, device="cuda", generator=torch.Generator(device="cuda").manual_seed(k)))
+        want = dense_group(x, [Weights(w, b) for w, b in zip(ws, bs)])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(ys, want))
