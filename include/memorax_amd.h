@@ -650,12 +650,29 @@ int mrx_dense_grads(void *stream, const void *x, const void *const *dys, const v
 
 /* ---- Dense layers over rows in float32 ----
  * y_l (rows, n_out[l]) = x W_l^T + b_l of up to MRX_DENSE_LAYERS layers on the rows x (rows, K), everything float32 (entries of `biases` may be NULL);
- * residual (rows, n), nullable: added to the one layer's result.  K a multiple of 8.  Products on the float16 matrix units, every value as the sum of
+ * residual (rows, n), nullable: added to the one layer's result; skip (n) and skip_x (rows, n), both or neither: so is skip[c] skip_x[r][c].
+ * mrx_dense_f32_input_grad: dx (rows, K) = sum_l dy_l W_l, + skip[c] skip_x[r][c] with skip (K), skip_x (rows, K).  K a multiple of 8.  Products on the float16 matrix units, every value as the sum of
  * two scaled float16 ones (22 bits and a sign, 2^-39 of its row's or column's largest value); infinities and NaN as float32 has them.
- * workspace: mrx_dense_f32_workspace(...) floats (0: sizes that are not served), overwritten.  x, weights, results and workspace on 16-byte boundaries. */
+ * workspace: mrx_dense_f32_workspace(...), mrx_dense_f32_input_grad_workspace(...) floats (0: sizes that are not served), overwritten.  x, weights, results and workspace on 16-byte boundaries. */
 int64_t mrx_dense_f32_workspace(const int64_t *n_out, int layers, int64_t K);
 int mrx_dense_f32(void *stream, const float *x, const void *const *weights, const void *const *biases, void *const *outs,
-                  const int64_t *n_out, int layers, const float *residual, int64_t rows, int64_t K, float *workspace);
+                  const int64_t *n_out, int layers, const float *residual, const float *skip, const float *skip_x, int64_t rows, int64_t K,
+                  float *workspace);
+int64_t mrx_dense_f32_input_grad_workspace(const int64_t *n_out, int layers, int64_t K);
+int mrx_dense_f32_input_grad(void *stream, const void *const *dys, const void *const *weights, const int64_t *n_out, int layers, const float *skip,
+                             const float *skip_x, float *dx, int64_t rows, int64_t K, float *workspace);
+
+/* ---- The LRU cell's parameters as its recurrence and its two products read them (lru.py:76-108), float32 ----
+ * params: HOST array of nu_log, theta_log, gamma_log (N), B_real, B_imag (N,F), C_real, C_imag (F,N);
+ * mrx_lru_params_fwd: decay (N) complex64 = exp(-exp(nu_log) + i exp(theta_log)); wb (2N,F), rows 2n and 2n + 1 = exp(gamma_log[n]) (B_real, B_imag)[n];
+ *   wc (F,2N), columns 2n and 2n + 1 = (C_real, -C_imag)[:, n].
+ * mrx_lru_params_bwd: from the gradients of those (ddecay: of the real and of the imaginary part) the parameters', in the same order (grads).
+ * mrx_column_product: out (D) = the column sums of a b, (rows, D) each; workspace: mrx_column_product_workspace(...) floats. */
+int mrx_lru_params_fwd(void *stream, const float *const *params, void *decay, float *wb, float *wc, int64_t N, int64_t F);
+int mrx_lru_params_bwd(void *stream, const float *const *params, const void *ddecay, const float *dwb, const float *dwc, float *const *grads,
+                       int64_t N, int64_t F);
+int64_t mrx_column_product_workspace(int64_t rows, int64_t D);
+int mrx_column_product(void *stream, const float *a, const float *b, float *out, float *workspace, int64_t rows, int64_t D);
 
 /* ---- The acting step of a gated recurrence up to what its closing layer reads ----
  * x (rows, K) float32, normalised as mrx_row_dense does (norm 0, 1, 2; K a multiple of 8 up to 512); weights (N, K) without biases in w_dtype;

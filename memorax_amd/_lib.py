@@ -71,7 +71,13 @@ SIGNATURES = {
     "mrx_dense_grads_workspace": (_L, [_L] * 2 + [_P] + [_I] * 2 + [ctypes.c_uint]),
     "mrx_dense_grads": (_I, [_P] * 5 + [_I] + [_P] * 3 + [_L] * 2 + [_I] * 2 + [ctypes.c_uint]),
     "mrx_dense_f32_workspace": (_L, [_P, _I, _L]),
-    "mrx_dense_f32": (_I, [_P] * 6 + [_I, _P] + [_L] * 2 + [_P]),
+    "mrx_dense_f32": (_I, [_P] * 6 + [_I] + [_P] * 3 + [_L] * 2 + [_P]),
+    "mrx_dense_f32_input_grad_workspace": (_L, [_P, _I, _L]),
+    "mrx_dense_f32_input_grad": (_I, [_P] * 4 + [_I] + [_P] * 3 + [_L] * 2 + [_P]),
+    "mrx_lru_params_fwd": (_I, [_P] * 5 + [_L] * 2),
+    "mrx_lru_params_bwd": (_I, [_P] * 6 + [_L] * 2),
+    "mrx_column_product_workspace": (_L, [_L] * 2),
+    "mrx_column_product": (_I, [_P] * 5 + [_L] * 2),
     "mrx_dense_rows_suit": (_I, [_L] * 2 + [_P, _I]),
     "mrx_dense_pack": (_I, [_P] * 3 + [_I, _L, _I] + [_P] * 2),
     "mrx_dense_rows": (_I, [_P] * 6 + [_I, _P] + [_L] * 2 + [_I]),

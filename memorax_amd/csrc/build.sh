@@ -16,7 +16,7 @@ cd "$(dirname "$0")"
 HIPCC=${HIPCC:-/opt/rocm/bin/hipcc}
 FLAGS=(--offload-arch=gfx950 -O3 -std=c++17 -fPIC -I../../include
        -Xclang -target-feature -Xclang -packed-fp32-ops -Wall -Wno-unused-function)
-SRCS=(api.hip scan.hip chunk_fwd.hip chunk_bwd.hip step.hip delta_tm.hip la_states.hip mlstm_gates.hip rms_norm.hip gate.hip conv_cells.hip row_dense.hip dense_grads.hip dense_rows.hip dense_split.hip act_cells.hip gated_step.hip)
+SRCS=(api.hip scan.hip chunk_fwd.hip chunk_bwd.hip step.hip delta_tm.hip la_states.hip mlstm_gates.hip rms_norm.hip gate.hip conv_cells.hip lru_cells.hip row_dense.hip dense_grads.hip dense_rows.hip dense_split.hip act_cells.hip gated_step.hip)
 pids=()
 compile() {  # compile <object suffix> <extra flags...>
     local suf=$1; shift

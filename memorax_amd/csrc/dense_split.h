@@ -14,6 +14,7 @@ struct SplitCall {
     const void *const *weights = nullptr, *const *biases = nullptr;
     void *const *outs = nullptr;
     const float *residual = nullptr;
+    const float *skip = nullptr, *skip_x = nullptr;   // skip[c] skip_x[r][c] is added to the one result
     void *dx = nullptr;
     bool dx_bf16 = false;
     const int64_t *n_out = nullptr;

@@ -1,7 +1,7 @@
 // Dense layers over rows in float32, forward and with respect to their input, on the float16 matrix units (split_f16.h):
 //
-//     y_l = x W_l^T + b_l      a group of layers that read the same rows;  y = residual + (x W^T + b) for one
-//     dx  = sum_l dy_l W_l     of such a group
+//     y_l = x W_l^T + b_l      a group of layers that read the same rows;  y = residual + (x W^T + b + skip z) for one
+//     dx  = sum_l dy_l W_l     of such a group, + skip z
 //
 // In float32 these are bound by the matrix units -- 154 TFLOP/s dense where float16 has sixteen times that -- and the array library runs
 // one product per layer and direction, at three quarters of the float32 rate over many rows, for 20 us of the host each.  Here a group is two
@@ -45,7 +45,7 @@ struct SplitArgs {
     SplitOut out[MRX_DENSE_LAYERS];  // what the columns belong to: the layers, or the input
     const f16x8 *packed;
     const int *exps;       // (steps, 16 tiles): exponent of each column
-    const float *residual;
+    const float *residual, *skip, *skip_x;
     int64_t rows;
     int ins, outs, steps, tiles, passes, groups, K;
     bool y_bf16;
@@ -223,6 +223,7 @@ template <int NT, bool ACROSS> __global__ void __launch_bounds__(SP_THREADS, NT 
     auto store = [&](int l, int64_t r, int c, float y) {
         const SplitOut &o = a.out[l];
         if (o.b) y += o.b[c];
+        if (a.skip) y = fmaf(a.skip[c], a.skip_x[r * o.n + c], y);
         if (a.residual) y += a.residual[r * o.n + c];
         if (ACROSS && a.y_bf16) static_cast<__bf16 *>(o.y)[r * o.n + c] = (__bf16)y;
         else static_cast<float *>(o.y)[r * o.n + c] = y;
@@ -341,6 +342,7 @@ template <int NT, bool ACROSS> __global__ void __launch_bounds__(SP_THREADS, NT 
                     if (c >= o.n) continue;
                     if (o.b) y += sf32x4{o.b[c], o.b[c + 1], o.b[c + 2], o.b[c + 3]};
                     const int64_t at = r * o.n + c;
+                    if (a.skip) y += *reinterpret_cast<const sf32x4 *>(a.skip + c) * *reinterpret_cast<const sf32x4 *>(a.skip_x + at);
                     if (a.residual) y += *reinterpret_cast<const sf32x4 *>(a.residual + at);
                     if (ACROSS && a.y_bf16) {
                         typedef __bf16 b4 __attribute__((ext_vector_type(4)));
@@ -407,7 +409,7 @@ int split_rows(hipStream_t st, const SplitCall &c)
     const Sizes z = sizes_of(c.n_out, c.layers, c.K, across);
     if (!z.ok || !c.workspace || !aligned(c.workspace, 16) || c.rows <= 0 || c.rows >= (1ll << 31)) return MRX_ERR_INVALID_ARG;
     SplitArgs a{};
-    a.rows = c.rows, a.K = (int)c.K, a.steps = (int)z.steps, a.tiles = (int)z.tiles, a.residual = c.residual, a.y_bf16 = c.dx_bf16;
+    a.rows = c.rows, a.K = (int)c.K, a.steps = (int)z.steps, a.tiles = (int)z.tiles, a.residual = c.residual, a.skip = c.skip, a.skip_x = c.skip_x, a.y_bf16 = c.dx_bf16;
     int64_t widest = 0;
     int step = 0, block = 0, tile = 0;
     auto in = [&](const float *x, const float *w, int64_t n) {
@@ -445,16 +447,34 @@ int split_rows(hipStream_t st, const SplitCall &c)
 extern "C" int64_t mrx_dense_f32_workspace(const int64_t *n_out, int layers, int64_t K) { return mrx::split_pack_floats(n_out, layers, K, false); }
 
 extern "C" int mrx_dense_f32(void *stream, const float *x, const void *const *weights, const void *const *biases, void *const *outs,
-                             const int64_t *n_out, int layers, const float *residual, int64_t rows, int64_t K, float *workspace)
+                             const int64_t *n_out, int layers, const float *residual, const float *skip, const float *skip_x, int64_t rows, int64_t K,
+                             float *workspace)
 {
     using namespace mrx;
+    if (!skip != !skip_x || (skip && layers != 1) || !aligned(skip, 16) || !aligned(skip_x, 16)) return MRX_ERR_INVALID_ARG;
     if (!x || !weights || !biases || !outs || !n_out || layers < 1 || layers > MRX_DENSE_LAYERS || !aligned(x, 16) || !aligned(residual, 16) || (residual && layers != 1))
         return MRX_ERR_INVALID_ARG;
     for (int l = 0; l < layers; ++l)
         if (!weights[l] || !outs[l] || !aligned(weights[l], 16) || !aligned(outs[l], 16) || !aligned(biases[l], 4)) return MRX_ERR_INVALID_ARG;
     if (const int rc = prepare_device(); rc != MRX_OK) return rc;
     SplitCall c;
-    c.x = x, c.weights = weights, c.biases = biases, c.outs = outs, c.residual = residual, c.n_out = n_out, c.layers = layers, c.rows = rows, c.K = K;
+    c.x = x, c.weights = weights, c.biases = biases, c.outs = outs, c.residual = residual, c.skip = skip, c.skip_x = skip_x, c.n_out = n_out, c.layers = layers, c.rows = rows, c.K = K;
+    c.workspace = workspace;
+    return split_rows(static_cast<hipStream_t>(stream), c);
+}
+
+extern "C" int64_t mrx_dense_f32_input_grad_workspace(const int64_t *n_out, int layers, int64_t K) { return mrx::split_pack_floats(n_out, layers, K, true); }
+
+extern "C" int mrx_dense_f32_input_grad(void *stream, const void *const *dys, const void *const *weights, const int64_t *n_out, int layers, const float *skip,
+                                        const float *skip_x, float *dx, int64_t rows, int64_t K, float *workspace)
+{
+    using namespace mrx;
+    if (!dys || !weights || !n_out || !dx || layers < 1 || layers > MRX_DENSE_LAYERS || !aligned(dx, 16) || !skip != !skip_x || !aligned(skip, 16) || !aligned(skip_x, 16))
+        return MRX_ERR_INVALID_ARG;
+    for (int l = 0; l < layers; ++l)
+        if (!dys[l] || !weights[l] || !aligned(dys[l], 4) || !aligned(weights[l], 16)) return MRX_ERR_INVALID_ARG;
+    SplitCall c;
+    c.dys = dys, c.weights = weights, c.dx = dx, c.skip = skip, c.skip_x = skip_x, c.n_out = n_out, c.layers = layers, c.rows = rows, c.K = K;
     c.workspace = workspace;
     return split_rows(static_cast<hipStream_t>(stream), c);
 }

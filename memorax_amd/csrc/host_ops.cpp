@@ -52,7 +52,8 @@ using torch::autograd::variable_list;
     X(mrx_mamba_elements_fwd) X(mrx_mamba_elements_bwd) X(mrx_decay_last) X(mrx_mamba_readout_fwd)                   \
     X(mrx_mamba_readout_bwd) X(mrx_deltanet_step) X(mrx_mingru_step) X(mrx_row_dense) X(mrx_dense_grads) X(mrx_dense_grads_workspace)                  \
     X(mrx_gated_recurrence_act)                                                                                       \
-    X(mrx_dense_f32_workspace) X(mrx_dense_f32) X(mrx_dense_rows_suit) X(mrx_dense_pack) X(mrx_dense_rows) X(mrx_dense_rows_input_grad)                          \
+    X(mrx_dense_f32_workspace) X(mrx_dense_f32) X(mrx_dense_f32_input_grad_workspace) X(mrx_dense_f32_input_grad) X(mrx_lru_params_fwd)                       \
+    X(mrx_lru_params_bwd) X(mrx_column_product_workspace) X(mrx_column_product) X(mrx_dense_rows_suit) X(mrx_dense_pack) X(mrx_dense_rows) X(mrx_dense_rows_input_grad)                          \
     X(mrx_lru_step) X(mrx_mlstm_step) X(mrx_linear_attn_norm_fwd_chunk_parallel) X(mrx_linear_attn_norm_bwd_chunk_parallel) \
     X(mrx_gated_linear_attn_fwd_chunk_parallel) X(mrx_gated_linear_attn_bwd_chunk_parallel)
 struct {
@@ -1700,7 +1701,8 @@ int row_layers(const Tensor &x, const std::vector<Tensor> &weights, const std::v
 }
 
 // The outputs of float32 layers on float32 rows (dense_split.hip), residual: added to the one layer's; nothing where the library does not serve them.
-std::vector<Tensor> dense_f32(const Tensor &x_, const std::vector<Tensor> &weights, const std::vector<OptTensor> &biases, const Tensor &residual)
+std::vector<Tensor> dense_f32(const Tensor &x_, const std::vector<Tensor> &weights, const std::vector<OptTensor> &biases, const Tensor &residual,
+                              const Tensor &skip = Tensor(), const Tensor &skip_x = Tensor())
 {
     std::vector<Tensor> out;
     std::array<int64_t, MRX_DENSE_LAYERS> n{};
@@ -1716,7 +1718,9 @@ std::vector<Tensor> dense_f32(const Tensor &x_, const std::vector<Tensor> &weigh
         out.push_back(fresh(shape, at::kFloat, x));
         w[l] = ptr(weights[l]), b[l] = ptr(biases[l]), y[l] = ptr(out[l]);
     }
-    check(lib.mrx_dense_f32(stream(), fptr(x), w.data(), b.data(), y.data(), n.data(), (int)out.size(), fptr(residual), rows, K, fptr(work)), "mrx_dense_f32");
+    check(lib.mrx_dense_f32(stream(), fptr(x), w.data(), b.data(), y.data(), n.data(), (int)out.size(), fptr(residual), fptr(skip), fptr(skip_x), rows, K,
+                            fptr(work)),
+          "mrx_dense_f32");
     return out;
 }
 
@@ -2089,7 +2093,8 @@ Tensor dense_onto(const Tensor &residual, const Tensor &x, const Tensor &weight,
     c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
     shape.back() = weight.size(0);
     const auto cast = autocast_dtype(x);
-    if (residual.sizes() != IntArrayRef(shape) || (cast.has_value() ? *cast : x.scalar_type()) != at::kBFloat16) return composed();
+    const auto product = cast.has_value() ? *cast : x.scalar_type();
+    if (residual.sizes() != IntArrayRef(shape) || (product != at::kBFloat16 && (cast.has_value() || product != at::kFloat))) return composed();
     const bool need_x = need_grad(x), need_params = need_grad(weight, bias);
     const bool need = (at::GradMode::is_enabled() && differentiable(residual)) || need_x || need_params;
     RowLayers layers;
@@ -2098,8 +2103,12 @@ Tensor dense_onto(const Tensor &residual, const Tensor &x, const Tensor &weight,
     {
         c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
         at::AutoDispatchBelowADInplaceOrView below;
-        xc = x.to(at::kBFloat16);
+        xc = x.to(product);
         const int suit = row_layers(xc, {weight}, {bias}, cast.has_value());
+        if (product == at::kFloat && need) {
+            out = dense_f32(xc, {weight}, {bias}, residual);
+            layers.weights = {weight};
+        }
         if (suit & MRX_DENSE_ROWS_RESIDUAL) {
             xc = dense16(xc);
             layers = pack_layers(suit, {weight}, need_x && x.scalar_type() == at::kBFloat16);
@@ -2109,6 +2118,107 @@ Tensor dense_onto(const Tensor &residual, const Tensor &x, const Tensor &weight,
     if (out.empty()) return composed();
     if (need) record_dense(x, xc, {weight}, {bias}, layers.weights, layers.transposed, residual, out);
     return out[0];
+}
+
+// ---- the LRU cell (lru_cells.hip around dense_split.hip and scan.hip)
+struct LruOp {
+    enum { X, H, H0, PARAMS, D_ = PARAMS + 7, DECAY, WB, WC, SAVED };   // the parameters in the order of lru_cells.hip, the skip vector behind them
+    static constexpr bool ONCE = true;
+    static const char *name() { return "MemoraxLruBackward"; }
+    Tensor done;
+    bool onto;   // a residual was added to the result
+    variable_list backward(OpNode<LruOp> &node, std::array<Tensor, SAVED> &s, variable_list &grads)
+    {
+        for (int i = 0; i < SAVED; ++i) {   // a hook on saved tensors may hand them on in another layout
+            s[i] = dense16(s[i]);
+            chk(s[i], "saved tensor", i == H || i == H0 || i == DECAY ? at::kComplexFloat : at::kFloat);
+        }
+        const Tensor &x = s[X], &h = s[H];
+        const int64_t B = x.size(0), T = x.size(1), F = x.size(2), N = h.size(2), rows = B * T;
+        variable_list out(10 + onto);   // x, eight parameters, h0 (, the residual)
+        if (onto) out.back() = grads[0];
+        const Tensor dy = dense16(grad_or_zeros(grads[0], x)).view({rows, F}), x2 = x.view({rows, F});
+        const auto read = dense_grads(at::view_as_real(h).view({rows, 2 * N}), {dy}, {s[WC]}, {false}, true, at::kFloat, true);
+        const auto r = scan_bwd(s[DECAY], h, done, some(s[H0]), at::view_as_complex(read[0].view({B, T, N, 2})), some(as(grads[1], at::kComplexFloat)), true);
+        const Tensor du = at::view_as_real(r.db).view({rows, 2 * N}), dwb = dense_grads(x2, {du}, {}, {false}, false, at::kFloat, true)[1];
+        out[9] = r.dh0;
+        if (node.wants(0)) {
+            const int64_t n = 2 * N;
+            const Tensor work = fresh({lib.mrx_dense_f32_input_grad_workspace(&n, 1, F)}, at::kFloat, x);
+            const void *dys = ptr(du), *ws = ptr(s[WB]);
+            out[0] = fresh_like(x);
+            check(lib.mrx_dense_f32_input_grad(stream(), &dys, &ws, &n, 1, fptr(s[D_]), fptr(dy), fptr(out[0]), rows, F, fptr(work)), "mrx_dense_f32_input_grad");
+        }
+        if (node.wants(1 + 7)) {
+            const int64_t floats = lib.mrx_column_product_workspace(rows, F);
+            const Tensor work = floats ? fresh({floats}, at::kFloat, x) : Tensor();
+            out[1 + 7] = fresh({F}, at::kFloat, x);
+            check(lib.mrx_column_product(stream(), fptr(dy), fptr(x2), fptr(out[1 + 7]), fptr(work), rows, F), "mrx_column_product");
+        }
+        const Tensor decay = sum_rows(r.da);
+        const float *params[7];
+        float *dparams[7];
+        for (int i = 0; i < 7; ++i) {
+            params[i] = fptr(s[PARAMS + i]);
+            out[1 + i] = fresh_like(s[PARAMS + i]);
+            dparams[i] = fptr(out[1 + i]);
+        }
+        check(lib.mrx_lru_params_bwd(stream(), params, ptr(decay), fptr(dwb), fptr(read[1]), dparams, N, F), "mrx_lru_params_bwd");
+        return out;
+    }
+};
+
+// x (B,T,F) float32 through the cell, residual (nullable, as x) added; p: nu_log, theta_log, gamma_log, B_real, B_imag, C_real, C_imag, D; the
+// carry's leaves (B,N) complex64.  y, and the carry's leaves afterwards.  F and 2 N multiples of eight.
+std::tuple<Tensor, Tensor, Tensor> lru_layer(const Tensor &x_, const OptTensor &residual_, const std::vector<Tensor> &p, const Tensor &done, const Tensor &h0_,
+                                             const Tensor &P0_)
+{
+    TORCH_CHECK_VALUE(x_.dim() == 3 && p.size() == 8 && p[3].dim() == 2, "lru_layer: x (B,T,F) and eight parameters");
+    const int64_t B = x_.size(0), T = x_.size(1), F = x_.size(2), N = p[3].size(0);
+    TORCH_CHECK_VALUE(F % 8 == 0 && N % 4 == 0 && B * T > 0, "lru_layer takes a multiple of eight features and of four states");
+    refuse(done, P0_);
+    bool need = need_grad(x_, residual_, h0_);
+    for (const Tensor &t : p) need = need_grad(t) || need;
+    chk_beside(x_, residual_, p, done, h0_, P0_);
+    Tensor x, residual, h0, decay, wb, wc, y;
+    std::vector<Tensor> q;
+    ScanOut r;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        x = dense16(x_), residual = dense16(residual_), h0 = h0_.contiguous();
+        for (const Tensor &t : p) q.push_back(dense16(t));
+        chk(x, "x", at::kFloat);
+        if (residual.defined()) chk(residual, "residual", at::kFloat, x.sizes());
+        const float *params[8];
+        const char *names[] = {"nu_log", "theta_log", "gamma_log", "B_real", "B_imag", "C_real", "C_imag", "D"};
+        const std::vector<int64_t> shapes[] = {{N}, {N}, {N}, {N, F}, {N, F}, {F, N}, {F, N}, {F}};
+        for (int i = 0; i < 8; ++i) chk(q[i], names[i], at::kFloat, shapes[i]), params[i] = fptr(q[i]);
+        decay = fresh({N}, at::kComplexFloat, x), wb = fresh({2 * N, F}, at::kFloat, x), wc = fresh({F, 2 * N}, at::kFloat, x);
+        check(lib.mrx_lru_params_fwd(stream(), params, ptr(decay), fptr(wb), fptr(wc), N, F), "mrx_lru_params_fwd");
+        const auto u = dense_f32(x, {wb}, {std::nullopt}, Tensor());
+        TORCH_CHECK_VALUE(!u.empty(), "lru_layer: sizes that the float32 products do not serve");
+        r = scan_fwd(decay, at::view_as_complex(u[0].view({B, T, N, 2})), done, some(h0), some(P0_.contiguous()), true);
+        y = dense_f32(at::view_as_real(r.h).view({B, T, 2 * N}), {wc}, {std::nullopt}, residual, q[7], x)[0];
+    }
+    if (need) {
+        auto node = std::shared_ptr<OpNode<LruOp>>(new OpNode<LruOp>(), torch::autograd::deleteNode);
+        node->op.done = done, node->op.onto = residual_.has_value();
+        torch::autograd::edge_list edges = torch::autograd::collect_next_edges(x_);
+        for (const Tensor &t : p) edges.push_back(torch::autograd::impl::gradient_edge(t));
+        edges.push_back(torch::autograd::impl::gradient_edge(h0_));
+        if (residual_.has_value()) edges.push_back(torch::autograd::impl::gradient_edge(*residual_));
+        node->set_next_edges(std::move(edges));
+        torch::autograd::set_history(y, node);
+        torch::autograd::set_history(r.h_last, node);
+        node->keep(LruOp::X, x);
+        node->keep(LruOp::H, r.h);
+        node->keep(LruOp::H0, h0);
+        for (int i = 0; i < 8; ++i) node->keep(LruOp::PARAMS + i, q[i]);
+        node->keep(LruOp::DECAY, decay);
+        node->keep(LruOp::WB, wb);
+        node->keep(LruOp::WC, wc);
+    }
+    return {y, r.h_last, r.P_last};
 }
 
 // ---- causal depthwise convolution over time with silu behind it (conv_cells.hip)
@@ -2454,6 +2564,7 @@ PYBIND11_MODULE(_native, m)
     def("params_suit", &params_suit);
     def("weight_gradient", &weight_gradient);
     def("weight_gradient_slices", &weight_gradient_slices);
+    def("lru_layer", &lru_layer);
     def("causal_conv_silu", &causal_conv_silu);
     def("mamba_mix", &mamba_mix);
 }

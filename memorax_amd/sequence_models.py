@@ -92,6 +92,10 @@ class MemoroidCellBase(nn.Module):
         """read(scan(self(x))) as one operation, (next_carry, y), where a cell has it for these arrays; else None."""
         return None
 
+    def whole_onto(self, residual, x, done, initial_carry):
+        """(next_carry, residual + y) with y as ``whole`` forms it, where a cell's last product takes the sum with it; else None."""
+        return None
+
     def acting(self, x, norm, done, carry):
         """(next_carry, x + read(scan(self(norm(x))))) for one time step without gradients (``_acts``), where a cell has its
         launches fused for these arrays; else None."""
@@ -185,10 +189,14 @@ class Memoroid(SequenceModel):
         return next_carry, y
 
     def onto(self, residual, inputs, done, carry):
-        if not (type(self).forward is Memoroid.forward and type(self.cell).whole is MemoroidCellBase.whole and self.cell.closes()):
+        if type(self).forward is not Memoroid.forward:
             return None
         if carry is None:
             carry = self.cell.initialize_carry(None, get_input_shape(inputs))
+        if type(self.cell).whole is not MemoroidCellBase.whole:
+            return self.cell.whole_onto(residual, inputs, done, carry)
+        if not self.cell.closes():
+            return None
         h, next_carry = self.cell.scan(self.cell(inputs), carry, done)
         layer, rows = self.cell.closing(h, inputs)
         return next_carry, native().dense_onto(residual, rows, layer.weight, layer.bias)
@@ -268,8 +276,30 @@ class LRUCell(_DiagonalCell):
     def read(self, h, x, **kwargs):
         return _real_read_out(h[0], torch.stack([self.C_real, -self.C_imag], -1)) + self.D * x
 
+    def _parameters_in_order(self):
+        return [self.nu_log, self.theta_log, self.gamma_log, self.B_real, self.B_imag, self.C_real, self.C_imag, self.D]
+
+    def whole(self, x, done, initial_carry):
+        """The layer as one native operation (lru_cells.hip around the products and the scan) where gradients are recorded: float32 on the
+        device, rows of whole vectors.  Of the composition's array operations two thirds make and differentiate small matrices of parameters."""
+        return self._layer(None, x, done, initial_carry)
+
+    def whole_onto(self, residual, x, done, initial_carry):
+        return self._layer(residual, x, done, initial_carry) if type(self).whole is LRUCell.whole else None
+
+    def _layer(self, residual, x, done, initial_carry):
+        params = self._parameters_in_order()
+        if not (torch.is_grad_enabled() and _as_written(self, LRUCell) and x.is_cuda and x.dtype is torch.float32 and x.dim() == 3
+                and autocast_dtype(x) is None and x.shape[0] * x.shape[1] >= _SPLIT_TERMS <= self.features and 2 * self.hidden_dim >= _SPLIT_TERMS
+                and x.shape[2] == self.features and self.features % 8 == 0 and self.hidden_dim % 4 == 0 and 2 * self.hidden_dim * self.features <= 1 << 20
+                and all(p.dtype is torch.float32 for p in params)):
+            return None
+        h0, P0 = initial_carry
+        y, h, P = native().lru_layer(x, residual, params, done, h0[:, 0], P0[:, 0])
+        return (h[:, None], P[:, None]), y
+
     def acting(self, x, norm, done, carry):
-        params = [self.nu_log, self.theta_log, self.gamma_log, self.B_real, self.B_imag, self.C_real, self.C_imag, self.D]
+        params = self._parameters_in_order()
         # fused / composed, in a graph and host-issued (us, features = hidden width): 1024 x 512 64 / 75 and 61 / 146, 4096 x 512 190 / 142 and
         # 180 / 147, 256 x 1024 66 / 78 and 64 / 146, 1024 x 1024 227 / 133 and 213 / 145
         if not (_as_written(self, LRUCell) and autocast_dtype(x) is None and self.hidden_dim % 8 == 0 and 2 * self.hidden_dim <= _RMS_NORM_MAX_D
@@ -486,6 +516,7 @@ class GatedLinearRecurrence(SequenceModel):
 # ----------------------------------------------------------------------------------
 # acting: one time step without gradients (ppo.py:105-143), rows = environments
 # ----------------------------------------------------------------------------------
+_SPLIT_TERMS = 64        # the fewest terms of a sum that csrc/host_ops.cpp (SPLIT_TERMS) gives to the float16 matrix units
 _ACTING_ROWS = 16384   # the most rows that csrc/host_ops.cpp (rows_pay) gives to the row kernels
 
 
@@ -816,6 +847,14 @@ class MambaCell(MemoroidCellBase):
         y, carry = self._mix(dense_group(x, [self.input_projection, self.B, self.C, self.dt]), done, initial_carry)
         return carry, self.output_projection(y)
 
+    def whole_onto(self, residual, x, done, initial_carry):
+        layer = self.output_projection
+        if not (type(self).whole is MambaCell.whole and self._native_sizes() and _as_written(self, MambaCell) and x.is_cuda and x.dtype == torch.float32
+                and x.dim() == 3 and x.shape[0] * x.shape[1] > 0 and autocast_dtype(x) is None):
+            return None
+        y, carry = self._mix(dense_group(x, [self.input_projection, self.B, self.C, self.dt]), done, initial_carry)
+        return carry, native().dense_onto(residual, y, layer.weight, layer.bias)
+
     def _native_sizes(self):
         P = self.head_dim
         return (type(self.norm) is _RMSNorm and self.norm.scale.dtype == torch.float32 and _plain(self.output_projection)
@@ -1122,7 +1161,7 @@ class Residual(nn.Module):
         if inputs.is_cuda and _forks(inner):   # x + f(norm(x)): one kernel takes both gradients of x
             inputs, normed = inner.norm.fork(inputs)
             if (isinstance(inner.module, SequenceModel) and not kwargs and inputs.is_cuda and inputs.dtype is torch.float32
-                    and normed.dtype is torch.bfloat16 and not _hooked(inner.module)):   # a mixed-precision block on a float32 stream
+                    and normed.dtype in (torch.bfloat16, torch.float32) and not _hooked(inner.module)):   # the closing layer adds to the stream
                 summed = inner.module.onto(inputs, normed, done, initial_carry)
                 if summed is not None:
                     return summed
