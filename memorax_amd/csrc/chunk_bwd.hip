@@ -6,8 +6,9 @@
 // triangular factor Tm (Tm_chk); everything else of the forward (U', masked QK^T) is
 // recomputed per chunk.  A chunk that
 // contains resets is processed once per episode, last episode first, with the rows
-// of the other episodes zeroed by select; dS only flows into the episode that
-// leaves the chunk and only out of the episode that enters it.
+// of the other episodes zeroed by select -- or all of its episodes at once, kept apart by masks
+// (chunk_common.h); dS only flows into the episode that leaves the chunk and only out of the
+// episode that enters it.
 //
 // Linear attention per pass (rows i >= j; all rows of one episode):
 //   Aqk = tril(Q K^T)                      dV  = Aqk^T dO + K dS^T
@@ -109,6 +110,7 @@ la_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restr
     using P4 = typename TT<T>::pack4;
     constexpr int LDD = L::LDD, LDC = L::LDC;
     extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ int sMixed[NW];   // of each wave: its part of the chunk fails the screen
     T *sQ = reinterpret_cast<T *>(smem + L::oQ);
     T *sK = reinterpret_cast<T *>(smem + L::oK);
     T *sV = reinterpret_cast<T *>(smem + L::oV);
@@ -343,23 +345,60 @@ la_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restr
             *reinterpret_cast<P4 *>(dst + (TMR::nt(w, j) * 16 + li) * LDD + TMR::mt(w, j) * 16 + 4 * lg) = h[j];
     };
 
-    for (int c = c_hi; c >= c_lo; --c) {
+    int c = c_hi, unit = -1, whole = 0;   // unit: of chunk c, the next to be done (-1: none yet); whole: it is the only one
+    // ONE: a unit of a chunk that holds resets; otherwise the chunks up to the next that does (chunk_common.h)
+    auto walk = [&](auto one, const int tid) __attribute__((always_inline)) {
+    constexpr bool ONE = decltype(one)::value;
+    const int lane = tid & 63, li = lane & 15, lg = lane >> 4;
+    for (; c >= c_lo; --c) {
         const int t0 = c * C;
         const unsigned long long dmask = __ballot(done_test(rdone, done_f32) && lane < C);
         const int nres = __popcll(dmask);
+        if (!ONE && __builtin_expect(nres != 0, 0)) break;
         const bool ckpt = PAR || !WALK || nres != 0 || (c > 0 && c % walk_anchor<T>() == 0);  // the entering state comes from S_chk
         if (WALK && !PAR)  // for the chunk prefetched during this one
             need_S = __ballot(done_test(rdone2, done_f32) && lane < C) != 0ull || (c >= 2 && (c - 1) % walk_anchor<T>() == 0);
-        for (int pass = nres; pass >= 0; --pass) {
-            auto live = [&](int r) { return nres == 0 || episode_of(dmask, r) == pass; };
-            // gated: cumulative log-decay of this pass's episode (as in the forward kernel)
+        if (ONE && unit < 0) {
+            bool ok = IO::within(rq, LA_MERGE_MAX) && IO::within(rk, LA_MERGE_MAX) && IO::within(rv, LA_MERGE_MAX) && IO::within(rdo, LA_MERGE_MAX);
+            if (NORM) {
+                ok = ok && IO::within(ro, LA_MERGE_MAX);
+#pragma unroll
+                for (int p = 0; p < IO::PASSES; ++p)
+                    ok = ok && rden[p] >= LA_MERGE_DEN && rden[p] <= LA_MERGE_DEN_MAX && fabsf(rdss[p]) <= LA_MERGE_MAX;
+            }
+            if (lane == 0) sMixed[w] = __ballot(!ok) != 0ull;
+            sync_lds();
+            whole = __builtin_amdgcn_readfirstlane(sMixed[0] | sMixed[1] | sMixed[2] | sMixed[3]) == 0;
+            unit = whole ? 0 : nres;
+        }
+        const bool mg = ONE && anew(whole);   // all episodes of this chunk in one unit
+        // rows below r_first: the episode that enters the chunk; from r_last on: the one that leaves it
+        const int r_first = mg ? (int)__builtin_ctzll(dmask) : C, r_last = mg ? 63 - (int)__builtin_clzll(dmask) : 0;
+        // of a [64][C] tile the columns (chunk rows) below or from `end` on, zeros elsewhere
+        auto keep_below = [&](f32x4 *acc, int end) {
+#pragma unroll
+            for (int j = 0; j < TMR::TPW; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[j][e] = TMR::nt(w, j) * 16 + li < end ? acc[j][e] : 0.f;
+        };
+        auto keep_from = [&](f32x4 *acc, int end) {
+#pragma unroll
+            for (int j = 0; j < TMR::TPW; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[j][e] = TMR::nt(w, j) * 16 + li >= end ? acc[j][e] : 0.f;
+        };
+        {
+            const int pass = ONE ? unit : 0;
+            auto live = [&](int r) { return nres == 0 || mg || episode_of(dmask, r) == pass; };
+            // gated: cumulative log-decay of this pass's episode (as in the forward kernel), of each of the chunk's if it is one unit
             float G = 0.f, Glast = 0.f;
             if (GATED) {
+                const int start = mg ? episode_start(dmask, lane) : 0;
                 G = (lane < C && live(lane) && !((dmask >> lane) & 1ull)) ? rg : 0.f;
 #pragma unroll
                 for (int off = 1; off < C; off <<= 1) {
                     const float up = __shfl_up(G, off);
-                    if (lane >= off) G += up;
+                    if (lane - off >= start) G += up;
                 }
                 Glast = __shfl(G, C - 1);
                 if (w == 0 && lane < C) {
@@ -374,7 +413,7 @@ la_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restr
                     IO::template fmap<FMAP>(fq);
                     IO::template fmap<FMAP>(fk);
                 }
-                if (nres != 0) {
+                if (nres != 0 && !mg) {
                     IO::mask_rows(fq, tid, live);
                     IO::mask_rows(fk, tid, live);
                     IO::mask_rows(fv, tid, live);
@@ -424,10 +463,10 @@ la_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restr
                     IOS::to_lds(fS, sS, LDD, tid);  // S[dv][dk]
                 }
             }
-            if (pass != nres) zero_acc<TMS::TPW>(dSacc);  // an episode that ends inside the chunk
+            if (pass != nres && !mg) zero_acc<TMS::TPW>(dSacc);  // an episode that ends inside the chunk
             store_acc<T, HD, HD, NW>(dSacc, sDS, LDD, w, lane);  // dS[dv][dk]
             if (NORM) {
-                if (pass != nres) zero_acc<TMS::MBW>(dzacc);
+                if (pass != nres && !mg) zero_acc<TMS::MBW>(dzacc);
                 if (w < TMS::WM && (VN ? lg == 0 : li == 0)) {
 #pragma unroll
                     for (int mi = 0; mi < TMS::MBW; ++mi) {
@@ -436,6 +475,10 @@ la_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restr
                         else *reinterpret_cast<f32x4 *>(dst + 4 * lg) = dzacc[mi];
                     }
                 }
+            }
+            if (mg) {  // what flows on past the chunk is the first episode's own
+                zero_acc<TMS::TPW>(dSacc);
+                zero_acc<TMS::MBW>(dzacc);
             }
             sync_lds();
             const bool pre = pass == 0 && c > c_lo;
@@ -450,16 +493,18 @@ la_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restr
 #pragma unroll
                     for (int j = 0; j < TMA::TPW; ++j) {
                         const int m = TMA::mt(w, j) * 16 + 4 * lg, n = TMA::nt(w, j) * 16 + li;
+                        const int start = mg ? episode_start(dmask, n) : 0;
+                        auto keep = [&](int e) { return ONE ? of_pair(m, e, n, start) : m + e <= n; };
                         float x[4];
                         const float dd = (NORM && add_dden) ? sDd[n] : 0.f;
                         if (GATED) {
                             const float gn = sG[n];
                             const f32x4 gm = *reinterpret_cast<const f32x4 *>(sG + m);
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) x[e] = (m + e <= n) ? a[j][e] * __expf(gn - gm[e]) : 0.f;
+                            for (int e = 0; e < 4; ++e) x[e] = keep(e) ? a[j][e] * __expf(gn - gm[e]) : 0.f;
                         } else {
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) x[e] = (m + e <= n) ? a[j][e] + dd : 0.f;
+                            for (int e = 0; e < 4; ++e) x[e] = keep(e) ? a[j][e] + dd : 0.f;
                         }
                         *reinterpret_cast<P4 *>(dst + n * LDC + m) = TT<T>::pack(x[0], x[1], x[2], x[3]);
                     }
@@ -518,10 +563,12 @@ la_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restr
             {
                 f32x4 acc[TMR::TPW];
                 zero_acc<TMR::TPW>(acc);
-                if (GATED) {  // the state term of row j carries b_j = exp(G_last - G_j)
+                if constexpr (GATED || ONE) {  // the state term of row j carries b_j = exp(G_last - G_j)
                     gemm<T, HD, C, HD, ROWK, ROWK, NW>(acc, sDS, LDD, sK, LDD, w, lane);
+                    if (GATED)
 #pragma unroll
-                    for (int j = 0; j < TMR::TPW; ++j) acc[j] *= __expf(Glast - sG[TMR::nt(w, j) * 16 + li]);
+                        for (int j = 0; j < TMR::TPW; ++j) acc[j] *= __expf(Glast - sG[TMR::nt(w, j) * 16 + li]);
+                    if (ONE) keep_from(acc, r_last);
                     gemm<T, HD, C, C, KROW, KROW, NW>(acc, sDO, LDD, sAqk, LDC, w, lane);
                 } else {
                     gemm<T, HD, C, C, KROW, KROW, NW>(acc, sDO, LDD, sAqk, LDC, w, lane);
@@ -539,13 +586,14 @@ la_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restr
 #pragma unroll
                     for (int j = 0; j < TMR::TPW; ++j) acc[j] *= __expf(sG[TMR::nt(w, j) * 16 + li]);
                 }
+                if (ONE) keep_below(acc, r_first);
                 gemm<T, HD, C, C, KROW, ROWK, NW>(acc, sK, LDD, sDAqk, LDC, w, lane);
                 if (GATED) rowdot(acc, sQ, 1.f);
                 if (NORM && pass == 0) {  // den_i = q_i . (z_in + ...): dQ_i += dden_i z_in
 #pragma unroll
                     for (int j = 0; j < TMR::TPW; ++j) {
                         const f32x4 zz = *reinterpret_cast<const f32x4 *>(sZf + TMR::mt(w, j) * 16 + 4 * lg);
-                        acc[j] += zz * sDd[TMR::nt(w, j) * 16 + li];
+                        acc[j] += zz * (!ONE || TMR::nt(w, j) * 16 + li < r_first ? sDd[TMR::nt(w, j) * 16 + li] : 0.f);
                     }
                 }
                 auto sc = [&](int r, int d0) {
@@ -559,20 +607,24 @@ la_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restr
             {
                 f32x4 acc[TMR::TPW];
                 zero_acc<TMR::TPW>(acc);
-                if (GATED) {
-                    gemm<T, HD, C, HD, KROW, ROWK, NW>(acc, sDS, LDD, sV, LDD, w, lane);
-#pragma unroll
-                    for (int j = 0; j < TMR::TPW; ++j) acc[j] *= __expf(Glast - sG[TMR::nt(w, j) * 16 + li]);
-                    gemm<T, HD, C, C, KROW, KROW, NW>(acc, sQ, LDD, sDAqk, LDC, w, lane);
-                    rowdot(acc, sK, -1.f);
-                } else {
-                    gemm<T, HD, C, C, KROW, KROW, NW>(acc, sQ, LDD, sDAqk, LDC, w, lane);
-                    gemm<T, HD, C, HD, KROW, ROWK, NW>(acc, sDS, LDD, sV, LDD, w, lane);
-                }
-                if (NORM && pass == nres) {  // every key of the leaving episode is part of the z that leaves
+                auto add_dz = [&]() {  // every key of the leaving episode is part of the z that leaves
 #pragma unroll
                     for (int j = 0; j < TMR::TPW; ++j)
                         acc[j] += *reinterpret_cast<const f32x4 *>(sDZ + TMR::mt(w, j) * 16 + 4 * lg);
+                };
+                if constexpr (GATED || ONE) {
+                    gemm<T, HD, C, HD, KROW, ROWK, NW>(acc, sDS, LDD, sV, LDD, w, lane);
+                    if (GATED)
+#pragma unroll
+                        for (int j = 0; j < TMR::TPW; ++j) acc[j] *= __expf(Glast - sG[TMR::nt(w, j) * 16 + li]);
+                    if (NORM && (mg || pass == nres)) add_dz();
+                    if (ONE) keep_from(acc, r_last);
+                    gemm<T, HD, C, C, KROW, KROW, NW>(acc, sQ, LDD, sDAqk, LDC, w, lane);
+                    if (GATED) rowdot(acc, sK, -1.f);
+                } else {
+                    gemm<T, HD, C, C, KROW, KROW, NW>(acc, sQ, LDD, sDAqk, LDC, w, lane);
+                    gemm<T, HD, C, HD, KROW, ROWK, NW>(acc, sDS, LDD, sV, LDD, w, lane);
+                    if (NORM && pass == nres) add_dz();
                 }
                 auto sc = [&](int r, int d0) {
                     const P4 x = *reinterpret_cast<const P4 *>(sK + r * LDD + d0);
@@ -583,7 +635,7 @@ la_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restr
             }
             // ---- dS^T[dk][dv] += sum_c Q[c][dk] dO[c][dv]  (gated: c dS + sum_c a_c Q[c] dO[c]) -----
             if (GATED) {
-                const float cl = __expf(Glast);
+                const float cl = mg ? 1.f : __expf(Glast);  // (one unit: what it would decay is zero)
 #pragma unroll
                 for (int j = 0; j < TMS::TPW; ++j) dSacc[j] *= cl;
 #pragma unroll
@@ -598,6 +650,7 @@ la_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restr
 #pragma unroll
             for (int mi = 0; mi < TMS::MBW; ++mi) dzpart[mi] = 0.f;
             auto dz_q = [&](int mi, int kb, Frag &xq) {
+                if (ONE && !GATED) keep_rows<T, true>(xq, kb, lg, r_first);
                 if (NORM) {  // dz[dk] += sum_i Q[i][dk] dden_i
                     if (VN) {
                         const float *dd = sDd + kb * TT<T>::KB + TT<T>::KP * lg;
@@ -611,6 +664,7 @@ la_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restr
                     const float *ea = sEa + kb * TT<T>::KB + TT<T>::KP * lg;
 #pragma unroll
                     for (int e = 0; e < TT<T>::KP; ++e) xq[e] = (T)((float)xq[e] * ea[e]);
+                    if (ONE) keep_rows<T, true>(xq, kb, lg, r_first);
                 }
             };
             if (!PAR) gemm<T, HD, HD, C, KROW, KROW, NW>(dSacc, sQ, LDD, sDO, LDD, w, lane, dz_q);
@@ -628,7 +682,7 @@ la_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restr
             park(hQ, sQ);
             park(hK, sK);
             pend_dmask = dmask;
-            pend_nres = nres;
+            pend_nres = mg ? 0 : nres;
             pend_pass = pass;
             pend_t0 = t0;
             sync_lds();
@@ -639,17 +693,28 @@ la_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restr
 #pragma unroll
                     for (int sl = 0; sl < TMR::WM; ++sl) x += sE[sl * C + lane];
                 }
-                // x_r <- sum over the rows i >= r of this pass's episode (its rows are consecutive)
+                // x_r <- sum over the rows i >= r of row r's episode (consecutive rows; of a pass only one episode's are not zero)
+                const int start = mg ? episode_start(dmask, lane) : 0;
 #pragma unroll
                 for (int off = 1; off < C; off <<= 1) {
                     const float up = __shfl_down(x, off);
-                    if (lane + off < C) x += up;
+                    if (lane + off < C && (!mg || episode_start(dmask, lane + off) == start)) x += up;
                 }
-                if (pass == nres) x += dg_carry;  // the episode that reaches the end of the chunk goes on into the later steps
+                if (mg ? lane >= r_last : pass == nres) x += dg_carry;  // the episode that reaches the end of the chunk goes on into the later steps
                 if (on && t0 + lane < Tlen) dg[((int64_t)b * Tlen + t0 + lane) * H + h] = ((dmask >> lane) & 1ull) ? 0.f : x;
                 if (pass == 0) dg_carry = (dmask & 1ull) ? 0.f : __shfl(x, 0);  // cut where the chunk opens with a reset
             }
         }
+        if (ONE) {
+            if (unit-- == 0) --c;
+            return;
+        }
+    }
+    };
+    for (;;) {
+        walk(std::false_type{}, tid);
+        if (__builtin_expect(c < c_lo, 1)) break;
+        walk(std::true_type{}, here(tid));
     }
     flush_pending();  // the last pass ended with a barrier
     if (dS0 && !PAR) {

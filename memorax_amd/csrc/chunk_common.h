@@ -68,6 +68,12 @@ template <typename T> constexpr int walk_anchor() { return sizeof(T) == 2 ? 128 
 // row dots behind dbeta, 2^6 x 2^6 x 2^110), inside the float32 range.
 constexpr float MERGE_IN_MAX = 64.f, MERGE_STATE_MAX = 1048576.f;
 
+// The same for linear attention and its forms, which have no chain of products: what a masked zero meets there are the staged rows alone
+// (and the weights dden of the normalised form's backward), everything else is dropped by select.  Inputs of at most LA_MERGE_MAX,
+// and denominators of at least LA_MERGE_DEN behind them, keep those finite: dout / den, with a gradient of the sums of squares
+// (2^20 + 2^41) 2^24, and dden 2^67 2^24.
+constexpr float LA_MERGE_MAX = 1048576.f, LA_MERGE_DEN = 5.9604645e-8f, LA_MERGE_DEN_MAX = 1.1529215e18f;
+
 // A 16-byte global load of data that no later kernel reads again (the residuals a backward call consumes):
 // non-temporal, so that it does not displace what the next kernels will read -- inputs, and the residuals the
 // forward call has just written -- from the last-level cache.  Row stores of results take the same hint
@@ -325,6 +331,17 @@ template <typename T, int R, int NTHR, int COLS = HD> struct TileIO {
         }
     }
 
+    // every element of this thread's at most `lim` in magnitude; false for NaN
+    static __device__ __forceinline__ bool within(const Regs &r, float lim)
+    {
+        bool ok = true;
+#pragma unroll
+        for (int p = 0; p < PASSES; ++p)
+#pragma unroll
+            for (int e = 0; e < KP; ++e) ok = ok && fabsf((float)r.v[p][e]) <= lim;
+        return ok;
+    }
+
     // zero the rows for which keep(row) is false (select, not multiply)
     template <typename KeepF> static __device__ __forceinline__ void mask_rows(Regs &r, int tid, KeepF keep)
     {
@@ -427,6 +444,56 @@ __device__ __forceinline__ int sequence_of_block(int i, int nblocks, int H)
 __device__ __forceinline__ int episode_of(unsigned long long dmask, int r)
 {
     return __popcll(dmask & ((2ull << r) - 1ull));
+}
+
+// The first row of row r's episode in the chunk (0: that of the episode that enters it).
+__device__ __forceinline__ int episode_start(unsigned long long dmask, int r)
+{
+    const unsigned long long before = dmask & ((2ull << r) - 1ull);
+    return before ? 63 - __builtin_clzll(before) : 0;
+}
+
+// ---- all episodes of a chunk in one unit (linear attention) -------------------------
+// A chunk with resets used to cost a unit of work per episode.  Masks do it in one: the [C][C] products keep pairs of one episode, what comes of the
+// state entering the chunk the rows of the first episode, what comes of the state's gradient leaving it those of the last, and the update takes the rows of
+// the one that goes on.  A masked zero then meets other episodes' rows in a product, so the chunk is screened first (LA_MERGE_MAX above); one that fails is
+// worked per episode, whose zeros are put in by select.
+// The masks stand in a copy of the unit of their own: chunks without resets run in a loop that ends at the first that has some, one unit of that is done
+// behind it, and so on.  In the same straight-line code they cost a chunk without resets 3 to 18 %; behind branches, or with the two units on the sides of one, 10
+// to 30 % or a hundred spilled registers (what the second side needs stays live across the first).  `here` and the expected end of the outer loop keep
+// what the second unit needs out of the first one's registers.
+// us, forward and backward, a unit per episode / one unit: float32 64 x 256 x 4 x 64 at a reset per 200 steps 108 / 86, per 33 154 / 93; bfloat16 64 x 512 x 4 x 64 74 / 60
+// and 126 / 71; gated 256 x 128 x 8 x 64, per 100, float32 349 / 292, bfloat16 152 / 119; normalised 382 / 349 and 163 / 143.  Without resets 0.96 to 1.0 of what
+// it took: a loop that knows there are none is the leaner one.
+__device__ __forceinline__ int here(int x)   // a value whose uses cannot be moved out of the loop they stand in
+{
+    asm volatile("" : "+v"(x));
+    return x;
+}
+__device__ __forceinline__ bool anew(int x)   // a wave-wide truth value that is another one at each use: no second copy of the code is made for it
+{
+    x = __builtin_amdgcn_readfirstlane(x);
+    asm volatile("" : "+s"(x));
+    return x != 0;
+}
+// Is row m + e of row n's episode, which starts at `start`, and not behind n?
+__device__ __forceinline__ bool of_pair(int m, int e, int n, int start) { return e <= n - m && e >= start - m; }
+// Elements of an operand fragment along the chunk's rows (element e of k block kb: row kb KB + KP lg + e): those of rows below `end` (BELOW)
+// or from `end` on, zeros elsewhere.
+template <typename T, bool BELOW> __device__ __forceinline__ void keep_rows(typename TT<T>::frag &x, int kb, int lg, int end)
+{
+    const int rel = end - TT<T>::KP * lg, r0 = kb * TT<T>::KB;
+    auto in = [&](int e) { return BELOW ? r0 + e < rel : r0 + e >= rel; };
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+        for (int e = 0; e < TT<T>::KP; ++e) x[e] = in(e) ? x[e] : 0.f;
+    } else {
+        typedef uint32_t words_t __attribute__((ext_vector_type(4)));
+        words_t v = __builtin_bit_cast(words_t, x);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] &= (in(2 * i) ? 0x0000ffffu : 0u) | (in(2 * i + 1) ? 0xffff0000u : 0u);
+        x = __builtin_bit_cast(typename TT<T>::frag, v);
+    }
 }
 
 // ---- inverse of a unit lower-triangular matrix (fp32 arithmetic) -----------------

@@ -11,7 +11,8 @@
 // with the rows of all other episodes replaced by zeros *by select*; the episode that
 // enters the chunk sees S, later episodes start from 0, and only the episode that
 // leaves the chunk updates S.  Inside a pass only the causal mask remains, and a
-// non-finite value can never meet a masked-out zero inside a matrix product.
+// non-finite value can never meet a masked-out zero inside a matrix product.  Where the
+// chunk's inputs rule one out, linear attention does all its episodes in one pass (chunk_common.h).
 // The state is kept transposed (S^T, d_k x d_v) in MFMA accumulators for the whole
 // sequence and re-staged to LDS as a T-typed d_v x d_k tile once per chunk.
 #include <type_traits>
@@ -113,6 +114,7 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
     using P4 = typename TT<T>::pack4;
     constexpr int LDD = L::LDD, LDC = L::LDC, LDA = L::LDA;
     extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ int sMixed[DELTA ? 1 : NW];   // of each wave: its part of the chunk fails the screen
     T *sQ = reinterpret_cast<T *>(smem + L::oQ);
     T *sK = reinterpret_cast<T *>(smem + L::oK);
     T *sV = reinterpret_cast<T *>(smem + L::oV);    // delta rule: holds beta_j V_j
@@ -262,10 +264,20 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
     };
     int64_t schk_off = (int64_t)bh * NC * dvw * dkw;                                 // S_chk[c]
     int64_t tmchk_off = (int64_t)bh * NC * C * C + (int64_t)tid * 4;                                  // row-major C x C
-    for (int c = c_first; c < c_end; ++c, schk_off += dvw * dkw, tmchk_off += C * C, den_off += C) {
+    // ONE (linear attention): a unit of a chunk that holds resets; otherwise the chunks up to the next that does (chunk_common.h)
+    int c = c_first;
+    [[maybe_unused]] int unit = -1, whole = 0;   // linear attention: of chunk c, the next to be done (-1: none yet); it is the only one
+    auto next_chunk = [&]() { ++c, schk_off += dvw * dkw, tmchk_off += C * C, den_off += C; };
+    auto walk = [&](auto one, const int tid) __attribute__((always_inline)) {
+    constexpr bool ONE = decltype(one)::value;
+    const int lane = tid & 63, li = lane & 15, lg = lane >> 4;
+    for (; c < c_end; next_chunk()) {
         const int t0 = c * C;
         const unsigned long long dmask = __ballot(done_test(rdone, done_f32) && lane < C);
         const int nres = __popcll(dmask);
+        if constexpr (!ONE && !DELTA) {
+            if (__builtin_expect(nres != 0, 0)) break;
+        }
         bool mg = false;  // this chunk's episodes in one unit
         if constexpr (MERGE) {
             if (nres != 0) {
@@ -295,20 +307,31 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
                 mg = sBeta[0] + sBeta[1] + sBeta[2] + sBeta[3] == 0.f;
             }
         }
+        if constexpr (ONE) {
+            if (unit < 0) {
+                const bool ok = IO::within(rq, LA_MERGE_MAX) && IO::within(rk, LA_MERGE_MAX) && IO::within(rv, LA_MERGE_MAX);
+                if (lane == 0) sMixed[w] = __ballot(!ok) != 0ull;
+                sync_lds();
+                whole = __builtin_amdgcn_readfirstlane(sMixed[0] | sMixed[1] | sMixed[2] | sMixed[3]) == 0;
+                unit = 0;
+            }
+            mg = anew(whole);
+        }
         const int npass = mg ? 0 : nres;
         const int r_first = mg ? (int)__builtin_ctzll(dmask) : C;        // rows below it: the episode that enters the chunk
         const int r_last = mg ? 63 - (int)__builtin_clzll(dmask) : 0;   // rows from it on: the episode that leaves it
-        for (int pass = 0; pass <= npass; ++pass) {
+        for (int pass = ONE ? unit : 0; pass <= (ONE ? unit : npass); ++pass) {   // (ONE: a unit a call)
             auto live = [&](int r) { return nres == 0 || mg || episode_of(dmask, r) == pass; };
             // gated: G_i = sum of the log-decays of this pass's episode up to row i (the decay of an
             // episode's first step multiplies a zero state and is left out); every wave scans its copy
             float G = 0.f, Glast = 0.f;
             if (GATED) {
+                const int start = ONE && mg ? episode_start(dmask, lane) : 0;   // one unit: of each of its episodes
                 G = (lane < C && live(lane) && !((dmask >> lane) & 1ull)) ? rg : 0.f;
 #pragma unroll
                 for (int off = 1; off < C; off <<= 1) {
                     const float up = __shfl_up(G, off);
-                    if (lane >= off) G += up;
+                    if (lane - off >= start) G += up;
                 }
                 Glast = __shfl(G, C - 1);
                 if (w == 0 && lane < C) {
@@ -417,6 +440,10 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
                     }
                 }
             }
+            if (ONE && mg) {  // the state that leaves is the last episode's own
+                zero_acc<TMS::TPW>(Sacc);
+                zero_acc<TMS::MBW>(zacc);
+            }
             const bool pre = pass == npass && c + 1 < c_end;
             if (pre) { prefetch_part(0); prefetch_part(1); }
             if (TMIN && pre) { prefetch_part(2); prefetch_part(3); }
@@ -458,11 +485,21 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
 #pragma unroll
                     for (int j = 0; j < TMA::TPW; ++j) {
                         const int m = TMA::mt(w, j) * 16 + 4 * lg, n = TMA::nt(w, j) * 16 + li;
+                        const int start = ONE && mg ? episode_start(dmask, n) : 0;
                         const float gn = sG[n];
                         const f32x4 gm = *reinterpret_cast<const f32x4 *>(sG + m);
                         float x[4];
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) x[e] = (m + e <= n) ? acc[j][e] * __expf(gn - gm[e]) : 0.f;
+                        for (int e = 0; e < 4; ++e) x[e] = (ONE ? of_pair(m, e, n, start) : m + e <= n) ? acc[j][e] * __expf(gn - gm[e]) : 0.f;
+                        *reinterpret_cast<P4 *>(sAqk + n * LDC + m) = TT<T>::pack(x[0], x[1], x[2], x[3]);
+                    }
+                } else if constexpr (ONE) {
+#pragma unroll
+                    for (int j = 0; j < TMA::TPW; ++j) {
+                        const int m = TMA::mt(w, j) * 16 + 4 * lg, n = TMA::nt(w, j) * 16 + li, start = mg ? episode_start(dmask, n) : 0;
+                        float x[4];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) x[e] = of_pair(m, e, n, start) ? acc[j][e] : 0.f;
                         *reinterpret_cast<P4 *>(sAqk + n * LDC + m) = TT<T>::pack(x[0], x[1], x[2], x[3]);
                     }
                 } else if (MERGE && mg) {
@@ -548,6 +585,17 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
 #pragma unroll
                 for (int j = 0; j < TMO::TPW; ++j) Oacc[j] *= __expf(sG[TMO::nt(w, j) * 16 + li]);
             }
+            if constexpr (ONE) {  // the entering state is the first episode's alone
+#pragma unroll
+                for (int j = 0; j < TMO::TPW; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) Oacc[j][e] = TMO::nt(w, j) * 16 + li < r_first ? Oacc[j][e] : 0.f;
+                if (NORM)
+#pragma unroll
+                    for (int ni = 0; ni < TMO::NBW; ++ni)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) dacc[ni][e] = TMO::nt(w, ni) * 16 + li < r_first ? dacc[ni][e] : 0.f;
+            }
             gemm<T, HD, C, C, KROW, ROWK, NW>(Oacc, sU, LDD, sAqk, LDC, w, lane, NoHook(), den_a);
             if (NORM) {
                 if (VN) {  // the lane groups hold partial sums over their k slots
@@ -598,7 +646,7 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
             if (pass == npass && !PAR) {
                 if (MERGE && mg) zero_acc<TMS::TPW>(Sacc);  // a chunk with resets: the state that leaves is the last episode's own
                 if (GATED) {  // S <- exp(G_last) S + sum_c exp(G_last - G_c) K[c] U'[c]
-                    const float cl = __expf(Glast);
+                    const float cl = ONE && mg ? 1.f : __expf(Glast);  // (one unit: what it would decay is zero)
 #pragma unroll
                     for (int j = 0; j < TMS::TPW; ++j) Sacc[j] *= cl;
                 }
@@ -606,6 +654,7 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
 #pragma unroll
                 for (int mi = 0; mi < TMS::MBW; ++mi) zpart[mi] = 0.f;
                 auto z_k = [&](int mi, int kb, Frag &xk) {
+                    if (ONE && !GATED) keep_rows<T, false>(xk, kb, lg, r_last);
                     if (NORM) {  // z[dk] += sum_c K[c][dk]
                         if (VN) {
 #pragma unroll
@@ -618,6 +667,7 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
                         const float *eb = sEb + kb * TT<T>::KB + TT<T>::KP * lg;
 #pragma unroll
                         for (int e = 0; e < TT<T>::KP; ++e) xk[e] = (T)((float)xk[e] * eb[e]);
+                        if (ONE) keep_rows<T, false>(xk, kb, lg, r_last);
                     }
                     if (MERGE && mg) {  // rows of the last episode only (element e of the fragment is chunk row k0 + e)
                         const int k0 = kb * TT<T>::KB + TT<T>::KP * lg;
@@ -645,6 +695,16 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
                 na.ss[(int64_t)bh * Tlen + t0 + tid] = x;  // the slots are next written after the next unit's barriers
             }
         }
+        if (ONE) {
+            if (unit++ == npass) unit = -1, next_chunk();
+            return;
+        }
+    }
+    };
+    for (;;) {
+        walk(std::false_type{}, tid);
+        if (DELTA || __builtin_expect(c >= c_end, 1)) break;
+        if constexpr (!DELTA) walk(std::true_type{}, here(tid));
     }
     flush_o();  // the last unit ended with a barrier
 
