@@ -74,13 +74,11 @@ typedef enum {
  *   every such chunk first (|q|, |k|, |v|, |beta|, |dout| and the factor's entries <= 2^6, the state's and its
  *   gradient's <= 2^20: bounds under which no intermediate can leave the float32 range) and fall back to
  *   the units per episode for a chunk that fails, so the results are those of MRX_RESETS_PASSES for any data.
- *   For callers whose episodes end every hundred steps or so (ppo.py:181-190): a chunk with a reset
- *   then costs what a chunk without one costs (measured, B=64 T=1024 H=8 bf16 at one reset per hundred steps:
- *   backward 197 -> 169 us; at one per five hundred the two are level, without resets the merged instance
- *   is 5 % behind).  The forward call merges where it takes the chunk-parallel factor kernel
- *   (mrx_factor_path), the backward call always; head dim 64 at full width, 32-row chunks -- elsewhere the
- *   argument is accepted and the units per episode run.  The two calls of a pair need not agree.
- * MRX_RESETS_AUTO: MRX_RESETS_PASSES. */
+ *   The forward call merges where it takes the chunk-parallel factor kernel (mrx_factor_path) at head dim 64 and full width: for
+ *   callers whose episodes end every hundred steps or so, a chunk without resets is 5 % behind there.  The backward call merges always
+ *   (32-row chunks), and chunks without resets pay nothing.  The two calls of a pair need not agree.
+ * MRX_RESETS_AUTO: the forward call as MRX_RESETS_PASSES; the backward call as MRX_RESETS_MERGED but for bfloat16 on fewer sequences than
+ *   the device has compute units. */
 typedef enum {
     MRX_RESETS_AUTO = 0,
     MRX_RESETS_PASSES = 1,

@@ -778,7 +778,8 @@ template <typename T, int C, int NW> struct DeltaBwdSmem : BwdDims<T, C> {
 static __device__ unsigned long long g_phase_clocks[4];
 #endif
 
-// MERGE: a chunk that holds resets is done in ONE unit instead of one per episode, as in the forward kernel
+// MERGE: a chunk that holds resets is done in ONE unit instead of one per episode, as in the forward kernel, in a copy of the unit beside the loop
+// over chunks without resets
 // (chunk_fwd_kernel): masks keep the episodes apart where they could meet -- Aqk, dAqk and dA (pairs of one
 // episode only), the three terms with the state entering the chunk (rows of the first episode), the two
 // terms with the gradient of the state leaving it (rows of the last episode) and the update of that
@@ -815,7 +816,6 @@ delta_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
     float *sKinv = reinterpret_cast<float *>(smem + L::oKinv);  // prologue: 1 / |k_row|
     float *sKd = sKinv + C;                                      // prologue: [NSLOT][C] partials of k_n . dk_n
     float *sFlag = reinterpret_cast<float *>(smem + L::oFlag);
-    static_assert(!MERGE || !NARROW, "merged episodes: full-width heads");
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -942,13 +942,20 @@ delta_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
         pend_db_on = false;
     };
 
-    for (int c = NC - 1; c >= 0; --c, dboff -= (int64_t)C * H) {
+    int c = NC - 1, unit = -1, whole = 0;   // unit: of chunk c, the next to be done (-1: none yet); whole: it is the only one
+    // MERGE: FREE the chunks up to the next that holds resets, UNIT one unit of that (chunk_common.h); EVERY chunk with its units per episode otherwise
+    enum Walk { EVERY, FREE, UNIT };
+    auto walk = [&](auto part, const int tid) __attribute__((always_inline)) {
+    constexpr Walk WALK = (Walk)decltype(part)::value;
+    constexpr bool RESETS = WALK == UNIT, MERGED = MERGE && RESETS;
+    const int lane = tid & 63, li = lane & 15, lg = lane >> 4;
+    for (; c >= 0; --c, dboff -= (int64_t)C * H) {
         const int t0 = c * C;
         const unsigned long long dmask = __ballot(done_test(rdone, done_f32) && lane < C);
         const int nres = __popcll(dmask);
-        bool mg = false;  // this chunk's episodes in one unit
-        if constexpr (MERGE) {
-            if (nres != 0) {
+        if (WALK == FREE && __builtin_expect(nres != 0, 0)) break;
+        if constexpr (MERGED) {
+            if (unit < 0) {
                 bool ok = true;
                 auto small = [](float x, float lim) { return fabsf(x) <= lim; };  // false for NaN
 #pragma unroll
@@ -980,18 +987,19 @@ delta_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
                 float bad = 0.f;
 #pragma unroll
                 for (int j = 0; j < NW; ++j) bad += sFlag[j];
-                mg = bad == 0.f;
+                whole = __builtin_amdgcn_readfirstlane(bad == 0.f);
             }
         }
+        if (RESETS && unit < 0) unit = whole ? 0 : nres;
+        const bool mg = MERGED && anew(whole);  // this chunk's episodes in one unit
         const int r_first = mg ? (int)__builtin_ctzll(dmask) : C;        // rows below it: the episode that enters the chunk
         const int r_last = mg ? 63 - (int)__builtin_clzll(dmask) : 0;   // rows from it on: the episode that leaves it
         auto one_episode = [&](int lo, int hi) { return (dmask & ((2ull << hi) - (2ull << lo))) == 0ull; };  // no reset in rows lo + 1 .. hi
         // One unit of work: the rows of one episode of the chunk (`pass` counts the episodes), or -- merged
         // episodes, MG -- all rows of a chunk that holds resets at once (pass 0).  In the instance that can
         // merge, the masks are part of the straight-line code of every unit (all-pass values where there is
-        // nothing to mask): a branch per mask would cut the phases into pieces the scheduler cannot overlap
-        // (measured: 10 % on chunks without resets), two copies of the unit do not fit the registers.
-        const bool MG = MERGE && mg;
+        // nothing to mask, of a chunk that fails the screen): a branch per mask would cut the phases into pieces the scheduler cannot overlap.
+        const bool MG = MERGED && mg;
         // ff / fl: 1 for the rows (nt * 16 + li of the wave's [C][64]-shaped tiles) of the first / last episode, else
         // 0; cw: the packed words of the wave's [C][C] tile j keep the bits of the elements that pair two rows of
         // one episode; fw: the words of an operand fragment read along the chunk rows (element e of the fragment of k block kb is
@@ -1059,7 +1067,7 @@ delta_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
                 *reinterpret_cast<words_t *>(dst + n * LDC + m) = wv;
             }
         };
-        for (int pass = MG ? 0 : nres; pass >= 0; --pass) {
+        for (int pass = WALK == EVERY ? nres : WALK == UNIT ? unit : 0, last = WALK == EVERY ? 0 : pass; pass >= last; --pass) {
             auto live = [&](int r) { return nres == 0 || MG || episode_of(dmask, r) == pass; };
             // ---- stage ---------------------------------------------------------------
             {
@@ -1119,7 +1127,7 @@ delta_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
                 f32x4 acc[TMA::TPW];
                 zero_acc<TMA::TPW>(acc);
                 gemm<T, C, C, HD, ROWK, ROWK, NW>(acc, sQ, LDD, sK, LDD, w, lane);
-                if constexpr (MERGE)
+                if constexpr (MERGED)
                     store_cc(acc, sAqk, [](int m, int n) { return m >= n; }, 1.f);
                 else
                     store_acc_f<T, C, C, NW>(acc, sAqk, LDC, w, lane, [](int m, int n, float x) { return m >= n ? x : 0.f; });
@@ -1136,9 +1144,9 @@ delta_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
                     const float bb = sBeta[r];
                     float y[4];
                     // merged episodes: the first one alone sees the entering state (a factor 0 on finite values)
-                    const float sees_S = MERGE ? ff[j % TMR::NBW] : 1.f;
+                    const float sees_S = MERGED ? ff[j % TMR::NBW] : 1.f;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) y[e] = MERGE ? (float)x[e] - sees_S * acc[j][e] : (float)x[e] - acc[j][e];
+                    for (int e = 0; e < 4; ++e) y[e] = MERGED ? (float)x[e] - sees_S * acc[j][e] : (float)x[e] - acc[j][e];
                     const P4 v0 = TT<T>::pack(y[0], y[1], y[2], y[3]);
                     *reinterpret_cast<P4 *>(sV + r * LDD + d0) = v0;
                     // V~ from the rounded V0, so that dbeta = rowdot(Z, V0) matches what U' was built from
@@ -1159,7 +1167,7 @@ delta_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
             {
                 f32x4 acc[TMR::TPW];
                 zero_acc<TMR::TPW>(acc);
-                if constexpr (MERGE) {  // the term with dS first, so that it can be confined to the rows of the last episode
+                if constexpr (MERGED) {  // the term with dS first, so that it can be confined to the rows of the last episode
                     gemm<T, HD, C, HD, ROWK, ROWK, NW>(acc, sDS, LDD, sK, LDD, w, lane);
 #pragma unroll
                     for (int j = 0; j < TMR::TPW; ++j) acc[j] *= fl[j % TMR::NBW];
@@ -1189,7 +1197,7 @@ delta_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
                 f32x4 acc[TMA::TPW];
                 zero_acc<TMA::TPW>(acc);
                 gemm<T, C, C, HD, ROWK, ROWK, NW>(acc, sU, LDD, sDO, LDD, w, lane);  // D[m = j][n = i]
-                if constexpr (MERGE)
+                if constexpr (MERGED)
                     store_cc(acc, sDAqk, [](int m, int n) { return m <= n; }, 1.f);
                 else
                     store_acc_f<T, C, C, NW>(acc, sDAqk, LDC, w, lane, tril);
@@ -1212,7 +1220,7 @@ delta_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
                 f32x4 acc[TMR::TPW];
                 zero_acc<TMR::TPW>(acc);
                 gemm<T, HD, C, HD, KROW, ROWK, NW>(acc, sS, LDD, sDO, LDD, w, lane);
-                if constexpr (MERGE) {
+                if constexpr (MERGED) {
 #pragma unroll
                     for (int j = 0; j < TMR::TPW; ++j) acc[j] *= ff[j % TMR::NBW];
                 }
@@ -1227,7 +1235,7 @@ delta_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
                 zero_acc<TMR::TPW>(acc);
                 zero_acc<TMR::TPW>(dKacc);
                 gemm<T, HD, C, HD, KROW, ROWK, NW>(acc, sS, LDD, sZb, LDD, w, lane);
-                if constexpr (MERGE) {  // the term with dS first: rows of the last episode; the term with S: rows of the first
+                if constexpr (MERGED) {  // the term with dS first: rows of the last episode; the term with S: rows of the first
                     gemm<T, HD, C, HD, KROW, ROWK, NW>(dKacc, sDS, LDD, sU, LDD, w, lane);
 #pragma unroll
                     for (int j = 0; j < TMR::TPW; ++j) dKacc[j] *= fl[j % TMR::NBW];
@@ -1245,7 +1253,7 @@ delta_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
             {
                 f32x4 acc[TMS::TPW];
                 zero_acc<TMS::TPW>(acc);
-                if constexpr (MERGE) {
+                if constexpr (MERGED) {
                     // a merged chunk: what flows on to the chunk before is the first episode's own sum -- the
                     // incoming gradient is dropped and the operand fragments keep the first episode's rows
                     // (straight-line: all-pass values in every other chunk)
@@ -1272,7 +1280,7 @@ delta_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
                 f32x4 acc[TMA::TPW];
                 zero_acc<TMA::TPW>(acc);
                 gemm<T, C, C, HD, ROWK, ROWK, NW>(acc, sU, LDD, sZ, LDD, w, lane);
-                if constexpr (MERGE)
+                if constexpr (MERGED)
                     store_cc(acc, sDA, [](int m, int n) { return m < n; }, -1.f);
                 else
                     store_acc_f<T, C, C, NW>(acc, sDA, LDC, w, lane, [](int m, int n, float x) { return m < n ? -x : 0.f; });
@@ -1352,7 +1360,19 @@ delta_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
             }
             // no barrier: sDb, sKd are not written again before the next pass's last phase
         }
+        if (RESETS) {
+            if (unit-- == 0) --c, whole = 0, dboff -= (int64_t)C * H;
+            return;
+        }
     }
+    };
+    if constexpr (!MERGE) walk(std::integral_constant<int, EVERY>{}, tid);
+    else
+        for (;;) {
+            walk(std::integral_constant<int, FREE>{}, tid);
+            if (__builtin_expect(c < 0, 1)) break;
+            walk(std::integral_constant<int, UNIT>{}, here(tid));
+        }
     sync_lds();
     flush_pending();
 #ifdef MRX_PHASE_CLOCKS
@@ -1619,10 +1639,9 @@ int launch_delta_bwd(hipStream_t st, const void *q, const void *k, const void *v
 {
     if (const int rc = prepare_device(); rc != MRX_OK) return rc;
     auto go = [&](auto narrow) {
-        constexpr bool MG = MERGE && !decltype(narrow)::value;  // narrow heads keep the units per episode
-        using Reg = DeltaBwdReg<T, C, PRO, decltype(narrow)::value, MG>;
+        using Reg = DeltaBwdReg<T, C, PRO, decltype(narrow)::value, MERGE>;
         (void)&Reg::reg;  // the kernel is on the list mrx_init() walks
-        return launch_kernel(delta_bwd_kernel<T, C, Reg::NW, PRO, decltype(narrow)::value, MG>, dim3((unsigned)(B * H)),
+        return launch_kernel(delta_bwd_kernel<T, C, Reg::NW, PRO, decltype(narrow)::value, MERGE>, dim3((unsigned)(B * H)),
                              dim3(64 * Reg::NW), Reg::smem, st, (const T *)q, (const T *)k, (const T *)v, (const T *)beta,
                              done, done_dtype, (const T *)S_chk, (const T *)Tm_chk, (const T *)dout,
                              (const float *)dS_last, (T *)dq, (T *)dk_out, (T *)dv_out, (T *)dbeta, (float *)dS0, (int)T_,
@@ -1645,16 +1664,20 @@ int delta_bwd_entry(void *stream, const void *q, const void *k, const void *v, c
     if (reset_path != MRX_RESETS_AUTO && reset_path != MRX_RESETS_PASSES && reset_path != MRX_RESETS_MERGED)
         return MRX_ERR_INVALID_ARG;
     hipStream_t st = (hipStream_t)stream;
-#if MRX_HD == 64
-    // merged episodes: the build with 32-row chunks, whose bounds the screen was derived for
-    if (reset_path == MRX_RESETS_MERGED && DELTA_BF16_CHUNK == 32) {
+    int cus = 0;
+    if (const int rc2 = prepare_device(&cus); rc2 != MRX_OK) return rc2;
+    // Merged episodes: the build with 32-row chunks, whose bounds the screen was derived for.  Left to choose, everywhere but for bfloat16 on fewer
+    // sequences than compute units: with one workgroup on a unit its loop over chunks without resets is 3 % the slower (us, forward and backward,
+    // merged / a unit per episode: 16 x 512 x 4 x 64 without resets 87.1 / 84.7, at one per 200 steps 109 / 111; 64 x 1024 x 8 x 64 243 / 243, one per
+    // 500 261 / 268, per 100 296 / 320, per 33 355 / 444; float32 64 x 256 x 8 x 64 233 / 238 and, per 100, 288 / 348; 64 x 512 x 4 x 48 95 / 97 and 136 / 148).
+    const bool merged = reset_path == MRX_RESETS_MERGED || (reset_path == MRX_RESETS_AUTO && (dtype == MRX_F32 || B * H >= cus));
+    if (merged && DELTA_BF16_CHUNK == 32) {
         if (dtype == MRX_BF16)
             return launch_delta_bwd<__bf16, 32, PRO, true>(st, q, k, v, beta, done, done_dtype, S_chk, Tm_chk, dout,
                                                            dS_last, dq, dk_out, dv_out, dbeta, dS0, B, T, H, dk, dv);
         return launch_delta_bwd<float, 32, PRO, true>(st, q, k, v, beta, done, done_dtype, S_chk, Tm_chk, dout, dS_last, dq,
                                                       dk_out, dv_out, dbeta, dS0, B, T, H, dk, dv);
     }
-#endif
     if (dtype == MRX_BF16)
         return launch_delta_bwd<__bf16, DELTA_BF16_CHUNK, PRO>(st, q, k, v, beta, done, done_dtype, S_chk, Tm_chk, dout,
                                                                dS_last, dq, dk_out, dv_out, dbeta, dS0, B, T, H, dk, dv);

@@ -165,3 +165,23 @@ def test_merged_at_the_torso_shape_through_the_functional_layer():
         assert relerr(a, b_.detach().float().cpu().numpy()) <= 4e-3
     with pytest.raises(KeyError):
         F.deltanet(q, k, v, b, done, S0, resets="sometimes")
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("B, d", [(64, 64), (64, 48), (64, 32), (2, 64), (2, 48)])
+def test_the_backward_left_to_choose(dtype, B, d):
+    """Few and many sequences, head dims of each build: what the call chooses against a unit per episode (the order of two sums)."""
+    from memorax_amd import kernels as K
+    T, H = 70, 4
+    rng = np.random.default_rng(B + d)
+    done = rng.random((B, T)) < 0.06
+    done[0, [0, 31, 32, 69]] = True
+    td = torch.bfloat16 if dtype == "bf16" else torch.float32
+    x = attn_inputs(B, T, H, d=d, seed=d, delta=True)
+    q, k, v, beta = (dev(x[n], td) for n in ("q", "k", "v", "beta"))
+    do = dev(rng.standard_normal((B, T, H, d)).astype(np.float32), td)
+    print(f"case auto resets dtype={dtype} B={B} d={d}", flush=True)
+    o, Sl, chk = K.delta_rule_fwd(q, k, v, beta, dev(done), dev(x["S0"]), factor_path="parallel")
+    a, b = (K.delta_rule_bwd(q, k, v, beta, dev(done), chk, do, None, reset_path=r, want_dS0=True) for r in ("auto", "passes"))
+    for n, s, t in zip(("dq", "dk", "dv", "dbeta", "dS0"), a, b):
+        assert relerr(s, t.float().cpu().numpy()) <= (4e-3 if dtype == "bf16" else 2e-6), (n, relerr(s, t.float().cpu().numpy()))
