@@ -366,7 +366,8 @@ la_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restr
                 for (int p = 0; p < IO::PASSES; ++p)
                     ok = ok && rden[p] >= LA_MERGE_DEN && rden[p] <= LA_MERGE_DEN_MAX && fabsf(rdss[p]) <= LA_MERGE_MAX;
             }
-            if (lane == 0) sMixed[w] = __ballot(!ok) != 0ull;
+            const bool fails = __ballot(!ok) != 0ull;  // of all lanes: taken before the branch
+            if (lane == 0) sMixed[w] = fails;
             sync_lds();
             whole = __builtin_amdgcn_readfirstlane(sMixed[0] | sMixed[1] | sMixed[2] | sMixed[3]) == 0;
             unit = whole ? 0 : nres;
@@ -982,7 +983,8 @@ delta_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
                 for (int j = 0; j < TMS::TPW; ++j)
 #pragma unroll
                     for (int e = 0; e < 4; ++e) ok = ok && small(dSacc[j][e], MERGE_STATE_MAX);
-                if (lane == 0) sFlag[w] = __ballot(!ok) != 0ull ? 1.f : 0.f;
+                const bool fails = __ballot(!ok) != 0ull;  // of all lanes: taken before the branch
+                if (lane == 0) sFlag[w] = fails ? 1.f : 0.f;
                 sync_lds();
                 float bad = 0.f;
 #pragma unroll

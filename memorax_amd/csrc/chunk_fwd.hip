@@ -302,7 +302,8 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
 #pragma unroll
                     for (int e = 0; e < 4; ++e) ok = ok && small(Sacc[j][e], MERGE_STATE_MAX);
                 // sBeta is free in this variant (the factors arrive ready): one flag per wave
-                if (lane == 0) sBeta[w] = __ballot(!ok) != 0ull ? 1.f : 0.f;
+                const bool fails = __ballot(!ok) != 0ull;  // of all lanes: taken before the branch
+                if (lane == 0) sBeta[w] = fails ? 1.f : 0.f;
                 sync_lds();
                 mg = sBeta[0] + sBeta[1] + sBeta[2] + sBeta[3] == 0.f;
             }
@@ -310,7 +311,8 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
         if constexpr (ONE) {
             if (unit < 0) {
                 const bool ok = IO::within(rq, LA_MERGE_MAX) && IO::within(rk, LA_MERGE_MAX) && IO::within(rv, LA_MERGE_MAX);
-                if (lane == 0) sMixed[w] = __ballot(!ok) != 0ull;
+                const bool fails = __ballot(!ok) != 0ull;  // of all lanes: taken before the branch
+                if (lane == 0) sMixed[w] = fails;
                 sync_lds();
                 whole = __builtin_amdgcn_readfirstlane(sMixed[0] | sMixed[1] | sMixed[2] | sMixed[3]) == 0;
                 unit = 0;

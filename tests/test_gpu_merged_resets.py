@@ -185,3 +185,24 @@ def test_the_backward_left_to_choose(dtype, B, d):
     a, b = (K.delta_rule_bwd(q, k, v, beta, dev(done), chk, do, None, reset_path=r, want_dS0=True) for r in ("auto", "passes"))
     for n, s, t in zip(("dq", "dk", "dv", "dbeta", "dS0"), a, b):
         assert relerr(s, t.float().cpu().numpy()) <= (4e-3 if dtype == "bf16" else 2e-6), (n, relerr(s, t.float().cpu().numpy()))
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("name", ["q", "k", "v", "beta", "do"])
+def test_one_element_beyond_the_screen(dtype, name):
+    """The screen sees what every lane of every wave holds: a single NaN leaves the other episodes of its chunk as the unit per episode does."""
+    from memorax_amd import kernels as K
+    B, T, H = 1, 96, 1
+    done = np.zeros((B, T), bool)
+    done[0, [40, 50]] = True
+    keep = np.r_[0:40, 50:96]
+    for at in ((40, 63), (43, 0), (44, 33), (49, 20)):
+        x = _case(B, T, H, 15, dtype, done)
+        x[name][(0, at[0], 0) if name == "beta" else (0, at[0], 0, at[1])] = np.nan
+        print(f"case merged element dtype={dtype} of={name} at={at}", flush=True)
+        a, b = (_run(K, x, dtype, r, dSl=False) for r in ("merged", "passes"))
+        for n in ("o", "dq", "dk", "dv", "dbeta"):
+            s, t = (r[n][:, keep].float().cpu().numpy() for r in (a, b))
+            assert np.isfinite(t).all() and relerr(s, t) <= (4e-3 if dtype == "bf16" else 2e-6), n
+        for n in ("S_last", "S_chk", "dS0"):
+            assert relerr(a[n], b[n].float().cpu().numpy()) <= (4e-3 if dtype == "bf16" else 2e-6), n

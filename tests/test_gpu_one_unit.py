@@ -111,3 +111,26 @@ def test_an_episode_beyond_the_screen_stays_by_itself(form, dtype, what):
     for n in a:
         u, w = (t[:, keep] if t.dim() >= 3 and t.shape[1] == T else t for t in (a[n], b[n]))
         assert torch.equal(u, w), n
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("name", ["q", "k", "v", "do"])
+def test_one_element_beyond_the_screen(form, dtype, name):
+    """The screen sees what every lane of every wave holds, not the first lane's share of the chunk."""
+    C = 64 if dtype == "bf16" else 32
+    T, lo, hi = 2 * C, C + 10, C + 20
+    done = np.zeros((1, T), bool)
+    done[0, [lo, hi]] = True
+    x = _case(1, T, 2, 64, dtype, 6)
+    good = _run(form, x, done, dtype)
+    keep = np.ones(T, bool)
+    keep[lo:hi] = False
+    for row, col in ((lo, 63), (lo + 3, 0), (lo + 4, 33), (hi - 1, 20)):
+        bad = dict(x, **{name: x[name].copy()})
+        bad[name][0, row, 1, col] = np.nan
+        print(f"case one_unit element form={form} dtype={dtype} of={name} at={row},{col}", flush=True)
+        got = _run(form, bad, done, dtype)
+        for n in good:
+            u, w = (t[:, keep] if t.dim() >= 3 and t.shape[1] == T else t for t in (good[n], got[n]))
+            assert torch.equal(u, w), n
