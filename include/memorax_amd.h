@@ -74,11 +74,13 @@ typedef enum {
  *   every such chunk first (|q|, |k|, |v|, |beta|, |dout| and the factor's entries <= 2^6, the state's and its
  *   gradient's <= 2^20: bounds under which no intermediate can leave the float32 range) and fall back to
  *   the units per episode for a chunk that fails, so the results are those of MRX_RESETS_PASSES for any data.
- *   The forward call merges where it takes the chunk-parallel factor kernel (mrx_factor_path) at head dim 64 and full width: for
- *   callers whose episodes end every hundred steps or so, a chunk without resets is 5 % behind there.  The backward call merges always
- *   (32-row chunks), and chunks without resets pay nothing.  The two calls of a pair need not agree.
- * MRX_RESETS_AUTO: the forward call as MRX_RESETS_PASSES; the backward call as MRX_RESETS_MERGED but for bfloat16 on fewer sequences than
- *   the device has compute units. */
+ *   The forward call merges where it takes the chunk-parallel factor kernel (mrx_factor_path), the backward call always (32-row
+ *   chunks).  For callers whose episodes end every hundred steps or so: at head dim 64 and full width the masks are part of the code for
+ *   every chunk, which is 2 to 7 % faster than MRX_RESETS_AUTO from there on and 2 to 14 % slower where resets are rare.
+ *   The two calls of a pair need not agree.
+ * MRX_RESETS_AUTO: one unit per chunk behind the same screen, in a loop of its own beside that over the chunks without resets, which pay
+ *   nothing: the forward call where it takes the chunk-parallel factor kernel, the backward call but for bfloat16 on fewer sequences than
+ *   the device has compute units.  The rest as MRX_RESETS_PASSES. */
 typedef enum {
     MRX_RESETS_AUTO = 0,
     MRX_RESETS_PASSES = 1,

@@ -786,7 +786,7 @@ static __device__ unsigned long long g_phase_clocks[4];
 // terms with the gradient of the state leaving it (rows of the last episode) and the update of that
 // gradient (rows of the first episode) -- after a screen of the chunk's inputs that rules out any
 // non-finite intermediate (chunk_common.h); a chunk that fails the screen takes the units per episode.
-template <typename T, int C, int NW, bool PRO, bool NARROW = false, bool MERGE = false>
+template <typename T, int C, int NW, bool PRO, bool NARROW = false, int MERGE = MERGE_NONE>
 __global__ void __launch_bounds__(64 * NW, sizeof(T) == 2 ? 2 : 1)
 delta_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restrict__ v,
                  const T *__restrict__ beta, const void *__restrict__ done, int done_f32,
@@ -944,11 +944,11 @@ delta_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
     };
 
     int c = NC - 1, unit = -1, whole = 0;   // unit: of chunk c, the next to be done (-1: none yet); whole: it is the only one
-    // MERGE: FREE the chunks up to the next that holds resets, UNIT one unit of that (chunk_common.h); EVERY chunk with its units per episode otherwise
+    // FREE: the chunks up to the next that holds resets; UNIT: one unit of that (chunk_common.h); EVERY: all chunks with all their units
     enum Walk { EVERY, FREE, UNIT };
     auto walk = [&](auto part, const int tid) __attribute__((always_inline)) {
     constexpr Walk WALK = (Walk)decltype(part)::value;
-    constexpr bool RESETS = WALK == UNIT, MERGED = MERGE && RESETS;
+    constexpr bool RESETS = WALK == UNIT, MERGED = RESETS || MERGE == MERGE_EVERY;
     const int lane = tid & 63, li = lane & 15, lg = lane >> 4;
     for (; c >= 0; --c, dboff -= (int64_t)C * H) {
         const int t0 = c * C;
@@ -956,7 +956,7 @@ delta_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
         const int nres = __popcll(dmask);
         if (WALK == FREE && __builtin_expect(nres != 0, 0)) break;
         if constexpr (MERGED) {
-            if (unit < 0) {
+            if (RESETS ? unit < 0 : nres != 0) {
                 bool ok = true;
                 auto small = [](float x, float lim) { return fabsf(x) <= lim; };  // false for NaN
 #pragma unroll
@@ -990,10 +990,12 @@ delta_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
 #pragma unroll
                 for (int j = 0; j < NW; ++j) bad += sFlag[j];
                 whole = __builtin_amdgcn_readfirstlane(bad == 0.f);
+            } else if (!RESETS) {
+                whole = 0;
             }
         }
         if (RESETS && unit < 0) unit = whole ? 0 : nres;
-        const bool mg = MERGED && anew(whole);  // this chunk's episodes in one unit
+        const bool mg = MERGED && (RESETS ? anew(whole) : whole != 0);  // this chunk's episodes in one unit
         const int r_first = mg ? (int)__builtin_ctzll(dmask) : C;        // rows below it: the episode that enters the chunk
         const int r_last = mg ? 63 - (int)__builtin_clzll(dmask) : 0;   // rows from it on: the episode that leaves it
         auto one_episode = [&](int lo, int hi) { return (dmask & ((2ull << hi) - (2ull << lo))) == 0ull; };  // no reset in rows lo + 1 .. hi
@@ -1069,7 +1071,7 @@ delta_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
                 *reinterpret_cast<words_t *>(dst + n * LDC + m) = wv;
             }
         };
-        for (int pass = WALK == EVERY ? nres : WALK == UNIT ? unit : 0, last = WALK == EVERY ? 0 : pass; pass >= last; --pass) {
+        for (int pass = WALK == EVERY ? (mg ? 0 : nres) : WALK == UNIT ? unit : 0, last = WALK == EVERY ? 0 : pass; pass >= last; --pass) {
             auto live = [&](int r) { return nres == 0 || MG || episode_of(dmask, r) == pass; };
             // ---- stage ---------------------------------------------------------------
             {
@@ -1368,7 +1370,7 @@ delta_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
         }
     }
     };
-    if constexpr (!MERGE) walk(std::integral_constant<int, EVERY>{}, tid);
+    if constexpr (MERGE != MERGE_BESIDE) walk(std::integral_constant<int, EVERY>{}, tid);
     else
         for (;;) {
             walk(std::integral_constant<int, FREE>{}, tid);
@@ -1627,13 +1629,13 @@ MRX_EXPORT int MRX_API(mrx_gated_linear_attn_bwd)(void *stream, const void *q, c
 namespace {
 inline namespace MRX_HD_NS {
 
-template <typename T, int C, bool PRO, bool NARROW, bool MERGE> struct DeltaBwdReg {
+template <typename T, int C, bool PRO, bool NARROW, int MERGE> struct DeltaBwdReg {
     static constexpr int NW = 4;
     static constexpr int smem = DeltaBwdSmem<T, C, NW>::total;
     static inline KernelRegistrar reg{reinterpret_cast<const void *>(delta_bwd_kernel<T, C, NW, PRO, NARROW, MERGE>), smem};
 };
 
-template <typename T, int C, bool PRO, bool MERGE = false>
+template <typename T, int C, bool PRO, int MERGE = MERGE_NONE>
 int launch_delta_bwd(hipStream_t st, const void *q, const void *k, const void *v, const void *beta,
                      const void *done, int done_dtype, const void *S_chk, const void *Tm_chk, const void *dout,
                      const void *dS_last, void *dq, void *dk_out, void *dv_out, void *dbeta, void *dS0, int64_t B,
@@ -1641,9 +1643,10 @@ int launch_delta_bwd(hipStream_t st, const void *q, const void *k, const void *v
 {
     if (const int rc = prepare_device(); rc != MRX_OK) return rc;
     auto go = [&](auto narrow) {
-        using Reg = DeltaBwdReg<T, C, PRO, decltype(narrow)::value, MERGE>;
+        constexpr int MG = decltype(narrow)::value && MERGE == MERGE_EVERY ? (int)MERGE_BESIDE : MERGE;
+        using Reg = DeltaBwdReg<T, C, PRO, decltype(narrow)::value, MG>;
         (void)&Reg::reg;  // the kernel is on the list mrx_init() walks
-        return launch_kernel(delta_bwd_kernel<T, C, Reg::NW, PRO, decltype(narrow)::value, MERGE>, dim3((unsigned)(B * H)),
+        return launch_kernel(delta_bwd_kernel<T, C, Reg::NW, PRO, decltype(narrow)::value, MG>, dim3((unsigned)(B * H)),
                              dim3(64 * Reg::NW), Reg::smem, st, (const T *)q, (const T *)k, (const T *)v, (const T *)beta,
                              done, done_dtype, (const T *)S_chk, (const T *)Tm_chk, (const T *)dout,
                              (const float *)dS_last, (T *)dq, (T *)dk_out, (T *)dv_out, (T *)dbeta, (float *)dS0, (int)T_,
@@ -1674,11 +1677,14 @@ int delta_bwd_entry(void *stream, const void *q, const void *k, const void *v, c
     // 500 261 / 268, per 100 296 / 320, per 33 355 / 444; float32 64 x 256 x 8 x 64 233 / 238 and, per 100, 288 / 348; 64 x 512 x 4 x 48 95 / 97 and 136 / 148).
     const bool merged = reset_path == MRX_RESETS_MERGED || (reset_path == MRX_RESETS_AUTO && (dtype == MRX_F32 || B * H >= cus));
     if (merged && DELTA_BF16_CHUNK == 32) {
-        if (dtype == MRX_BF16)
-            return launch_delta_bwd<__bf16, 32, PRO, true>(st, q, k, v, beta, done, done_dtype, S_chk, Tm_chk, dout,
-                                                           dS_last, dq, dk_out, dv_out, dbeta, dS0, B, T, H, dk, dv);
-        return launch_delta_bwd<float, 32, PRO, true>(st, q, k, v, beta, done, done_dtype, S_chk, Tm_chk, dout, dS_last, dq,
-                                                      dk_out, dv_out, dbeta, dS0, B, T, H, dk, dv);
+        auto go = [&](auto t, auto how) {
+            return launch_delta_bwd<decltype(t), 32, PRO, decltype(how)::value>(st, q, k, v, beta, done, done_dtype, S_chk, Tm_chk, dout, dS_last, dq,
+                                                                               dk_out, dv_out, dbeta, dS0, B, T, H, dk, dv);
+        };
+        using Beside = std::integral_constant<int, MERGE_BESIDE>;
+        using Asked = std::integral_constant<int, MRX_HD == 64 ? (int)MERGE_EVERY : (int)MERGE_BESIDE>;
+        if (reset_path == MRX_RESETS_MERGED) return dtype == MRX_BF16 ? go(__bf16(), Asked{}) : go(float(), Asked{});
+        return dtype == MRX_BF16 ? go(__bf16(), Beside{}) : go(float(), Beside{});
     }
     if (dtype == MRX_BF16)
         return launch_delta_bwd<__bf16, DELTA_BF16_CHUNK, PRO>(st, q, k, v, beta, done, done_dtype, S_chk, Tm_chk, dout,

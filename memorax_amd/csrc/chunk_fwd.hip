@@ -92,8 +92,9 @@ struct NormArgs {
 // magnitude and the state at most MERGE_STATE_MAX (bounds under which no intermediate of the chunk can
 // leave the float32 range, so a non-finite value cannot arise either), else the chunk takes the units
 // per episode, whose zeros are put in by select.  Results equal those of the units per episode.
+// MERGE_BESIDE walks chunks without resets and chunks with them in two loops, as linear attention does (SPLIT below).
 template <typename T, int C, bool DELTA, bool FMAP, bool GATED, bool NORM, bool PRO = false, bool TMIN = false,
-          bool PAR = false, bool NARROW = false, bool MERGE = false>
+          bool PAR = false, bool NARROW = false, int MERGE = MERGE_NONE>
 __global__ void __launch_bounds__(NTHR, 2)  // 2 waves per SIMD: two workgroups share a CU
 chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restrict__ v,
                  const T *__restrict__ beta, const float *__restrict__ glog,
@@ -106,7 +107,8 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
     static_assert(!PRO || DELTA, "the prologue belongs to the delta rule");
     static_assert(!TMIN || (DELTA && C == 32), "precomputed factors belong to the delta rule's 32-row chunks");
     static_assert(!PAR || !DELTA, "one workgroup per chunk: linear attention only");
-    static_assert(!MERGE || (TMIN && !NARROW), "merged episodes: the delta rule on precomputed factors, full-width heads");
+    static_assert(!MERGE || TMIN, "merged episodes of the delta rule: on precomputed factors");
+    constexpr bool SPLIT = !DELTA || MERGE == MERGE_BESIDE;  // chunks with resets apart from those without
     using IOT = TileIO<T, C, NTHR, C>;  // the [C][C] triangular factor
     using L = FwdSmem<T, C, DELTA, GATED, NORM>;
     using Frag = typename TT<T>::frag;
@@ -264,23 +266,23 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
     };
     int64_t schk_off = (int64_t)bh * NC * dvw * dkw;                                 // S_chk[c]
     int64_t tmchk_off = (int64_t)bh * NC * C * C + (int64_t)tid * 4;                                  // row-major C x C
-    // ONE (linear attention): a unit of a chunk that holds resets; otherwise the chunks up to the next that does (chunk_common.h)
+    // SPLIT: one UNIT of a chunk that holds resets, or the chunks up to the next that does (chunk_common.h).  ONE: with the masks for all episodes at once
     int c = c_first;
-    [[maybe_unused]] int unit = -1, whole = 0;   // linear attention: of chunk c, the next to be done (-1: none yet); it is the only one
+    [[maybe_unused]] int unit = -1, whole = 0;   // of chunk c, the next to be done (-1: none yet); it is the only one
     auto next_chunk = [&]() { ++c, schk_off += dvw * dkw, tmchk_off += C * C, den_off += C; };
-    auto walk = [&](auto one, const int tid) __attribute__((always_inline)) {
-    constexpr bool ONE = decltype(one)::value;
+    auto walk = [&](auto resets, const int tid) __attribute__((always_inline)) {
+    constexpr bool UNIT = decltype(resets)::value, ONE = UNIT || MERGE == MERGE_EVERY;
     const int lane = tid & 63, li = lane & 15, lg = lane >> 4;
     for (; c < c_end; next_chunk()) {
         const int t0 = c * C;
         const unsigned long long dmask = __ballot(done_test(rdone, done_f32) && lane < C);
         const int nres = __popcll(dmask);
-        if constexpr (!ONE && !DELTA) {
+        if constexpr (!UNIT && SPLIT) {
             if (__builtin_expect(nres != 0, 0)) break;
         }
         bool mg = false;  // this chunk's episodes in one unit
-        if constexpr (MERGE) {
-            if (nres != 0) {
+        if constexpr (ONE && DELTA) {
+            if (UNIT ? unit < 0 : nres != 0) {
                 bool ok = true;
                 auto small = [](float x, float lim) { return fabsf(x) <= lim; };  // false for NaN
 #pragma unroll
@@ -305,10 +307,14 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
                 const bool fails = __ballot(!ok) != 0ull;  // of all lanes: taken before the branch
                 if (lane == 0) sBeta[w] = fails ? 1.f : 0.f;
                 sync_lds();
-                mg = sBeta[0] + sBeta[1] + sBeta[2] + sBeta[3] == 0.f;
+                whole = __builtin_amdgcn_readfirstlane(sBeta[0] + sBeta[1] + sBeta[2] + sBeta[3] == 0.f);
+                unit = 0;
+            } else if (!UNIT) {
+                whole = 0;
             }
+            mg = UNIT ? anew(whole) : whole != 0;
         }
-        if constexpr (ONE) {
+        if constexpr (ONE && !DELTA) {
             if (unit < 0) {
                 const bool ok = IO::within(rq, LA_MERGE_MAX) && IO::within(rk, LA_MERGE_MAX) && IO::within(rv, LA_MERGE_MAX);
                 const bool fails = __ballot(!ok) != 0ull;  // of all lanes: taken before the branch
@@ -322,7 +328,7 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
         const int npass = mg ? 0 : nres;
         const int r_first = mg ? (int)__builtin_ctzll(dmask) : C;        // rows below it: the episode that enters the chunk
         const int r_last = mg ? 63 - (int)__builtin_clzll(dmask) : 0;   // rows from it on: the episode that leaves it
-        for (int pass = ONE ? unit : 0; pass <= (ONE ? unit : npass); ++pass) {   // (ONE: a unit a call)
+        for (int pass = UNIT ? unit : 0; pass <= (UNIT ? unit : npass); ++pass) {
             auto live = [&](int r) { return nres == 0 || mg || episode_of(dmask, r) == pass; };
             // gated: G_i = sum of the log-decays of this pass's episode up to row i (the decay of an
             // episode's first step multiplies a zero state and is left out); every wave scans its copy
@@ -504,11 +510,6 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
                         for (int e = 0; e < 4; ++e) x[e] = of_pair(m, e, n, start) ? acc[j][e] : 0.f;
                         *reinterpret_cast<P4 *>(sAqk + n * LDC + m) = TT<T>::pack(x[0], x[1], x[2], x[3]);
                     }
-                } else if (MERGE && mg) {
-                    // pairs (i = n, j = m <= n) of one episode only: no reset in rows m + 1 .. n
-                    store_acc_f<T, C, C, NW>(acc, sAqk, LDC, w, lane, [&](int m, int n, float x) {
-                        return m <= n && (dmask & ((2ull << n) - (2ull << m))) == 0ull ? x : 0.f;
-                    });
                 } else {
                     store_acc_f<T, C, C, NW>(acc, sAqk, LDC, w, lane,
                                              [](int m, int n, float x) { return m <= n ? x : 0.f; });
@@ -544,7 +545,7 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
 #pragma unroll
                     for (int j = 0; j < TMO::TPW; ++j) {
                         // merged episodes: only the rows of the episode that entered the chunk see its state
-                        if (!(MERGE && mg) || TMO::nt(w, j) * 16 + li < r_first) Uacc[j] -= acc[j];
+                        if (!ONE || TMO::nt(w, j) * 16 + li < r_first) Uacc[j] -= acc[j];
                     }
                     store_acc<T, HD, C, NW>(Uacc, sU, LDD, w, lane);
                 }
@@ -578,11 +579,6 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
                 }
             };
             gemm<T, HD, C, HD, ROWK, ROWK, NW>(Oacc, sS, LDD, sQ, LDD, w, lane, NoHook(), den_q);
-            if (MERGE && mg) {
-#pragma unroll
-                for (int j = 0; j < TMO::TPW; ++j)
-                    if (TMO::nt(w, j) * 16 + li >= r_first) Oacc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-            }
             if (GATED) {  // the incoming state reaches row i decayed by exp(G_i)
 #pragma unroll
                 for (int j = 0; j < TMO::TPW; ++j) Oacc[j] *= __expf(sG[TMO::nt(w, j) * 16 + li]);
@@ -646,7 +642,6 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
             pend_t0 = t0;
             // ---- S^T[dk][dv] += sum_c K[c][dk] U'[c][dv]  (only the episode that leaves the chunk)
             if (pass == npass && !PAR) {
-                if (MERGE && mg) zero_acc<TMS::TPW>(Sacc);  // a chunk with resets: the state that leaves is the last episode's own
                 if (GATED) {  // S <- exp(G_last) S + sum_c exp(G_last - G_c) K[c] U'[c]
                     const float cl = ONE && mg ? 1.f : __expf(Glast);  // (one unit: what it would decay is zero)
 #pragma unroll
@@ -671,12 +666,6 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
                         for (int e = 0; e < TT<T>::KP; ++e) xk[e] = (T)((float)xk[e] * eb[e]);
                         if (ONE) keep_rows<T, false>(xk, kb, lg, r_last);
                     }
-                    if (MERGE && mg) {  // rows of the last episode only (element e of the fragment is chunk row k0 + e)
-                        const int k0 = kb * TT<T>::KB + TT<T>::KP * lg;
-#pragma unroll
-                        for (int e = 0; e < TT<T>::KP; ++e)
-                            if (k0 + e < r_last) xk[e] = (T)0.f;
-                    }
                 };
                 gemm<T, HD, HD, C, KROW, KROW, NW>(Sacc, sK, LDD, sU, LDD, w, lane, z_k);
                 if (NORM && VN) {
@@ -697,7 +686,7 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
                 na.ss[(int64_t)bh * Tlen + t0 + tid] = x;  // the slots are next written after the next unit's barriers
             }
         }
-        if (ONE) {
+        if (UNIT) {
             if (unit++ == npass) unit = -1, next_chunk();
             return;
         }
@@ -705,8 +694,8 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
     };
     for (;;) {
         walk(std::false_type{}, tid);
-        if (DELTA || __builtin_expect(c >= c_end, 1)) break;
-        if constexpr (!DELTA) walk(std::true_type{}, here(tid));
+        if (!SPLIT || __builtin_expect(c >= c_end, 1)) break;
+        if constexpr (SPLIT) walk(std::true_type{}, here(tid));
     }
     flush_o();  // the last unit ended with a barrier
 
@@ -729,7 +718,7 @@ chunk_fwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__re
     }
 }
 
-template <typename T, int C, bool DELTA, bool FMAP, bool GATED, bool NORM, bool PRO, bool TMIN, bool PAR, bool NARROW, bool MERGE> struct FwdReg {
+template <typename T, int C, bool DELTA, bool FMAP, bool GATED, bool NORM, bool PRO, bool TMIN, bool PAR, bool NARROW, int MERGE> struct FwdReg {
     static constexpr int smem = FwdSmem<T, C, DELTA, GATED, NORM>::total;
     static inline KernelRegistrar reg{
         reinterpret_cast<const void *>(chunk_fwd_kernel<T, C, DELTA, FMAP, GATED, NORM, PRO, TMIN, PAR, NARROW, MERGE>), smem};
@@ -738,7 +727,7 @@ template <typename T, int C, bool DELTA, bool FMAP, bool GATED, bool NORM, bool 
 // dka, dva: widths of the q/k and v/o rows in memory; less than the build's head dim (narrow heads)
 // selects the kernel instance that pads on the fly.
 template <typename T, int C, bool DELTA, bool FMAP, bool GATED = false, bool NORM = false, bool PRO = false,
-          bool TMIN = false, bool PAR = false, bool MERGE = false>
+          bool TMIN = false, bool PAR = false, int MERGE = MERGE_NONE>
 int launch(hipStream_t st, const void *q, const void *k, const void *v, const void *beta,
            const void *done, int done_f32, const void *S0, void *o, void *S_last, void *S_chk,
            void *Tm_chk, int64_t B, int64_t Tlen, int64_t H, const void *glog = nullptr, NormArgs na = NormArgs{},
@@ -749,7 +738,7 @@ int launch(hipStream_t st, const void *q, const void *k, const void *v, const vo
     if (PAR && NC > 65535) return MRX_ERR_INVALID_ARG;
     auto go = [&](auto narrow) {
         constexpr bool NARROW = decltype(narrow)::value;
-        constexpr bool MG = MERGE && !NARROW;  // narrow heads keep the units per episode
+        constexpr int MG = NARROW && MERGE == MERGE_EVERY ? (int)MERGE_BESIDE : MERGE;
         using Reg = FwdReg<T, C, DELTA, FMAP, GATED, NORM, PRO, TMIN, PAR, NARROW, MG>;
         (void)&Reg::reg;  // the kernel is on the list mrx_init() walks
         return launch_kernel(chunk_fwd_kernel<T, C, DELTA, FMAP, GATED, NORM, PRO, TMIN, PAR, NARROW, MG>,
@@ -811,19 +800,23 @@ int delta_fwd_dispatch(hipStream_t st, const void *q, const void *k, const void 
     // merged episodes run on precomputed factors (which arrive block diagonal by episode, and screened like any
     // other input): where the factor path is the chunk-parallel kernel; with the inverse inside the sequential
     // kernel the units per episode stay (on a full device, where that path is the rule, a chunk with resets
-    // costs the forward a few per cent, less than the factor kernel would)
-    const bool merged = MRX_HD == 64 && TM_KERNEL && reset_path == MRX_RESETS_MERGED && parallel;
-    (void)merged;  // the head-dim-32 build has no merged instances
+    // costs the forward a few per cent, less than the factor kernel would).  Left to choose the two loops beside each other: without resets they
+    // are no slower than the one that knows passes (us, forward and backward, a unit per episode / merged: bf16 64 x 1024 x 8 x 64 no resets
+    // 243 / 245, one per 500 steps 265 / 256, per 100 317 / 288, per 33 443 / 326; 16 x 512 x 4 x 64 85 / 83 and 130 / 129; float32 64 x 256 x 8 x 64
+    // 238 / 232 and, per 100, 349 / 274; 64 x 512 x 4 x 48 97 / 93 and 149 / 138; 64 x 512 x 8 x 32 81 / 79 and 114 / 105; the backward's share included)
+    const bool merged = parallel && reset_path != MRX_RESETS_PASSES;
     if (!TM_KERNEL && factor_path == MRX_FACTORS_PARALLEL) return MRX_ERR_UNSUPPORTED;
     if constexpr (TM_KERNEL) if (parallel) {
         const int rc = launch_delta_tm(st, k, beta, done, done_dtype, Tm_chk, B, T, H, dtype, PRO, dk);
         if (rc != MRX_OK) return rc;
 #define MRX_ARGS st, q, k, v, beta, done, done_dtype, S0, o, S_last, S_chk, Tm_chk, B, T, H, nullptr, NormArgs{}, dk, dv
-#if MRX_HD == 64
-        if (merged)
-            return dtype == MRX_BF16 ? launch<__bf16, 32, true, false, false, false, PRO, true, false, true>(MRX_ARGS)
-                                     : launch<float, 32, true, false, false, false, PRO, true, false, true>(MRX_ARGS);
-#endif
+        if (merged) {
+            auto go = [&](auto t, auto how) { return launch<decltype(t), 32, true, false, false, false, PRO, true, false, decltype(how)::value>(MRX_ARGS); };
+            using Beside = std::integral_constant<int, MERGE_BESIDE>;
+            using Asked = std::integral_constant<int, MRX_HD == 64 ? (int)MERGE_EVERY : (int)MERGE_BESIDE>;
+            if (reset_path == MRX_RESETS_MERGED) return dtype == MRX_BF16 ? go(__bf16(), Asked{}) : go(float(), Asked{});
+            return dtype == MRX_BF16 ? go(__bf16(), Beside{}) : go(float(), Beside{});
+        }
         if (dtype == MRX_BF16) return launch<__bf16, 32, true, false, false, false, PRO, true>(MRX_ARGS);
         return launch<float, 32, true, false, false, false, PRO, true>(MRX_ARGS);
 #undef MRX_ARGS

@@ -269,7 +269,7 @@ def delta_rule(q, k, v, beta, done, S0=None, resets=None):
     """DeltaNet recurrence S_t = r_t S_{t-1}(I - beta_t k_t k_t^T) + beta_t v_t k_t^T,
     o_t = S_t q_t, in chunked WY form.  Returns (o, S_last).
     resets: None / "passes" / "merged" -- how the kernels treat a chunk that holds resets
-    (mrx_reset_path; "merged" for callers whose episodes end every hundred steps or so)."""
+    (mrx_reset_path; None for any reset rate, "merged" a few per cent faster where episodes end every hundred steps or so)."""
     if _no_steps(q):
         return _attention_without_steps(q, v, S0)
     if _native_heads(q, v):

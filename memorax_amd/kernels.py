@@ -174,8 +174,8 @@ def delta_rule_fwd(q, k, v, beta, done, S0=None, save_chk=True, out=None, prolog
     anyway, which lets it compute them chunk-parallel.  None: when the library would use it (float32;
     bf16 with B*H at most two sequences per compute unit).
     factor_path: None / "auto" (by occupancy), "parallel" or "inline" (mrx_factor_path).
-    reset_path: None / "auto", "passes" (one unit of work per episode of a chunk) or "merged" (one per chunk
-    behind a screen of its inputs: mrx_reset_path); the backward call takes the same argument."""
+    reset_path: "passes" (one unit of work per episode of a chunk), "merged" (one per chunk behind a screen of its inputs, in code for
+    short episodes) or None / "auto" (the library's choice: mrx_reset_path); the backward call takes the same argument."""
     if out is not None:
         save_chk = out[2] is not None
     o, S_last, S_chk, Tm_chk = _lib.native().delta_rule_fwd(q, k, v, beta, done, S0, save_chk, out, prologue, tm_scratch,

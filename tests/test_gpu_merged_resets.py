@@ -167,6 +167,30 @@ def test_merged_at_the_torso_shape_through_the_functional_layer():
         F.deltanet(q, k, v, b, done, S0, resets="sometimes")
 
 
+@pytest.mark.parametrize("poison", [False, True])
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("T, d", [(70, 64), (70, 48), (33, 32), (64, 24), (1, 64)])
+def test_the_forward_left_to_choose(dtype, T, d, poison):
+    """The one unit adds exact zeros where the units per episode have none: outputs, states and residuals bit for bit; with a value above the
+    screen's bound, an infinity and a NaN in middle episodes the unit per episode is what runs."""
+    from memorax_amd import kernels as K
+    B, H = 5, 3
+    rng = np.random.default_rng(T + d)
+    done = rng.random((B, T)) < 0.06
+    done[0, [t for t in (0, 1, 31, 32, 63) if t < T]] = True
+    done[1] = True
+    done[2, 5:9] = True
+    td = torch.bfloat16 if dtype == "bf16" else torch.float32
+    x = attn_inputs(B, T, H, d=d, seed=d, delta=True)
+    if poison and T > 8:
+        x["v"][2, 6, 0, 3], x["q"][2, 7, 1, 0], x["v"][2, 5, 2, 1] = 100., np.inf, np.nan
+    q, k, v, beta = (dev(x[n], td) for n in ("q", "k", "v", "beta"))
+    print(f"case auto resets forward dtype={dtype} T={T} d={d} poison={poison}", flush=True)
+    a, b = (K.delta_rule_fwd(q, k, v, beta, dev(done), dev(x["S0"]), factor_path="parallel", reset_path=r) for r in ("auto", "passes"))
+    for s, t in zip((a[0], a[1], *a[2]), (b[0], b[1], *b[2])):
+        np.testing.assert_array_equal(s.float().cpu().numpy(), t.float().cpu().numpy())
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 @pytest.mark.parametrize("B, d", [(64, 64), (64, 48), (64, 32), (2, 64), (2, 48)])
 def test_the_backward_left_to_choose(dtype, B, d):
