@@ -30,3 +30,16 @@ def test_gradient_of_a_broadcast_coefficient(B, D, dtype):
         bound = bound + 2.0 ** -8 * want.abs()
     assert got.dtype == dtype and got.shape == a.shape
     assert ((got.to(wide) - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("rows", [511, 512, 513, 575, 1023, 1025, 4097])
+@pytest.mark.parametrize("columns", [1, 15, 16, 17, 256, 4096, 4097])
+def test_many_rows(rows, columns):
+    """Either side of the rule by which few columns take sixteen per workgroup: 64 threads a column, eight sums each."""
+    from memorax_amd import _lib
+    print(f"case column sum of many rows {rows} {columns}", flush=True)
+    x = torch.randn(rows, columns, device="cuda", generator=torch.Generator(device="cuda").manual_seed(rows + columns))
+    out = torch.full((columns + 1,), 7.0, device="cuda")
+    assert _lib.load().mrx_column_sum(torch.cuda.current_stream().cuda_stream, x.data_ptr(), out.data_ptr(), rows, columns) == 0
+    bound = 2.0 ** -23 * (rows // 64 + 2 + 6) * x.double().abs().sum(0)   # the longest chain of sums, of either kernel
+    assert ((out[:-1].double() - x.double().sum(0)).abs() <= bound).all() and out[-1] == 7.0
