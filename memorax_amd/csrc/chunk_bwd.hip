@@ -593,8 +593,14 @@ la_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restr
                 if (NORM && pass == 0) {  // den_i = q_i . (z_in + ...): dQ_i += dden_i z_in
 #pragma unroll
                     for (int j = 0; j < TMR::TPW; ++j) {
-                        const f32x4 zz = *reinterpret_cast<const f32x4 *>(sZf + TMR::mt(w, j) * 16 + 4 * lg);
-                        acc[j] += zz * (!ONE || TMR::nt(w, j) * 16 + li < r_first ? sDd[TMR::nt(w, j) * 16 + li] : 0.f);
+                        const int r = TMR::nt(w, j) * 16 + li;
+                        const f32x4 zz = *reinterpret_cast<const f32x4 *>(sZf + TMR::mt(w, j) * 16 + 4 * lg) * sDd[r];
+                        if constexpr (ONE) {  // the product goes, not a factor: z is the first episode's and may be anything
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) acc[j][e] += r < r_first ? zz[e] : 0.f;
+                        } else {
+                            acc[j] += zz;
+                        }
                     }
                 }
                 auto sc = [&](int r, int d0) {

@@ -134,3 +134,26 @@ def test_one_element_beyond_the_screen(form, dtype, name):
         for n in good:
             u, w = (t[:, keep] if t.dim() >= 3 and t.shape[1] == T else t for t in (good[n], got[n]))
             assert torch.equal(u, w), n
+
+
+@pytest.mark.parametrize("chunks", [3, 12])   # a workgroup per sequence, a workgroup per chunk
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("form", FORMS)
+def test_a_reset_on_a_chunk_s_first_row_drops_what_enters_it(form, dtype, chunks):
+    """The episode that ends with a chunk leaves a state, and a sum of keys, that is not finite: no row of the next chunk is of that episode, and its
+    inputs pass the screen."""
+    C = 64 if dtype == "bf16" else 32
+    T = chunks * C
+    done = np.zeros((1, T), bool)
+    done[0, [C, 2 * C + 7]] = True
+    x = _case(1, T, 2, 64, dtype, 7)
+    print(f"case one_unit first row form={form} dtype={dtype} chunks={chunks}", flush=True)
+    good = _run(form, x, done, dtype)
+    for what in (float("nan"), float("inf")):
+        bad = {n: a.copy() for n, a in x.items()}
+        bad["k"][0, C - 5, 0, 11] = what
+        got = _run(form, bad, done, dtype)
+        for n in good:
+            u, w = (t[:, C:] if t.dim() >= 3 and t.shape[1] == T else t for t in (good[n], got[n]))
+            if n not in ("dS0", "dz0"):   # of the episode that enters the sequence
+                assert torch.equal(u, w), n
