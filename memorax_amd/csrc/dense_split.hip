@@ -188,6 +188,7 @@ template <int NT, bool ACROSS> __global__ void __launch_bounds__(SP_THREADS, NT 
     const int first = (int)((int64_t)a.passes * group / a.groups), last = (int)((int64_t)a.passes * (group + 1) / a.groups);
     const int row = tid >> 5, k8 = tid & 31;
     if (tid == 0) infinite = 0;
+    sync_lds();   // before any wave sets it
 
     constexpr int UNITS = SP_ROWS * 32 / SP_THREADS, APART = SP_THREADS / 32;
     sf32x4 v[UNITS][2];

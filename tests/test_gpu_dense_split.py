@@ -103,6 +103,17 @@ def test_what_is_not_finite(bad):
     assert not torch.isfinite(dws[0][9]).any() and torch.isfinite(dws[1]).all() and torch.isfinite(dws[0][:9]).all()
 
 
+@pytest.mark.parametrize("at", [63, 37, 16])
+def test_an_infinity_in_every_tile_of_rows(at):
+    """Whichever wave of a workgroup meets it: each tile's row has infinite sums, none of them NaN."""
+    x, ws, bs, _ = _case(64 * 700, 64, [64, 64])
+    x[at::64, 3] = float("inf")
+    ws = [w.requires_grad_() for w in ws]
+    for y, w in zip(dense_group(x, [Weights(w, b) for w, b in zip(ws, bs)]), ws):
+        assert torch.equal(y[at::64], (w[:, 3].sign() * float("inf")).expand(700, -1))
+        assert int(torch.isfinite(y).sum()) == 63 * 700 * 64
+
+
 def test_residual_and_bfloat16_results():
     """The C entry's residual sum, and an input gradient that is asked for in bfloat16."""
     x, ws, _, dys = _case(1000, 128, [96])
