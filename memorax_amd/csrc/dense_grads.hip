@@ -293,7 +293,9 @@ template <int TN, int TK> __global__ void __launch_bounds__(DG_THREADS, 2) split
 #pragma unroll
             for (int p = 0; p < SplitTile<TN>::Rows::PASSES; ++p) part += __builtin_bit_cast(sf32x4, ty.rows.v[p]);
             const sf32x4 y = part - bias_low, s = bias_sum + y;
-            bias_low = (s - bias_sum) - y, bias_sum = s;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) bias_low[q] = fabsf(s[q]) <= 3.402823466e38f ? (s[q] - bias_sum[q]) - y[q] : 0.f;   // an infinite sum rounds nothing off
+            bias_sum = s;
         }
         sync_lds();   // the buffer two steps back has been read by every wave that reaches the barrier
         if (beyond[buf] == step) {

@@ -114,6 +114,21 @@ def test_an_infinity_in_every_tile_of_rows(at):
         assert int(torch.isfinite(y).sum()) == 63 * 700 * 64
 
 
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("row", [0, 70, 199])
+def test_bias_gradients_of_what_is_not_finite(bad, row):
+    """An infinity among the rows is the sum of its column, as in the array library's sums; opposite ones and NaN are NaN."""
+    x, ws, _, dys = _case(200, 128, [64, 72])
+    dys[0][row, 9], dys[1][row, 3], dys[1][5, 4], dys[1][190, 4] = bad, 1.0, bad, -bad
+    bs = [torch.zeros(w.shape[0], device="cuda", requires_grad=True) for w in ws]
+    torch.autograd.backward(dense_group(x, [Weights(w, b) for w, b in zip(ws, bs)]), dys)
+    for b, dy in zip(bs, dys):
+        want = dy.double().sum(0)
+        fine = torch.isfinite(want)
+        assert torch.equal(torch.isnan(b.grad), torch.isnan(want)) and torch.equal(b.grad.double()[torch.isinf(want)], want[torch.isinf(want)])
+        assert (b.grad.double() - want)[fine].abs().max() <= 8 * EPS * 200 ** 0.5
+
+
 def test_residual_and_bfloat16_results():
     """The C entry's residual sum, and an input gradient that is asked for in bfloat16."""
     x, ws, _, dys = _case(1000, 128, [96])
