@@ -1643,6 +1643,9 @@ std::optional<ScalarType> autocast_dtype(const Tensor &x)
 // Sums of fewer than SPLIT_TERMS products stay float32's, whose error is that of their few additions: 64 terms 1.0e-7 here, 1.4e-7 there, 8 terms
 // 1.0e-7 and 0.3e-7.
 constexpr int64_t SPLIT_TERMS = 64, SPLIT_WIDEST = 1 << 20;
+// What mrx_dense_grads and mrx_dense_f32 take: features of a row and outputs of a layer up to DENSE_WIDEST, rows that 32 bits count.
+constexpr int64_t DENSE_WIDEST = 1 << 16;
+bool dense_takes(int64_t rows, int64_t K, int64_t widest) { return rows < (1ll << 31) && K <= DENSE_WIDEST && widest <= DENSE_WIDEST; }
 bool params_suit(ScalarType dt, int64_t rows, int64_t K, int64_t widest, size_t, size_t)
 {
     return dt == at::kBFloat16 ? K * widest <= 512 * 512 : rows >= SPLIT_TERMS && K * widest <= 256 * 256;
@@ -1808,7 +1811,7 @@ struct DenseOp {
             regular = regular && ws.back().device() == x.device() && ws.back().scalar_type() == dt && ws.back().is_contiguous() && ws.back().size(0) > 0 && reinterpret_cast<uintptr_t>(ws.back().data_ptr()) % 16 == 0;
         }
         if (used.empty()) return out;
-        regular = regular && used.size() <= MRX_DENSE_LAYERS && x2.is_contiguous() && reinterpret_cast<uintptr_t>(x2.data_ptr()) % 16 == 0;
+        regular = regular && used.size() <= MRX_DENSE_LAYERS && dense_takes(x2.size(0), x2.size(1), widest) && x2.is_contiguous() && reinterpret_cast<uintptr_t>(x2.data_ptr()) % 16 == 0;
         const bool rows_dx = across.defined() && used.size() == n && regular && input_from_rows(dys, ws, across, x2.size(1), want_params, out);
         for (Tensor &dy : dys) dy = dy.to(dt);   // (a residual stream's gradient: unless that has left its rounded copy)
         const bool own_params = want_params && regular &&

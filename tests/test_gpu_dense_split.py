@@ -129,6 +129,27 @@ def test_bias_gradients_of_what_is_not_finite(bad, row):
         assert (b.grad.double() - want)[fine].abs().max() <= 8 * EPS * 200 ** 0.5
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,K,outs", [(64, 131072, [1]), (70, 65544, [3, 1]), (16, 8, [65537, 16]), (300, 8, [131072])])
+def test_widths_beyond_the_kernels(rows, K, outs, dtype):
+    """More features or outputs than the kernels' 65536: the array library's products, as small as the layers are otherwise."""
+    x, ws, _, dys = _case(rows, K, outs)
+    x, ws, dys = x.to(dtype), [w.to(dtype) for w in ws], [d.to(dtype) for d in dys]
+    print(f"case dense split wide rows={rows} K={K} outs={outs} {dtype}", flush=True)
+    _, dx, dws = _run(x, ws, [None] * len(ws), dys)
+    if dtype == torch.float32:
+        _close(dx, torch.cat(dys, 1), torch.cat(ws))
+    else:   # each layer's share, and their sum, is rounded
+        want, size = sum(d.double() @ w.double() for d, w in zip(dys, ws)), sum((d.double().abs() @ w.double().abs()) for d, w in zip(dys, ws))
+        assert ((dx.double() - want).abs() <= 2.0 ** -7 * size).all()
+    for dw, dy in zip(dws, dys):
+        if dtype == torch.float32:
+            _close(dw, dy.t(), x)
+        else:
+            want = dy.double().t() @ x.double()
+            assert ((dw.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-3).all()
+
+
 def test_residual_and_bfloat16_results():
     """The C entry's residual sum, and an input gradient that is asked for in bfloat16."""
     x, ws, _, dys = _case(1000, 128, [96])
