@@ -651,8 +651,8 @@ int mrx_dense_grads(void *stream, const void *x, const void *const *dys, const v
 /* ---- Dense layers over rows in float32 ----
  * y_l (rows, n_out[l]) = x W_l^T + b_l of up to MRX_DENSE_LAYERS layers on the rows x (rows, K), everything float32 (entries of `biases` may be NULL);
  * residual (rows, n), nullable: added to the one layer's result; skip (n) and skip_x (rows, n), both or neither: so is skip[c] skip_x[r][c].
- * mrx_dense_f32_input_grad: dx (rows, K) = sum_l dy_l W_l, + skip[c] skip_x[r][c] with skip (K), skip_x (rows, K).  K a multiple of 8.  Products on the float16 matrix units, every value as the sum of
- * two scaled float16 ones (22 bits and a sign, 2^-39 of its row's or column's largest value); infinities and NaN as float32 has them.
+ * mrx_dense_f32_input_grad: dx (rows, K) = sum_l dy_l W_l, + skip[c] skip_x[r][c] with skip (K), skip_x (rows, K).  K a multiple of 8.  Products on the bfloat16 matrix units, every value as the
+ * exact sum of three bfloat16 ones (below 2^-110 in magnitude: within 2^-134), a product within 2^-26 of itself; infinities and NaN as float32 has them.
  * workspace: mrx_dense_f32_workspace(...), mrx_dense_f32_input_grad_workspace(...) floats (0: sizes that are not served), overwritten.  x, weights, results and workspace on 16-byte boundaries. */
 int64_t mrx_dense_f32_workspace(const int64_t *n_out, int layers, int64_t K);
 int mrx_dense_f32(void *stream, const float *x, const void *const *weights, const void *const *biases, void *const *outs,

@@ -20,7 +20,7 @@
 #include "col_sum.h"
 #include "dense_split.h"
 #include "row_dma.h"
-#include "split_f16.h"
+#include "split_bf16.h"
 
 #include <type_traits>
 
@@ -166,35 +166,22 @@ __global__ void __launch_bounds__(DG_THREADS, 2) dense_weight_grad_kernel(DenseG
     }
 }
 
-// ---- weight gradients in float32 on the float16 matrix units (split_f16.h)
-// The same tiles, slices and steps; a step's rows are split into two float16 tiles each on their way into LDS, every column with a power of two
-// of its own.  A column's scale leaves room for values 16 times the largest so far: where a step goes beyond, the workgroup finds the columns'
-// largest values again, brings the running sums to the new scales and splits the step once more (the first step does).
-// us, here / on float32 products before: 32768 x 256 -> 1024 + 512 + 512 + 8 199 / 305 (the array library), 131072 x 256 -> 3 x 256 + 4 315 / 576, 4096 x 256 ->
-// 3 x 256 35 / 53.  Without the products the first takes 170, without the splitting 165, without the loads 145: two workgroups of a compute
-// unit in turn, each a trip to L2, the split, a barrier and the products a step.  Three (half the LDS, a second barrier) spill.
-template <int W> __device__ __forceinline__ f16x8 split_fragment(const _Float16 *tile, int c0, int lane)
+// ---- weight gradients in float32 on the bfloat16 matrix units (split_bf16.h)
+// The same tiles and slices; a step's 32 rows are split into three bfloat16 tiles an operand on their way into LDS, 55 KB of them, one step at a time: two
+// workgroups of a compute unit take turns, one on its way to memory and splitting while the other multiplies (two buffers leave room for one workgroup: 365 us).
+// us, here / the array library: 32768 x 256 -> 1024 + 512 + 512 + 8 259 / 289, 131072 x 256 -> 3 x 256 + 4 412 / 414, 131072 x 128 -> 3 x 128 104 / 125, 4096 x 256
+// -> 3 x 256 36 / 79.  What bounds the first are a step's 1536 cycles of products, 1200 of splitting and about as many of LDS, in two workgroups' turns.
+template <int W> __device__ __forceinline__ bf16x8 split_fragment(const __bf16 *tile, int c0, int lane)
 {
-    constexpr int LD = W + 16;   // as RowTile::LD
-    const int i = lane & 15, g = lane >> 4;
-    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-    const _Float16 *p = tile + (8 * g + (i >> 2)) * LD + c0 + 4 * (i & 3);
-    union {
-        s16x4 h[2];
-        f16x8 f;
-    } u;
-    u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)p);
-    u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(p + 4 * LD));
-    return u.f;
+    return TT<__bf16>::template load<KROW>(tile, W + 16, c0, 0, lane);   // (as RowTile::LD)
 }
 
-// One operand's step: 32 rows x W columns in registers, and the scales of this thread's four columns.
+// One operand's step: 32 rows x W columns in registers.
 template <int W> struct SplitTile {
     using Rows = RowTile<float, 32, W, KROW>;
-    static constexpr int LD = W + 16, HALF = 32 * LD;   // float16 between rows; of the high, then of the low parts
+    static constexpr int LD = W + 16, PART = 32 * LD;   // bfloat16 between rows; of one part
     static constexpr int COLS = W / 4;                  // threads across
     Rows rows;
-    float scale[4];
     // columns past the last count nothing
     __device__ __forceinline__ void mask(int tid)
     {
@@ -206,52 +193,34 @@ template <int W> struct SplitTile {
                 for (int q = 0; q < 4; ++q)
                     if (q >= have) rows.v[p][q] = 0u;
     }
-    // the largest scaled value of this thread's part; in (hi, lo) tiles
-    __device__ __forceinline__ float to_lds(_Float16 *dst, int tid)
+    // the largest of this thread's values; in three tiles
+    __device__ __forceinline__ float to_lds(__bf16 *dst, int tid)
     {
-        float m = 0.f;
-        const sf32x4 s = {scale[0], scale[1], scale[2], scale[3]};
+        float most = 0.f;
 #pragma unroll
         for (int p = 0; p < Rows::PASSES; ++p) {
-            const sf32x4 x = __builtin_bit_cast(sf32x4, rows.v[p]) * s;
-            m = max4(m, x);
-            const Split4 y = split4(x, 1.f);
+            const f32x4 x = __builtin_bit_cast(f32x4, rows.v[p]);
+            most = max4(most, x);
+            Words<2>::type parts[PARTS];
+            split_parts<2>(&x, parts);
             const int at = (tid / COLS + p * (DG_THREADS / COLS)) * LD + tid % COLS * 4;
-            *reinterpret_cast<f16x4 *>(dst + at) = y.hi;
-            *reinterpret_cast<f16x4 *>(dst + HALF + at) = y.lo;
+#pragma unroll
+            for (int h = 0; h < PARTS; ++h) *reinterpret_cast<Words<2>::type *>(dst + h * PART + at) = parts[h];
         }
-        return m;
-    }
-    __device__ __forceinline__ void peaks(int *top, int tid) const   // of each of this thread's columns
-    {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            float m = 0.f;
-#pragma unroll
-            for (int p = 0; p < Rows::PASSES; ++p) m = fmaxf(m, fabsf(__uint_as_float(rows.v[p][q])));
-            atomicMax(&top[tid % COLS * 4 + q], (int)(__float_as_uint(m) & 0x7fffffffu));
-        }
-    }
-    __device__ __forceinline__ void rescale(const int *log_scale, int tid)
-    {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) scale[q] = power_of_two(log_scale[tid % COLS * 4 + q]);
+        return most;
     }
 };
-constexpr int SG_TOP = 10;            // the largest of a column so far lies in [2^10, 2^11) when its scale is chosen
-constexpr float SG_LIMIT = 32768.f;
 
-template <int TN, int TK> constexpr size_t split_lds() { return 2 * 2 * (SplitTile<TN>::HALF + SplitTile<TK>::HALF) * sizeof(_Float16); }
+template <int TN, int TK> constexpr size_t split_lds() { return PARTS * (SplitTile<TN>::PART + SplitTile<TK>::PART) * sizeof(__bf16); }
 
 template <int TN, int TK> __global__ void __launch_bounds__(DG_THREADS, 2) split_weight_grad_kernel(DenseGradArgs a)
 {
     constexpr int RC = SG_STEP, MBW = TK / 32, NBW = TN / 32;
     using TM = TileMap<TK, TN, DG_WAVES, MBW>;
-    constexpr int BUF = 2 * (SplitTile<TK>::HALF + SplitTile<TN>::HALF);
     static_assert(RC == 32, "one block of the contraction a step");
     extern __shared__ __align__(16) unsigned char smem[];
-    __shared__ int top[TK + TN], log_scale[TK + TN], change[TK + TN], beyond[2], infinite;
-    _Float16 *const lds = reinterpret_cast<_Float16 *>(smem);
+    __shared__ int beyond;   // a value without parts is among the operands
+    __bf16 *const sx = reinterpret_cast<__bf16 *>(smem), *const sy = sx + PARTS * SplitTile<TK>::PART;
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), i16 = lane & 15, g = lane >> 4;
     const int tiles = a.first_tile[a.layers] * a.ktiles;
     const int64_t task = task_of((int64_t)tiles * a.slices);
@@ -264,89 +233,64 @@ template <int TN, int TK> __global__ void __launch_bounds__(DG_THREADS, 2) split
     const int64_t r0 = slice * a.slice_rows, r1 = r0 + a.slice_rows < a.rows ? r0 + a.slice_rows : a.rows;
     const float *x = static_cast<const float *>(a.x), *dy = static_cast<const float *>(a.dy[l]);
     const bool bias = a.b_at[l] >= 0 && kt == 0;
-    if (tid < TK + TN) top[tid] = 0, log_scale[tid] = 126;
-    if (tid == 0) beyond[0] = beyond[1] = infinite = 0;
+    if (tid == 0) beyond = 0;
+    sync_lds();   // before any wave sets it
 
     f32x4 acc[TM::TPW];
     zero_acc<TM::TPW>(acc);
     // the bias gradient, a step's sum at a time with what its additions round off
-    sf32x4 bias_sum = {0.f, 0.f, 0.f, 0.f}, bias_low = bias_sum;
+    f32x4 bias_sum = {0.f, 0.f, 0.f, 0.f}, bias_low = bias_sum;
     SplitTile<TK> tx;
     SplitTile<TN> ty;
-    sync_lds();
-    tx.rescale(log_scale, tid);
-    ty.rescale(log_scale + TK, tid);
     auto load = [&](int64_t r) {
         tx.rows.load(x, r, r1, a.rows, k0, a.K, tid);
         ty.rows.load(dy, r, r1, a.rows, n0, N, tid);
     };
     load(r0);
-    int buf = 0, step = 0;
-    for (int64_t r = r0; r < r1; r += RC, buf ^= 1) {
-        _Float16 *const sx = lds + buf * BUF, *const sy = sx + 2 * SplitTile<TK>::HALF;
-        ++step;
+    float most = 0.f;
+    for (int64_t r = r0; r < r1; r += RC) {
         tx.mask(tid);
         ty.mask(tid);
-        if (fmaxf(tx.to_lds(sx, tid), ty.to_lds(sy, tid)) >= SG_LIMIT) beyond[buf] = step;
         if (bias) {
-            sf32x4 part = {0.f, 0.f, 0.f, 0.f};
+            f32x4 part = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int p = 0; p < SplitTile<TN>::Rows::PASSES; ++p) part += __builtin_bit_cast(sf32x4, ty.rows.v[p]);
-            const sf32x4 y = part - bias_low, s = bias_sum + y;
+            for (int p = 0; p < SplitTile<TN>::Rows::PASSES; ++p) part += __builtin_bit_cast(f32x4, ty.rows.v[p]);
+            const f32x4 y = part - bias_low, s = bias_sum + y;
 #pragma unroll
             for (int q = 0; q < 4; ++q) bias_low[q] = fabsf(s[q]) <= 3.402823466e38f ? (s[q] - bias_sum[q]) - y[q] : 0.f;   // an infinite sum rounds nothing off
             bias_sum = s;
         }
-        sync_lds();   // the buffer two steps back has been read by every wave that reaches the barrier
-        if (beyond[buf] == step) {
-            tx.peaks(top, tid);
-            ty.peaks(top + TK, tid);
-            sync_lds();
-            if (tid < TK + TN) {
-                const int e = exponent(__uint_as_float((uint32_t)top[tid])), was = log_scale[tid];
-                int now = SG_TOP - e;
-                now = now < was ? now : was;
-                now = now < -126 ? -126 : now;
-                change[tid] = now - was, log_scale[tid] = now;
-                if (e == 128) infinite = 1;
-            }
-            sync_lds();
-#pragma unroll
-            for (int j = 0; j < TM::TPW; ++j)
-#pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    acc[j][v] = __builtin_ldexpf(acc[j][v], change[TM::mt(w, j) * 16 + 4 * g + v] + change[TK + TM::nt(w, j) * 16 + i16]);
-            tx.rescale(log_scale, tid);
-            ty.rescale(log_scale + TK, tid);
-            tx.to_lds(sx, tid);
-            ty.to_lds(sy, tid);
-            sync_lds();
-        }
+        if (r > r0) sync_lds();   // the step before has been read
+        most = fmaxf(most, fmaxf(tx.to_lds(sx, tid), ty.to_lds(sy, tid)));
         if (r + RC < r1) load(r + RC);
-        f16x8 fx[MBW][2];
+        sync_lds();
+        bf16x8 fx[MBW][PARTS];
 #pragma unroll
         for (int m = 0; m < MBW; ++m)
 #pragma unroll
-            for (int h = 0; h < 2; ++h) fx[m][h] = split_fragment<TK>(sx + h * SplitTile<TK>::HALF, TM::mt(w, m * TM::NBW) * 16, lane);
+            for (int h = 0; h < PARTS; ++h) fx[m][h] = split_fragment<TK>(sx + h * SplitTile<TK>::PART, TM::mt(w, m * TM::NBW) * 16, lane);
 #pragma unroll
         for (int n = 0; n < NBW; ++n) {
-            f16x8 fy[2];
+            bf16x8 fy[PARTS];
 #pragma unroll
-            for (int h = 0; h < 2; ++h) fy[h] = split_fragment<TN>(sy + h * SplitTile<TN>::HALF, TM::nt(w, n) * 16, lane);
-            // the small products by themselves first: two roundings of the running sum a step instead of three
+            for (int h = 0; h < PARTS; ++h) fy[h] = split_fragment<TN>(sy + h * SplitTile<TN>::PART, TM::nt(w, n) * 16, lane);
+            // the small products by themselves first: two roundings of the running sum a step
             f32x4 low[MBW];
 #pragma unroll
-            for (int m = 0; m < MBW; ++m) low[m] = mma_f16(fx[m][1], fy[0], f32x4{0.f, 0.f, 0.f, 0.f});
+            for (int q = 0; q < PRODUCTS; ++q)
 #pragma unroll
-            for (int m = 0; m < MBW; ++m) low[m] = mma_f16(fx[m][0], fy[1], low[m]);
-#pragma unroll
-            for (int m = 0; m < MBW; ++m) acc[m * TM::NBW + n] = mma_f16(fx[m][0], fy[0], acc[m * TM::NBW + n]);
+                for (int m = 0; m < MBW; ++m) {
+                    if (q + 1 < PRODUCTS) low[m] = mma_bf16(fx[m][PART_A[q]], fy[PART_B[q]], q ? low[m] : f32x4{0.f, 0.f, 0.f, 0.f});
+                    else acc[m * TM::NBW + n] = mma_bf16(fx[m][0], fy[0], acc[m * TM::NBW + n]);
+                }
 #pragma unroll
             for (int m = 0; m < MBW; ++m) acc[m * TM::NBW + n] += low[m];
         }
     }
+    if (most > BF16_MOST) beyond = 1;
+    sync_lds();
     float *const out = a.out + slice * a.total;
-    if (infinite) {   // sums one by one: what an infinity makes of them is float32's
+    if (beyond) {   // sums one by one: what an infinity makes of them is float32's
         for (int e = tid; e < TN * TK; e += DG_THREADS) {
             const int n = n0 + e / TK, k = k0 + e % TK;
             if (n >= N || k >= a.K) continue;
@@ -359,8 +303,6 @@ template <int TN, int TK> __global__ void __launch_bounds__(DG_THREADS, 2) split
         for (int j = 0; j < TM::TPW; ++j) {
             const int ki = TM::mt(w, j) * 16 + 4 * g, ni = TM::nt(w, j) * 16 + i16;
             if (k0 + ki >= a.K || n0 + ni >= N) continue;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc[j][v] = __builtin_ldexpf(acc[j][v], -(log_scale[ki + v] + log_scale[TK + ni]));
             *reinterpret_cast<f32x4 *>(out + a.w_at[l] + (int64_t)(n0 + ni) * a.K + k0 + ki) = acc[j];
         }
     }
@@ -368,7 +310,7 @@ template <int TN, int TK> __global__ void __launch_bounds__(DG_THREADS, 2) split
         constexpr int SHARES = DG_THREADS / SplitTile<TN>::COLS;
         float *const part = reinterpret_cast<float *>(smem);
         sync_lds();
-        *reinterpret_cast<sf32x4 *>(part + tid / SplitTile<TN>::COLS * TN + tid % SplitTile<TN>::COLS * 4) = bias_sum;
+        *reinterpret_cast<f32x4 *>(part + tid / SplitTile<TN>::COLS * TN + tid % SplitTile<TN>::COLS * 4) = bias_sum;
         sync_lds();
         if (tid < TN && n0 + tid < N) {
             float t[SHARES];
@@ -604,7 +546,8 @@ struct WeightPlan {
 // shorter than four steps of a workgroup, and a whole number of such rounds where a slice would have more than CHAIN rows: a running
 // sum in float32 errs in proportion to its length.  131072 rows, three layers of 256 x 256 and one of 256 x 4, error of the weights against
 // float64: bfloat16 (3648 rows a slice) 8.4e-8 -> 4.5e-8, where the array library's slices have 5.2e-8, 132 -> 134 us.  A float32 slice may be longer
-// than on float32 products (512), with a quarter of their roundings: 32768 x 256 -> 2056 outputs 512 rows a slice 2.7e-7 and 220 us, 1152 2.6e-7 and 199 us.
+// than on float32 products (512 rows, 3.9e-7), with a quarter of their roundings: 32768 x 256 -> 2056 outputs 512 rows a slice 1.5e-7 and 280 us, 1152 2.3e-7 and
+// 259 us; the array library 8.1e-7.
 constexpr int64_t CHAIN_BF16 = 2048, CHAIN_F32 = 1152;
 
 constexpr int64_t WIDE_WORK = 3 << 16;

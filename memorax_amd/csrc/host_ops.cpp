@@ -1635,7 +1635,7 @@ std::optional<ScalarType> autocast_dtype(const Tensor &x)
 // bfloat16.  Parameters: while they are bound by reading the rows, i.e. up to widths where the array library's larger tiles take over (us,
 // here / there: 131072 x 256 -> 3 x 256 105 / 277, 11455 x 128 -> 3 x 256 26 / 225, 32768 x 1024 -> 1024 148 / 121).  The input: several layers at
 // once, as narrow (68200 x 128 -> 3 x 64 + 2 25 / 69, 131072 x 256 -> 3 x 256 + 4 118 / 150), or few rows, where the host's calls are what it costs.
-// float32, on the float16 matrix units (split_f16.h), in graphs and thus without the 20 us of the host that a product of the array library costs:
+// float32, on the bfloat16 matrix units (split_bf16.h), in graphs and thus without the 20 us of the host that a product of the array library costs:
 // parameters 4096 x 128 -> 3 x 128 23 / 78, 4096 x 256 -> 3 x 256 35 / 79, 32768 x 256 -> 256 39 / 49, 131072 x 256 -> 3 x 256 + 4 315 / 425.  Wider
 // layers 256 x 512 -> 512 25 / 14, 1024 x 512 -> 512 29 / 15, 4096 x 512 -> 512 38 / 32, 4096 x 512 -> 3 x 512 65 / 83, 4096 x 1024 -> 1024 78 / 74, 16384 x
 // 1024 -> 1024 189 / 252, 32768 x 1024 -> 1024 357 / 504.  The input 4096 x 128 -> 3 x 128 26 / 22, 4096 x 256 -> 3 x 256 30 / 33, 131072 x 256 -> 3 x 256 +

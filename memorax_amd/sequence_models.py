@@ -516,7 +516,7 @@ class GatedLinearRecurrence(SequenceModel):
 # ----------------------------------------------------------------------------------
 # acting: one time step without gradients (ppo.py:105-143), rows = environments
 # ----------------------------------------------------------------------------------
-_SPLIT_TERMS = 64        # the fewest terms of a sum that csrc/host_ops.cpp (SPLIT_TERMS) gives to the float16 matrix units
+_SPLIT_TERMS = 64        # the fewest terms of a sum that csrc/host_ops.cpp (SPLIT_TERMS) gives to the bfloat16 matrix units
 _ACTING_ROWS = 16384   # the most rows that csrc/host_ops.cpp (rows_pay) gives to the row kernels
 
 

@@ -1,4 +1,4 @@
-"""Float32 dense layers on the float16 matrix units (csrc/dense_split.hip, the float32 kernels of csrc/dense_grads.hip) against double
+"""Float32 dense layers on the bfloat16 matrix units (csrc/dense_split.hip, the float32 kernels of csrc/dense_grads.hip) against double
 precision: sizes around their tiles and steps, rows and columns of very different magnitudes, infinities and NaN."""
 import pytest
 import torch
@@ -25,7 +25,7 @@ def _run(x, ws, bs, dys):
 
 
 def _close(got, a, b, add=None):
-    """got = a b (+ add) with a (m, k), b (k, n): an element is out by what splitting leaves of each product (2^-22) and by the roundings of
+    """got = a b (+ add) with a (m, k), b (k, n): an element is out by what splitting leaves of each product (2^-26) and by the roundings of
     its running sum, together within 16 eps of the products' 2-norm -- eight times what they are on average."""
     want = a.double() @ b.double()
     size = (a.double().abs() ** 2 @ b.double().abs() ** 2).sqrt()
@@ -48,7 +48,7 @@ def test_sizes(rows, K, outs):
 
 
 def test_magnitudes():
-    """Every row, and every column of the weights, has its own scale; a step of a longer contraction may be far larger or smaller than the one before."""
+    """Rows, columns of the weights and steps of a longer contraction of very different magnitudes."""
     x, ws, bs, dys = _case(500, 520, [300, 16])
     rows, feats = (torch.randint(-40, 40, (n,), generator=torch.Generator().manual_seed(n)).cuda() for n in (500, 300))
     x = torch.ldexp(x, rows[:, None])
@@ -63,9 +63,32 @@ def test_magnitudes():
     _close(dx, torch.cat(dys, 1), torch.cat(ws))
 
 
+@pytest.mark.parametrize("big", [2.0 ** 20, 1e12, 1e18])
+def test_outliers_that_meet_zeros(big):
+    """A value takes nothing from its row's or column's others, however far above or below them it lies: what the operands hold is in the products,
+    also where the large ones meet zeros."""
+    x, ws, bs, dys = _case(700, 200, [96, 24])
+    x[:, 5], ws[0][:, 5], ws[1][:, 5] = big, 0., 0.                       # a feature that no layer uses
+    x[33, 9], ws[0][:, 9], ws[1][:, 9] = -big, 0., 0.
+    ws[0][3], ws[0][4], ws[1][2] = ws[0][3] * 2.0 ** -50, ws[0][4] * 1e-28, ws[1][2] * 2.0 ** 41
+    ws[0][7, ::2] *= big                                                # a column of wide range
+    x[100:164, ::2] = 0.
+    x[300:310], x[310:320] = x[300:310] * 2.0 ** -60, x[310:320] * 2.0 ** -90
+    dys[0][400:420], dys[1][400:420], x[400:420, 7] = 0., 0., big      # rows without gradients
+    dys[0][:, 11], ws[0][11] = dys[0][:, 11] * big, 0.
+    dys[0][500:600, 12], x[500:600, 13] = big, 0.
+    _, dx, dws = _run(x, ws, bs, dys)
+    _close(dx, torch.cat(dys, 1), torch.cat(ws))
+    for dw, dy in zip(dws, dys):
+        _close(dw, dy.t(), x)
+    ys, _, _ = _run(x, ws, bs, dys)
+    for y, w, b in zip(ys, ws, bs):
+        _close(y, x, w.t(), b)
+
+
 @pytest.mark.parametrize("late", [False, True])
 def test_columns_that_grow_along_the_rows(late):
-    """The parameters' gradients rescale a column when a later step goes beyond the earlier ones, zeros first among them."""
+    """The parameters' gradients where a later step of rows goes far beyond the earlier ones, zeros first among them."""
     x, ws, bs, dys = _case(2000, 64, [64, 8])
     x[:, 5], dys[0][:, 9] = 0., 0.
     at = slice(700, None) if late else slice(0, 40)
