@@ -594,13 +594,11 @@ la_bwd_kernel(const T *__restrict__ q, const T *__restrict__ k, const T *__restr
 #pragma unroll
                     for (int j = 0; j < TMR::TPW; ++j) {
                         const int r = TMR::nt(w, j) * 16 + li;
-                        const f32x4 zz = *reinterpret_cast<const f32x4 *>(sZf + TMR::mt(w, j) * 16 + 4 * lg) * sDd[r];
-                        if constexpr (ONE) {  // the product goes, not a factor: z is the first episode's and may be anything
+                        const f32x4 zz = *reinterpret_cast<const f32x4 *>(sZf + TMR::mt(w, j) * 16 + 4 * lg);
+                        const float dd = sDd[r];
+                        // one unit: selected, not multiplied by zero: z is the first episode's and may be anything
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) acc[j][e] += r < r_first ? zz[e] : 0.f;
-                        } else {
-                            acc[j] += zz;
-                        }
+                        for (int e = 0; e < 4; ++e) acc[j][e] = !ONE || r < r_first ? fmaf(zz[e], dd, acc[j][e]) : acc[j][e];
                     }
                 }
                 auto sc = [&](int r, int d0) {
