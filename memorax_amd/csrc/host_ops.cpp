@@ -24,6 +24,7 @@
 #include <torch/csrc/utils/pybind.h>
 
 #include <array>
+#include <numeric>
 
 #include "memorax_amd.h"
 
@@ -1631,34 +1632,37 @@ std::optional<ScalarType> autocast_dtype(const Tensor &x)
     return std::nullopt;
 }
 
-// Which of a group's gradients the library's kernels form.
+// What the library's kernels form of a group of dense layers on `rows` rows of K features, `widest` the most outputs of a layer and `outputs` those of all; the
+// rest are the array library's products.
 // bfloat16.  Parameters: while they are bound by reading the rows, i.e. up to widths where the array library's larger tiles take over (us,
 // here / there: 131072 x 256 -> 3 x 256 105 / 277, 11455 x 128 -> 3 x 256 26 / 225, 32768 x 1024 -> 1024 148 / 121).  The input: several layers at
 // once, as narrow (68200 x 128 -> 3 x 64 + 2 25 / 69, 131072 x 256 -> 3 x 256 + 4 118 / 150), or few rows, where the host's calls are what it costs.
-// float32, on the bfloat16 matrix units (split_bf16.h), in graphs and thus without the 20 us of the host that a product of the array library costs:
-// parameters 4096 x 128 -> 3 x 128 23 / 78, 4096 x 256 -> 3 x 256 35 / 79, 32768 x 256 -> 256 39 / 49, 131072 x 256 -> 3 x 256 + 4 315 / 425.  Wider
-// layers 256 x 512 -> 512 25 / 14, 1024 x 512 -> 512 29 / 15, 4096 x 512 -> 512 38 / 32, 4096 x 512 -> 3 x 512 65 / 83, 4096 x 1024 -> 1024 78 / 74, 16384 x
-// 1024 -> 1024 189 / 252, 32768 x 1024 -> 1024 357 / 504.  The input 4096 x 128 -> 3 x 128 26 / 22, 4096 x 256 -> 3 x 256 30 / 33, 131072 x 256 -> 3 x 256 +
-// 4 261 / 520; one layer 256 x 512 -> 512 24 / 15, 1024 x 512 -> 512 24 / 15, 4096 x 512 -> 512 26 / 27, 4096 x 1024 -> 1024 53 / 75, 32768 x 512 -> 256 47 / 83.
-// Sums of fewer than SPLIT_TERMS products stay float32's, whose error is that of their few additions: 64 terms 1.0e-7 here, 1.4e-7 there, 8 terms
-// 1.0e-7 and 0.3e-7.
+// float32, on the bfloat16 matrix units (split_bf16.h).  Times in graphs, i.e. without the 20 us of the host that a product of the array library costs beside;
+// sizes are taken where these are no longer here, and groups up to 512 x 512 on few rows, whose gradient of the input has always been one call of the host's.
+//   forward     1024 x 128 -> 3 x 128 15 / 18, 1024 x 256 -> 3 x 256 19 / 21, 4096 x 512 -> 512 30 / 31, 4096 x 512 -> 3 x 512 50 / 63, 4096 x 1024 -> 1024 62 / 77;
+//               not 256 x 512 -> 512 21 / 15, 1024 x 512 -> 3 x 512 33 / 28, 1024 x 1024 -> 1024 38 / 28
+//   parameters  1024 x 256 -> 3 x 256 28 / 32, 12288 x 128 -> 256 28 / 28, 32768 x 256 -> 256 45 / 43, 131072 x 256 -> 3 x 256 + 4 412 / 414; groups 4096 x 512 -> 3 x 512
+//               76 / 80, 32768 x 256 -> 1024 + 512 + 512 + 8 259 / 289; with a bias 8192 x 512 -> 512 51 / 76, 32768 x 512 -> 256 74 / 100, without 50 / 58 and 73 / 75; not
+//               1024 x 512 -> 3 x 512 52 / 32, 4096 x 512 -> 512 38 / 30, 16384 x 1024 -> 1024 246 / 238
+//   input       4096 x 1024 -> 1024 62 / 69, 32768 x 256 -> 256 35 / 43, 131072 x 256 -> 3 x 256 + 4 303 / 504; groups 4096 x 256 -> 3 x 256 29 / 32, 1024 x 256 ->
+//               3 x 256 25 / 19, 1024 x 512 -> 3 x 512 43 / 31, 256 x 512 -> 3 x 512 43 / 23; not 12288 x 128 -> 256 21 / 17, 4096 x 512 -> 512 29 / 24, 1024 x 1024 -> 3 x 1024 88 / 62
+// Sums of fewer than SPLIT_TERMS products stay float32's, whose error is that of their few additions.
 constexpr int64_t SPLIT_TERMS = 64, SPLIT_WIDEST = 1 << 20;
 // What mrx_dense_grads and mrx_dense_f32 take: features of a row and outputs of a layer up to DENSE_WIDEST, rows that 32 bits count.
 constexpr int64_t DENSE_WIDEST = 1 << 16;
-bool dense_takes(int64_t rows, int64_t K, int64_t widest) { return rows < (1ll << 31) && K <= DENSE_WIDEST && widest <= DENSE_WIDEST; }
-bool params_suit(ScalarType dt, int64_t rows, int64_t K, int64_t widest, size_t, size_t)
+struct DenseRoutes {
+    bool forward, params, input;
+};
+DenseRoutes dense_routes(ScalarType dt, int64_t rows, int64_t K, int64_t widest, int64_t outputs, int64_t layers)
 {
-    return dt == at::kBFloat16 ? K * widest <= 512 * 512 : rows >= SPLIT_TERMS && K * widest <= 256 * 256;
-}
-// The same for float32 layers beyond that: results of many tiles, which the array library needs many rows to be slower at.
-bool wide_params_suit(ScalarType dt, int64_t rows, int64_t K, int64_t widest)
-{
-    return dt == at::kFloat && K * widest > 256 * 256 && K * widest <= SPLIT_WIDEST && (rows >= 4096 || (rows >= SPLIT_TERMS && K * widest <= 256 * 1024));
-}
-bool input_suits(ScalarType dt, int64_t rows, int64_t K, int64_t widest, int64_t outputs, size_t layers)
-{
-    if (dt == at::kFloat) return outputs >= SPLIT_TERMS && K * widest <= SPLIT_WIDEST && (layers > 1 || rows >= 4096 || K * widest <= 256 * 512);
-    return layers > 1 && ((K <= 256 && widest <= 256) || (rows <= 4096 && K * widest <= 512 * 512));
+    if (K % 8 != 0 || rows >= (1ll << 31) || K > DENSE_WIDEST || widest > DENSE_WIDEST || layers > MRX_DENSE_LAYERS) return {};
+    const int64_t size = K * widest;
+    const bool group = layers > 1, many = rows >= 4096, more = rows >= 8192;
+    if (dt == at::kBFloat16) return {false, size <= 512 * 512, group && ((K <= 256 && widest <= 256) || (rows <= 4096 && size <= 512 * 512))};
+    if (dt != at::kFloat || size > SPLIT_WIDEST) return {};
+    const bool small = size <= 256 * 256, middle = size <= 512 * 512;
+    return {K >= SPLIT_TERMS && (small || many), rows >= SPLIT_TERMS && (small || (middle && (group ? many : more))),
+            outputs >= SPLIT_TERMS && ((group && middle) || (many && rows * K * outputs >= 1ll << 31))};
 }
 
 // Layers in bfloat16 whose weights fit the registers of a compute unit: the rows pass all of them once, in either direction (dense_rows.hip).
@@ -1703,15 +1707,17 @@ int row_layers(const Tensor &x, const std::vector<Tensor> &weights, const std::v
     return lib.mrx_dense_rows_suit(x.numel() / x.size(-1), x.size(-1), n.data(), (int)weights.size());
 }
 
-// The outputs of float32 layers on float32 rows (dense_split.hip), residual: added to the one layer's; nothing where the library does not serve them.
+// The outputs of float32 layers on float32 rows (dense_split.hip), residual: added to the one layer's; nothing where the library does not serve them or -- unless
+// `any` size is to be -- they are the array library's (dense_routes).
 std::vector<Tensor> dense_f32(const Tensor &x_, const std::vector<Tensor> &weights, const std::vector<OptTensor> &biases, const Tensor &residual,
-                              const Tensor &skip = Tensor(), const Tensor &skip_x = Tensor())
+                              bool any = false, const Tensor &skip = Tensor(), const Tensor &skip_x = Tensor())
 {
     std::vector<Tensor> out;
     std::array<int64_t, MRX_DENSE_LAYERS> n{};
     if (x_.scalar_type() != at::kFloat || !plain_layers(x_, weights, biases, [](ScalarType dt) { return dt == at::kFloat; }, n)) return out;
     const int64_t K = x_.size(-1), rows = x_.numel() / K, floats = lib.mrx_dense_f32_workspace(n.data(), (int)weights.size(), K);
-    if (!floats || rows >= (1ll << 31) || K < SPLIT_TERMS || K * *std::max_element(n.begin(), n.end()) > SPLIT_WIDEST) return out;
+    const int64_t widest = *std::max_element(n.begin(), n.end()), outputs = std::accumulate(n.begin(), n.end(), int64_t(0));
+    if (!floats || rows >= (1ll << 31) || (!any && !dense_routes(at::kFloat, rows, K, widest, outputs, (int64_t)weights.size()).forward)) return out;
     const Tensor x = dense16(x_), work = fresh({floats}, at::kFloat, x);
     std::array<const void *, MRX_DENSE_LAYERS> w{}, b{};
     std::array<void *, MRX_DENSE_LAYERS> y{};
@@ -1811,14 +1817,11 @@ struct DenseOp {
             regular = regular && ws.back().device() == x.device() && ws.back().scalar_type() == dt && ws.back().is_contiguous() && ws.back().size(0) > 0 && reinterpret_cast<uintptr_t>(ws.back().data_ptr()) % 16 == 0;
         }
         if (used.empty()) return out;
-        regular = regular && used.size() <= MRX_DENSE_LAYERS && dense_takes(x2.size(0), x2.size(1), widest) && x2.is_contiguous() && reinterpret_cast<uintptr_t>(x2.data_ptr()) % 16 == 0;
+        regular = regular && used.size() <= MRX_DENSE_LAYERS && x2.is_contiguous() && reinterpret_cast<uintptr_t>(x2.data_ptr()) % 16 == 0;
         const bool rows_dx = across.defined() && used.size() == n && regular && input_from_rows(dys, ws, across, x2.size(1), want_params, out);
         for (Tensor &dy : dys) dy = dy.to(dt);   // (a residual stream's gradient: unless that has left its rounded copy)
-        const bool own_params = want_params && regular &&
-                                (params_suit(dt, x2.size(0), x2.size(1), widest, used.size(), std::count(bias.begin(), bias.end(), true)) ||
-                                 wide_params_suit(dt, x2.size(0), x2.size(1), widest)),
-                   own_dx = node.wants(0) && !rows_dx && regular && (x_dtype == at::kFloat || x_dtype == at::kBFloat16) &&
-                            input_suits(dt, x2.size(0), x2.size(1), widest, outputs, used.size());
+        const DenseRoutes routes = regular ? dense_routes(dt, x2.size(0), x2.size(1), widest, outputs, (int64_t)used.size()) : DenseRoutes{};
+        const bool own_params = want_params && routes.params, own_dx = node.wants(0) && !rows_dx && routes.input && (x_dtype == at::kFloat || x_dtype == at::kBFloat16);
         if (own_params || own_dx) {
             auto r = dense_grads(x2, dys, ws, bias, own_dx, x_dtype, own_params);
             if (own_dx) out[0] = r[0];
@@ -1941,8 +1944,8 @@ struct HeadMapsOp {
         int64_t widest = 0;
         for (const Tensor &dy : dys) widest = std::max(widest, dy.size(1));
         std::vector<Tensor> whole;
-        if (x2.size(1) % 8 == 0 && dys.size() <= MRX_DENSE_LAYERS && reinterpret_cast<uintptr_t>(x2.data_ptr()) % 16 == 0 &&
-            params_suit(x2.scalar_type(), x2.size(0), x2.size(1), widest, dys.size(), 0)) {
+        if (reinterpret_cast<uintptr_t>(x2.data_ptr()) % 16 == 0 &&
+            dense_routes(x2.scalar_type(), x2.size(0), x2.size(1), widest, widest, (int64_t)dys.size()).params) {
             whole = dense_grads(x2, dys, {}, std::vector<bool>(dys.size(), false), false, x2.scalar_type(), true);
             whole.erase(whole.begin());
         } else {
@@ -2198,10 +2201,10 @@ std::tuple<Tensor, Tensor, Tensor> lru_layer(const Tensor &x_, const OptTensor &
         for (int i = 0; i < 8; ++i) chk(q[i], names[i], at::kFloat, shapes[i]), params[i] = fptr(q[i]);
         decay = fresh({N}, at::kComplexFloat, x), wb = fresh({2 * N, F}, at::kFloat, x), wc = fresh({F, 2 * N}, at::kFloat, x);
         check(lib.mrx_lru_params_fwd(stream(), params, ptr(decay), fptr(wb), fptr(wc), N, F), "mrx_lru_params_fwd");
-        const auto u = dense_f32(x, {wb}, {std::nullopt}, Tensor());
+        const auto u = dense_f32(x, {wb}, {std::nullopt}, Tensor(), true);
         TORCH_CHECK_VALUE(!u.empty(), "lru_layer: sizes that the float32 products do not serve");
         r = scan_fwd(decay, at::view_as_complex(u[0].view({B, T, N, 2})), done, some(h0), some(P0_.contiguous()), true);
-        y = dense_f32(at::view_as_real(r.h).view({B, T, 2 * N}), {wc}, {std::nullopt}, residual, q[7], x)[0];
+        y = dense_f32(at::view_as_real(r.h).view({B, T, 2 * N}), {wc}, {std::nullopt}, residual, true, q[7], x)[0];
     }
     if (need) {
         auto node = std::shared_ptr<OpNode<LruOp>>(new OpNode<LruOp>(), torch::autograd::deleteNode);
@@ -2564,7 +2567,10 @@ PYBIND11_MODULE(_native, m)
     def("dense_onto", &dense_onto);
     def("head_maps", &head_maps);
     def("dense_grads", &dense_grads);
-    def("params_suit", &params_suit);
+    def("dense_routes", +[](ScalarType dt, int64_t rows, int64_t K, int64_t widest, int64_t outputs, int64_t layers) {
+        const DenseRoutes r = dense_routes(dt, rows, K, widest, outputs, layers);
+        return std::make_tuple(r.forward, r.params, r.input);
+    });
     def("weight_gradient", &weight_gradient);
     def("weight_gradient_slices", &weight_gradient_slices);
     def("lru_layer", &lru_layer);

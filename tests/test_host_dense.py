@@ -119,14 +119,32 @@ def test_dense_group_on_the_device_under_autocast():
         assert (m.weight.grad.double() - dw).abs().max().item() <= 1e-4 * dw.abs().max().item()
 
 
-@pytest.mark.parametrize("rows", [8192, 16384, 32768, 50000, 65536, 131072])
-def test_the_choice_of_the_parameter_kernels_has_no_place_for_one_width(rows):
-    """Layers a little narrower than 256 x 256 and 128 x 256 take the route of those widths; no narrower layer is refused what a wider
-    one gets."""
+FORWARD, PARAMS, INPUT = 1, 2, 4
+
+
+@pytest.mark.parametrize("rows,K,outs,routes", [
+    # float32 sums of few products, features that are no whole pieces
+    (63, 64, [64, 64], FORWARD | INPUT), (64, 64, [64, 64], FORWARD | PARAMS | INPUT), (64, 56, [64], PARAMS), (64, 56, [40, 24], PARAMS | INPUT),
+    (64, 56, [40, 23], PARAMS), (64, 60, [64, 64], 0), (1 << 31, 64, [64, 64], 0),
+    # one layer, few rows and many, up to 256 x 256, 512 x 512 and 1024 x 1024
+    (64, 256, [256], FORWARD | PARAMS), (64, 256, [264], 0), (4095, 1024, [1024], 0), (4096, 1024, [1024], FORWARD | INPUT), (4096, 1024, [1032], 0),
+    (32768, 256, [256], FORWARD | PARAMS | INPUT), (32760, 256, [256], FORWARD | PARAMS), (8191, 512, [512], FORWARD), (8192, 512, [512], FORWARD | PARAMS | INPUT), (8192, 512, [520], FORWARD | INPUT),
+    # groups
+    (64, 256, [256, 8], FORWARD | PARAMS | INPUT), (4095, 256, [264, 8], INPUT), (4096, 256, [264, 8], FORWARD | PARAMS | INPUT), (4096, 512, [512, 512], FORWARD | PARAMS | INPUT),
+    (4095, 512, [520, 8], 0), (4096, 512, [520, 8], FORWARD), (4096, 512, [520, 520], FORWARD | INPUT), (64, 128, [128] * 8, FORWARD | PARAMS | INPUT), (64, 128, [128] * 9, 0),
+    # wider than the kernels take
+    (64, 65536, [1], FORWARD | PARAMS), (64, 65544, [1], 0), (64, 131072, [1], 0), (4096, 8, [65536, 8], INPUT), (4096, 8, [65544, 8], 0),
+])
+def test_which_float32_layers_the_library_s_kernels_take(rows, K, outs, routes):
     from memorax_amd._lib import native
-    suits = lambda K, n, biases=0: native().params_suit(torch.float32, rows, K, n, 3, biases)  # noqa: E731
-    assert suits(256, 256) == suits(256, 248) == suits(248, 256) == suits(200, 256)
-    routes = [suits(K, n) for K, n in sorted([(64, 64), (128, 128), (128, 184), (128, 200), (160, 200), (160, 256), (224, 256), (256, 256), (256, 264)],
-                                             key=lambda s: s[0] * s[1])]
-    assert routes == sorted(routes, reverse=True)
-    assert suits(256, 256, 2) and suits(128, 128) and not suits(256, 264, 3)
+    forward, params, dx = native().dense_routes(torch.float32, rows, K, max(outs), sum(outs), len(outs))
+    assert forward * FORWARD + params * PARAMS + dx * INPUT == routes
+
+
+def test_which_bfloat16_layers_the_library_s_kernels_take():
+    from memorax_amd._lib import native
+    routes = lambda rows, K, *outs: native().dense_routes(torch.bfloat16, rows, K, max(outs), sum(outs), len(outs))  # noqa: E731
+    assert routes(32768, 1024, 256) == (False, True, False) and routes(32768, 1024, 264) == (False, False, False)
+    assert routes(32768, 256, 256, 256) == (False, True, True) and routes(4097, 256, 264, 8) == (False, True, False)
+    assert routes(4096, 512, 512, 8) == (False, True, True) and routes(64, 131072, 1) == routes(64, 65544, 1) == (False, False, False)
+    assert native().dense_routes(torch.float64, 4096, 64, 64, 64, 1) == (False, False, False)
