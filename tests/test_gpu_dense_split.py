@@ -1,5 +1,7 @@
 """Float32 dense layers on the bfloat16 matrix units (csrc/dense_split.hip, the float32 kernels of csrc/dense_grads.hip) against double
 precision: sizes around their tiles and steps, rows and columns of very different magnitudes, infinities and NaN."""
+import ctypes
+
 import pytest
 import torch
 
@@ -18,9 +20,13 @@ def _case(rows, K, outs, seed=0):
 
 
 def _run(x, ws, bs, dys):
-    x, ws = x.clone().requires_grad_(), [w.clone().requires_grad_() for w in ws]
+    x, ws, bs = (t.clone().requires_grad_() if torch.is_tensor(t) else [None if u is None else u.clone().requires_grad_() for u in t] for t in (x, ws, bs))
     ys = dense_group(x, [Weights(w, b) for w, b in zip(ws, bs)])
     torch.autograd.backward(ys, dys)
+    for b, dy in zip(bs, dys):   # a sum of rows: sqrt(rows) roundings of a few terms' size, twice over
+        if b is not None and bool(torch.isfinite(dy).all()) and dy.dtype == torch.float32:
+            d = dy.double()
+            assert ((b.grad.double() - d.sum(0)).abs() <= 2 * EPS * (dy.shape[0] * (d ** 2).sum(0)).sqrt() + 1e-38).all()
     return [y.detach() for y in ys], x.grad, [w.grad for w in ws]
 
 
@@ -35,7 +41,8 @@ def _close(got, a, b, add=None):
 
 
 @pytest.mark.parametrize("rows,K,outs", [(1, 64, [64, 3]), (63, 64, [1, 16, 17]), (65, 72, [130, 256]), (128, 256, [64, 64, 64, 2]), (129, 264, [48, 260]),
-                                         (300, 520, [16, 5, 16]), (4097, 256, [512, 256, 8]), (9000, 128, [128] * 8)])
+                                         (300, 520, [16, 5, 16]), (4097, 256, [512, 256, 8]), (9000, 128, [128] * 8),
+                                         (40000, 64, [64, 8]), (17000, 200, [300, 40])])
 def test_sizes(rows, K, outs):
     x, ws, bs, dys = _case(rows, K, outs)
     print(f"case dense split rows={rows} K={K} outs={outs}", flush=True)
@@ -173,12 +180,66 @@ def test_widths_beyond_the_kernels(rows, K, outs, dtype):
             assert ((dw.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-3).all()
 
 
-def test_residual_and_bfloat16_results():
-    """The C entry's residual sum, and an input gradient that is asked for in bfloat16."""
+def test_bfloat16_input_gradients():
+    """An input gradient that is asked for in bfloat16."""
     x, ws, _, dys = _case(1000, 128, [96])
     got = _lib.native().dense_grads(x, dys, ws, [False], True, torch.bfloat16, False)[0]
     want = dys[0].double() @ ws[0].double()
     assert got.dtype == torch.bfloat16 and ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all()
+
+
+def _pointers(*ts):
+    return (ctypes.c_void_p * len(ts))(*(None if t is None else t.data_ptr() for t in ts))
+
+
+@pytest.mark.parametrize("bad", [None, float("inf")])
+@pytest.mark.parametrize("n", [17, 64])
+@pytest.mark.parametrize("rows", [70, 20000])
+def test_what_is_added_to_a_layer_s_result(rows, n, bad):
+    """The C entries' residual and skip, with and without a bias, in rows of whole 16-byte pieces and others, also where the sums are formed one by one."""
+    lib, K = _lib.load(), 72
+    x, (w,), _, (dy,) = _case(rows, K, [n])
+    g = torch.Generator(device="cuda").manual_seed(n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    residual, skip, z, b, sx = rnd(rows, n), rnd(n), rnd(rows, n), rnd(n), rnd(K)
+    zx = rnd(rows, K)
+    if bad is not None:
+        x[13, 3], dy[13, 5] = bad, bad
+    sizes = (ctypes.c_int64 * 1)(n)
+    work = torch.empty(max(lib.mrx_dense_f32_workspace(sizes, 1, K), lib.mrx_dense_f32_input_grad_workspace(sizes, 1, K)), device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    at = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    fine = torch.arange(rows, device="cuda") != (13 if bad is not None else -1)
+    for add, sk, bias in [(residual, None, b), (None, skip, None), (residual, skip, b), (None, None, None)]:
+        y = torch.full((rows, n), -7.0, device="cuda")
+        assert lib.mrx_dense_f32(stream, at(x), _pointers(w), _pointers(bias), _pointers(y), sizes, 1, at(add), at(sk), None if sk is None else at(z), rows, K, at(work)) == 0
+        more = sum((t for t in (add, None if sk is None else sk * z, bias) if t is not None), torch.zeros(rows, n, device="cuda"))
+        size = more.abs() + (0 if add is None else add.abs()) + (0 if bias is None else bias.abs())
+        want = x.double() @ w.double().t() + more.double()
+        room = 16 * EPS * (K ** 0.25 * (x.double() ** 2 @ (w.double() ** 2).t()).sqrt() + size)
+        assert ((y.double() - want).abs() <= room)[fine].all()
+        assert bad is None or torch.equal(y[13].double(), want[13])
+    for sk in (None, sx):
+        dx = torch.full((rows, K), -7.0, device="cuda")
+        assert lib.mrx_dense_f32_input_grad(stream, _pointers(dy), _pointers(w), sizes, 1, at(sk), None if sk is None else at(zx), at(dx), rows, K, at(work)) == 0
+        want = dy.double() @ w.double() + (0 if sk is None else (sk * zx).double())
+        room = 16 * EPS * (n ** 0.25 * (dy.double() ** 2 @ w.double() ** 2).sqrt() + (0 if sk is None else (sk * zx).abs()))
+        assert ((dx.double() - want).abs() <= room)[fine].all()
+        assert bad is None or torch.equal(dx[13].double(), want[13])
+
+
+@pytest.mark.parametrize("rows", [15, 16, 17, 1024, 1025, 2048, 2049, 4096, 4097])
+def test_few_rows(rows):
+    """Tiles of 16, 32 and 64 rows, and one or two of a workgroup's columns to a wave."""
+    for K, outs in ((128, [128, 120, 8]), (256, [256, 40]), (64, [64, 64])):
+        x, ws, bs, dys = _case(rows, K, outs)
+        print(f"case dense split few rows={rows} K={K} outs={outs}", flush=True)
+        ys, dx, dws = _run(x, ws, bs, dys)
+        for y, w, b in zip(ys, ws, bs):
+            _close(y, x, w.t(), b)
+        _close(dx, torch.cat(dys, 1), torch.cat(ws))
+        for dw, dy in zip(dws, dys):
+            _close(dw, dy.t(), x)
 
 
 def test_graph_replays():
