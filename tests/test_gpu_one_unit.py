@@ -157,3 +157,46 @@ def test_a_reset_on_a_chunk_s_first_row_drops_what_enters_it(form, dtype, chunks
             u, w = (t[:, C:] if t.dim() >= 3 and t.shape[1] == T else t for t in (good[n], got[n]))
             if n not in ("dS0", "dz0"):   # of the episode that enters the sequence
                 assert torch.equal(u, w), n
+
+
+@pytest.mark.parametrize("chunks", [4, 12])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("form", FORMS)
+def test_a_reset_drops_what_comes_back_from_later_chunks(form, dtype, chunks):
+    """The gradient of the state that leaves a chunk is not finite, the chunk's own rows pass the screen: it reaches the chunk's last episode and no other."""
+    C = 64 if dtype == "bf16" else 32
+    T = chunks * C
+    done = np.zeros((1, T), bool)
+    done[0, [C, 2 * C + 7]] = True
+    x = _case(1, T, 2, 64, dtype, 8)
+    print(f"case one_unit later chunk form={form} dtype={dtype} chunks={chunks}", flush=True)
+    good = _run(form, x, done, dtype)
+    for what in (float("nan"), float("inf")):
+        bad = dict(x, do=x["do"].copy())
+        bad["do"][0, 3 * C + 3, 1, 40] = what
+        got = _run(form, bad, done, dtype)
+        for n in good:
+            u, w = (t[:, :2 * C + 7] if t.dim() >= 3 and t.shape[1] == T else t for t in (good[n], got[n]))
+            assert torch.equal(u, w), n
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("what", [float("nan"), float("inf"), 200.0])
+def test_a_gate_beyond_bounds_stays_in_its_episode(what, dtype):
+    """Gates are not screened: what they make of a step's decay meets the rows of its own episode only."""
+    C = 64 if dtype == "bf16" else 32
+    T, lo, hi = 3 * C, C + 10, C + 20
+    done = np.zeros((1, T), bool)
+    done[0, [5, lo, hi, 2 * C]] = True
+    x = _case(1, T, 2, 64, dtype, 9)
+    good = _run("gated", x, done, dtype)
+    keep = np.ones(T, bool)
+    keep[lo:hi] = False
+    for row in (lo + 1, lo + 4, hi - 1):
+        bad = dict(x, g=x["g"].copy())
+        bad["g"][0, row, 1] = what
+        print(f"case one_unit gate dtype={dtype} what={what} row={row}", flush=True)
+        got = _run("gated", bad, done, dtype)
+        for n in good:
+            u, w = (t[:, keep] if t.dim() >= 3 and t.shape[1] == T else t for t in (good[n], got[n]))
+            assert torch.equal(u, w), n
