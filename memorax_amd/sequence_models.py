@@ -93,7 +93,8 @@ class MemoroidCellBase(nn.Module):
         return None
 
     def whole_onto(self, residual, x, done, initial_carry):
-        """(next_carry, residual + y) with y as ``whole`` forms it, where a cell's last product takes the sum with it; else None."""
+        """(next_carry, residual + y) with y as ``whole`` forms it, where a cell's last product takes the sum with it; else None.
+        initial_carry: None where the cell is to make it."""
         return None
 
     def acting(self, x, norm, done, carry):
@@ -191,12 +192,12 @@ class Memoroid(SequenceModel):
     def onto(self, residual, inputs, done, carry):
         if type(self).forward is not Memoroid.forward:
             return None
-        if carry is None:
-            carry = self.cell.initialize_carry(None, get_input_shape(inputs))
         if type(self.cell).whole is not MemoroidCellBase.whole:
             return self.cell.whole_onto(residual, inputs, done, carry)
         if not self.cell.closes():
             return None
+        if carry is None:
+            carry = self.cell.initialize_carry(None, get_input_shape(inputs))
         h, next_carry = self.cell.scan(self.cell(inputs), carry, done)
         layer, rows = self.cell.closing(h, inputs)
         return next_carry, native().dense_onto(residual, rows, layer.weight, layer.bias)
@@ -294,7 +295,7 @@ class LRUCell(_DiagonalCell):
                 and x.shape[2] == self.features and self.features % 8 == 0 and self.hidden_dim % 4 == 0 and 2 * self.hidden_dim * self.features <= 1 << 20
                 and all(p.dtype is torch.float32 for p in params)):
             return None
-        h0, P0 = initial_carry
+        h0, P0 = self.initialize_carry(None, get_input_shape(x)) if initial_carry is None else initial_carry
         y, h, P = native().lru_layer(x, residual, params, done, h0[:, 0], P0[:, 0])
         return (h[:, None], P[:, None]), y
 
@@ -852,6 +853,8 @@ class MambaCell(MemoroidCellBase):
         if not (type(self).whole is MambaCell.whole and self._native_sizes() and _as_written(self, MambaCell) and x.is_cuda and x.dtype == torch.float32
                 and x.dim() == 3 and x.shape[0] * x.shape[1] > 0 and autocast_dtype(x) is None):
             return None
+        if initial_carry is None:
+            initial_carry = self.initialize_carry(None, get_input_shape(x))
         y, carry = self._mix(dense_group(x, [self.input_projection, self.B, self.C, self.dt]), done, initial_carry)
         return carry, native().dense_onto(residual, y, layer.weight, layer.bias)
 

@@ -84,6 +84,27 @@ def test_blocks_on_a_float32_stream(cell):
         assert _err(a.double(), b.double()) <= 2e-5
 
 
+@pytest.mark.parametrize("cell", ["lru", "lru of few rows", "s5", "mamba", "linear_attention", "recurrence"])
+def test_a_block_makes_its_carry_once(cell):
+    """Whether the closing layer takes the sum with the stream, or the block finds that it does not."""
+    make = {"lru": lambda: sm.Memoroid(sm.LRUCell(64, 64)), "s5": lambda: sm.Memoroid(sm.S5Cell(64, 32)),
+            "mamba": lambda: sm.Memoroid(sm.MambaCell(64, num_heads=2, head_dim=32, state_dim=16)),
+            "linear_attention": lambda: sm.Memoroid(sm.LinearAttentionCell(64, 32, 2)), "recurrence": lambda: sm.GatedLinearRecurrence(64)}[cell.split(" of")[0]]
+    block = sm.Residual(sm.PreNorm(make(), 64)).cuda()
+    rows, steps, inner = 3 if "few" in cell else 9, 20, block.module.module.cell
+    made, init = [], type(inner).initialize_carry
+
+    class Counting(type(inner)):
+        def initialize_carry(self, key, input_shape):
+            made.append(input_shape)
+            return init(self, key, input_shape)
+
+    inner.__class__ = Counting
+    x, done = torch.randn(rows, steps, 64, device="cuda"), torch.rand(rows, steps, device="cuda") < 0.05
+    block(x.requires_grad_(), done)
+    assert len(made) == 1
+
+
 def test_saved_tensors_in_another_layout():
     """A hook on saved tensors may hand them back with other strides."""
     torch.manual_seed(4)
