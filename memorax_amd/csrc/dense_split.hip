@@ -11,8 +11,8 @@
 // rows are narrower.  Along the layers' outputs a step is 128 features, so that two workgroups share a compute unit and one multiplies while the other stages
 // (32768 rows, below: 256 features 211 us, 128 185).  Longer contractions go on in steps, the layers of an input gradient one after the other.
 // us, here / the array library: 32768 x 256 -> 1024 + 512 + 512 + 8 forward 184 / 297 (188 TFLOP/s of float32 products, 1.1 PFLOP/s of bfloat16 ones),
-// their input gradient 180 / 280; 131072 x 256 -> 3 x 256 + 4 290 / 448 and 303 / 504; 4096 x 256 -> 3 x 256 31 / 34 and 29 / 32.  The bfloat16 products alone
-// are 83 us of the first at the nominal rate; a wave's six products of a tile follow each other while its neighbours' loads are on their way.
+// their input gradient 180 / 280; 131072 x 256 -> 3 x 256 + 4 290 / 448 and 303 / 504; 4096 x 256 -> 3 x 256 31 / 34 and 29 / 32.  The matrix units are
+// busy 58 % of the first's cycles and 52 % of its input gradient's, the vector ALU 18 and 24 %, LDS 15 and 17.
 #include "dense_split.h"
 
 #include "chunk_common.h"
