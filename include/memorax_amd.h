@@ -73,7 +73,8 @@ typedef enum {
  *   multiplies values of other episodes, which is exact while those are finite; the kernels therefore screen
  *   every such chunk first (|q|, |k|, |v|, |beta|, |dout| and the factor's entries <= 2^6, the state's and its
  *   gradient's <= 2^20: bounds under which no intermediate can leave the float32 range) and fall back to
- *   the units per episode for a chunk that fails, so the results are those of MRX_RESETS_PASSES for any data.
+ *   the units per episode for a chunk that fails, so the results are those of MRX_RESETS_PASSES for any data (backward: up to
+ *   the order of two sums).
  *   The forward call merges where it takes the chunk-parallel factor kernel (mrx_factor_path), the backward call always (32-row
  *   chunks).  For callers whose episodes end every hundred steps or so: at head dim 64 and full width the masks are part of the code for
  *   every chunk, which is 2 to 7 % faster than MRX_RESETS_AUTO from there on and 2 to 14 % slower where resets are rare.

@@ -397,6 +397,7 @@ int split_rows(hipStream_t st, const SplitCall &c)
     const bool across = c.dys != nullptr;
     const Sizes z = sizes_of(c.n_out, c.layers, c.K, across);
     if (!z.ok || !c.workspace || !aligned(c.workspace, 16) || c.rows <= 0 || c.rows >= (1ll << 31)) return MRX_ERR_INVALID_ARG;
+    if (const int rc = prepare_device(); rc != MRX_OK) return rc;
     SplitArgs a{};
     a.rows = c.rows, a.K = (int)c.K, a.steps = (int)z.steps, a.tiles = (int)z.tiles, a.residual = c.residual, a.skip = c.skip, a.skip_x = c.skip_x, a.y_bf16 = c.dx_bf16;
     const int SP_K = step_features(across);
@@ -442,7 +443,6 @@ extern "C" int mrx_dense_f32(void *stream, const float *x, const void *const *we
         return MRX_ERR_INVALID_ARG;
     for (int l = 0; l < layers; ++l)
         if (!weights[l] || !outs[l] || !aligned(weights[l], 16) || !aligned(outs[l], 16) || !aligned(biases[l], 4)) return MRX_ERR_INVALID_ARG;
-    if (const int rc = prepare_device(); rc != MRX_OK) return rc;
     SplitCall c;
     c.x = x, c.weights = weights, c.biases = biases, c.outs = outs, c.residual = residual, c.skip = skip, c.skip_x = skip_x, c.n_out = n_out, c.layers = layers, c.rows = rows, c.K = K;
     c.workspace = workspace;
