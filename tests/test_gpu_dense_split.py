@@ -80,7 +80,7 @@ def test_outliers_that_meet_zeros(big):
     ws[0][3], ws[0][4], ws[1][2] = ws[0][3] * 2.0 ** -50, ws[0][4] * 1e-28, ws[1][2] * 2.0 ** 41
     ws[0][7, ::2] *= big                                                # a column of wide range
     x[100:164, ::2] = 0.
-    x[300:310], x[310:320] = x[300:310] * 2.0 ** -60, x[310:320] * 2.0 ** -90
+    x[300:310], x[310:320], x[320:330] = x[300:310] * 2.0 ** -60, x[310:320] * 2.0 ** -90, x[320:330].sign() * (x[320:330].abs() + 1) * 2.0 ** -110
     dys[0][400:420], dys[1][400:420], x[400:420, 7] = 0., 0., big      # rows without gradients
     dys[0][:, 11], ws[0][11] = dys[0][:, 11] * big, 0.
     dys[0][500:600, 12], x[500:600, 13] = big, 0.
