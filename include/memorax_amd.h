@@ -524,13 +524,14 @@ int mrx_mingru_scan_bwd(void *stream, const void *z, const void *h_tilde, const 
                         void *dz, void *dh_tilde, void *dh0, int64_t B, int64_t T, int64_t D,
                         int dtype, int done_dtype);
 /* The same with the read-out of the block around the recurrence, y = h silu(gate), and the carry as the cell keeps it, in logarithms: gate, y (B,T,D) in
- * `dtype`; log_state, log_decay and their successors (B,D) float32.  Backward: dy, the gradients of z, h~ and the gate, and (nullable) that of log_state;
- * g_last (nullable): the gradient of the last state itself. */
+ * `dtype`; log_state, log_decay and their successors (B,D) float32.  ends (2,B,D) float32: the states before the first step and behind the last one, left by the
+ * forward (nullable) for the backward.  Backward: dy, the gradients of z, h~ and the gate, and (nullable) that of log_state; g_last (nullable): the
+ * gradient of log_state's successor. */
 int mrx_gated_scan_fwd(void *stream, const void *z, const void *h_tilde, const void *gate, const void *done, const float *log_state,
-                       const float *log_decay, void *h, void *y, float *log_state_out, float *log_decay_out, int64_t B, int64_t T,
-                       int64_t D, int dtype, int done_dtype);
+                       const float *log_decay, void *h, void *y, float *log_state_out, float *log_decay_out, float *ends, int64_t B,
+                       int64_t T, int64_t D, int dtype, int done_dtype);
 int mrx_gated_scan_bwd(void *stream, const void *z, const void *h_tilde, const void *gate, const void *h, const void *done,
-                       const float *log_state, const void *dy, const float *g_last, void *dz, void *dh_tilde, void *dgate,
+                       const float *ends, const void *dy, const float *g_last, void *dz, void *dh_tilde, void *dgate,
                        float *dlog_state, int64_t B, int64_t T, int64_t D, int dtype, int done_dtype);
 /* with a workspace (see mrx_scan_workspace) */
 int mrx_mingru_scan_fwd_segmented(void *stream, const void *z, const void *h_tilde, const void *done, const void *h0,

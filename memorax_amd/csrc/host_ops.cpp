@@ -1496,12 +1496,12 @@ Tensor silu_gate(const Tensor &h, const Tensor &g)
 
 // A gated recurrence between its projections and its closing layer (scan.hip, GATE).
 struct GatedScanOp {
-    static constexpr int SAVED = 6;   // z, h~, gate, h, log_state, its successor
+    static constexpr int SAVED = 5;   // z, h~, gate, h, the states at both ends
     static constexpr bool ONCE = true;
     static const char *name() { return "MemoraxGatedScanBackward"; }
     Tensor done;
     ScalarType carried;
-    variable_list backward(OpNode<GatedScanOp> &node, std::array<Tensor, 6> &s, variable_list &grads)
+    variable_list backward(OpNode<GatedScanOp> &node, std::array<Tensor, SAVED> &s, variable_list &grads)
     {
         const Tensor &z = s[0];
         const int64_t B = z.size(0), T = z.size(1), D = z.size(2);
@@ -1510,9 +1510,9 @@ struct GatedScanOp {
         chk(s[2], "gate", z.scalar_type(), z.sizes());
         chk(s[3], "h", z.scalar_type(), z.sizes());
         chk(z, "z");
-        chk(s[4], "log_state", at::kFloat, {B, D});
+        chk(s[4], "ends", at::kFloat, {2, B, D});
         chk(dy, "dy", z.scalar_type(), z.sizes());
-        const Tensor g_last = grads[1].defined() ? (grads[1].to(at::kFloat) / s[5].exp()).view({B, D}).contiguous() : Tensor();
+        const Tensor g_last = as(grads[1], at::kFloat);
         const Tensor dz = fresh_like(z), dx = fresh_like(z), dg = fresh_like(z), dls = node.wants(3) ? fresh({B, D}, at::kFloat, z) : Tensor();
         const Done flags(done, B, T);
         check(lib.mrx_gated_scan_bwd(stream(), ptr(z), ptr(s[1]), ptr(s[2]), ptr(s[3]), flags.p(), fptr(s[4]), ptr(dy), fptr(g_last), ptr(dz), ptr(dx), ptr(dg),
@@ -1528,22 +1528,21 @@ std::tuple<Tensor, Tensor, Tensor> gated_scan(const Tensor &z, const Tensor &x, 
 {
     refuse(done, log_decay);
     const bool need = need_grad(z, x, gate, log_state);
-    TORCH_CHECK_VALUE(z.dim() == 3 && log_state.dim() == 3 && log_state.size(1) == 1 && log_decay.dim() == 3 && log_decay.size(1) == 1,
-                      "z must be (B,T,D), the carry (B,1,D)");
+    TORCH_CHECK_VALUE(z.dim() == 3 && log_state.dim() == 3 && log_decay.dim() == 3, "z must be (B,T,D), the carry (B,1,D)");
     const int64_t B = z.size(0), T = z.size(1), D = z.size(2);
     const auto dt = z.scalar_type();
     chk_scan_dtype(dt, false, "gated_scan");
-    // long sequences over few columns run in segments, which know nothing of gates: the operations this stands for
-    if (lib.mrx_scan_workspace(B, T, D, code(dt), MRX_SCAN_MINGRU) || (need && lib.mrx_scan_workspace(B, T, D, code(dt), MRX_SCAN_MINGRU | MRX_SCAN_BACKWARD))) {
+    // long sequences over few columns run in segments, which know nothing of gates: the operations this stands for; a carry of more than one step likewise
+    if (log_state.size(1) != 1 || log_decay.size(1) != 1 || lib.mrx_scan_workspace(B, T, D, code(dt), MRX_SCAN_MINGRU) ||
+        (need && lib.mrx_scan_workspace(B, T, D, code(dt), MRX_SCAN_MINGRU | MRX_SCAN_BACKWARD))) {
         const auto [h, h_last, P_last] = mingru_scan(z, x, done, log_state.exp().select(1, 0), log_decay.exp().select(1, 0));
         return {silu_gate(h, gate), h_last.unsqueeze(1).log(), P_last.unsqueeze(1).log()};
     }
-    Tensor z_, x_, g_, ls, h, y, ls_out, ld_out;
+    Tensor z_, x_, g_, h, y, ls_out, ld_out, ends;
     {
         at::AutoDispatchBelowADInplaceOrView below;
         z_ = z.contiguous(), x_ = as(x, dt), g_ = as(gate, dt);
-        ls = as(log_state, at::kFloat).view({B, D});
-        const Tensor ld = as(log_decay, at::kFloat).view({B, D});
+        const Tensor ls = as(log_state.select(1, 0), at::kFloat), ld = as(log_decay.select(1, 0), at::kFloat);
         chk(z_, "z");
         chk(x_, "h_tilde", dt, z.sizes());
         chk(g_, "gate", dt, z.sizes());
@@ -1551,7 +1550,8 @@ std::tuple<Tensor, Tensor, Tensor> gated_scan(const Tensor &z, const Tensor &x, 
         chk(ld, "log_decay", at::kFloat, {B, D});
         const Done flags(done, B, T);
         h = fresh_like(z_), y = fresh_like(z_), ls_out = fresh({B, 1, D}, at::kFloat, z_), ld_out = fresh({B, 1, D}, at::kFloat, z_);
-        check(lib.mrx_gated_scan_fwd(stream(), ptr(z_), ptr(x_), ptr(g_), flags.p(), fptr(ls), fptr(ld), ptr(h), ptr(y), fptr(ls_out), fptr(ld_out), B, T, D,
+        if (need) ends = fresh({2, B, D}, at::kFloat, z_);
+        check(lib.mrx_gated_scan_fwd(stream(), ptr(z_), ptr(x_), ptr(g_), flags.p(), fptr(ls), fptr(ld), ptr(h), ptr(y), fptr(ls_out), fptr(ld_out), fptr(ends), B, T, D,
                                      code(dt), flags.dtype),
               "mrx_gated_scan_fwd");
     }
@@ -1559,9 +1559,8 @@ std::tuple<Tensor, Tensor, Tensor> gated_scan(const Tensor &z, const Tensor &x, 
         auto node = record(GatedScanOp{done, log_state.scalar_type()}, z, x, gate, log_state);
         torch::autograd::set_history(y, node);
         torch::autograd::set_history(ls_out, node);
-        const Tensor *kept[] = {&z_, &x_, &g_, &h, &ls};
-        for (int i = 0; i < 5; ++i) node->keep(i, *kept[i]);
-        node->keep(5, ls_out, true);
+        const Tensor *kept[] = {&z_, &x_, &g_, &h, &ends};
+        for (int i = 0; i < GatedScanOp::SAVED; ++i) node->keep(i, *kept[i]);
     }
     return {y, ls_out, ld_out};
 }

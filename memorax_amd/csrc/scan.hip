@@ -279,9 +279,12 @@ constexpr int MAX_SEGMENTS = 64;
 // element of bfloat16 arrays instead of eight, besides the scan's own), backward dh is neither written nor read, nor h a second time (sixteen instead
 // of twenty-two), and four launches over the carries.  1024 x 128 x 256 bfloat16, us, the launches it stands for / one: forward 43 + 31
 // + 4 x 4.7 / 77, backward 76 + 55 / 105.
+// The backward reads the states before the first step and behind the last one (first, last: (B,D)) as the forward leaves them for it, not the carries
+// in the caller's hands: those may be overwritten meanwhile, and a state is not what comes back from its logarithm.
 template <typename S> struct Gate {
     const S *gate;
     S *y, *dgate;
+    float *first, *last;
 };
 template <typename S, int VEC> __device__ __forceinline__ Vec<float, VEC> gated(const Vec<float, VEC> &h, const raw_t<S, VEC> &gate)
 {
@@ -308,6 +311,17 @@ template <typename E, int VEC, typename F> __device__ __forceinline__ Vec<E, VEC
 {
 #pragma unroll
     for (int i = 0; i < VEC; ++i) x.v[i] = f(x.v[i]);
+    return x;
+}
+// the gradient of the last state, of its logarithm's (LOG)
+template <bool LOG, typename E, int VEC> __device__ __forceinline__ Vec<E, VEC> carry_grad(const E *g, [[maybe_unused]] const float *last, int64_t at)
+{
+    Vec<E, VEC> x = ldc<E, VEC>(g + at);
+    if constexpr (LOG) {
+        const Vec<E, VEC> h = ldc<E, VEC>(last + at);
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) x.v[i] /= h.v[i];
+    }
     return x;
 }
 template <bool LOG, typename E, int VEC> __device__ __forceinline__ Vec<E, VEC> carry_in(const E *p)
@@ -360,6 +374,8 @@ diag_scan_fwd_kernel(const S *__restrict__ a, const S *__restrict__ b,
     V carry_h = vfill<E, VEC>(O::zero()), carry_p = vfill<E, VEC>(O::one());
     if (act && SEG != SUMMARISE) {
         if (h0) carry_h = carry_in<GATE, E, VEC>(h0 + bi * D + col);
+        if constexpr (GATE)
+            if (gt.first && w == 0) stc<E, VEC>(gt.first + bi * D + col, carry_h);
         if (P0) carry_p = carry_in<GATE, E, VEC>(P0 + bi * D + col);
     }
 
@@ -545,6 +561,8 @@ diag_scan_fwd_kernel(const S *__restrict__ a, const S *__restrict__ b,
     }
     if (w == 0 && act && t_end == T) {
         if (h_last) carry_out<GATE, E, VEC>(h_last + bi * D + col, carry_h);
+        if constexpr (GATE)
+            if (gt.last) stc<E, VEC>(gt.last + bi * D + col, carry_h);
         if (P_last) carry_out<GATE, E, VEC>(P_last + bi * D + col, carry_p);
     }
 }
@@ -586,7 +604,7 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
     constexpr bool ONCE = GATE;   // z_{t+1} of a step is the z_t of the one before: read once
 
     V carry = vfill<E, VEC>(O::zero());  // lam_{t+1} entering from the right
-    if (act && g_last && SEG != SUMMARISE) carry = ldc<E, VEC>(g_last + bi * D + col);
+    if (act && g_last && SEG != SUMMARISE) carry = carry_grad<GATE, E, VEC>(g_last, gt.last, bi * D + col);
     // da_sum (time-invariant a): da is (B,D), the sum of the per-step terms over the sequence -- what the
     // gradient of a broadcast coefficient needs -- kept in registers instead of written per step
     V dsum = vfill<E, VEC>(O::zero());
@@ -614,7 +632,7 @@ diag_scan_bwd_kernel(const S *__restrict__ a, const S *__restrict__ hx, const S 
         buf = 1;
     }
     [[maybe_unused]] V h0v = vfill<E, VEC>(O::zero());   // h_{-1}: what step 0 multiplies its lam with
-    if (SEG != SUMMARISE && h0) h0v = carry_in<GATE, E, VEC>(h0 + bi * D + col);
+    if (SEG != SUMMARISE && h0) h0v = ldc<E, VEC>(h0 + bi * D + col);
     [[maybe_unused]] V p_all;                            // a broadcast coefficient
     if constexpr (ATI) {
         p_all = ldv<S, E, VEC>(a + col);
@@ -912,6 +930,8 @@ diag_scan_fwd_stream_kernel(const S *__restrict__ a, const S *__restrict__ b,
     const int64_t row0 = bi * T;
     V ch = vfill<E, VEC>(O::zero()), cp = vfill<E, VEC>(O::one());
     if (h0) ch = carry_in<GATE, E, VEC>(h0 + bi * D + col);
+    if constexpr (GATE)
+        if (gt.first) stc<E, VEC>(gt.first + bi * D + col, ch);
     if (P0) cp = carry_in<GATE, E, VEC>(P0 + bi * D + col);
 
     using R = raw_t<S, VEC>;  // prefetched values stay as stored until they are consumed
@@ -962,6 +982,8 @@ diag_scan_fwd_stream_kernel(const S *__restrict__ a, const S *__restrict__ b,
             for (int s = 0; s < SG; ++s) xg[s] = ng[s];
     }
     if (h_last) carry_out<GATE, E, VEC>(h_last + bi * D + col, ch);
+    if constexpr (GATE)
+        if (gt.last) stc<E, VEC>(gt.last + bi * D + col, ch);
     if (P_last) carry_out<GATE, E, VEC>(P_last + bi * D + col, cp);
 }
 
@@ -1050,7 +1072,7 @@ diag_scan_bwd_stream_kernel(const S *__restrict__ a, const S *__restrict__ hx, c
     const int64_t row0 = bi * T;
     V dsum = vfill<E, VEC>(O::zero());  // da_sum: the per-step terms summed over the sequence, da is (B,D)
     V lam = vfill<E, VEC>(O::zero());  // conj(abar_{t+1}) lam_{t+1} entering step t
-    if (g_last) lam = ldc<E, VEC>(g_last + bi * D + col);
+    if (g_last) lam = carry_grad<GATE, E, VEC>(g_last, gt.last, bi * D + col);
 
     // step r (reversed index), t = T-1-r: needs g_t, a_t (for the carry to t-1), h_{t-1}, done_t
     using R = raw_t<S, VEC>;  // prefetched values stay as stored until they are consumed
@@ -1060,7 +1082,7 @@ diag_scan_bwd_stream_kernel(const S *__restrict__ a, const S *__restrict__ hx, c
     R xx[MG ? SG : 1], nx[MG ? SG : 1];
     uint32_t xd[SG], nd[SG];
     V h0v = vfill<E, VEC>(O::zero());  // h_{-1}: what step 0 multiplies its lam with
-    if (h0) h0v = carry_in<GATE, E, VEC>(h0 + bi * D + col);
+    if (h0) h0v = ldc<E, VEC>(h0 + bi * D + col);
     [[maybe_unused]] R xq[GATE ? SG : 1], nq[GATE ? SG : 1];   // gates
     [[maybe_unused]] V top;                                    // the state of the step at hand
     if constexpr (GATE && !RECOMP) top = ldv<S, E, VEC>(hfw + (row0 + T - 1) * D + col);
@@ -1831,7 +1853,7 @@ extern "C" int mrx_linear_scan_last(void *stream, const void *a, const void *b, 
 
 namespace {
 
-int mingru_scan_fwd(void *stream, const void *gate, void *y, const void *z, const void *h_tilde, const void *done, const void *h0, const void *P0, void *h, void
+int mingru_scan_fwd(void *stream, const void *gate, void *y, float *ends, const void *z, const void *h_tilde, const void *done, const void *h0, const void *P0, void *h, void
                     *h_last, void *P_last, int64_t B, int64_t T, int64_t D, int dtype, int done_dtype, void *workspace)
 {
     if (!z || !h_tilde || !done || !h) return MRX_ERR_INVALID_ARG;
@@ -1842,12 +1864,13 @@ int mingru_scan_fwd(void *stream, const void *gate, void *y, const void *z, cons
     const size_t ea = dtype == MRX_BF16 ? 2 : 4;  // z, h~, h in `dtype`; the carries in float32
     for (const void *p : {z, h_tilde, (const void *)h, gate, (const void *)y})
         if (!aligned(p, ea)) return MRX_ERR_INVALID_ARG;
-    for (const void *p : {h0, P0, (const void *)h_last, (const void *)P_last})
+    for (const void *p : {h0, P0, (const void *)h_last, (const void *)P_last, (const void *)ends})
         if (!aligned(p, 4)) return MRX_ERR_INVALID_ARG;
+    float *const last = ends ? ends + B * D : nullptr;
     if (dtype == MRX_BF16)
-        return launch_fwd<float, true, __bf16>((hipStream_t)stream, {(const __bf16 *)gate, (__bf16 *)y, nullptr}, z, h_tilde, done, done_dtype, h0, P0, h, h_last,
-                                               P_last, B, T, D, 0, workspace);
-    return launch_fwd<float, true>((hipStream_t)stream, {(const float *)gate, (float *)y, nullptr}, z, h_tilde, done, done_dtype, h0, P0, h, h_last, P_last, B, T,
+        return launch_fwd<float, true, __bf16>((hipStream_t)stream, {(const __bf16 *)gate, (__bf16 *)y, nullptr, ends, last}, z, h_tilde, done, done_dtype, h0, P0, h,
+                                               h_last, P_last, B, T, D, 0, workspace);
+    return launch_fwd<float, true>((hipStream_t)stream, {(const float *)gate, (float *)y, nullptr, ends, last}, z, h_tilde, done, done_dtype, h0, P0, h, h_last, P_last, B, T,
                                    D, 0, workspace);
 }
 
@@ -1856,7 +1879,7 @@ int mingru_scan_fwd(void *stream, const void *gate, void *y, const void *z, cons
 extern "C" int mrx_mingru_scan_fwd(void *stream, const void *z, const void *h_tilde, const void *done, const void *h0, const void *P0,
                                    void *h, void *h_last, void *P_last, int64_t B, int64_t T, int64_t D, int dtype, int done_dtype)
 {
-    return mingru_scan_fwd(stream, nullptr, nullptr, z, h_tilde, done, h0, P0, h, h_last, P_last, B, T, D, dtype, done_dtype, nullptr);
+    return mingru_scan_fwd(stream, nullptr, nullptr, nullptr, z, h_tilde, done, h0, P0, h, h_last, P_last, B, T, D, dtype, done_dtype, nullptr);
 }
 
 extern "C" int mrx_mingru_scan_fwd_segmented(void *stream, const void *z, const void *h_tilde, const void *done, const void *h0, const
@@ -1864,12 +1887,12 @@ extern "C" int mrx_mingru_scan_fwd_segmented(void *stream, const void *z, const 
                                              int done_dtype, void *workspace)
 {
     if (!aligned(workspace, 8)) return MRX_ERR_INVALID_ARG;
-    return mingru_scan_fwd(stream, nullptr, nullptr, z, h_tilde, done, h0, P0, h, h_last, P_last, B, T, D, dtype, done_dtype, workspace);
+    return mingru_scan_fwd(stream, nullptr, nullptr, nullptr, z, h_tilde, done, h0, P0, h, h_last, P_last, B, T, D, dtype, done_dtype, workspace);
 }
 
 namespace {
 
-int mingru_scan_bwd(void *stream, const void *gate, void *dgate, const void *z, const void *h_tilde, const void *h, const void *done, const void *h0, const void *g,
+int mingru_scan_bwd(void *stream, const void *gate, void *dgate, const float *ends, const void *z, const void *h_tilde, const void *h, const void *done, const void *h0, const void *g,
                     const void *g_last, void *dz, void *dh_tilde, void *dh0, int64_t B, int64_t T, int64_t D, int dtype, int done_dtype,
                     void *workspace)
 {
@@ -1881,12 +1904,13 @@ int mingru_scan_bwd(void *stream, const void *gate, void *dgate, const void *z, 
     const size_t ea = dtype == MRX_BF16 ? 2 : 4;  // z, h~, h, g, dz, dh~ in `dtype`; the carries in float32
     for (const void *p : {z, h_tilde, h, g, (const void *)dz, (const void *)dh_tilde, gate, (const void *)dgate})
         if (!aligned(p, ea)) return MRX_ERR_INVALID_ARG;
-    for (const void *p : {h0, g_last, (const void *)dh0})
+    for (const void *p : {h0, g_last, (const void *)dh0, (const void *)ends})
         if (!aligned(p, 4)) return MRX_ERR_INVALID_ARG;
+    float *const last = ends ? const_cast<float *>(ends) + B * D : nullptr;   // (read only)
     if (dtype == MRX_BF16)
-        return launch_bwd<float, true, __bf16>((hipStream_t)stream, {(const __bf16 *)gate, nullptr, (__bf16 *)dgate}, z, h_tilde, h, done, done_dtype, h0, g, g_last, dz,
+        return launch_bwd<float, true, __bf16>((hipStream_t)stream, {(const __bf16 *)gate, nullptr, (__bf16 *)dgate, nullptr, last}, z, h_tilde, h, done, done_dtype, h0, g, g_last, dz,
                                                dh_tilde, dh0, B, T, D, 0, 0, workspace);
-    return launch_bwd<float, true>((hipStream_t)stream, {(const float *)gate, nullptr, (float *)dgate}, z, h_tilde, h, done, done_dtype, h0, g, g_last, dz, dh_tilde,
+    return launch_bwd<float, true>((hipStream_t)stream, {(const float *)gate, nullptr, (float *)dgate, nullptr, last}, z, h_tilde, h, done, done_dtype, h0, g, g_last, dz, dh_tilde,
                                    dh0, B, T, D, 0, 0, workspace);
 }
 
@@ -1896,7 +1920,7 @@ extern "C" int mrx_mingru_scan_bwd(void *stream, const void *z, const void *h_ti
                                    const void *g, const void *g_last, void *dz, void *dh_tilde, void *dh0, int64_t B, int64_t T, int64_t
                                    D, int dtype, int done_dtype)
 {
-    return mingru_scan_bwd(stream, nullptr, nullptr, z, h_tilde, h, done, h0, g, g_last, dz, dh_tilde, dh0, B, T, D, dtype, done_dtype, nullptr);
+    return mingru_scan_bwd(stream, nullptr, nullptr, nullptr, z, h_tilde, h, done, h0, g, g_last, dz, dh_tilde, dh0, B, T, D, dtype, done_dtype, nullptr);
 }
 
 extern "C" int mrx_mingru_scan_bwd_segmented(void *stream, const void *z, const void *h_tilde, const void *h, const void *done, const void
@@ -1904,23 +1928,23 @@ extern "C" int mrx_mingru_scan_bwd_segmented(void *stream, const void *z, const 
                                              int64_t T, int64_t D, int dtype, int done_dtype, void *workspace)
 {
     if (!aligned(workspace, 8)) return MRX_ERR_INVALID_ARG;
-    return mingru_scan_bwd(stream, nullptr, nullptr, z, h_tilde, h, done, h0, g, g_last, dz, dh_tilde, dh0, B, T, D, dtype, done_dtype, workspace);
+    return mingru_scan_bwd(stream, nullptr, nullptr, nullptr, z, h_tilde, h, done, h0, g, g_last, dz, dh_tilde, dh0, B, T, D, dtype, done_dtype, workspace);
 }
 
 extern "C" int mrx_gated_scan_fwd(void *stream, const void *z, const void *h_tilde, const void *gate, const void *done, const float *log_state,
-                                  const float *log_decay, void *h, void *y, float *log_state_out, float *log_decay_out, int64_t B, int64_t T, int64_t D,
-                                  int dtype, int done_dtype)
+                                  const float *log_decay, void *h, void *y, float *log_state_out, float *log_decay_out, float *ends, int64_t B, int64_t T,
+                                  int64_t D, int dtype, int done_dtype)
 {
     if (!gate || !y) return MRX_ERR_INVALID_ARG;
-    return mingru_scan_fwd(stream, gate, y, z, h_tilde, done, log_state, log_decay, h, log_state_out, log_decay_out, B, T, D, dtype, done_dtype, nullptr);
+    return mingru_scan_fwd(stream, gate, y, ends, z, h_tilde, done, log_state, log_decay, h, log_state_out, log_decay_out, B, T, D, dtype, done_dtype, nullptr);
 }
 
 extern "C" int mrx_gated_scan_bwd(void *stream, const void *z, const void *h_tilde, const void *gate, const void *h, const void *done,
-                                  const float *log_state, const void *dy, const float *g_last, void *dz, void *dh_tilde, void *dgate,
+                                  const float *ends, const void *dy, const float *g_last, void *dz, void *dh_tilde, void *dgate,
                                   float *dlog_state, int64_t B, int64_t T, int64_t D, int dtype, int done_dtype)
 {
-    if (!gate || !dgate) return MRX_ERR_INVALID_ARG;
-    return mingru_scan_bwd(stream, gate, dgate, z, h_tilde, h, done, log_state, dy, g_last, dz, dh_tilde, dlog_state, B, T, D, dtype, done_dtype, nullptr);
+    if (!gate || !dgate || !ends) return MRX_ERR_INVALID_ARG;
+    return mingru_scan_bwd(stream, gate, dgate, ends, z, h_tilde, h, done, ends, dy, g_last, dz, dh_tilde, dlog_state, B, T, D, dtype, done_dtype, nullptr);
 }
 
 namespace {

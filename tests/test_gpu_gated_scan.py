@@ -52,6 +52,51 @@ def test_gated_scan_equals_its_operations(B, T, D, dt):
             assert relerr(a, _np(b)) <= 2 * tol
 
 
+def _operations(z, x, gate, done, ls, ld):
+    from memorax_amd import functional as Fn
+    h, hl, Pl = Fn.mingru_scan(z, x, done, ls.exp()[:, 0], ld.exp()[:, 0])
+    return Fn.silu_gate(h, gate), hl[:, None].log(), Pl[:, None].log()
+
+
+@pytest.mark.parametrize("B,T,D", [(3, 5, 7), (300, 40, 256), (1100, 33, 130)])   # wave-split, and whole rows streaming
+def test_carries_overwritten_between_the_passes(B, T, D):
+    """A program that keeps its carry in one buffer writes the next one over it, or clears what it was handed, before the backward."""
+    from memorax_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(D)
+    z, x, gate = (torch.randn(B, T, D, device="cuda", generator=g).requires_grad_() for _ in range(3))
+    ls, ld = torch.randn(B, 1, D, device="cuda", generator=g), torch.zeros(B, 1, D, device="cuda")
+    done, dy, dl = torch.rand(B, T, device="cuda", generator=g) < 0.1, torch.randn(B, T, D, device="cuda", generator=g), torch.randn(B, 1, D, device="cuda", generator=g)
+    want = torch.autograd.grad(_operations(z, x, gate, done, ls.clone(), ld)[:2], (z, x, gate), (dy, dl))
+    print(f"case gated scan overwritten {B} {T} {D}", flush=True)
+    y, s, d = _lib.native().gated_scan(z, x, gate, done, ls, ld)
+    ls.copy_(s.detach())
+    ld.copy_(d)
+    s.detach().zero_()
+    for a, b in zip(torch.autograd.grad((y, s), (z, x, gate), (dy, dl)), want):
+        assert relerr(a, _np(b)) <= 2e-5   # as above
+
+
+def test_gradient_of_the_carry_handed_on():
+    """d log h_T / d log h_0 is h_0 / h_T to within a division's and two products' roundings, however far the logarithm is from zero: with every gate shut it is 1."""
+    from memorax_amd import _lib
+    B, T, D = 40, 3, 96
+    ls = torch.rand(B, 1, D, device="cuda") * 160 - 80
+    ls.requires_grad_()
+    z, x, gate = torch.full((B, T, D), -200.0, device="cuda"), torch.randn(B, T, D, device="cuda"), torch.randn(B, T, D, device="cuda")
+    _, s, _ = _lib.native().gated_scan(z, x, gate, torch.zeros(B, T, dtype=torch.bool, device="cuda"), ls, torch.zeros(B, 1, D, device="cuda"))
+    (got,) = torch.autograd.grad(s.sum(), ls)
+    assert (got - 1).abs().max() <= 3 * 2.0 ** -24
+
+
+def test_a_carry_of_several_steps_gives_its_first():
+    from memorax_amd import _lib
+    z, x, gate = (torch.randn(6, 9, 40, device="cuda").requires_grad_() for _ in range(3))
+    ls, ld, done = torch.randn(6, 2, 40, device="cuda"), -torch.rand(6, 2, 40, device="cuda"), torch.rand(6, 9, device="cuda") < 0.2
+    got, want = _lib.native().gated_scan(z, x, gate, done, ls, ld), _operations(z, x, gate, done, ls, ld)
+    for a, b in zip(got, want):
+        assert a.shape == b.shape and relerr(a, _np(b)) <= 1e-5
+
+
 def test_cells_of_their_own_keep_their_scan():
     from memorax_amd import sequence_models as sm
     seen = []
