@@ -5,17 +5,17 @@
 //     z, h~, gate = norm(x') W^T -> MinGRU step -> gated state  (a gated recurrence: mrx_gated_recurrence_act)
 //
 // Few rows, one per environment.  A workgroup of eight waves owns 16 rows and 64 (gated: of each of its three layers) or 256 columns of
-// the opening layers, and computes the closing layer for its rows whole: what that costs is reading W_c once more for each of the
-// (mostly four) workgroups of a row tile.  Bound by its trips to memory -- a matrix state's traffic has pushed the weights out of L2 -- and
+// the opening layers, and computes the closing layer for its rows whole: what that costs is reading W_c once more for each
+// workgroup of a row tile.  Bound by its trips to memory -- a matrix state's traffic has pushed the weights out of L2 -- and
 // by the 64 bytes a clock that a compute unit takes in.  So the rows and the weights of either product are requested in the order
 // they are needed and go to LDS without passing through registers, in steps through slots of each wave's own: 128 bytes of k of the wave's
 // 16 (up to 3) weight rows, fetched as whole lines of eight lanes (read as the matrix instruction wants them, 16 lanes on 16 lines, 128 KB take
 // 2.9 us instead of 1.0).  Only the wave that requested a slot reads it, after a wait of its own; the workgroup meets at the barriers of the norms.
 //
-// In a graph behind a matrix state's step (134 MB), 256 features, bfloat16 (us; closing layer in a launch of its own + opening / one launch):
-//     gated recurrence     32 rows 5.5 + 8.2 / 12.5, 1024 5.7 + 8.8 / 13.2, 2048 9.0 + 18.7 / 27.4 (before: 5.5 + 10.0, 5.7 + 10.9, 9.0 + 18.9)
-//     q, k, v and beta     32 rows 5.5 + 6.0 / 11.6, 1024 5.7 + 9.1 / 12.0, 2048 9.0 + 12.0 / 21.2
-// More rows than a workgroup for each compute unit takes are better off apart: the callers' rule.
+// In a graph behind 512 MB of other traffic, 256 features, bfloat16 (us; the closing layer in a launch of its own and then the opening / one launch):
+//     gated recurrence     32 rows 12.2 / 11.8, 1024 14.2 / 13.8, 2048 18.4 / 19.3
+//     q, k, v and beta     32 rows 9.4 / 10.7, 1024 14.0 / 11.8, 2048 18.1 / 16.2
+// Which of the two is the callers' rule (host_ops.cpp, chain_pays).
 // (A matrix state's projections and its step in one launch, the states on their way meanwhile, gain nothing: whole rows of states are 256 KB a
 // workgroup, one workgroup a compute unit, and the slowest of them ends 40 % after the mean: 31 us, as two launches 31; few rows 9.2 / 7.7.)
 //
@@ -36,7 +36,7 @@ constexpr int AC_PIECE = 16 * 128;            // bytes: 128 of k of 16 weight ro
 constexpr int AC_REGION = 8 * AC_PIECE;       // of a wave's steps on their way, at most
 constexpr int AC_MOST_X = 256;                // features of x' behind a closing layer
 constexpr int AC_MOST_K = 512;                // features of a normalised row
-constexpr int AC_MOST_LDS = 160 * 1024;
+constexpr int AC_MOST_LDS = 160 * 1024, AC_UNITS = 256;
 
 // Where things lie in LDS.
 struct ChainLds {
@@ -186,7 +186,7 @@ template <typename T, bool WBF, int CT> struct WeightStream {
     {
         return SHARED ? i / BLOCK * (2 * BLOCK) + half * BLOCK + i % BLOCK : i;
     }
-    template <bool SHARED> static __device__ __forceinline__ int steps_of(int K, int half)
+    template <bool SHARED> static __host__ __device__ __forceinline__ int steps_of(int K, int half)
     {
         const int all = (K + KPIECE - 1) / KPIECE, pairs = all / (2 * BLOCK), rest = all - pairs * 2 * BLOCK - half * BLOCK;
         return SHARED ? pairs * BLOCK + (rest < 0 ? 0 : rest < BLOCK ? rest : BLOCK) : all;
@@ -506,9 +506,21 @@ template <typename T, bool WBF, bool GATED> int launch_chain(hipStream_t st, Cha
     if (grid >= (1ll << 31)) return MRX_ERR_INVALID_ARG;
     auto go = [&](auto ct1) -> int {
         constexpr int CT1 = decltype(ct1)::value, CT2 = GATED ? 3 : 2;
-        int region = AC_REGION;
+        // No more than the steps there are; and room for a second workgroup on the compute unit where there are workgroups for it and the rows leave it: with
+        // one of 160 KB a grid of more than the compute units loses to smaller workgroups.  A gated recurrence alone, bfloat16, us, four waves with
+        // their weights in registers / one workgroup a unit / two: 256 features and columns 4096 rows 24.7 / 26.4 / 20.2, 16 384 74 / 90 / 62; 256 by 1024 columns
+        // 2048 rows 41 / 48 / 34; float32 128 by 256 columns 8192 rows 49 / 56 / 41.  (Rows of 320 to 500 features leave none: 384, 8192 rows 79 / 82.)
+        using Closing = WeightStream<T, WBF, CT1 ? CT1 : 1>;
+        using Opening = WeightStream<T, WBF, CT2>;
+        const int need1 = CT1 * Closing::template steps_of<false>(a.in.K, 0), need2 = CT2 * Opening::template steps_of<GATED>(a.F, 0), need = need1 > need2 ? need1 : need2;
+        int region = need * AC_PIECE < AC_REGION ? need * AC_PIECE : AC_REGION;
         while (region > 0 && !lay_out(a, closing, CT1, CT2, sizeof(T), region)) region -= AC_PIECE;
         if (region <= 0) return MRX_ERR_UNSUPPORTED;
+        if (grid > AC_UNITS) {
+            int less = region;
+            while (less > 0 && !(lay_out(a, closing, CT1, CT2, sizeof(T), less) && a.at.bytes <= AC_MOST_LDS / 2)) less -= AC_PIECE;
+            if (less <= 0) lay_out(a, closing, CT1, CT2, sizeof(T), region);
+        }
         return launch_kernel(ChainKernel<T, WBF, CT1, GATED>::get(), dim3((unsigned)grid), dim3(AC_THREADS), a.at.bytes, st, a);
     };
     if constexpr (GATED)

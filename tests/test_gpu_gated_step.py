@@ -15,6 +15,7 @@ def _np(t):
 
 
 @pytest.mark.parametrize("rows,K,N", [(1, 8, 8), (15, 24, 56), (16, 256, 64), (17, 264, 72), (33, 512, 200), (130, 136, 256),
+                                      (4112, 72, 64), (1040, 128, 256), (1040, 512, 264),   # more workgroups than compute units, two on each and one
                                       (5, 520, 64)])   # the last: past its features
 @pytest.mark.parametrize("wd,product", [(F32, F32), (F32, BF), (BF, BF)])
 @pytest.mark.parametrize("norm,bias", [(0, False), (1, False), (2, False), (1, True)])
