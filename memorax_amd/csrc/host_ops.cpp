@@ -2772,8 +2772,29 @@ bool act_block(ActBlock &k, const Tensor &x, const py::tuple &spec, const py::tu
            k.D <= 64 && k.D % (k.dtype == at::kBFloat16 ? 8 : 4) == 0;
 }
 
-// Rows from which on a closing layer is a launch of its own: sixteen rows and (mostly) four workgroups for them, one to a compute unit (act_chain.hip).
-constexpr int64_t CHAINED_ROWS = 1024;
+// Whether the closing layer (K -> F) in the launch of what it opens -- layers of n columns, or a gated recurrence's -- takes less time than before it.  Each
+// workgroup of the opening (act_chain.hip: 16 rows and 256 or, gated, 64 columns of three layers) forms the closing layer for its rows again, at the price of reading all
+// of its weights; what is saved is a launch and a trip to memory.  Behind 512 MB of other traffic, us, apart / as one, weights and products in bfloat16 unless said:
+//     beyond a workgroup for each compute unit      qkv 512 wide 64 features 2048 rows 20.8 / 21.3, gated 512 wide 1024 rows 17.2 / 21.2, 1024 wide 23.6 / 37.7
+//     gated recurrences, by the bytes of weights a workgroup reads
+//                                                   256 wide 256 features 32 rows 12.2 / 11.8, weights in float32 (448 KB) 15.2 / 15.3, 512 wide (704 KB) 17.9 / 19.3;
+//                                                   float32 products 512 wide 128 features (352 KB) 19.4 / 18.8, 256 wide 256 features (448 KB) 16.4 / 18.2
+//     other layers, half the compute units at work  256 wide 256 features 1024 rows 14.0 / 11.8, weights in float32 512 wide 512 rows (768 KB) 18.5 / 18.2;
+//                                                   float32 products 512 wide 128 features 512 rows (384 KB) 19.0 / 17.5, 256 wide 256 features 1024 rows (512 KB) 19.5 / 20.5
+//     fewer: apart, the closing layer has more workgroups than rows fill here, and its weights come in by all of them
+//                                                   256 wide 256 features 32 rows 9.4 / 10.7, 128 features 9.2 / 7.4, 64 wide 256 features 8.9 / 8.7;
+//                                                   float32 products 64 wide 128 features 9.1 / 9.9, 256 wide 64 features 10.8 / 10.2
+bool chain_pays(int64_t B, int64_t F, int64_t K, IntArrayRef n, bool gated, int64_t weight_bytes, bool bf16, int64_t units)
+{
+    int64_t columns = 0;
+    for (const int64_t c : n) columns += (c + 15) / 16 * 16;
+    const int64_t groups = gated ? (n[0] + 63) / 64 : (columns + 255) / 256, wgs = (B + 15) / 16 * groups;
+    if (wgs > units) return false;
+    const int64_t read = weight_bytes * F * (K + (gated ? 192 : std::min<int64_t>(columns, 256)));
+    if (gated) return read <= (bf16 ? 448 : 352) << 10;
+    if (2 * wgs >= units) return read <= (bf16 ? 768 : 384) << 10;
+    return F <= (bf16 ? 128 : 64) || (bf16 && groups == 1);
+}
 
 void run_act(const Tensor &x0, std::vector<ActBlock> &blocks, const Done &done, ScalarType product, bool in_place, Tensor &y)
 {
@@ -2810,10 +2831,13 @@ void run_act(const Tensor &x0, std::vector<ActBlock> &blocks, const Done &done, 
         pending.any = false;
     };
     // opens a block on what the pending closing layer leaves, in one launch if that pays and is taken
-    auto open = [&](int wd, auto chained, auto alone) {
+    const int64_t units = compute_units(x0);
+    auto open = [&](const ActBlock &k, int wd, auto chained, auto alone) {
         if (pending.any) {
             x = pending.c.out;
-            if (B <= CHAINED_ROWS && F <= 256 && pending.wd == wd) {
+            if (F <= 256 && pending.wd == wd &&
+                chain_pays(B, F, pending.c.K, IntArrayRef(k.n).slice(0, k.n.size() - 1), k.kind == ActBlock::GATED, wd == MRX_F32 ? 4 : 2, product == at::kBFloat16,
+                           units)) {
                 const int rc = chained(&pending.c);
                 if (rc != MRX_ERR_UNSUPPORTED) {
                     check(rc, "mrx_closing");
@@ -2847,7 +2871,7 @@ void run_act(const Tensor &x0, std::vector<ActBlock> &blocks, const Done &done, 
                                                            done.p(), fptr(k.carry[0]), fptr(k.carry[1]), ptr(k.z), rows, fptr(k.next[0]), fptr(k.next[1]), B, F,
                                                            k.N, wd, pc, done.dtype, (float)k.eps);
             };
-            open(wd, launch, [&] { check(launch(nullptr), "mrx_closed_gated_recurrence_act"); });
+            open(k, wd, launch, [&] { check(launch(nullptr), "mrx_closed_gated_recurrence_act"); });
         } else {
             std::array<const void *, MRX_ROW_DENSE_LAYERS> w{}, b{};
             std::array<void *, MRX_ROW_DENSE_LAYERS> u{};
@@ -2856,7 +2880,7 @@ void run_act(const Tensor &x0, std::vector<ActBlock> &blocks, const Done &done, 
                 w[l] = ptr(k.w[l]), b[l] = ptr(k.b[l]), u[l] = take(B * k.n[l], k.dtype);
                 if (k.b[l].defined()) bd = code(k.b[l].scalar_type());
             }
-            open(wd, [&](const mrx_closing *c) {
+            open(k, wd, [&](const mrx_closing *c) {
                 return lib.mrx_closed_row_dense(st, c, fptr(k.scale), fptr(k.nbias), k.norm, w.data(), b.data(), u.data(), k.n.data(), (int)last, B, F, wd, bd,
                                                 code(k.dtype), pc, (float)k.eps);
             }, [&] {

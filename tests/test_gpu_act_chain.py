@@ -35,7 +35,8 @@ def _leaves(t):
 
 
 @pytest.mark.parametrize("kinds", [("delta", "gated", "delta", "gated"), ("linear", "linear", "wide"), ("gated", "lru", "delta"), ("wide", "gated")])
-@pytest.mark.parametrize("B,F,H,d", [(1, 8, 1, 8), (17, 64, 2, 16), (33, 72, 2, 24), (130, 136, 3, 40), (1024, 256, 4, 64), (1030, 256, 8, 64), (16, 264, 2, 32)])
+@pytest.mark.parametrize("B,F,H,d", [(1, 8, 1, 8), (17, 64, 2, 16), (33, 72, 2, 24), (130, 136, 3, 40), (1024, 256, 4, 64), (1030, 256, 8, 64), (16, 264, 2, 32),
+                                     (4096, 64, 2, 16), (4097, 64, 2, 16)])   # a workgroup for each compute unit, and one more
 @pytest.mark.parametrize("rms,autocast", [(True, True), (False, True), (True, False)])
 def test_stack_acts_as_its_blocks(kinds, B, F, H, d, rms, autocast):
     from memorax_amd import sequence_models as sm
