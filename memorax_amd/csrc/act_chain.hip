@@ -542,7 +542,8 @@ int chain_input(ChainArgs &a, const mrx_closing *c, const float *x, const float 
 {
     if (!known(w_dtype) || !known(product_dtype) || norm < 0 || norm > 2 || rows <= 0 || rows >= (1ll << 31) || K <= 0) return MRX_ERR_INVALID_ARG;
     if (!aligned(scale, 16) || !aligned(norm_bias, 16)) return MRX_ERR_INVALID_ARG;
-    if (K % 8 != 0 || K > AC_MOST_K || (product_dtype == MRX_F32 && w_dtype != MRX_F32)) return MRX_ERR_UNSUPPORTED;
+    if (K > AC_MOST_K || (product_dtype == MRX_F32 && w_dtype != MRX_F32)) return MRX_ERR_UNSUPPORTED;
+    if (K % 8 != 0) return MRX_ERR_INVALID_ARG;
     a.F = (int)K, a.inv_F = 1.f / (float)K, a.eps = eps, a.norm = norm;
     if (!c) {
         if (!x || !aligned(x, 16)) return MRX_ERR_INVALID_ARG;
