@@ -742,7 +742,7 @@ typedef struct mrx_closing {
     const float *scale;      /* (K) or NULL */
     const void *weight, *bias;   /* (n, K); (n) in bias_dtype, or NULL */
     const float *residual;   /* (rows, n) */
-    float *out;              /* (rows, n), not the residual's memory */
+    float *out;              /* (rows, n), no memory of rows or residual (an invalid argument) */
     int64_t K;
     int norm, round_norm, row_dtype, bias_dtype;
     float eps;

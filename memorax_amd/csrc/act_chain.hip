@@ -554,7 +554,14 @@ int chain_input(ChainArgs &a, const mrx_closing *c, const float *x, const float 
     const void *arrays[] = {c->rows, c->scale, c->weight, c->bias, c->residual, c->out};
     for (const void *p : arrays)
         if (!aligned(p, 16)) return MRX_ERR_INVALID_ARG;
-    if (K > AC_MOST_X || c->K % 8 != 0 || c->K > AC_MOST_K) return MRX_ERR_UNSUPPORTED;
+    if (K > AC_MOST_X || c->K > AC_MOST_K) return MRX_ERR_UNSUPPORTED;
+    if (c->K % 8 != 0) return MRX_ERR_INVALID_ARG;
+    // the first workgroup of a row tile writes `out` while the others still read what it comes from
+    auto apart = [&](const void *p, int64_t bytes) {
+        const uintptr_t from = reinterpret_cast<uintptr_t>(p), out = reinterpret_cast<uintptr_t>(c->out);
+        return from + bytes <= out || out + rows * K * 4 <= from;
+    };
+    if (!apart(c->residual, rows * K * 4) || !apart(c->rows, rows * c->K * (c->row_dtype == MRX_BF16 ? 2 : 4))) return MRX_ERR_INVALID_ARG;
     a.in = RowInput{c->rows, c->scale, nullptr, rows, (int)c->K, c->norm ? 1 : 0, c->eps, 1.f / (float)c->K, c->round_norm != 0};
     a.wc = c->weight, a.bc = c->bias, a.residual = c->residual, a.x_out = c->out, a.scale = scale, a.nbias = norm_bias;
     a.x_bf16 = c->row_dtype == MRX_BF16, a.bc_bf16 = c->bias_dtype == MRX_BF16;
