@@ -2915,6 +2915,7 @@ py::tuple stack_act(const Tensor &x, const py::list &specs, const py::tuple &typ
     blocks.reserve(specs.size());
     if (!tracing() && !x.key_set().has(c10::DispatchKey::Python) && !transformed(x) && !transformed(done_) && x.dim() == 3 && x.size(1) == 1 && x.is_cuda() &&
         x.scalar_type() == at::kFloat && x.is_contiguous() && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 && !x._fw_grad(0).defined() &&
+        !done_._fw_grad(0).defined() && !done_.key_set().has(c10::DispatchKey::Python) &&
         (product == at::kFloat || product == at::kBFloat16) && done_.device() == x.device() && done_.dim() == 2 && done_.size(0) == x.size(0) && done_.size(1) == 1)
         for (const auto &spec : specs) {
             blocks.emplace_back();

@@ -89,6 +89,21 @@ def test_an_acting_block_refuses_tangents(cell, dual):
             torch.func.functional_call(block, params, (x, done, carry))
 
 
+@pytest.mark.parametrize("dual", ["input", "flags", "carry"])
+@pytest.mark.parametrize("cell", ["delta", "linear_attention", "recurrence"])
+def test_an_acting_stack_refuses_tangents(cell, dual):
+    block = _block(cell) if cell in CELLS else sm.Residual(sm.PreNorm(sm.GatedLinearRecurrence(64), 64)).cuda()
+    stack = sm.Stack([block, sm.Residual(sm.PreNorm(sm.GatedLinearRecurrence(64), 64)).cuda()])
+    x, done, carry = torch.randn(6, 1, 64, device="cuda"), torch.zeros(6, 1, device="cuda"), stack.initialize_carry(None, (6, 64))
+    make = lambda t: torch.autograd.forward_ad.make_dual(t, torch.ones_like(t))  # noqa: E731
+    with torch.no_grad(), torch.autograd.forward_ad.dual_level():
+        x, done = make(x) if dual == "input" else x, make(done) if dual == "flags" else done
+        if dual == "carry":
+            carry = (carry[0], (make(carry[1][0]), carry[1][1]))
+        with pytest.raises(NotImplementedError, match="forward-mode"):
+            stack(x, done, carry)
+
+
 @pytest.mark.parametrize("cell", ["lru", "mlstm", "recurrence"])
 def test_blocks_wider_than_the_row_kernel_act_on_their_composition(cell):
     Fe = 2056
