@@ -527,6 +527,8 @@ int mrx_mingru_scan_bwd(void *stream, const void *z, const void *h_tilde, const 
  * `dtype`; log_state, log_decay and their successors (B,D) float32.  ends (2,B,D) float32: the states before the first step and behind the last one, left by the
  * forward (nullable) for the backward.  Backward: dy, the gradients of z, h~ and the gate, and (nullable) that of log_state; g_last (nullable): the
  * gradient of log_state's successor. */
+/* mrx_gated_scan_pays: 1 where the library's own rule expects less time of them than of the scan and the gate apart (a question of time, not of coverage) */
+int mrx_gated_scan_pays(int64_t B, int64_t T, int64_t D, int dtype, int backward);
 int mrx_gated_scan_fwd(void *stream, const void *z, const void *h_tilde, const void *gate, const void *done, const float *log_state,
                        const float *log_decay, void *h, void *y, float *log_state_out, float *log_decay_out, float *ends, int64_t B,
                        int64_t T, int64_t D, int dtype, int done_dtype);

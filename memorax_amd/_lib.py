@@ -65,6 +65,7 @@ SIGNATURES = {
     "mrx_deltanet_step": (_I, [_P] * 9 + [_L] * 4 + [_I] * 2),
     "mrx_mingru_step": (_I, [_P] * 10 + [_L] * 2 + [_I] * 2),
     "mrx_row_dense": (_I, [_P] * 4 + [_I] * 2 + [_P] * 4 + [_I, _P] + [_L] * 2 + [_I] * 5 + [ctypes.c_float, _P, _L, _P, _P]),
+    "mrx_gated_scan_pays": (_I, [_L] * 3 + [_I] * 2),
     "mrx_gated_scan_fwd": (_I, [_P] * 12 + [_L] * 3 + [_I] * 2),
     "mrx_gated_scan_bwd": (_I, [_P] * 13 + [_L] * 3 + [_I] * 2),
     "mrx_closed_row_dense": (_I, [_P] * 4 + [_I] + [_P] * 4 + [_I] + [_L] * 2 + [_I] * 4 + [ctypes.c_float]),

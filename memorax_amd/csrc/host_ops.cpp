@@ -42,7 +42,7 @@ using torch::autograd::variable_list;
 // ------------------------------------------------------------------------------------------------ entry points
 #define MRX_BOUND(X)                                                                                                 \
     X(mrx_status_string) X(mrx_chunk_size) X(mrx_delta_chunk_size) X(mrx_scan_workspace) X(mrx_column_sum) X(mrx_linear_scan_fwd_segmented) X(mrx_linear_scan_bwd_segmented)     \
-    X(mrx_linear_scan_last) X(mrx_mingru_scan_fwd_segmented) X(mrx_mingru_scan_bwd_segmented) X(mrx_mlstm_gates_fwd)                     \
+    X(mrx_linear_scan_last) X(mrx_mingru_scan_fwd) X(mrx_mingru_scan_fwd_segmented) X(mrx_mingru_scan_bwd_segmented) X(mrx_mlstm_gates_fwd)                     \
     X(mrx_place_inputs) X(mrx_mlstm_gate_rows_fwd) X(mrx_mlstm_gate_rows_bwd)                                                           \
     X(mrx_mlstm_keys_fwd) X(mrx_mlstm_keys_bwd) X(mrx_mlstm_read_fwd) X(mrx_mlstm_read_bwd)                         \
     X(mrx_mlstm_gates_bwd) X(mrx_rms_norm_fwd) X(mrx_rms_norm_bwd) X(mrx_layer_norm_fwd) X(mrx_layer_norm_bwd)       \
@@ -54,7 +54,7 @@ using torch::autograd::variable_list;
     X(mrx_gated_linear_attn_step) X(mrx_delta_rule_step) X(mrx_causal_conv_silu_fwd) X(mrx_causal_conv_silu_bwd)     \
     X(mrx_mamba_elements_fwd) X(mrx_mamba_elements_bwd) X(mrx_decay_last) X(mrx_mamba_readout_fwd)                   \
     X(mrx_mamba_readout_bwd) X(mrx_deltanet_step) X(mrx_mingru_step) X(mrx_row_dense) X(mrx_dense_grads) X(mrx_dense_grads_workspace)                  \
-    X(mrx_gated_recurrence_act) X(mrx_closed_row_dense) X(mrx_closed_gated_recurrence_act) X(mrx_gated_scan_fwd) X(mrx_gated_scan_bwd)                                                                                       \
+    X(mrx_gated_recurrence_act) X(mrx_closed_row_dense) X(mrx_closed_gated_recurrence_act) X(mrx_gated_scan_pays) X(mrx_gated_scan_fwd) X(mrx_gated_scan_bwd)                                                                                       \
     X(mrx_dense_f32_workspace) X(mrx_dense_f32) X(mrx_dense_f32_input_grad_workspace) X(mrx_dense_f32_input_grad) X(mrx_lru_params_fwd)                       \
     X(mrx_lru_params_bwd) X(mrx_column_product_workspace) X(mrx_column_product) X(mrx_dense_rows_suit) X(mrx_dense_pack) X(mrx_dense_rows) X(mrx_dense_rows_input_grad)                          \
     X(mrx_lru_step) X(mrx_mlstm_step) X(mrx_linear_attn_norm_fwd_chunk_parallel) X(mrx_linear_attn_norm_bwd_chunk_parallel) \
@@ -1512,7 +1512,15 @@ struct GatedScanOp {
         chk(z, "z");
         chk(s[4], "ends", at::kFloat, {2, B, D});
         chk(dy, "dy", z.scalar_type(), z.sizes());
-        const Tensor g_last = as(grads[1], at::kFloat);
+        Tensor g_last = as(grads[1], at::kFloat);
+        if (!lib.mrx_gated_scan_pays(B, T, D, code(z.scalar_type()), true)) {   // the gate's backward, and then the scan's
+            const auto d = silu_gate_bwd(dense16(s[3]), dense16(s[2]), dense16(dy));
+            const Tensor first = s[4].select(0, 0);
+            if (g_last.defined()) g_last = g_last.view({B, D}) / s[4].select(0, 1);
+            auto r = mingru_bwd(z, s[1], s[3], done, first, d[0], some(g_last));
+            return {unless(!node.wants(0), r.da), unless(!node.wants(1), r.db), unless(!node.wants(2), d[1]),
+                    node.wants(3) ? r.dh0.mul_(first).view({B, 1, D}).to(carried) : Tensor()};
+        }
         const Tensor dz = fresh_like(z), dx = fresh_like(z), dg = fresh_like(z), dls = node.wants(3) ? fresh({B, D}, at::kFloat, z) : Tensor();
         const Done flags(done, B, T);
         check(lib.mrx_gated_scan_bwd(stream(), ptr(z), ptr(s[1]), ptr(s[2]), ptr(s[3]), flags.p(), fptr(s[4]), ptr(dy), fptr(g_last), ptr(dz), ptr(dx), ptr(dg),
@@ -1549,11 +1557,24 @@ std::tuple<Tensor, Tensor, Tensor> gated_scan(const Tensor &z, const Tensor &x, 
         chk(ls, "log_state", at::kFloat, {B, D});
         chk(ld, "log_decay", at::kFloat, {B, D});
         const Done flags(done, B, T);
-        h = fresh_like(z_), y = fresh_like(z_), ls_out = fresh({B, 1, D}, at::kFloat, z_), ld_out = fresh({B, 1, D}, at::kFloat, z_);
-        if (need) ends = fresh({2, B, D}, at::kFloat, z_);
-        check(lib.mrx_gated_scan_fwd(stream(), ptr(z_), ptr(x_), ptr(g_), flags.p(), fptr(ls), fptr(ld), ptr(h), ptr(y), fptr(ls_out), fptr(ld_out), fptr(ends), B, T, D,
-                                     code(dt), flags.dtype),
-              "mrx_gated_scan_fwd");
+        h = fresh_like(z_);
+        if (lib.mrx_gated_scan_pays(B, T, D, code(dt), false)) {
+            y = fresh_like(z_), ls_out = fresh({B, 1, D}, at::kFloat, z_), ld_out = fresh({B, 1, D}, at::kFloat, z_);
+            if (need) ends = fresh({2, B, D}, at::kFloat, z_);
+            check(lib.mrx_gated_scan_fwd(stream(), ptr(z_), ptr(x_), ptr(g_), flags.p(), fptr(ls), fptr(ld), ptr(h), ptr(y), fptr(ls_out), fptr(ld_out), fptr(ends), B,
+                                         T, D, code(dt), flags.dtype),
+                  "mrx_gated_scan_fwd");
+        } else {   // the scan, and then the gate
+            ends = fresh({2, B, D}, at::kFloat, z_);
+            Tensor first = ends.select(0, 0), last = ends.select(0, 1);
+            at::exp_out(first, ls);
+            const Tensor decay = ld.exp(), decay_last = fresh_like(decay);
+            check(lib.mrx_mingru_scan_fwd(stream(), ptr(z_), ptr(x_), flags.p(), fptr(first), fptr(decay), ptr(h), fptr(last), fptr(decay_last), B, T, D, code(dt),
+                                          flags.dtype),
+                  "mrx_mingru_scan_fwd");
+            y = silu_gate_fwd(h, dense16(g_));
+            ls_out = last.unsqueeze(1).log(), ld_out = decay_last.unsqueeze(1).log();
+        }
     }
     if (need) {
         auto node = record(GatedScanOp{done, log_state.scalar_type()}, z, x, gate, log_state);

@@ -1630,7 +1630,7 @@ int launch_bwd(hipStream_t st, const Gate<S> &gt, const void *a, const void *hx,
         return rc;
     }
     ScanPlan pl = plan_scan(B, T, D, sizeof(E), true, MG, !std::is_same<S, E>::value, a_ti);
-    // five float32 arrays of four elements a lane and eight steps do not fit the wave-split kernel's registers
+    // five float32 arrays of four elements a lane and eight steps do not fit the wave-split kernel's registers (mrx_gated_scan_pays has what that costs)
     if (gt.gate && std::is_same<S, E>::value && !pl.stream && pl.vec == 4) pl.vec = 2, pl.tiles = (int)((D + 127) / 128);
     int rc = MRX_ERR_LAUNCH;
     if (pl.stream) {
@@ -1929,6 +1929,33 @@ extern "C" int mrx_mingru_scan_bwd_segmented(void *stream, const void *z, const 
 {
     if (!aligned(workspace, 8)) return MRX_ERR_INVALID_ARG;
     return mingru_scan_bwd(stream, nullptr, nullptr, nullptr, z, h_tilde, h, done, h0, g, g_last, dz, dh_tilde, dh0, B, T, D, dtype, done_dtype, workspace);
+}
+
+// Where the gate inside the scan takes less time than the operations that it stands for, which read and write flat arrays in whole lines whatever the rows
+// are.  Behind 512 MB of other traffic, us, operations / one; shapes drawn over 3 to 120 million elements, 32 to 1024 columns: of 290 drawn once the rule stood,
+// time by it over time apart is 0.88 forward and 0.91 backward in float32, 0.94 and 0.93 in bfloat16, worst 1.12, 26 of 580 above 1.03.
+extern "C" int mrx_gated_scan_pays(int64_t B, int64_t T, int64_t D, int dtype, int backward)
+{
+    if (!scan_shape_ok(B, T, D) || (dtype != MRX_F32 && dtype != MRX_BF16)) return 0;
+    const bool half = dtype == MRX_BF16;
+    const ScanPlan pl = plan_scan(B, T, D, 4, backward != 0, true, half, false);
+    const int64_t n = B * T * D, row = D * (half ? 2 : 4);
+    if (!backward) {
+        if (n < (half ? 10000000 : 12000000)) return 1;   // launches saved weigh more: bfloat16 878 x 245 x 39 50 / 48, float32 268 x 195 x 86 50 / 49
+        // One more array each way of loads and stores that begin in the middle of a line.  bfloat16, wave-split, rows of no whole lines: 2010 x 675 x 34 191 / 264,
+        // 1006 x 266 x 144 134 / 159, 170 x 521 x 810 235 / 279, at 10 to 15 million 0.97 to 1.11; whole lines 896 x 442 x 192 204 / 204, 1024 x 512 x 256 325 / 271.
+        // Streams of two elements a lane are even (0.87 to 1.06), of one 68282 x 25 x 37 269 / 317.
+        if (half) return row % 128 == 0 || (pl.stream && pl.vec > 1);
+        // float32: single elements, unless a row is one wave's: 4274 x 38 x 131 145 / 173, 271 x 963 x 68 155 / 184, 25735 x 26 x 44 194 / 213; 28605 x 70 x 43 503 / 463,
+        // rows of whole half lines 17302 x 23 x 144 305 / 259, two elements and more 0.59 to 1.06
+        return pl.vec > 1 || row % 64 == 0 || (!pl.stream && D <= 64);
+    }
+    // whole rows streaming, few columns each: single elements of rows narrower than a wave, bfloat16 68282 x 25 x 37 394 / 449, float32 1416 x 449 x 49 456 / 515 (43772 x 30 x 40
+    // 521 / 495), bfloat16 also four elements of rows narrower than two, 6904 x 106 x 41 281 / 340, 2514 x 125 x 124 260 / 281; whole half lines 16384 x 64 x 128 533 / 380
+    if (pl.stream && row % 64 && n >= 9000000 && ((pl.vec == 1 && D < 64) || (half && pl.vec == 4 && D < 128))) return 0;
+    // float32 plans of four elements run with two (launch_bwd): a second column tile that is half empty costs more than the pass, 917 x 141 x 165 200 / 250, 2843 x 220 x 158
+    // 935 / 1075, 674 x 76 x 147 81 / 87; whole half lines 563 x 667 x 144 590 / 502, wider rows 3939 x 115 x 216 876 / 832
+    return half || pl.stream || pl.vec < 4 || D > 208 || row % 64 == 0 || n < 6000000;
 }
 
 extern "C" int mrx_gated_scan_fwd(void *stream, const void *z, const void *h_tilde, const void *gate, const void *done, const float *log_state,

@@ -1,5 +1,6 @@
-"""The gated recurrence in one launch each way (gated_scan: scan.hip with the gate inside) against the operations it stands for -- exp of the carry, the MinGRU
-scan, the gate, the logarithms -- on every kernel that the planner takes for it, at ragged widths, short and long sequences, and with a carry of zero."""
+"""The gated recurrence in one launch each way (gated_scan: scan.hip with the gate inside), or the scan and the gate apart where that is faster, against the operations
+it stands for -- exp of the carry, the MinGRU scan, the gate, the logarithms: the planner's kinds of kernel (wave-split with one, two and four elements a lane, eight and sixteen
+waves, eight and sixteen steps; streams; streams that form the states again), ragged widths, short and long sequences, and a carry of zero."""
 import pytest
 import torch
 
@@ -13,8 +14,12 @@ def _np(t):
     return t.detach().float().cpu().numpy()
 
 
-# few columns and sixteen waves, eight, four; streams; the recomputing stream (2400 x 64 x 700); segments; one step
-SHAPES = [(3, 5, 7), (2, 1, 64), (9, 129, 100), (40, 64, 257), (64, 200, 192), (300, 40, 256), (1100, 33, 130), (700, 70, 512), (4, 900, 48), (600, 24, 4), (2400, 64, 700)]
+# few columns and sixteen waves, eight, four; streams; segments; one step; float32 on four elements a lane, backward on two (300 x 64 x 200, 146 x 113 x 265); streams of two and
+# four elements; states formed again (2400 x 64 x 700, 1024 x 128 x 256 float32); apart forward (380 x 240 x 136 bfloat16, 2100 x 45 x 131 float32), backward (280 x 140 x 165
+# float32) or both ways (7000 x 30 x 59 and 4700 x 64 x 61 bfloat16)
+SHAPES = [(3, 5, 7), (2, 1, 64), (9, 129, 100), (40, 64, 257), (64, 200, 192), (300, 40, 256), (1100, 33, 130), (700, 70, 512), (4, 900, 48), (600, 24, 4), (2400, 64, 700),
+          (300, 64, 200), (146, 113, 265), (32, 128, 256), (200, 520, 70), (5894, 21, 120), (3000, 16, 200), (1024, 128, 256), (380, 240, 136), (2100, 45, 131), (7000, 30, 59),
+          (280, 140, 165), (4700, 64, 61)]
 
 
 @pytest.mark.parametrize("B,T,D", SHAPES)
