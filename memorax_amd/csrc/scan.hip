@@ -1673,7 +1673,7 @@ int launch_bwd(hipStream_t st, const Gate<S> &gt, const void *a, const void *hx,
                                    (const E *)g_last, (S *)da, (S *)db, (E *)dh0, (int)T, D, pl.tiles, pl.nw, a_ti, da_sum, Segments<E>{}, gt);
             };
             auto go = [&](auto ti, auto paced) {
-                if constexpr (MG && !decltype(paced)::value)
+                if constexpr (MG && !decltype(paced)::value && (!std::is_same<S, E>::value || decltype(vc)::value < 4))
                     if (gt.gate) return launch(ti, paced, std::true_type{});
                 launch(ti, paced, std::false_type{});
             };
