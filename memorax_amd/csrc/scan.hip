@@ -1261,20 +1261,24 @@ ScanPlan plan_scan(int64_t B, int64_t T, int64_t D, size_t esize, bool bwd, bool
         // along time on wide vectors gained most -- a workgroup's registers then leave room for others beside it.  us, before -> now.
         const int64_t covered4 = 256 * ntiles(4);
         const bool full = ntiles(4) == 1 ? D >= 176 : 10 * D >= 9 * covered4;
-        // Three rules for float32, each timed against the plan it replaces over shapes drawn after it was fixed, but that the first lost its MinGRU backward by
-        // that draw (n shapes: geometric mean of new / old time, worst; us old -> new).
+        // Three rules for float32, each timed against the plan it replaces over shapes drawn after it was fixed (n shapes: geometric mean of new / old time, worst;
+        // us old -> new); what lost there keeps the old plan, and was drawn again by itself.
         const bool f32 = esize == 4 && !half_storage;
-        // Rows of 65 to 111 floats fit one wave of two elements a lane, half the load instructions of two waves of one.  Forward, MinGRU too: n 67, 0.87, 1.09
-        // (969 x 947 x 72 306 -> 195, 454 x 884 x 88 167 -> 101; 321 x 80 x 104 12.0 -> 13.1); plain backward: n 20, 0.83, 1.06 (902 x 787 x 103 373 -> 217).  Not the
-        // backward of MinGRU: 0.91 over 43, but 812 x 566 x 80 207 -> 298.
+        // Rows of 65 to 111 floats fit one wave of two elements a lane, half the load instructions of two waves of one (96 and more had that before, on eight
+        // waves).  Forward, MinGRU too: n 210, 0.81, 1.06 (969 x 947 x 72 306 -> 195, 454 x 884 x 88 167 -> 101); plain backward: n 110, 0.70, 0.95 (902 x 787 x 103 373 -> 217).
+        // Not the backward of MinGRU: 0.91 over 43, but 812 x 566 x 80 207 -> 298.  Eight waves along time where rows give fewer than two workgroups a compute unit: from
+        // 256 steps on below 700 (646 x 300 x 104 as before), forward from 96 floats on at any length up to 512 (four: 456 x 122 x 102 17.3 -> 19.5, 341 x 255 x 102 MinGRU
+        // 32.1 -> 35.7; 534 x 154 x 105 31.9 -> 29.2).
         if (f32 && D > 64 && D < 112 && T < 128 * TS_MIN && waves2 >= 256 && !(mg && bwd)) {
-            return split(2, nw8 > 4 && T >= 256 && B < 700 ? 8 : nw8 < 4 ? nw8 : 4);
+            const bool eight = T >= 256 ? B < 700 : !bwd && D >= 96 && B <= 512;
+            return split(2, nw8 > 4 && eight ? 8 : nw8 < 4 ? nw8 : 4);
         }
         if (f32 && ragged && bwd) {
-            // MinGRU streams: n 55, 0.85, 1.06 (263 x 469 x 272 315 -> 205, 132 x 274 x 872 238 -> 164; 489 x 339 x 200 180 -> 190).  From 1024 on 10 of 68
-            // shapes lost, up to 1.18.
-            if (mg && D >= 192 && T >= 64 && waves2 >= 512 && waves2 < 1024) return flow(2);
-            // four elements a lane from half as many columns on: n 39, 0.93, 1.01 (254 x 526 x 219 179 -> 136, 179 x 203 x 197 51 -> 41)
+            // MinGRU streams: n 150, 0.92, 1.08 (263 x 469 x 272 315 -> 205, 132 x 274 x 872 238 -> 164).  Not where four elements a lane make between 340 and 512 workgroups and a
+            // row is one of them (33 of 37 shapes lost, 433 x 242 x 234 138 -> 162; 340 x 1414 x 253 784 -> 768, 527 x 189 x 244 168 -> 161) or the sequence is short (246 x 110 x 505
+            // 80 -> 87).  From 1024 on 10 of 68 shapes lost, up to 1.18.
+            if (mg && D >= 192 && T >= 64 && waves2 >= 512 && waves2 < 1024 && !(cols(4) > 340 && cols(4) <= 512 && (ntiles(4) == 1 || T < 128))) return flow(2);
+            // four elements a lane from half as many columns on: n 60, 0.87, 1.01 (254 x 526 x 219 179 -> 136, 179 x 203 x 197 51 -> 41)
             if (!mg && T >= 128 && waves2 >= 256 && waves2 < 512) return split(4, nw8);
         }
         // (*) bfloat16 backward: single elements are 2-byte loads, three or four arrays of them; two per lane and 16 steps
