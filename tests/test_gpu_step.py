@@ -202,6 +202,60 @@ def test_normalised_and_gated_steps_in_place_equal_the_steps_out_of_place(dtype,
         assert torch.equal(og2, og) and torch.equal(Sg_in, Sg), step
 
 
+def _reference_step(kind, q, k, v, beta, g, done, S, z):
+    """One step in float64: (o, S', z')."""
+    q, k, v, S, z = (t.double() for t in (q, k, v, S, z))
+    keep = 1.0 - done.double()[:, None, None, None]
+    if kind == "normalised":
+        q, k = (torch.where(t > 0, t + 1, t.exp()) for t in (q, k))
+    if kind == "deltanet":
+        k, beta = torch.nn.functional.normalize(k, dim=-1), torch.sigmoid(beta.double())
+    S = S * keep * (g.double().exp()[..., None, None] if kind == "gated" else 1.0)
+    u = beta.double()[..., None] * (v - torch.einsum("bhvk,bhk->bhv", S, k)) if kind.startswith("delta") else v
+    S, z = S + u[..., None] * k[:, :, None], z * keep[..., 0] + k
+    o = torch.einsum("bhvk,bhk->bhv", S, q)
+    return (o / (q * z).sum(-1, keepdim=True).clamp_min(1e-6) if kind == "normalised" else o), S, z
+
+
+@pytest.mark.parametrize("dims", [(32, 32), (16, 16), (8, 24), (32, 8)])
+@pytest.mark.parametrize("B", [255, 256])   # four heads: just below the 1024 states from which on one wave has a narrow state, and there
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("kind", ["normalised", "gated", "delta", "deltanet"])
+def test_steps_of_many_narrow_states(kind, dtype, B, dims):
+    """Rows of a state by one wave and by four, of every form: against float64, and where the state (and the key sum) is updated in place."""
+    from memorax_amd import _lib
+    from memorax_amd import kernels as K
+    (dk, dv), H = dims, 4
+    gen = torch.Generator(device="cuda").manual_seed(B + dk + dv)
+    rand = lambda *s: torch.randn(*s, device="cuda", generator=gen)  # noqa: E731
+    q, k, v, beta = rand(B, H, dk).to(dtype), rand(B, H, dk).to(dtype), rand(B, H, dv).to(dtype), torch.rand(B, H, device="cuda", generator=gen).to(dtype)
+    g, done, S, z = -torch.rand(B, H, device="cuda", generator=gen), torch.rand(B, device="cuda", generator=gen) < 0.2, rand(B, H, dv, dk), rand(B, H, dk).abs() + 1.0
+    if kind == "delta":
+        k = torch.nn.functional.normalize(k.float(), dim=-1).to(dtype)
+    want_o, want_S, want_z = _reference_step(kind, q, k, v, beta, g, done, S, z)
+    print(f"case many narrow states {kind} {dtype} {B} {dims}", flush=True)
+
+    def step(S, z, inplace):
+        if kind == "normalised":
+            return K.linear_attn_step(q, k, v, done, S, z, "elu1", True, 1e-6, inplace=inplace)
+        if kind == "gated":
+            return *K.gated_linear_attn_step(q, k, v, g, done, S, inplace=inplace), None
+        if kind == "delta":
+            return *K.delta_rule_step(q, k, v, beta, done, S, inplace=inplace), None
+        o, to = torch.empty_like(v), S if inplace else torch.empty_like(S)
+        p = [t.data_ptr() for t in (q, k, v, beta, done, S, o, to)]
+        assert _lib.load().mrx_deltanet_step(torch.cuda.current_stream().cuda_stream, *p, B, H, dk, dv, int(dtype == torch.bfloat16), 0) == 0
+        return o, to, None
+
+    o, S2, z2 = step(S, z, False)
+    tol = TOL_BF16 if dtype == torch.bfloat16 else 1e-5
+    assert relerr(o, want_o.cpu().numpy()) <= tol
+    assert relerr(S2, want_S.cpu().numpy()) <= (tol if kind == "deltanet" else 1e-5)   # (there bfloat16 rounds the normalised key and the gate)
+    assert z2 is None or relerr(z2, want_z.cpu().numpy()) <= 1e-5
+    o3, S3, z3 = step(S, z, True)
+    assert S3.data_ptr() == S.data_ptr() and torch.equal(o3, o) and torch.equal(S3, S2) and (z3 is None or torch.equal(z3, z2))
+
+
 def test_step_rejects_bad_arguments():
     from memorax_amd import _lib
     lib = _lib.load()
