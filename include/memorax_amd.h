@@ -737,8 +737,8 @@ int mrx_gated_recurrence_act(void *stream, const float *x, const float *scale, c
  * most 256 with a closing layer; its own K a multiple of 8 up to 512; norm: an RMS norm, or none).
  * mrx_closed_row_dense: out, and then mrx_row_dense of its rows.  y_l: (rows, n_out[l]) in y_dtype.
  * mrx_closed_gated_recurrence_act: out, and then mrx_gated_recurrence_act of its rows; without closing (NULL) of x.
- * Weights of both layers in w_dtype; every array on a 16-byte boundary (biases of the opening layers as their type is).  MRX_ERR_UNSUPPORTED: sizes whose
- * rows do not fit a workgroup's LDS beside the weights. */
+ * Weights of both layers in w_dtype; every array on a 16-byte boundary (biases of the opening layers as their type is).  MRX_ERR_UNSUPPORTED: sizes beyond
+ * these (what is within them fits a workgroup's LDS). */
 typedef struct mrx_closing {
     const void *rows;        /* (rows, K) in row_dtype */
     const float *scale;      /* (K) or NULL */

@@ -133,10 +133,45 @@ def test_closed_row_dense(rows, K, F, ns, wd, product, xd, norm):
     rc = lib.mrx_closed_row_dense(stream, ctypes.byref(c), p(scale), p(nbias), norm, arr([p(w) for w in ws]), arr([p(b) for b in bs]), arr([p(y) for y in ys]),
                                   (ctypes.c_int64 * len(ns))(*ns), len(ns), rows, F, code(wd), 0, code(xd), code(product), 1e-5)
     torch.cuda.synchronize()
-    assert rc in (0, -2) and (rc == 0 or K > 256)   # wide float32 rows need not fit
-    if rc == 0:
-        # float32 sums of up to 512 products in another order; with bfloat16 roundings behind them a result may round the other way
-        tol = 1e-5 if product == F32 and xd == F32 else 1e-2
-        assert relerr(out, _np(want_x)) <= tol
-        for y, w in zip(ys, want):
-            assert relerr(y, _np(w)) <= tol
+    assert rc == 0
+    # float32 sums of up to 512 products in another order; with bfloat16 roundings behind them a result may round the other way
+    tol = 1e-5 if product == F32 and xd == F32 else 1e-2
+    assert relerr(out, _np(want_x)) <= tol
+    for y, w in zip(ys, want):
+        assert relerr(y, _np(w)) <= tol
+
+
+@pytest.mark.parametrize("rows,K,F,N", [(1, 8, 8, 8), (15, 24, 56, 60), (16, 512, 64, 64), (17, 72, 128, 200), (33, 264, 136, 68), (49, 256, 256, 256), (16, 512, 256, 512),
+                                        (1040, 128, 128, 256)])   # the last: two workgroups on a compute unit
+@pytest.mark.parametrize("wd,product", [(F32, F32), (F32, BF), (BF, BF)])
+@pytest.mark.parametrize("norm", [0, 1, 2])
+def test_closed_gated_recurrence(rows, K, F, N, wd, product, norm):
+    """The closing layer and the gated step in one launch against the row kernel and then the gated step alone."""
+    from memorax_amd import _lib
+    lib, n = _lib.load(), _lib.native()
+    g = torch.Generator(device="cuda").manual_seed(rows + K + F + N)
+    rand = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    code = lambda dt: 0 if dt == F32 else 1  # noqa: E731
+    h, res = rand(rows, 1, K).to(product), rand(rows, 1, F)
+    cs, cw, cb = rand(K), (rand(F, K) * K ** -0.5).to(wd), rand(F)
+    scale, nbias = rand(F) if norm else None, rand(F) if norm == 2 else None
+    ws = [(rand(N, F) * F ** -0.5).to(wd) for _ in range(3)]
+    done = torch.rand(rows, 1, device="cuda", generator=g) < 0.3
+    ls, ld = rand(rows, 1, N), -torch.rand(rows, 1, N, device="cuda", generator=g)
+    ls[0] = -float("inf")   # a carry of zero
+    p = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    st = torch.cuda.current_stream().cuda_stream
+    fresh = lambda: [torch.full((rows, 1, N), float("nan"), device="cuda", dtype=dt) for dt in (product, product, F32, F32)]  # noqa: E731
+    print(f"case closed gated {rows} {K} {F} {N} {wd} {product} {norm}", flush=True)
+    want_x = n.row_dense(h, norm % 2, cs if norm % 2 else None, None, 1e-6, product == BF, [cw], [cb], product, F32, res)[0]
+    want, got, out = fresh(), fresh(), torch.full_like(want_x, float("nan"))
+    tail = lambda o: (*(p(w) for w in ws), p(done), p(ls), p(ld), *(p(t) for t in o), rows, F, N, code(wd), code(product), 0, 1e-5)  # noqa: E731
+    assert lib.mrx_gated_recurrence_act(st, p(want_x), p(scale), p(nbias), norm, *tail(want)) == 0
+    c = _Closing(p(h), p(cs) if norm % 2 else None, p(cw), p(cb), p(res), p(out), K, norm % 2, product == BF, code(product), 0, 1e-6)
+    assert lib.mrx_closed_gated_recurrence_act(st, ctypes.byref(c), None, p(scale), p(nbias), norm, *tail(got)) == 0
+    torch.cuda.synchronize()
+    # each on its own scale: x' as above; z, the gated state and the state's exponential behind one more product of up to 256 terms and its roundings
+    tol = 1e-5 if product == F32 else 1e-2
+    assert relerr(out, _np(want_x)) <= tol
+    for a, b in ((got[0], want[0]), (got[1], want[1]), (got[2].exp(), want[2].exp()), (got[3], want[3])):
+        assert relerr(a, _np(b)) <= 2 * tol
