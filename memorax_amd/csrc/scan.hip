@@ -278,7 +278,8 @@ constexpr int MAX_SEGMENTS = 64;
 // and the gate's gradient beside the others; and the carry in the cell's logarithms.  What that saves is a pass: forward h is not read back (six bytes an
 // element of bfloat16 arrays instead of eight, besides the scan's own), backward dh is neither written nor read, nor h a second time (sixteen instead
 // of twenty-two), and four launches over the carries.  1024 x 128 x 256 bfloat16, us, the launches it stands for / one: forward 43 + 31
-// + 4 x 4.7 / 77, backward 76 + 55 / 105.
+// + 4 x 4.7 / 77, backward 76 + 55 / 105.  float32, behind 512 MB of other traffic: 157 / 125 and 255 / 189; 512 x 1024 x 512, where the scan by itself is the paced
+// kernel, 1256 / 903 and 2210 / 1484.  Where it does not pay: mrx_gated_scan_pays.
 // The backward reads the states before the first step and behind the last one (first, last: (B,D)) as the forward leaves them for it, not the carries
 // in the caller's hands: those may be overwritten meanwhile, and a state is not what comes back from its logarithm.
 template <typename S> struct Gate {
@@ -1262,23 +1263,27 @@ ScanPlan plan_scan(int64_t B, int64_t T, int64_t D, size_t esize, bool bwd, bool
         const int64_t covered4 = 256 * ntiles(4);
         const bool full = ntiles(4) == 1 ? D >= 176 : 10 * D >= 9 * covered4;
         // Three rules for float32, each timed against the plan it replaces over shapes drawn after it was fixed (n shapes: geometric mean of new / old time, worst;
-        // us old -> new); what lost there keeps the old plan, and was drawn again by itself.
+        // us old -> new).  What lost in earlier draws keeps the old plan; the figures are of a last one.
         const bool f32 = esize == 4 && !half_storage;
         // Rows of 65 to 111 floats fit one wave of two elements a lane, half the load instructions of two waves of one (96 and more had that before, on eight
-        // waves).  Forward, MinGRU too: n 210, 0.81, 1.06 (969 x 947 x 72 306 -> 195, 454 x 884 x 88 167 -> 101); plain backward: n 110, 0.70, 0.95 (902 x 787 x 103 373 -> 217).
-        // Not the backward of MinGRU: 0.91 over 43, but 812 x 566 x 80 207 -> 298.  Eight waves along time where rows give fewer than two workgroups a compute unit: from
-        // 256 steps on below 700 (646 x 300 x 104 as before), forward from 96 floats on at any length up to 512 (four: 456 x 122 x 102 17.3 -> 19.5, 341 x 255 x 102 MinGRU
-        // 32.1 -> 35.7; 534 x 154 x 105 31.9 -> 29.2).
+        // waves).  Forward, MinGRU too: n 240, 0.78, 1.05 (969 x 947 x 72 306 -> 195, 454 x 884 x 88 167 -> 101); plain backward: n 120, 0.69, 1.02 (902 x 787 x 103 373 -> 217).
+        // Not the backward of MinGRU: 0.91 over 43, but 812 x 566 x 80 207 -> 298.  Eight waves along time where rows give no
+        // more than two workgroups a compute unit (eight / four: 512 x 600 x 70 67 / 71, MinGRU 69 / 76, backward 122 / 129; 690 x 600 x 90 111 / 107, 116 / 105, 223 / 194): from
+        // 256 steps on, forward from 96 floats on at any length (456 x 122 x 102 17.3 / 19.5, 341 x 255 x 102 MinGRU 32.1 / 35.7; 534 x 154 x 105 31.9 / 29.2) and beyond
+        // 1024 rows as before (1273 x 230 x 101 81 / 85, 1094 x 123 x 107 MinGRU 42 / 45, 2420 x 1022 x 100 630 / 642).
         if (f32 && D > 64 && D < 112 && T < 128 * TS_MIN && waves2 >= 256 && !(mg && bwd)) {
-            const bool eight = T >= 256 ? B < 700 : !bwd && D >= 96 && B <= 512;
+            const bool eight = !bwd && D >= 96 ? B <= 512 || B > 1024 : B <= 512 && T >= 256;
             return split(2, nw8 > 4 && eight ? 8 : nw8 < 4 ? nw8 : 4);
         }
         if (f32 && ragged && bwd) {
-            // MinGRU streams: n 150, 0.92, 1.08 (263 x 469 x 272 315 -> 205, 132 x 274 x 872 238 -> 164).  Not where four elements a lane make between 340 and 512 workgroups and a
-            // row is one of them (33 of 37 shapes lost, 433 x 242 x 234 138 -> 162; 340 x 1414 x 253 784 -> 768, 527 x 189 x 244 168 -> 161) or the sequence is short (246 x 110 x 505
-            // 80 -> 87).  From 1024 on 10 of 68 shapes lost, up to 1.18.
-            if (mg && D >= 192 && T >= 64 && waves2 >= 512 && waves2 < 1024 && !(cols(4) > 340 && cols(4) <= 512 && (ntiles(4) == 1 || T < 128))) return flow(2);
-            // four elements a lane from half as many columns on: n 60, 0.87, 1.01 (254 x 526 x 219 179 -> 136, 179 x 203 x 197 51 -> 41)
+            // MinGRU streams: n 120, 0.89, 1.04 (263 x 469 x 272 315 -> 205, 132 x 274 x 872 238 -> 164, 622 x 1037 x 208 864 -> 613).  Not where four elements a lane make between 340
+            // and 512 workgroups and a row is one of them (33 of 37 shapes lost, 433 x 242 x 234 138 -> 162; 340 x 1414 x 253 784 -> 768, 527 x 189 x 244 168 -> 161), nor, where
+            // either is so, in short sequences (246 x 110 x 505 80 -> 87, 676 x 146 x 193 118 -> 145).  From 1024 on 10 of 68 shapes lost, up to 1.18.
+            if (mg && D >= 192 && T >= 64 && waves2 >= 512 && waves2 < 1024) {
+                const bool between = cols(4) > 340 && cols(4) <= 512, one = ntiles(4) == 1;
+                if (!(between && one) && (T >= 256 || !(between || one))) return flow(2);
+            }
+            // four elements a lane from half as many columns on: n 120, 0.87, 1.02 (254 x 526 x 219 179 -> 136, 179 x 203 x 197 51 -> 41)
             if (!mg && T >= 128 && waves2 >= 256 && waves2 < 512) return split(4, nw8);
         }
         // (*) bfloat16 backward: single elements are 2-byte loads, three or four arrays of them; two per lane and 16 steps
