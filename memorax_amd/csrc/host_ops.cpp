@@ -2799,7 +2799,7 @@ bool act_block(ActBlock &k, const Tensor &x, const py::tuple &spec, const py::tu
 //     beyond a workgroup for each compute unit      qkv 512 wide 64 features 2048 rows 20.8 / 21.3, gated 512 wide 1024 rows 17.2 / 21.2, 1024 wide 23.6 / 37.7
 //     gated recurrences, by the bytes of weights a workgroup reads
 //                                                   256 wide 256 features 32 rows 12.2 / 11.8, weights in float32 (448 KB) 15.2 / 15.3, 512 wide (704 KB) 17.9 / 19.3;
-//                                                   float32 products 512 wide 128 features (352 KB) 19.4 / 18.8, 256 wide 256 features (448 KB) 16.4 / 18.2
+//                                                   float32 products 1024 wide 128 features 256 rows (352 KB) 19.4 / 18.8, 256 wide 256 features (448 KB) 16.4 / 18.2
 //     other layers, half the compute units at work  256 wide 256 features 1024 rows 14.0 / 11.8, weights in float32 512 wide 512 rows (768 KB) 18.5 / 18.2;
 //                                                   float32 products 512 wide 128 features 512 rows (384 KB) 19.0 / 17.5, 256 wide 256 features 1024 rows (512 KB) 19.5 / 20.5
 //     fewer: apart, the closing layer has more workgroups than rows fill here, and its weights come in by all of them
