@@ -8,8 +8,8 @@ synthetic batch of benchmark configuration 4 (B=64, H=8, T=1024, d=64, bf16 inpu
 fp32 state, reset mask Bernoulli(0.002)); inputs are resident in HBM before the
 timed region.  Prints ONE JSON line.  Only one GPU is used: --gpus > 1 exits.
 
-The other configurations (diagonal scan: configs[0]; linear attention: configs[1], configs[2];
-the sequence kernels of the torso: configs[4]) are timed first and reported as secondary blocks of
+The other configurations (1: diagonal scan; 2 and 3: linear attention;
+5: the sequence kernels of the torso) are timed first and reported as secondary blocks of
 the same line; the headline step is timed after them, on a device that is already at its clocks.
 """
 from __future__ import annotations
@@ -232,7 +232,7 @@ def main() -> int:
         "dtype": "bf16",
         "data": "synthetic",
         "clock_ramp_ms": args.ramp_ms,
-        "config": {"workload": "configs[3]: DeltaNet delta rule fwd+bwd, B=64 H=8 T=1024 d=64, "
+        "config": {"workload": "DeltaNet delta rule fwd+bwd, B=64 H=8 T=1024 d=64, "
                                f"bf16 in / fp32 state, chunk {C}, resets p=0.002"
                                },
         "ms_per_step_merged_resets": None if dt_merged is None else dt_merged * 1e3,
@@ -528,7 +528,7 @@ def bench_scan(torch, K):
 
 
 def bench_linear_attention(torch, K, np, dev):
-    """Configuration 2 (configs[1]: fp32, elu+1, resets) and configuration 3 (configs[2]: bf16, no resets),
+    """Configuration 2 (64x256x4x64 fp32, elu+1, resets) and configuration 3 (256x4096x8x64 bf16, no resets),
     forward + backward, with the fractions of the roofline that binds each on paper: the fp32 matrix
     peak for configuration 2 (41 flop/B against a balance of 20), HBM for configuration 3."""
     res = {}
@@ -763,7 +763,7 @@ def bench_block_kernels(torch, K):
 
 
 def bench_torso_kernels(torch, K):
-    """Configuration 5 (configs[4]), the sequence kernels of one update: 4 blocks x (DeltaNet H=4, d=64
+    """Configuration 5, the sequence kernels of one update: 4 blocks x (DeltaNet H=4, d=64
     forward + backward, diagonal recurrence forward + backward) over B=1024 envs x T=128, done p=0.01.
     The DeltaNet cell calls the kernels with its prologue inside (key normalisation and gate sigmoid on
     the raw projections, gradients taken back through them): that is the figure reported; the plain
@@ -863,7 +863,7 @@ def cpu_baseline(np, x, do_np):
     dt = (time.perf_counter() - t0) / reps
     T = sl["q"].shape[1]
     return {"value": Bs * T / dt, "unit": "tokens/s", "cores": cores, "kind": "port",
-            "sample": f"all {Bs} batch rows of configs[3] (H=8, T={T}, d=64), fwd+bwd, mean of {reps} runs after "
+            "sample": f"all {Bs} batch rows of the step's workload (H=8, T={T}, d=64), fwd+bwd, mean of {reps} runs after "
                       f"a warm-up, sequential recurrence in C (fp32 state), OpenMP over (b,h); {dt:.2f} s per run"}
 
 

@@ -2,7 +2,7 @@
 
 TEST INFRASTRUCTURE ONLY.  Nothing under this package is part of the shipped
 product: it is imported by ``tests/``, by ``__graft_entry__.smoke()`` and by the
-``cpu_baseline`` leg of ``bench.py`` as the checker / the timed CPU baseline,
+``cpu_baseline`` leg of ``bench.py`` as the oracle / the timed CPU baseline,
 never by ``memorax_amd``.
 
 Contents

@@ -2,7 +2,7 @@
  * (forward + analytic backward).
  *
  * TEST INFRASTRUCTURE ONLY: loaded by tests/, __graft_entry__.smoke() and the
- * cpu_baseline leg of bench.py as the checker / timed CPU baseline.  The product
+ * cpu_baseline leg of bench.py as the oracle / timed CPU baseline.  The product
  * library never links or loads it.
  *
  * Each function is pinned (tests/test_oracle_c.py) against the NumPy fp64
